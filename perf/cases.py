@@ -14,7 +14,9 @@ their real width (every layer of a stack costs the same) and their whole vocabul
 
 Weights are random and the same in every case of a model (a server loads them once); prompts, contexts, cached keys
 and values and candidates come from the seed.  Cached rows hold what the projections of normalised rows give (normal,
-standard deviation 1.28); routers are as decisive as trained ones (logits a few units apart).
+standard deviation 1.28); routers are as decisive as trained ones (logits a few units apart); the embeddings of the fp8
+and routed models are scaled so that a layer changes the residual stream by a fraction, as in trained ones (else the
+rounding of e4m3 activations compounds from layer to layer until two correct runs have little in common).
 """
 import gc
 import json
@@ -45,6 +47,7 @@ BLOCK = 16                     # tokens per cache block, the engine's default
 WEIGHT_SEED = 1234
 KV_STD = 1.28                  # 0.02 * sqrt(4096): keys and values of unit-RMS rows
 LAYERS = {"llama": 4, "mixtral": 2, "mixtral-fp8": 2, "e5": 3}
+STREAM = {"mixtral": 256.0, "mixtral-fp8": 256.0, "e5": 256.0}   # embedding scale (a power of two: exact in bf16)
 MAX_POS = 8192
 MODEL_LEN = 4096               # the engine's default limit: how wide its block tables are
 ENCODERS = {"bge-small": "bge-small-en-v1.5", "bge-base": "bge-base-en-v1.5", "bge-large": "bge-large-en-v1.5"}
@@ -253,9 +256,12 @@ def _make(name):
     if name == "llama":
         return LlamaModel(_decoder_cfg(name), device=DEV, seed=WEIGHT_SEED, max_position=MAX_POS)
     if name.startswith("mixtral"):
-        return MixtralModel(_decoder_cfg(name), device=DEV, seed=WEIGHT_SEED, max_position=MAX_POS, fp8=name == "mixtral-fp8")
+        m = MixtralModel(_decoder_cfg(name), device=DEV, seed=WEIGHT_SEED, max_position=MAX_POS, fp8=name == "mixtral-fp8")
+        m.embed.mul_(STREAM[name])
+        return m
     if name == "e5":
         m = LlamaModel(_decoder_cfg(name), device=DEV, seed=WEIGHT_SEED, max_position=MAX_POS, fp8_dense=True, fold_norms=False)
+        m.embed.mul_(STREAM[name])
         return DecoderEmbedder(m, max_tokens=512)
     return _make_layer_list(name)
 
@@ -679,6 +685,12 @@ def _rope(x, positions, base, dims, scaling=None, pairs="half"):
     return torch.cat([r, x[..., dims:]], -1)
 
 
+def _fp8(w):
+    """What e4m3 weights with one scale per output channel hold."""
+    s = w.float().abs().amax(-1).clamp(min=1e-12) / 448.0
+    return (w.float() / s.unsqueeze(-1)).to(torch.float8_e4m3fn).to(F64) * s.to(F64).unsqueeze(-1)
+
+
 def _experts(h, z_ids, z_w, weights):
     out = torch.zeros_like(h)
     for e, (gate, up, down) in enumerate(weights):
@@ -689,9 +701,9 @@ def _experts(h, z_ids, z_w, weights):
     return out
 
 
-def _exact_llama(name, x_ids, positions, attend, keep):
+def _exact_llama(name, x_ids, positions, attend, keep, logits=True):
     """Llama-family forward; ``attend(layer, q, k, v)`` runs the attention.  The weights are drawn as the models draw
-    theirs from a seed."""
+    theirs from a seed (fp8: the rounded weights; activations stay as they are)."""
     c = _decoder_cfg(name)
     g = torch.Generator(device=DEV).manual_seed(WEIGHT_SEED)
     d, D, H, G, std = c.hidden, c.head_dim, c.heads, c.kv_heads, 0.02
@@ -700,10 +712,10 @@ def _exact_llama(name, x_ids, positions, attend, keep):
         return (torch.randn(*shape, generator=g, device=DEV, dtype=F32) * s).to(BF16)
 
     small = std / math.sqrt(2 * c.layers)
-    cast = lambda w: w.to(F64)  # noqa: E731
-    x = rnd(c.vocab_size, d)[x_ids].to(F64)
+    cast = _fp8 if name in ("mixtral-fp8", "e5") else (lambda w: w.to(F64))
+    x = rnd(c.vocab_size, d)[x_ids].to(F64) * STREAM.get(name, 1.0)
     for li in range(c.layers):
-        if name == "mixtral":
+        if c.num_experts:
             wqkv = torch.cat([rnd(H * D, d), rnd(G * D, d), rnd(G * D, d)])
             wo, router = rnd(d, H * D, s=small), rnd(c.num_experts, d, s=0.1)
             w1, w3, w2 = rnd(c.num_experts, c.ffn, d), rnd(c.num_experts, c.ffn, d), rnd(c.num_experts, d, c.ffn, s=small)
@@ -717,14 +729,15 @@ def _exact_llama(name, x_ids, positions, attend, keep):
             a, x = a[keep], x[keep]
         x = x + a.reshape(x.shape[0], -1) @ cast(wo).T
         h = _unit(x, c.rms_eps)
-        if name == "mixtral":
+        if c.num_experts:
             top = torch.topk(h @ router.to(F64).T, c.experts_per_token, -1)
             x = x + _experts(h, top.indices, torch.softmax(top.values, -1),
                              [(lambda e=e: cast(w1[e]), lambda e=e: cast(w3[e]), lambda e=e: cast(w2[e])) for e in range(c.num_experts)])
         else:
             w = cast(gu)
             x = x + (_silu(h @ w[:c.ffn].T) * (h @ w[c.ffn:].T)) @ cast(w2).T
-    return _unit(x, c.rms_eps) @ rnd(c.vocab_size, d).to(F64).T
+    h = _unit(x, c.rms_eps)
+    return h @ rnd(c.vocab_size, d).to(F64).T if logits else h
 
 
 def _exact_decode_llama(case, seed):
@@ -924,8 +937,6 @@ def _exact_bert(name, texts):
 
 def exact(case, seed):
     path, name = case["path"], case.get("model")
-    if name in ("mixtral-fp8", "e5"):
-        return None   # activations of three mantissa bits: 64 bits are 0.1 to 0.3 away from any fp8 kernels, which measures the format
     if path == "sample":
         if not case["logprobs"]:
             return None     # whole numbers only
@@ -934,6 +945,10 @@ def exact(case, seed):
         return {"token": None, "logprob": None, "top_ids": None, "top_logprobs": top}
     if path in ("embed", "consensus"):
         texts = _texts(case, seed)
+        if name == "e5":
+            lens, ids, pos, last = _packed([np.asarray(t, np.int64) for t in texts[0]])
+            h = _exact_llama("e5", ids, pos, lambda li, q, k, v: _attend(q, k, v, lens, 128 ** -0.5, True), last, logits=False)
+            return {"embedding": torch.nn.functional.normalize(h, dim=-1)}
         E = _exact_bert(name, [t for r in texts for t in r])
         if path == "embed":
             return {"embedding": E}
