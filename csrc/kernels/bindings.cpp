@@ -32,6 +32,8 @@ int lwc_rms_rowsumsq(const void*, float*, int, int, hipStream_t);
 int lwc_skinny_gemm(const void*, const void*, void*, const void*, int, int, int, int, int, int, hipStream_t);
 int lwc_gemm8g_fp8(const void*, const void*, void*, const int*, const int*, const float*, const float*, int, int, int,
                    int, int, int, int, int, int, const void*, void*, int, hipStream_t);
+int lwc_gemm8g_bf16(const void*, const void*, void*, const int*, const int*, int, int, int, int, int, int, int, int, int,
+                    hipStream_t);
 int lwc_moe_route(const void*, int, int, int, int*, float*, int*, int*, int*, hipStream_t);
 int lwc_moe_router(const void*, int, const void*, int, int, int, int, int*, float*, int*, int*, int*, void*,
                    hipStream_t);
@@ -489,6 +491,32 @@ void rms_rowsumsq(const at::Tensor& x, at::Tensor& ss) {
   TORCH_CHECK(x.dim() == 2 && ss.numel() >= x.size(0), "rms_rowsumsq: x [M, d], ss [>= M]");
   CHECK_RC(lwc_rms_rowsumsq(x.data_ptr(), ss.data_ptr<float>(), (int)x.size(0), (int)x.size(1), cur_stream()),
            "rms_rowsumsq");
+}
+
+// grouped bf16 GEMM on the 8-phase schedule (gemm8g.hip): A [rows_a, K], W [G, N, K], C [rows, N] (swiglu: [rows, N / 2],
+// W's rows gate / up interleaved in blocks of 32); row_off [G + 1] int32 and a_rows [rows] int32 on the device.
+void gemm8g_bf16(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const at::Tensor& row_off, int64_t max_slots,
+                 const c10::optional<at::Tensor>& a_rows, bool swiglu) {
+  CHECK_GPU(A); CHECK_GPU(W); CHECK_GPU(C); CHECK_BF16(A); CHECK_BF16(W); CHECK_BF16(C); CHECK_CONTIG(W);
+  CHECK_DTYPE(row_off, at::kInt); CHECK_CONTIG(row_off);
+  TORCH_CHECK(A.dim() == 2 && A.stride(1) == 1 && C.dim() == 2 && C.stride(1) == 1 && W.dim() == 3, "gemm8g_bf16: layouts");
+  const int G = (int)W.size(0), N = (int)W.size(1), K = (int)W.size(2);
+  TORCH_CHECK(row_off.numel() == G + 1, "gemm8g_bf16: row_off must have G + 1 entries");
+  TORCH_CHECK(A.size(1) == K && C.size(1) == (swiglu ? N / 2 : N), "gemm8g_bf16: shape mismatch");
+  TORCH_CHECK(max_slots >= 0 && max_slots < (int64_t(1) << 24), "gemm8g_bf16: slots");
+  const auto aligned = [](const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.data_ptr()) % 16 == 0; };
+  TORCH_CHECK(aligned(A) && aligned(W) && aligned(C), "gemm8g_bf16: 16-byte aligned operands");
+  const int* ar = nullptr;
+  if (a_rows.has_value() && a_rows->defined()) {
+    CHECK_DTYPE(*a_rows, at::kInt); CHECK_CONTIG(*a_rows);
+    TORCH_CHECK(a_rows->numel() >= C.size(0), "gemm8g_bf16: a_rows shorter than the output rows");
+    ar = a_rows->data_ptr<int>();
+  } else {
+    TORCH_CHECK(C.size(0) <= A.size(0), "gemm8g_bf16: more output rows than A rows");
+  }
+  CHECK_RC(lwc_gemm8g_bf16(A.data_ptr(), W.data_ptr(), C.data_ptr(), row_off.data_ptr<int>(), ar, G, (int)max_slots, N, K,
+                           (int)A.stride(0), (int)C.stride(0), (int)A.size(0), (int)C.size(0), swiglu ? 1 : 0, cur_stream()),
+           "gemm8g_bf16");
 }
 
 void gemm8g_fp8(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::optional<at::Tensor>& row_off,
@@ -971,6 +999,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("knn_topk", &knn_topk);
   m.def("vote_tally", &vote_tally);
   m.def("gemm8g_fp8", &gemm8g_fp8);
+  m.def("gemm8g_bf16", &gemm8g_bf16);
   m.def("ar_alloc", &ar_alloc);
   m.def("ar_open", &ar_open);
   m.def("ar_close", &ar_close);

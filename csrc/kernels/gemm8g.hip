@@ -1,4 +1,4 @@
-// K6g' grouped fp8 GEMM on the 8-phase 256x256 schedule (the MoE expert FFNs of config 5):
+// K6g' grouped GEMM on the 8-phase 256x256 schedule (the MoE expert FFNs), fp8 and bf16:
 //   C[r, :] = (A[a_rows[r], :] . W_g^T) * a_scale[a_rows[r]] * w_scale[g, :]   for rows r of group g
 // with groups = the experts' contiguous row segments row_off[g]..row_off[g+1] (device table, no host
 // sync, graph-capturable) and A gathered through a_rows (MoE dispatch without a permute copy).
@@ -23,6 +23,11 @@
 // XCDs, and XCD x walks the n-tiles n = x (mod 8) with all m-tiles of an n-tile consecutive, so the
 // weight tile of an expert is read from HBM once per XCD and reused from its L2 by the expert's other
 // m-tiles.  Surplus slots (routing decides the m-tile count at run time) exit immediately.
+//
+// bf16 (kBf16 / kBf16Swiglu): the same bytes move through the same pipeline — a K tile of 128 bytes is 64 bf16, a
+// phase's 8 double-length fp8 MFMAs become 16 bf16 ones as in gemm8p — without scales.  Bound by the matrix cores:
+// 8 experts of 4096 rows, [14336, 4096] weights 2988 us (1.29 PF/s; the 128-row kernel 4720), [4096, 7168] 1481 us
+// (1.30 PF/s; 2376), one MI355X.
 #include "common.h"
 
 namespace lwc {
@@ -43,7 +48,7 @@ struct Params {
   const int* a_rows;      // [rows] or null
   const float* a_scale;   // [rows_a]
   const float* w_scale;   // [G][N]
-  int G, N, K, lda, ldc;  // K in elements (= bytes), lda in elements
+  int G, N, K, lda, ldc;  // K and lda in BYTES of A / W rows, ldc in elements of C
   int rows_a;             // rows of A (DMA bounds)
   int slots, n_tiles;     // m-tile slots per n-tile, n-tiles
   int rows_c;             // output rows when row_off is null (dense: G = 1)
@@ -63,6 +68,8 @@ constexpr int kPlain = 0;   // bf16 out, A per-row scaled
 constexpr int kSwiglu = 1;  // SwiGLU epilogue, bf16 out
 constexpr int kMxOut = 2;   // SwiGLU epilogue, e4m3 out with MX block scales (feeds a kMxA GEMM)
 constexpr int kMxA = 3;     // bf16 out, A carries MX block scales
+constexpr int kBf16 = 4;        // bf16 A and W, bf16 out
+constexpr int kBf16Swiglu = 5;  // bf16 A and W, SwiGLU epilogue, bf16 out
 constexpr int kMxLds = 4096;  // kMxA: the two K buffers' scale tiles (256 rows x 4 blocks, twice: see the DMA)
 
 // A block-scaled: the lane's e8m0 scale is byte OP of sa (its row's scale for the lane's K block)
@@ -78,6 +85,12 @@ LWC_DEVICE float4v mfma8s(const uint4v& a0, const uint4v& a1, const uint4v& b0, 
 LWC_DEVICE float quad_max(float x) {
   x = fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, false)));  // ^1
   return fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xF, 0xF, false)));  // ^2
+}
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+LWC_DEVICE float4v mfma16(const uint4v& a, const uint4v& b, const float4v& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                 0, 0);
 }
 
 LWC_DEVICE float4v mfma8(const uint4v& a0, const uint4v& a1, const uint4v& b0, const uint4v& b1, const float4v& c) {
@@ -99,8 +112,9 @@ LWC_DEVICE float silu8(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(
 // silu(gate) * up, and writes [rows, N / 2] bf16 — the [rows, N] gate|up intermediate never reaches HBM.
 template <int MODE>
 __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
-  constexpr bool SWIGLU = MODE == kSwiglu || MODE == kMxOut;
+  constexpr bool SWIGLU = MODE == kSwiglu || MODE == kMxOut || MODE == kBf16Swiglu;
   constexpr bool MXA = MODE == kMxA;
+  constexpr bool BF = MODE == kBf16 || MODE == kBf16Swiglu;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   // ---- work item: XCD-grouped (n-tile, m-slot), then (group, m-tile) of the slot ----
   const int id = blockIdx.x, xcd = id & 7, local = id >> 3;
@@ -207,7 +221,14 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
   uint4v a[4][2], b0[2][2], b1[2][2];
   int sc[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // kMxA: this K tile's scale (block q) of the lane's 8 row fragments
   auto mma = [&](int i0, int j0, const uint4v (&bb)[2][2]) {
-    if constexpr (MXA) {
+    if constexpr (BF) {
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int jj = 0; jj < 2; ++jj) acc[i0 + i][j0 + jj] = mfma16(a[i][s], bb[jj][s], acc[i0 + i][j0 + jj]);
+    } else if constexpr (MXA) {
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -294,23 +315,25 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
   // ---- epilogue: scales in registers, per wave 128 rows x 64 bf16 columns through LDS, 16 B stores ----
   // (row loop outermost: one activation scale live at a time — hoisting all 32 of them spills)
   __builtin_amdgcn_sched_barrier(0);
-  float ws[4];
+  if constexpr (!BF) {
+    float ws[4];
 #pragma unroll
-  for (int jj = 0; jj < 4; ++jj) {
-    const int col = n0 + wc * 64 + jj * 16 + r16;
-    ws[jj] = col < p.N ? p.w_scale[(size_t)g * p.N + col] : 0.f;
-  }
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int rr = 0; rr < 4; ++rr) {
-      int row = m_begin + wr * 128 + i * 16 + 4 * q + rr;
-      if (row >= m_end) row = m_begin;
-      const float as = MXA ? 1.f : p.a_scale[p.a_rows ? p.a_rows[row] : row];
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) acc[i][jj][rr] *= as * ws[jj];
-      __builtin_amdgcn_sched_barrier(0);  // one scale load in flight at a time: no 32-load VGPR burst
+    for (int jj = 0; jj < 4; ++jj) {
+      const int col = n0 + wc * 64 + jj * 16 + r16;
+      ws[jj] = col < p.N ? p.w_scale[(size_t)g * p.N + col] : 0.f;
     }
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int rr = 0; rr < 4; ++rr) {
+        int row = m_begin + wr * 128 + i * 16 + 4 * q + rr;
+        if (row >= m_end) row = m_begin;
+        const float as = MXA ? 1.f : p.a_scale[p.a_rows ? p.a_rows[row] : row];
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) acc[i][jj][rr] *= as * ws[jj];
+        __builtin_amdgcn_sched_barrier(0);  // one scale load in flight at a time: no 32-load VGPR burst
+      }
+  }
   if constexpr (SWIGLU) {
     // columns jj 0, 1 of the wave are gate, jj 2, 3 the matching up columns: 32 outputs per row
     constexpr int CW = 32;
@@ -439,5 +462,33 @@ extern "C" int lwc_gemm8g_fp8(const void* A, const void* W, void* C, const int* 
     gemm8g_kernel<kSwiglu><<<grid, 512, kLdsB, s>>>(p);
   else
     gemm8g_kernel<kPlain><<<grid, 512, kLdsB, s>>>(p);
+  return (int)hipGetLastError();
+}
+
+// Grouped bf16 GEMM on the same schedule: C[r, :] = A[a_rows[r], :] . W_g^T for rows r of group g (a_rows null: A's row
+// r), or with swiglu = 1 silu(gate) * up over rows interleaved in blocks of 32, C [rows, N / 2].  Requires K % 64 == 0,
+// N % 8 == 0 (SwiGLU: N % 64 == 0), lda % 8 == 0, ldc % 8 == 0, rows_a * lda * 2 < 2^31 and 512 * K < 2^31; max_slots >=
+// sum_g ceil(M_g / 256).
+extern "C" int lwc_gemm8g_bf16(const void* A, const void* W, void* C, const int* row_off, const int* a_rows, int G,
+                               int max_slots, int N, int K, int lda, int ldc, int rows_a, int rows_c, int swiglu,
+                               hipStream_t s) {
+  using namespace lwc::g8g;
+  if (!row_off || K % 64 != 0 || K < 64 || N % (swiglu ? 64 : 8) != 0 || lda % 8 != 0 || ldc % 8 != 0 || G < 1) return -1;
+  if ((long long)rows_a * lda * 2 >= (1LL << 31) || 512LL * K >= (1LL << 31)) return -1;
+  if (max_slots <= 0) return 0;
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute((const void*)gemm8g_kernel<kBf16>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsB);
+    (void)hipFuncSetAttribute((const void*)gemm8g_kernel<kBf16Swiglu>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsB);
+    attr = true;
+  }
+  const int n_tiles = (N + 255) / 256, nj = (n_tiles + 7) / 8;
+  Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, nullptr, nullptr,
+           G, N, K * 2, lda * 2, ldc, rows_a, max_slots, n_tiles, rows_c, nj, 1, nullptr, nullptr, 0};
+  const unsigned grid = (unsigned)(nj * max_slots * 8);
+  if (swiglu)
+    gemm8g_kernel<kBf16Swiglu><<<grid, 512, kLdsB, s>>>(p);
+  else
+    gemm8g_kernel<kBf16><<<grid, 512, kLdsB, s>>>(p);
   return (int)hipGetLastError();
 }

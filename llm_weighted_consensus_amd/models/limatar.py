@@ -167,7 +167,9 @@ class LimatarModel(LatentDecoder):
             elif isinstance(e, TopkExpertsSpec):
                 self._router_weight(x, f32(p + "mlp.router"))
                 x["router_b"] = f32(p + "mlp.router.b")
-                x["w_gu"] = torch.stack([torch.cat([t(f"{p}mlp.e{j}.gate"), t(f"{p}mlp.e{j}.up")], 0)
+                # (the grouped GEMMs' epilogue pairs gate and up rows interleaved in blocks of 32)
+                lay = ops.swiglu_interleave if self._use_grouped(cfg.hidden, e.ff) else torch.Tensor.contiguous
+                x["w_gu"] = torch.stack([lay(torch.cat([t(f"{p}mlp.e{j}.gate"), t(f"{p}mlp.e{j}.up")], 0))
                                          for j in range(e.experts)]).contiguous()
                 x["w_down"] = torch.stack([t(f"{p}mlp.e{j}.down") for j in range(e.experts)]).contiguous()
                 if e.shared_ff:
@@ -231,8 +233,8 @@ class LimatarModel(LatentDecoder):
         z = self._router_logits(h2, x)
         _ids, w, row_off, src, row_expert, inv = res32.router(z, None, e.experts, e.top, bias=x["router_b"], renorm=True)
         if self._use_grouped(self.cfg.hidden, e.ff):
-            gu = ops.grouped_gemm(h2, x["w_gu"], row_off, a_rows=src, rows=src.numel())
-            Y = ops.grouped_gemm(res32.glu(gu), x["w_down"], row_off)
+            act = ops.grouped_gemm(h2, x["w_gu"], row_off, a_rows=src, rows=src.numel(), swiglu=True)
+            Y = ops.grouped_gemm(act, x["w_down"], row_off)
         else:
             Y = res32.expert_rows(h2, src, row_expert, row_off, x["w_gu"], x["w_down"])
         shared = None

@@ -216,7 +216,9 @@ class MerudraModel:
                 else:
                     self._mm32 = False
                 if e.experts:
-                    extra["w_gu"] = torch.stack([torch.cat([t(f"{p}mlp.e{x}.gate"), t(f"{p}mlp.e{x}.up")], 0)
+                    # (the grouped GEMMs' epilogue pairs gate and up rows interleaved in blocks of 32)
+                    lay = ops.swiglu_interleave if self._use_grouped(e) else torch.Tensor.contiguous
+                    extra["w_gu"] = torch.stack([lay(torch.cat([t(f"{p}mlp.e{x}.gate"), t(f"{p}mlp.e{x}.up")], 0))
                                                  for x in range(e.experts)]).contiguous()
                     extra["w_down"] = torch.stack([t(f"{p}mlp.e{x}.down") for x in range(e.experts)]).contiguous()
                 else:
@@ -297,6 +299,12 @@ class MerudraModel:
         return RecurrentStatePool.bytes_per_slot(self.state_fields())
 
     # ------------------------------------------------------------------ forward
+    def _use_grouped(self, e) -> bool:
+        """Whether a layer's experts run on the grouped matrix-core GEMMs."""
+        d = self.cfg.hidden
+        return bool(self.dtype == torch.bfloat16 and e.experts and d * e.ff >= self.GROUPED_MIN and d % 64 == 0
+                    and e.ff % 64 == 0 and ops.available())
+
     def _experts(self, h2: torch.Tensor, L: MerudraLayer, e) -> torch.Tensor:
         """Routed experts of the rows h2 -> fp32 [T, d]."""
         x = L.extra
@@ -305,12 +313,9 @@ class MerudraModel:
         else:
             z = F.linear(h2.float(), x["router"])  # router logits in fp32
         _ids, w, row_off, src, row_expert, inv = res32.router(z, x["correction"], e.experts, e.top)
-        d = self.cfg.hidden
-        if (self.dtype == torch.bfloat16 and e.experts and d * e.ff >= self.GROUPED_MIN and d % 64 == 0 and e.ff % 64 == 0
-                and ops.available()):
-            rows = src.numel()
-            gu = ops.grouped_gemm(h2, x["w_gu"], row_off, a_rows=src, rows=rows)
-            Y = ops.grouped_gemm(ops.silu_mul(gu), x["w_down"], row_off)
+        if self._use_grouped(e):
+            act = ops.grouped_gemm(h2, x["w_gu"], row_off, a_rows=src, rows=src.numel(), swiglu=True)
+            Y = ops.grouped_gemm(act, x["w_down"], row_off)
         else:
             Y = res32.expert_rows(h2, src, row_expert, row_off, x["w_gu"], x["w_down"])
         return res32.moe_combine(Y, inv, w, h2)

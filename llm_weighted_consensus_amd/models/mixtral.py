@@ -55,7 +55,7 @@ class MoELayerWeights:
     w2: torch.Tensor              # [E, d, F_local]
     s13: Optional[torch.Tensor]   # fp8 per-channel scales [E, 2F_local]
     s2: Optional[torch.Tensor]    # [E, d]
-    gu_block: int = 0             # >0: w13 rows interleave gate|up in blocks of this size (fp8 path)
+    gu_block: int = 0             # >0: w13 rows interleave gate|up in blocks of this size
 
 
 class MixtralModel(LlamaModel):
@@ -121,16 +121,18 @@ class MixtralModel(LlamaModel):
         w13 = torch.cat([w1[:, r * fl:(r + 1) * fl], w3[:, r * fl:(r + 1) * fl]], dim=1).contiguous()  # [E,2fl,d]
         w2_s = w2[:, :, r * fl:(r + 1) * fl].contiguous()                                             # [E,d,fl]
         s13 = s2 = None
-        if self.fp8:
-            # gate / up rows interleaved in blocks of 32 per expert: the grouped fp8 GEMM applies the SwiGLU
-            # in its epilogue (no [rows, 2F] intermediate), then one per-row e4m3 pass feeds the down GEMM
+        # gate / up rows interleaved in blocks of 32 per expert: the grouped GEMMs of large batches apply the SwiGLU
+        # in their epilogue (no [rows, 2F] intermediate; fp8: then one per-row e4m3 pass feeds the down GEMM)
+        block = 32 if self.fp8 or (w13.is_cuda and fl % 32 == 0) else 0
+        if block:
             w13 = torch.stack([ops.swiglu_interleave(w13[e]) for e in range(w13.shape[0])])
+        if self.fp8:
             w13, s13 = ops.quant_fp8_weight(w13)
             w2_s, s2 = ops.quant_fp8_weight(w2_s)
             # the attention projections are fp8 too (config 5: fp8 MFMA throughout; router and lm_head bf16)
             wqkv, wo_s = ops.Fp8Weight(wqkv), ops.Fp8Weight(wo_s)
         return MoELayerWeights(attn_norm, wqkv, wo_s, mlp_norm, router.contiguous(), w13, w2_s, s13, s2,
-                               32 if self.fp8 else 0)
+                               block)
 
     def _random_init(self, seed: int) -> None:
         cfg, dev, dt = self.full_cfg, self.device, self.dtype
@@ -237,8 +239,11 @@ class MixtralModel(LlamaModel):
                                    swiglu=True)
             aq, as_ = ops.quant_fp8_rows(act)
             return ops.grouped_gemm(aq, L.w2, row_off, a_scale=as_, w_scale=L.s2)
-        gu = ops.grouped_gemm(x, L.w13, row_off, a_rows=a_rows, rows=rows)
-        return ops.grouped_gemm(ops.silu_mul(gu), L.w2, row_off)
+        if L.gu_block == 32:
+            act = ops.grouped_gemm(x, L.w13, row_off, a_rows=a_rows, rows=rows, swiglu=True)
+        else:
+            act = ops.silu_mul(ops.grouped_gemm(x, L.w13, row_off, a_rows=a_rows, rows=rows))
+        return ops.grouped_gemm(act, L.w2, row_off)
 
     _mlp_reads_bf16 = True  # the router projects the bf16 rows
 

@@ -305,7 +305,7 @@ def grouped_gemm(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tensor, max_sl
     (default: ceil(rows/128) + G, enough for any split of the rows into G groups).  ``splits`` > 1 splits
     K over that many workgroups per tile (fp32 atomics into a workspace, then one bf16 pass); default:
     chosen so a small-M launch (MoE decode down projection: 8 experts x 32 column tiles) still puts
-    ~4 workgroups on every CU.  ``swiglu=True``: W's rows are gate / up interleaved in blocks of 32
+    ~4 workgroups on every CU.  Large batches run on the 8-phase 256-row tiles (csrc/kernels/gemm8g.hip), fp8 and bf16.  ``swiglu=True``: W's rows are gate / up interleaved in blocks of 32
     (:func:`swiglu_interleave` per group) and the result is silu(gate) * up [rows, N/2] — from the 8-phase
     kernel's epilogue when it takes the batch, else GEMM + the SwiGLU pass.  ``a_mx`` [K/128, rows, 4] uint8:
     A carries MX block scales (from :func:`grouped_gemm_swiglu_mx`) instead of ``a_scale`` — 8-phase kernel
@@ -317,6 +317,11 @@ def grouped_gemm(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tensor, max_sl
         if out is None:
             out = torch.empty(rows, N, dtype=torch.bfloat16, device=A.device)
         kernels().gemm8g_fp8(A, W, out, row_off, -(-rows // 256) + G, None, None, w_scale.contiguous(), 0, a_mx, None)
+        return out
+    if _use_gemm8g_bf16(A, W, rows, G, N, K, bias, splits, out) and (not swiglu or N % 64 == 0):
+        if out is None:
+            out = torch.empty(rows, N // 2 if swiglu else N, dtype=torch.bfloat16, device=A.device)
+        kernels().gemm8g_bf16(A, W, out, row_off, -(-rows // 256) + G, a_rows, bool(swiglu))
         return out
     if _use_gemm8g(A, W, rows, G, N, K, bias, splits, out) and (not swiglu or N % 64 == 0):
         # large fp8 expert batches (>= ~1 full 256-row tile per expert on average): the 8-phase kernel
@@ -370,6 +375,25 @@ def moe_mx_ok(A: torch.Tensor, W13: torch.Tensor, W2: torch.Tensor, rows: int) -
     if N % 256 or W2.shape[2] != N // 2 or not _use_gemm8g(A, W13, rows, G, N, K, None, None, None):
         return False
     return rows * (N // 2) < (1 << 31) and (N // 256) * rows * 4 < (1 << 31)
+
+
+# rows per group (on average) from which bf16 groups take the 8-phase 256-row tiles.  Below, the 128-row kernel with K split
+# over workgroups reads the weights faster; 8 experts, one MI355X, 128-row kernel / 8-phase, us: [14336, 4096] weights
+# 64 rows a group 235 / 236, 128 rows 336 / 245, 4096 rows 4720 / 2988; [4096, 7168] 133 / 143, 200 / 148, 2376 / 1481
+GROUPED_BF16_8PHASE_ROWS = 96
+
+
+def _use_gemm8g_bf16(A, W, rows, G, N, K, bias, splits, out) -> bool:
+    """Whether bf16 groups run on the 8-phase kernel: enough rows per group, 16-byte rows, 32-bit spans."""
+    if A.dtype != torch.bfloat16 or W.dtype != torch.bfloat16 or bias is not None or (splits or 1) > 1:
+        return False
+    if K % 64 or N % 8 or A.stride(1) != 1 or A.stride(0) % 8 or A.data_ptr() % 16 or W.data_ptr() % 16:
+        return False
+    if A.shape[0] * A.stride(0) * 2 >= (1 << 31) or 512 * K >= (1 << 31):
+        return False
+    if out is not None and (out.stride(1) != 1 or out.stride(0) % 8 or out.data_ptr() % 16):
+        return False
+    return rows >= GROUPED_BF16_8PHASE_ROWS * G
 
 
 def _use_gemm8g(A, W, rows, G, N, K, bias, splits, out) -> bool:

@@ -931,6 +931,39 @@ def test_gemm8g_grouped_fp8_matches_reference(gpu, gather, monkeypatch):
     _close(out, classic, 2e-2, 2e-2)
 
 
+@pytest.mark.parametrize("swiglu", [False, True])
+@pytest.mark.parametrize("gather", [False, True])
+@pytest.mark.parametrize("sizes,N,K", [([300, 0, 17, 700, 256], 640, 192), ([1, 255, 257, 512], 64, 64), ([97, 0, 96], 328, 448)])
+def test_grouped_gemm_bf16_8phase(gpu, sizes, N, K, gather, swiglu, monkeypatch):
+    """bf16 groups on the 8-phase kernel (gemm8g.hip): empty groups, groups of less than, exactly and more than whole
+    256-row tiles, N past the last whole tile, one to seven K tiles, a gathered A, the SwiGLU epilogue; vs fp32 products
+    of the same operands.  Bound: one bf16 rounding (2^-9 relative, doubled) and fp32 sums of K terms."""
+    from llm_weighted_consensus_amd import ops
+
+    if swiglu and N % 64:
+        N = 384
+    monkeypatch.setattr(ops, "GROUPED_BF16_8PHASE_ROWS", 0)
+    torch.manual_seed(12)
+    G, rows = len(sizes), sum(sizes)
+    off = torch.tensor([0] + list(np.cumsum(sizes)), dtype=torch.int32, device=gpu)
+    big = torch.randn(rows + 37, K + 8, device=gpu).to(torch.bfloat16)
+    A = big[:, :K]   # rows of a wider matrix
+    W = (torch.randn(G, N, K, device=gpu) * K ** -0.5).to(torch.bfloat16)
+    a_rows = torch.randperm(rows + 37, device=gpu)[:rows].to(torch.int32) if gather else None
+    Aq = A if gather else A[:rows]
+    guard = torch.full((rows + 2, N // 2 if swiglu else N), float("nan"), dtype=torch.bfloat16, device=gpu)
+    out = ops.grouped_gemm(Aq, W, off, a_rows=a_rows, rows=rows, swiglu=swiglu, out=guard[:rows])
+    assert torch.isnan(guard[rows:]).all() and not torch.isnan(out).any()
+    Ar = A[a_rows.long()].float() if gather else A[:rows].float()
+    o = off.tolist()
+    for g in range(G):
+        ref = Ar[o[g]:o[g + 1]] @ W[g].float().t()
+        if swiglu:
+            v = ref.view(-1, N // 64, 2, 32)
+            ref = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(-1, N // 2)
+        torch.testing.assert_close(out[o[g]:o[g + 1]].float(), ref, rtol=2 ** -8, atol=2e-5)
+
+
 @pytest.mark.parametrize("sizes", [[300, 0, 77, 520], [100, 200, 129, 128]])
 @pytest.mark.parametrize("gather", [False, True])
 @pytest.mark.parametrize("moe_gemm", ["g8", "classic"])
