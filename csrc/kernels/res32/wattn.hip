@@ -184,8 +184,8 @@ extern "C" int r32_window_attn(const float* q, const void* k_cache, const void* 
 // ---------------------------------------------------------------------------------------------------------
 // window_attn_mfma_kernel: prompt portions on the matrix cores (bf16 cache, D = 32 ND, Dv = 16 NV).
 //
-// Workgroup = 4 waves = 64 consecutive query rows of one (item, head); wave w owns rows 16w .. 16w+15 and all
-// four walk the 32-key tiles of the rows' windows, staged through LDS (K row-major; V transposed with the keys
+// Workgroup = 4 waves = 64 QS consecutive query rows of one (item, head); wave w owns rows 16 QS w .. in QS blocks of 16
+// and all four walk the 32-key tiles of the rows' windows, staged through LDS (K row-major; V transposed with the keys
 // permuted so that a lane's eight k-slots of one value column are one 16-byte read).  mfma_f32_16x16x32_bf16, lane l:
 // r16 = l & 15, g = l >> 4:
 //   S^T = K Q^T : A = K rows from LDS, B = Q^T in registers; C reg r = S^T[key 4g + r][query r16], two 16-key
@@ -196,6 +196,12 @@ extern "C" int r32_window_attn(const float* q, const void* k_cache, const void* 
 // The distance bias comes from a table bias[h][i - j] (fp32, built once from r1, r2).  Online softmax in fp32;
 // masked scores never enter it (weights forced to 0), rows are finite-initialised.
 // Positions ascend by one along an item's rows (a portion of a prompt).
+//
+// Bound by the matrix cores and the LDS reads that feed them: the two halves of q and of the weights double the products,
+// and with one 16-row block per wave every product read its own 1 KiB fragment.  Two blocks (QS 2) share it; the row sums
+// stay in their lanes until the end, the reference maximum moves only past 2^8, the four lanes of a row meet by lane swaps,
+// and without a distance bias none is read.  8 x 2048 tokens, 32 heads, one MI355X: 192 / 128 entries, 32 key heads 2270 ->
+// 974 us; 128 / 128, 8 key heads 1462 -> 830 us; one block: 2 x 512 tokens 52 -> 38 us and 44 -> 35 us.
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 
@@ -225,30 +231,35 @@ struct WAttnMfmaParams {
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
+constexpr long long kWideFrom = 512;  // workgroups of 128 rows: two per CU (1 x 2048 tokens x 32 heads: 228 -> 145 us)
 constexpr int kVPad = 40;  // keys per V^T row in LDS (32 + 8: rows stay 16-byte aligned, banks spread)
 
-template <int ND, int NV>
-__global__ void __launch_bounds__(256) window_attn_mfma_kernel(const WAttnMfmaParams p) {
-  constexpr int D = 32 * ND, DV = 16 * NV, KLD = D + 8;
+template <int ND, int NV, int QS, bool BIAS>
+__global__ void __launch_bounds__(256, 2) window_attn_mfma_kernel(const WAttnMfmaParams p) {
+  constexpr int D = 32 * ND, DV = 16 * NV, KLD = D + 8, ROWS = 64 * QS, NB = ROWS + 32;
   constexpr int KCH = (32 * (D / 8) + 255) / 256, VCH = (8 * (DV / 2) + 255) / 256;  // 16-byte words per thread and tile
+  constexpr float kLazy = 8.0f;  // a row's reference maximum moves only when a score passes it by 2^8 (weights stay <= 256)
   // two images of every staged tile: tile kt + 1 is written while tile kt is read (one barrier per tile)
   __shared__ __attribute__((aligned(16))) bf16_t K_s2[2][32 * KLD];
   __shared__ __attribute__((aligned(16))) bf16_t Vt_s2[2][DV * kVPad];
-  __shared__ float bias_s2[2][96];  // the tile's bias by (row - key + 31): rows 0..63 of the workgroup, keys 0..31 of the tile
+  __shared__ float bias_s2[2][BIAS ? NB : 1];  // the tile's bias by (row - key + 31): the workgroup's rows, keys 0..31 of the tile
   extern __shared__ int pages_s[];  // the item's block table over this workgroup's key range (dynamic size)
-  // the last row tiles of an item see the most keys: they start first
-  const int it = blockIdx.x / p.tiles_per_item, tile = p.tiles_per_item - 1 - blockIdx.x % p.tiles_per_item;
+  // all row tiles of one (item, head) on one XCD, so its keys and values pass through one L2; of these the last rows see
+  // the most keys: they start first
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  const int pair = id / p.tiles_per_item, tile = p.tiles_per_item - 1 - id % p.tiles_per_item;
+  const int it = pair / p.H, h = pair % p.H;
   const int q_begin = p.cu_q[it], q_end = p.cu_q[it + 1];
-  const int row0 = q_begin + tile * 64;
+  const int row0 = q_begin + tile * ROWS;
   if (row0 >= q_end) return;
-  const int h = blockIdx.y, H = p.H, g = h / (H / p.G), G = p.G;
-  const int nrows = min(64, q_end - row0);
+  const int H = p.H, g = h / (H / p.G), G = p.G;
+  const int nrows = min(ROWS, q_end - row0);
   const int k_len = p.k_lens[it];
   const int pos0 = p.positions[row0], pos_last = pos0 + nrows - 1;  // positions ascend by one along the rows
   // first visible key of the row at position i: the later of its window's and its chunk's start (ascends with i)
   auto lo_of = [&](int i) { return max(max(0, i - p.window + 1), p.chunk > 0 ? i - i % p.chunk : 0); };
   const int j_lo = lo_of(pos0), j_hi = min(pos_last, k_len - 1);
-  const int tid = threadIdx.x, w = tid >> 6, lane = tid & 63, r16 = lane & 15, g4 = lane >> 4;
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, r16 = lane & 15, g4 = lane >> 4;
   const int* table = p.block_tables + (size_t)it * p.bt_width;
   const int BS = p.block_size, bsh = p.bs_shift;
   // page and offset of key j (a runtime division would cost tens of instructions per load)
@@ -256,31 +267,41 @@ __global__ void __launch_bounds__(256) window_attn_mfma_kernel(const WAttnMfmaPa
   auto page_off = [&](int j) { return j & (BS - 1); };
   typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
 
-  const int qrow = 16 * w + r16;
-  const bool q_valid = qrow < nrows;
-  const int i_q = pos0 + qrow;
-  short8 qhi[ND], qlo[ND];
+  const int wrow = 16 * QS * w;  // this wave's first row; lane r16 of row block qs: row wrow + 16 qs + r16
+  short8 qhi[QS][ND], qlo[QS][ND];
 #pragma unroll
-  for (int kd = 0; kd < ND; ++kd) {
+  for (int qs = 0; qs < QS; ++qs)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float x = 0.f;
-      if (q_valid) x = p.q[((size_t)(row0 + qrow) * H + h) * D + kd * 32 + 8 * g4 + e];
-      const bf16_t hi = f2bf(x);
-      qhi[kd][e] = (short)hi;
-      qlo[kd][e] = (short)f2bf(x - bf2f(hi));
+    for (int kd = 0; kd < ND; ++kd) {
+      float x[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+      const int qrow = wrow + 16 * qs + r16;
+      if (qrow < nrows) {
+        const float* qp = p.q + ((size_t)(row0 + qrow) * H + h) * D + kd * 32 + 8 * g4;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = qp[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const bf16_t hi = f2bf(x[e]);
+        qhi[qs][kd][e] = (short)hi;
+        qlo[qs][kd][e] = (short)f2bf(x[e] - bf2f(hi));
+      }
     }
-  }
-  const int w_min = pos0 + 16 * w, w_max = min(pos0 + 16 * w + 15, pos_last);  // this wave's positions
-  const int w_lo_min = lo_of(w_min), w_lo_max = lo_of(max(w_max, w_min)), lo_q = lo_of(i_q);  // and their first visible keys
-  const bool wave_live = 16 * w < nrows;
+  const int w_min = pos0 + wrow, w_max = min(w_min + 16 * QS - 1, pos_last);  // this wave's positions
+  const int w_lo_min = lo_of(w_min), w_lo_max = lo_of(max(w_max, w_min));     // and their first visible keys
+  const bool wave_live = wrow < nrows, wave_full = w_max - w_min == 16 * QS - 1;
   const float cap_k = p.cap > 0.f ? 2.0f * kLog2e / p.cap : 0.f;
 
-  float4v O[NV];
+  float4v O[QS][NV];
+  float m[QS], l[QS];  // l: this lane's share of the row's sum (its keys only; the four lanes of a row meet at the end)
 #pragma unroll
-  for (int n = 0; n < NV; ++n) O[n] = float4v{0.f, 0.f, 0.f, 0.f};
-  float m = -1e30f, l = 0.f;
-  const float* bias_h = p.bias ? p.bias + (size_t)h * p.window : nullptr;  // no table: no distance bias
+  for (int qs = 0; qs < QS; ++qs) {
+    m[qs] = -1e30f;
+    l[qs] = 0.f;
+#pragma unroll
+    for (int n = 0; n < NV; ++n) O[qs][n] = float4v{0.f, 0.f, 0.f, 0.f};
+  }
+  const float* bias_h = BIAS ? p.bias + (size_t)h * p.window : nullptr;
 
   const int pg0 = page_ix((j_lo / 32) * 32);  // first page of the workgroup's key range
   // a tile's words are fetched into registers one tile ahead (the loads fly while the previous tile is computed)
@@ -311,15 +332,16 @@ __global__ void __launch_bounds__(256) window_attn_mfma_kernel(const WAttnMfmaPa
                                                    4LL * (g * DV + 2 * dc));
       }
     }
-    if (tid < 96) {
-      const int dist = pos0 - kt * 32 - 31 + tid;  // (row - key + 31) = tid
-      breg = bias_h && dist >= 0 && dist < p.window ? bias_h[dist] * kLog2e : 0.f;  // the softmax runs in the log2 domain
+    if constexpr (BIAS) {
+      if (tid < NB) {
+        const int dist = pos0 - kt * 32 - 31 + tid;  // (row - key + 31) = tid
+        breg = dist >= 0 && dist < p.window ? bias_h[dist] * kLog2e : 0.f;  // the softmax runs in the log2 domain
+      }
     }
   };
   auto stash = [&](int buf) {
     bf16_t* K_s = K_s2[buf];
     bf16_t* Vt_s = Vt_s2[buf];
-    float* bias_s = bias_s2[buf];
 #pragma unroll
     for (int u = 0; u < KCH; ++u) {
       const int c = tid + 256 * u;
@@ -336,7 +358,9 @@ __global__ void __launch_bounds__(256) window_attn_mfma_kernel(const WAttnMfmaPa
         *reinterpret_cast<uint2v*>(&Vt_s[(2 * dc + 1) * kVPad + at]) = uint2v{vreg[u][2], vreg[u][3]};
       }
     }
-    if (tid < 96) bias_s[tid] = breg;
+    if constexpr (BIAS) {
+      if (tid < NB) bias_s2[buf][tid] = breg;
+    }
   };
 
   const int kt_lo = j_lo / 32, kt_hi = j_hi / 32;
@@ -355,121 +379,130 @@ __global__ void __launch_bounds__(256) window_attn_mfma_kernel(const WAttnMfmaPa
     if (kt < kt_hi) fetch(kt + 1);
     // the tile's keys [32 kt, 32 kt + 31] against this wave's rows: nothing visible -> nothing to compute
     if (wave_live && kt * 32 <= w_max && kt * 32 + 31 >= w_lo_min) {
-    float4v sacc[2];
+      // a K fragment read from LDS serves QS row blocks
+      float4v sacc[QS][2];
 #pragma unroll
-    for (int sub = 0; sub < 2; ++sub) {
-      sacc[sub] = float4v{0.f, 0.f, 0.f, 0.f};
+      for (int sub = 0; sub < 2; ++sub) {
 #pragma unroll
-      for (int kd = 0; kd < ND; ++kd) {
-        const short8 a = *reinterpret_cast<const short8*>(&K_s[(sub * 16 + r16) * KLD + kd * 32 + 8 * g4]);
-        sacc[sub] = mfma16(a, qhi[kd], sacc[sub]);
-        sacc[sub] = mfma16(a, qlo[kd], sacc[sub]);
+        for (int qs = 0; qs < QS; ++qs) sacc[qs][sub] = float4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kd = 0; kd < ND; ++kd) {
+          const short8 a = *reinterpret_cast<const short8*>(&K_s[(sub * 16 + r16) * KLD + kd * 32 + 8 * g4]);
+#pragma unroll
+          for (int qs = 0; qs < QS; ++qs) sacc[qs][sub] = mfma16(a, qhi[qs][kd], sacc[qs][sub]);
+#pragma unroll
+          for (int qs = 0; qs < QS; ++qs) sacc[qs][sub] = mfma16(a, qlo[qs][kd], sacc[qs][sub]);
+        }
       }
-    }
-    if (p.cap > 0.f) {
+      // every key of the tile visible to every row of the wave: no masks
+      const bool inner = kt * 32 + 31 <= w_min && kt * 32 >= w_lo_max && wave_full;
+      short8 ph[QS], pl[QS];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) sacc[e >> 2][e & 3] = softcap_f(sacc[e >> 2][e & 3], p.cap, cap_k);
-    }
-    // every key of the tile visible to every row of the wave: no masks
-    const bool inner = kt * 32 + 31 <= w_min && kt * 32 >= w_lo_max && w_max - w_min == 15;
-    float s[8];
-    float mx = -1e30f;
-    const float* brow = bias_s + (qrow + 31 - 4 * g4);
-    if (inner) {
+      for (int qs = 0; qs < QS; ++qs) {
+        const int qrow = wrow + 16 * qs + r16, i_q = pos0 + qrow;
+        float s[8];
+        float mx = -1e30f;
+        if (p.cap > 0.f) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        s[e] = fmaf(sacc[e >> 2][e & 3], kLog2e, -brow[-((e >> 2) * 16 + (e & 3))]);
-        mx = fmaxf(mx, s[e]);
+          for (int e = 0; e < 8; ++e) sacc[qs][e >> 2][e & 3] = softcap_f(sacc[qs][e >> 2][e & 3], p.cap, cap_k);
+        }
+        const float* brow = BIAS ? bias_s + (qrow + 31 - 4 * g4) : nullptr;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float x = sacc[qs][e >> 2][e & 3];
+          if constexpr (BIAS) s[e] = fmaf(x, kLog2e, -brow[-((e >> 2) * 16 + (e & 3))]);
+          else s[e] = x * kLog2e;
+        }
+        if (!inner) {
+          const int lo_q = lo_of(i_q);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const int j = kt * 32 + (e >> 2) * 16 + 4 * g4 + (e & 3);
+            if (!(qrow < nrows && j <= i_q && j >= lo_q)) s[e] = -1e30f;
+          }
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) mx = fmaxf(mx, s[e]);
+        mx = row_max4(mx);
+        if (__any(mx > m[qs] + kLazy)) {   // (wave-uniform; the running maxima settle after the first tiles)
+          const float m_new = fmaxf(m[qs], mx);
+          const float alpha = __builtin_amdgcn_exp2f(m[qs] - m_new);
+          m[qs] = m_new;
+          l[qs] *= alpha;
+          float ar[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, 4 * g4 + r, 64);
+#pragma unroll
+          for (int n = 0; n < NV; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) O[qs][n][r] *= ar[r];
+        }
+        float pe[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) pe[e] = __builtin_amdgcn_exp2f(s[e] - m[qs]);
+        if (!inner) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) pe[e] = s[e] > -1e29f ? pe[e] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e) l[qs] += pe[e];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const bf16_t hi = f2bf(pe[e]);
+          ph[qs][e] = (short)hi;
+          pl[qs][e] = (short)f2bf(pe[e] - bf2f(hi));
+        }
       }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int jl = (e >> 2) * 16 + 4 * g4 + (e & 3);
-        const int dist = i_q - (kt * 32 + jl);
-        const bool ok = q_valid && dist >= 0 && kt * 32 + jl >= lo_q;
-        s[e] = ok ? fmaf(sacc[e >> 2][e & 3], kLog2e, -brow[-((e >> 2) * 16 + (e & 3))]) : -1e30f;
-        mx = fmaxf(mx, s[e]);
-      }
-    }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m, mx);
-    const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-    float pe[8], psum = 0.f;
-    if (inner) {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pe[e] = __builtin_amdgcn_exp2f(s[e] - m_new);
-        psum += pe[e];
-      }
-    } else {
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        pe[e] = s[e] > -1e29f ? __builtin_amdgcn_exp2f(s[e] - m_new) : 0.f;
-        psum += pe[e];
-      }
-    }
-    psum += __shfl_xor(psum, 16, 64);
-    psum += __shfl_xor(psum, 32, 64);
-    l = l * alpha + psum;
-    m = m_new;
-    short8 ph, pl;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const bf16_t hi = f2bf(pe[e]);
-      ph[e] = (short)hi;
-      pl[e] = (short)f2bf(pe[e] - bf2f(hi));
-    }
-    float ar[4];
-#pragma unroll
-    for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, 4 * g4 + r, 64);
-    // (the running maxima settle after the first tiles: most tiles rescale nothing)
-    if (__any(alpha != 1.0f)) {
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
+        const short8 b = *reinterpret_cast<const short8*>(&Vt_s[(n * 16 + r16) * kVPad + 8 * g4]);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) O[n][r] *= ar[r];
+        for (int qs = 0; qs < QS; ++qs) O[qs][n] = mfma16(ph[qs], b, O[qs][n]);
+#pragma unroll
+        for (int qs = 0; qs < QS; ++qs) O[qs][n] = mfma16(pl[qs], b, O[qs][n]);
       }
-    }
-#pragma unroll
-    for (int n = 0; n < NV; ++n) {
-      const short8 b = *reinterpret_cast<const short8*>(&Vt_s[(n * 16 + r16) * kVPad + 8 * g4]);
-      O[n] = mfma16(ph, b, O[n]);
-      O[n] = mfma16(pl, b, O[n]);
-    }
     }  // (this wave's work on the tile)
     if (kt < kt_hi) stash(cur ^ 1);  // every wave left that image at the previous barrier
     __syncthreads();
   }
   if (!wave_live) return;
-  float a_fin = 1.0f;
-  if (p.sink) {  // the sink's share: one more term of the denominator, nothing added to O
-    const float sk = p.sink[h] * kLog2e, mf = fmaxf(m, sk);
-    a_fin = __builtin_amdgcn_exp2f(m - mf);
-    l = l * a_fin + __builtin_amdgcn_exp2f(sk - mf);
-  }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float lr = __shfl(l, 4 * g4 + r, 64);
-    const float inv = (lr > 0.f ? 1.0f / lr : 0.f) * __shfl(a_fin, 4 * g4 + r, 64);
-    const int row = 16 * w + 4 * g4 + r;
-    if (row < nrows) {
-      bf16_t* orow = p.out + (size_t)(row0 + row) * p.ldo + (size_t)h * DV;
+  for (int qs = 0; qs < QS; ++qs) {
+    float ls = row_sum4(l[qs]), a_fin = 1.0f;
+    if (p.sink) {  // the sink's share: one more term of the denominator, nothing added to O
+      const float sk = p.sink[h] * kLog2e, mf = fmaxf(m[qs], sk);
+      a_fin = __builtin_amdgcn_exp2f(m[qs] - mf);
+      ls = ls * a_fin + __builtin_amdgcn_exp2f(sk - mf);
+    }
 #pragma unroll
-      for (int n = 0; n < NV; ++n) orow[n * 16 + r16] = f2bf(O[n][r] * inv);
+    for (int r = 0; r < 4; ++r) {
+      const float lr = __shfl(ls, 4 * g4 + r, 64);
+      const float inv = (lr > 0.f ? 1.0f / lr : 0.f) * __shfl(a_fin, 4 * g4 + r, 64);
+      const int row = wrow + 16 * qs + 4 * g4 + r;
+      if (row < nrows) {
+        bf16_t* orow = p.out + (size_t)(row0 + row) * p.ldo + (size_t)h * DV;
+#pragma unroll
+        for (int n = 0; n < NV; ++n) orow[n * 16 + r16] = f2bf(O[qs][n][r] * inv);
+      }
     }
   }
 }
 
-template <int ND>
-int launch_mfma_nv(const WAttnMfmaParams& p, int nv, dim3 grid, size_t shm, hipStream_t s) {
+template <int ND, int QS, bool BIAS>
+int launch_mfma_nv(const WAttnMfmaParams& p, int nv, unsigned grid, size_t shm, hipStream_t s) {
   switch (nv) {
-    case 2: window_attn_mfma_kernel<ND, 2><<<grid, 256, shm, s>>>(p); break;
-    case 4: window_attn_mfma_kernel<ND, 4><<<grid, 256, shm, s>>>(p); break;
-    case 8: window_attn_mfma_kernel<ND, 8><<<grid, 256, shm, s>>>(p); break;
+    case 2: window_attn_mfma_kernel<ND, 2, QS, BIAS><<<grid, 256, shm, s>>>(p); break;
+    case 4: window_attn_mfma_kernel<ND, 4, QS, BIAS><<<grid, 256, shm, s>>>(p); break;
+    case 8: window_attn_mfma_kernel<ND, 8, QS, BIAS><<<grid, 256, shm, s>>>(p); break;
     default: return -1;
   }
   return (int)hipGetLastError();
+}
+
+template <int ND>
+int launch_mfma_qs(const WAttnMfmaParams& p, int qs, int nv, unsigned grid, size_t shm, hipStream_t s) {
+  if (qs == 2) return p.bias ? launch_mfma_nv<ND, 2, true>(p, nv, grid, shm, s) : launch_mfma_nv<ND, 2, false>(p, nv, grid, shm, s);
+  return p.bias ? launch_mfma_nv<ND, 1, true>(p, nv, grid, shm, s) : launch_mfma_nv<ND, 1, false>(p, nv, grid, shm, s);
 }
 
 // Whether the matrix-core kernel takes these sizes (bf16 cache only).
@@ -490,19 +523,25 @@ extern "C" int r32_window_attn_mfma(const float* q, const void* k_cache, const v
   p.bs_shift = -1;
   for (int b = 0; b < 20; ++b)
     if ((1 << b) == block_size) p.bs_shift = b;
-  p.cu_q = cu_q; p.k_lens = k_lens; p.tiles_per_item = (max_q + 63) / 64; p.block_tables = block_tables;
+  // two row blocks per wave (128 rows a workgroup) halve the LDS reads per product; one (64 rows) while that leaves
+  // compute units without a workgroup
+  const long long wide = (long long)n_items * ((max_q + 127) / 128) * H;
+  const int qs = wide >= kWideFrom ? 2 : 1;
+  p.cu_q = cu_q; p.k_lens = k_lens; p.tiles_per_item = (max_q + 64 * qs - 1) / (64 * qs); p.block_tables = block_tables;
   p.bt_width = bt_width; p.bias = bias; p.sink = sink; p.window = window; p.chunk = chunk; p.cap = cap; p.out = (bf16_t*)out; p.ldo = ldo; p.H = H; p.G = G;
-  const dim3 grid(n_items * p.tiles_per_item, H);
-  // a workgroup's keys span at most window + 63 positions (from a 32-aligned start: + 31) and never more than the table
-  long long span = (long long)window + 63 + 31;
+  const long long wgs = (long long)n_items * p.tiles_per_item * H;
+  if (wgs >= (1LL << 31)) return -3;
+  const unsigned grid = (unsigned)wgs;
+  // a workgroup's keys span at most window + its rows - 1 positions (from a 32-aligned start: + 31) and never more than the table
+  long long span = (long long)window + 64 * qs - 1 + 31;
   if (span > (long long)bt_width * block_size) span = (long long)bt_width * block_size;
   const size_t shm = (size_t)(span / block_size + 2) * sizeof(int);
   if (shm > 48 * 1024) return -2;
   switch (D / 32) {
-    case 1: return launch_mfma_nv<1>(p, Dv / 16, grid, shm, s);
-    case 2: return launch_mfma_nv<2>(p, Dv / 16, grid, shm, s);
-    case 4: return launch_mfma_nv<4>(p, Dv / 16, grid, shm, s);
-    case 6: return launch_mfma_nv<6>(p, Dv / 16, grid, shm, s);
+    case 1: return launch_mfma_qs<1>(p, qs, Dv / 16, grid, shm, s);
+    case 2: return launch_mfma_qs<2>(p, qs, Dv / 16, grid, shm, s);
+    case 4: return launch_mfma_qs<4>(p, qs, Dv / 16, grid, shm, s);
+    case 6: return launch_mfma_qs<6>(p, qs, Dv / 16, grid, shm, s);
   }
   return -1;
 }

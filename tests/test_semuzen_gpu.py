@@ -232,6 +232,64 @@ def test_capped_scores(gpu, dtype, tol, H, G, D, Dv, cap):
     assert (out.cpu().double().view(n - a, H, Dv) - ref[a:]).abs().max() < tol * 4
 
 
+@pytest.mark.parametrize("D,Dv", [(32, 32), (128, 128), (192, 128)])
+@pytest.mark.parametrize("window,chunk,cap,sink,biased", [(NO_WINDOW, 0, 0.0, False, False), (70, 0, 0.0, True, True),
+                                                          (NO_WINDOW, 50, 4.0, False, False), (33, 0, 0.0, False, False)])
+def test_portions_of_many_rows(gpu, D, Dv, window, chunk, cap, sink, biased):
+    """Enough rows and heads for two row blocks per wave: portions of whole, nearly whole and barely begun 128-row tiles,
+    behind cached keys and not, scores that keep rising along the keys.  Bound: the bf16 result's rounding (2^-9, doubled)
+    plus the 2^-16 of the weights' two bf16 halves, over values of up to 4."""
+    from llm_weighted_consensus_amd.models.cache import PagedLayerCache
+    from llm_weighted_consensus_amd.ops import res32
+
+    H, G, bs = 96, 6, 16
+    lens, k_lens = [257, 1, 128, 130], [257, 40, 333, 130]   # rows of the portion, keys they end at
+    g = torch.Generator().manual_seed(D + window % 1000)
+    nb = [-(-n // bs) for n in k_lens]
+    cache = PagedLayerCache([(G * D, G * Dv)], sum(nb), bs, gpu, BF16)
+    perm = torch.randperm(sum(nb), generator=g)
+    width = 2 * -(-max(k_lens) // (2 * bs))
+    tables = torch.zeros(len(lens), width, dtype=torch.int32)
+    r1, r2 = torch.rand(H, generator=g), torch.rand(H, generator=g)
+    z = torch.randn(H, generator=g).to(gpu)
+    Ks, Vs, qs, pos, at = [], [], [], [], 0
+    for i, n in enumerate(k_lens):
+        blk = perm[at:at + nb[i]]
+        at += nb[i]
+        tables[i, :nb[i]] = blk.to(torch.int32)
+        sl = (blk[:, None] * bs + torch.arange(bs)).reshape(-1)[:n]
+        K = (torch.randn(n, G, D, generator=g) * (0.2 + 3.0 * torch.arange(n)[:, None, None] / n)).to(BF16)
+        V = torch.randn(n, G, Dv, generator=g).clamp(-4, 4).to(BF16)
+        cache.set_rows(0, sl.to(gpu), K.view(n, -1).to(gpu), V.view(n, -1).to(gpu))
+        Ks.append(K)
+        Vs.append(V)
+        qs.append(torch.randn(lens[i], H, D, generator=g) * 2 * D ** -0.5)
+        pos.append(torch.arange(n - lens[i], n))
+    q = torch.cat(qs).to(gpu)
+    out = torch.empty(sum(lens), H * Dv, dtype=BF16, device=gpu)
+    zero = torch.zeros(H, device=gpu)
+    cu = torch.tensor(np.concatenate([[0], np.cumsum(lens)]), dtype=torch.int32, device=gpu)
+    res32.window_attn(q.view(len(q), -1), cache.k[0], cache.v[0], torch.cat(pos).to(torch.int32).to(gpu), tables.to(gpu), zero, zero, window, out,
+                      H, G, cu_q=cu, k_lens=torch.tensor(k_lens, dtype=torch.int32, device=gpu), max_q=max(lens), cores=True, chunk=chunk, cap=cap,
+                      bias=res32.distance_bias(r1.to(gpu), r2.to(gpu), window) if biased else None, sink=z if sink else None)
+    a = 0
+    for i, n in enumerate(k_lens):
+        K, V = (t[i].to(gpu).double().repeat_interleave(H // G, 1) for t in (Ks, Vs))
+        s = torch.einsum("ihd,jhd->hij", qs[i].to(gpu).double(), K)
+        if cap:
+            s = cap * torch.tanh(s / cap)
+        p, j = pos[i].to(gpu)[:, None], torch.arange(n, device=gpu)[None]
+        if biased:
+            s = s - r1.to(gpu).double()[:, None, None] * torch.log1p(r2.to(gpu).double()[:, None, None] * (p - j).clamp(min=0))
+        ok = (j <= p) & (j > p - window) & ((j >= p - p % chunk) if chunk else True)
+        s = s.masked_fill(~ok, -float("inf"))
+        if sink:
+            s = torch.cat([s, z.double()[:, None, None].expand(H, lens[i], 1)], -1)
+        ref = torch.einsum("hij,jhv->ihv", s.softmax(-1)[..., :n], V).reshape(lens[i], -1)
+        torch.testing.assert_close(out[a:a + lens[i]].double(), ref, rtol=2 ** -8, atol=4 * 2 ** -15)
+        a += lens[i]
+
+
 # ------------------------------------------------------------------ the model through the engine
 def _configs():
     return {
