@@ -472,14 +472,13 @@ void gemm4w(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::
            "gemm4w");
 }
 
-// skinny GEMM (decode-sized M <= 64): C = A . W^T (epi 0), R + A . W^T (epi 1, R may be C) or the SwiGLU of
-// a 32-row gate/up interleaved W (epi 2, C [M, N / 2])
+// skinny GEMM (M <= 256): C = A . W^T (epi 0), R + A . W^T (epi 1, R may be C), the SwiGLU of a 32-row gate/up
+// interleaved W (epi 2, C [M, N / 2]), A . W^T + bias (epi 3, R = bias [N]) or its GELU (epi 4)
 void skinny_gemm(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::optional<at::Tensor>& R,
                  int64_t epi) {
-  TORCH_CHECK(epi >= 0 && epi <= 2, "skinny_gemm: epi 0 (plain), 1 (residual) or 2 (SwiGLU)");
   const void* r = gemm_operands(A, W, C, R, epi);
   const int M = (int)A.size(0), K = (int)A.size(1), N = (int)W.size(0);
-  TORCH_CHECK(M <= 64 && K % 2048 == 0 && N % 16 == 0, "skinny_gemm: needs M <= 64, K % 2048 == 0, N % 16 == 0");
+  TORCH_CHECK(M <= 256 && N % 16 == 0, "skinny_gemm: needs M <= 256, N % 16 == 0");
   CHECK_RC(lwc_skinny_gemm(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, M, N, K, (int)A.stride(0), (int)C.stride(0),
                            (int)epi, cur_stream()),
            "skinny_gemm");

@@ -83,6 +83,16 @@ LWC_DEVICE float block_max(float v, float* scratch) {
   return wave_max(r);
 }
 
+// erf by Abramowitz & Stegun 7.1.26 (|error| < 1.5e-7, far below bf16's resolution): one exp, one rcp and a
+// 5-term polynomial — the libm erff's branches made the fused epilogue cost more than a separate pass.
+LWC_DEVICE float erf_as(float x) {
+  const float a = fabsf(x);
+  const float t = __builtin_amdgcn_rcpf(1.f + 0.3275911f * a);  // v_rcp_f32 (1 ulp): __frcp_rn is a full division sequence
+  const float y = t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
+  return copysignf(1.f - y * __expf(-a * a), x);
+}
+LWC_DEVICE float gelu_erf(float x) { return 0.5f * x * (1.f + erf_as(x * 0.70710678118654752f)); }
+
 // Reductions over the 4 lanes {l, l^16, l^32, l^48} holding one query row's tokens: two VALU
 // half-swaps (v_permlane32_swap / v_permlane16_swap, gfx950) instead of LDS ds_bpermute round trips.
 LWC_DEVICE float row_max4(float v) {

@@ -86,16 +86,6 @@ LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
 // v_div_fixup around an rcp: ~9 VALU per element in an epilogue of 256 per lane); the result is rounded
 // to bf16 (or e4m3) anyway.  x -> -inf: rcp(inf) = 0, x * 0 = -0 as the division gives
 LWC_DEVICE float silu(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
-// erf by Abramowitz & Stegun 7.1.26 (|error| < 1.5e-7, far below bf16's resolution): one exp, one rcp and a
-// 5-term polynomial — the libm erff's branches made the fused epilogue cost more than a separate pass.
-LWC_DEVICE float erf_as(float x) {
-  const float a = fabsf(x);
-  const float t = __builtin_amdgcn_rcpf(1.f + 0.3275911f * a);  // v_rcp_f32 (1 ulp): __frcp_rn is a full division sequence
-  const float y = t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
-  return copysignf(1.f - y * __expf(-a * a), x);
-}
-LWC_DEVICE float gelu_erf(float x) { return 0.5f * x * (1.f + erf_as(x * 0.70710678118654752f)); }
-
 // K-iteration range [a, e) of stream-K workgroup j (of wpx) on XCD x.
 LWC_DEVICE void sk_range(const Params& p, int x, int j, int& a, int& e) {
   const int t0 = p.sk_tiles * x / 8, t1 = p.sk_tiles * (x + 1) / 8;

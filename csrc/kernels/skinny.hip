@@ -1,5 +1,5 @@
-// K6 skinny projection GEMM for decode-sized row counts (M <= 64): C[M, N] (+ R) = A[M, K] . W[N, K]^T, bf16
-// in / out, fp32 accumulation.
+// K6 skinny projection GEMM for small row counts: C[M, N] = A[M, K] . W[N, K]^T (+ residual, + bias, + bias and
+// exact-erf GELU, or SwiGLU), bf16 in / out, fp32 accumulation.
 //
 // At a serving decode step (a few to 64 sequences) every projection is a weight stream: o (N = K = 4096)
 // reads 33.5 MB of W for 0.5 MFLOP per weight row.  The 256 x 256-tile cores (gemm4w / gemm8p) leave all
@@ -15,11 +15,19 @@
 //     accumulator of lane (r16, q) holds output row 16 mt + r16, columns n0 + 4q .. 4q + 3 (4 consecutive
 //     output columns: one 8-byte store, one 8-byte residual load);
 //   * the 8 waves' partial tiles meet in LDS (8 x MT x 1 KiB) and MT waves finish: sum in wave order,
-//     + residual (or SwiGLU of the gate and up tiles, EPI 2), bf16, store.
-// Rows past M read zeros (buffer offsets past the activation resource's end) and are not stored.
+//     + residual / bias (GELU) (or SwiGLU of the gate and up tiles, EPI 2), bf16, store.
+// Rows past M read zeros (buffer offsets past the activation resource's end) and are not stored.  Rows past 64 go in
+// chunks of 64 over grid y (encoders: a few texts, whose weights stay in the caches).
 //
-// Requires K % 2048 == 0 (8 waves x an even number of 4-step batches of 32), N % 16 == 0, M <= 64, lda / ldc % 4 == 0; the
-// planner (ops/gemm_plan.py, backend "gv") times it against hipBLASLt per decode bucket.
+// K is cut into steps of 32, ceil(K / 256) of them per wave; the FULL build (K % 2048 == 0, every wave the same even
+// number of whole batches) has no masks, the other sends the steps past a wave's share to offsets past the resources'
+// ends, which load zeros without a memory request.  A bge-small text of 12 tokens (K 384 / 1536, N 384 .. 1536): the
+// 256-row tiles ran 8 workgroups, 14.3 us plain and 22.1 us with GELU; here 3.3 and
+// 3.4 us (hipBLASLt 3.8, with 2-3 times the host time per call); from 64 rows on the library catches up (activations
+// are read once per 16 columns), which the planners' timings see.
+//
+// Requires K % 32 == 0, N % 16 == 0, lda / ldc % 4 == 0; the planners (ops/gemm_plan.py, backend "gv") time it against
+// hipBLASLt per decode bucket and per encoder token bucket.
 #include "common.h"
 
 namespace lwc {
@@ -38,7 +46,7 @@ struct Params {
   const bf16_t* A;
   const bf16_t* W;
   bf16_t* C;
-  const bf16_t* R;  // residual [M, ldc] (EPI 1) — may alias C
+  const bf16_t* R;  // residual [M, ldc] (EPI 1) — may alias C; bias [N] (EPI 3, 4)
   int M, N, K, lda, ldc;
 };
 
@@ -47,9 +55,9 @@ struct Params {
 // 16 (x % 2) + [0, 16) and the up rows 32 further (NW = 2); the plain / residual forms take 16 (NW = 1) or 32
 // adjacent output columns (NW = 2: half the workgroups, so half the activation re-reads from L2 — past 16
 // rows those loads, M / 16 times the weight bytes, are what limits the NW = 1 form)
-template <int MT, int EPI, int NW>
+template <int MT, int EPI, int NW, bool FULL>
 __global__ void __launch_bounds__(512) skinny_kernel(Params p) {
-  constexpr int U = 4;  // k-steps per load batch: nb = K / 1024 batches, even for K % 2048 == 0
+  constexpr int U = 4;  // k-steps per load batch (FULL: nb = K / 1024 batches, even for K % 2048 == 0)
   static_assert(EPI != 2 || NW == 2, "SwiGLU pairs a gate and an up tile");
   constexpr int TS = EPI == 2 ? 32 : 16;  // W rows between the NW tiles
   __shared__ float4v red[KS][NW][MT][64];
@@ -58,16 +66,22 @@ __global__ void __launch_bounds__(512) skinny_kernel(Params p) {
   const int r16 = lane & 15, g = lane >> 4;
   const int n0 = blockIdx.x * (EPI == 2 ? 16 : 16 * NW);  // first output column
   const int wrow = EPI == 2 ? 64 * (blockIdx.x >> 1) + 16 * (blockIdx.x & 1) : n0;  // first W row
-  const int Kw = p.K / KS;          // this wave's K range [w Kw, (w + 1) Kw)
-  const int nb = Kw / (32 * U);     // load batches
+  const int m0 = blockIdx.y * 64;   // this chunk's first row
+  const int M = min(p.M - m0, 64);
+  const int steps = p.K / 32, per = (steps + KS - 1) / KS;   // this wave's k-steps: [w per, w per + cnt)
+  const int cnt = max(0, min(per, steps - w * per));
+  const int nb = FULL ? per / U : ((per + U - 1) / U + 1) & ~1;   // load batches, an even number
+  const int k0 = w * per * 32;
   const __amdgpu_buffer_rsrc_t rW = uniform_rsrc(p.W + (size_t)wrow * p.K, (16 + TS * (NW - 1)) * p.K * 2);
-  const __amdgpu_buffer_rsrc_t rA = uniform_rsrc(p.A, p.M * p.lda * 2);
+  const __amdgpu_buffer_rsrc_t rA = uniform_rsrc(p.A + (size_t)m0 * p.lda, M * p.lda * 2);
+  constexpr uint32_t kPast = 0x7ffffff0u;  // past every resource: loads zeros
   uint32_t voW[NW];
 #pragma unroll
-  for (int t = 0; t < NW; ++t) voW[t] = (uint32_t)(((r16 + TS * t) * p.K + w * Kw + 8 * g) * 2);
+  for (int t = 0; t < NW; ++t) voW[t] = (uint32_t)(((r16 + TS * t) * p.K + k0 + 8 * g) * 2);
+  // (rows past M of the last row's stride would reach past the rows' own end when lda > K: sent past the resource too)
   uint32_t voA[MT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt) voA[mt] = (uint32_t)(((mt * 16 + r16) * p.lda + w * Kw + 8 * g) * 2);
+  for (int mt = 0; mt < MT; ++mt) voA[mt] = mt * 16 + r16 < M ? (uint32_t)(((mt * 16 + r16) * p.lda + k0 + 8 * g) * 2) : kPast;
 
   float4v acc[NW][MT];
 #pragma unroll
@@ -80,13 +94,14 @@ __global__ void __launch_bounds__(512) skinny_kernel(Params p) {
   auto load = [&](int b, uint4v(&wb)[U][NW], uint4v(&ab)[U][MT]) {
 #pragma unroll
     for (int s = 0; s < U; ++s) {
-      const int so = (b * U + s) * 64;  // 32 k of bf16 per step (wave-uniform: soffset)
+      const bool in = FULL || b * U + s < cnt;    // wave-uniform
+      const int so = in ? (b * U + s) * 64 : 0;   // 32 k of bf16 per step (soffset)
 #pragma unroll
       for (int t = 0; t < NW; ++t)
-        wb[s][t] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rW, voW[t], so, 0));
+        wb[s][t] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rW, in ? voW[t] : kPast, so, 0));
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt)
-        ab[s][mt] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rA, voA[mt], so, 0));
+        ab[s][mt] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rA, in ? voA[mt] : kPast, so, 0));
     }
   };
   auto compute = [&](const uint4v(&wb)[U][NW], const uint4v(&ab)[U][MT]) {
@@ -134,11 +149,19 @@ __global__ void __launch_bounds__(512) skinny_kernel(Params p) {
       for (int e = 0; e < 4; ++e) sum[0][e] = sum[0][e] * __builtin_amdgcn_rcpf(1.f + __expf(-sum[0][e])) * sum[1][e];
     }
     const int m = w * 16 + r16;
-    if (m < p.M) {
+    if (m < M) {
 #pragma unroll
       for (int t = 0; t < NO; ++t) {
-        const size_t off = (size_t)m * p.ldc + n0 + 16 * t + 4 * g;
+        const size_t off = (size_t)(m0 + m) * p.ldc + n0 + 16 * t + 4 * g;
         float v[4] = {sum[t][0], sum[t][1], sum[t][2], sum[t][3]};
+        if constexpr (EPI == 3 || EPI == 4) {
+          const bf16_t* b = p.R + n0 + 16 * t + 4 * g;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            v[e] += bf2f(b[e]);
+            if constexpr (EPI == 4) v[e] = gelu_erf(v[e]);
+          }
+        }
         if constexpr (EPI == 1) {
           const uint2 rr = *reinterpret_cast<const uint2*>(p.R + off);
           v[0] += __uint_as_float(rr.x << 16);
@@ -155,18 +178,23 @@ __global__ void __launch_bounds__(512) skinny_kernel(Params p) {
   }
 }
 
-template <int EPI, int NW>
-int launch_nw(const Params& p, hipStream_t s) {
-  const int mt = (p.M + 15) / 16;
-  const dim3 grid(EPI == 2 ? p.N / 32 : p.N / (16 * NW));  // SwiGLU: N / 2 output columns, 16 per workgroup
+template <int EPI, int NW, bool FULL>
+int launch_full(const Params& p, hipStream_t s) {
+  const int mt = (min(p.M, 64) + 15) / 16;
+  const dim3 grid(EPI == 2 ? p.N / 32 : p.N / (16 * NW), (p.M + 63) / 64);  // SwiGLU: N / 2 output columns, 16 per workgroup
   switch (mt) {
-    case 1: skinny_kernel<1, EPI, NW><<<grid, 512, 0, s>>>(p); break;
-    case 2: skinny_kernel<2, EPI, NW><<<grid, 512, 0, s>>>(p); break;
+    case 1: skinny_kernel<1, EPI, NW, FULL><<<grid, 512, 0, s>>>(p); break;
+    case 2: skinny_kernel<2, EPI, NW, FULL><<<grid, 512, 0, s>>>(p); break;
     case 3:
-    case 4: skinny_kernel<4, EPI, NW><<<grid, 512, 0, s>>>(p); break;
+    case 4: skinny_kernel<4, EPI, NW, FULL><<<grid, 512, 0, s>>>(p); break;
     default: return -1;
   }
   return (int)hipGetLastError();
+}
+
+template <int EPI, int NW>
+int launch_nw(const Params& p, hipStream_t s) {
+  return p.K % 2048 == 0 ? launch_full<EPI, NW, true>(p, s) : launch_full<EPI, NW, false>(p, s);
 }
 
 // plain / residual: 32 output columns per workgroup past 16 rows when that still leaves >= 192 workgroups
@@ -185,19 +213,26 @@ int launch(const Params& p, hipStream_t s) {
 }  // namespace skinny
 }  // namespace lwc
 
-// C = A . W^T (epi 0), R + A . W^T (epi 1; R may be C) or silu(A . Wg^T) * (A . Wu^T) over a 32-row gate/up
-// interleaved W [N, K] (epi 2, C [M, N / 2]) for M <= 64 rows.  -1: shape not taken.
+// C = A . W^T (epi 0), R + A . W^T (epi 1; R may be C), silu(A . Wg^T) * (A . Wu^T) over a 32-row gate/up interleaved
+// W [N, K] (epi 2, C [M, N / 2]), A . W^T + bias (epi 3; R = bias [N]) or gelu(A . W^T + bias) (epi 4) for M <= 256 rows.
+// -1: shape not taken.
 extern "C" int lwc_skinny_gemm(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda,
                                int ldc, int epi, hipStream_t s) {
   using namespace lwc::skinny;
   const int NC = epi == 2 ? N / 2 : N;
-  if (M < 0 || M > 64 || K % 2048 != 0 || N % (epi == 2 ? 64 : 16) != 0 || lda % 4 != 0 || ldc % 4 != 0 ||
+  if (M < 0 || M > 256 || K < 32 || K % 32 != 0 || N % (epi == 2 ? 64 : 16) != 0 || lda % 4 != 0 || ldc % 4 != 0 ||
       lda < K || ldc < NC)
     return -1;
-  if (epi < 0 || epi > 2) return -1;
-  if (epi == 1 && R == nullptr) return -1;
-  if ((long long)48 * K * 2 >= (1LL << 31) || (long long)M * lda * 2 >= (1LL << 31)) return -1;
+  if (epi < 0 || epi > 4) return -1;
+  if ((epi == 1 || epi >= 3) && R == nullptr) return -1;
+  if ((long long)48 * K * 2 >= 0x7ffffff0LL || (long long)64 * lda * 2 >= 0x7ffffff0LL) return -1;
   if (M == 0 || N == 0) return 0;
   Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc};
-  return epi == 1 ? launch<1>(p, s) : (epi == 2 ? launch<2>(p, s) : launch<0>(p, s));
+  switch (epi) {
+    case 0: return launch<0>(p, s);
+    case 1: return launch<1>(p, s);
+    case 2: return launch<2>(p, s);
+    case 3: return launch<3>(p, s);
+  }
+  return launch<4>(p, s);
 }

@@ -10,8 +10,8 @@ Backends computing ``A . W^T`` for the dense projections:
 * ``g4p``    — gemm4w 256 x 256 with the VAR 64 schedule: each persistent workgroup DMAs its next tile's
   first two K tiles inside its last two main-loop iterations and runs the wave-local epilogue on the
   transposed accumulator layout (``profiles/gemm4w_stamps_r5.md``).
-* ``gv``     — the skinny weight-stream GEMM for decode-sized row counts (M <= 64; plain, residual and
-  SwiGLU epilogues; ``csrc/kernels/skinny.hip``): the serving path's small decode steps.
+* ``gv``     — the skinny weight-stream GEMM for few rows (M <= 256; plain, residual, SwiGLU and bias (+ GELU)
+  epilogues; ``csrc/kernels/skinny.hip``): the serving path's small decode steps, the encoders' few short texts.
 * ``g4s``    — gemm4w VAR 64 with split-K (``ops.split_plan``): shapes whose tiles leave CUs idle (the
   serving path's mid-size row counts: o / down at M = 2048 are 128 tiles for 256 CUs) run every tile as 2-4
   K-range units, a ragged last round (lm_head) splits only that round's tiles.
@@ -151,7 +151,7 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = 
     N = w.shape[0]
     epi = "bias_gelu" if gelu else "bias"
     key = (_m_bucket(M), N, K, epi)
-    c = MODE if MODE in ("blas", "g8", "g4", "g4p") else _CHOICE.get(key)
+    c = MODE if MODE in ("blas", "g8", "g4", "g4p", "gv") else _CHOICE.get(key)
     # gemm8p addresses A through one 32-bit buffer range (operands of 2 GiB or more take the other backends);
     # gemm4w runs such an A as row blocks
     ok = _g8_ok(N, K, epi) and x.stride(1) == 1 and x.is_cuda
@@ -162,6 +162,8 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = 
         runs.update({"g4": lambda: gemm4w(x, w, bias=b, gelu=gelu), "g4p": lambda: gemm4w(x, w, bias=b, gelu=gelu, var=64)})
     if small_a:
         runs["g8"] = lambda: gemm8p(x, w, bias=b, gelu=gelu, ws=ws)
+    if ok and _own_ok("gv", x, N, K, epi):
+        runs["gv"] = lambda: skinny_gemm(x, w, bias=b, gelu=gelu)
     if c is None:
         if not ok or torch.cuda.is_current_stream_capturing():
             c = "blas"
@@ -183,7 +185,7 @@ def linear_residual_(x: torch.Tensor, w: torch.Tensor, acc: torch.Tensor, ws=Non
     M, K = x.shape
     N = w.shape[0]
     key = (_m_bucket(M), N, K, "enc_residual")
-    c = MODE if MODE in ("blas", "g8", "g4", "g4p") else _CHOICE.get(key)
+    c = MODE if MODE in ("blas", "g8", "g4", "g4p", "gv") else _CHOICE.get(key)
     ok = _g8_ok(N, K, "residual") and x.stride(1) == 1 and x.is_cuda and acc.is_contiguous()
     small_a = M * x.stride(0) * 2 < (1 << 31)
 
@@ -193,6 +195,8 @@ def linear_residual_(x: torch.Tensor, w: torch.Tensor, acc: torch.Tensor, ws=Non
             r.update({"g4": lambda: gemm4w(x, w, residual=a, out=a), "g4p": lambda: gemm4w(x, w, residual=a, out=a, var=64)})
         if small_a:
             r["g8"] = lambda: gemm8p(x, w, residual=a, out=a, ws=ws)
+        if ok and _own_ok("gv", x, N, K, "residual"):
+            r["gv"] = lambda: skinny_gemm(x, w, residual=a, out=a)
         return r
 
     if c is None:

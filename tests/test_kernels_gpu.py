@@ -1464,6 +1464,39 @@ def test_knn_topk(gpu, n, d, k):
         assert r.index(best) < r.index(n - 3)  # ties: lower row first
 
 
+@pytest.mark.parametrize("M", [1, 12, 64, 65, 130, 256])
+@pytest.mark.parametrize("N,K", [(1152, 384), (384, 1536), (48, 64), (80, 448), (3072, 1024), (208, 7168)])
+@pytest.mark.parametrize("epi", ["plain", "residual", "bias", "gelu"])
+def test_skinny_gemm_any_k(gpu, M, N, K, epi):
+    """K that gives the waves unequal shares, partial last batches or nothing at all; rows over several chunks of 64; A and
+    C as columns of wider matrices; vs fp64 of the same operands.  Bound: one bf16 rounding (2^-9, doubled), fp32 sums of
+    K terms of about 1 / sqrt(K), for GELU its erf polynomial's 1.5e-7."""
+    from llm_weighted_consensus_amd import ops
+
+    torch.manual_seed(M + N + K)
+    A = torch.randn(M, K + 64, device=gpu).to(torch.bfloat16)
+    A[:, K:] = float("nan")   # columns past K are never read
+    A = A[:, :K]
+    W = (torch.randn(N, K, device=gpu) * K ** -0.5).to(torch.bfloat16)
+    R = torch.randn(M, N, device=gpu).to(torch.bfloat16)
+    b = torch.randn(N, device=gpu).to(torch.bfloat16)
+    ref = A.double() @ W.double().t()
+    if epi == "residual":
+        ref += R.double()
+        out = ops.skinny_gemm(A, W, residual=R, out=R)
+        assert out is R
+    elif epi == "plain":
+        wide = torch.full((M + 1, N + 8), float("nan"), dtype=torch.bfloat16, device=gpu)
+        out = ops.skinny_gemm(A, W, out=wide[:M, :N])
+        assert torch.isnan(wide[M:]).all() and torch.isnan(wide[:, N:]).all()
+    else:
+        ref += b.double()
+        if epi == "gelu":
+            ref = torch.nn.functional.gelu(ref)
+        out = ops.skinny_gemm(A, W, bias=b, gelu=epi == "gelu")
+    torch.testing.assert_close(out.double(), ref, rtol=2 ** -8, atol=2e-5)
+
+
 @pytest.mark.parametrize("M", [1, 7, 16, 33, 64])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (6144, 4096), (4096, 14336), (1040, 2048)])
 @pytest.mark.parametrize("res", [False, True])
