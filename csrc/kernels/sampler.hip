@@ -1,6 +1,12 @@
 // K8a+K8b+K8c+K8d fused: logits processing, raw log-softmax + top-k logprobs, and top-k / top-p /
 // min-p / top-a filtered multinomial sampling (or greedy argmax) in ONE pass over each logits row.
 //
+// Bound by the one row a compute unit can hold (64 of 128 registers per lane), so that the row's load, 11 us at the CU's
+// share of the memory rate, and its passes take turns; every pass and every barrier counts.  4096 rows, one MI355X, us,
+// before -> after the passes lost their spilled registers (a row written to and read from scratch once more) and the
+// reductions their shuffles: vocabulary 128256 greedy 472 -> 208, temperature 0.8 345 -> 255, with top-p 0.95 452 -> 347,
+// with 20 logprobs 781 -> 592; vocabulary 32000 72 -> 43, 147 -> 63, 205 -> 97, 390 -> 240.
+//
 // One 1024-thread workgroup per row.  The row (bf16, V <= 8*1024*SLOTS) is loaded ONCE from HBM into
 // registers as packed bf16 (16 B per load, SLOTS loads per thread) and every later phase — raw max and
 // log-sum-exp, the top-K selection for `top_logprobs`, penalties/bias/grammar mask, the filter
@@ -79,6 +85,8 @@ LWC_DEVICE float key2f(uint32_t k) {
   return __uint_as_float(b << 16);
 }
 
+// (Passes under a condition have it in front of the condition: inside, the two paths' rows are two values and meet in
+// copies of the whole row, spilled.)
 // Keep the packed row opaque at the top of every pass: otherwise LICM hoists the 8*SLOTS unpacked
 // floats (or their keys) out of the binary-search loops and the kernel spills (1024 threads leave
 // 128 VGPRs per lane; the packed row alone is 4*SLOTS of them).
@@ -140,27 +148,96 @@ LWC_DEVICE float dot_read(float acc) {
 }
 LWC_DEVICE uint32_t thr1x2(uint32_t key) { return ((key - 1u) & 0xffffu) * 0x10001u; }  // key >= 1
 
-LWC_DEVICE int block_sum_i(int v, int* scratch) {
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  __syncthreads();
-  if (lane == 0) scratch[wid] = v;
-  __syncthreads();
-  int r = lane < (kSampT / 64) ? scratch[lane] : 0;
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) r += __shfl_xor(r, o, 64);
-  return r;
+// ---- reductions by lane swaps and DPP (a shuffle is a trip through LDS, six of them per reduction) ----
+#define LWC_DPP(x, ctrl) __builtin_amdgcn_mov_dpp((x), (ctrl), 0xF, 0xF, false)
+LWC_DEVICE float row16_sum(float x) {
+  x += __int_as_float(LWC_DPP(__float_as_int(x), 0xB1));
+  x += __int_as_float(LWC_DPP(__float_as_int(x), 0x4E));
+  x += __int_as_float(LWC_DPP(__float_as_int(x), 0x141));
+  return x + __int_as_float(LWC_DPP(__float_as_int(x), 0x140));
+}
+LWC_DEVICE int row16_sum_i(int x) {
+  x += LWC_DPP(x, 0xB1);
+  x += LWC_DPP(x, 0x4E);
+  x += LWC_DPP(x, 0x141);
+  return x + LWC_DPP(x, 0x140);
+}
+LWC_DEVICE int row_sum4_i(int v) {
+  auto r = __builtin_amdgcn_permlane32_swap((uint32_t)v, (uint32_t)v, false, false);
+  v = (int)(r[0] + r[1]);
+  auto q = __builtin_amdgcn_permlane16_swap((uint32_t)v, (uint32_t)v, false, false);
+  return (int)(q[0] + q[1]);
+}
+// inclusive sum over the wave's lanes: within rows of 16, then row 0 into 1 and 2 into 3, then the lower half into the upper
+LWC_DEVICE float wave_scan(float x) {
+#define LWC_SCAN(ctrl, rows) \
+  x += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), ctrl, rows, 0xF, false))
+  LWC_SCAN(0x111, 0xF);
+  LWC_SCAN(0x112, 0xF);
+  LWC_SCAN(0x114, 0xF);
+  LWC_SCAN(0x118, 0xF);
+  LWC_SCAN(0x142, 0xA);
+  LWC_SCAN(0x143, 0xC);
+#undef LWC_SCAN
+  return x;
 }
 
-template <int SLOTS>
+// Block-wide reductions over two alternating sets of partials: one barrier each (a set is written again only behind the
+// next reduction's barrier, which every reader of it has passed)
+struct Red {
+  float* f;  // [2][32]
+  int ph;
+  LWC_DEVICE float* set() { return f + 32 * (ph++ & 1); }
+  LWC_DEVICE float sum(float v) {
+    float* sc = set();
+    v = row_sum4(row16_sum(v));
+    if ((threadIdx.x & 63) == 0) sc[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return row16_sum(sc[threadIdx.x & 15]);
+  }
+  LWC_DEVICE float max(float v) {
+    float* sc = set();
+    v = row_max4(row16_max(v));
+    if ((threadIdx.x & 63) == 0) sc[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return row16_max(sc[threadIdx.x & 15]);
+  }
+  LWC_DEVICE int sum_i(int v) {
+    int* sc = reinterpret_cast<int*>(set());
+    v = row_sum4_i(row16_sum_i(v));
+    if ((threadIdx.x & 63) == 0) sc[threadIdx.x >> 6] = v;
+    __syncthreads();
+    return row16_sum_i(sc[threadIdx.x & 15]);
+  }
+};
+static_assert(kSampT == 1024, "the reductions meet over 16 waves");
+
+// Lowest index among the thread's elements for which TEST(j, e) holds, 0x7fffffff if none.  Slot and element are kept
+// apart: both are inline constants, while an index per element would be 8 * SLOTS literals, each in a register of its own
+// ahead of the loop (100 spilled registers in the SLOTS = 16 build).
+#define LOWEST_INDEX(TEST, OUT)                                     \
+  do {                                                              \
+    int _bj = -1, _be = 0;                                          \
+    _Pragma("unroll") for (int j = SLOTS - 1; j >= 0; --j) {        \
+      int _e = 8;                                                   \
+      _Pragma("unroll") for (int e = 7; e >= 0; --e) _e = (TEST) ? e : _e; \
+      _bj = _e < 8 ? j : _bj;                                       \
+      _be = _e < 8 ? _e : _be;                                      \
+      __builtin_amdgcn_sched_barrier(0);                            \
+    }                                                               \
+    OUT = _bj >= 0 ? (_bj * kSampT + t) * 8 + _be : 0x7fffffff;     \
+  } while (0)
+
+// PROC: a bias, a mask or penalties may apply to the rows; TOPK: num_logprobs > 0.  Builds of their own, so that a step
+// that asks for neither carries neither's registers.
+template <int SLOTS, bool PROC, bool TOPK>
 __global__ void __launch_bounds__(kSampT) sample_kernel(SampleParams p) {
-  __shared__ float sred[32];
+  __shared__ float sred[2 * 32];
   __shared__ int sredi[32];
+  __shared__ int s_owner;
   __shared__ float s_cval[kCollect];
   __shared__ int s_cidx[kCollect];
   __shared__ int s_ccount;
-  __shared__ float s_scan[kSampT / 64];
   __shared__ uint32_t s_tkey[kSampT];
   __shared__ uint32_t s_lb, s_fkey;
   __shared__ uint32_t s_own[SLOTS * 4];
@@ -169,13 +246,14 @@ __global__ void __launch_bounds__(kSampT) sample_kernel(SampleParams p) {
 
   const int b = blockIdx.x;
   const int t = threadIdx.x;
+  Red red{sred, 0};
   const bf16_t* lrow = p.logits + (size_t)b * p.ld;
   const int nvec = p.V >> 3;
 
   // ---- load the raw row once ----
   uint4v row[SLOTS];
   const uint32_t* lmask =
-      (p.mask_logprobs && p.mask && p.mask_rows[b] >= 0) ? p.mask + (size_t)p.mask_rows[b] * (p.V >> 5) : nullptr;
+      (PROC && p.mask_logprobs && p.mask && p.mask_rows[b] >= 0) ? p.mask + (size_t)p.mask_rows[b] * (p.V >> 5) : nullptr;
 #pragma unroll
   for (int j = 0; j < SLOTS; ++j) {
     const int vi = j * kSampT + t;
@@ -194,13 +272,15 @@ __global__ void __launch_bounds__(kSampT) sample_kernel(SampleParams p) {
   float mx = -INFINITY;
 OPAQUE_ROW(row);
 #pragma unroll
-  for (int j = 0; j < SLOTS; ++j)
+  for (int j = 0; j < SLOTS; ++j) {
 #pragma unroll
     for (int e = 0; e < 8; ++e) mx = fmaxf(mx, GET(row, j, e));
+    __builtin_amdgcn_sched_barrier(0);  // one slot's values live at a time
+  }
   const uint32_t my_maxkey = f2key(mx);
-  const float raw_max = block_max(mx, sred);
+  const float raw_max = red.max(mx);
   const int lane = t & 63, wid = t >> 6;
-  const int K = p.num_logprobs;
+  const int K = TOPK ? p.num_logprobs : 0;
   // The raw log-sum-exp (the denominator of every reported logprob) is only computed when some output
   // needs it, and its exp sum rides along in a pass that runs anyway: the processed-row pass, or the
   // sampling pass's exp when the row is unprocessed (then its max IS the raw max).  Only a greedy
@@ -210,7 +290,7 @@ OPAQUE_ROW(row);
 
   // ---- raw top-K (for top_logprobs): candidates collected here, ranked and written once the
   // log-sum-exp is known ----
-  if (K > 0) {
+  if constexpr (TOPK) {
     // Bound first: the K largest per-thread maxima are K distinct elements, so the K-th largest element
     // of the row is >= the K-th largest thread max (lb).  One wave finds lb over the 1024 thread maxima
     // (no block barriers inside the search); the elements >= lb — rarely more than a few dozen — are
@@ -221,13 +301,16 @@ OPAQUE_ROW(row);
     s_tkey[t] = my_maxkey;
     __syncthreads();
     if (t < 64) {
+      uint32_t tk[kSampT / 64];
+#pragma unroll
+      for (int i = 0; i < kSampT / 64; ++i) tk[i] = s_tkey[i * 64 + t];
       uint32_t lo = 0x80u, hi = 0xffffu;
       while (lo < hi) {
         const uint32_t mid = (lo + hi + 1) >> 1;
-        float c = 0.f;
+        int c = 0;
 #pragma unroll
-        for (int i = 0; i < kSampT / 64; ++i) c += s_tkey[i * 64 + t] >= mid ? 1.f : 0.f;
-        if (wave_sum(c) >= (float)K)
+        for (int i = 0; i < kSampT / 64; ++i) c += __popcll(__builtin_amdgcn_ballot_w64(tk[i] >= mid));
+        if (c >= K)
           lo = mid;
         else
           hi = mid - 1;
@@ -245,10 +328,12 @@ OPAQUE_ROW(row);
           int c = 0;
 OPAQUE_ROW(row);
 #pragma unroll
-          for (int j = 0; j < SLOTS; ++j)
+          for (int j = 0; j < SLOTS; ++j) {
 #pragma unroll
             for (int e = 0; e < 8; ++e) c += f2key(GET(row, j, e)) >= mid;
-          if (block_sum_i(c, sredi) >= K)
+            __builtin_amdgcn_sched_barrier(0);  // one slot's values live at a time
+          }
+          if (red.sum_i(c) >= K)
             lo = mid;
           else
             hi = mid - 1;
@@ -257,41 +342,44 @@ OPAQUE_ROW(row);
         if (t == 0) s_ccount = 0;
         __syncthreads();
       }
-      // candidates are sparse (a few dozen of 128k): one float compare per element and a wave-uniform
-      // branch on its ballot; only an element position where some lane of the wave hits runs the exact
-      // key test and the LDS append (key2f(lo) is the smallest value with key >= lo, so the float test
+      // candidates are sparse (a few dozen of 128k): one compare of a slot's largest value and a wave-uniform
+      // branch on its ballot; only a slot where some lane of the wave hits looks at its elements one by one, and only
+      // an element position that hits runs the exact key test and the LDS append (key2f(lo) is the smallest value with key >= lo, so the float test
       // passes a superset: -0 next to +0)
       const float thr = key2f(lo);
 OPAQUE_ROW(row);
 #pragma unroll
-      for (int j = 0; j < SLOTS; ++j)
+      for (int j = 0; j < SLOTS; ++j) {
+        float top = GET(row, j, 0);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float v = GET(row, j, e);
-          const bool h = v >= thr;
-          if (__builtin_amdgcn_ballot_w64(h)) {
-            const int idx = (j * kSampT + t) * 8 + e;
-            if (h && f2key(v) >= lo) {  // padding past V holds -inf (key 0x7f < lo): never collected
+        for (int e = 1; e < 8; ++e) top = fmaxf(top, GET(row, j, e));
+        if (__builtin_amdgcn_ballot_w64(top >= thr)) {
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            const float v = GET(row, j, e);
+            if (v >= thr && f2key(v) >= lo) {  // padding past V holds -inf (key 0x7f < lo): never collected
               const int slot = atomicAdd(&s_ccount, 1);
               if (slot < kCollect) {
                 s_cval[slot] = v;
-                s_cidx[slot] = idx;
+                s_cidx[slot] = (j * kSampT + t) * 8 + e;
               }
             }
           }
         }
+        __builtin_amdgcn_sched_barrier(0);
+      }
       __syncthreads();
       if (s_ccount <= kCollect) break;  // block-uniform
     }
   }
 
   // ---- processed values y = raw + bias - penalties (masked -> -inf), stored back as bf16 ----
-  const float* brow = (p.bias && p.bias_rows[b] >= 0) ? p.bias + (size_t)p.bias_rows[b] * p.V : nullptr;
-  const uint32_t* mrow = (p.mask && p.mask_rows[b] >= 0) ? p.mask + (size_t)p.mask_rows[b] * (p.V >> 5) : nullptr;
-  const int crow_i = p.counts ? (p.count_rows ? p.count_rows[b] : b) : -1;
+  const float* brow = (PROC && p.bias && p.bias_rows[b] >= 0) ? p.bias + (size_t)p.bias_rows[b] * p.V : nullptr;
+  const uint32_t* mrow = (PROC && p.mask && p.mask_rows[b] >= 0) ? p.mask + (size_t)p.mask_rows[b] * (p.V >> 5) : nullptr;
+  const int crow_i = PROC && p.counts ? (p.count_rows ? p.count_rows[b] : b) : -1;
   const uint16_t* crow = crow_i >= 0 ? p.counts + (size_t)crow_i * p.V : nullptr;
-  const float fpen = p.freq_pen ? p.freq_pen[b] : 0.f, ppen = p.pres_pen ? p.pres_pen[b] : 0.f;
-  const float rpen = p.rep_pen ? p.rep_pen[b] : 1.f;
+  const float fpen = PROC && p.freq_pen ? p.freq_pen[b] : 0.f, ppen = PROC && p.pres_pen ? p.pres_pen[b] : 0.f;
+  const float rpen = PROC && p.rep_pen ? p.rep_pen[b] : 1.f;
   const bool use_pen = crow && (fpen != 0.f || ppen != 0.f || rpen != 1.f);
   const bool processed = brow || mrow || use_pen;
   if (processed) {
@@ -337,17 +425,17 @@ OPAQUE_ROW(row);
   const float T = p.temperature[b];
   int token = 0;
   float raw_lse = __builtin_nanf("");
-  if (T <= 0.f) {
-    if (need_lse) {
-      if (!processed) {
 OPAQUE_ROW(row);
+  if (need_lse && !processed) {  // (in the passes below it would double their live values: spills)
 #pragma unroll
-        for (int j = 0; j < SLOTS; ++j)
+    for (int j = 0; j < SLOTS; ++j) {
 #pragma unroll
-          for (int e = 0; e < 8; ++e) se += __expf(GET(row, j, e) - raw_max);
-      }
-      raw_lse = raw_max + __logf(block_sum(se, sred));
+      for (int e = 0; e < 8; ++e) se += __expf(GET(row, j, e) - raw_max);
+      __builtin_amdgcn_sched_barrier(0);
     }
+  }
+  if (T <= 0.f) {
+    if (need_lse) raw_lse = raw_max + __logf(red.sum(se));
     // ---- greedy: argmax (lowest index on ties).  The row maximum is known (the raw max; a processed row
     // takes one max pass), so the argmax is the lowest index holding it — instead of a value-and-index
     // compare chain with a branch per element.  (Padding past V holds -inf: it can only match
@@ -355,24 +443,19 @@ OPAQUE_ROW(row);
     float gm = raw_max;
     if (processed) {
       float ym = -INFINITY;
-OPAQUE_ROW(row);
 #pragma unroll
-      for (int j = 0; j < SLOTS; ++j)
+      for (int j = 0; j < SLOTS; ++j) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) ym = fmaxf(ym, GET(row, j, e));
-      gm = block_max(ym, sred);
+        __builtin_amdgcn_sched_barrier(0);  // one slot's values live at a time
+      }
+      gm = red.max(ym);
     }
     // the thread's elements visited from its highest index down, the last match wins: its lowest index,
     // one compare + one select per element, no branch
-    int bi = 0x7fffffff;
-OPAQUE_ROW(row);
-#pragma unroll
-    for (int j = SLOTS - 1; j >= 0; --j)
-#pragma unroll
-      for (int e = 7; e >= 0; --e) {
-        bi = GET(row, j, e) == gm ? (j * kSampT + t) * 8 + e : bi;
-      }
-    int cand = bi;
+    int cand;
+    if constexpr (PROC) { OPAQUE_ROW(row); }
+    LOWEST_INDEX(GET(row, j, e) == gm, cand);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, 64));
     __syncthreads();
@@ -385,14 +468,16 @@ OPAQUE_ROW(row);
   } else {
     const float invT = 1.f / T;
     float ymax = raw_max;  // unprocessed row: the processed max IS the raw max (no extra pass)
+OPAQUE_ROW(row);
     if (processed) {
       float ym = -INFINITY;
-OPAQUE_ROW(row);
 #pragma unroll
-      for (int j = 0; j < SLOTS; ++j)
+      for (int j = 0; j < SLOTS; ++j) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) ym = fmaxf(ym, GET(row, j, e));
-      ymax = block_max(ym, sred);
+        __builtin_amdgcn_sched_barrier(0);  // one slot's values live at a time
+      }
+      ymax = red.max(ym);
     }
     if (!(ymax > -INFINITY)) ymax = 0.f;  // every token masked: all u = 0 (the argmax fallback below)
     const uint32_t kOne2 = 0x00010001u, kH1 = 0x3C003C00u;
@@ -401,15 +486,6 @@ OPAQUE_ROW(row);
     // raw 16-bit keys and sums fp16 values: no transcendental inside the searches.  The same pass
     // sums this thread's share of Z (over the ROUNDED values, as every later mass is).
     float zloc = 0.f;
-    // unprocessed row + logprobs wanted: the raw exp sum needs its own pass over the raw values (fusing
-    // it into the pass below doubles that pass's live values and the SLOTS=16 instance spills)
-    if (need_lse && !processed) {
-OPAQUE_ROW(row);
-#pragma unroll
-      for (int j = 0; j < SLOTS; ++j)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) se += __expf(GET(row, j, e) - raw_max);
-    }
     // u = 2^(y * c1 + c0), c1 = log2(e) / T, c0 ~ -ymax * c1 rounded so that the exponent of y = ymax is
     // >= 0: with v_cvt_pkrtz (round toward zero) the max element is exactly 1.0 (0x3C00) and every other
     // element (at least one bf16 ulp below it, far above the fp32 rounding of c0) below 1; y = -inf gives
@@ -432,21 +508,16 @@ OPAQUE_ROW(row);
         zloc = __builtin_amdgcn_fdot2(as_h2(w), ones2, zloc, false);
         row[j][c] = w;
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
-    float Z;
-    if (need_lse) {  // both sums in one block reduction
-      const float zw = wave_sum(zloc), sw = wave_sum(se);
-      __syncthreads();
-      if (lane == 0) {
-        sred[wid] = zw;
-        sred[16 + wid] = sw;
-      }
-      __syncthreads();
-      Z = wave_sum(lane < kSampT / 64 ? sred[lane] : 0.f);
-      raw_lse = raw_max + __logf(wave_sum(lane < kSampT / 64 ? sred[16 + lane] : 0.f));
-    } else {
-      Z = block_sum(zloc, sred);
-    }
+    // Z: from the scan of the first draw where that runs over every element and nothing needs it earlier (no top-k,
+    // no top-a: the usual case), else a reduction of its own
+    const int k = p.top_k[b];
+    const float mp = p.min_p[b], ta = p.top_a[b];
+    const bool z_from_scan = k <= 0 && !(ta > 0.f) && !(mp > 0.f);
+    float Z = 0.f;
+    if (need_lse) raw_lse = raw_max + __logf(red.sum(se));
+    if (!z_from_scan) Z = red.sum(zloc);
     // mass of the elements with key >= KEY (macro, not a lambda: a by-reference capture of `row`
     // makes it addressable and sends it to scratch)
 #define MASS_LOCAL(KEY, OUT)                                                           \
@@ -464,10 +535,9 @@ OPAQUE_ROW(row);
   do {                           \
     float _l;                    \
     MASS_LOCAL(KEY, _l);         \
-    OUT = block_sum(_l, sred);   \
+    OUT = red.sum(_l);           \
   } while (0)
     uint32_t tau_k = 0;  // top-k: keep elements with key >= tau_k
-    const int k = p.top_k[b];
     if (k > 0) {
       uint32_t lo = 0, hi = 0x3C00u;  // keys of [0, 1.0]
       while (lo < hi) {
@@ -480,7 +550,7 @@ OPAQUE_ROW(row);
           count2(c2, row[j][0], row[j][1], t2, kOne2);
           count2(c2, row[j][2], row[j][3], t2, kOne2);
         }
-        if (block_sum_i((int)((c2 & 0xffffu) + (c2 >> 16)), sredi) >= k)
+        if (red.sum_i((int)((c2 & 0xffffu) + (c2 >> 16))) >= k)
           lo = mid;
         else
           hi = mid - 1;
@@ -489,9 +559,7 @@ OPAQUE_ROW(row);
     }
     // the filters other than top-p are plain lower bounds on the key
     uint32_t L0 = tau_k;
-    const float mp = p.min_p[b];
     if (mp > 0.f) L0 = max(L0, (uint32_t)h2bits(mp));        // u_i >= min_p  (u_max = 1)
-    const float ta = p.top_a[b];
     if (ta > 0.f) L0 = max(L0, (uint32_t)h2bits(fminf(ta / Z, 1.f)));  // p_i >= top_a p_max^2 <=> u_i >= top_a / Z
     if (L0 > 0x3C00u) L0 = 0x3C00u;                            // never filter out the argmax (u = 1)
     if (L0 == 0u) L0 = 1u;                                     // zero-mass elements are never kept
@@ -504,7 +572,7 @@ OPAQUE_ROW(row);
     // the common case.
     const float tp = p.top_p[b];
     float target = 0.f;
-    if (tp < 1.f) {
+    if (tp < 1.f && !z_from_scan) {
       float mk = Z;
       if (tau_k > 0u) MASS_GE(tau_k, mk);
       target = tp * mk;
@@ -523,61 +591,54 @@ OPAQUE_ROW(row);
       else
         MASS_LOCAL(tau, local);
       // exclusive scan of `local` over threads
-      float incl = local;
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const float n = __shfl_up(incl, o, 64);
-        if (lane >= o) incl += n;
-      }
-      __syncthreads();
-      if (lane == 63) s_scan[wid] = incl;
+      const float incl = wave_scan(local);
+      float* sc = red.set();
+      if (lane == 63) sc[wid] = incl;
+      if (t == 0) s_owner = 0x7fffffff;
       __syncthreads();
       float wave_off = 0.f, total = 0.f;
+#pragma unroll
       for (int w = 0; w < kSampT / 64; ++w) {
-        const float sw = s_scan[w];
+        const float sw = sc[w];
         if (w < wid) wave_off += sw;
         total += sw;
       }
+      if (z_from_scan && attempt == 0) target = tp * total;  // (the first draw's total is Z)
       const float excl = wave_off + incl - local;
       const float u01 = (((attempt == 0 ? ctr[0] : ctr[1]) >> 8) + 0.5f) * (1.0f / 16777216.0f);
       const float u = u01 * total;
       // The owner: the lowest thread whose [excl, excl + local) holds u — or, when rounding put u at or
       // past the end, the last thread with mass (its last kept element is taken).  Its packed u go to
-      // LDS and ONE wave walks them (two elements per dword, an exclusive scan over the lanes) instead
+      // LDS and its wave walks them (two elements per dword, an exclusive scan over the lanes) instead
       // of a single lane stepping through 8 * SLOTS elements with a branch each.
-      int cand = (local > 0.f && u >= excl && u < excl + local) ? t : 0x7fffffff;
-      int lastt = local > 0.f ? t : -1;
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        cand = min(cand, __shfl_xor(cand, o, 64));
-        lastt = max(lastt, __shfl_xor(lastt, o, 64));
-      }
+      if (local > 0.f && u >= excl && u < excl + local) atomicMin(&s_owner, t);
       __syncthreads();
-      if (lane == 0) {
-        sredi[wid] = cand;
-        sredi[16 + wid] = lastt;
-      }
-      __syncthreads();
-      cand = lane < (kSampT / 64) ? sredi[lane] : 0x7fffffff;
-      lastt = lane < (kSampT / 64) ? sredi[16 + lane] : -1;
+      int owner = s_owner;  // block-uniform
+      const bool past_end = owner == 0x7fffffff;
+      if (past_end) {
+        int lastt = local > 0.f ? t : -1;
 #pragma unroll
-      for (int o = 32; o > 0; o >>= 1) {
-        cand = min(cand, __shfl_xor(cand, o, 64));
-        lastt = max(lastt, __shfl_xor(lastt, o, 64));
+        for (int o = 32; o > 0; o >>= 1) lastt = max(lastt, __shfl_xor(lastt, o, 64));
+        if (lane == 0) sredi[wid] = lastt;
+        __syncthreads();
+        lastt = lane < (kSampT / 64) ? sredi[lane] : -1;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) lastt = max(lastt, __shfl_xor(lastt, o, 64));
+        owner = lastt;
       }
-      const bool past_end = cand == 0x7fffffff;
-      const int owner = past_end ? lastt : cand;  // block-uniform
       found = 0x7fffffff;
       if (owner >= 0) {
-        if (t == owner) {
+        if (wid == (owner >> 6)) {  // the owner's wave: its LDS writes are its own reads' (in order, no barrier)
+          if (t == owner) {
 #pragma unroll
-          for (int j = 0; j < SLOTS; ++j)
+            for (int j = 0; j < SLOTS; ++j)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) s_own[j * 4 + c] = row[j][c];
-          s_oexcl = excl;
-        }
-        __syncthreads();
-        if (t < 64) {
+              for (int c = 0; c < 4; ++c) s_own[j * 4 + c] = row[j][c];
+            s_oexcl = excl;
+          }
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
           constexpr int ND = SLOTS * 4, P = (ND + 63) / 64;  // lane: dwords [lane*P, lane*P + P)
           float v[2 * P];
           float sl = 0.f;
@@ -593,13 +654,7 @@ OPAQUE_ROW(row);
               sl += v[2 * q + h];
             }
           }
-          float incl = sl;
-#pragma unroll
-          for (int o = 1; o < 64; o <<= 1) {
-            const float n = __shfl_up(incl, o, 64);
-            if (lane >= o) incl += n;
-          }
-          float acc = s_oexcl + incl - sl;
+          float acc = s_oexcl + wave_scan(sl) - sl;
           int mine = -1, lastk = -1;
 #pragma unroll
           for (int e = 0; e < 2 * P; ++e)
@@ -632,21 +687,15 @@ OPAQUE_ROW(row);
         // u landed past the last kept element through rounding: fall back to argmax (key 0x3C00: always
         // inside the nucleus)
         float bv = -INFINITY;
-        int bi = 0x7fffffff;
 OPAQUE_ROW(row);
 #pragma unroll
         for (int j = 0; j < SLOTS; ++j)
 #pragma unroll
-          for (int e = 0; e < 8; ++e) {
-            const float v = GETU(row, j, e);
-            const int idx = (j * kSampT + t) * 8 + e;
-            if (v > bv || (v == bv && idx < bi)) {  // padding past V has u = 0 < u_max = 1
-              bv = v;
-              bi = idx;
-            }
-          }
-        const float gm = block_max(bv, sred);
-        int cand = (bv == gm) ? bi : 0x7fffffff;
+          for (int e = 0; e < 8; ++e) bv = fmaxf(bv, GETU(row, j, e));  // padding past V has u = 0 < u_max = 1
+        const float gm = red.max(bv);
+        int cand;
+OPAQUE_ROW(row);
+        LOWEST_INDEX(GETU(row, j, e) == gm, cand);
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, 64));
         __syncthreads();
@@ -681,7 +730,7 @@ OPAQUE_ROW(row);
 #undef MASS_GE
     token = found;
   }
-  if (K > 0 && t < 64) {  // one wave: rank-sort the collected top-K candidates (value desc, index asc)
+  if (TOPK && t < 64) {  // one wave: rank-sort the collected top-K candidates (value desc, index asc)
     const int n = min(s_ccount, kCollect);
     for (int r = n + t; r < K; r += 64) {  // fewer finite values than K: empty slots
       p.out_topk_ids[(size_t)b * K + r] = -1;
@@ -704,7 +753,7 @@ OPAQUE_ROW(row);
   if (t == 0) {
     p.out_token[b] = token;
     p.out_logprob[b] = bf2f(lrow[token]) - raw_lse;
-    if (p.counts && crow_i >= 0) {
+    if (PROC && p.counts && crow_i >= 0) {
       uint16_t* c = p.counts + (size_t)crow_i * p.V + token;
       if (*c < 0xffffu) *c += 1;
     }
@@ -728,15 +777,24 @@ extern "C" int lwc_sample(const void* logits, int ld, int V, int B, const float*
                  mask_logprobs, need_logprob, out_token, out_logprob, out_topk_ids, out_topk_lp};
   const int nvec = V / 8;
   const int slots = (nvec + kSampT - 1) / kSampT;
+  const bool proc = bias || mask || counts;
+#define LWC_SAMPLE(S)                                                                                                \
+  do {                                                                                                               \
+    if (proc && num_logprobs > 0) sample_kernel<S, true, true><<<B, kSampT, 0, s>>>(p);                              \
+    else if (proc) sample_kernel<S, true, false><<<B, kSampT, 0, s>>>(p);                                            \
+    else if (num_logprobs > 0) sample_kernel<S, false, true><<<B, kSampT, 0, s>>>(p);                                \
+    else sample_kernel<S, false, false><<<B, kSampT, 0, s>>>(p);                                                     \
+  } while (0)
   if (slots <= 4)
-    sample_kernel<4><<<B, kSampT, 0, s>>>(p);
+    LWC_SAMPLE(4);
   else if (slots <= 8)
-    sample_kernel<8><<<B, kSampT, 0, s>>>(p);
+    LWC_SAMPLE(8);
   else if (slots <= 16)
-    sample_kernel<16><<<B, kSampT, 0, s>>>(p);
+    LWC_SAMPLE(16);
   else if (slots <= 20)
-    sample_kernel<20><<<B, kSampT, 0, s>>>(p);
+    LWC_SAMPLE(20);
   else
     return -1;
+#undef LWC_SAMPLE
   return (int)hipGetLastError();
 }

@@ -630,6 +630,77 @@ def test_sample_bias_mask_penalty(gpu):
     assert counts[0, tok[0].long()].item() == 1  # the sampled token was counted
 
 
+def _philox_uniform(seed, offset):
+    """First word of Philox4x32-10 for a (seed, step) pair as the sampler's uniform in (0, 1)."""
+    c, k = [offset & 0xffffffff, offset >> 32, 0, 0], [seed & 0xffffffff, seed >> 32]
+    for _ in range(10):
+        a, b = 0xD2511F53 * c[0], 0xCD9E8D57 * c[2]
+        c = [(b >> 32) ^ c[1] ^ k[0], b & 0xffffffff, (a >> 32) ^ c[3] ^ k[1], a & 0xffffffff]
+        k = [(k[0] + 0x9E3779B9) & 0xffffffff, (k[1] + 0xBB67AE85) & 0xffffffff]
+    return ((c[0] >> 8) + 0.5) / 16777216.0
+
+
+@pytest.mark.parametrize("V", [32, 8192, 32768, 40000, 128256, 163840])
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("K", [0, 20])
+def test_sample_draws_follow_the_uniform(gpu, V, masked, K):
+    """Every build of the sampler (rows of 4 to 20 slots, with and without masks and logprobs): the drawn token is the one
+    whose share of the cumulative mass, in the kernel's order of elements, holds the row's Philox uniform.  The masses
+    are fp16 values (2^-10 relative, rounded toward zero) and fp32 sums: the cumulative share is off by at most 2^-10 of
+    itself.  Greedy rows take the lowest index among equal maxima."""
+    from llm_weighted_consensus_amd import ops
+
+    B, T = 12, 0.7
+    g = torch.Generator(device=gpu).manual_seed(V + K)
+    x = (torch.randn(B, V, generator=g, device=gpu) * 2).to(torch.bfloat16)
+    x[0, V // 2] = x[0, V - 1] = 20.0    # equal maxima
+    x[1] = 0.0                           # every token alike
+    x[2, :] = -60.0
+    x[2, V - 3] = 5.0                    # one token has all the mass
+    seeds = torch.arange(3, 3 + B, dtype=torch.int64, device=gpu) * 0x123456789
+    offs = torch.arange(B, dtype=torch.int64, device=gpu) + (1 << 33)
+    f = lambda v, dt=torch.float32: torch.full((B,), v, dtype=dt, device=gpu)  # noqa: E731
+    mask = rows = None
+    ok = torch.ones(B, V, dtype=torch.bool, device=gpu)
+    if masked:
+        bits = torch.rand(B, V, generator=g, device=gpu) < 0.5
+        bits[:, V - 3] = True
+        w = (bits.view(B, V // 32, 32).long() << torch.arange(32, device=gpu)).sum(-1)
+        mask, rows = torch.where(w >= 1 << 31, w - (1 << 32), w).to(torch.int32), torch.arange(B, dtype=torch.int32, device=gpu)
+        rows[5] = -1
+        ok = bits.clone()
+        ok[5] = True
+
+    def run(temp, top_p=1.0):
+        return ops.sample(x, f(temp), f(top_p), f(0, torch.int32), f(0.0), f(0.0), seeds, offs, num_logprobs=K, mask=mask, mask_rows=rows,
+                          need_logprob=K > 0)
+
+    y = x.float().masked_fill(~ok, -float("inf"))
+    assert run(0.0)[0].tolist() == [int((y[b] == y[b].max()).nonzero()[0]) for b in range(B)]
+    tok, lp, ids, lps = run(T)
+    slots = next(s for s in (4, 8, 16, 20) if V <= 8 * 1024 * s)
+    i = torch.arange(V, device=gpu)
+    order = torch.argsort((i // 8 % 1024) * (slots * 8) + (i // 8192) * 8 + i % 8)     # thread, slot, element
+    m = torch.exp((y.double() - y.max(-1, keepdim=True).values.double()) / T)
+    m[m < 2.0 ** -24] = 0.0
+    c = m[:, order].cumsum(-1)
+    for b in range(B):
+        at = int((order == int(tok[b])).nonzero())
+        lo, hi = (c[b, at] - m[b, order[at]]).item() / c[b, -1].item(), c[b, at].item() / c[b, -1].item()
+        u = _philox_uniform(int(seeds[b]), int(offs[b]))
+        assert bool(ok[b, tok[b]]) and lo * (1 - 2 ** -10) - 1e-6 <= u <= hi * (1 + 2 ** -10) + 1e-6, (b, lo, u, hi)
+    nucleus = run(T, 0.6)[0]
+    for b in range(B):
+        above = m[b][m[b] > m[b, nucleus[b]] * (1 + 2 ** -9)].sum() / m[b].sum()
+        assert above < 0.6 + 1e-3
+    if K:
+        full = torch.log_softmax(x.double(), -1)
+        torch.testing.assert_close(lp.double(), full.gather(1, tok.long()[:, None])[:, 0], rtol=1e-5, atol=1e-4)
+        n, r = min(K, V), [b for b in range(B) if b not in (1, 2)]   # (not the rows of thousands of equal values)
+        torch.testing.assert_close(lps[r, :n].double(), full[r].topk(n).values, rtol=1e-5, atol=1e-4)
+        assert torch.equal(x[r].gather(1, ids[r, :n].long()), x[r].topk(n).values)
+
+
 def test_sample_reproducible(gpu):
     logits = _bf(8, 32000, dev=gpu, scale=2.0)
     a, *_ = _sample(logits, gpu, top_p=0.9)
