@@ -24,7 +24,7 @@ int r32_window_attn_mfma(const float*, const void*, const void*, long long, long
 int r32_window_attn_decode_ok(int, int, int);
 int r32_window_attn_decode_splits(int, int, int, int, int);
 int r32_window_attn_decode(const float*, const void*, const void*, long long, long long, int, const int*, const int*, int,
-                           const float*, const float*, int, int, float, float*, float*, int, int, void*, int, int, int, int, int, int, int,
+                           const float*, const float*, int, int, float, float*, float*, int, void*, int, int, int, int, int, int, int,
                            hipStream_t);
 int r32_conv_hist(const void*, int, const float*, int, int, float*, long long, const int*, const int*, const int*,
                   const int*, void*, int, void*, int, int, int, int, int, int, int, hipStream_t);
@@ -347,7 +347,7 @@ void window_attn_decode(Tensor q, Tensor k_cache, Tensor v_cache, Tensor positio
                               (long long)v_cache.stride(0), BS, positions.data_ptr<int>(), block_tables.data_ptr<int>(),
                               (int)block_tables.size(1), bias.has_value() ? bias->data_ptr<float>() : nullptr,
                               sink_ptr(sink, H, "window_attn_decode"), (int)window, (int)chunk, (float)cap, po, po + (int64_t)B * H * S * Dv, S,
-                              (int)max_keys, out.data_ptr(), ldo, B, (int)H, (int)G, D, Dv, values_in_keys ? 1 : 0, stream()),
+                              out.data_ptr(), ldo, B, (int)H, (int)G, D, Dv, values_in_keys ? 1 : 0, stream()),
        "window_attn_decode");
 }
 

@@ -12,26 +12,48 @@ extern "C" int r32_window_attn_decode_ok(int D, int Dv, int vk) {
 extern "C" int r32_window_attn_decode_wide_launch(const WAttnDecodeParams* p, int D, int gx, int gy, int gz, int chunks_per_group,
                                                   hipStream_t s);
 
-// out[b, h, :] = sum_s exp(m_s - M) o_s / sum_s exp(m_s - M) l_s  (splits that saw no key have l = 0)
+// out[b, h, :] = sum_s exp(m_s - M) o_s / sum_s exp(m_s - M) l_s  (splits that saw no key have l = 0, and no o)
 // sink (or null): exp(sink_h) joins the denominator.
+// Lane s of every wave weighs split s (S <= 64), so the loop over the splits only has loads that do not wait for one
+// another: at 64 splits of one row the step (both kernels) took 59 us with the
+// weights formed inside the loop, 26 now.
 __global__ void window_attn_reduce_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                           const float* __restrict__ sink, bf16_t* __restrict__ out, int ldo, int H, int S,
                                           int Dv) {
-  const int b = blockIdx.x, h = blockIdx.y;
-  const float* ml = part_ml + ((size_t)b * H + h) * S * 2;
-  float M = -1e30f;
-  for (int s = 0; s < S; ++s)
-    if (ml[2 * s + 1] > 0.f) M = fmaxf(M, ml[2 * s]);
+  const int b = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
+  float m = -1e30f, l = 0.f;
+  if (lane < S) {
+    const float* ml = part_ml + (((size_t)b * H + h) * S + lane) * 2;
+    m = ml[0];
+    l = ml[1];
+  }
+  const bool seen = l > 0.f;
+  float M = seen ? m : -1e30f;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
   if (sink) M = fmaxf(M, sink[h]);
-  float L = sink ? expf(sink[h] - M) : 0.f;
-  for (int s = 0; s < S; ++s)
-    if (ml[2 * s + 1] > 0.f) L += expf(ml[2 * s] - M) * ml[2 * s + 1];
+  const float w = seen ? expf(m - M) : 0.f;
+  float L = seen ? w * l : 0.f;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) L += __shfl_xor(L, o, 64);
+  if (sink) L += expf(sink[h] - M);
   const float inv = L > 0.f ? 1.0f / L : 0.f;
-  for (int dv = threadIdx.x; dv < Dv; dv += blockDim.x) {
-    float acc = 0.f;
-    for (int s = 0; s < S; ++s)
-      if (ml[2 * s + 1] > 0.f) acc += expf(ml[2 * s] - M) * part_o[(((size_t)b * H + h) * S + s) * Dv + dv];
-    out[(size_t)b * ldo + (size_t)h * Dv + dv] = f2bf(acc * inv);
+  const unsigned long long live = __ballot(seen);
+  const int n = live ? 64 - __builtin_clzll(live) : 0;  // splits fill from the first
+  const float* po = part_o + ((size_t)b * H + h) * S * Dv;
+  const int dv = 2 * threadIdx.x;
+  float2 acc = {0.f, 0.f};
+  if (dv < Dv)
+#pragma unroll 8
+    for (int s = 0; s < n; ++s) {
+      const float ws = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, w), s));
+      const float2 o = *reinterpret_cast<const float2*>(po + (size_t)s * Dv + dv);
+      acc.x += ws != 0.f ? ws * o.x : 0.f;  // (a split without keys has left its row as it was)
+      acc.y += ws != 0.f ? ws * o.y : 0.f;
+    }
+  if (dv < Dv) {
+    out[(size_t)b * ldo + (size_t)h * Dv + dv] = f2bf(acc.x * inv);
+    out[(size_t)b * ldo + (size_t)h * Dv + dv + 1] = f2bf(acc.y * inv);
   }
 }
 
@@ -46,12 +68,12 @@ int launch_decode_nv(const WAttnDecodeParams& p, int nv, dim3 grid, hipStream_t 
   return (int)hipGetLastError();
 }
 
-// Splits for a decode step of B sequences whose windows hold at most max_keys keys: about 2048 waves (two per SIMD),
-// at least 64 keys each.  Measured at 64 sequences x 8 kv heads x 2048 keys of 128: 3 splits 150 us, 4 splits
-// (2048 waves) 130 us, 8 splits 155 us, 16 splits 146 us (shorter key runs per wave, larger partials to merge).
+// Splits for a decode step of B sequences whose windows hold at most max_keys keys: about 2048 waves (two per SIMD, the
+// registers' limit).  Measured with contexts of 500 to 1500 keys of 128, 8 kv heads: at 64 sequences 2 splits 65 us, 4
+// (2048 waves) 54 us, 6 61 us, 8 56 us, 16 66 us; at 8 sequences 8 splits 22 us, 16 19 us, 32 (2048 waves) 20 us, 64 22 us.
 // Wide rows (D = 320, 576): workgroups of four waves, about 512 of them, or of eight (more than 16 heads), at most 256 of them
-// (one per CU: at 64 sequences x 32 heads x 576 / 512 over 2048 keys 4 splits take 105 us where 8 take 139 us), at least 128
-// keys each (their partials are large).
+// (one per CU: at 64 sequences x 32 heads x 576 / 512 4 splits take 74 us where 8 take 94 us), at least 128 keys each (their
+// partials are large).
 extern "C" int r32_window_attn_decode_splits(int B, int G, int Hg, int max_keys, int D) {
   const bool wide = D > 192;
   const int chunks = (Hg + 15) / 16;
@@ -63,12 +85,11 @@ extern "C" int r32_window_attn_decode_splits(int B, int G, int Hg, int max_keys,
   return s < 1 ? 1 : s;
 }
 
-// part_o: fp32 [B * H * S * Dv], part_ml: fp32 [B * H * S * 2] scratch of the caller.  max_keys: an upper bound of
-// the keys any row sees (min(window, longest context)), known on the host.
+// part_o: fp32 [B * H * S * Dv], part_ml: fp32 [B * H * S * 2] scratch of the caller.
 extern "C" int r32_window_attn_decode(const float* q, const void* k_cache, const void* v_cache, long long kb_stride,
                                       long long vb_stride, int block_size, const int* positions, const int* block_tables,
                                       int bt_width, const float* bias, const float* sink, int window, int chunk, float cap, float* part_o,
-                                      float* part_ml, int S, int max_keys, void* out, int ldo, int B, int H, int G, int D,
+                                      float* part_ml, int S, void* out, int ldo, int B, int H, int G, int D,
                                       int Dv, int vk, hipStream_t s) {
   if (B <= 0) return 0;
   if (!r32_window_attn_decode_ok(D, Dv, vk) || H % G != 0 || S < 1 || (block_size & (block_size - 1)) != 0) return -1;
@@ -80,8 +101,7 @@ extern "C" int r32_window_attn_decode(const float* q, const void* k_cache, const
     if ((1 << b) == block_size) p.bs_shift = b;
   p.bt_width = bt_width; p.bias = bias; p.window = window; p.chunk = chunk; p.cap = cap; p.part_o = part_o; p.part_ml = part_ml; p.H = H; p.G = G;
   p.S = S;
-  // a row's keys start at a multiple of 32 at or below its window's first key: up to max_keys + 31 keys to cover
-  p.keys_per_split = (((max_keys + 31 + S - 1) / S) + 31) / 32 * 32;
+  p.min_keys = D > 192 ? 128 : 64;
   const int Hg = H / G;
   const dim3 grid(B, G * ((Hg + 15) / 16), S);
   int rc = -1;
@@ -97,6 +117,6 @@ extern "C" int r32_window_attn_decode(const float* q, const void* k_cache, const
     }
   }
   if (rc != 0) return rc;
-  window_attn_reduce_kernel<<<dim3(B, H), 64, 0, s>>>(part_o, part_ml, sink, (bf16_t*)out, ldo, H, S, Dv);
+  window_attn_reduce_kernel<<<dim3(B, H), Dv <= 128 ? 64 : Dv / 2, 0, s>>>(part_o, part_ml, sink, (bf16_t*)out, ldo, H, S, Dv);
   return (int)hipGetLastError();
 }

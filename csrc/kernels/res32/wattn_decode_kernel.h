@@ -17,7 +17,10 @@ LWC_DEVICE float4v mfma16(const short8& a, const short8& b, const float4v& c) {
 // (up to 16) query heads that share head g, so K and V are read ONCE for all of them, straight from the paged
 // cache into the operands — no LDS: a K row's 16 bytes are an A operand as they lie, the interleaved V word is a
 // B operand as it lies.  Same arithmetic as the portion kernel (hi + lo halves of q and of the weights, bias
-// table, fp32 online softmax).  Each split leaves an unnormalised partial (o, m, l); the reduce kernel merges
+// table, fp32 online softmax).  Bound by the reads of the cache: 64 sequences of 500 to 1500 keys (1000 on average), 32
+// heads over 8 of 128 entries, take 54 us for 258 MB (42 us at the rate of a plain read of memory) in tables of 4096 keys.
+// With the splits cut for the table's width and every load of a tile waited for on its own it took 137 us, and 189 instead
+// of 104 us at 2048 keys each.  Each split leaves an unnormalised partial (o, m, l); the reduce kernel merges
 // them (splits == 1: still through the reduce, which then only normalises).
 struct WAttnDecodeParams {
   const float* q;          // [B, H*D]
@@ -34,7 +37,7 @@ struct WAttnDecodeParams {
   float cap;               // > 0: scores become cap tanh(score / cap)
   float* part_o;           // [B, H, S, Dv]
   float* part_ml;          // [B, H, S, 2]
-  int H, G, S, keys_per_split;  // keys_per_split: a multiple of 32
+  int H, G, S, min_keys;  // min_keys: the fewest keys a split takes before the next one gets any (a multiple of 32)
 };
 
 // NW waves per workgroup share one (sequence, head chunk, split).  With NW > 1 a tile's 32 key rows go through LDS
@@ -62,8 +65,12 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
   const int r16 = lane & 15, g4 = lane >> 4;
   const int i = p.positions[b];
   const int j_lo = max(max(0, i - p.window + 1), p.chunk > 0 ? i - i % p.chunk : 0);
-  const int base = (j_lo / 32) * 32 + split * p.keys_per_split;  // this split's first key (a multiple of 32)
-  const int last = min(i, base + p.keys_per_split - 1);
+  // The row's own keys divide among the splits (a multiple of 32 each): the host only knows the longest context there
+  // could be, and ranges cut for that one would leave the whole row to the first split.
+  const int first = (j_lo / 32) * 32, n_keys = max(i + 1 - first, 0);
+  const int keys_per_split = max(((n_keys + p.S - 1) / p.S + 31) / 32 * 32, p.min_keys);
+  const int base = first + split * keys_per_split;  // this split's first key (a multiple of 32)
+  const int last = min(i, base + keys_per_split - 1);
   const int* table = p.block_tables + (size_t)b * p.bt_width;
   const int BS = p.block_size, bsh = p.bs_shift;
   auto page_ix = [&](int j) { return j >> bsh; };
@@ -71,7 +78,7 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
   // the split's pages, one per lane, fetched once: a key's page then comes from a lane exchange instead of a table
   // load that every K / V load would have to wait for (splits longer than 64 pages look the table up directly)
   const int pg_base = page_ix(base);
-  const bool pages_in_lanes = page_ix(base + p.keys_per_split - 1) - pg_base < 64;
+  const bool pages_in_lanes = page_ix(base + keys_per_split - 1) - pg_base < 64;
   int my_page = 0;
   if (pages_in_lanes && pg_base + lane <= page_ix(max(i, 0)) && base <= i) my_page = table[pg_base + lane];
   auto page_of = [&](int j) { return pages_in_lanes ? __shfl(my_page, page_ix(j) - pg_base, 64) : table[page_ix(j)]; };
@@ -132,8 +139,49 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
     __syncthreads();
   }
 
+  // One wave alone (no LDS): a tile's value words and the next tile's key rows are in flight while the scores and the
+  // weights of the tile are formed.  (Rows past the split's keys are masked below: any valid row does.)
+  short8 kf[kStage ? 1 : 2 * ND];
+  short4v vf[kStage ? 1 : 2 * NVW];
+  auto load_keys = [&](int t0) {
+#pragma unroll
+    for (int sub = 0; sub < 2; ++sub) {
+      const int j = min(t0 + sub * 16 + r16, last);
+      const bf16_t* kr = p.k_cache + (long long)page_of(j) * p.kb_stride + ((long long)page_off(j) * G + g) * D + 8 * g4;
+#pragma unroll
+      for (int kd = 0; kd < ND; ++kd) kf[sub * ND + kd] = *reinterpret_cast<const short8*>(kr + kd * 32);
+    }
+  };
+  auto value_row = [&](int j) {
+    return p.v_cache + (long long)page_of(j) * p.vb_stride + (long long)(page_off(j) >> 2) * (4LL * G * DV) + 4LL * (g * DV + r16);
+  };
+  if constexpr (!kStage) {
+    if (base <= last) load_keys(base);
+  }
+
   for (int t0 = base; t0 <= last; t0 += 32) {  // (base and last are the same for every wave of the workgroup)
     if (kStage && t0 + 32 <= last) fetch(t0 + 32);
+    // the lane's two 4-key groups: keys t0 + 4 g4 .. and t0 + 16 + 4 g4 .. (groups past the token: any valid one,
+    // their weights are 0)
+    const int ja = min(t0 + 4 * g4, (i / 4) * 4), jb = min(t0 + 16 + 4 * g4, (i / 4) * 4);
+    const bf16_t *va = nullptr, *vb = nullptr;
+    if constexpr (!VK) {
+      va = value_row(ja);
+      vb = value_row(jb);
+    }
+    float bias_e[8];
+    if (bias_h) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) bias_e[e] = bias_h[min(max(i - (t0 + (e >> 2) * 16 + 4 * g4 + (e & 3)), 0), p.window - 1)];
+    }
+    if constexpr (!kStage) {
+#pragma unroll
+      for (int n = 0; n < NVW; ++n) {
+        vf[2 * n] = *reinterpret_cast<const short4v*>(va + 64 * n);
+        vf[2 * n + 1] = *reinterpret_cast<const short4v*>(vb + 64 * n);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
     float4v sacc[2];
     if constexpr (kSplitQK) {
       float4v part = float4v{0.f, 0.f, 0.f, 0.f};
@@ -160,17 +208,19 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
           if (QLO) sacc[sub] = mfma16(a, qlo[kd], sacc[sub]);
         }
       } else {
-        const int j = min(t0 + sub * 16 + r16, i);  // (rows past the token are masked below: any valid row does)
-        const bf16_t* kr = p.k_cache + (long long)page_of(j) * p.kb_stride + ((long long)page_off(j) * G + g) * D + 8 * g4;
 #pragma unroll
         for (int kd = 0; kd < ND; ++kd) {
-          const short8 a = *reinterpret_cast<const short8*>(kr + kd * 32);
-          sacc[sub] = mfma16(a, qhi[kd], sacc[sub]);
-          if (QLO) sacc[sub] = mfma16(a, qlo[kd], sacc[sub]);
+          sacc[sub] = mfma16(kf[sub * ND + kd], qhi[kd], sacc[sub]);
+          if (QLO) sacc[sub] = mfma16(kf[sub * ND + kd], qlo[kd], sacc[sub]);
         }
       }
     }
     }  // (scores without the split)
+    if constexpr (!kStage) {
+      __builtin_amdgcn_sched_barrier(0);
+      load_keys(t0 + 32);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     if (p.cap > 0.f) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) sacc[e >> 2][e & 3] = softcap_f(sacc[e >> 2][e & 3], p.cap, cap_k);
@@ -183,7 +233,7 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
       const int j = t0 + (e >> 2) * 16 + 4 * g4 + (e & 3);
       const int dist = i - j;
       ok[e] = h_valid && dist >= 0 && j >= j_lo && j <= last;
-      s[e] = ok[e] ? sacc[e >> 2][e & 3] - (bias_h ? bias_h[dist] : 0.f) : -1e30f;
+      s[e] = ok[e] ? sacc[e >> 2][e & 3] - (bias_h ? bias_e[e] : 0.f) : -1e30f;
       mx = fmaxf(mx, s[e]);
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -210,11 +260,6 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
     float ar[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, 4 * g4 + r, 64);
-    // the lane's two 4-key groups: keys t0 + 4 g4 .. and t0 + 16 + 4 g4 .. (groups past the token: any valid one,
-    // their weights are 0)
-    const int ja = min(t0 + 4 * g4, (i / 4) * 4), jb = min(t0 + 16 + 4 * g4, (i / 4) * 4);
-    const bf16_t* va = p.v_cache + (long long)page_of(ja) * p.vb_stride + (long long)(page_off(ja) >> 2) * (4LL * G * DV) + 4LL * (g * DV + r16);
-    const bf16_t* vb = p.v_cache + (long long)page_of(jb) * p.vb_stride + (long long)(page_off(jb) >> 2) * (4LL * G * DV) + 4LL * (g * DV + r16);
 #pragma unroll
     for (int n = 0; n < NVW; ++n) {
 #pragma unroll
@@ -227,6 +272,9 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
           bb[e] = (short)col[e * KLD];
           bb[4 + e] = (short)col[(16 + e) * KLD];
         }
+      } else if constexpr (!kStage) {
+        const short4v b0 = vf[2 * n], b1 = vf[2 * n + 1];
+        bb = short8{b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
       } else {
         const short4v b0 = *reinterpret_cast<const short4v*>(va + 64 * (wv * NVW + n));
         const short4v b1 = *reinterpret_cast<const short4v*>(vb + 64 * (wv * NVW + n));
@@ -241,11 +289,11 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
       __syncthreads();
     }
   }
-  // partials: O rows are heads 4 g4 + r, columns dv 16 n + r16
+  // partials: O rows are heads 4 g4 + r, columns dv 16 n + r16 (a split without keys leaves l = 0 and no row)
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int hr = 4 * g4 + r;
-    if (hr < nh) {
+    if (hr < nh && base <= last) {
       float* po = p.part_o + (((size_t)b * H + h0 + hr) * p.S + split) * DV;
 #pragma unroll
       for (int n = 0; n < NVW; ++n) po[(wv * NVW + n) * 16 + r16] = O[n][r];

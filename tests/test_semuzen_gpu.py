@@ -232,6 +232,55 @@ def test_capped_scores(gpu, dtype, tol, H, G, D, Dv, cap):
     assert (out.cpu().double().view(n - a, H, Dv) - ref[a:]).abs().max() < tol * 4
 
 
+@pytest.mark.parametrize("D,Dv", [(32, 32), (64, 128), (128, 128), (192, 128), (320, 256), (576, 512)])
+@pytest.mark.parametrize("window,splits,biased", [(NO_WINDOW, 0, False), (NO_WINDOW, 3, False), (NO_WINDOW, 64, False), (100, 5, True),
+                                                  (1000, 1, True)])
+def test_decode_splits_follow_each_rows_own_keys(gpu, D, Dv, window, splits, biased):
+    """Contexts from one key to the table's whole width, around the edges of a 32-key tile and of a split's least share, in
+    tables far wider than most of them.  Bound: the bf16 result's rounding (2^-9, doubled) plus, at D = 576, q's own (2^-9
+    relative, random over the entries: 2^-8 in a score of up to 5), over values of up to 4."""
+    from llm_weighted_consensus_amd.models.cache import PagedLayerCache
+    from llm_weighted_consensus_amd.ops import res32
+
+    wide = D > 192
+    H, G, bs, wpages = (20, 1, 16, 64) if wide else (12, 2, 16, 64)
+    lens = [1, 2, 31, 32, 33, 63, 64, 65, 127, 129, 200, 257, 1000, 1024]
+    g = torch.Generator().manual_seed(D + window % 1000)
+    nb = [-(-n // bs) for n in lens]
+    cache = PagedLayerCache([(G * D, G * Dv)], sum(nb), bs, gpu, BF16)
+    perm = torch.randperm(sum(nb), generator=g)
+    tables = torch.zeros(len(lens), wpages, dtype=torch.int32)
+    r1, r2 = torch.rand(H, generator=g), torch.rand(H, generator=g)
+    sink = torch.randn(H, generator=g)
+    Ks, Vs, at = [], [], 0
+    for i, n in enumerate(lens):
+        blk = perm[at:at + nb[i]]
+        at += nb[i]
+        tables[i, :nb[i]] = blk.to(torch.int32)
+        sl = (blk[:, None] * bs + torch.arange(bs)).reshape(-1)[:n]
+        K = (torch.randn(n, G, D, generator=g) * (0.2 + 1.5 * torch.arange(n)[:, None, None] / n)).clamp(-4, 4).to(BF16)
+        V = K[..., :Dv] if wide else torch.randn(n, G, Dv, generator=g).clamp(-4, 4).to(BF16)
+        cache.set_rows(0, sl.to(gpu), K.reshape(n, -1).to(gpu), V.reshape(n, -1).to(gpu))
+        Ks.append(K)
+        Vs.append(V)
+    q = torch.randn(len(lens), H, D, generator=g) * D ** -0.5
+    out = torch.empty(len(lens), H * Dv, dtype=BF16, device=gpu)
+    z = torch.zeros(H, device=gpu)
+    res32.window_attn(q.view(len(lens), -1).to(gpu), cache.k[0], cache.v[0], torch.tensor(lens, dtype=torch.int32, device=gpu) - 1,
+                      tables.to(gpu), z, z, window, out, H, G, cores=True, splits=splits, values_in_keys=wide, sink=sink.to(gpu),
+                      bias=res32.distance_bias(r1.to(gpu), r2.to(gpu), window) if biased else None)
+    got, tol = out.cpu().double().view(len(lens), H, Dv), 4 * (2 ** -8 + (2 ** -8 if D == 576 else 0))
+    for i, n in enumerate(lens):
+        K, V = (t[i].double().repeat_interleave(H // G, 1) for t in (Ks, Vs))
+        s = torch.einsum("hd,jhd->hj", q[i].double(), K)
+        dist = n - 1 - torch.arange(n)
+        if biased:
+            s = s - r1.double()[:, None] * torch.log1p(r2.double()[:, None] * dist)
+        s = s.masked_fill((dist >= window)[None], -1e300)
+        w = torch.cat([s, sink.double()[:, None]], 1).softmax(-1)[:, :-1]
+        assert (got[i] - torch.einsum("hj,jhv->hv", w, V)).abs().max() < tol, n
+
+
 @pytest.mark.parametrize("D,Dv", [(32, 32), (128, 128), (192, 128)])
 @pytest.mark.parametrize("window,chunk,cap,sink,biased", [(NO_WINDOW, 0, 0.0, False, False), (70, 0, 0.0, True, True),
                                                           (NO_WINDOW, 50, 4.0, False, False), (33, 0, 0.0, False, False)])
