@@ -66,7 +66,7 @@ int r32_retention_max_dim();
 int r32_retention_prep(const void*, int, int, const float*, float, const int*, float*, int, int, int, int, float, int, int,
                        hipStream_t);
 int r32_retention(const float*, const void*, int, const float*, float*, long long, const int*, const int*, const int*, float*,
-                  int, int, int, int, int, int, int, hipStream_t);
+                  int, int, int, int, int, int, int, int, hipStream_t);
 int r32_glu(const void*, int, void*, int, int, int, int, float, float, int, hipStream_t);
 int r32_act(const void*, int, void*, int, int, int, int, int, hipStream_t);
 int r32_hyper_max_streams();
@@ -867,7 +867,7 @@ void retention(Tensor proj, int64_t k_off, Tensor v, Tensor freq, double mult, i
        "retention_prep");
   done(r32_retention(qk.data_ptr<float>(), v.data_ptr(), ldv, decay.data_ptr<float>(), state.data_ptr<float>(),
                      (long long)state.stride(0), cu.data_ptr<int>(), item_slot.data_ptr<int>(), positions.data_ptr<int>(),
-                     out.data_ptr<float>(), ldo, (int)item_slot.numel(), (int)H, D, Dv, act ? 1 : 0, f, stream()), "retention");
+                     out.data_ptr<float>(), ldo, (int)item_slot.numel(), T, (int)H, D, Dv, act ? 1 : 0, f, stream()), "retention");
 }
 
 // in rows [gate (n) | up (n)], out rows of n; mode 0 silu(g) u, 1 the clamped unit g' sigmoid(alpha g') (u' + 1)

@@ -247,6 +247,47 @@ def test_retention_portions_single_tokens_and_stale_slots(gpu, dtype, tol, H, D,
         assert (state[slot[k]].cpu().double() - ref_S[k]).abs().max() < tol * 4 * max(1.0, float(ref_S[k].abs().max())), k
 
 
+@pytest.mark.parametrize("H,D,Dv,dtype", [(2, 128, 128, torch.bfloat16), (3, 32, 16, torch.float32), (2, 24, 40, torch.bfloat16),
+                                          (1, 64, 130, torch.float32), (2, 200, 72, torch.float32), (1, 256, 64, torch.bfloat16)])
+@pytest.mark.parametrize("act", [False, True])
+def test_retention_chunks(gpu, H, D, Dv, dtype, act):
+    """Portions around the edges of a 32-token chunk, fresh and behind earlier tokens, beside single rows; decays of 0, 1 and
+    between.  An infinite value reaches no token before it.  Bound: 64 roundings of 2^-24 over the sum of the terms' sizes (a
+    term passes two contractions of at most 64 entries, its powers, and one decay per chunk)."""
+    from llm_weighted_consensus_amd.ops import res32
+
+    g = torch.Generator().manual_seed(D + Dv)
+    lens = [1, 31, 32, 33, 64, 95, 257, 3]
+    decay = torch.tensor([0.98, 1.0, 0.0][:H] if H > 1 else [0.7])
+    f = torch.zeros(0, device=gpu)
+    nq, nv, T = H * D, H * Dv, sum(lens)
+    x = torch.randn(T, 2 * nq + nv, generator=g).to(dtype)
+    slots, start = list(range(len(lens)))[::-1], [0, 0, 7, 0, 5, 0, 0, 9]
+    state = torch.randn(len(lens), H, D, Dv, generator=g) * 3
+    first = state.clone()
+    state = state.to(gpu)
+    k_scale = 1.0 if act else D ** -0.5
+    run = lambda x: res32.retention(x.to(gpu), nq, x.to(gpu)[:, 2 * nq:], f, 1.0, 0, decay.to(gpu), state,
+                                    _items(lens, slots, start, gpu), H, k_scale=k_scale, act=act)
+    got = run(x).cpu().double()
+    z = x.double()
+    z = z * torch.sigmoid(z) if act else z
+    at = 0
+    for n, s, p in zip(lens, slots, start):
+        q, k, v = (z[at:at + n, a:b].reshape(n, H, -1) for a, b in ((0, nq), (nq, 2 * nq), (2 * nq, None)))
+        S0 = first[s].double() if p else torch.zeros(H, D, Dv, dtype=torch.float64)
+        dec = [float(d) for d in decay]
+        o, S = O.retention_scan(q, k * k_scale, v, dec, S=S0.clone())
+        ob, Sb = O.retention_scan(q.abs(), k.abs() * k_scale, v.abs(), dec, S=S0.abs())
+        assert ((got[at:at + n].view(n, H, Dv) - o).abs() <= 2 ** -18 * ob).all(), n
+        assert ((state[s].cpu().double() - S).abs() <= 2 ** -18 * Sb).all(), n
+        at += n
+    at = sum(lens[:6])
+    x[at + 40, 2 * nq] = float("inf")
+    again = run(x).cpu()
+    assert (again[at:at + 40].double() - got[at:at + 40]).abs().max() < 1e-6 * got[at:at + 40].abs().max() and not again[at + 40, 0].isfinite()
+
+
 def test_retention_far_token_survives_a_slow_decay(gpu):
     """One early token made large: after hundreds of tokens its share of the result is a^n times its value, for a fast
     and a slow head (prompt portion, then single tokens)."""
