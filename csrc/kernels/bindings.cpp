@@ -26,6 +26,8 @@ int lwc_grouped_gemm(const void*, const void*, void*, const int*, const float*, 
                      int, int, int, int, int, int, long long, int, float*, int, long long, hipStream_t);
 int lwc_gemm8p(const void*, const void*, void*, const void*, float*, int*, int, int, int, int, int, int, hipStream_t);
 int lwc_gemm8p_slots();
+void lwc_gemm2w_plan(int, int, int, int, long long, int*, int*);
+int lwc_gemm2w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, int, float*, int*, hipStream_t);
 int lwc_gemm4w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, float*, int, int, int,
                float, int, int, int, int, float*, int*, hipStream_t);
 int lwc_rms_rowsumsq(const void*, float*, int, int, hipStream_t);
@@ -427,6 +429,31 @@ void gemm8p(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::
   CHECK_RC(lwc_gemm8p(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, ws.data_ptr<float>(), flags.data_ptr<int>(), M, N,
                       K, (int)A.stride(0), (int)C.stride(0), (int)epi, cur_stream()),
            "gemm8p");
+}
+
+// gemm2w: tiles of 128 x 128 (tile 0), 192 x 128 (1), 128 x 192 (2) or 64 x 64 (3, in splits K ranges: part and count, the
+// latter zero between calls); tile -1: by the sizes, K ranges only with part and count
+void gemm2w(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::optional<at::Tensor>& R, int64_t epi,
+            int64_t tile, int64_t splits, const c10::optional<at::Tensor>& part, const c10::optional<at::Tensor>& count) {
+  const void* r = gemm_operands(A, W, C, R, epi);
+  const int M = (int)A.size(0), K = (int)A.size(1), N = (int)W.size(0);
+  if (tile < 0) {
+    int t = 0, s = 1;
+    const bool ws = part.has_value() && count.has_value();
+    lwc_gemm2w_plan(M, N, K, (int)epi, ws ? part->numel() / 4096 : 0, &t, &s);
+    tile = t, splits = s;
+  }
+  if (splits > 1) {
+    const int64_t tiles = ((int64_t)M + 63) / 64 * ((N + 63) / 64);
+    TORCH_CHECK(part.has_value() && count.has_value(), "gemm2w: K ranges need part and count");
+    CHECK_GPU(*part); CHECK_DTYPE(*part, at::kFloat); CHECK_CONTIG(*part);
+    CHECK_GPU(*count); CHECK_DTYPE(*count, at::kInt); CHECK_CONTIG(*count);
+    TORCH_CHECK(part->numel() >= tiles * splits * 4096 && count->numel() >= tiles, "gemm2w: workspace too small");
+  }
+  CHECK_RC(lwc_gemm2w(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, M, N, K, (int)A.stride(0), (int)C.stride(0), (int)epi,
+                      (int)tile, (int)splits, splits > 1 ? part->data_ptr<float>() : nullptr,
+                      splits > 1 ? count->data_ptr<int>() : nullptr, cur_stream()),
+           "gemm2w");
 }
 
 // gemm4w: the 4-wave interleaved core (one wave per SIMD, data-parallel tiles of 256 x bn, bn = 256 | 192).
@@ -975,6 +1002,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_decode", &paged_decode);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("gemm8p", &gemm8p);
+  m.def("gemm2w", &gemm2w);
   m.def("gemm4w", &gemm4w);
   m.def("skinny_gemm", &skinny_gemm);
   m.def("rms_rowsumsq", &rms_rowsumsq);

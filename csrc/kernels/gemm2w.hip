@@ -1,0 +1,300 @@
+// bf16 GEMM in tiles for two independent workgroups per CU (gfx950): C = A W^T with the epilogues of gemm8p.
+//
+// gemm8p's persistent 256 x 256 tiles leave CUs idle below some 8000 rows, hand partial tiles over through memory, and no
+// other work covers a tile's prologue and epilogue.  Here a workgroup is four waves with a tile of 64 to 192 rows or columns,
+// at most 80 KiB of LDS and 256 registers, so that two share a CU: one's MFMAs run while the other waits for its first rows,
+// reads operands or stores.  Rows arrive by LDS-DMA, 64 entries (a whole 128-byte line: with 32 the rate halves) at a time;
+// accumulators hold eight consecutive columns of a row, so the epilogue needs no LDS.
+// What bounds it: the rate at which rows reach LDS (12 to 15 TB/s over the chip), so the larger tiles at many rows, where it
+// stays behind the library's 256 x 256; below, the time of a K step on a CU that has one workgroup (0.33 us), which the K
+// ranges of few tiles shorten.
+// Measured against gemm8p and the library (us): 1000 rows x 4096 x K 1024, bias + GELU: 43 and 22 -> 16; 3600 x 1024 x 1024: 46 and
+// 20 -> 8 to 16; 7155 x 1024 x 1024: 40 and 24 -> 21; 61 x 4096 x 4096 (weights from memory): skinny 20, library 18 -> 13;
+// 61 x 28672 x 4096 SwiGLU 61 (library) -> 51; 61 x 4096 x 14336 39 (library) -> 28; 65536 x 4096 x 1024: 641 and 515, here 634.
+#include <algorithm>
+
+#include "common.h"
+
+namespace lwc {
+namespace g2w {
+
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4 };
+
+struct Params {
+  const bf16_t* A;
+  const bf16_t* W;
+  bf16_t* C;
+  const bf16_t* R;  // EPI_RESIDUAL: residual [M, ldc] (may be C); EPI_BIAS / EPI_BIAS_GELU: bias [N]
+  int M, N, K, lda, ldc;
+  int tiles_m, tiles_n;
+  int splits;   // K ranges per tile
+  float* part;  // splits > 1: [tiles][splits][TM * TN] partial tiles
+  int* count;   // [tiles] finished ranges (zero between launches)
+};
+
+LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
+LWC_DEVICE float silu(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+
+LWC_DEVICE void dma16(const __amdgpu_buffer_rsrc_t& r, uint8_t* dst, uint32_t vo, int so) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, 0);
+}
+
+// every outstanding load but the last N, and all LDS reads
+template <int N>
+LWC_DEVICE void wait_rows() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
+constexpr int kGroupM = 8;
+
+template <int EPI, int TM, int TN, int NST>
+__global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
+  constexpr int WC = EPI == EPI_SWIGLU && TN == 64 ? 1 : 2, WR = 4 / WC;  // waves across the tile's columns and rows
+  constexpr int kA = TM * 128, kStage = kA + TN * 128;  // bytes of a 64-deep K step: A rows, then W rows, 128 bytes each
+  constexpr int IA = TM / 32, IW = TN / 32;             // DMA instructions per wave and step
+  constexpr int MI = TM / WR / 16, NP = TN / WC / 32;   // the wave's 16-row tiles and its groups of 32 columns
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, q = lane >> 4, wr = wid / WC, wc = wid % WC;
+
+  // (the ranges of a tile are neighbours: they run on one XCD, and their partial sums meet in its L2)
+  const int u = xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n * p.splits), t = u / p.splits, split = u % p.splits;
+  const int first_m = t / (kGroupM * p.tiles_n) * kGroupM, gsz = min(p.tiles_m - first_m, kGroupM);
+  const int in = t % (kGroupM * p.tiles_n);
+  const int m0 = (first_m + in % gsz) * TM, n0 = in / gsz * TN;
+
+  // DMA: a wave's instruction fills 8 rows; lane l carries row l / 8 and the chunk of it that belongs at position l % 8:
+  // chunk c of A row r lies at c ^ (r / 2 % 8), of W row r at c ^ (r / 8 % 4 * 2 + r / 2 % 2), so that the 16-lane groups
+  // in which an operand read is served meet every bank once
+  const int rows_m = min(p.M - m0, TM), rows_n = min(p.N - n0, TN);
+  const __amdgpu_buffer_rsrc_t rA = uniform_rsrc(p.A + (size_t)m0 * p.lda, ((rows_m - 1) * p.lda + p.K) * 2);
+  const __amdgpu_buffer_rsrc_t rW = uniform_rsrc(p.W + (size_t)n0 * p.K, rows_n * p.K * 2);
+  uint32_t voA[IA], voW[IW];
+#pragma unroll
+  for (int i = 0; i < IA; ++i) {
+    const int row = (i * 4 + wid) * 8 + (lane >> 3);
+    voA[i] = row < rows_m ? (uint32_t)(row * p.lda * 2 + (((lane & 7) ^ ((row >> 1) & 7)) << 4)) : 0x7fffffffu;
+  }
+#pragma unroll
+  for (int i = 0; i < IW; ++i) {
+    const int row = (i * 4 + wid) * 8 + (lane >> 3);
+    voW[i] = row < rows_n ? (uint32_t)(row * p.K * 2 + (((lane & 7) ^ ((row >> 3 & 3) * 2 + (row >> 1 & 1))) << 4)) : 0x7fffffffu;
+  }
+  auto stage = [&](uint8_t* buf, int kt) {
+#pragma unroll
+    for (int i = 0; i < IA; ++i) dma16(rA, buf + (i * 4 + wid) * 1024, voA[i], kt * 128);
+#pragma unroll
+    for (int i = 0; i < IW; ++i) dma16(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], kt * 128);
+  };
+  // operand reads: A tile i holds rows 16 i + r16; W tile (g, h) holds rows 32 g + 8 (r16 / 4) + 4 h + r16 % 4, so that a
+  // lane's accumulators of the pair h = 0, 1 are the eight consecutive columns 32 g + 8 q .. of output row r16
+  const int pos0 = (q ^ (r16 >> 1)) << 4, pos1 = pos0 ^ 64;
+  const int offA = (wr * (TM / WR) + r16) * 128;
+  const int offW = kA + (wc * (TN / WC) + 8 * (r16 >> 2) + (r16 & 3)) * 128;
+
+  float4v acc[MI][NP][2];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int g = 0; g < NP; ++g)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) acc[i][g][h] = float4v{0.f, 0.f, 0.f, 0.f};
+
+  const int KT = p.K / 64, k0 = KT * split / p.splits, nk = KT * (split + 1) / p.splits - k0;
+#pragma unroll
+  for (int k = 0; k < NST; ++k)
+    if (k < nk) stage(smem + k * kStage, k0 + k);
+  int at = 0;
+  for (int kt = 0; kt < nk; ++kt) {
+    uint8_t* buf = smem + at;
+    at = at == (NST - 1) * kStage ? 0 : at + kStage;
+    // this step's rows have landed, the following steps' may be in flight
+    if (kt + NST <= nk) wait_rows<(NST - 1) * (IA + IW)>();
+    else if (NST > 2 && kt + 3 <= nk) wait_rows<2 * (IA + IW)>();
+    else if (kt + 2 <= nk) wait_rows<IA + IW>();
+    else wait_rows<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    uint4v a[2][MI], w[2][NP][2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+      const int pos = s ? pos1 : pos0;
+#pragma unroll
+      for (int i = 0; i < MI; ++i) a[s][i] = *reinterpret_cast<const uint4v*>(buf + offA + pos + i * 2048);
+#pragma unroll
+      for (int g = 0; g < NP; ++g)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) w[s][g][h] = *reinterpret_cast<const uint4v*>(buf + offW + pos + g * 4096 + h * 512);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();  // every wave holds the step's operands: its buffer takes the step after next
+    asm volatile("" ::: "memory");
+    if (kt + NST < nk) stage(buf, k0 + kt + NST);
+    __builtin_amdgcn_sched_barrier(0);
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int g = 0; g < NP; ++g)
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+          for (int i = 0; i < MI; ++i) acc[i][g][h] = mfma(w[s][g][h], a[s][i], acc[i][g][h]);
+    __builtin_amdgcn_s_setprio(0);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+
+  if constexpr (TM == 64)
+  if (p.splits > 1) {  // the last range to arrive adds all of them up, in their order, and writes the output
+    // (partial sums pass the caches by stores and loads of device scope: a fence per workgroup writes the whole L2 back and
+    // took 10 us and more)
+    constexpr int kAcc = MI * NP * 8;  // accumulators per lane
+    float* mine = p.part + ((size_t)t * p.splits + split) * (TM * TN) + tid;
+#pragma unroll
+    for (int e = 0; e < kAcc; ++e)
+      __hip_atomic_store(mine + e * 256, acc[e / (NP * 8)][e / 8 % NP][e / 4 % 2][e % 4], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // they have arrived
+    __syncthreads();
+    int* flag = reinterpret_cast<int*>(smem);
+    if (tid == 0) {
+      const int n = __hip_atomic_fetch_add(p.count + t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (n == p.splits - 1) __hip_atomic_store(p.count + t, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *flag = n;
+    }
+    __syncthreads();
+    if (*flag != p.splits - 1) return;
+    float sum[kAcc];
+#pragma unroll
+    for (int e = 0; e < kAcc; ++e) sum[e] = 0.f;
+    for (int s = 0; s < p.splits; ++s) {
+      const float* part = p.part + ((size_t)t * p.splits + s) * (TM * TN) + tid;
+      float x[kAcc];
+#pragma unroll
+      for (int e = 0; e < kAcc; ++e) x[e] = __hip_atomic_load(part + e * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+      for (int e = 0; e < kAcc; ++e) sum[e] += x[e];
+    }
+#pragma unroll
+    for (int e = 0; e < kAcc; ++e) acc[e / (NP * 8)][e / 8 % NP][e / 4 % 2][e % 4] = sum[e];
+  }
+
+  const int mrow = m0 + wr * (TM / WR) + r16;
+  if constexpr (EPI == EPI_SWIGLU) {  // groups 2 g: gate columns, 2 g + 1: the matching up columns
+#pragma unroll
+    for (int g = 0; g < NP / 2; ++g) {
+      const int col = (n0 + wc * (TN / WC)) / 2 + g * 32 + 8 * q;
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        float x[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = silu(acc[i][2 * g][e >> 2][e & 3]) * acc[i][2 * g + 1][e >> 2][e & 3];
+        if (mrow + 16 * i < p.M && col < p.N / 2) *reinterpret_cast<uint4v*>(p.C + (size_t)(mrow + 16 * i) * p.ldc + col) = pack8(x);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int g = 0; g < NP; ++g) {
+      const int col = n0 + wc * (TN / WC) + g * 32 + 8 * q;
+      if (col >= p.N) continue;
+      float b[8];
+      if (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) unpack8(*reinterpret_cast<const uint4v*>(p.R + col), b);
+      uint4v rv[MI];
+      if (EPI == EPI_RESIDUAL) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+          rv[i] = *reinterpret_cast<const uint4v*>(p.R + (size_t)min(mrow + 16 * i, p.M - 1) * p.ldc + col);
+      }
+#pragma unroll
+      for (int i = 0; i < MI; ++i) {
+        float x[8];
+        if (EPI == EPI_RESIDUAL) unpack8(rv[i], b);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          x[e] = acc[i][g][e >> 2][e & 3];
+          if (EPI != EPI_PLAIN) x[e] += b[e];
+          if (EPI == EPI_BIAS_GELU) x[e] = gelu_erf(x[e]);
+        }
+        if (mrow + 16 * i < p.M) *reinterpret_cast<uint4v*>(p.C + (size_t)(mrow + 16 * i) * p.ldc + col) = pack8(x);
+      }
+    }
+  }
+}
+
+template <int EPI, int TM, int TN, int NST>
+int launch(Params p, hipStream_t s) {
+  constexpr int kLds = NST * (TM + TN) * 128;
+  static const hipError_t attr =
+      hipFuncSetAttribute((const void*)gemm2w_kernel<EPI, TM, TN, NST>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+  (void)attr;
+  p.tiles_m = (p.M + TM - 1) / TM;
+  p.tiles_n = (p.N + TN - 1) / TN;
+  gemm2w_kernel<EPI, TM, TN, NST><<<p.tiles_m * p.tiles_n * p.splits, 256, kLds, s>>>(p);
+  return (int)hipGetLastError();
+}
+
+}  // namespace g2w
+}  // namespace lwc
+
+// epi 0: C = A W^T; 1: C = A W^T + R (R may be C); 2: C[:, :N/2] = silu(gate) * up over 32-row interleaved W (N % 64 == 0);
+// 3: C = A W^T + bias (R = bias [N]); 4: C = gelu(A W^T + bias) (exact erf GELU).
+// tile 0: 128 x 128, 1: 192 x 128, 2: 128 x 192 (not epi 2), 3: 64 x 64, there with splits K ranges per tile (part: tiles x
+// splits x 4096 floats, count: tiles ints, zero on the first call; the kernel leaves them zero).
+// Requires K % 64 == 0, K / 64 >= splits, N % 8 == 0 and 16-byte rows and pointers.
+// The tile and the K ranges of a call (max_splits: what the caller's workspace holds, in 64 x 64 partial tiles).
+// 64 x 64 up to 512 tiles (two workgroups per CU) and for any call of up to 64 rows.  Measured (us, 64 x 64 against 128 x 128):
+// 512 rows x 4096 x K 1024 9.9 / 14.8, 512 x 4096 x 4096 35.5 / 42.8, 1000 x 3072 x 1024 (768 tiles) 14.9 / 13.8, 1000 x 4096 x
+// 4096 (1024 tiles) 62 / 44.  Its K ranges: as many as fit one workgroup per CU, none below 16 steps.  Measured, one / two /
+// four / eight ranges: 61 x 4096 x 4096 21.9 / 15.6 / 12.9 / 15.5, 61 x 6144 x 4096 22.2 / 17.0 / 17.6 / 21.3, 61 x 4096 x 14336
+// 70 / 42 / 28 / 32, 128 x 4096 x 4096 22.1 / 16.1 / 17.3 / 25.4, 256 x 1024 x 4096 21.1 / 14.9 / 12.2 / 13.7, 61 x 3072 x 1024
+// 7.4 / 7.9 / 8.2.
+// Larger ones: the tile that takes the least time in whole rounds of two workgroups per CU, the larger of two that tie.
+// Measured (128 x 128 against 128 x 192): 3600 x 2304 x 768 (522 and 348 tiles) 25.3 / 20.3, 3600 x 4096 x 1024 (928 and
+// 638) 40.8 / 46.7, 7155 x 3072 x 768 (1344 and 896) 51.5 / 48.1.
+extern "C" void lwc_gemm2w_plan(int M, int N, int K, int epi, long long max_splits, int* tile, int* splits) {
+  auto tiles = [&](int tm, int tn) { return ((long long)M + tm - 1) / tm * ((N + tn - 1) / tn); };
+  *splits = 1;
+  const long long small = tiles(64, 64);
+  if (M <= 64 || small <= 512) {
+    *tile = 3;
+    const long long s = std::min(std::min(256 / std::max(small, 1LL), (long long)K / 1024), max_splits / std::max(small, 1LL));
+    *splits = (int)std::max(1LL, s);
+    return;
+  }
+  const long long square = (tiles(128, 128) + 511) / 512 * (128 * 128);
+  const int wide = epi != lwc::g2w::EPI_SWIGLU ? 2 : 1;
+  const long long rect = ((wide == 2 ? tiles(128, 192) : tiles(192, 128)) + 511) / 512 * (128 * 192);
+  *tile = rect <= square ? wide : 0;
+}
+
+extern "C" int lwc_gemm2w(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda, int ldc, int epi,
+                          int tile, int splits, float* part, int* count, hipStream_t s) {
+  using namespace lwc::g2w;
+  if (K % 64 != 0 || K < 64 || N % 8 != 0 || lda % 8 != 0 || ldc % 8 != 0 || tile < 0 || tile > 3) return -1;
+  if (192LL * (lda + K) * 2 >= (1LL << 31)) return -1;  // 32-bit buffer offsets in a tile
+  if (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C | (uintptr_t)R) & 15) return -1;
+  if (splits < 1 || splits > K / 64 || (splits > 1 && (tile != 3 || part == nullptr || count == nullptr))) return -1;
+  if (epi == EPI_SWIGLU && (N % 64 != 0 || tile == 2)) return -1;
+  if (epi != EPI_PLAIN && epi != EPI_SWIGLU && R == nullptr) return -1;
+  if (M == 0 || N == 0) return 0;
+  if (((long long)M + 63) / 64 * ((N + 63) / 64) * splits >= (1LL << 31)) return -1;
+  const Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc, 0, 0,
+                 splits, part, count};
+#define LWC_G2W(E)                                                                     \
+  case E:                                                                              \
+    if constexpr (E != EPI_SWIGLU)                                                     \
+      if (tile == 2) return launch<E, 128, 192, 2>(p, s);                              \
+    return tile == 3 ? launch<E, 64, 64, 4>(p, s) : tile == 1 ? launch<E, 192, 128, 2>(p, s) : launch<E, 128, 128, 2>(p, s);
+  switch (epi) {
+    LWC_G2W(EPI_PLAIN)
+    LWC_G2W(EPI_RESIDUAL)
+    LWC_G2W(EPI_SWIGLU)
+    LWC_G2W(EPI_BIAS)
+    LWC_G2W(EPI_BIAS_GELU)
+  }
+#undef LWC_G2W
+  return -1;
+}

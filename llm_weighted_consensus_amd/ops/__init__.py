@@ -432,6 +432,35 @@ def gemm8p(A: torch.Tensor, W: torch.Tensor, residual: Optional[torch.Tensor] = 
     return out
 
 
+def gemm2w(A: torch.Tensor, W: torch.Tensor, residual: Optional[torch.Tensor] = None,
+           out: Optional[torch.Tensor] = None, swiglu: bool = False, bias: Optional[torch.Tensor] = None,
+           gelu: bool = False, tile: int = -1, splits: int = 1, ws=None) -> torch.Tensor:
+    """MFMA GEMM in tiles for two workgroups per CU (K6, csrc/kernels/gemm2w.hip): the calls and epilogues of
+    :func:`gemm8p`, rows and pointers at 16 bytes (:func:`gemm2w_ok`).  ``tile`` 0: 128 x 128, 1: 192 x 128, 2: 128 x 192 (not
+    SwiGLU), 3: 64 x 64, there with ``splits`` K ranges per tile over the workspace ``ws`` (gemm8p's; default: the one of
+    the current stream); -1: by the sizes."""
+    if (swiglu and residual is not None) or (bias is not None and (swiglu or residual is not None)):
+        raise ValueError("gemm2w: swiglu, residual and bias do not combine")
+    if gelu and bias is None:
+        raise ValueError("gemm2w: gelu needs a bias")
+    if out is None:
+        out = torch.empty(A.shape[0], W.shape[0] // 2 if swiglu else W.shape[0], dtype=torch.bfloat16, device=A.device)
+    epi = 2 if swiglu else 1 if residual is not None else 0 if bias is None else 4 if gelu else 3
+    if ws is None and (tile < 0 or splits > 1):
+        ws = _G8_WS.get((A.device.index, torch.cuda.current_stream(A.device).cuda_stream))
+        if ws is None and not torch.cuda.is_current_stream_capturing():
+            ws = gemm8p_workspace(A.device)
+    part, count = ws if ws is not None else (None, None)   # (none under capture: unsplit)
+    kernels().gemm2w(A, W, out, bias if bias is not None else residual, epi, int(tile), int(splits), part, count)
+    return out
+
+
+def gemm2w_ok(N: int, K: int, *operands: Optional[torch.Tensor], swiglu: bool = False) -> bool:
+    """Whether :func:`gemm2w` takes a call: its sizes, and 16-byte rows and pointers of every operand."""
+    return K % 64 == 0 and N % (64 if swiglu else 8) == 0 and all(
+        t is None or (t.data_ptr() % 16 == 0 and (t.dim() == 1 or (t.stride(1) == 1 and t.stride(0) % 8 == 0))) for t in operands)
+
+
 def skinny_gemm(A: torch.Tensor, W: torch.Tensor, residual: Optional[torch.Tensor] = None,
                 out: Optional[torch.Tensor] = None, swiglu: bool = False, bias: Optional[torch.Tensor] = None,
                 gelu: bool = False) -> torch.Tensor:

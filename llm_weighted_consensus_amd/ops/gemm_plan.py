@@ -12,6 +12,9 @@ Backends computing ``A . W^T`` for the dense projections:
   transposed accumulator layout (``profiles/gemm4w_stamps_r5.md``).
 * ``gv``     — the skinny weight-stream GEMM for few rows (M <= 256; plain, residual, SwiGLU and bias (+ GELU)
   epilogues; ``csrc/kernels/skinny.hip``): the serving path's small decode steps, the encoders' few short texts.
+* ``g2``     — tiles for two workgroups per CU (``csrc/kernels/gemm2w.hip``), 64 x 64 with K ranges up to 192 x 128 by the
+  sizes: up to 8192 rows (above, the 256 x 256 tiles of ``g8`` and of the library are always faster: 65536 rows x 3072 x
+  1024 418 us against 387 and 322), from a few dozen rows on.
 * ``g4s``    — gemm4w VAR 64 with split-K (``ops.split_plan``): shapes whose tiles leave CUs idle (the
   serving path's mid-size row counts: o / down at M = 2048 are 128 tiles for 256 CUs) run every tile as 2-4
   K-range units, a ragged last round (lm_head) splits only that round's tiles.
@@ -34,10 +37,11 @@ from typing import Dict, Optional, Tuple
 import torch
 import torch.nn.functional as F
 
-from . import GEMM4W, gemm4w, gemm8p, silu_mul, skinny_gemm, skinny_ok, split_plan
+from . import GEMM4W, gemm2w, gemm2w_ok, gemm4w, gemm8p, silu_mul, skinny_gemm, skinny_ok, split_plan
 
 MODE = os.environ.get("LWC_GEMM", "auto")
-BACKENDS = ("blas", "g8", "g4", "g4n192", "g4p", "gv", "g4s")
+BACKENDS = ("blas", "g8", "g4", "g4n192", "g4p", "gv", "g2", "g4s")
+G2_ROWS = 8192
 # a hand-written core is chosen when it is at least as fast as the library in the isolated timings (no
 # bias either way: the decode step's plan is then settled by the engine's in-step A/B of whole captured steps,
 # engine.LLMEngine._step_ab, which sees the step's clock and cache state)
@@ -83,6 +87,8 @@ def _own_ok(b: str, x: torch.Tensor, N: int, K: int, epi: str) -> bool:
         return False
     if b == "gv":
         return SKINNY and skinny_ok(x.shape[0], N, K, swiglu=epi == "swiglu")
+    if b == "g2":
+        return x.is_cuda and x.shape[0] <= G2_ROWS and gemm2w_ok(N, K, x, swiglu=epi == "swiglu")
     if b == "g4s":  # VAR 64, split-K wherever split_plan splits this M (else unsplit: a bucket's M varies)
         return x.is_cuda
     return not (b == "g4n192" and epi == "swiglu")
@@ -93,6 +99,8 @@ def _own(b: str, x: torch.Tensor, w: torch.Tensor, ws=None, **kw) -> torch.Tenso
         return gemm8p(x, w, ws=ws, **kw)
     if b == "gv":
         return skinny_gemm(x, w, **kw)
+    if b == "g2":
+        return gemm2w(x, w, ws=ws, **kw)
     if b == "g4s":
         s_, f_ = split_plan(x.shape[0], w.shape[0], x.shape[1])
         return gemm4w(x, w, var=64, splits=s_, split_from=f_, **kw)
@@ -117,7 +125,7 @@ def linear_add_(x: torch.Tensor, w: torch.Tensor, acc: torch.Tensor, ws=None) ->
     M, K = x.shape
     N = w.shape[0]
     b = choice(M, N, K, "residual")
-    if _own_ok(b, x, N, K, "residual") and acc.is_contiguous():
+    if _own_ok(b, x, N, K, "residual") and acc.is_contiguous() and (b != "g2" or acc.data_ptr() % 16 == 0):
         return _own(b, x, w, ws, residual=acc, out=acc)
     return acc.addmm_(x, w.t())
 
@@ -151,30 +159,38 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = 
     N = w.shape[0]
     epi = "bias_gelu" if gelu else "bias"
     key = (_m_bucket(M), N, K, epi)
-    c = MODE if MODE in ("blas", "g8", "g4", "g4p", "gv") else _CHOICE.get(key)
-    # gemm8p addresses A through one 32-bit buffer range (operands of 2 GiB or more take the other backends);
-    # gemm4w runs such an A as row blocks
-    ok = _g8_ok(N, K, epi) and x.stride(1) == 1 and x.is_cuda
-    small_a = M * x.stride(0) * 2 < (1 << 31)
-    runs = {"blas": ((lambda: torch._addmm_activation(b, x, w.t(), use_gelu=True)) if gelu
-                     else (lambda: F.linear(x, w, b)))}
-    if GEMM4W:
-        runs.update({"g4": lambda: gemm4w(x, w, bias=b, gelu=gelu), "g4p": lambda: gemm4w(x, w, bias=b, gelu=gelu, var=64)})
-    if small_a:
-        runs["g8"] = lambda: gemm8p(x, w, bias=b, gelu=gelu, ws=ws)
-    if ok and _own_ok("gv", x, N, K, epi):
-        runs["gv"] = lambda: skinny_gemm(x, w, bias=b, gelu=gelu)
+    c = MODE if MODE in ENC_BACKENDS else _CHOICE.get(key)
+    blas = (lambda: torch._addmm_activation(b, x, w.t(), use_gelu=True)) if gelu else (lambda: F.linear(x, w, b))
     if c is None:
-        if not ok or torch.cuda.is_current_stream_capturing():
+        if not (x.is_cuda and x.stride(1) == 1 and _g8_ok(N, K, epi)) or torch.cuda.is_current_stream_capturing():
             c = "blas"
         else:
-            t = {name: _time(fn, iters=2, rounds=3) for name, fn in runs.items()}
-            TIMINGS[key] = t
-            own = min((n for n in t if n != "blas"), key=lambda n: t[n], default="blas")
-            c = own if t[own] <= t["blas"] * (1 + OWN_MARGIN) else "blas"
+            runs = {"blas": blas}
+            runs.update({n: (lambda n=n: _own(n, x, w, ws, bias=b, gelu=gelu)) for n in ENC_BACKENDS[1:] if _enc_ok(n, x, w, epi, b)})
+            c = _pick(key, runs)
         _CHOICE[key] = c
-    # (a choice made for the token bucket at a smaller A may name gemm8p, which a 2 GiB A cannot take)
-    return runs[c]() if c != "blas" and ok and c in runs else runs["blas"]()
+    # (a choice made for the token bucket may name a core that does not take this call: a 2 GiB A, an odd alignment)
+    return _own(c, x, w, ws, bias=b, gelu=gelu) if c != "blas" and _enc_ok(c, x, w, epi, b) else blas()
+
+
+ENC_BACKENDS = ("blas", "g4", "g4p", "g8", "gv", "g2")
+
+
+def _enc_ok(n: str, x: torch.Tensor, w: torch.Tensor, epi: str, other: torch.Tensor) -> bool:
+    """Whether core ``n`` takes an encoder projection (``other``: its bias, or the stream it adds into)."""
+    N, K = w.shape
+    if not x.is_cuda or not _own_ok(n, x, N, K, epi):
+        return False
+    if n == "g8":  # addresses A through one 32-bit buffer range (gemm4w runs an A of 2 GiB or more as row blocks)
+        return x.shape[0] * x.stride(0) * 2 < (1 << 31)
+    return n != "g2" or gemm2w_ok(N, K, w, other)
+
+
+def _pick(key, runs) -> str:
+    t = {name: _time(fn, iters=2, rounds=3) for name, fn in runs.items()}
+    TIMINGS[key] = t
+    own = min((n for n in t if n != "blas"), key=lambda n: t[n], default="blas")
+    return own if t[own] <= t["blas"] * (1 + OWN_MARGIN) else "blas"
 
 
 def linear_residual_(x: torch.Tensor, w: torch.Tensor, acc: torch.Tensor, ws=None) -> torch.Tensor:
@@ -185,34 +201,20 @@ def linear_residual_(x: torch.Tensor, w: torch.Tensor, acc: torch.Tensor, ws=Non
     M, K = x.shape
     N = w.shape[0]
     key = (_m_bucket(M), N, K, "enc_residual")
-    c = MODE if MODE in ("blas", "g8", "g4", "g4p", "gv") else _CHOICE.get(key)
-    ok = _g8_ok(N, K, "residual") and x.stride(1) == 1 and x.is_cuda and acc.is_contiguous()
-    small_a = M * x.stride(0) * 2 < (1 << 31)
-
-    def runs_on(a):
-        r = {"blas": lambda: a.addmm_(x, w.t())}
-        if GEMM4W:
-            r.update({"g4": lambda: gemm4w(x, w, residual=a, out=a), "g4p": lambda: gemm4w(x, w, residual=a, out=a, var=64)})
-        if small_a:
-            r["g8"] = lambda: gemm8p(x, w, residual=a, out=a, ws=ws)
-        if ok and _own_ok("gv", x, N, K, "residual"):
-            r["gv"] = lambda: skinny_gemm(x, w, residual=a, out=a)
-        return r
-
+    c = MODE if MODE in ENC_BACKENDS else _CHOICE.get(key)
+    takes = lambda n: acc.is_contiguous() and _enc_ok(n, x, w, "residual", acc)
     if c is None:
-        if not ok or torch.cuda.is_current_stream_capturing():
+        if not (x.is_cuda and x.stride(1) == 1 and _g8_ok(N, K, "residual") and acc.is_contiguous()) or \
+                torch.cuda.is_current_stream_capturing():
             c = "blas"
         else:
-            scratch = acc.clone()  # the timing runs add into a copy, never into the stream
-            t = {name: _time(fn, iters=2, rounds=3) for name, fn in runs_on(scratch).items()}
-            del scratch
-            TIMINGS[key] = t
-            own = min((n for n in t if n != "blas"), key=lambda n: t[n], default="blas")
-            c = own if t[own] <= t["blas"] * (1 + OWN_MARGIN) else "blas"
+            a = acc.clone()  # the timing runs add into a copy, never into the stream
+            runs = {"blas": lambda: a.addmm_(x, w.t())}
+            runs.update({n: (lambda n=n: _own(n, x, w, ws, residual=a, out=a)) for n in ENC_BACKENDS[1:] if takes(n)})
+            c = _pick(key, runs)
+            del a, runs
         _CHOICE[key] = c
-    runs = runs_on(acc)
-    runs[c if c != "blas" and ok and c in runs else "blas"]()
-    return acc
+    return _own(c, x, w, ws, residual=acc, out=acc) if c != "blas" and takes(c) else acc.addmm_(x, w.t())
 
 
 def _time(fn, iters: int = 5, rounds: int = 3) -> float:

@@ -1568,6 +1568,50 @@ def test_skinny_gemm_any_k(gpu, M, N, K, epi):
     torch.testing.assert_close(out.double(), ref, rtol=2 ** -8, atol=2e-5)
 
 
+@pytest.mark.parametrize("tile,splits", [(0, 1), (1, 1), (2, 1), (3, 1), (3, 5), (-1, 0)])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 64), (64, 8, 128), (129, 200, 320), (192, 384, 192), (515, 704, 1024), (61, 1024, 4096),
+                                   (1500, 2304, 448)])
+@pytest.mark.parametrize("epi", ["plain", "residual", "bias", "gelu", "swiglu"])
+def test_gemm2w(gpu, M, N, K, epi, tile, splits):
+    """Tiles with rows and columns to spare, one K step to many, K ranges of unequal length (twice over one workspace, whose
+    counters go back to zero), the sizes' own choice; A and C as columns of wider matrices; vs fp64 of the same operands.
+    Bound: one bf16 rounding (2^-9, doubled), fp32 sums of K terms of about 1 / sqrt(K), for GELU its erf polynomial's 1.5e-7,
+    for SwiGLU the fast exp and reciprocal (2^-20 of values up to 16)."""
+    from llm_weighted_consensus_amd import ops
+
+    if epi == "swiglu" and (N % 64 or tile == 2):
+        pytest.skip("not a call the tile takes")
+    torch.manual_seed(M + N + K)
+    A = torch.randn(M, K + 64, device=gpu).to(torch.bfloat16)
+    A[:, K:] = float("nan")   # columns past K are never read
+    A = A[:, :K]
+    W = (torch.randn(N, K, device=gpu) * K ** -0.5).to(torch.bfloat16)
+    R = torch.randn(M, N, device=gpu).to(torch.bfloat16)
+    b = torch.randn(N, device=gpu).to(torch.bfloat16)
+    ref = A.double() @ W.double().t()
+    ws = ops.new_gemm8p_workspace(gpu)
+    kw = dict(tile=tile, splits=max(1, min(splits, K // 64)) if M < 1000 else 1, ws=ws)   # (256 counters: up to 256 tiles)
+    for again in range(2):
+        if epi == "residual":
+            want, C = ref + R.double(), R.clone()
+            out = ops.gemm2w(A, W, residual=C, out=C, **kw)
+            assert out is C
+        elif epi == "plain":
+            wide = torch.full((M + 1, N + 8), float("nan"), dtype=torch.bfloat16, device=gpu)
+            want, out = ref, ops.gemm2w(A, W, out=wide[:M, :N], **kw)
+            assert torch.isnan(wide[M:]).all() and torch.isnan(wide[:, N:]).all()
+        elif epi == "swiglu":
+            v = ref.view(M, N // 64, 2, 32)
+            want = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+            out = ops.gemm2w(A, W, swiglu=True, **kw)
+        else:
+            want = ref + b.double()
+            want = torch.nn.functional.gelu(want) if epi == "gelu" else want
+            out = ops.gemm2w(A, W, bias=b, gelu=epi == "gelu", **kw)
+        torch.testing.assert_close(out.double(), want, rtol=2 ** -8, atol=3e-5)
+        assert not ws[1].any()
+
+
 @pytest.mark.parametrize("M", [1, 7, 16, 33, 64])
 @pytest.mark.parametrize("N,K", [(4096, 4096), (6144, 4096), (4096, 14336), (1040, 2048)])
 @pytest.mark.parametrize("res", [False, True])
