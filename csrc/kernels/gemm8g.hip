@@ -415,6 +415,14 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
 }  // namespace g8g
 }  // namespace lwc
 
+extern "C" int lwc_gemm2g_fp8(const void*, const void*, void*, const int*, const int*, const float*, const float*, int, int, int, int,
+                              int, int, int, int, const void*, void*, int, hipStream_t);
+
+// rows per group up to which the weights bound a grouped call and gemm2g.hip takes it.  us, 8-phase / gemm2g: SwiGLU to MX
+// [28672, 4096] x 8 at 128 rows a group 270 / 217, 175 rows 272 / 237, 256 rows 293 / 344; from MX [4096, 14336] x 8 at 128 rows
+// 155 / 115, 175 rows (a group of 219 needs a second tile, 288 for 256 CUs) 161 / 188
+constexpr int kSmallRows = 144, kSmallRowsSwiglu = 176;
+
 // Grouped fp8 GEMM on the 8-phase schedule.  Requires K % 128 == 0, N % 8 == 0, lda / ldc % 16 == 0 (bytes
 // / elements: 16-byte rows), rows_a * lda < 2^31 and 256 * K < 2^31 (32-bit buffer offsets); max_slots >=
 // sum_g ceil(M_g / 256) (ceil(rows / 256) + G always is).  row_off == null: dense, G = 1, rows [0, rows_c).
@@ -434,6 +442,9 @@ extern "C" int lwc_gemm8g_fp8(const void* A, const void* W, void* C, const int* 
   if (mode == 2 && (N % 256 != 0 || !mx_out || s_rows < rows_c || ldc % 16 != 0)) return -1;
   if (a_mx && (mode != 0 || a_rows || s_rows < rows_a || (long long)(K / 128) * s_rows * 4 >= (1LL << 31))) return -1;
   if (max_slots <= 0) return 0;
+  if (row_off && rows_c > 0 && rows_c <= (swiglu ? kSmallRowsSwiglu : kSmallRows) * (long long)G)
+    return lwc_gemm2g_fp8(A, W, C, row_off, a_rows, a_scale, w_scale, G, N, K, lda, ldc, rows_a, rows_c, a_mx ? 3 : mode, a_mx, mx_out,
+                          s_rows, s);
   static bool attr = false;
   if (!attr) {
     (void)hipFuncSetAttribute((const void*)gemm8g_kernel<kPlain>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsB);

@@ -1195,6 +1195,56 @@ def test_grouped_fp8_mx_a_matches_reference(gpu, sizes):
             assert ((out[o[g]:o[g + 1]].float() - ref_).norm() / ref_.norm()).item() < 1e-2
 
 
+@pytest.mark.parametrize("sizes", [[1, 0, 2, 40], [64, 65, 0, 16], [128, 129, 90, 17], [192, 193, 100, 60]])
+@pytest.mark.parametrize("N,K", [(128, 128), (256, 640), (11264, 256)])
+@pytest.mark.parametrize("mode", ["plain", "swiglu", "mx_out", "mx_a"])
+def test_grouped_fp8_of_few_rows(gpu, sizes, N, K, mode):
+    """Groups of few rows (gemm2g.hip): row tiles of 64, 128 and 192 with rows to spare and beyond, fewer K steps than the
+    stages hold and more, few tiles and many; vs fp64 of the dequantised operands.  Bound: the bf16 result's rounding (2^-8
+    relative with its double rounding), the matrix core's sum of a 128-term slice (2^-13 of the row's largest output), for
+    e4m3 outputs half its last bit (2^-4 of the block's largest)."""
+    from llm_weighted_consensus_amd import ops
+
+    if mode == "mx_out" and N % 256:
+        pytest.skip("MX output needs whole slices")
+    torch.manual_seed(sum(sizes) + N)
+    G, rows = len(sizes), sum(sizes)
+    off = torch.tensor([0] + list(np.cumsum(sizes)), dtype=torch.int32, device=gpu)
+    Aq = (torch.randn(rows + 3, K, device=gpu) * 60).clamp(-448, 448).to(torch.float8_e4m3fn)
+    Wq = (torch.randn(G, N, K, device=gpu) * 60).clamp(-448, 448).to(torch.float8_e4m3fn)
+    ws = torch.rand(G, N, device=gpu) * K ** -0.5 / 60 + 1e-4
+    xs = torch.rand(rows + 3, device=gpu) / 60 + 1e-3
+    a_rows = torch.randperm(rows + 3, device=gpu)[:rows].to(torch.int32)
+    slots = -(-rows // 256) + G
+    out = torch.full((rows + 1, N // (1 if mode in ("plain", "mx_a") else 2)), 7.0, device=gpu).to(torch.float8_e4m3fn if mode == "mx_out" else torch.bfloat16)
+    C, mx = out[:rows], None
+    if mode == "mx_a":
+        mx = torch.randint(124, 131, (K // 128, rows, 4), dtype=torch.uint8, device=gpu)
+        ops.kernels().gemm8g_fp8(Aq[:rows], Wq, C, off, slots, None, None, ws, 0, mx, None)
+        A = Aq[:rows].double() * _mx_scale_map(mx, K).double()
+    else:
+        if mode == "mx_out":
+            mx = torch.zeros(N // 256, rows, 4, dtype=torch.uint8, device=gpu)
+        ops.kernels().gemm8g_fp8(Aq, Wq, C, off, slots, a_rows, xs, ws, {"plain": 0, "swiglu": 1, "mx_out": 2}[mode], None, mx)
+        A = (Aq.double() * xs.double()[:, None])[a_rows.long()]
+    assert (out[rows:].float() == 7).all()
+    got = C.double() * _mx_scale_map(mx, N // 2).double() if mode == "mx_out" else C.double()
+    o = off.tolist()
+    for g in range(G):
+        y = A[o[g]:o[g + 1]] @ (Wq[g].double() * ws[g].double()[:, None]).t()
+        if not len(y):
+            continue
+        slack = 2 ** -13 * y.abs().amax(1, keepdim=True)
+        if mode in ("swiglu", "mx_out"):
+            v = y.view(len(y), -1, 2, 32)
+            y = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(len(y), -1)
+            slack = slack * v.abs().amax((1, 2, 3))[:, None] * 2
+        bound = 2 ** -8 * y.abs() + slack
+        if mode == "mx_out":
+            bound = bound + (2 ** -4 * y.abs().view(len(y), -1, 32).amax(-1, keepdim=True)).expand(-1, -1, 32).reshape(y.shape)
+        assert ((got[o[g]:o[g + 1]] - y).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("sizes", [[300, 0, 77, 520], [100, 200, 129, 128]])
 @pytest.mark.parametrize("gather", [False, True])
 def test_grouped_fp8_swiglu_mx_matches_reference(gpu, gather, sizes):
