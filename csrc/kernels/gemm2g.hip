@@ -9,7 +9,7 @@
 // Measured, 8 experts, us, 8-phase kernel -> here ([28672, 4096] SwiGLU to MX, [4096, 14336] from MX; 154 and 77 at the rate of
 // a plain read): 4 rows an expert 257 -> 182, 144 -> 81; 32 rows 259 -> 189, 145 -> 84; 64 rows 264 -> 200, 150 -> 90; 128 rows
 // 270 -> 217, 155 -> 115.  In steps in flight: one workgroup of six (four) steps for the first GEMM 189 to 257, two workgroups of
-// three (two) steps for the second 123 to 175.
+// three (two) steps for the second 123 to 175.  Dense calls of few tiles likewise: 512 rows x 4096 x K 4096 from MX 45 -> 21.
 #include "common.h"
 
 namespace lwc {
@@ -27,7 +27,7 @@ struct Params {
   const int* a_rows;
   const float* a_scale;
   const float* w_scale;
-  int G, N, K, lda, ldc, rows_a;
+  int G, N, K, lda, ldc, rows_a, rows;
   int slots, n_tiles;
   const uint8_t* a_mx;
   uint8_t* mx_out;
@@ -81,7 +81,7 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
   if (ntile >= p.n_tiles) return;
   int slot = local / nj, g = 0, m_begin = 0, m_end = 0;
   for (; g < p.G; ++g) {
-    const int r0 = p.row_off[g], r1 = p.row_off[g + 1], nt = (r1 - r0 + TM - 1) / TM;
+    const int r0 = p.row_off ? p.row_off[g] : 0, r1 = p.row_off ? p.row_off[g + 1] : p.rows, nt = (r1 - r0 + TM - 1) / TM;
     if (slot < nt) {
       m_begin = r0 + slot * TM;
       m_end = min(r1, m_begin + TM);
@@ -245,17 +245,21 @@ int launch(Params p, int rows, hipStream_t s) {
 }  // namespace g2g
 }  // namespace lwc
 
-// The operands of lwc_gemm8g_fp8 (checked there) with a row table; mode 3: A carries MX scales.  rows: all groups' rows.
+// The operands of lwc_gemm8g_fp8 (checked there), row_off null for a dense call; mode 3: A carries MX scales.  rows: all groups' rows.
 extern "C" int lwc_gemm2g_fp8(const void* A, const void* W, void* C, const int* row_off, const int* a_rows,
                               const float* a_scale, const float* w_scale, int G, int N, int K, int lda, int ldc, int rows_a,
                               int rows, int mode, const void* a_mx, void* mx_out, int s_rows, hipStream_t s) {
   using namespace lwc::g2g;
-  if (!row_off || K % 128 != 0 || K < 128 || N % 8 != 0 || rows <= 0) return -1;
+  if ((!row_off && G != 1) || K % 128 != 0 || K < 128 || N % 8 != 0 || rows <= 0) return -1;
   const Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, a_scale, w_scale, G, N, K, lda, ldc, rows_a,
-                 0, 0, (const uint8_t*)a_mx, (uint8_t*)mx_out, s_rows};
+                 rows, 0, 0, (const uint8_t*)a_mx, (uint8_t*)mx_out, s_rows};
   // The tile that most groups' rows fit, with room for an uneven routing (a second tile reads the weights again).
-  const int per = (rows + G - 1) / G, tm = per <= 44 ? 64 : per <= 104 ? 128 : 192;
-  const bool deep = (long long)((N + 127) / 128) * G * ((per + tm - 1) / tm) <= 320;  // (256 CUs)
+  // Dense (no table): whole tiles of 64 rows while they give a CU two workgroups at most, then of 128, then of 192.
+  const int per = (rows + G - 1) / G;
+  const long long nt = (N + 127) / 128;
+  int tm = per <= 44 ? 64 : per <= 104 ? 128 : 192;
+  if (!row_off) tm = nt * ((rows + 63) / 64) <= 512 ? 64 : nt * ((rows + 127) / 128) <= 512 ? 128 : 192;
+  const bool deep = nt * G * ((per + tm - 1) / tm) <= 320;  // (256 CUs)
 #define LWC_G2G(M, D64, D128, D192)                                                                                       \
   case M:                                                                                                                 \
     if (deep) return tm == 64 ? launch<M, 64, D64>(p, rows, s) : tm == 128 ? launch<M, 128, D128>(p, rows, s) : launch<M, 192, D192>(p, rows, s); \

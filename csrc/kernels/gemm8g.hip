@@ -422,6 +422,9 @@ extern "C" int lwc_gemm2g_fp8(const void*, const void*, void*, const int*, const
 // [28672, 4096] x 8 at 128 rows a group 270 / 217, 175 rows 272 / 237, 256 rows 293 / 344; from MX [4096, 14336] x 8 at 128 rows
 // 155 / 115, 175 rows (a group of 219 needs a second tile, 288 for 256 CUs) 161 / 188
 constexpr int kSmallRows = 144, kSmallRowsSwiglu = 176;
+// and the dense calls: up to this many 256 x 256 tiles.  us, 8-phase / gemm2g, K 4096: 512 rows x 4096 (32 tiles) 45 / 21, 2048 x
+// 4096 (128) 48 / 34, 256 x 28672 SwiGLU to MX (112) 51 / 43, 2048 x 6144 (192) 49 / 66, 512 x 28672 (224) 61 / 73
+constexpr long long kSmallTiles = 128;
 
 // Grouped fp8 GEMM on the 8-phase schedule.  Requires K % 128 == 0, N % 8 == 0, lda / ldc % 16 == 0 (bytes
 // / elements: 16-byte rows), rows_a * lda < 2^31 and 256 * K < 2^31 (32-bit buffer offsets); max_slots >=
@@ -442,7 +445,9 @@ extern "C" int lwc_gemm8g_fp8(const void* A, const void* W, void* C, const int* 
   if (mode == 2 && (N % 256 != 0 || !mx_out || s_rows < rows_c || ldc % 16 != 0)) return -1;
   if (a_mx && (mode != 0 || a_rows || s_rows < rows_a || (long long)(K / 128) * s_rows * 4 >= (1LL << 31))) return -1;
   if (max_slots <= 0) return 0;
-  if (row_off && rows_c > 0 && rows_c <= (swiglu ? kSmallRowsSwiglu : kSmallRows) * (long long)G)
+  const bool small = row_off ? rows_c <= (swiglu ? kSmallRowsSwiglu : kSmallRows) * (long long)G
+                             : (long long)((rows_c + 255) / 256) * ((N + 255) / 256) <= kSmallTiles;
+  if (small && rows_c > 0)
     return lwc_gemm2g_fp8(A, W, C, row_off, a_rows, a_scale, w_scale, G, N, K, lda, ldc, rows_a, rows_c, a_mx ? 3 : mode, a_mx, mx_out,
                           s_rows, s);
   static bool attr = false;

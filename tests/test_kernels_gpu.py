@@ -1195,7 +1195,9 @@ def test_grouped_fp8_mx_a_matches_reference(gpu, sizes):
             assert ((out[o[g]:o[g + 1]].float() - ref_).norm() / ref_.norm()).item() < 1e-2
 
 
-@pytest.mark.parametrize("sizes", [[1, 0, 2, 40], [64, 65, 0, 16], [128, 129, 90, 17], [192, 193, 100, 60]])
+@pytest.mark.parametrize("sizes", [[1, 0, 2, 40], [64, 65, 0, 16], [128, 129, 90, 17], [192, 193, 100, 60],
+                                   # (one group: a dense call without a table)
+                                   [3], [64], [200], [1000]])
 @pytest.mark.parametrize("N,K", [(128, 128), (256, 640), (11264, 256)])
 @pytest.mark.parametrize("mode", ["plain", "swiglu", "mx_out", "mx_a"])
 def test_grouped_fp8_of_few_rows(gpu, sizes, N, K, mode):
@@ -1214,19 +1216,21 @@ def test_grouped_fp8_of_few_rows(gpu, sizes, N, K, mode):
     Wq = (torch.randn(G, N, K, device=gpu) * 60).clamp(-448, 448).to(torch.float8_e4m3fn)
     ws = torch.rand(G, N, device=gpu) * K ** -0.5 / 60 + 1e-4
     xs = torch.rand(rows + 3, device=gpu) / 60 + 1e-3
-    a_rows = torch.randperm(rows + 3, device=gpu)[:rows].to(torch.int32)
-    slots = -(-rows // 256) + G
+    a_rows = torch.randperm(rows + 3, device=gpu)[:rows].to(torch.int32) if G > 1 else None
+    slots = -(-rows // 256) + (G if G > 1 else 0)
+    ro = off if G > 1 else None
     out = torch.full((rows + 1, N // (1 if mode in ("plain", "mx_a") else 2)), 7.0, device=gpu).to(torch.float8_e4m3fn if mode == "mx_out" else torch.bfloat16)
     C, mx = out[:rows], None
     if mode == "mx_a":
         mx = torch.randint(124, 131, (K // 128, rows, 4), dtype=torch.uint8, device=gpu)
-        ops.kernels().gemm8g_fp8(Aq[:rows], Wq, C, off, slots, None, None, ws, 0, mx, None)
+        ops.kernels().gemm8g_fp8(Aq[:rows], Wq, C, ro, slots, None, None, ws, 0, mx, None)
         A = Aq[:rows].double() * _mx_scale_map(mx, K).double()
     else:
         if mode == "mx_out":
             mx = torch.zeros(N // 256, rows, 4, dtype=torch.uint8, device=gpu)
-        ops.kernels().gemm8g_fp8(Aq, Wq, C, off, slots, a_rows, xs, ws, {"plain": 0, "swiglu": 1, "mx_out": 2}[mode], None, mx)
-        A = (Aq.double() * xs.double()[:, None])[a_rows.long()]
+        ops.kernels().gemm8g_fp8(Aq, Wq, C, ro, slots, a_rows, xs, ws, {"plain": 0, "swiglu": 1, "mx_out": 2}[mode], None, mx)
+        A = Aq.double() * xs.double()[:, None]
+        A = A[:rows] if a_rows is None else A[a_rows.long()]
     assert (out[rows:].float() == 7).all()
     got = C.double() * _mx_scale_map(mx, N // 2).double() if mode == "mx_out" else C.double()
     o = off.tolist()
