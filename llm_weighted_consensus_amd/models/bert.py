@@ -21,6 +21,7 @@ GPU whose kernels failed to load.
 from __future__ import annotations
 
 import math
+import operator
 import os
 from dataclasses import dataclass
 from typing import Optional, Sequence
@@ -50,6 +51,9 @@ class EncLayer:
     b2: torch.Tensor
     ln2_g: torch.Tensor
     ln2_b: torch.Tensor
+
+
+_layer_tensors = operator.attrgetter(*EncLayer.__dataclass_fields__)
 
 
 class BertEncoder:
@@ -160,6 +164,15 @@ class BertEncoder:
         # but not under o's K = 768 (+119 us): profiles/round6_ab.md
         mode = self.fused_residual if d <= 1024 else "0"
         fuse_o, fuse_f = mode == "all", mode in ("all", "ffn2")
+        if x.dtype == torch.bfloat16 and self.layers:
+            L = self.layers[0]
+            cores = gemm_plan.encoder_cores(T, ((L.wqkv, L.bqkv, "bias"), (L.wo, None if fuse_o else L.bo, "enc_residual" if fuse_o else "bias"),
+                                                (L.w1, L.b1, "bias_gelu"),
+                                                (L.w2, None if fuse_f else L.b2, "enc_residual" if fuse_f else "bias")))
+            y = None if cores is None else ops.encoder_layers(x, [t for L in self.layers for t in _layer_tensors(L)], cu, max_len, H, Dh,
+                                                              self.scale, c.ln_eps, cores, fuse_o, fuse_f)
+            if y is not None:
+                return y
         for L in self.layers:
             qkv = lin(x, L.wqkv, L.bqkv)
             a = ops.prefill_attention(qkv[:, :d], qkv[:, d:2 * d], qkv[:, 2 * d:], cu, max_len, H, H, Dh, self.scale,

@@ -447,12 +447,26 @@ def gemm2w(A: torch.Tensor, W: torch.Tensor, residual: Optional[torch.Tensor] = 
         out = torch.empty(A.shape[0], W.shape[0] // 2 if swiglu else W.shape[0], dtype=torch.bfloat16, device=A.device)
     epi = 2 if swiglu else 1 if residual is not None else 0 if bias is None else 4 if gelu else 3
     if ws is None and (tile < 0 or splits > 1):
-        ws = _G8_WS.get((A.device.index, torch.cuda.current_stream(A.device).cuda_stream))
-        if ws is None and not torch.cuda.is_current_stream_capturing():
-            ws = gemm8p_workspace(A.device)
-    part, count = ws if ws is not None else (None, None)   # (none under capture: unsplit)
+        ws = _split_workspace(A.device)
+    part, count = ws if ws is not None else (None, None)   # (none: unsplit)
     kernels().gemm2w(A, W, out, bias if bias is not None else residual, epi, int(tile), int(splits), part, count)
     return out
+
+
+def _split_workspace(device: torch.device):
+    """gemm8p's workspace of the current stream, created if need be; None where it cannot be (under capture)."""
+    ws = _G8_WS.get((device.index, torch.cuda.current_stream(device).cuda_stream))
+    return gemm8p_workspace(device) if ws is None and not torch.cuda.is_current_stream_capturing() else ws
+
+
+def encoder_layers(x: torch.Tensor, weights: Sequence[torch.Tensor], cu: torch.Tensor, max_len: int, H: int, Dh: int,
+                   scale: float, eps: float, cores: Sequence[int], fuse_o: bool, fuse_f: bool) -> Optional[torch.Tensor]:
+    """The layers of a post-norm encoder (``models/bert.py``) launched from native code: ``weights`` 12 tensors a layer,
+    ``cores`` the cores of its four projections (:func:`gemm_plan.encoder_cores`).  ``x`` is overwritten.
+    None, and nothing done, if a weight is not laid out as those cores read it."""
+    part, count = _split_workspace(x.device) or (None, None)
+    return kernels().encoder_layers(x, weights, cu, int(max_len), int(H), int(Dh), float(scale), float(eps), cores, bool(fuse_o),
+                                    bool(fuse_f), part, count)
 
 
 def gemm2w_ok(N: int, K: int, *operands: Optional[torch.Tensor], swiglu: bool = False) -> bool:

@@ -174,6 +174,24 @@ def linear_bias(x: torch.Tensor, w: torch.Tensor, b: torch.Tensor, gelu: bool = 
 
 
 ENC_BACKENDS = ("blas", "g4", "g4p", "g8", "gv", "g2")
+_NATIVE = {"gv": 1, "g2": 2}
+
+
+def encoder_cores(M: int, projections) -> Optional[list]:
+    """The cores of an encoder layer's projections ((weight, its bias or None where it adds into the stream, epilogue
+    name) each) at M rows as ``ops.encoder_layers`` numbers them; None until all are timed, or if one's choice is another
+    core or does not take the call."""
+    out = []
+    for w, b, epi in projections:
+        N, K = w.shape
+        c = MODE if MODE in ENC_BACKENDS else _CHOICE.get((_m_bucket(M), N, K, epi))
+        n = _NATIVE.get(c)
+        if n is None or not _g8_ok(N, K, epi) or c in EXCLUDE:
+            return None
+        if not (SKINNY and skinny_ok(M, N, K) if n == 1 else M <= G2_ROWS and gemm2w_ok(N, K, w, b)):
+            return None
+        out.append(n)
+    return out
 
 
 def _enc_ok(n: str, x: torch.Tensor, w: torch.Tensor, epi: str, other: torch.Tensor) -> bool:

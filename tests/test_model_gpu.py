@@ -130,6 +130,40 @@ def test_engine_export_import_prefill_equivalence(tiny, gpu):
     assert b.bm.num_free == 256
 
 
+@pytest.mark.parametrize("core,lens", [("gv", [5, 1, 40]), ("g2", [5, 1, 40]), ("g2", [300, 2, 64, 129])])
+@pytest.mark.parametrize("fused", ["0", "ffn2", "all"])
+def test_encoder_layers_launched_natively(gpu, monkeypatch, core, lens, fused):
+    """The natively launched layers run the loop's kernels: the same bits, and the loop itself where a weight lies at an odd
+    address or a projection has another core."""
+    from llm_weighted_consensus_amd import ops
+    from llm_weighted_consensus_amd.models.bert import BertEncoder
+    from llm_weighted_consensus_amd.models.config import encoder_config
+    from llm_weighted_consensus_amd.ops import gemm_plan
+
+    m = BertEncoder(encoder_config("bge-small-en-v1.5"), device=gpu, seed=5)
+    m.fused_residual = fused
+    args = m.pack([[(7 * i + j) % 900 + 1 for j in range(n)] for i, n in enumerate(lens)])
+    monkeypatch.setattr(gemm_plan, "MODE", core)
+    taken, native = [], ops.encoder_layers
+    monkeypatch.setattr(ops, "encoder_layers", lambda *a: taken.append(native(*a)) or taken[-1])
+    y = m.forward_packed(*args)
+    assert len(taken) == 1 and taken[0] is not None
+    monkeypatch.setattr(ops, "encoder_layers", lambda *a: None)
+    assert torch.equal(y, m.forward_packed(*args))
+    monkeypatch.setattr(ops, "encoder_layers", lambda *a: taken.append(native(*a)) or taken[-1])
+    w = m.layers[1].w2
+    m.layers[1].w2 = torch.cat([w.flatten()[:1], w.flatten()])[1:].view(w.shape)   # two bytes off
+    if core == "gv":
+        torch.testing.assert_close(y, m.forward_packed(*args))
+    else:
+        assert torch.isfinite(m.forward_packed(*args).float()).all()
+    assert len(taken) == 2 and taken[1] is None
+    m.layers[1].w2 = w
+    monkeypatch.setattr(gemm_plan, "MODE", "blas")
+    m.forward_packed(*args)
+    assert len(taken) == 2
+
+
 @pytest.mark.parametrize("fused", ["ffn2", "all", "0"])
 @pytest.mark.parametrize("arch", ["bge-small-en-v1.5", "bert-tiny"])
 def test_bert_encoder_matches_reference(gpu, arch, fused):
