@@ -1,4 +1,4 @@
-// Grouped fp8 GEMM of few rows per group (gfx950): the calls of the 8-phase kernel (gemm8g.hip: the same operands, epilogues
+// Grouped fp8 and bf16 GEMM of few rows per group (gfx950): the calls of the 8-phase kernel (gemm8g.hip: the same operands, epilogues
 // and MX form) while the weights, not the matrix cores, bound them.
 //
 // The 8-phase kernel keeps one workgroup per CU with 32 KiB of weights on their way, and hands its CU over with nothing in
@@ -10,6 +10,8 @@
 // a plain read): 4 rows an expert 257 -> 182, 144 -> 81; 32 rows 259 -> 189, 145 -> 84; 64 rows 264 -> 200, 150 -> 90; 128 rows
 // 270 -> 217, 155 -> 115.  In steps in flight: one workgroup of six (four) steps for the first GEMM 189 to 257, two workgroups of
 // three (two) steps for the second 123 to 175.  Dense calls of few tiles likewise: 512 rows x 4096 x K 4096 from MX 45 -> 21.
+// bf16, 8 experts of 16 rows: [14336, 4096] 194 (the 128-row kernel with split K, its clear and its conversion 204), [4096, 7168] 82
+// (103).
 #include "common.h"
 
 namespace lwc {
@@ -17,11 +19,11 @@ namespace g2g {
 
 typedef int v8i32 __attribute__((ext_vector_type(8)));
 
-constexpr int kPlain = 0, kSwiglu = 1, kMxOut = 2, kMxA = 3;  // as in gemm8g.hip
+constexpr int kPlain = 0, kSwiglu = 1, kMxOut = 2, kMxA = 3, kBf16 = 4, kBf16Swiglu = 5;  // as in gemm8g.hip
 
 struct Params {
-  const uint8_t* A;      // [rows_a, lda] e4m3
-  const uint8_t* W;      // [G][N, K] e4m3
+  const uint8_t* A;      // [rows_a, lda] e4m3 or bf16 (lda, K in bytes)
+  const uint8_t* W;      // [G][N, K]
   bf16_t* C;
   const int* row_off;
   const int* a_rows;
@@ -38,6 +40,10 @@ LWC_DEVICE float4v mfma8(const uint4v& a0, const uint4v& a1, const uint4v& b0, c
   const v8i32 av = {(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w, (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
   const v8i32 bv = {(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w, (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, 0, 127, 0, sb);
+}
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+LWC_DEVICE float4v mfma16(const uint4v& a, const uint4v& b, const float4v& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 LWC_DEVICE float silu8(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 LWC_DEVICE void dma16(const __amdgpu_buffer_rsrc_t& r, uint8_t* dst, uint32_t vo, int so) {
@@ -67,7 +73,7 @@ LWC_DEVICE void wait_steps(int n) {
 
 template <int MODE, int TM, int NST>
 __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
-  constexpr bool MXA = MODE == kMxA;
+  constexpr bool MXA = MODE == kMxA, BF = MODE == kBf16 || MODE == kBf16Swiglu;
   constexpr int TN = 128, kA = TM * 128, kS = kA + TN * 128, kStage = kS + (MXA ? 1024 : 0);  // rows, weights, scales
   constexpr int IA = TM / 32, IW = TN / 32, MI = TM / 32;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -173,7 +179,10 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
 #pragma unroll
         for (int c = 0; c < 2; ++c)
 #pragma unroll
-          for (int h = 0; h < 2; ++h) acc[i][c][h] = mfma8(w[0][c][h], w[1][c][h], a[0][i], a[1][i], acc[i][c][h], MXA ? sc[i] : 127);
+          for (int h = 0; h < 2; ++h) {
+            if constexpr (BF) acc[i][c][h] = mfma16(w[1][c][h], a[1][i], mfma16(w[0][c][h], a[0][i], acc[i][c][h]));
+            else acc[i][c][h] = mfma8(w[0][c][h], w[1][c][h], a[0][i], a[1][i], acc[i][c][h], MXA ? sc[i] : 127);
+          }
       }
     __builtin_amdgcn_s_setprio(0);
     __builtin_amdgcn_sched_barrier(0);
@@ -184,17 +193,17 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
 #pragma unroll
   for (int c = 0; c < 2; ++c)
 #pragma unroll
-    for (int e = 0; e < 8; ++e) ws[c][e] = col0 + 32 * c < p.N ? p.w_scale[(size_t)g * p.N + col0 + 32 * c + e] : 0.f;
+    for (int e = 0; e < 8; ++e) ws[c][e] = !BF && col0 + 32 * c < p.N ? p.w_scale[(size_t)g * p.N + col0 + 32 * c + e] : 0.f;
 #pragma unroll
   for (int i = 0; i < MI; ++i) {
     const int m = m_begin + (2 * i + wr) * 16 + r16;
-    const float as = MXA ? 1.f : p.a_scale[p.a_rows ? p.a_rows[src_row[i]] : src_row[i]];
+    const float as = MXA || BF ? 1.f : p.a_scale[p.a_rows ? p.a_rows[src_row[i]] : src_row[i]];
     float x[2][8];
 #pragma unroll
     for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) x[c][e] = acc[i][c][e >> 2][e & 3] * (as * ws[c][e]);
-    if constexpr (MODE == kPlain || MODE == kMxA) {
+      for (int e = 0; e < 8; ++e) x[c][e] = BF ? acc[i][c][e >> 2][e & 3] : acc[i][c][e >> 2][e & 3] * (as * ws[c][e]);
+    if constexpr (MODE == kPlain || MODE == kMxA || MODE == kBf16) {
 #pragma unroll
       for (int c = 0; c < 2; ++c)
         if (m < m_end && col0 + 32 * c < p.N) *reinterpret_cast<uint4v*>(p.C + (size_t)m * p.ldc + col0 + 32 * c) = pack8(x[c]);
@@ -204,7 +213,7 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) y[e] = silu8(x[0][e]) * x[1][e];
       const uint4v packed = pack8(y);
-      if constexpr (MODE == kSwiglu) {
+      if constexpr (MODE == kSwiglu || MODE == kBf16Swiglu) {
         if (m < m_end && col < p.N / 2) *reinterpret_cast<uint4v*>(p.C + (size_t)m * p.ldc + col) = packed;
       } else {  // e4m3 rows, one e8m0 scale per row and block of 32: four lanes hold a block
         float v[8];
@@ -245,8 +254,9 @@ int launch(Params p, int rows, hipStream_t s) {
 }  // namespace g2g
 }  // namespace lwc
 
-// The operands of lwc_gemm8g_fp8 (checked there), row_off null for a dense call; mode 3: A carries MX scales.  rows: all groups' rows.
-extern "C" int lwc_gemm2g_fp8(const void* A, const void* W, void* C, const int* row_off, const int* a_rows,
+// The operands of lwc_gemm8g_fp8 (checked there), row_off null for a dense call, or of lwc_gemm8g_bf16 (K and lda in bytes);
+// mode 3: A carries MX scales; 4, 5: bf16.  rows: all groups' rows.
+extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_off, const int* a_rows,
                               const float* a_scale, const float* w_scale, int G, int N, int K, int lda, int ldc, int rows_a,
                               int rows, int mode, const void* a_mx, void* mx_out, int s_rows, hipStream_t s) {
   using namespace lwc::g2g;
@@ -269,6 +279,8 @@ extern "C" int lwc_gemm2g_fp8(const void* A, const void* W, void* C, const int* 
     LWC_G2G(kSwiglu, 6, 5, 4)
     LWC_G2G(kMxOut, 6, 5, 4)
     LWC_G2G(kMxA, 6, 4, 3)
+    LWC_G2G(kBf16, 6, 5, 4)
+    LWC_G2G(kBf16Swiglu, 6, 5, 4)
   }
 #undef LWC_G2G
   return -1;

@@ -415,13 +415,14 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
 }  // namespace g8g
 }  // namespace lwc
 
-extern "C" int lwc_gemm2g_fp8(const void*, const void*, void*, const int*, const int*, const float*, const float*, int, int, int, int,
+extern "C" int lwc_gemm2g(const void*, const void*, void*, const int*, const int*, const float*, const float*, int, int, int, int,
                               int, int, int, int, const void*, void*, int, hipStream_t);
 
 // rows per group up to which the weights bound a grouped call and gemm2g.hip takes it.  us, 8-phase / gemm2g: SwiGLU to MX
 // [28672, 4096] x 8 at 128 rows a group 270 / 217, 175 rows 272 / 237, 256 rows 293 / 344; from MX [4096, 14336] x 8 at 128 rows
-// 155 / 115, 175 rows (a group of 219 needs a second tile, 288 for 256 CUs) 161 / 188
-constexpr int kSmallRows = 144, kSmallRowsSwiglu = 176;
+// 155 / 115, 175 rows (a group of 219 needs a second tile, 288 for 256 CUs) 161 / 188; bf16 [14336, 4096] x 8 at 128 rows a group
+// 245 / 223, 162 rows 245 / 233, [4096, 7168] x 8 148 / 115, 148 / 120
+constexpr int kSmallRows = 144, kSmallRowsSwiglu = 176, kSmallRowsBf16 = 176;
 // and the dense calls: up to this many 256 x 256 tiles.  us, 8-phase / gemm2g, K 4096: 512 rows x 4096 (32 tiles) 45 / 21, 2048 x
 // 4096 (128) 48 / 34, 256 x 28672 SwiGLU to MX (112) 51 / 43, 2048 x 6144 (192) 49 / 66, 512 x 28672 (224) 61 / 73
 constexpr long long kSmallTiles = 128;
@@ -448,7 +449,7 @@ extern "C" int lwc_gemm8g_fp8(const void* A, const void* W, void* C, const int* 
   const bool small = row_off ? rows_c <= (swiglu ? kSmallRowsSwiglu : kSmallRows) * (long long)G
                              : (long long)((rows_c + 255) / 256) * ((N + 255) / 256) <= kSmallTiles;
   if (small && rows_c > 0)
-    return lwc_gemm2g_fp8(A, W, C, row_off, a_rows, a_scale, w_scale, G, N, K, lda, ldc, rows_a, rows_c, a_mx ? 3 : mode, a_mx, mx_out,
+    return lwc_gemm2g(A, W, C, row_off, a_rows, a_scale, w_scale, G, N, K, lda, ldc, rows_a, rows_c, a_mx ? 3 : mode, a_mx, mx_out,
                           s_rows, s);
   static bool attr = false;
   if (!attr) {
@@ -492,6 +493,9 @@ extern "C" int lwc_gemm8g_bf16(const void* A, const void* W, void* C, const int*
   if (!row_off || K % 64 != 0 || K < 64 || N % (swiglu ? 64 : 8) != 0 || lda % 8 != 0 || ldc % 8 != 0 || G < 1) return -1;
   if ((long long)rows_a * lda * 2 >= (1LL << 31) || 512LL * K >= (1LL << 31)) return -1;
   if (max_slots <= 0) return 0;
+  if (rows_c > 0 && rows_c <= kSmallRowsBf16 * (long long)G)
+    return lwc_gemm2g(A, W, C, row_off, a_rows, nullptr, nullptr, G, N, K * 2, lda * 2, ldc, rows_a, rows_c, swiglu ? 5 : 4, nullptr,
+                      nullptr, 0, s);
   static bool attr = false;
   if (!attr) {
     (void)hipFuncSetAttribute((const void*)gemm8g_kernel<kBf16>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsB);

@@ -305,7 +305,8 @@ def grouped_gemm(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tensor, max_sl
     (default: ceil(rows/128) + G, enough for any split of the rows into G groups).  ``splits`` > 1 splits
     K over that many workgroups per tile (fp32 atomics into a workspace, then one bf16 pass); default:
     chosen so a small-M launch (MoE decode down projection: 8 experts x 32 column tiles) still puts
-    ~4 workgroups on every CU.  Large batches run on the 8-phase 256-row tiles (csrc/kernels/gemm8g.hip), fp8 and bf16.  ``swiglu=True``: W's rows are gate / up interleaved in blocks of 32
+    ~4 workgroups on every CU.  Batches of at least a row per group run on tiles of 64 to 192 rows
+    (csrc/kernels/gemm2g.hip) or the 8-phase 256-row tiles (csrc/kernels/gemm8g.hip), fp8 and bf16.  ``swiglu=True``: W's rows are gate / up interleaved in blocks of 32
     (:func:`swiglu_interleave` per group) and the result is silu(gate) * up [rows, N/2] — from the 8-phase
     kernel's epilogue when it takes the batch, else GEMM + the SwiGLU pass.  ``a_mx`` [K/128, rows, 4] uint8:
     A carries MX block scales (from :func:`grouped_gemm_swiglu_mx`) instead of ``a_scale`` — 8-phase kernel
@@ -377,14 +378,15 @@ def moe_mx_ok(A: torch.Tensor, W13: torch.Tensor, W2: torch.Tensor, rows: int) -
     return rows * (N // 2) < (1 << 31) and (N // 256) * rows * 4 < (1 << 31)
 
 
-# rows per group (on average) from which bf16 groups take the 8-phase 256-row tiles.  Below, the 128-row kernel with K split
-# over workgroups reads the weights faster; 8 experts, one MI355X, 128-row kernel / 8-phase, us: [14336, 4096] weights
-# 64 rows a group 235 / 236, 128 rows 336 / 245, 4096 rows 4720 / 2988; [4096, 7168] 133 / 143, 200 / 148, 2376 / 1481
-GROUPED_BF16_8PHASE_ROWS = 96
+# rows per group (on average) from which bf16 groups take the small-tile and 8-phase kernels (csrc/kernels/gemm2g.hip,
+# gemm8g.hip; which of the two is decided there).  Below, few groups have a row at all, and the 128-row kernel's split of K over
+# workgroups is what reads their weights; 8 experts, one MI355X, 128-row kernel / here, us: [14336, 4096] weights 2 rows in all
+# 51 / 34, 8 rows 124 / 125, 128 rows 204 / 194, 1024 rows 336 / 223; [4096, 7168] 32 / 44, 93 / 71, 103 / 82, 201 / 115
+GROUPED_BF16_ROWS = 1
 
 
 def _use_gemm8g_bf16(A, W, rows, G, N, K, bias, splits, out) -> bool:
-    """Whether bf16 groups run on the 8-phase kernel: enough rows per group, 16-byte rows, 32-bit spans."""
+    """Whether bf16 groups run on the small-tile / 8-phase kernels: enough rows per group, 16-byte rows, 32-bit spans."""
     if A.dtype != torch.bfloat16 or W.dtype != torch.bfloat16 or bias is not None or (splits or 1) > 1:
         return False
     if K % 64 or N % 8 or A.stride(1) != 1 or A.stride(0) % 8 or A.data_ptr() % 16 or W.data_ptr() % 16:
@@ -393,7 +395,7 @@ def _use_gemm8g_bf16(A, W, rows, G, N, K, bias, splits, out) -> bool:
         return False
     if out is not None and (out.stride(1) != 1 or out.stride(0) % 8 or out.data_ptr() % 16):
         return False
-    return rows >= GROUPED_BF16_8PHASE_ROWS * G
+    return rows >= GROUPED_BF16_ROWS * G
 
 
 def _use_gemm8g(A, W, rows, G, N, K, bias, splits, out) -> bool:
