@@ -165,6 +165,70 @@ latent_expand_write_kernel(const AT* __restrict__ kv, int ldk, const AT* __restr
   }
 }
 
+// The same four entries at a time.  Four tokens share the words of the interleaved value rows: where a token's slot begins such a
+// word and the next three tokens fill it, its workgroup writes the values of all four (the others only their keys), else
+// every token its own.  Bound by its writes: 16384 tokens, 32 heads of 128 + 64 and 128, took 324 us with two-byte stores into words
+// that four workgroups shared, 233 so (600 MB).
+template <typename AT>
+__global__ void __launch_bounds__(256)
+latent_expand_write_vec_kernel(const AT* __restrict__ kv, int ldk, const AT* __restrict__ lat, int ldl, int rot_off,
+                               const long long* __restrict__ slots, AT* __restrict__ k_cache, AT* __restrict__ v_cache,
+                               long long kb_stride, long long vb_stride, int block_size, int N, int H, int D, int R, int Dv, int dk, int dv) {
+  typedef AT AT4 __attribute__((ext_vector_type(4)));
+  typedef AT AT8 __attribute__((ext_vector_type(8), aligned(16)));
+  const int t = blockIdx.x;
+  long long near[7];  // (the neighbours' slots at once: one trip to memory instead of five)
+#pragma unroll
+  for (int i = 0; i < 7; ++i) near[i] = slots[min(max(t + i - 3, 0), N - 1)];
+  const long long slot = near[3];
+  if (slot < 0) return;
+  const unsigned blk = (unsigned)slot / (unsigned)block_size, off = (unsigned)slot % (unsigned)block_size;
+  const int sub = (int)(slot & 3);
+  bool four = t >= sub && t - sub + 3 < N;
+#pragma unroll
+  for (int i = 0; i < 7; ++i) four = four && (i + sub < 3 || i + sub > 6 || near[i] == slot + i - 3);
+  const AT4 zero = {0, 0, 0, 0};
+  const AT* kr = kv + (size_t)t * ldk;
+  const AT* lr = lat + (size_t)t * ldl + rot_off;
+  AT* kc = k_cache + (long long)blk * kb_stride + off * ((long long)H * dk);
+  const int k4 = dk / 4, v4 = dv / 4;
+  // (a group's head and entry, stepped instead of divided out each time)
+  struct At {
+    int h, i, dh, di, n;
+    LWC_DEVICE At(int n) : h(threadIdx.x / n), i(threadIdx.x % n), dh(256 / n), di(256 % n), n(n) {}
+    LWC_DEVICE void step() {
+      h += dh, i += di;
+      if (i >= n) i -= n, ++h;
+    }
+  };
+#pragma unroll 4
+  for (At a(k4); a.h < H; a.step()) {
+    const int i = 4 * a.i;
+    *reinterpret_cast<AT4*>(kc + (size_t)a.h * dk + i) = i < D ? *reinterpret_cast<const AT4*>(kr + a.h * D + i)
+                                                         : i < D + R ? *reinterpret_cast<const AT4*>(lr + i - D) : zero;
+  }
+  if (four && sub != 0) return;
+  AT* vc = v_cache + (long long)blk * vb_stride + (off >> 2) * (4LL * H * dv);
+  const AT* vr = kr + H * D;
+#pragma unroll 2
+  for (At a(v4); a.h < H; a.step()) {
+    const int h = a.h, i = 4 * a.i;
+    AT* o = vc + 16 * ((size_t)h * v4 + a.i);
+    if (four) {
+      AT4 x[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[j] = i < Dv ? *reinterpret_cast<const AT4*>(vr + (size_t)j * ldk + h * Dv + i) : zero;
+#pragma unroll
+      for (int c = 0; c < 4; c += 2)
+        *reinterpret_cast<AT8*>(o + 4 * c) = AT8{x[0][c], x[1][c], x[2][c], x[3][c], x[0][c + 1], x[1][c + 1], x[2][c + 1], x[3][c + 1]};
+    } else {
+      const AT4 x = i < Dv ? *reinterpret_cast<const AT4*>(vr + h * Dv + i) : zero;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[4 * c + sub] = x[c];
+    }
+  }
+}
+
 // ENTRY: a gate per entry (gate rows [H Dv]), else per head (gate rows [H])
 template <typename AT, bool ENTRY>
 __global__ void __launch_bounds__(256) head_gate_rows_kernel(const AT* __restrict__ o, long long row_stride, long long head_stride,
@@ -234,6 +298,18 @@ extern "C" int r32_latent_expand_write(const void* kv, int ldk, const void* lat,
                                        int N, int H, int D, int R, int Dv, int dk, int dv, int f32, hipStream_t s) {
   if (N <= 0) return 0;
   if (dk < D + R || dv < Dv) return -1;
+  const int a4 = f32 ? 16 : 8;
+  if (((D | R | Dv | dk | dv | ldk | ldl | rot_off | block_size) & 3) == 0 && ((kb_stride | vb_stride) & 3) == 0 && aligned_to(kv, a4) &&
+      aligned_to(lat, a4) && aligned_to(k_cache, a4) && aligned_to(v_cache, 16) && (vb_stride & 7) == 0) {
+    if (f32)
+      latent_expand_write_vec_kernel<float><<<N, 256, 0, s>>>((const float*)kv, ldk, (const float*)lat, ldl, rot_off, slots, (float*)k_cache,
+                                                              (float*)v_cache, kb_stride, vb_stride, block_size, N, H, D, R, Dv, dk, dv);
+    else
+      latent_expand_write_vec_kernel<bf16_t><<<N, 256, 0, s>>>((const bf16_t*)kv, ldk, (const bf16_t*)lat, ldl, rot_off, slots, (bf16_t*)k_cache,
+                                                               (bf16_t*)v_cache, kb_stride, vb_stride, block_size, N, H, D, R, Dv, dk, dv);
+    LWC_CHECK_LAUNCH();
+    return 0;
+  }
   if (f32)
     latent_expand_write_kernel<float><<<N, 256, 0, s>>>((const float*)kv, ldk, (const float*)lat, ldl, rot_off, slots,
                                                         (float*)k_cache, (float*)v_cache, kb_stride, vb_stride, block_size, H, D,

@@ -247,6 +247,32 @@ def test_retention_portions_single_tokens_and_stale_slots(gpu, dtype, tol, H, D,
         assert (state[slot[k]].cpu().double() - ref_S[k]).abs().max() < tol * 4 * max(1.0, float(ref_S[k].abs().max())), k
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,D,R,Dv,dk,dv", [(3, 16, 8, 12, 32, 16), (2, 128, 64, 128, 192, 128), (2, 10, 6, 9, 16, 12)])
+def test_expanded_pages(gpu, dtype, H, D, R, Dv, dk, dv):
+    """Keys and values of sequences that begin anywhere in a word of four tokens, end anywhere in one, lie side by side or
+    apart: every entry of their slots, and no other, is written, bit for bit."""
+    from llm_weighted_consensus_amd.models.cache import PagedLayerCache
+    from llm_weighted_consensus_amd.ops import res32
+
+    g = torch.Generator().manual_seed(D)
+    runs = [(0, 9), (11, 2), (13, 3), (18, 14), (35, 1), (40, 4), (45, 19)]   # first slot, tokens
+    slots = torch.cat([torch.arange(a, a + n) for a, n in runs])
+    N = len(slots)
+    kv = torch.randn(N, H * (D + Dv) + 4, generator=g).to(dtype)[:, :H * (D + Dv)].to(gpu)
+    lat = torch.randn(N, 8 + R + 4, generator=g).to(dtype).to(gpu)
+    cache = PagedLayerCache([(H * dk, H * dv)], 5, 16, gpu, dtype)
+    cache.pool.fill_(7.0)
+    res32.latent_expand_write(kv, lat, 8, R, slots.to(gpu), cache.k[0], cache.v[0], H, D, Dv)
+    K, V = (x.float().cpu() for x in cache.rows(0, torch.arange(80, device=gpu)))
+    wk, wv = torch.full((80, H, dk), 7.0), torch.full((80, H, dv), 7.0)
+    wk[slots], wv[slots] = 0.0, 0.0
+    wk[slots, :, :D] = kv[:, :H * D].float().cpu().view(N, H, D)
+    wk[slots, :, D:D + R] = lat[:, 8:8 + R].float().cpu()[:, None]
+    wv[slots, :, :Dv] = kv[:, H * D:].float().cpu().view(N, H, Dv)
+    assert torch.equal(K.view(80, H, dk), wk) and torch.equal(V.view(80, H, dv), wv)
+
+
 @pytest.mark.parametrize("H,D,Dv,dtype", [(2, 128, 128, torch.bfloat16), (3, 32, 16, torch.float32), (2, 24, 40, torch.bfloat16),
                                           (1, 64, 130, torch.float32), (2, 200, 72, torch.float32), (1, 256, 64, torch.bfloat16)])
 @pytest.mark.parametrize("act", [False, True])
