@@ -305,7 +305,7 @@ def grouped_gemm(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tensor, max_sl
     (default: ceil(rows/128) + G, enough for any split of the rows into G groups).  ``splits`` > 1 splits
     K over that many workgroups per tile (fp32 atomics into a workspace, then one bf16 pass); default:
     chosen so a small-M launch (MoE decode down projection: 8 experts x 32 column tiles) still puts
-    ~4 workgroups on every CU.  Batches of at least a row per group run on tiles of 64 to 192 rows
+    ~4 workgroups on every CU.  Batches of at least four rows per group run on tiles of 64 to 192 rows
     (csrc/kernels/gemm2g.hip) or the 8-phase 256-row tiles (csrc/kernels/gemm8g.hip), fp8 and bf16.  ``swiglu=True``: W's rows are gate / up interleaved in blocks of 32
     (:func:`swiglu_interleave` per group) and the result is silu(gate) * up [rows, N/2] — from the 8-phase
     kernel's epilogue when it takes the batch, else GEMM + the SwiGLU pass.  ``a_mx`` [K/128, rows, 4] uint8:
@@ -379,10 +379,11 @@ def moe_mx_ok(A: torch.Tensor, W13: torch.Tensor, W2: torch.Tensor, rows: int) -
 
 
 # rows per group (on average) from which bf16 groups take the small-tile and 8-phase kernels (csrc/kernels/gemm2g.hip,
-# gemm8g.hip; which of the two is decided there).  Below, few groups have a row at all, and the 128-row kernel's split of K over
-# workgroups is what reads their weights; 8 experts, one MI355X, 128-row kernel / here, us: [14336, 4096] weights 2 rows in all
-# 51 / 34, 8 rows 124 / 125, 128 rows 204 / 194, 1024 rows 336 / 223; [4096, 7168] 32 / 44, 93 / 71, 103 / 82, 201 / 115
-GROUPED_BF16_ROWS = 1
+# gemm8g.hip; which of the two is decided there).  Below, the two GEMMs of an expert together gain little or nothing, and the
+# 128-row kernel's split of K over workgroups stays; 8 experts, one MI355X, 128-row kernel / here, us, [14336, 4096] (whose SwiGLU pass
+# of 5 the epilogue saves) and [4096, 7168]: 16 rows in all 157 / 175 and 99 / 81, 32 rows 184 / 191 and 100 / 82, 128 rows 204 / 194
+# and 103 / 82, 1024 rows 336 / 223 and 201 / 115
+GROUPED_BF16_ROWS = 4
 
 
 def _use_gemm8g_bf16(A, W, rows, G, N, K, bias, splits, out) -> bool:

@@ -1008,7 +1008,7 @@ def test_gemm8g_grouped_fp8_matches_reference(gpu, gather, monkeypatch):
                                          # groups of few rows (gemm2g.hip): tiles of 64, 128, 192 rows, few tiles and many
                                          ([2, 0, 3], 256, 128), ([64, 65, 40, 3], 640, 1536), ([192, 193, 100], 328, 448),
                                          ([30, 50, 40, 9], 10560, 64)])
-def test_grouped_gemm_bf16_8phase(gpu, sizes, N, K, gather, swiglu):
+def test_grouped_gemm_bf16_8phase(gpu, sizes, N, K, gather, swiglu, monkeypatch):
     """bf16 groups on the 8-phase kernel (gemm8g.hip): empty groups, groups of less than, exactly and more than whole
     256-row tiles, N past the last whole tile, one to seven K tiles, a gathered A, the SwiGLU epilogue; vs fp32 products
     of the same operands.  Bound: one bf16 rounding (2^-9 relative, doubled) and fp32 sums of K terms."""
@@ -1016,6 +1016,7 @@ def test_grouped_gemm_bf16_8phase(gpu, sizes, N, K, gather, swiglu):
 
     if swiglu and N % 64:
         N = 384
+    monkeypatch.setattr(ops, "GROUPED_BF16_ROWS", 0)
     torch.manual_seed(12)
     G, rows = len(sizes), sum(sizes)
     off = torch.tensor([0] + list(np.cumsum(sizes)), dtype=torch.int32, device=gpu)
