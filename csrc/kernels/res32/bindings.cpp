@@ -46,6 +46,7 @@ int r32_rmsnorm_rows(const float*, const long long*, const float*, void*, int, i
 int r32_gelu_mul_rows(const void*, int, const void*, int, int, const int*, int, void*, int, int, int, hipStream_t);
 int r32_stack_mix(const float*, long long, const float*, int, float*, long long, hipStream_t);
 int r32_router_max_outputs();
+int r32_router_one_group(int, int);
 int r32_router(const float*, int, const float*, const float*, int, int, float, float, int, int, int, int, int, int, int*, float*,
                int*, int*, int*, int*, int*, int*, hipStream_t);
 int r32_expert_rows(const void*, int, const int*, const int*, const int*, int, const void*, const void*, float*, int, int,
@@ -626,7 +627,8 @@ std::vector<Tensor> router(Tensor z, c10::optional<Tensor> corr, int64_t E, int6
   auto oi = z.options().dtype(torch::kInt32);
   Tensor ids = torch::empty({T, k}, oi), w = torch::empty({T, k}, z.options()), rank = torch::empty({T, k}, oi);
   const int64_t Ec = std::max<int64_t>(E, 1);
-  Tensor zeroed = torch::zeros({Ec + 2 * (int64_t)T * k}, oi);  // counts | src | row_expert: one fill
+  const int64_t ints = Ec + 2 * (int64_t)T * k;  // counts | src | row_expert: one fill where the kernels need one
+  Tensor zeroed = r32_router_one_group(T, NE) ? torch::empty({ints}, oi) : torch::zeros({ints}, oi);
   Tensor counts = zeroed.narrow(0, 0, Ec), src = zeroed.narrow(0, Ec, T * k), row_expert = zeroed.narrow(0, Ec + T * k, T * k);
   Tensor row_off = torch::empty({E + 1}, oi), inv = torch::empty({T * k}, oi);
   done(r32_router(z.data_ptr<float>(), ldz, corr.has_value() ? corr->data_ptr<float>() : nullptr,

@@ -17,6 +17,7 @@ namespace lwc {
 namespace {
 
 constexpr int kMaxPerLane = 8;  // router outputs per lane: NE <= 512
+constexpr int kOneGroup = 512;   // tokens that one workgroup routes (router_one_group_kernel)
 
 // How scores become choices and weights.
 struct RouterRule {
@@ -146,13 +147,29 @@ __global__ void router_topk_kernel(const float* __restrict__ z, const float* __r
     for (int j = 0; j < k; ++j) wts[(size_t)t * k + j] *= rule.scale / (rule.renorm ? chosen + rule.floor : 1.0f);
 }
 
-// Few router outputs (NE <= NMAX): one THREAD per token, the scores in registers.
+// This lane's rank within expert x, for a wave whose lanes hold one choice each: lane e's `next` is the rank that the first
+// of them to choose expert e takes, and moves past them all.  -1 where x is no real expert or the lane is not live.
+__device__ __forceinline__ int expert_rank(int x, bool live, int E, int& next) {
+  const int lane = threadIdx.x & 63;
+  int r = -1;
+  for (int e = 0; e < E; ++e) {
+    const unsigned long long m = __ballot(live && x == e);
+    if (m == 0ull) continue;
+    const int first = __builtin_amdgcn_readlane(next, e);
+    if (live && x == e) r = first + __popcll(m & ((1ull << lane) - 1ull));
+    if (lane == e) next += __popcll(m);
+  }
+  return r;
+}
+
+// Few router outputs (NE <= NMAX): one THREAD per token t0, the scores in registers.  Writes ids and weights and returns
+// the k choices, four bits each.  mine, in lane e < E: how many choices of this wave's tokens are expert e.
 template <int NMAX>
-__global__ void router_topk_thread_kernel(const float* __restrict__ z, const float* __restrict__ corr,
-                                          const float* __restrict__ bias, int ldz, RouterRule rule, int NE, int E, int k,
-                                          int* __restrict__ ids, float* __restrict__ wts, int* __restrict__ counts,
-                                          int* __restrict__ rank, int T) {
-  const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ unsigned long long route_token(const float* __restrict__ z, const float* __restrict__ corr,
+                                                          const float* __restrict__ bias, int ldz, RouterRule rule, int NE,
+                                                          int E, int k, int* __restrict__ ids, float* __restrict__ wts,
+                                                          int t0, int T, int& mine) {
+  static_assert(NMAX <= 16, "a choice takes four bits");
   const bool live = t0 < T;  // lanes past the last token go along (wave-wide votes below) and write nothing
   const int t = live ? t0 : T - 1;
   const float* zr = z + (size_t)t * ldz;
@@ -209,6 +226,8 @@ __global__ void router_topk_thread_kernel(const float* __restrict__ z, const flo
       if (!((open >> i) & 1u)) c[i] = -INFINITY;
   }
   float chosen = 0.f;
+  unsigned long long picks = 0;
+  mine = 0;
   for (int j = 0; j < k; ++j) {
     float best = -INFINITY, sc = 0.f;
     int bi = 0;
@@ -219,26 +238,72 @@ __global__ void router_topk_thread_kernel(const float* __restrict__ z, const flo
     for (int i = 0; i < NMAX; ++i)
       if (i == bi) c[i] = -INFINITY;
     chosen += sc;
+    picks |= (unsigned long long)bi << (4 * j);
+    expert_rank(bi, live, E, mine);
     if (live) {
       ids[(size_t)t * k + j] = bi;
       wts[(size_t)t * k + j] = sc;
     }
-    // one atomic per (wave, expert) instead of one per token: the wave's tokens that chose expert e take
-    // consecutive ranks in lane order
-    int rk = -1;
-    for (int e = 0; e < E; ++e) {
-      const unsigned long long m = __ballot(live && bi == e);
-      if (m == 0ull) continue;
-      const int leader = __ffsll((long long)m) - 1;
-      int base = 0;
-      if ((int)(threadIdx.x & 63) == leader) base = atomicAdd(counts + e, __popcll(m));
-      base = __shfl(base, leader, 64);
-      if (live && bi == e) rk = base + __popcll(m & ((1ull << (threadIdx.x & 63)) - 1ull));
-    }
-    if (live) rank[(size_t)t * k + j] = rk;
   }
   if (live && (rule.renorm || rule.scale != 1.0f))
     for (int j = 0; j < k; ++j) wts[(size_t)t * k + j] *= rule.scale / (rule.renorm ? chosen + rule.floor : 1.0f);
+  return picks;
+}
+
+// One atomic per (wave, expert): lane e takes as many ranks of expert e as its wave's tokens have chosen it, and the
+// tokens take them choice by choice, in lane order.  (An atomic per wave, choice AND expert, each waited for: 16.8 us for
+// 1024 tokens, top 2 of 8; 73 us for top 8 of 16.  So: 12.3 and 32 us, with the fill, offsets and scatter.)
+template <int NMAX>
+__global__ void router_topk_thread_kernel(const float* __restrict__ z, const float* __restrict__ corr,
+                                          const float* __restrict__ bias, int ldz, RouterRule rule, int NE, int E, int k,
+                                          int* __restrict__ ids, float* __restrict__ wts, int* __restrict__ counts,
+                                          int* __restrict__ rank, int T) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x, lane = threadIdx.x & 63;
+  int next;
+  const unsigned long long picks = route_token<NMAX>(z, corr, bias, ldz, rule, NE, E, k, ids, wts, t, T, next);
+  next = lane < E && next ? atomicAdd(counts + lane, next) : 0;
+  for (int j = 0; j < k; ++j) {
+    const int r = expert_rank((int)(picks >> (4 * j)) & 15, t < T, E, next);
+    if (t < T) rank[(size_t)t * k + j] = r;
+  }
+}
+
+// The whole routing of at most kOneGroup tokens in ONE workgroup: choice, counts, offsets and expert-major rows.
+// Few tokens are all latency: apart, a fill, the choice, the offsets and the scatter cost 14.3 us (64 tokens, 8 of 10 outputs
+// real, top 2), most of it launches and one dependent atomic in memory per choice and expert; here 6.9 us, the counts in LDS.
+// kOneGroup: 512 tokens take 8.4 us here and 12.3 in three kernels, 1024 take 11.7 to 13.1 and 11.9 (16 outputs, top 8:
+// 30 and 32, 41 and 29): beyond it one CU has too many waves to run one after the other.
+template <int NMAX>
+__global__ void __launch_bounds__(kOneGroup) router_one_group_kernel(const float* __restrict__ z, const float* __restrict__ corr,
+                                                                     const float* __restrict__ bias, int ldz, RouterRule rule,
+                                                                     int NE, int E, int k, int* __restrict__ ids,
+                                                                     float* __restrict__ wts, int* __restrict__ row_off,
+                                                                     int* __restrict__ src, int* __restrict__ row_expert,
+                                                                     int* __restrict__ inv, int T) {
+  __shared__ int counts[NMAX];
+  const int t = threadIdx.x, lane = t & 63;
+  if (t < NMAX) counts[t] = 0;
+  __syncthreads();
+  int next;
+  const unsigned long long picks = route_token<NMAX>(z, corr, bias, ldz, rule, NE, E, k, ids, wts, t, T, next);
+  next = lane < E && next ? atomicAdd(counts + lane, next) : 0;
+  __syncthreads();
+  const int c = lane < E ? counts[lane] : 0;
+  int off = c;  // lane e < NMAX: where expert e's rows end
+#pragma unroll
+  for (int o = 1; o < NMAX; o <<= 1) {
+    const int before = __shfl_up(off, o, 64);
+    if (lane >= o) off += before;
+  }
+  const int rows = __shfl(off, NMAX - 1, 64);
+  next += off - c;
+  if (t <= E) row_off[t] = t == E ? rows : off - c;
+  for (int j = 0; j < k; ++j) {
+    const int x = (int)(picks >> (4 * j)) & 15, row = expert_rank(x, t < T, E, next);
+    if (t < T) inv[t * k + j] = row;
+    if (t < T && row >= 0) src[row] = t, row_expert[row] = x;
+  }
+  for (int r = rows + t; r < T * k; r += blockDim.x) src[r] = 0, row_expert[r] = 0;  // rows of no expert
 }
 
 __global__ void router_offsets_kernel(const int* __restrict__ counts, int E, int* __restrict__ row_off) {
@@ -358,7 +423,10 @@ using namespace lwc;
 
 extern "C" int r32_router_max_outputs() { return 64 * kMaxPerLane; }
 
-// counts must be zero on entry (E ints)
+// Whether a router of these sizes runs in one workgroup: counts is not used then, and src and row_expert need no clearing.
+extern "C" int r32_router_one_group(int T, int NE) { return T <= kOneGroup && NE <= 16; }
+
+// counts, src and row_expert must be zero on entry (E, T k, T k ints) unless r32_router_one_group(T, NE)
 // z rows have leading dimension ldz; corr (added to the scores for the choice only) and bias (added to the logits) may be
 // null; sigmoid, renorm, floor, scale, groups, keep: RouterRule
 extern "C" int r32_router(const float* z, int ldz, const float* corr, const float* bias, int sigmoid, int renorm, float floor,
@@ -369,6 +437,12 @@ extern "C" int r32_router(const float* z, int ldz, const float* corr, const floa
   if (NE > 64 * kMaxPerLane || k < 1 || k > NE || E > NE) return -1;
   if (groups > 1 && (NE % groups != 0 || keep < 1 || keep > groups || k > keep * (NE / groups))) return -1;
   const RouterRule rule{sigmoid, renorm, floor, scale, groups, keep};
+  if (r32_router_one_group(T, NE)) {
+    router_one_group_kernel<16><<<1, (T + 63) / 64 * 64, 0, s>>>(z, corr, bias, ldz, rule, NE, E, k, ids, wts, row_off, src, row_expert,
+                                                                inv, T);
+    LWC_CHECK_LAUNCH();
+    return 0;
+  }
   if (NE <= 16) router_topk_thread_kernel<16><<<(T + 63) / 64, 64, 0, s>>>(z, corr, bias, ldz, rule, NE, E, k, ids, wts, counts, rank, T);
   else if (NE <= 64) router_topk_kernel<1><<<(T + 3) / 4, 256, 0, s>>>(z, corr, bias, ldz, rule, NE, E, k, ids, wts, counts, rank, T);
   else router_topk_kernel<kMaxPerLane><<<(T + 3) / 4, 256, 0, s>>>(z, corr, bias, ldz, rule, NE, E, k, ids, wts, counts, rank, T);

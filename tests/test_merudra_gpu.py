@@ -353,6 +353,29 @@ def test_router_identity_experts_and_correction(gpu, E, I, top, d):
     assert (out.cpu().double() - ref).abs().max() < 2e-5
 
 
+@pytest.mark.parametrize("T", [1, 63, 64, 65, 500, 512, 513])
+@pytest.mark.parametrize("E,NE,top", [(8, 10, 2), (16, 16, 16), (0, 3, 2), (1, 1, 1)])
+def test_router_of_few_tokens(gpu, T, E, NE, top):
+    """Up to 512 tokens are routed by one workgroup: ids and weights are those of a longer batch's rows (bit for bit),
+    the rows of the experts cover every real choice once, and rows of no expert name token 0 and expert 0."""
+    from llm_weighted_consensus_amd.ops import res32
+
+    g = torch.Generator().manual_seed(T + NE)
+    z, corr = torch.randn(1100, NE, generator=g).to(gpu), (torch.randn(NE, generator=g) * 0.1).to(gpu)
+    full = [x.cpu() for x in res32.router(z, corr, E, top, renorm=True)]
+    ids, w, row_off, src, row_expert, inv = (x.cpu() for x in res32.router(z[:T], corr, E, top, renorm=True))
+    assert torch.equal(ids, full[0][:T]) and torch.equal(w, full[1][:T])
+    real = ids.flatten() < E
+    n = int(real.sum())
+    counts = torch.bincount(ids.flatten()[real].long(), minlength=E)[:E]
+    assert torch.equal(row_off.long(), torch.cat([torch.zeros(1, dtype=torch.long), counts.cumsum(0)]))
+    rows = inv[real].long()
+    assert torch.equal(rows.sort().values, torch.arange(n)) and bool((inv[~real] == -1).all())
+    tokens = torch.arange(T).repeat_interleave(top)[real]
+    assert torch.equal(src[rows].long(), tokens) and torch.equal(row_expert[rows], ids.flatten()[real])
+    assert not bool(src[n:].any()) and not bool(row_expert[n:].any())
+
+
 # ------------------------------------------------------------------ the model through the engine
 A = dict(type="attention", heads=4, kv_heads=2, dim=12, every=7, mlp=dict(experts=5, identity=2, top=3, ff=24))
 CONFIGS = {
