@@ -250,6 +250,22 @@ def _time(fn, iters: int = 5, rounds: int = 3) -> float:
     return sorted(ts)[len(ts) // 2]
 
 
+def _time_step(fn, x: torch.Tensor, evict: torch.Tensor, iters: int = 5) -> float:
+    """Mean time of ``fn`` as a step finds its operands: the weights passed through by a read of ``evict``, the rows ``x`` just
+    touched.  (The read also keeps the device busy while the host enqueues the call.)"""
+    marks = []
+    for _ in range(iters):
+        evict.sum()
+        x.clone()
+        s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        s.record()
+        fn()
+        e.record()
+        marks.append((s, e))
+    torch.cuda.synchronize()
+    return sum(s.elapsed_time(e) for s, e in marks) / iters * 1e3
+
+
 def tune(x: torch.Tensor, w: torch.Tensor, epi: str = "plain", block: int = 0, ws=None,
          bucket: bool = False) -> Optional[str]:
     """Time every applicable backend for this (M, N, K, epi) and record the choice (no-op under graph
@@ -317,12 +333,20 @@ def _tune(x, w, epi, block, ws, M, N, K, key, lo=None) -> str:
                 continue  # a backend must take the whole bucket
             fns.append(run(b, x[:lo]))
         runs[b] = fns
+    # A decode step reads each layer's weight from memory (the last-level cache holds 256 MB, a step's weights are more);
+    # repeated calls find it cached, and that favours the cores that read it more often: 4096 rows x 6144 x 4096 took
+    # gemm2w 164 us against 169 of gemm8p there, and 180 against 172 in the step.
+    try:
+        evict = torch.ones(1 << 27, device=x.device)
+    except torch.cuda.OutOfMemoryError:
+        evict = None
+    rows = (x, x if lo is None else x[:lo])
     ts = {b: [] for b in runs}
     # 5 interleaved rounds of 5 calls: o and gate|up are within 1-3 % between backends, and 3 x 3 calls
     # flipped the choice from run to run (profiles/bench_r64_round3.md); runs before graph capture only
     for _ in range(5):
         for b, fns in runs.items():
-            ts[b].append(sum(_time(fn, iters=5, rounds=1) for fn in fns))
+            ts[b].append(sum(_time(fn, iters=5, rounds=1) if evict is None else _time_step(fn, r, evict) for fn, r in zip(fns, rows)))
     med = {b: sorted(t)[len(t) // 2] for b, t in ts.items()}
     TIMINGS[key] = med
     own = min((b for b in med if b != "blas"), key=lambda b: med[b], default=None)
