@@ -26,8 +26,8 @@ down projections (:func:`linear_add_`), into their epilogue.  None wins everywhe
 (``profiles/gemm4w.md``), so the choice is made per (M, N, K, epilogue) by timing every applicable
 backend on the device, once, before a decode bucket's hipGraph is captured (:meth:`LlamaModel.tune_gemms`);
 a hand-written core is taken when it is at least as fast as the library (``OWN_MARGIN``, 0); for a decode bucket
-the engine then A/Bs whole captured steps (planner / all-library / all-own, ``LlamaModel.step_plans``).  Untuned shapes (prefill,
-encode) use hipBLASLt.  ``LWC_GEMM=blas|g8|g4|g4n192`` forces one backend (``auto`` = measured, the default).
+the engine then A/Bs whole captured steps (planner / all-library / all-own, ``LlamaModel.step_plans``).  Untuned shapes (prefill)
+use hipBLASLt, but for few rows (:func:`_few_rows`).  ``LWC_GEMM=blas|g8|g4|g4n192`` forces one backend (``auto`` = measured, the default).
 """
 from __future__ import annotations
 
@@ -76,6 +76,37 @@ def choice(M: int, N: int, K: int, epi: str) -> str:
     return "blas"
 
 
+def _few_rows(M: int, N: int, K: int, epi: str) -> str:
+    """The backend of a shape that no one tuned (prefill: a batch of prompts' last layer runs on their last tokens only, and
+    short prompts on few rows everywhere), where its rows are few and the weight's read bounds it.  us, weights from memory,
+    library -> here: gate|up of 28672 x 4096, 5 rows 67 -> 46 (the library needs a SwiGLU pass after it), 64 rows 55 -> 51,
+    16384 x 2048 19.4 -> 16.8; 4096 x 4096 5 rows 15.4 -> 8.7, 3072 x 2048 11.1 -> 5.7, 64 rows of 4096 x 14336 39 -> 28,
+    of 6144 x 4096 17.5 -> 16.6.  Beyond these sizes both are within a few per cent, or the library is ahead (10240 x 8192, 8
+    rows: 35 and 41 to 46; 57344 x 8192, 48 rows: 170 and 182); below, they are not of a size to matter."""
+    size = N * K
+    if epi == "swiglu":
+        return "g2" if M <= 64 and 1 << 25 <= size <= 1 << 27 else "blas"
+    if M <= 16 and K <= 4096 and 1 << 22 <= size <= 1 << 24:
+        return "gv"
+    return "g2" if 32 < M <= 64 and 1 << 24 <= size <= 1 << 26 else "blas"
+
+
+def _backend(x: torch.Tensor, w: torch.Tensor, epi: str, ws):
+    """(backend, its workspace) of a call: as tuned or forced with the caller's, else :func:`_few_rows` with the current
+    stream's own (a model's workspace belongs to the stream of its steps).  The library keeps what only it takes (a gradient
+    to record, operands off 16 bytes, a strided weight) and, untuned, what is captured."""
+    (M, K), N = x.shape, w.shape[0]
+    b = choice(M, N, K, epi)
+    if M > 64 or b != "blas" or MODE != "auto" or (M, N, K, epi) in _CHOICE or (N, K, epi) in _BUCKETS:
+        return b, ws
+    own = _few_rows(M, N, K, epi)
+    if own == "blas" or not (x.is_cuda and w.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous()
+                             and x.stride(0) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0) or \
+            (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)) or torch.cuda.is_current_stream_capturing():
+        return b, ws
+    return own, None
+
+
 def _g8_ok(N: int, K: int, epi: str) -> bool:
     return K % 64 == 0 and N % (64 if epi == "swiglu" else 8) == 0
 
@@ -111,7 +142,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, ws=None) -> torch.Tensor:
     """x [M, K] . w[N, K]^T -> [M, N] bf16 on the chosen backend."""
     M, K = x.shape
     N = w.shape[0]
-    b = choice(M, N, K, "plain")
+    b, ws = _backend(x, w, "plain", ws)
     if _own_ok(b, x, N, K, "plain"):
         return _own(b, x, w, ws)
     return F.linear(x, w)
@@ -124,8 +155,8 @@ def linear_add_(x: torch.Tensor, w: torch.Tensor, acc: torch.Tensor, ws=None) ->
     lane).  Saves the separate residual add's read and write of the [M, N] projection output."""
     M, K = x.shape
     N = w.shape[0]
-    b = choice(M, N, K, "residual")
-    if _own_ok(b, x, N, K, "residual") and acc.is_contiguous() and (b != "g2" or acc.data_ptr() % 16 == 0):
+    b, ws = _backend(x, w, "residual", ws)
+    if _own_ok(b, x, N, K, "residual") and acc.is_contiguous() and (b not in ("g2", "gv") or acc.data_ptr() % 16 == 0):
         return _own(b, x, w, ws, residual=acc, out=acc)
     return acc.addmm_(x, w.t())
 
@@ -135,7 +166,7 @@ def swiglu(x: torch.Tensor, w_gu: torch.Tensor, block: int, ws=None) -> torch.Te
     (block 0) or interleaved in blocks of ``block`` (ops.swiglu_interleave; required by g8)."""
     M, K = x.shape
     N = w_gu.shape[0]
-    b = choice(M, N, K, "swiglu")
+    b, ws = _backend(x, w_gu, "swiglu", ws)
     if block == 32 and _own_ok(b, x, N, K, "swiglu"):
         return _own(b, x, w_gu, ws, swiglu=True)
     return silu_mul(F.linear(x, w_gu), block=block)

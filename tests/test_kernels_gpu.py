@@ -1625,6 +1625,38 @@ def test_skinny_gemm_any_k(gpu, M, N, K, epi):
     torch.testing.assert_close(out.double(), ref, rtol=2 ** -8, atol=2e-5)
 
 
+@pytest.mark.parametrize("epi,N,K,rows", [("swiglu", 8192, 4096, {1: "g2", 64: "g2", 65: "blas"}),
+                                          ("swiglu", 8128, 4096, {8: "blas"}),
+                                          ("residual", 4096, 1024, {1: "gv", 16: "gv", 17: "blas"}),
+                                          ("plain", 4096, 4096, {16: "gv", 32: "blas", 33: "g2", 64: "g2", 65: "blas"}),
+                                          ("plain", 4160, 4096, {16: "blas", 33: "g2"}),
+                                          ("residual", 4096, 16384, {16: "blas", 64: "g2"}),
+                                          ("residual", 4104, 16384, {64: "blas"})])
+def test_untuned_gemms_of_few_rows(gpu, epi, N, K, rows):
+    """The edges of the rule for shapes that no one tuned, and its results against fp64 of the same operands (bounds: one bf16
+    rounding, doubled; the library's SwiGLU rounds gate and up before it, three; fp32 sums)."""
+    from llm_weighted_consensus_amd import ops
+    from llm_weighted_consensus_amd.ops import gemm_plan
+
+    g = torch.Generator().manual_seed(N)
+    W = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).to(gpu)
+    for M, core in rows.items():
+        A, C = (torch.randn(M, n, generator=g).to(torch.bfloat16).to(gpu) for n in (K, N))
+        if (M, N, K, epi) not in gemm_plan._CHOICE and (N, K, epi) not in gemm_plan._BUCKETS and gemm_plan.MODE == "auto":
+            assert gemm_plan._backend(A, W, epi, None)[0] == core
+            assert gemm_plan._backend(A, W.t().contiguous().t(), epi, None)[0] == "blas"
+        ref = A.double() @ W.double().t()
+        if epi == "swiglu":
+            v = ref.view(M, N // 64, 2, 32)
+            ref = (torch.nn.functional.silu(v[:, :, 0]) * v[:, :, 1]).reshape(M, N // 2)
+            out = gemm_plan.swiglu(A, W, 32)
+        elif epi == "residual":
+            ref, out = ref + C.double(), gemm_plan.linear_add_(A, W, C)
+        else:
+            out = gemm_plan.linear(A, W)
+        torch.testing.assert_close(out.double(), ref, rtol=2 ** -6 if epi == "swiglu" else 2 ** -8, atol=2e-4)
+
+
 @pytest.mark.parametrize("tile,splits", [(0, 1), (1, 1), (2, 1), (3, 1), (3, 5), (-1, 0)])
 @pytest.mark.parametrize("M,N,K", [(1, 64, 64), (64, 8, 128), (129, 200, 320), (192, 384, 192), (515, 704, 1024), (61, 1024, 4096),
                                    (1500, 2304, 448)])
