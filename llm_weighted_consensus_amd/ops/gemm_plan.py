@@ -27,7 +27,7 @@ down projections (:func:`linear_add_`), into their epilogue.  None wins everywhe
 backend on the device, once, before a decode bucket's hipGraph is captured (:meth:`LlamaModel.tune_gemms`);
 a hand-written core is taken when it is at least as fast as the library (``OWN_MARGIN``, 0); for a decode bucket
 the engine then A/Bs whole captured steps (planner / all-library / all-own, ``LlamaModel.step_plans``).  Untuned shapes (prefill)
-use hipBLASLt, but for few rows (:func:`_few_rows`).  ``LWC_GEMM=blas|g8|g4|g4n192`` forces one backend (``auto`` = measured, the default).
+use hipBLASLt, but where :func:`_untuned` names a core.  ``LWC_GEMM=blas|g8|g4|g4n192`` forces one backend (``auto`` = measured, the default).
 """
 from __future__ import annotations
 
@@ -76,15 +76,24 @@ def choice(M: int, N: int, K: int, epi: str) -> str:
     return "blas"
 
 
-def _few_rows(M: int, N: int, K: int, epi: str) -> str:
-    """The backend of a shape that no one tuned (prefill: a batch of prompts' last layer runs on their last tokens only, and
-    short prompts on few rows everywhere), where its rows are few and the weight's read bounds it.  us, weights from memory,
+def _untuned(M: int, N: int, K: int, epi: str) -> str:
+    """The backend of a shape that no one tuned.
+
+    Many rows of a gate|up projection: the library needs a SwiGLU pass over its [M, N] result, gemm8p none.  us, 28672 x 4096 and
+    16384 x 2048, library -> gemm8p: 5000 rows 1013 -> 921 and 301 -> 270, 7000 rows 1296 -> 1242 and 412 -> 372, 16384 rows
+    2893 -> 2855 and 936 -> 842.  Fewer rows: a last round of half empty tiles decides, either way (4500: 817 and 840, 2200:
+    416 and 459, 3333: 706 and 622).  8192 x 1024, 4700 rows: 120 -> 104; 1024 x 512 21 and 36, 57344 x 8192 3281 and 3239.
+
+    Few rows (prefill: a batch of prompts' last layer runs on their last tokens only, and short prompts on few rows everywhere):
+    the weight's read bounds them.  us, weights from memory,
     library -> here: gate|up of 28672 x 4096, 5 rows 67 -> 46 (the library needs a SwiGLU pass after it), 64 rows 55 -> 51,
     16384 x 2048 19.4 -> 16.8; 4096 x 4096 5 rows 15.4 -> 8.7, 3072 x 2048 11.1 -> 5.7, 64 rows of 4096 x 14336 39 -> 28,
     of 6144 x 4096 17.5 -> 16.6.  Beyond these sizes both are within a few per cent, or the library is ahead (10240 x 8192, 8
     rows: 35 and 41 to 46; 57344 x 8192, 48 rows: 170 and 182); below, they are not of a size to matter."""
     size = N * K
     if epi == "swiglu":
+        if M > 4608:
+            return "g8" if 1 << 23 <= size <= 1 << 28 and M * N < 1 << 30 else "blas"   # (32-bit byte offsets)
         return "g2" if M <= 64 and 1 << 25 <= size <= 1 << 27 else "blas"
     if M <= 16 and K <= 4096 and 1 << 22 <= size <= 1 << 24:
         return "gv"
@@ -92,16 +101,16 @@ def _few_rows(M: int, N: int, K: int, epi: str) -> str:
 
 
 def _backend(x: torch.Tensor, w: torch.Tensor, epi: str, ws):
-    """(backend, its workspace) of a call: as tuned or forced with the caller's, else :func:`_few_rows` with the current
+    """(backend, its workspace) of a call: as tuned or forced with the caller's, else :func:`_untuned` with the current
     stream's own (a model's workspace belongs to the stream of its steps).  The library keeps what only it takes (a gradient
     to record, operands off 16 bytes, a strided weight) and, untuned, what is captured."""
     (M, K), N = x.shape, w.shape[0]
     b = choice(M, N, K, epi)
-    if M > 64 or b != "blas" or MODE != "auto" or (M, N, K, epi) in _CHOICE or (N, K, epi) in _BUCKETS:
+    if b != "blas" or MODE != "auto" or (M, N, K, epi) in _CHOICE or (N, K, epi) in _BUCKETS:
         return b, ws
-    own = _few_rows(M, N, K, epi)
+    own = _untuned(M, N, K, epi)
     if own == "blas" or not (x.is_cuda and w.is_cuda and x.dtype == w.dtype == torch.bfloat16 and w.is_contiguous()
-                             and x.stride(0) % 8 == 0 and (x.data_ptr() | w.data_ptr()) % 16 == 0) or \
+                             and x.stride(0) % 8 == 0 and M * x.stride(0) < 1 << 30 and (x.data_ptr() | w.data_ptr()) % 16 == 0) or \
             (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)) or torch.cuda.is_current_stream_capturing():
         return b, ws
     return own, None

@@ -1627,6 +1627,7 @@ def test_skinny_gemm_any_k(gpu, M, N, K, epi):
 
 @pytest.mark.parametrize("epi,N,K,rows", [("swiglu", 8192, 4096, {1: "g2", 64: "g2", 65: "blas"}),
                                           ("swiglu", 8128, 4096, {8: "blas"}),
+                                          ("swiglu", 8192, 1024, {64: "blas", 4608: "blas", 4609: "g8", 5001: "g8"}),
                                           ("residual", 4096, 1024, {1: "gv", 16: "gv", 17: "blas"}),
                                           ("plain", 4096, 4096, {16: "gv", 32: "blas", 33: "g2", 64: "g2", 65: "blas"}),
                                           ("plain", 4160, 4096, {16: "blas", 33: "g2"}),
