@@ -25,6 +25,7 @@
 // blocks are read ONCE per tile instead of once per sequence: for N candidates of one prompt this
 // removes (N-1)/N of the prompt's KV traffic and finally uses the MFMA rows; each sequence's own
 // blocks follow in the same launch, softmax states merged in registers.
+#include <algorithm>
 #include <cstdlib>
 
 #include "common.h"
@@ -66,6 +67,7 @@ struct DecodeParams {
   const float* rope_cos;
   const float* rope_sin;
   const int* positions;
+  int* counts = nullptr;  // [B, Hkv] finished splits, zero between calls: the last split of a sequence's KV head adds them up
 };
 
 // K and V registers of one PAIR of 16-token blocks for one wave (K: 8 x 16 B, V: 16 x 8 B per lane).
@@ -296,9 +298,35 @@ LWC_DEVICE void load_q(short8 (&qf)[4], const DecodeParams& p, int row_seq0, int
   }
 }
 
-// blockIdx.x = sequence.  4 waves split the sequence's block pairs and combine through LDS: the
-// long-context / small-batch path.
-__global__ void __launch_bounds__(256)
+// out[bh] = sum_s 2^(lse_s - LSE) o_s / sum_s 2^(lse_s - LSE) over the first n of bh's S splits, in their order: one wave, two
+// dims a lane.  (Loads of device scope: the sums may come from workgroups of the same launch.)
+LWC_DEVICE void split_sum(const float* part_o, const float* part_lse, bf16_t* out, size_t bh, int S, int n, int lane) {
+  const float* lse = part_lse + bh * S;
+  float M = -INFINITY;
+  for (int s = 0; s < n; ++s) M = fmaxf(M, __hip_atomic_load(lse + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+  float L = 0.f, x = 0.f, y = 0.f;
+  if (M != -INFINITY) {
+#pragma unroll 4
+    for (int s = 0; s < n; ++s) {
+      const float f = exp2f(__hip_atomic_load(lse + s, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - M);
+      const unsigned long long v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(part_o + (bh * S + s) * kD) + lane,
+                                                     __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      L += f;
+      x += f * __uint_as_float((uint32_t)v);
+      y += f * __uint_as_float((uint32_t)(v >> 32));
+    }
+  }
+  const float inv = L > 0.f ? 1.f / L : 0.f;
+  reinterpret_cast<uint32_t*>(out + bh * kD)[lane] = pack_bf16x2(x * inv, y * inv);
+}
+
+// blockIdx.x = sequence.  W waves split the sequence's block pairs and combine through LDS: the long-context / small-batch
+// path.  A sequence takes as many of the grid's splits as have a pair for every wave, so that most contexts need one workgroup
+// and its waves meet in LDS (a second kernel that adds splits up takes 5 to 7 us of a step, whatever the batch; the last split
+// to finish doing it, about as much behind the longest sequence); with counts the splits there are meet in this launch.
+// Dynamic LDS: [W][G] running maxima and sums, [W][G][kD + 4] output rows.
+template <int W>
+__global__ void __launch_bounds__(64 * W, 4)
     paged_decode_kernel(DecodeParams p, const int* __restrict__ block_tables, const int* __restrict__ ctx_lens) {
   const int item = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
   // wid through readfirstlane: the compiler then knows everything derived from it (sequence, block
@@ -310,66 +338,105 @@ __global__ void __launch_bounds__(256)
   const int nrows = p.G;
   const int ctx = ctx_lens[item];
   const int nblk_total = (ctx + kBS - 1) / kBS;
-  const int per_split = (nblk_total + p.num_splits - 1) / p.num_splits;
+  const int per_split = max((nblk_total + p.num_splits - 1) / p.num_splits, 2 * W);
+  const int splits = max(1, (nblk_total + per_split - 1) / per_split);
+  if (split >= splits) return;
   const int blk_begin = split * per_split;
   const int blk_end = min(nblk_total, blk_begin + per_split);
   const int* bt = block_tables + (size_t)item * p.max_blocks;
 
-  short8 qf[4];
-  load_q<false>(qf, p, item, nrows, kvh, r16, g);
+  // q goes through LDS, rotated once by the last wave while the others' first pairs are on their way, and is read from there for
+  // every pair: held in registers it took the kernel past the 128 that two workgroups of eight waves per CU allow
+  __shared__ uint4v s_q[4][64];
   const float sl2 = p.scale * kLog2e;
+  int pair = blk_begin + 2 * wid;
+  PairRegs r;
+  if (wid == W - 1) {  // (ahead of the wave's own pair, which would hold q and its angles back: 9.5 -> 7 us for one sequence)
+    short8 qf[4];
+    load_q<false>(qf, p, item, nrows, kvh, r16, g);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) s_q[s][lane] = __builtin_bit_cast(uint4v, qf[s]);
+  }
+  if (pair < blk_end) load_pair(r, p, bt, kvh, pair, pair + 1 < blk_end, r16, g, ctx);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 
   float4v o[8];
 #pragma unroll
   for (int n = 0; n < 8; ++n) o[n] = float4v{0.f, 0.f, 0.f, 0.f};
   float m = -1e30f, l = 0.f;  // running max / sum (log2 domain) for row r16
 
-  for (int pair = blk_begin + 2 * wid; pair < blk_end; pair += 2 * kWaves) {
-    PairRegs r;
-    const bool hasB = pair + 1 < blk_end;
-    load_pair(r, p, bt, kvh, pair, hasB, r16, g, ctx);
-    attend_pair(r, pair, hasB, ctx, qf, sl2, g, o, m, l);
+  while (pair < blk_end) {
+    int at = lane;
+    asm volatile("" : "+v"(at));  // (read here, not kept)
+    short8 qf[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) qf[s] = __builtin_bit_cast(short8, s_q[s][at]);
+    attend_pair(r, pair, pair + 1 < blk_end, ctx, qf, sl2, g, o, m, l);
+    pair += 2 * W;
+    if (pair < blk_end) load_pair(r, p, bt, kvh, pair, pair + 1 < blk_end, r16, g, ctx);
   }
 
-  // ---- combine the 4 waves through LDS ----
-  __shared__ float s_m[kWaves][16], s_l[kWaves][16];
-  __shared__ float s_o[kWaves][16][kD + 4];
-  if (g == 0) {
-    s_m[wid][r16] = m;
-    s_l[wid][r16] = l;
+  // ---- combine the waves through LDS: wave w takes rows w, w + W, ..., a lane two dims ----
+  extern __shared__ __attribute__((aligned(16))) float s_mem[];
+  constexpr int kRow = kD + 4;
+  float *s_m = s_mem, *s_l = s_mem + W * nrows, *s_o = s_mem + 2 * W * nrows;
+  if (g == 0 && r16 < nrows) {
+    s_m[wid * nrows + r16] = m;
+    s_l[wid * nrows + r16] = l;
   }
 #pragma unroll
-  for (int n = 0; n < 8; ++n)
+  for (int r = 0; r < 4; ++r)
+    if (4 * g + r < nrows) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) s_o[wid][4 * g + r][odim(n, r16)] = o[n][r];
+      for (int n = 0; n < 8; ++n) s_o[(wid * nrows + 4 * g + r) * kRow + odim(n, r16)] = o[n][r];
+    }
   __syncthreads();
-  // thread t: row h = t / 16 (< nrows), dims 8*(t%16) .. +8
-  const int t = threadIdx.x;
-  const int h = t >> 4, dc = (t & 15) * 8;
-  if (h < nrows) {
-    const int hq = kvh * p.G + h;
+  typedef unsigned long long u64;
+  for (int h = wid; h < nrows; h += W) {
+    const size_t bh = (size_t)item * p.Hq + kvh * p.G + h;
     float M = -1e30f;
-    for (int w = 0; w < kWaves; ++w) M = fmaxf(M, s_m[w][h]);
-    float L = 0.f, acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (int w = 0; w < kWaves; ++w) {
-      const float f = exp2f(s_m[w][h] - M);
-      L += f * s_l[w][h];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[j] += f * s_o[w][h][dc + j];
+    for (int w = 0; w < W; ++w) M = fmaxf(M, s_m[w * nrows + h]);
+    float L = 0.f, x = 0.f, y = 0.f;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      const float f = exp2f(s_m[w * nrows + h] - M);
+      const float2 v = *reinterpret_cast<const float2*>(s_o + (w * nrows + h) * kRow + 2 * lane);
+      L += f * s_l[w * nrows + h];
+      x += f * v.x;
+      y += f * v.y;
     }
     const float inv = L > 0.f ? 1.f / L : 0.f;
-    if (p.num_splits == 1) {
-      float outv[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) outv[j] = acc[j] * inv;
-      *reinterpret_cast<uint4v*>(p.out + ((size_t)item * p.Hq + hq) * kD + dc) = pack8(outv);
-    } else {
-      float* po = p.part_o + (((size_t)item * p.Hq + hq) * p.num_splits + split) * kD + dc;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) po[j] = acc[j] * inv;
-      if ((t & 15) == 0)
-        p.part_lse[((size_t)item * p.Hq + hq) * p.num_splits + split] = L > 0.f ? M + log2f(L) : -INFINITY;
+    x *= inv;
+    y *= inv;
+    if (splits == 1) {
+      reinterpret_cast<uint32_t*>(p.out + bh * kD)[lane] = pack_bf16x2(x, y);
+      continue;
     }
+    // (read by another workgroup of this launch, or by the reduction's: stores of device scope, past the caches of this XCD)
+    const size_t at = bh * p.num_splits + split;
+    __hip_atomic_store(reinterpret_cast<u64*>(p.part_o + at * kD) + lane,
+                       (u64)__float_as_uint(x) | (u64)__float_as_uint(y) << 32, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (lane == 0)
+      __hip_atomic_store(p.part_lse + at, L > 0.f ? M + log2f(L) : -INFINITY, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (splits == 1 || !p.counts) return;
+  // ---- the last split to finish adds them all up, in their order ----
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this split's sums have arrived
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int* n = p.counts + (size_t)item * p.Hkv + kvh;
+    const bool last = __hip_atomic_fetch_add(n, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == splits - 1;
+    if (last) __hip_atomic_store(n, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    s_mem[0] = last ? 1.f : 0.f;
+  }
+  __syncthreads();
+  if (s_mem[0] == 0.f) return;
+  for (int h = wid; h < nrows; h += W) {
+    const size_t bh = (size_t)item * p.Hq + kvh * p.G + h;
+    split_sum(p.part_o, p.part_lse, p.out, bh, p.num_splits, splits, lane);
   }
 }
 
@@ -734,24 +801,20 @@ __global__ void __launch_bounds__(kCWaves * 64)
   }
 }
 
-// Combine split-K partials: out[b, hq, :] = sum_s 2^(lse_s - LSE) o_s / sum_s 2^(lse_s - LSE)
-__global__ void __launch_bounds__(128) paged_decode_reduce_kernel(const float* __restrict__ part_o,
-                                                                  const float* __restrict__ part_lse,
-                                                                  bf16_t* __restrict__ out, int S) {
-  const int bh = blockIdx.x;  // b * Hq + hq
-  const int d = threadIdx.x;  // 0..127
-  const float* lse = part_lse + (size_t)bh * S;
-  float M = -INFINITY;
-  for (int s = 0; s < S; ++s) M = fmaxf(M, lse[s]);
-  float L = 0.f, acc = 0.f;
-  if (M != -INFINITY) {
-    for (int s = 0; s < S; ++s) {
-      const float f = exp2f(lse[s] - M);
-      L += f;
-      acc += f * part_o[((size_t)bh * S + s) * kD + d];
-    }
+// The splits of the wave-per-item kernel, and those of paged_decode_kernel<W> where the caller has no counters (there a
+// sequence has as many as hold a pair per wave, and one has written its output already).  One wave per (sequence, head).
+__global__ void __launch_bounds__(256) paged_decode_reduce_kernel(const float* __restrict__ part_o, const float* __restrict__ part_lse,
+                                                                  bf16_t* __restrict__ out, const int* __restrict__ ctx_lens, int rows,
+                                                                  int Hq, int S, int waves) {
+  const int bh = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // b * Hq + hq
+  if (bh >= rows) return;
+  int n = S;
+  if (waves > 1) {
+    const int nblk = (ctx_lens[bh / Hq] + kBS - 1) / kBS, per = max((nblk + S - 1) / S, 2 * waves);
+    n = max(1, (nblk + per - 1) / per);
+    if (n == 1) return;
   }
-  out[(size_t)bh * kD + d] = f2bf(L > 0.f ? acc / L : 0.f);
+  split_sum(part_o, part_lse, out, bh, S, n, threadIdx.x & 63);
 }
 
 }  // namespace lwc
@@ -767,7 +830,8 @@ extern "C" int lwc_set_decode_wave_min_items(int n) {
 extern "C" int lwc_paged_decode(const void* q, int q_stride, const void* kc, const void* vc, const int* block_tables,
                                 const int* ctx_lens, void* out, float* part_o, float* part_lse, int B, int Hq,
                                 int Hkv, int D, int BS, int max_blocks, int num_splits, float scale,
-                                const float* rope_cos, const float* rope_sin, const int* positions, hipStream_t s) {
+                                const float* rope_cos, const float* rope_sin, const int* positions, int* counts,
+                                hipStream_t s) {
   using namespace lwc;
   if (D != kD || BS != kBS || Hq % Hkv != 0 || Hq / Hkv > 16 || num_splits < 1) return -1;
   if (num_splits > 1 && (!part_o || !part_lse)) return -2;
@@ -775,14 +839,38 @@ extern "C" int lwc_paged_decode(const void* q, int q_stride, const void* kc, con
   DecodeParams p{(const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, block_tables, ctx_lens, (bf16_t*)out,
                  part_o, part_lse, q_stride, Hq, Hkv, Hq / Hkv, max_blocks, num_splits, scale,
                  rope_cos, rope_sin, positions};
+  int waves = 1;
   if ((long)B * Hkv * num_splits >= g_wave_min_items) {
     const int items = B * num_splits;
     paged_decode_wave_kernel<<<dim3((items + kWaves - 1) / kWaves, Hkv), 256, 0, s>>>(p, items, block_tables,
                                                                                       ctx_lens);
   } else {
-    paged_decode_kernel<<<dim3(B, Hkv, num_splits), 256, 0, s>>>(p, block_tables, ctx_lens);
+    // As many waves per (sequence, KV head) as num_splits workgroups of four, in workgroups of up to 16, and further workgroups
+    // while there are fewer than CUs; of eight where the CUs have room for half the splits (a CU reads 50 to 60 GB/s, and one
+    // sequence of 2000 keys took 14.4 us in 16s, 13.5 in 16 splits of four).  Against splits of four waves and a second kernel
+    // (us, 32 heads on 8): 1 x 247 keys 12.2 -> 9, 8 x 900 19.0 -> 16.1, 32 x 900 30.0 -> 25.6, 64 x 60 13.0 -> 8.5, 64 x 900
+    // 53.2 -> 45.5, 128 x 600 (one split) 64.3 -> 61.1.
+    const int room = 256 / std::max(1, B * Hkv);
+    waves = num_splits == 1 ? 4 : num_splits == 2 || room >= (num_splits + 1) / 2 ? 8 : 16;
+    p.num_splits = std::min(num_splits, std::max((4 * num_splits + waves - 1) / waves, room));
+    p.counts = p.num_splits > 1 ? counts : nullptr;
+    num_splits = p.num_splits;
+    const dim3 grid(B, Hkv, p.num_splits);
+    const int lds = waves * p.G * (2 + kD + 4) * 4;
+    if (waves == 4) paged_decode_kernel<4><<<grid, 256, lds, s>>>(p, block_tables, ctx_lens);
+    else if (waves == 8) {
+      static const hipError_t attr = hipFuncSetAttribute((const void*)paged_decode_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, 8 * 16 * 134 * 4);
+      (void)attr;
+      paged_decode_kernel<8><<<grid, 512, lds, s>>>(p, block_tables, ctx_lens);
+    } else {
+      static const hipError_t attr = hipFuncSetAttribute((const void*)paged_decode_kernel<16>, hipFuncAttributeMaxDynamicSharedMemorySize, 16 * 16 * 134 * 4);
+      (void)attr;
+      paged_decode_kernel<16><<<grid, 1024, lds, s>>>(p, block_tables, ctx_lens);
+    }
+    if (p.counts) return (int)hipGetLastError();
   }
-  if (num_splits > 1) paged_decode_reduce_kernel<<<B * Hq, kD, 0, s>>>(part_o, part_lse, (bf16_t*)out, num_splits);
+  if (num_splits > 1)
+    paged_decode_reduce_kernel<<<(B * Hq + 3) / 4, 256, 0, s>>>(part_o, part_lse, (bf16_t*)out, ctx_lens, B * Hq, Hq, num_splits, waves);
   return (int)hipGetLastError();
 }
 

@@ -6,6 +6,8 @@
 #include <c10/hip/HIPStream.h>
 #include <hip/hip_runtime.h>
 
+#include "step_fuse_args.h"
+
 extern "C" {
 int lwc_rmsnorm(const void*, void*, const void*, void*, int, int, float, hipStream_t);
 int lwc_rmsnorm_quant_fp8(const void*, void*, const void*, void*, int, int, float, void*, float*, hipStream_t);
@@ -14,10 +16,11 @@ int lwc_rope_kv_write(void*, const int*, const int*, const float*, const float*,
                       int, int, hipStream_t);
 int lwc_silu_mul(const void*, void*, int, int, int, hipStream_t);
 int lwc_embedding_gather(const void*, const int*, void*, int, int, int, hipStream_t);
+int lwc_embedding_step(const void*, const int*, void*, float*, int*, int, int, int, int, hipStream_t);
 int lwc_kv_block_copy(void*, const int*, int, int, int, long long, hipStream_t);
 int lwc_kv_gather(const void*, const void*, const long long*, void*, void*, int, int, int, int, hipStream_t);
 int lwc_paged_decode(const void*, int, const void*, const void*, const int*, const int*, void*, float*, float*, int,
-                     int, int, int, int, int, int, float, const float*, const float*, const int*, hipStream_t);
+                     int, int, int, int, int, int, float, const float*, const float*, const int*, int*, hipStream_t);
 int lwc_set_decode_wave_min_items(int);
 int lwc_paged_decode_cascade(const void*, int, const void*, const void*, const int*, const int*, const int*, int, void*,
                              int, int, int, int, int, float, const float*, const float*, const int*, void*, void*, int, hipStream_t);
@@ -27,11 +30,13 @@ int lwc_grouped_gemm(const void*, const void*, void*, const int*, const float*, 
 int lwc_gemm8p(const void*, const void*, void*, const void*, float*, int*, int, int, int, int, int, int, hipStream_t);
 int lwc_gemm8p_slots();
 void lwc_gemm2w_plan(int, int, int, int, long long, int*, int*);
-int lwc_gemm2w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, int, float*, int*, hipStream_t);
+int lwc_gemm2w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, int, float*, int*,
+               const lwc::RowSumsq*, const lwc::RopeKV*, hipStream_t);
 int lwc_gemm4w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, float*, int, int, int,
                float, int, int, int, int, float*, int*, hipStream_t);
 int lwc_rms_rowsumsq(const void*, float*, int, int, hipStream_t);
-int lwc_skinny_gemm(const void*, const void*, void*, const void*, int, int, int, int, int, int, hipStream_t);
+int lwc_skinny_gemm(const void*, const void*, void*, const void*, int, int, int, int, int, int, const lwc::RowSumsq*,
+                    const lwc::RopeKV*, hipStream_t);
 int lwc_gemm8g_fp8(const void*, const void*, void*, const int*, const int*, const float*, const float*, int, int, int,
                    int, int, int, int, int, int, const void*, void*, int, int, hipStream_t);
 int lwc_gemm8g_bf16(const void*, const void*, void*, const int*, const int*, int, int, int, int, int, int, int, int, int,
@@ -234,6 +239,20 @@ void embedding(const at::Tensor& table, const at::Tensor& ids, at::Tensor& out) 
            "embedding");
 }
 
+// The same for a decode step: ss [T, 4] fp32, each row's sum of squares in four partials; counts [T, per] int32, cleared
+void embedding_step(const at::Tensor& table, const at::Tensor& ids, at::Tensor& out, at::Tensor& ss, at::Tensor& counts) {
+  CHECK_BF16(table); CHECK_BF16(out); CHECK_CONTIG(table); CHECK_CONTIG(out);
+  CHECK_GPU(ids); CHECK_DTYPE(ids, at::kInt);
+  CHECK_GPU(ss); CHECK_DTYPE(ss, at::kFloat); CHECK_CONTIG(ss);
+  CHECK_GPU(counts); CHECK_DTYPE(counts, at::kInt); CHECK_CONTIG(counts);
+  const int T = (int)ids.numel(), d = (int)table.size(1);
+  TORCH_CHECK(out.numel() == (int64_t)T * d && ss.numel() == (int64_t)T * 4 && counts.dim() == 2 && counts.size(0) == T,
+              "embedding_step: output shapes");
+  CHECK_RC(lwc_embedding_step(table.data_ptr(), ids.data_ptr<int>(), out.data_ptr(), ss.data_ptr<float>(), counts.data_ptr<int>(),
+                              (int)counts.size(1), T, d, (int)table.size(0), cur_stream()),
+           "embedding_step");
+}
+
 void kv_gather(const at::Tensor& kc, const at::Tensor& vc, const at::Tensor& slots, at::Tensor& ko, at::Tensor& vo) {
   // kc [NB, Hkv, BS, D], vc [NB, Hkv, BS/4, D, 4] (one layer), slots [n] int64 (< NB*BS, checked by the
   // caller's block manager), ko/vo [n, Hkv*D] contiguous bf16
@@ -264,8 +283,9 @@ void paged_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Tens
                   const at::Tensor& block_tables, const at::Tensor& ctx_lens, at::Tensor& out,
                   const c10::optional<at::Tensor>& part_o, const c10::optional<at::Tensor>& part_lse,
                   int64_t num_splits, double scale, const c10::optional<at::Tensor>& rope_cos,
-                  const c10::optional<at::Tensor>& rope_sin, const c10::optional<at::Tensor>& positions) {
-  // q: [B, >= Hq*D] with row stride; out: [B, Hq, D]
+                  const c10::optional<at::Tensor>& rope_sin, const c10::optional<at::Tensor>& positions,
+                  const c10::optional<at::Tensor>& counts) {
+  // q: [B, >= Hq*D] with row stride; out: [B, Hq, D]; counts [B, Hkv], zero: the splits are added up in the same launch
   CHECK_BF16(q); CHECK_BF16(k_cache); CHECK_BF16(v_cache); CHECK_BF16(out);
   CHECK_DTYPE(block_tables, at::kInt); CHECK_DTYPE(ctx_lens, at::kInt);
   CHECK_CONTIG(block_tables); CHECK_CONTIG(ctx_lens); CHECK_CONTIG(out);
@@ -284,11 +304,17 @@ void paged_decode(const at::Tensor& q, const at::Tensor& k_cache, const at::Tens
     po = part_o->data_ptr<float>();
     pl = part_lse->data_ptr<float>();
   }
+  int* cn = nullptr;
+  if (counts.has_value() && counts->defined()) {
+    CHECK_GPU(*counts); CHECK_DTYPE(*counts, at::kInt); CHECK_CONTIG(*counts);
+    TORCH_CHECK(counts->numel() >= (int64_t)B * Hkv, "paged_decode: counts too small");
+    cn = counts->data_ptr<int>();
+  }
   const QRope qr = q_rope(rope_cos, rope_sin, positions, B, D, "paged_decode");
   CHECK_RC(lwc_paged_decode(q.data_ptr(), (int)q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
                             block_tables.data_ptr<int>(), ctx_lens.data_ptr<int>(), out.data_ptr(), po, pl, B, Hq, Hkv,
                             D, BS, (int)block_tables.size(1), (int)num_splits, (float)scale, qr.cos, qr.sin, qr.pos,
-                            cur_stream()),
+                            cn, cur_stream()),
            "paged_decode");
 }
 
@@ -452,7 +478,7 @@ void gemm2w(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::
   }
   CHECK_RC(lwc_gemm2w(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, M, N, K, (int)A.stride(0), (int)C.stride(0), (int)epi,
                       (int)tile, (int)splits, splits > 1 ? part->data_ptr<float>() : nullptr,
-                      splits > 1 ? count->data_ptr<int>() : nullptr, cur_stream()),
+                      splits > 1 ? count->data_ptr<int>() : nullptr, nullptr, nullptr, cur_stream()),
            "gemm2w");
 }
 
@@ -507,8 +533,65 @@ void skinny_gemm(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const 
   const int M = (int)A.size(0), K = (int)A.size(1), N = (int)W.size(0);
   TORCH_CHECK(M <= 256 && N % 16 == 0, "skinny_gemm: needs M <= 256, N % 16 == 0");
   CHECK_RC(lwc_skinny_gemm(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, M, N, K, (int)A.stride(0), (int)C.stride(0),
-                           (int)epi, cur_stream()),
+                           (int)epi, nullptr, nullptr, cur_stream()),
            "skinny_gemm");
+}
+
+// A projection of a decode step of at most 64 rows with what lies between it and its neighbours (step_fuse.h), on the weight
+// stream (core 1, skinny.hip) or the 64 x 64 tiles (core 2, gemm2w.hip).  epi 0 plain, 1 residual (R; may be C), 2 SwiGLU:
+// ss [M, P] fp32 partial sums of squares scale the rows of 0 and 2 and are left by 1 (P = N / 16 of core 1, N / 32 of core 2).
+void step_gemm(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::optional<at::Tensor>& R, int64_t epi, int64_t core,
+               const at::Tensor& ss, double eps, const lwc::RopeKV* kv, const c10::optional<at::Tensor>& part,
+               const c10::optional<at::Tensor>& count) {
+  const int M = (int)A.size(0), K = (int)A.size(1), N = (int)W.size(0);
+  TORCH_CHECK(M <= 64 && (core == 1 || core == 2), "step_gemm: at most 64 rows, core 1 or 2");
+  CHECK_GPU(ss); CHECK_DTYPE(ss, at::kFloat); CHECK_CONTIG(ss);
+  TORCH_CHECK(ss.dim() == 2 && ss.size(0) == M && ((uintptr_t)ss.data_ptr() & 15) == 0, "step_gemm: ss must be [M, P]");
+  const lwc::RowSumsq rs{ss.data_ptr<float>(), (int)ss.size(1), (float)eps};
+  const void* r = R.has_value() && R->defined() ? R->data_ptr() : nullptr;
+  int tile = 3, splits = 1;
+  if (core == 2 && part.has_value() && count.has_value()) {
+    CHECK_GPU(*part); CHECK_DTYPE(*part, at::kFloat); CHECK_CONTIG(*part);
+    CHECK_GPU(*count); CHECK_DTYPE(*count, at::kInt); CHECK_CONTIG(*count);
+    lwc_gemm2w_plan(M, N, K, (int)epi, std::min<int64_t>(part->numel() / 4096, count->numel()), &tile, &splits);
+  }
+  CHECK_RC(core == 1 ? lwc_skinny_gemm(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, M, N, K, (int)A.stride(0), (int)C.stride(0),
+                                       (int)epi, &rs, kv, cur_stream())
+                     : lwc_gemm2w(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, M, N, K, (int)A.stride(0), (int)C.stride(0), (int)epi,
+                                  tile, splits, splits > 1 ? part->data_ptr<float>() : nullptr,
+                                  splits > 1 ? count->data_ptr<int>() : nullptr, &rs, kv, cur_stream()),
+           "step_gemm");
+}
+
+void step_project(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::optional<at::Tensor>& R, int64_t epi, int64_t core,
+                  const at::Tensor& ss, double eps, const c10::optional<at::Tensor>& part, const c10::optional<at::Tensor>& count) {
+  gemm_operands(A, W, C, R, epi);
+  TORCH_CHECK(epi <= 2, "step_project: epi must be 0..2");
+  step_gemm(A, W, C, R, epi, core, ss, eps, nullptr, part, count);
+}
+
+// The qkv projection of such a step: q [M, Hq * D] un-rotated into out, k rotated and v into the paged cache at slots.
+void step_qkv(const at::Tensor& A, const at::Tensor& W, at::Tensor& out, const at::Tensor& positions, const at::Tensor& slots,
+              const at::Tensor& cos_t, const at::Tensor& sin_t, at::Tensor& k_cache, at::Tensor& v_cache, int64_t core,
+              const at::Tensor& ss, double eps, const c10::optional<at::Tensor>& part, const c10::optional<at::Tensor>& count) {
+  CHECK_BF16(A); CHECK_BF16(W); CHECK_BF16(out); CHECK_CONTIG(W); CHECK_BF16(k_cache); CHECK_BF16(v_cache);
+  CHECK_GPU(positions); CHECK_DTYPE(positions, at::kInt); CHECK_CONTIG(positions);
+  CHECK_GPU(slots); CHECK_DTYPE(slots, at::kInt); CHECK_CONTIG(slots);
+  CHECK_DTYPE(cos_t, at::kFloat); CHECK_DTYPE(sin_t, at::kFloat); CHECK_CONTIG(cos_t); CHECK_CONTIG(sin_t);
+  TORCH_CHECK(A.dim() == 2 && A.stride(1) == 1 && A.stride(0) % 8 == 0 && out.dim() == 2 && out.stride(1) == 1 && out.stride(0) % 8 == 0,
+              "step_qkv: 2-D rows of 16-byte strides");
+  TORCH_CHECK(k_cache.dim() == 4 && k_cache.is_contiguous(), "step_qkv: k_cache [NB, Hkv, BS, D]");
+  check_v_cache(v_cache, k_cache, "step_qkv");
+  const int64_t M = A.size(0), Hkv = k_cache.size(1), BS = k_cache.size(2), D = k_cache.size(3), Hq = out.size(1) / std::max<int64_t>(D, 1);
+  TORCH_CHECK(W.size(1) == A.size(1) && W.size(0) == (Hq + 2 * Hkv) * D && out.size(0) == M && out.size(1) == Hq * D, "step_qkv: shapes");
+  TORCH_CHECK(positions.numel() == M && slots.numel() == M, "step_qkv: positions and slots");
+  TORCH_CHECK(cos_t.size(1) == D / 2 && sin_t.size(1) == D / 2, "step_qkv: cos/sin table width");
+  lwc::RopeKV kv;
+  kv.positions = positions.data_ptr<int>(), kv.slots = slots.data_ptr<int>();
+  kv.cos = cos_t.data_ptr<float>(), kv.sin = sin_t.data_ptr<float>();
+  kv.kc = (uint16_t*)k_cache.data_ptr(), kv.vc = (uint16_t*)v_cache.data_ptr();
+  kv.Hq = (int)Hq, kv.Hkv = (int)Hkv, kv.D = (int)D, kv.BS = (int)BS;
+  step_gemm(A, W, out, c10::nullopt, 5, core, ss, eps, &kv, part, count);
 }
 
 // ss[r] = sum(x[r]^2): the single partial of the folded RMSNorm for the first projection of a chain
@@ -1055,6 +1138,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm2w", &gemm2w);
   m.def("gemm4w", &gemm4w);
   m.def("skinny_gemm", &skinny_gemm);
+  m.def("step_project", &step_project);
+  m.def("step_qkv", &step_qkv);
+  m.def("embedding_step", &embedding_step);
   m.def("rms_rowsumsq", &rms_rowsumsq);
   m.def("gemm8p_slots", &lwc_gemm8p_slots);
   m.def("moe_route", &moe_route);

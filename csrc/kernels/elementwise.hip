@@ -119,6 +119,30 @@ __global__ void embedding_gather_kernel(const bf16_t* __restrict__ table, const 
   for (int i = threadIdx.x; i < (d >> 3); i += blockDim.x) dst[i] = src[i];
 }
 
+// The rows of a decode step: the same gather, with each row's sum of squares in four partials (step_fuse.h) and the step's
+// split counters cleared (paged_decode_kernel), [T, per]
+__global__ void __launch_bounds__(256) embedding_step_kernel(const bf16_t* __restrict__ table, const int* __restrict__ ids,
+                                                             bf16_t* __restrict__ out, float* __restrict__ ss,
+                                                             int* __restrict__ counts, int per, int d, int V) {
+  const int t = blockIdx.x, lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int id = ids[t];
+  id = id < 0 ? 0 : (id >= V ? V - 1 : id);
+  const uint4v* src = reinterpret_cast<const uint4v*>(table + (size_t)id * d);
+  uint4v* dst = reinterpret_cast<uint4v*>(out + (size_t)t * d);
+  float s = 0.f;
+  for (int i = threadIdx.x; i < (d >> 3); i += 256) {
+    const uint4v v = src[i];
+    dst[i] = v;
+    float x[8];
+    unpack8(v, x);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s += x[e] * x[e];
+  }
+  s = wave_sum(s);
+  if (lane == 0) ss[(size_t)t * 4 + w] = s;
+  for (int i = threadIdx.x; i < per; i += 256) counts[(size_t)t * per + i] = 0;
+}
+
 // cache: [L, 2, NB, block_elems]; pairs: [P, 2] (src, dst) int32
 __global__ void kv_block_copy_kernel(bf16_t* __restrict__ cache, const int* __restrict__ pairs, int NB,
                                      int64_t block_elems) {
@@ -195,6 +219,15 @@ extern "C" int lwc_embedding_gather(const void* table, const int* ids, void* out
   if (d % 8 != 0) return -1;
   if (T == 0) return 0;
   embedding_gather_kernel<<<T, 128, 0, s>>>((const bf16_t*)table, ids, (bf16_t*)out, d, V);
+  return (int)hipGetLastError();
+}
+
+extern "C" int lwc_embedding_step(const void* table, const int* ids, void* out, float* ss, int* counts, int per, int T, int d,
+                                  int V, hipStream_t s) {
+  using namespace lwc;
+  if (d % 8 != 0 || per < 0) return -1;
+  if (T == 0) return 0;
+  embedding_step_kernel<<<T, 256, 0, s>>>((const bf16_t*)table, ids, (bf16_t*)out, ss, counts, per, d, V);
   return (int)hipGetLastError();
 }
 

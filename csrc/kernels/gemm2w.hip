@@ -14,13 +14,14 @@
 #include <algorithm>
 
 #include "common.h"
+#include "step_fuse.h"
 
 namespace lwc {
 namespace g2w {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
-enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4 };
+enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4, EPI_ROPE_KV = 5 };
 
 struct Params {
   const bf16_t* A;
@@ -32,6 +33,8 @@ struct Params {
   int splits;   // K ranges per tile
   float* part;  // splits > 1: [tiles][splits][TM * TN] partial tiles
   int* count;   // [tiles] finished ranges (zero between launches)
+  RowSumsq ss;  // NORM: read by EPI_PLAIN, EPI_SWIGLU and EPI_ROPE_KV, written by EPI_RESIDUAL
+  RopeKV kv;    // EPI_ROPE_KV
 };
 
 LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
@@ -51,9 +54,13 @@ LWC_DEVICE void wait_rows() {
 
 constexpr int kGroupM = 8;
 
-template <int EPI, int TM, int TN, int NST>
+// EPI_ROPE_KV (64 x 64 tiles, step_fuse.h): a tile takes 32 columns of a head and the 32 that rotate with them, D / 2 further.
+// NORM (64 x 64 tiles): the folded RMSNorm of step_fuse.h.
+template <int EPI, int TM, int TN, int NST, bool NORM>
 __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
-  constexpr int WC = EPI == EPI_SWIGLU && TN == 64 ? 1 : 2, WR = 4 / WC;  // waves across the tile's columns and rows
+  static_assert((!NORM && EPI != EPI_ROPE_KV) || (TM == 64 && TN == 64), "one row of partial sums per lane group");
+  constexpr bool kPairs = EPI == EPI_SWIGLU || EPI == EPI_ROPE_KV;  // columns that meet in a lane: groups of 32, two by two
+  constexpr int WC = kPairs && TN == 64 ? 1 : 2, WR = 4 / WC;  // waves across the tile's columns and rows
   constexpr int kA = TM * 128, kStage = kA + TN * 128;  // bytes of a 64-deep K step: A rows, then W rows, 128 bytes each
   constexpr int IA = TM / 32, IW = TN / 32;             // DMA instructions per wave and step
   constexpr int MI = TM / WR / 16, NP = TN / WC / 32;   // the wave's 16-row tiles and its groups of 32 columns
@@ -65,14 +72,20 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
   const int u = xcd_remap(blockIdx.x, p.tiles_m * p.tiles_n * p.splits), t = u / p.splits, split = u % p.splits;
   const int first_m = t / (kGroupM * p.tiles_n) * kGroupM, gsz = min(p.tiles_m - first_m, kGroupM);
   const int in = t % (kGroupM * p.tiles_n);
-  const int m0 = (first_m + in % gsz) * TM, n0 = in / gsz * TN;
+  const int m0 = (first_m + in % gsz) * TM;
+  int n0 = in / gsz * TN, far = 0;  // far: W rows between the tile's two halves beyond those of a contiguous tile
+  if constexpr (EPI == EPI_ROPE_KV) {
+    const int strips = p.kv.D / 64, h = in / gsz / strips;
+    n0 = h * p.kv.D + in / gsz % strips * 32;
+    far = p.kv.D / 2 - 32;
+  }
 
   // DMA: a wave's instruction fills 8 rows; lane l carries row l / 8 and the chunk of it that belongs at position l % 8:
   // chunk c of A row r lies at c ^ (r / 2 % 8), of W row r at c ^ (r / 8 % 4 * 2 + r / 2 % 2), so that the 16-lane groups
   // in which an operand read is served meet every bank once
-  const int rows_m = min(p.M - m0, TM), rows_n = min(p.N - n0, TN);
+  const int rows_m = min(p.M - m0, TM), rows_n = EPI == EPI_ROPE_KV ? TN : min(p.N - n0, TN);
   const __amdgpu_buffer_rsrc_t rA = uniform_rsrc(p.A + (size_t)m0 * p.lda, ((rows_m - 1) * p.lda + p.K) * 2);
-  const __amdgpu_buffer_rsrc_t rW = uniform_rsrc(p.W + (size_t)n0 * p.K, rows_n * p.K * 2);
+  const __amdgpu_buffer_rsrc_t rW = uniform_rsrc(p.W + (size_t)n0 * p.K, (rows_n + far) * p.K * 2);
   uint32_t voA[IA], voW[IW];
 #pragma unroll
   for (int i = 0; i < IA; ++i) {
@@ -82,7 +95,7 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
 #pragma unroll
   for (int i = 0; i < IW; ++i) {
     const int row = (i * 4 + wid) * 8 + (lane >> 3);
-    voW[i] = row < rows_n ? (uint32_t)(row * p.K * 2 + (((lane & 7) ^ ((row >> 3 & 3) * 2 + (row >> 1 & 1))) << 4)) : 0x7fffffffu;
+    voW[i] = row < rows_n ? (uint32_t)((row + (EPI == EPI_ROPE_KV && row >= 32 ? far : 0)) * p.K * 2 + (((lane & 7) ^ ((row >> 3 & 3) * 2 + (row >> 1 & 1))) << 4)) : 0x7fffffffu;
   }
   auto stage = [&](uint8_t* buf, int kt) {
 #pragma unroll
@@ -104,10 +117,40 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) acc[i][g][h] = float4v{0.f, 0.f, 0.f, 0.f};
 
+  // The rows' partial sums of squares go out ahead of the first K steps and are added up while those are on their way, each
+  // wave its own rows: 16 lanes per row, four rows at a time.  (In registers: a store to LDS waits for every row on its way
+  // there, 1.6 us.)  So do a row's slot and position; the angles follow the first K steps.
+  constexpr bool kScale = NORM && EPI != EPI_RESIDUAL;
+  float4v ssv[kScale ? 4 * MI : 1][4];
+  float sumsq[kScale ? 4 * MI : 1];
+  if constexpr (kScale) {
+    const __amdgpu_buffer_rsrc_t rS = uniform_rsrc(p.ss.ss + (size_t)m0 * p.ss.P, rows_m * p.ss.P * 4);
+#pragma unroll
+    for (int i = 0; i < 4 * MI; ++i)
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        ssv[i][c] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(
+            rS, 64 * c + 4 * r16 < p.ss.P ? ((wr * (TM / WR) + 4 * i + q) * p.ss.P + 64 * c + 4 * r16) * 4 : 0x7fffffff, 0, 0));
+  }
+  RopeAhead<8> ahead;
+  if constexpr (EPI == EPI_ROPE_KV) rope_kv_row(p.kv, ahead, min(m0 + wr * 16 + r16, p.M - 1), n0 / p.kv.D);
+  __builtin_amdgcn_sched_barrier(0);
   const int KT = p.K / 64, k0 = KT * split / p.splits, nk = KT * (split + 1) / p.splits - k0;
 #pragma unroll
-  for (int k = 0; k < NST; ++k)
-    if (k < nk) stage(smem + k * kStage, k0 + k);
+  for (int k = 0; k < NST; ++k)  // (NORM: steps past the range too, rows that nothing reads: behind a branch the sums would wait for all)
+    if (NORM || k < nk) stage(smem + k * kStage, k0 + k);
+  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (EPI == EPI_ROPE_KV) rope_kv_angles(p.kv, ahead, n0 / p.kv.D, n0 % p.kv.D + 8 * q);
+  if constexpr (kScale) {
+#pragma unroll
+    for (int i = 0; i < 4 * MI; ++i) {
+      float t = 0.f;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) t += (ssv[i][c][0] + ssv[i][c][1]) + (ssv[i][c][2] + ssv[i][c][3]);
+      sumsq[i] = row16_sum(t);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   int at = 0;
   for (int kt = 0; kt < nk; ++kt) {
     uint8_t* buf = smem + at;
@@ -183,7 +226,49 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
   }
 
   const int mrow = m0 + wr * (TM / WR) + r16;
-  if constexpr (EPI == EPI_SWIGLU) {  // groups 2 g: gate columns, 2 g + 1: the matching up columns
+  if constexpr (kScale) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      float t = 0.f;  // row r16 = 4 j + q' was added up by lane group q' of the j-th four
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float u = __shfl(sumsq[4 * i + j], 16 * (r16 & 3), 64);
+        t = r16 >> 2 == j ? u : t;
+      }
+      const float f = rsqrtf(t / p.K + p.ss.eps);
+#pragma unroll
+      for (int g = 0; g < NP; ++g)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) acc[i][g][h] *= f;
+    }
+  }
+  if constexpr (EPI == EPI_ROPE_KV) {
+    const int head = n0 / p.kv.D, c0 = n0 % p.kv.D;
+    if (head >= p.kv.Hq + p.kv.Hkv) {
+      // v: its entries lie four tokens apart, so a row's 64 are turned through LDS to go out side by side, a sector of four
+      // per 32 bytes (as the lanes hold them every one was a sector of its own: 61 rows x 6144 x 4096 22 -> 18 us)
+      bf16_t* turn = reinterpret_cast<bf16_t*>(smem) + 64 + wid * 16 * 72;  // (behind the splits' flag; the wave's own)
+      float x[8];
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) x[e] = acc[0][h][e >> 2][e & 3];
+        *reinterpret_cast<uint4v*>(turn + r16 * 72 + h * 32 + 8 * q) = pack8(x);
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      const int c = c0 + (lane & 31) + (lane >= 32 ? p.kv.D / 2 : 0);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const int slot = __builtin_amdgcn_readlane(ahead.slot, r), row = m0 + wr * 16 + r;
+        if (row < p.M && slot >= 0) rope_v_row(p.kv, slot, head)[4 * c] = turn[r * 72 + lane];
+      }
+      return;
+    }
+    float x[8], y[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = acc[0][0][e >> 2][e & 3], y[e] = acc[0][1][e >> 2][e & 3];
+    if (mrow < p.M) rope_kv_store<8>(p.kv, ahead, p.C, p.ldc, mrow, head, c0 + 8 * q, x, y);
+  } else if constexpr (EPI == EPI_SWIGLU) {  // groups 2 g: gate columns, 2 g + 1: the matching up columns
 #pragma unroll
     for (int g = 0; g < NP / 2; ++g) {
       const int col = (n0 + wc * (TN / WC)) / 2 + g * 32 + 8 * q;
@@ -218,21 +303,30 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
           if (EPI != EPI_PLAIN) x[e] += b[e];
           if (EPI == EPI_BIAS_GELU) x[e] = gelu_erf(x[e]);
         }
-        if (mrow + 16 * i < p.M) *reinterpret_cast<uint4v*>(p.C + (size_t)(mrow + 16 * i) * p.ldc + col) = pack8(x);
+        const uint4v o = pack8(x);
+        if (mrow + 16 * i < p.M) *reinterpret_cast<uint4v*>(p.C + (size_t)(mrow + 16 * i) * p.ldc + col) = o;
+        if constexpr (EPI == EPI_RESIDUAL && NORM) {  // of the row as stored: one partial per 32 columns
+          unpack8(o, x);
+          float t2 = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t2 += x[e] * x[e];
+          t2 = row_sum4(t2);
+          if (q == 0 && mrow + 16 * i < p.M) p.ss.ss[(size_t)(mrow + 16 * i) * p.ss.P + (n0 + wc * (TN / WC)) / 32 + g] = t2;
+        }
       }
     }
   }
 }
 
-template <int EPI, int TM, int TN, int NST>
+template <int EPI, int TM, int TN, int NST, bool NORM = false>
 int launch(Params p, hipStream_t s) {
   constexpr int kLds = NST * (TM + TN) * 128;
   static const hipError_t attr =
-      hipFuncSetAttribute((const void*)gemm2w_kernel<EPI, TM, TN, NST>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+      hipFuncSetAttribute((const void*)gemm2w_kernel<EPI, TM, TN, NST, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   (void)attr;
   p.tiles_m = (p.M + TM - 1) / TM;
   p.tiles_n = (p.N + TN - 1) / TN;
-  gemm2w_kernel<EPI, TM, TN, NST><<<p.tiles_m * p.tiles_n * p.splits, 256, kLds, s>>>(p);
+  gemm2w_kernel<EPI, TM, TN, NST, NORM><<<p.tiles_m * p.tiles_n * p.splits, 256, kLds, s>>>(p);
   return (int)hipGetLastError();
 }
 
@@ -243,6 +337,8 @@ int launch(Params p, hipStream_t s) {
 // 3: C = A W^T + bias (R = bias [N]); 4: C = gelu(A W^T + bias) (exact erf GELU).
 // tile 0: 128 x 128, 1: 192 x 128, 2: 128 x 192 (not epi 2), 3: 64 x 64, there with splits K ranges per tile (part: tiles x
 // splits x 4096 floats, count: tiles ints, zero on the first call; the kernel leaves them zero).
+// epi 5: the qkv projection with k and v written into the paged cache (kv; tile 3).  ss (tile 3): the folded RMSNorm: epi 0, 2
+// and 5 scale their rows by it (epi 5 always), epi 1 writes N / 32 partials per row (N % 32 == 0).
 // Requires K % 64 == 0, K / 64 >= splits, N % 8 == 0 and 16-byte rows and pointers.
 // The tile and the K ranges of a call (max_splits: what the caller's workspace holds, in 64 x 64 partial tiles).
 // 64 x 64 up to 512 tiles (two workgroups per CU) and for any call of up to 64 rows.  Measured (us, 64 x 64 against 128 x 128):
@@ -271,18 +367,28 @@ extern "C" void lwc_gemm2w_plan(int M, int N, int K, int epi, long long max_spli
 }
 
 extern "C" int lwc_gemm2w(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda, int ldc, int epi,
-                          int tile, int splits, float* part, int* count, hipStream_t s) {
+                          int tile, int splits, float* part, int* count, const lwc::RowSumsq* ss, const lwc::RopeKV* kv,
+                          hipStream_t s) {
   using namespace lwc::g2w;
   if (K % 64 != 0 || K < 64 || N % 8 != 0 || lda % 8 != 0 || ldc % 8 != 0 || tile < 0 || tile > 3) return -1;
   if (192LL * (lda + K) * 2 >= (1LL << 31)) return -1;  // 32-bit buffer offsets in a tile
   if (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C | (uintptr_t)R) & 15) return -1;
   if (splits < 1 || splits > K / 64 || (splits > 1 && (tile != 3 || part == nullptr || count == nullptr))) return -1;
   if (epi == EPI_SWIGLU && (N % 64 != 0 || tile == 2)) return -1;
-  if (epi != EPI_PLAIN && epi != EPI_SWIGLU && R == nullptr) return -1;
+  if ((epi == EPI_RESIDUAL || epi == EPI_BIAS || epi == EPI_BIAS_GELU) && R == nullptr) return -1;
+  if (ss != nullptr && (tile != 3 || epi == EPI_BIAS || epi == EPI_BIAS_GELU || ss->P < 4 || ss->P % 4 != 0 || ss->P > 256 ||
+                        (epi == EPI_RESIDUAL && (N % 32 != 0 || ss->P != N / 32)))) return -1;
+  if (epi == EPI_ROPE_KV && (ss == nullptr || kv == nullptr || !lwc::rope_kv_ok(*kv, N) || (64LL + kv->D) * K * 2 >= (1LL << 31))) return -1;
   if (M == 0 || N == 0) return 0;
   if (((long long)M + 63) / 64 * ((N + 63) / 64) * splits >= (1LL << 31)) return -1;
   const Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc, 0, 0,
-                 splits, part, count};
+                 splits, part, count, ss != nullptr ? *ss : lwc::RowSumsq{}, kv != nullptr ? *kv : lwc::RopeKV{}};
+  if (ss != nullptr) switch (epi) {
+    case EPI_PLAIN: return launch<EPI_PLAIN, 64, 64, 4, true>(p, s);
+    case EPI_RESIDUAL: return launch<EPI_RESIDUAL, 64, 64, 4, true>(p, s);
+    case EPI_SWIGLU: return launch<EPI_SWIGLU, 64, 64, 4, true>(p, s);
+    default: return launch<EPI_ROPE_KV, 64, 64, 4, true>(p, s);
+  }
 #define LWC_G2W(E)                                                                     \
   case E:                                                                              \
     if constexpr (E != EPI_SWIGLU)                                                     \

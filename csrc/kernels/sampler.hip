@@ -150,12 +150,6 @@ LWC_DEVICE uint32_t thr1x2(uint32_t key) { return ((key - 1u) & 0xffffu) * 0x100
 
 // ---- reductions by lane swaps and DPP (a shuffle is a trip through LDS, six of them per reduction) ----
 #define LWC_DPP(x, ctrl) __builtin_amdgcn_mov_dpp((x), (ctrl), 0xF, 0xF, false)
-LWC_DEVICE float row16_sum(float x) {
-  x += __int_as_float(LWC_DPP(__float_as_int(x), 0xB1));
-  x += __int_as_float(LWC_DPP(__float_as_int(x), 0x4E));
-  x += __int_as_float(LWC_DPP(__float_as_int(x), 0x141));
-  return x + __int_as_float(LWC_DPP(__float_as_int(x), 0x140));
-}
 LWC_DEVICE int row16_sum_i(int x) {
   x += LWC_DPP(x, 0xB1);
   x += LWC_DPP(x, 0x4E);

@@ -29,6 +29,7 @@
 // Requires K % 32 == 0, N % 16 == 0, lda / ldc % 4 == 0; the planners (ops/gemm_plan.py, backend "gv") time it against
 // hipBLASLt per decode bucket and per encoder token bucket.
 #include "common.h"
+#include "step_fuse.h"
 
 namespace lwc {
 namespace skinny {
@@ -48,6 +49,8 @@ struct Params {
   bf16_t* C;
   const bf16_t* R;  // residual [M, ldc] (EPI 1) — may alias C; bias [N] (EPI 3, 4)
   int M, N, K, lda, ldc;
+  RowSumsq ss;  // NORM: read by EPI 0, 2, 5, written by EPI 1
+  RopeKV kv;    // EPI 5
 };
 
 // NW weight tiles of 16 rows per workgroup, on the same activation fragments: EPI 2 (SwiGLU, W = [gate; up]
@@ -55,16 +58,21 @@ struct Params {
 // 16 (x % 2) + [0, 16) and the up rows 32 further (NW = 2); the plain / residual forms take 16 (NW = 1) or 32
 // adjacent output columns (NW = 2: half the workgroups, so half the activation re-reads from L2 — past 16
 // rows those loads, M / 16 times the weight bytes, are what limits the NW = 1 form)
-template <int MT, int EPI, int NW, bool FULL>
+// EPI 5 (the qkv projection of a decode step, step_fuse.h): the two tiles are the halves of a head that rotate together.
+// NORM: the folded RMSNorm of step_fuse.h.
+template <int MT, int EPI, int NW, bool FULL, bool NORM>
 __global__ void __launch_bounds__(512) skinny_kernel(Params p) {
   constexpr int U = 4;  // k-steps per load batch (FULL: nb = K / 1024 batches, even for K % 2048 == 0)
-  static_assert(EPI != 2 || NW == 2, "SwiGLU pairs a gate and an up tile");
-  constexpr int TS = EPI == 2 ? 32 : 16;  // W rows between the NW tiles
+  static_assert((EPI != 2 && EPI != 5) || NW == 2, "SwiGLU pairs a gate and an up tile, RoPE the halves of a head");
+  const int TS = EPI == 2 ? 32 : EPI == 5 ? p.kv.D / 2 : 16;  // W rows between the NW tiles
   __shared__ float4v red[KS][NW][MT][64];
+  __shared__ float rowscale[NORM ? MT * 16 : 1];
   const int lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
-  const int n0 = blockIdx.x * (EPI == 2 ? 16 : 16 * NW);  // first output column
+  const int strips = EPI == 5 ? p.kv.D / 32 : 1;  // (EPI 5: workgroups per head)
+  const int n0 = EPI == 5 ? blockIdx.x / strips * p.kv.D + blockIdx.x % strips * 16
+                          : blockIdx.x * (EPI == 2 ? 16 : 16 * NW);  // first output column
   const int wrow = EPI == 2 ? 64 * (blockIdx.x >> 1) + 16 * (blockIdx.x & 1) : n0;  // first W row
   const int m0 = blockIdx.y * 64;   // this chunk's first row
   const int M = min(p.M - m0, 64);
@@ -112,9 +120,32 @@ __global__ void __launch_bounds__(512) skinny_kernel(Params p) {
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[t][mt] = mfma(wb[s][t], ab[s][mt], acc[t][mt]);
   };
+  // the rows' partial sums of squares go out ahead of the first weights and are added up while those are on their way
+  constexpr bool kScale = NORM && EPI != 1;
+  constexpr int NR = 2 * MT;  // rows per wave
+  float4v ssv[NR];
+  if constexpr (kScale) {
+    const __amdgpu_buffer_rsrc_t rS = uniform_rsrc(p.ss.ss + (size_t)m0 * p.ss.P, M * p.ss.P * 4);
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+      ssv[i] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(
+                                               rS, 4 * lane < p.ss.P ? ((w + 8 * i) * p.ss.P + 4 * lane) * 4 : kPast, 0, 0));
+  }
+  RopeAhead<4> ahead;  // (waves past the m tiles and rows past M: row m0's, unused)
+  if constexpr (EPI == 5) rope_kv_row(p.kv, ahead, m0 + (w < MT && w * 16 + r16 < M ? w * 16 + r16 : 0), blockIdx.x / strips);
   // straight-line pairs (no conditional loads: a load under a branch made the wait before every compute a
   // vmcnt(0)); nb is even
   load(0, wf[0], af[0]);
+  if constexpr (EPI == 5) rope_kv_angles(p.kv, ahead, blockIdx.x / strips, blockIdx.x % strips * 16 + 4 * g);
+  if constexpr (kScale) {
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < NR; ++i) {
+      const float t = wave_sum((ssv[i][0] + ssv[i][1]) + (ssv[i][2] + ssv[i][3]));
+      if (lane == 0) rowscale[w + 8 * i] = rsqrtf(t / p.K + p.ss.eps);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
   for (int b = 0; b + 2 < nb; b += 2) {
     load(b + 1, wf[1], af[1]);
     __builtin_amdgcn_sched_barrier(0);
@@ -144,12 +175,21 @@ __global__ void __launch_bounds__(512) skinny_kernel(Params p) {
       for (int k = 1; k < KS; ++k) sum[t] += red[k][t][w][lane];
     }
     constexpr int NO = EPI == 2 ? 1 : NW;  // 16-column output groups
+    if constexpr (kScale) {
+#pragma unroll
+      for (int t = 0; t < NW; ++t) sum[t] *= rowscale[w * 16 + r16];
+    }
     if constexpr (EPI == 2) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) sum[0][e] = sum[0][e] * __builtin_amdgcn_rcpf(1.f + __expf(-sum[0][e])) * sum[1][e];
     }
     const int m = w * 16 + r16;
-    if (m < M) {
+    if constexpr (EPI == 5) {
+      if (m < M) {
+        const float x[4] = {sum[0][0], sum[0][1], sum[0][2], sum[0][3]}, y[4] = {sum[1][0], sum[1][1], sum[1][2], sum[1][3]};
+        rope_kv_store<4>(p.kv, ahead, p.C, p.ldc, m0 + m, blockIdx.x / strips, blockIdx.x % strips * 16 + 4 * g, x, y);
+      }
+    } else if (m < M) {
 #pragma unroll
       for (int t = 0; t < NO; ++t) {
         const size_t off = (size_t)(m0 + m) * p.ldc + n0 + 16 * t + 4 * g;
@@ -173,40 +213,46 @@ __global__ void __launch_bounds__(512) skinny_kernel(Params p) {
         o.x = pack_bf16x2(v[0], v[1]);
         o.y = pack_bf16x2(v[2], v[3]);
         *reinterpret_cast<uint2*>(p.C + off) = o;
+        if constexpr (EPI == 1 && NORM) {  // of the row as stored: one partial per 16 columns
+          const float a = __uint_as_float(o.x << 16), b = __uint_as_float(o.x & 0xffff0000u), c = __uint_as_float(o.y << 16),
+                      d = __uint_as_float(o.y & 0xffff0000u);
+          const float t2 = row_sum4((a * a + b * b) + (c * c + d * d));
+          if (g == 0) p.ss.ss[(size_t)(m0 + m) * p.ss.P + n0 / 16 + t] = t2;
+        }
       }
     }
   }
 }
 
-template <int EPI, int NW, bool FULL>
+template <int EPI, int NW, bool FULL, bool NORM>
 int launch_full(const Params& p, hipStream_t s) {
   const int mt = (min(p.M, 64) + 15) / 16;
   const dim3 grid(EPI == 2 ? p.N / 32 : p.N / (16 * NW), (p.M + 63) / 64);  // SwiGLU: N / 2 output columns, 16 per workgroup
   switch (mt) {
-    case 1: skinny_kernel<1, EPI, NW, FULL><<<grid, 512, 0, s>>>(p); break;
-    case 2: skinny_kernel<2, EPI, NW, FULL><<<grid, 512, 0, s>>>(p); break;
+    case 1: skinny_kernel<1, EPI, NW, FULL, NORM><<<grid, 512, 0, s>>>(p); break;
+    case 2: skinny_kernel<2, EPI, NW, FULL, NORM><<<grid, 512, 0, s>>>(p); break;
     case 3:
-    case 4: skinny_kernel<4, EPI, NW, FULL><<<grid, 512, 0, s>>>(p); break;
+    case 4: skinny_kernel<4, EPI, NW, FULL, NORM><<<grid, 512, 0, s>>>(p); break;
     default: return -1;
   }
   return (int)hipGetLastError();
 }
 
-template <int EPI, int NW>
+template <int EPI, int NW, bool NORM>
 int launch_nw(const Params& p, hipStream_t s) {
-  return p.K % 2048 == 0 ? launch_full<EPI, NW, true>(p, s) : launch_full<EPI, NW, false>(p, s);
+  return p.K % 2048 == 0 ? launch_full<EPI, NW, true, NORM>(p, s) : launch_full<EPI, NW, false, NORM>(p, s);
 }
 
 // plain / residual: 32 output columns per workgroup past 16 rows when that still leaves >= 192 workgroups
 // (M / 16 activation re-reads halved: qkv at M = 32 23.9 -> 17.9 us), else 16 (o, N = 4096: 128 workgroups
 // of 32 columns ran 17.6 us against 13.8 with 256 of 16 — too little of the weight stream in flight)
-template <int EPI>
+template <int EPI, bool NORM = false>
 int launch(const Params& p, hipStream_t s) {
-  if constexpr (EPI == 2) {
-    return launch_nw<2, 2>(p, s);
+  if constexpr (EPI == 2 || EPI == 5) {
+    return launch_nw<EPI, 2, NORM>(p, s);
   } else {
-    if (p.M > 16 && p.N % 32 == 0 && p.N / 32 >= 192) return launch_nw<EPI, 2>(p, s);
-    return launch_nw<EPI, 1>(p, s);
+    if (p.M > 16 && p.N % 32 == 0 && p.N / 32 >= 192) return launch_nw<EPI, 2, NORM>(p, s);
+    return launch_nw<EPI, 1, NORM>(p, s);
   }
 }
 
@@ -214,20 +260,30 @@ int launch(const Params& p, hipStream_t s) {
 }  // namespace lwc
 
 // C = A . W^T (epi 0), R + A . W^T (epi 1; R may be C), silu(A . Wg^T) * (A . Wu^T) over a 32-row gate/up interleaved
-// W [N, K] (epi 2, C [M, N / 2]), A . W^T + bias (epi 3; R = bias [N]) or gelu(A . W^T + bias) (epi 4) for M <= 256 rows.
-// -1: shape not taken.
+// W [N, K] (epi 2, C [M, N / 2]), A . W^T + bias (epi 3; R = bias [N]) or gelu(A . W^T + bias) (epi 4) for M <= 256 rows;
+// epi 5: the qkv projection with k and v written into the paged cache (kv).  ss: the folded RMSNorm (epi 0, 2 and 5 scale
+// their rows by it, epi 5 always; epi 1 writes N / 16 partials per row).  -1: shape not taken.
 extern "C" int lwc_skinny_gemm(const void* A, const void* W, void* C, const void* R, int M, int N, int K, int lda,
-                               int ldc, int epi, hipStream_t s) {
+                               int ldc, int epi, const lwc::RowSumsq* ss, const lwc::RopeKV* kv, hipStream_t s) {
   using namespace lwc::skinny;
-  const int NC = epi == 2 ? N / 2 : N;
+  const int NC = epi == 2 ? N / 2 : epi == 5 && kv != nullptr ? kv->Hq * kv->D : N;
   if (M < 0 || M > 256 || K < 32 || K % 32 != 0 || N % (epi == 2 ? 64 : 16) != 0 || lda % 4 != 0 || ldc % 4 != 0 ||
       lda < K || ldc < NC)
     return -1;
-  if (epi < 0 || epi > 4) return -1;
-  if ((epi == 1 || epi >= 3) && R == nullptr) return -1;
-  if ((long long)48 * K * 2 >= 0x7ffffff0LL || (long long)64 * lda * 2 >= 0x7ffffff0LL) return -1;
+  if (epi < 0 || epi > 5) return -1;
+  if ((epi == 1 || epi == 3 || epi == 4) && R == nullptr) return -1;
+  if (ss != nullptr && (epi == 3 || epi == 4 || ss->P < 4 || ss->P % 4 != 0 || ss->P > 256 || (epi == 1 && ss->P != N / 16))) return -1;
+  if (epi == 5 && (ss == nullptr || kv == nullptr || !lwc::rope_kv_ok(*kv, N))) return -1;
+  if ((long long)(16 + (epi == 5 ? kv->D / 2 : 32)) * K * 2 >= 0x7ffffff0LL || (long long)64 * lda * 2 >= 0x7ffffff0LL) return -1;
   if (M == 0 || N == 0) return 0;
-  Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc};
+  Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc,
+           ss != nullptr ? *ss : lwc::RowSumsq{}, kv != nullptr ? *kv : lwc::RopeKV{}};
+  if (ss != nullptr) switch (epi) {
+    case 0: return launch<0, true>(p, s);
+    case 1: return launch<1, true>(p, s);
+    case 2: return launch<2, true>(p, s);
+    default: return launch<5, true>(p, s);
+  }
   switch (epi) {
     case 0: return launch<0>(p, s);
     case 1: return launch<1>(p, s);

@@ -291,6 +291,59 @@ class LlamaModel:
             return ops.gemm4w(x_res, self.lm_head, chain=ch, var=lv, splits=sk[0], split_from=sk[1])
         return self._proj(ops.rmsnorm(x_res, ones, eps), self.lm_head)
 
+    def _step_ok(self, positions: torch.Tensor, slots: torch.Tensor, cache) -> bool:
+        """Whether a decode step runs as :meth:`_decode_step`: few rows (the launches between its GEMMs count), the norms
+        folded, and positions, slots and a cache that its kernels read."""
+        B = positions.numel()
+        return (self.norm_folded and self._dense_residual and self.g8_ws is not None and 0 < B <= gemm_plan.STEP_ROWS
+                and self.cfg.head_dim == 128 and self.layers[0].gu_block == 32 and not self.chain_ok(B) and slots is not None
+                and slots.numel() == B and all(t.dtype == torch.int32 and t.is_contiguous() for t in (positions, slots))
+                and cache.k[0].is_contiguous() and cache.v[0].is_contiguous())
+
+    def _decode_step(self, tokens, positions, slots, block_tables, ctx_lens, cache: KVCache, num_splits: int) -> torch.Tensor:
+        """A decode step of few rows without the kernels between its GEMMs (csrc/kernels/step_fuse.h): the residual
+        projections leave the rows' sums of squares and the next projection scales by them, the qkv projection writes k and
+        v into the cache, the attention adds up its splits.  A projection that is on another core keeps the norm (and RoPE)
+        kernel in front of it.  Llama-3-8B layers, four of them, and its lm_head: one row 621 -> 569 us, 61 rows of mixed
+        contexts 927 -> 880 (of both, half is the attention's reduction kernel)."""
+        cfg = self.cfg
+        B, Hq, Hkv, D, eps, ws = tokens.shape[0], cfg.heads, cfg.kv_heads, cfg.head_dim, cfg.rms_eps, self.g8_ws
+        x, ss, counts = ops.embedding_step(self.embed, tokens, Hkv)
+        part_o = part_lse = None
+        if num_splits > 1:
+            part_o = torch.empty(B * Hq * num_splits * D, dtype=torch.float32, device=x.device)
+            part_lse = torch.empty(B * Hq * num_splits, dtype=torch.float32, device=x.device)
+
+        def project(w, epi, ss):
+            core = gemm_plan.step_core(x, w, epi) if ss is not None else 0
+            if core:
+                return ops.step_project(x, w, core, ss, eps, swiglu=epi == "swiglu", ws=ws)
+            h = ops.rmsnorm(x, self.final_norm, eps)  # (every norm weight is ones after folding)
+            return gemm_plan.linear(h, w, ws=ws) if epi == "plain" else gemm_plan.swiglu(h, w, 32, ws=ws)
+
+        def add(inp, w):
+            core = gemm_plan.step_core(inp, w, "residual")
+            P = ops.step_partials(core, cfg.hidden) if core else 0
+            if not P:
+                gemm_plan.linear_add_(inp, w, x, ws=ws)
+                return None
+            part = torch.empty(B, P, dtype=torch.float32, device=x.device)
+            ops.step_project(inp, w, core, part, eps, residual=x, ws=ws)
+            return part
+
+        for li, L in enumerate(self.layers):
+            core = gemm_plan.step_core(x, L.wqkv, "plain") if ss is not None else 0
+            if core:
+                q = ops.step_qkv(x, L.wqkv, core, ss, eps, positions, slots, self.cos, self.sin, cache.k[li], cache.v[li], Hq, ws=ws)
+            else:
+                q = project(L.wqkv, "plain", None)
+                ops.rope_kv_write(q, positions, self.cos, self.sin, cache.k[li], cache.v[li], Hq, Hkv, D, slots=slots, rope_q=False)
+            attn = ops.paged_decode(q, cache.k[li], cache.v[li], block_tables, ctx_lens, Hq, self.scale, num_splits=num_splits,
+                                    part_o=part_o, part_lse=part_lse, rope=(self.cos, self.sin, positions), counts=counts)
+            ss = add(attn.view(B, Hq * D), L.wo)
+            ss = add(project(L.w_gate_up, "swiglu", ss), L.w_down)
+        return project(self.lm_head, "plain", ss)
+
     def chain_ok(self, M: int) -> bool:
         """Whether a decode step of M rows folds at least one norm (timed faster at M, before capture)."""
         c = self.chain_m.get(M)
@@ -664,12 +717,14 @@ class LlamaModel:
         the one-launch cascade kernel (shared prompt blocks read once per super-tile; the engine's
         large-batch path); otherwise split-K paged decode."""
         cfg = self.cfg
-        x = ops.embedding(self.embed, tokens)
         B = tokens.shape[0]
+        q_at_load = os.environ.get("LWC_DECODE_QROPE", "1") != "0"
+        if cascade_tiles is None and q_at_load and self._step_ok(positions, slots, cache):
+            return self._decode_step(tokens, positions, slots, block_tables, ctx_lens, cache, num_splits)
+        x = ops.embedding(self.embed, tokens)
         # q is rotated inside the attention kernels as they load it (rope_kv_write rotates and caches k
         # only): q's round trip through HBM in rope_kv_write (2/3 of its bytes at GQA 4) is gone.
         # LWC_DECODE_QROPE=0: the previous split (rope_kv_write rotates q in place), an A/B knob
-        q_at_load = os.environ.get("LWC_DECODE_QROPE", "1") != "0"
         rope = (self.cos, self.sin, positions) if q_at_load else None
         if cascade_tiles is not None:
             # fp8 o projection (config 5): the attention output leaves the kernel in MX form (ops.MXAct)

@@ -117,6 +117,17 @@ def embedding(table: torch.Tensor, ids: torch.Tensor, out: Optional[torch.Tensor
     return out
 
 
+def embedding_step(table: torch.Tensor, ids: torch.Tensor, per: int) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """The rows of a decode step: (rows [T, d] as :func:`embedding`, their sums of squares in partials [T, 4] for the first
+    projection (:func:`step_qkv`), cleared int32 counters [T, per] for :func:`paged_decode`)."""
+    T = ids.numel()
+    out = torch.empty(T, table.shape[1], dtype=table.dtype, device=table.device)
+    ss = torch.empty(T, 4, dtype=torch.float32, device=table.device)
+    counts = torch.empty(T, per, dtype=torch.int32, device=table.device)
+    kernels().embedding_step(table, ids, out, ss, counts)
+    return out, ss, counts
+
+
 def rope_kv_write(qkv: torch.Tensor, positions: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
                   k_cache: torch.Tensor, v_cache: torch.Tensor, Hq: int, Hkv: int, D: int,
                   slots: Optional[torch.Tensor] = None, rope_q: bool = True) -> None:
@@ -151,10 +162,12 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
                  ctx_lens: torch.Tensor, Hq: int, scale: float, num_splits: int = 1,
                  out: Optional[torch.Tensor] = None, part_o: Optional[torch.Tensor] = None,
                  part_lse: Optional[torch.Tensor] = None,
-                 rope: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None) -> torch.Tensor:
+                 rope: Optional[Tuple[torch.Tensor, torch.Tensor, torch.Tensor]] = None,
+                 counts: Optional[torch.Tensor] = None) -> torch.Tensor:
     """One-token paged GQA split-K decode attention (K3).  q: [B, >=Hq*D] (row stride allowed).  The
     engine's large batches of forked candidates use :func:`paged_decode_cascade` instead.  ``rope`` =
-    (cos, sin, positions [B] int32): q arrives un-rotated and is rotated at load."""
+    (cos, sin, positions [B] int32): q arrives un-rotated and is rotated at load.  ``counts`` [B, Hkv] int32, zero (and
+    left zero): the splits' sums meet in the same launch; calls that may run at once need counters of their own."""
     B = q.shape[0]
     D = k_cache.shape[-1]
     if out is None:
@@ -164,7 +177,7 @@ def paged_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, 
         part_lse = torch.empty(B * Hq * num_splits, dtype=torch.float32, device=q.device)
     rc, rs, rp = rope if rope is not None else (None, None, None)
     kernels().paged_decode(q, k_cache, v_cache, block_tables, ctx_lens, out, part_o, part_lse, int(num_splits),
-                           float(scale), rc, rs, rp)
+                           float(scale), rc, rs, rp, counts)
     return out
 
 
@@ -544,6 +557,37 @@ def skinny_gemm(A: torch.Tensor, W: torch.Tensor, residual: Optional[torch.Tenso
 
 def skinny_ok(M: int, N: int, K: int, swiglu: bool = False) -> bool:
     return 0 < M <= 256 and K % 64 == 0 and N % (64 if swiglu else 16) == 0
+
+
+def step_partials(core: int, d: int) -> int:
+    """Partial sums of squares per row that core 1 (:func:`skinny_gemm`) or 2 (:func:`gemm2w`) leaves of d columns; 0 where
+    the next projection does not take as many."""
+    n = 16 if core == 1 else 32
+    return d // n if d % (4 * n) == 0 and d // n <= 256 else 0
+
+
+def step_project(x: torch.Tensor, w: torch.Tensor, core: int, ss: torch.Tensor, eps: float, residual: Optional[torch.Tensor] = None,
+                 swiglu: bool = False, ws=None) -> torch.Tensor:
+    """A projection of a decode step of at most 64 rows with the RMSNorm folded into it (csrc/kernels/step_fuse.h): scales the
+    rows of ``x w^T`` (or of its gate and up halves, ``swiglu``) by 1 / rms from the partials ``ss`` [M, P], or adds into
+    ``residual`` in place and leaves its partials in ``ss``.  ``core``: 1 the weight stream, 2 the 64 x 64 tiles (with K ranges
+    over the workspace ``ws``)."""
+    out = residual if residual is not None else torch.empty(x.shape[0], w.shape[0] // 2 if swiglu else w.shape[0], dtype=x.dtype,
+                                                            device=x.device)
+    part, count = ws if ws is not None else (None, None)
+    kernels().step_project(x, w, out, residual, 2 if swiglu else 0 if residual is None else 1, int(core), ss, float(eps), part, count)
+    return out
+
+
+def step_qkv(x: torch.Tensor, w: torch.Tensor, core: int, ss: torch.Tensor, eps: float, positions: torch.Tensor, slots: torch.Tensor,
+             cos: torch.Tensor, sin: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, Hq: int, ws=None) -> torch.Tensor:
+    """The qkv projection of such a step: returns q [M, Hq * D], un-rotated (``rope=`` of :func:`paged_decode`); k is rotated,
+    k and v go into the paged cache at ``slots`` (< 0: nowhere).  The same rows as a norm, a projection and
+    :func:`rope_kv_write` leave, without the normalised rows' rounding."""
+    out = torch.empty(x.shape[0], Hq * k_cache.shape[3], dtype=x.dtype, device=x.device)
+    part, count = ws if ws is not None else (None, None)
+    kernels().step_qkv(x, w, out, positions, slots, cos, sin, k_cache, v_cache, int(core), ss, float(eps), part, count)
+    return out
 
 
 # gemm4w is switched off: its main loop was rewritten and the first headline run of the new build ended in a GPU fault

@@ -204,6 +204,17 @@ def swiglu(x: torch.Tensor, w_gu: torch.Tensor, block: int, ws=None) -> torch.Te
     return silu_mul(F.linear(x, w_gu), block=block)
 
 
+STEP_ROWS = 64
+
+
+def step_core(x: torch.Tensor, w: torch.Tensor, epi: str) -> int:
+    """The core of a decode step's projection as ``ops.step_project`` and ``ops.step_qkv`` number them, 0 where the choice at
+    these sizes is another one (the library; a shape no one tuned)."""
+    M, N = x.shape[0], w.shape[0]
+    b = choice(M, N, x.shape[1], epi)
+    return _NATIVE.get(b, 0) if M <= STEP_ROWS and _own_ok(b, x, N, x.shape[1], epi) else 0
+
+
 def _m_bucket(M: int) -> int:
     """Encoder token counts vary per call: tune per power-of-two bucket (everything >= 64k tokens is one)."""
     return min(1 << max(M - 1, 1).bit_length(), 1 << 16)
