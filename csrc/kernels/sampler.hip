@@ -1,21 +1,22 @@
 // K8a+K8b+K8c+K8d fused: logits processing, raw log-softmax + top-k logprobs, and top-k / top-p /
 // min-p / top-a filtered multinomial sampling (or greedy argmax) in ONE pass over each logits row.
 //
-// Bound by the one row a compute unit can hold (64 of 128 registers per lane), so that the row's load, 11 us at the CU's
-// share of the memory rate, and its passes take turns; every pass and every barrier counts.  4096 rows, one MI355X, us,
-// before -> after the passes lost their spilled registers (a row written to and read from scratch once more) and the
-// reductions their shuffles: vocabulary 128256 greedy 472 -> 208, temperature 0.8 345 -> 255, with top-p 0.95 452 -> 347,
-// with 20 logprobs 781 -> 592; vocabulary 32000 72 -> 43, 147 -> 63, 205 -> 97, 390 -> 240.
+// Bound by the row a compute unit holds: its load takes 11 us at the CU's share of the memory rate, its passes 8 us and more
+// (a round of exps 6, of masses 2).  Large batches of large vocabularies hold two rows per CU, 512 threads each with 23 of 32
+// slots in registers and 9 in LDS, so that the two overlap; thresholds are searched in a list of the few elements that can
+// matter, and a draw that carries 1 - top_p by itself is accepted without a pass.  4096 rows, one MI355X, us, before -> after
+// these: vocabulary 128256 greedy 208 -> 206, temperature 0.8 258 -> 229, with top-p 0.95 344 -> 280, with top-k 40 and top-p
+// 0.9 818 -> 403, with 20 logprobs 589 -> 399; vocabulary 32000 top-p 0.95 99 -> 83, top-k 240 -> 161, 20 logprobs 239 -> 166.
 //
-// One 1024-thread workgroup per row.  The row (bf16, V <= 8*1024*SLOTS) is loaded ONCE from HBM into
-// registers as packed bf16 (16 B per load, SLOTS loads per thread) and every later phase — raw max and
+// One workgroup per row, of 1024 threads or of 512 that stand for two each.  The row (bf16, V <= 8*1024*SLOTS) is
+// loaded ONCE from HBM as packed bf16 (16 B per load, SLOTS loads per thread) and every later phase — raw max and
 // log-sum-exp, the top-K selection for `top_logprobs`, penalties/bias/grammar mask, the filter
 // thresholds and the inverse-CDF draw — works on those registers plus block reductions.
 // Element index of (thread t, slot j, lane-element e) = (j*1024 + t)*8 + e.
 //
 // Thresholds are found by exact binary search over the 16-bit order-preserving key of the bf16 value
-// (16 block-reduction rounds), so top-p / top-k are exact (ties at the threshold are kept, as in the
-// usual "keep >= threshold" convention).  Randomness: Philox4x32-10 keyed by the per-sequence seed,
+// (over a list of the candidates, else 14 block-reduction rounds over the row), so top-p / top-k are exact (ties at the
+// threshold are kept, as in the usual "keep >= threshold" convention).  Randomness: Philox4x32-10 keyed by the per-sequence seed,
 // counter = per-sequence step — reproducible per (seed, step) independent of batch composition.
 //
 // Reference fields served: temperature/top_p/min_p/top_a/top_k/frequency_penalty/presence_penalty/
@@ -29,6 +30,7 @@ namespace lwc {
 constexpr int kSampT = 1024;
 constexpr int kMaxTopK = 20;
 constexpr int kCollect = 64;
+constexpr int kRegSlots = 23;  // of the 32 slots of the 512-thread build
 
 struct SampleParams {
   const bf16_t* logits;  // [B, ld]
@@ -90,19 +92,32 @@ LWC_DEVICE float key2f(uint32_t k) {
 // Keep the packed row opaque at the top of every pass: otherwise LICM hoists the 8*SLOTS unpacked
 // floats (or their keys) out of the binary-search loops and the kernel spills (1024 threads leave
 // 128 VGPRs per lane; the packed row alone is 4*SLOTS of them).
-#define OPAQUE_ROW(row)                                   \
-  _Pragma("unroll") for (int _j = 0; _j < SLOTS; ++_j) { \
-    asm volatile("" : "+v"(row[_j]));                     \
-  }
+#define OPAQUE_ROW(row)                                \
+  _Pragma("unroll") for (int _j = 0; _j < RS; ++_j) { \
+    asm volatile("" : "+v"(row[_j]));                  \
+  }                                                    \
+  if constexpr (LS > 0) asm volatile("" ::: "memory")  /* nor keep what an earlier pass read from LDS */
 
-// value of element e (0..7) of the row vector held in slot j (compile-time j, e: stays in VGPRs)
-#define GET(row, j, e) \
-  (((e)&1) ? __uint_as_float((row)[j][(e) >> 1] & 0xffff0000u) : __uint_as_float((row)[j][(e) >> 1] << 16))
+// The thread's slot s (compile-time s): the first RS in registers, the others in its own cells of LDS
+#define SLOT(s) ((s) < RS ? row[(s) < RS ? (s) : 0] : held[((s) < RS ? 0 : (s)-RS) * T + t])
+#define SET_SLOT(s, x)                                  \
+  do {                                                  \
+    if ((s) < RS) row[(s) < RS ? (s) : 0] = (x);        \
+    else held[((s) < RS ? 0 : (s)-RS) * T + t] = (x);   \
+  } while (0)
+// one slot's values live at a time, LDS slots read when their turn comes
+#define NEXT_SLOT()                                       \
+  do {                                                    \
+    __builtin_amdgcn_sched_barrier(0);                    \
+    if constexpr (LS > 0) asm volatile("" ::: "memory");  \
+  } while (0)
+// value of element e (0..7) of a slot (compile-time e)
+#define GET(x, e) (((e)&1) ? __uint_as_float((x)[(e) >> 1] & 0xffff0000u) : __uint_as_float((x)[(e) >> 1] << 16))
 
 // fp16 helpers for the probability form of the row (u in [0,1] as packed fp16)
 LWC_DEVICE uint16_t h2bits(float f) { return __builtin_bit_cast(uint16_t, (_Float16)f); }
-#define KEYU(row, j, e) ((((e)&1) ? ((row)[j][(e) >> 1] >> 16) : ((row)[j][(e) >> 1] & 0xffffu)))
-#define GETU(row, j, e) ((float)__builtin_bit_cast(_Float16, (uint16_t)KEYU(row, j, e)))
+#define KEYU(x, e) ((((e)&1) ? ((x)[(e) >> 1] >> 16) : ((x)[(e) >> 1] & 0xffffu)))
+#define GETU(x, e) ((float)__builtin_bit_cast(_Float16, (uint16_t)KEYU(x, e)))
 
 // Packed selection over the probability form (two non-negative fp16 u per register: their bit patterns
 // order like the values).  Per pair: a saturating 16-bit subtract against (threshold - 1) is >= 1 exactly
@@ -177,15 +192,21 @@ LWC_DEVICE float wave_scan(float x) {
 }
 
 // Block-wide reductions over two alternating sets of partials: one barrier each (a set is written again only behind the
-// next reduction's barrier, which every reader of it has passed)
+// next reduction's barrier, which every reader of it has passed).  The partials are those of the 16 waves of 1024 threads:
+// a thread that stands for two of them brings two values, so that a sum's order does not depend on the workgroup's size
+template <int VT>
 struct Red {
+  static constexpr int kW = kSampT / 64 / VT;  // waves
   float* f;  // [2][32]
   int ph;
   LWC_DEVICE float* set() { return f + 32 * (ph++ & 1); }
-  LWC_DEVICE float sum(float v) {
+  LWC_DEVICE float sum(const float (&x)[VT]) {
     float* sc = set();
-    v = row_sum4(row16_sum(v));
-    if ((threadIdx.x & 63) == 0) sc[threadIdx.x >> 6] = v;
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+      const float w = row_sum4(row16_sum(x[v]));
+      if ((threadIdx.x & 63) == 0) sc[(threadIdx.x >> 6) + v * kW] = w;
+    }
     __syncthreads();
     return row16_sum(sc[threadIdx.x & 15]);
   }
@@ -194,45 +215,95 @@ struct Red {
     v = row_max4(row16_max(v));
     if ((threadIdx.x & 63) == 0) sc[threadIdx.x >> 6] = v;
     __syncthreads();
-    return row16_max(sc[threadIdx.x & 15]);
+    return row16_max(sc[threadIdx.x & (kW - 1)]);
   }
   LWC_DEVICE int sum_i(int v) {
     int* sc = reinterpret_cast<int*>(set());
     v = row_sum4_i(row16_sum_i(v));
     if ((threadIdx.x & 63) == 0) sc[threadIdx.x >> 6] = v;
     __syncthreads();
-    return row16_sum_i(sc[threadIdx.x & 15]);
+    return row16_sum_i((threadIdx.x & 15) < kW ? sc[threadIdx.x & (kW - 1)] : 0);
+  }
+  // hi * 4096 + lo of the block, exact: |hi| < 2^21, 0 <= lo < 2^21 each
+  LWC_DEVICE double sum_wide(int hi, int lo) {
+    int* sc = reinterpret_cast<int*>(set());
+    hi = row_sum4_i(row16_sum_i(hi));
+    lo = row_sum4_i(row16_sum_i(lo));
+    if ((threadIdx.x & 63) == 0) {
+      sc[threadIdx.x >> 6] = hi;
+      sc[16 + (threadIdx.x >> 6)] = lo;
+    }
+    __syncthreads();
+    const bool on = (threadIdx.x & 15) < kW;
+    return (double)row16_sum_i(on ? sc[threadIdx.x & (kW - 1)] : 0) * 4096.0 + (double)row16_sum_i(on ? sc[16 + (threadIdx.x & (kW - 1))] : 0);
   }
 };
 static_assert(kSampT == 1024, "the reductions meet over 16 waves");
 
-// Lowest index among the thread's elements for which TEST(j, e) holds, 0x7fffffff if none.  Slot and element are kept
+// Lowest index among the thread's elements for which TEST(x, e) holds, 0x7fffffff if none.  Slot and element are kept
 // apart: both are inline constants, while an index per element would be 8 * SLOTS literals, each in a register of its own
 // ahead of the loop (100 spilled registers in the SLOTS = 16 build).
-#define LOWEST_INDEX(TEST, OUT)                                     \
-  do {                                                              \
-    int _bj = -1, _be = 0;                                          \
-    _Pragma("unroll") for (int j = SLOTS - 1; j >= 0; --j) {        \
-      int _e = 8;                                                   \
-      _Pragma("unroll") for (int e = 7; e >= 0; --e) _e = (TEST) ? e : _e; \
-      _bj = _e < 8 ? j : _bj;                                       \
-      _be = _e < 8 ? _e : _be;                                      \
-      __builtin_amdgcn_sched_barrier(0);                            \
-    }                                                               \
-    OUT = _bj >= 0 ? (_bj * kSampT + t) * 8 + _be : 0x7fffffff;     \
+#define LOWEST_INDEX(TEST, OUT)                                                  \
+  do {                                                                           \
+    OUT = 0x7fffffff;                                                            \
+    _Pragma("unroll") for (int v = 0; v < VT; ++v) {                             \
+      int _bj = -1, _be = 0;                                                     \
+      _Pragma("unroll") for (int j = SLOTS - 1; j >= 0; --j) {                   \
+        const uint4v x = SLOT(v * SLOTS + j);                                    \
+        int _e = 8;                                                              \
+        _Pragma("unroll") for (int e = 7; e >= 0; --e) _e = (TEST) ? e : _e;     \
+        _bj = _e < 8 ? j : _bj;                                                  \
+        _be = _e < 8 ? _e : _be;                                                 \
+        NEXT_SLOT();                                                             \
+      }                                                                          \
+      OUT = min(OUT, _bj >= 0 ? (_bj * kSampT + v * T + t) * 8 + _be : 0x7fffffff); \
+    }                                                                            \
   } while (0)
+
+// One wave: the largest key in [lo, hi] that at least K of the 1024 keys reach (lo if no larger one does)
+LWC_DEVICE uint32_t kth_of_1024(const uint32_t* keys, int lane, int K, uint32_t lo, uint32_t hi) {
+  uint32_t tk[kSampT / 64];
+#pragma unroll
+  for (int i = 0; i < kSampT / 64; ++i) tk[i] = keys[i * 64 + lane];
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi + 1) >> 1;
+    int c = 0;
+#pragma unroll
+    for (int i = 0; i < kSampT / 64; ++i) c += __popcll(__builtin_amdgcn_ballot_w64(tk[i] >= mid));
+    if (c >= K)
+      lo = mid;
+    else
+      hi = mid - 1;
+  }
+  return lo;
+}
+
+// A row's scalar as what it is, the same in every lane: loaded plainly the compiler takes it for a lane's own, both sides of
+// a branch on it are run one after the other, and the row stays live, in copies, through the side that does not need it
+LWC_DEVICE float uniform_f(float x) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(x))); }
 
 // PROC: a bias, a mask or penalties may apply to the rows; TOPK: num_logprobs > 0.  Builds of their own, so that a step
 // that asks for neither carries neither's registers.
-template <int SLOTS, bool PROC, bool TOPK>
-__global__ void __launch_bounds__(kSampT) sample_kernel(SampleParams p) {
+// T threads: 1024, or 512 of which each stands for two of the 1024 (element order, sums and draws are those of 1024: slot
+// v * SLOTS + j of thread t is slot j of thread v * T + t).  RS of the VT * SLOTS slots are in registers, the rest in LDS.
+template <int T, int SLOTS, int RS, bool PROC, bool TOPK>
+__global__ void __launch_bounds__(T, RS < SLOTS * (kSampT / T) ? 4 : SLOTS <= 4 && !PROC ? 8 : 4) sample_kernel(SampleParams p) {
+  constexpr int VT = kSampT / T, NS = SLOTS * VT, LS = NS - RS;
+  static_assert(!PROC || VT == 1, "processed rows are held by 1024 threads");
+  __shared__ uint4v held[LS > 0 ? LS * T : 1];
   __shared__ float sred[2 * 32];
   __shared__ int sredi[32];
   __shared__ int s_owner;
   __shared__ float s_cval[kCollect];
   __shared__ int s_cidx[kCollect];
   __shared__ int s_ccount;
-  __shared__ uint32_t s_tkey[kSampT];
+  // Two workgroups per compute unit: a threshold search over a list is one wave's, the other row has the unit meanwhile.
+  // One: every thread's (64 rows, top-p 0.95, 50 us by one wave, 35 by all; 4096 rows of 32000 in pairs 83 by one, 92 by all)
+  constexpr bool kPairs = LS > 0 || SLOTS <= 4;
+  constexpr int kList = LS > 0 ? 3456 : kPairs ? 2048 : 8192;  // 16-bit keys in LDS, which the pairs share
+  __shared__ uint32_t s_tkey[kList / 2];
+  uint16_t* const s_list = reinterpret_cast<uint16_t*>(s_tkey);
+  static_assert(kList >= 2 * kSampT, "s_tkey holds the maxima of 1024 threads too");
   __shared__ uint32_t s_lb, s_fkey;
   __shared__ uint32_t s_own[SLOTS * 4];
   __shared__ float s_oexcl;
@@ -240,38 +311,64 @@ __global__ void __launch_bounds__(kSampT) sample_kernel(SampleParams p) {
 
   const int b = blockIdx.x;
   const int t = threadIdx.x;
-  Red red{sred, 0};
+  Red<VT> red{sred, 0};
   const bf16_t* lrow = p.logits + (size_t)b * p.ld;
   const int nvec = p.V >> 3;
 
   // ---- load the raw row once ----
-  uint4v row[SLOTS];
+  uint4v row[RS];
   const uint32_t* lmask =
       (PROC && p.mask_logprobs && p.mask && p.mask_rows[b] >= 0) ? p.mask + (size_t)p.mask_rows[b] * (p.V >> 5) : nullptr;
+  if constexpr (VT == 1) {
 #pragma unroll
-  for (int j = 0; j < SLOTS; ++j) {
-    const int vi = j * kSampT + t;
-    row[j] = vi < nvec ? *reinterpret_cast<const uint4v*>(lrow + (size_t)vi * 8) : uint4v{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
-    if (lmask && vi < nvec) {  // constrained logprobs: disallowed tokens are -inf from the start
-      const uint32_t bits = (lmask[vi >> 2] >> ((vi & 3) * 8)) & 0xffu;
+    for (int j = 0; j < SLOTS; ++j) {
+      const int vi = j * kSampT + t;
+      row[j] = vi < nvec ? *reinterpret_cast<const uint4v*>(lrow + (size_t)vi * 8) : uint4v{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+      if (lmask && vi < nvec) {  // constrained logprobs: disallowed tokens are -inf from the start
+        const uint32_t bits = (lmask[vi >> 2] >> ((vi & 3) * 8)) & 0xffu;
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const uint32_t lo = (bits >> (2 * c)) & 1u ? (row[j][c] & 0xffffu) : 0xff80u;
-        const uint32_t hi = (bits >> (2 * c + 1)) & 1u ? (row[j][c] >> 16) : 0xff80u;
-        row[j][c] = lo | (hi << 16);
+        for (int c = 0; c < 4; ++c) {
+          const uint32_t lo = (bits >> (2 * c)) & 1u ? (row[j][c] & 0xffffu) : 0xff80u;
+          const uint32_t hi = (bits >> (2 * c + 1)) & 1u ? (row[j][c] >> 16) : 0xff80u;
+          row[j][c] = lo | (hi << 16);
+        }
       }
+    }
+  } else {
+    // the LDS slots by LDS-DMA first, then the registers'; vectors past the row's end read nothing (and become -inf below)
+    // (a resource per slot: one lane offset serves all of them)
+    const int w0 = __builtin_amdgcn_readfirstlane(t >> 6) * 64;
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      const int s = i < LS ? RS + i : i - LS, v0 = s % SLOTS * kSampT + s / SLOTS * T;
+      const __amdgpu_buffer_rsrc_t r = uniform_rsrc(lrow + v0 * 8, max(0, nvec - v0) * 16);
+      if (i < LS)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(held + i * T + w0), 16, t * 16, 0, 0, 0);
+      else
+        row[i < LS ? 0 : s] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(r, t * 16, 0, 0));
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RS) : "memory");
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      const int v0 = s % SLOTS * kSampT + s / SLOTS * T;
+      if (v0 + T > nvec && v0 + t >= nvec) SET_SLOT(s, (uint4v{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u}));
     }
   }
   // ---- raw max (+ each thread's own max key: the top-K search bound) and log-sum-exp ----
-  float mx = -INFINITY;
+  float mxv[VT];
 OPAQUE_ROW(row);
 #pragma unroll
-  for (int j = 0; j < SLOTS; ++j) {
+  for (int v = 0; v < VT; ++v) {
+    mxv[v] = -INFINITY;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) mx = fmaxf(mx, GET(row, j, e));
-    __builtin_amdgcn_sched_barrier(0);  // one slot's values live at a time
+    for (int j = 0; j < SLOTS; ++j) {
+      const uint4v x = SLOT(v * SLOTS + j);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) mxv[v] = fmaxf(mxv[v], GET(x, e));
+      NEXT_SLOT();  // one slot's values live at a time
+    }
   }
-  const uint32_t my_maxkey = f2key(mx);
+  const float mx = VT == 1 ? mxv[0] : fmaxf(mxv[0], mxv[VT - 1]);
   const float raw_max = red.max(mx);
   const int lane = t & 63, wid = t >> 6;
   const int K = TOPK ? p.num_logprobs : 0;
@@ -280,7 +377,7 @@ OPAQUE_ROW(row);
   // pass of its own, sampled ones too: formed in the sampling pass it doubles that pass's live values, and
   // the row spills.
   const bool need_lse = p.need_logprob || K > 0;
-  float se = 0.f;
+  float se[VT] = {};
 
   // ---- raw top-K (for top_logprobs): candidates collected here, ranked and written once the
   // log-sum-exp is known ----
@@ -292,24 +389,12 @@ OPAQUE_ROW(row);
     // search over the whole row run (starting from lb).  Masked (-inf, key 0x7f) entries are never
     // candidates: a row with < K finite values returns fewer (rest: id -1).
     if (t == 0) s_ccount = 0;
-    s_tkey[t] = my_maxkey;
+#pragma unroll
+    for (int v = 0; v < VT; ++v) s_tkey[v * T + t] = f2key(mxv[v]);
     __syncthreads();
     if (t < 64) {
-      uint32_t tk[kSampT / 64];
-#pragma unroll
-      for (int i = 0; i < kSampT / 64; ++i) tk[i] = s_tkey[i * 64 + t];
-      uint32_t lo = 0x80u, hi = 0xffffu;
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        int c = 0;
-#pragma unroll
-        for (int i = 0; i < kSampT / 64; ++i) c += __popcll(__builtin_amdgcn_ballot_w64(tk[i] >= mid));
-        if (c >= K)
-          lo = mid;
-        else
-          hi = mid - 1;
-      }
-      if (t == 0) s_lb = lo;
+      const uint32_t lb = kth_of_1024(s_tkey, lane, K, 0x80u, 0xffffu);
+      if (t == 0) s_lb = lb;
     }
     __syncthreads();
     uint32_t lo = s_lb;
@@ -322,10 +407,11 @@ OPAQUE_ROW(row);
           int c = 0;
 OPAQUE_ROW(row);
 #pragma unroll
-          for (int j = 0; j < SLOTS; ++j) {
+          for (int s = 0; s < NS; ++s) {
+            const uint4v x = SLOT(s);
 #pragma unroll
-            for (int e = 0; e < 8; ++e) c += f2key(GET(row, j, e)) >= mid;
-            __builtin_amdgcn_sched_barrier(0);  // one slot's values live at a time
+            for (int e = 0; e < 8; ++e) c += f2key(GET(x, e)) >= mid;
+            NEXT_SLOT();  // one slot's values live at a time
           }
           if (red.sum_i(c) >= K)
             lo = mid;
@@ -343,24 +429,25 @@ OPAQUE_ROW(row);
       const float thr = key2f(lo);
 OPAQUE_ROW(row);
 #pragma unroll
-      for (int j = 0; j < SLOTS; ++j) {
-        float top = GET(row, j, 0);
+      for (int s = 0; s < NS; ++s) {
+        const uint4v x = SLOT(s);
+        float top = GET(x, 0);
 #pragma unroll
-        for (int e = 1; e < 8; ++e) top = fmaxf(top, GET(row, j, e));
+        for (int e = 1; e < 8; ++e) top = fmaxf(top, GET(x, e));
         if (__builtin_amdgcn_ballot_w64(top >= thr)) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
-            const float v = GET(row, j, e);
+            const float v = GET(x, e);
             if (v >= thr && f2key(v) >= lo) {  // padding past V holds -inf (key 0x7f < lo): never collected
               const int slot = atomicAdd(&s_ccount, 1);
               if (slot < kCollect) {
                 s_cval[slot] = v;
-                s_cidx[slot] = (j * kSampT + t) * 8 + e;
+                s_cidx[slot] = (s % SLOTS * kSampT + s / SLOTS * T + t) * 8 + e;
               }
             }
           }
         }
-        __builtin_amdgcn_sched_barrier(0);
+        NEXT_SLOT();
       }
       __syncthreads();
       if (s_ccount <= kCollect) break;  // block-uniform
@@ -384,10 +471,10 @@ OPAQUE_ROW(row);
       if (vi >= nvec) continue;
       float y[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) y[e] = GET(row, j, e);
+      for (int e = 0; e < 8; ++e) y[e] = GET(row[j], e);
       if (need_lse) {
 #pragma unroll
-        for (int e = 0; e < 8; ++e) se += __expf(y[e] - raw_max);
+        for (int e = 0; e < 8; ++e) se[0] += __expf(y[e] - raw_max);
       }
       if (brow) {
         const float4 b0 = reinterpret_cast<const float4*>(brow + (size_t)vi * 8)[0];
@@ -416,19 +503,20 @@ OPAQUE_ROW(row);
     }
   }
 
-  const float T = p.temperature[b];
+  const float temp = uniform_f(p.temperature[b]);
   int token = 0;
   float raw_lse = __builtin_nanf("");
 OPAQUE_ROW(row);
   if (need_lse && !processed) {  // (in the passes below it would double their live values: spills)
 #pragma unroll
-    for (int j = 0; j < SLOTS; ++j) {
+    for (int s = 0; s < NS; ++s) {
+      const uint4v x = SLOT(s);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) se += __expf(GET(row, j, e) - raw_max);
-      __builtin_amdgcn_sched_barrier(0);
+      for (int e = 0; e < 8; ++e) se[s / SLOTS] += __expf(GET(x, e) - raw_max);
+      NEXT_SLOT();
     }
   }
-  if (T <= 0.f) {
+  if (temp <= 0.f) {
     if (need_lse) raw_lse = raw_max + __logf(red.sum(se));
     // ---- greedy: argmax (lowest index on ties).  The row maximum is known (the raw max; a processed row
     // takes one max pass), so the argmax is the lowest index holding it — instead of a value-and-index
@@ -438,10 +526,11 @@ OPAQUE_ROW(row);
     if (processed) {
       float ym = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < SLOTS; ++j) {
+      for (int s = 0; s < NS; ++s) {
+        const uint4v x = SLOT(s);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ym = fmaxf(ym, GET(row, j, e));
-        __builtin_amdgcn_sched_barrier(0);  // one slot's values live at a time
+        for (int e = 0; e < 8; ++e) ym = fmaxf(ym, GET(x, e));
+        NEXT_SLOT();  // one slot's values live at a time
       }
       gm = red.max(ym);
     }
@@ -449,29 +538,32 @@ OPAQUE_ROW(row);
     // one compare + one select per element, no branch
     int cand;
     if constexpr (PROC) { OPAQUE_ROW(row); }
-    LOWEST_INDEX(GET(row, j, e) == gm, cand);
+    NEXT_SLOT();
+    LOWEST_INDEX(GET(x, e) == gm, cand);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, 64));
     __syncthreads();
     if ((t & 63) == 0) sredi[t >> 6] = cand;
     __syncthreads();
-    cand = (t & 63) < (kSampT / 64) ? sredi[t & 63] : 0x7fffffff;
+    cand = (t & 63) < T / 64 ? sredi[t & 63] : 0x7fffffff;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, 64));
     token = cand == 0x7fffffff ? 0 : cand;
   } else {
-    const float invT = 1.f / T;
+    const float invT = 1.f / temp;
     float ymax = raw_max;  // unprocessed row: the processed max IS the raw max (no extra pass)
 OPAQUE_ROW(row);
     if (processed) {
       float ym = -INFINITY;
 #pragma unroll
-      for (int j = 0; j < SLOTS; ++j) {
+      for (int s = 0; s < NS; ++s) {
+        const uint4v x = SLOT(s);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) ym = fmaxf(ym, GET(row, j, e));
-        __builtin_amdgcn_sched_barrier(0);  // one slot's values live at a time
+        for (int e = 0; e < 8; ++e) ym = fmaxf(ym, GET(x, e));
+        NEXT_SLOT();  // one slot's values live at a time
       }
       ymax = red.max(ym);
+      mxv[0] = ym;
     }
     if (!(ymax > -INFINITY)) ymax = 0.f;  // every token masked: all u = 0 (the argmax fallback below)
     const uint32_t kOne2 = 0x00010001u, kH1 = 0x3C003C00u;
@@ -479,7 +571,7 @@ OPAQUE_ROW(row);
     // Non-negative fp16 bit patterns are order-preserving, so every later threshold search compares
     // raw 16-bit keys and sums fp16 values: no transcendental inside the searches.  The same pass
     // sums this thread's share of Z (over the ROUNDED values, as every later mass is).
-    float zloc = 0.f;
+    float zloc[VT] = {};
     // u = 2^(y * c1 + c0), c1 = log2(e) / T, c0 ~ -ymax * c1 rounded so that the exponent of y = ymax is
     // >= 0: with v_cvt_pkrtz (round toward zero) the max element is exactly 1.0 (0x3C00) and every other
     // element (at least one bf16 ulp below it, far above the fp32 rounding of c0) below 1; y = -inf gives
@@ -492,22 +584,29 @@ OPAQUE_ROW(row);
     const half2v ones2 = {(_Float16)1.f, (_Float16)1.f};
 OPAQUE_ROW(row);
 #pragma unroll
-    for (int j = 0; j < SLOTS; ++j) {
+    for (int s = 0; s < NS; ++s) {
+      uint4v x = SLOT(s);
+      float y[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = __builtin_fmaf(GET(x, e), c1, c0);
+      if constexpr (LS > 0) __builtin_amdgcn_sched_barrier(0);  // (8 exps in a row: two waves per SIMD wait for each other's)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = __builtin_amdgcn_exp2f(y[e]);
+      if constexpr (LS > 0) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
-        const float y0 = GET(row, j, 2 * c), y1 = GET(row, j, 2 * c + 1);
-        const auto h = __builtin_amdgcn_cvt_pkrtz(__builtin_amdgcn_exp2f(__builtin_fmaf(y0, c1, c0)),
-                                                  __builtin_amdgcn_exp2f(__builtin_fmaf(y1, c1, c0)));
-        const uint32_t w = __builtin_bit_cast(uint32_t, h);
-        zloc = __builtin_amdgcn_fdot2(as_h2(w), ones2, zloc, false);
-        row[j][c] = w;
+        const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(y[2 * c], y[2 * c + 1]));
+        zloc[s / SLOTS] = __builtin_amdgcn_fdot2(as_h2(w), ones2, zloc[s / SLOTS], false);
+        x[c] = w;
       }
-      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (LS > 0) asm volatile("" : "+v"(zloc[s / SLOTS]));  // (else the sums wait for the end, with every slot live)
+      SET_SLOT(s, x);
+      NEXT_SLOT();
     }
     // Z: from the scan of the first draw where that runs over every element and nothing needs it earlier (no top-k,
     // no top-a: the usual case), else a reduction of its own
-    const int k = p.top_k[b];
-    const float mp = p.min_p[b], ta = p.top_a[b];
+    const int k = __builtin_amdgcn_readfirstlane(p.top_k[b]);
+    const float mp = uniform_f(p.min_p[b]), ta = uniform_f(p.top_a[b]);
     const bool z_from_scan = k <= 0 && !(ta > 0.f) && !(mp > 0.f);
     float Z = 0.f;
     if (need_lse) raw_lse = raw_max + __logf(red.sum(se));
@@ -518,31 +617,110 @@ OPAQUE_ROW(row);
   do {                                                                                 \
     OPAQUE_ROW(row);                                                                   \
     const uint32_t _t2 = thr1x2(KEY);                                                  \
-    float _s = 0.f;                                                                    \
-    _Pragma("unroll") for (int j = 0; j < SLOTS; ++j) {                                \
-      mass2(_s, row[j][0], row[j][1], _t2, kOne2, kH1);                                \
-      mass2(_s, row[j][2], row[j][3], _t2, kOne2, kH1);                                \
+    _Pragma("unroll") for (int v = 0; v < VT; ++v) {                                   \
+      float _s = 0.f;                                                                  \
+      _Pragma("unroll") for (int j = 0; j < SLOTS; ++j) {                              \
+        const uint4v x = SLOT(v * SLOTS + j);                                          \
+        mass2(_s, x[0], x[1], _t2, kOne2, kH1);                                        \
+        mass2(_s, x[2], x[3], _t2, kOne2, kH1);                                        \
+      }                                                                                \
+      OUT[v] = dot_read(_s);                                                           \
     }                                                                                  \
-    OUT = dot_read(_s);                                                                \
   } while (0)
 #define MASS_GE(KEY, OUT)        \
   do {                           \
-    float _l;                    \
+    float _l[VT];                \
     MASS_LOCAL(KEY, _l);         \
     OUT = red.sum(_l);           \
+  } while (0)
+    // The keys in [LO, HI] (LO >= 1) go to s_list if they are at most kList, thread by thread; N: how many they are.  A search
+    // over the list takes 2 us, over the row 14 rounds of 1.3 (counts) or 2 us (masses).
+#define COLLECT(LO, HI, N)                                                             \
+  do {                                                                                 \
+    OPAQUE_ROW(row);                                                                   \
+    const uint32_t _a = thr1x2(LO), _b = thr1x2((HI) + 1u);                            \
+    uint32_t _ca = 0u, _cb = 0u;                                                       \
+    _Pragma("unroll") for (int s = 0; s < NS; ++s) {                                   \
+      const uint4v x = SLOT(s);                                                        \
+      count2(_ca, x[0], x[1], _a, kOne2);                                              \
+      count2(_ca, x[2], x[3], _a, kOne2);                                              \
+      count2(_cb, x[0], x[1], _b, kOne2);                                              \
+      count2(_cb, x[2], x[3], _b, kOne2);                                              \
+      NEXT_SLOT();                                                                     \
+    }                                                                                  \
+    const float _c = (float)((int)((_ca & 0xffffu) + (_ca >> 16)) - (int)((_cb & 0xffffu) + (_cb >> 16))); \
+    const float _i = wave_scan(_c);                                                    \
+    float* _sc = red.set();                                                            \
+    if (lane == 63) _sc[wid] = _i;                                                     \
+    __syncthreads();                                                                   \
+    float _off = _i - _c, _tot = 0.f;                                                  \
+    for (int w = 0; w < T / 64; ++w) {                                                 \
+      const float sw = _sc[w];                                                         \
+      _off += w < wid ? sw : 0.f;                                                      \
+      _tot += sw;                                                                      \
+    }                                                                                  \
+    N = __builtin_amdgcn_readfirstlane((int)_tot);                                     \
+    if (N <= kList && __builtin_amdgcn_ballot_w64(_c > 0.f)) {                         \
+      int _p = (int)_off;                                                              \
+      _Pragma("unroll") for (int s = 0; s < NS; ++s) {                                 \
+        const uint4v x = SLOT(s);                                                      \
+        _Pragma("unroll") for (int e = 0; e < 8; ++e) {                                \
+          const uint32_t kk = KEYU(x, e);                                              \
+          if (kk - (LO) <= (HI) - (LO)) s_list[_p++] = (uint16_t)kk;                   \
+        }                                                                              \
+        NEXT_SLOT();                                                                   \
+      }                                                                                \
+    }                                                                                  \
+    __syncthreads();                                                                   \
   } while (0)
     uint32_t tau_k = 0;  // top-k: keep elements with key >= tau_k
     if (k > 0) {
       uint32_t lo = 0, hi = 0x3C00u;  // keys of [0, 1.0]
+      // Few (k <= 1024): the k largest of the threads' own maxima bound the k-th largest element from below (0: fewer than
+      // k threads hold any mass); the elements from there on, rarely more than a few times k, are searched in a list
+      if (k <= kSampT) {
+#pragma unroll
+        for (int v = 0; v < VT; ++v) {
+          const float um = __builtin_amdgcn_exp2f(__builtin_fmaf(mxv[v], c1, c0));
+          s_tkey[v * T + t] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_pkrtz(um, um)) & 0xffffu;
+        }
+        __syncthreads();
+        if (t < 64) {
+          const uint32_t lb = kth_of_1024(s_tkey, lane, k, 0u, hi);
+          if (t == 0) s_lb = lb;
+        }
+        __syncthreads();
+        lo = __builtin_amdgcn_readfirstlane(s_lb);
+        const uint32_t from = max(lo, 1u);
+        int n;
+        COLLECT(from, hi, n);
+        if (n <= kList) {
+          if (t < 64) {  // (one wave: the list is short)
+            while (lo < hi) {
+              const uint32_t mid = (lo + hi + 1) >> 1;
+              int c = 0;
+              for (int i = 0; i < n; i += 64) c += __popcll(__builtin_amdgcn_ballot_w64(i + lane < n && s_list[i + lane] >= mid));
+              if (c >= k)
+                lo = mid;
+              else
+                hi = mid - 1;
+            }
+            if (t == 0) s_lb = lo;
+          }
+          __syncthreads();
+          lo = hi = __builtin_amdgcn_readfirstlane(s_lb);
+        }
+      }
       while (lo < hi) {
         const uint32_t mid = (lo + hi + 1) >> 1;
         const uint32_t t2 = thr1x2(mid);
         uint32_t c2 = 0u;
 OPAQUE_ROW(row);
 #pragma unroll
-        for (int j = 0; j < SLOTS; ++j) {
-          count2(c2, row[j][0], row[j][1], t2, kOne2);
-          count2(c2, row[j][2], row[j][3], t2, kOne2);
+        for (int s = 0; s < NS; ++s) {
+          const uint4v x = SLOT(s);
+          count2(c2, x[0], x[1], t2, kOne2);
+          count2(c2, x[2], x[3], t2, kOne2);
         }
         if (red.sum_i((int)((c2 & 0xffffu) + (c2 >> 16))) >= k)
           lo = mid;
@@ -564,9 +742,11 @@ OPAQUE_ROW(row);
     // over {key >= max(tau_p, L0)} — the result is again exactly distributed (the fallback does not
     // depend on the rejected draw).  Saves the ~14 block-wide passes of a threshold search per row in
     // the common case.
-    const float tp = p.top_p[b];
+    const float tp = uniform_f(p.top_p[b]);
     float target = 0.f;
-    if (tp < 1.f && !z_from_scan) {
+    // (where the first draw runs over exactly the top-k set its total is that mass)
+    const bool target_from_scan = z_from_scan || (tau_k > 0u && L0 == tau_k);
+    if (tp < 1.f && !target_from_scan) {
       float mk = Z;
       if (tau_k > 0u) MASS_GE(tau_k, mk);
       target = tp * mk;
@@ -579,57 +759,73 @@ OPAQUE_ROW(row);
 #pragma unroll 1
     for (int attempt = 0; attempt < 2; ++attempt) {
       // ---- inverse-CDF draw over {key >= tau} (order: thread-major, then slot, then element) ----
-      float local = 0.f;
-      if (tau <= 1u)
-        local = zloc;  // every positive element is kept: the thread's share of Z
-      else
+      float local[VT], excl[VT];
+      if (tau <= 1u) {
+#pragma unroll
+        for (int v = 0; v < VT; ++v) local[v] = zloc[v];  // every positive element is kept: the thread's share of Z
+      } else {
         MASS_LOCAL(tau, local);
+      }
       // exclusive scan of `local` over threads
-      const float incl = wave_scan(local);
       float* sc = red.set();
-      if (lane == 63) sc[wid] = incl;
+#pragma unroll
+      for (int v = 0; v < VT; ++v) {
+        excl[v] = wave_scan(local[v]);
+        if (lane == 63) sc[wid + v * (T / 64)] = excl[v];
+      }
       if (t == 0) s_owner = 0x7fffffff;
       __syncthreads();
-      float wave_off = 0.f, total = 0.f;
+      float wave_off[VT] = {}, total = 0.f;
 #pragma unroll
       for (int w = 0; w < kSampT / 64; ++w) {
         const float sw = sc[w];
-        if (w < wid) wave_off += sw;
+#pragma unroll
+        for (int v = 0; v < VT; ++v)
+          if (w < wid + v * (T / 64)) wave_off[v] += sw;
         total += sw;
       }
-      if (z_from_scan && attempt == 0) target = tp * total;  // (the first draw's total is Z)
-      const float excl = wave_off + incl - local;
+#pragma unroll
+      for (int v = 0; v < VT; ++v) excl[v] = wave_off[v] + excl[v] - local[v];
+      if (target_from_scan && attempt == 0) target = tp * total;
       const float u01 = (((attempt == 0 ? ctr[0] : ctr[1]) >> 8) + 0.5f) * (1.0f / 16777216.0f);
       const float u = u01 * total;
       // The owner: the lowest thread whose [excl, excl + local) holds u — or, when rounding put u at or
       // past the end, the last thread with mass (its last kept element is taken).  Its packed u go to
       // LDS and its wave walks them (two elements per dword, an exclusive scan over the lanes) instead
       // of a single lane stepping through 8 * SLOTS elements with a branch each.
-      if (local > 0.f && u >= excl && u < excl + local) atomicMin(&s_owner, t);
+#pragma unroll
+      for (int v = 0; v < VT; ++v)
+        if (local[v] > 0.f && u >= excl[v] && u < excl[v] + local[v]) atomicMin(&s_owner, v * T + t);
       __syncthreads();
       int owner = s_owner;  // block-uniform
       const bool past_end = owner == 0x7fffffff;
       if (past_end) {
-        int lastt = local > 0.f ? t : -1;
+        int lastt = -1;
+#pragma unroll
+        for (int v = 0; v < VT; ++v) lastt = local[v] > 0.f ? v * T + t : lastt;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) lastt = max(lastt, __shfl_xor(lastt, o, 64));
         if (lane == 0) sredi[wid] = lastt;
         __syncthreads();
-        lastt = lane < (kSampT / 64) ? sredi[lane] : -1;
+        lastt = lane < T / 64 ? sredi[lane] : -1;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) lastt = max(lastt, __shfl_xor(lastt, o, 64));
         owner = lastt;
       }
       found = 0x7fffffff;
       if (owner >= 0) {
-        if (wid == (owner >> 6)) {  // the owner's wave: its LDS writes are its own reads' (in order, no barrier)
-          if (t == owner) {
+        if (wid == ((owner & (T - 1)) >> 6)) {  // the owner's wave: its LDS writes are its own reads' (in order, no barrier)
 #pragma unroll
-            for (int j = 0; j < SLOTS; ++j)
+          for (int v = 0; v < VT; ++v)
+            if (v * T + t == owner) {
 #pragma unroll
-              for (int c = 0; c < 4; ++c) s_own[j * 4 + c] = row[j][c];
-            s_oexcl = excl;
-          }
+              for (int j = 0; j < SLOTS; ++j) {
+                const uint4v x = SLOT(v * SLOTS + j);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) s_own[j * 4 + c] = x[c];
+              }
+              s_oexcl = excl[v];
+            }
           __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
           __builtin_amdgcn_wave_barrier();
           __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
@@ -683,19 +879,21 @@ OPAQUE_ROW(row);
         float bv = -INFINITY;
 OPAQUE_ROW(row);
 #pragma unroll
-        for (int j = 0; j < SLOTS; ++j)
+        for (int s = 0; s < NS; ++s) {
+          const uint4v x = SLOT(s);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) bv = fmaxf(bv, GETU(row, j, e));  // padding past V has u = 0 < u_max = 1
+          for (int e = 0; e < 8; ++e) bv = fmaxf(bv, GETU(x, e));  // padding past V has u = 0 < u_max = 1
+        }
         const float gm = red.max(bv);
         int cand;
 OPAQUE_ROW(row);
-        LOWEST_INDEX(GETU(row, j, e) == gm, cand);
+        LOWEST_INDEX(GETU(x, e) == gm, cand);
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, 64));
         __syncthreads();
         if (lane == 0) sredi[wid] = cand;
         __syncthreads();
-        cand = lane < (kSampT / 64) ? sredi[lane] : 0x7fffffff;
+        cand = lane < T / 64 ? sredi[lane] : 0x7fffffff;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) cand = min(cand, __shfl_xor(cand, o, 64));
         found = cand == 0x7fffffff ? 0 : cand;
@@ -703,25 +901,68 @@ OPAQUE_ROW(row);
       }
       if (!check) break;
       // ---- nucleus test of the draw (s_fkey: the drawn element's key, written by the walk) ----
-      const uint32_t ks = s_fkey;
+      const uint32_t ks = __builtin_amdgcn_readfirstlane(s_fkey);
+      // What lies above is kept too, so it is no more than the rest: an element that carries enough itself needs no sum.
+      // (The margin is wider than the sums' rounding, 256 terms each: what the sum would answer is what this answers)
+      const float rest = total - (float)__builtin_bit_cast(_Float16, (uint16_t)ks);
+      if (__builtin_amdgcn_readfirstlane(rest * 1.0001f < target)) break;
       float above;
       MASS_GE(ks + 1u, above);
       if (above < target) break;  // accepted (block-uniform)
       // rejected: tau_p > ks.  Exact search for the largest key with mass(>= key) >= target.
+      // The keys left in the interval go to a list once they are few; until then rounds over the row halve it.
       uint32_t lo = ks + 1u, hi = 0x3C00u;
-      while (lo < hi) {
+      float over = 0.f;  // the mass above hi
+      for (int round = 0; lo < hi; ++round) {
+        if (round % 4 == 0) {
+          int n;
+          COLLECT(lo, hi, n);
+          if (n <= kList) {
+            // masses as whole numbers of 2^-24 (every fp16 u is one): exact in any order
+            const double want = ((double)target - (double)over) * 16777216.0;
+            if (!kPairs || t < 64) {
+              while (lo < hi) {
+                const uint32_t mid = (lo + hi + 1) >> 1;
+                uint32_t c = 0;
+#pragma unroll 4
+                for (int i = t; i < n; i += kPairs ? 64 : T) {
+                  const uint16_t kk = s_list[i];
+                  c += kk >= mid ? (uint32_t)((float)__builtin_bit_cast(_Float16, kk) * 16777216.f) : 0u;
+                }
+                double m;
+                if constexpr (kPairs)
+                  m = (double)row_sum4_i(row16_sum_i((int)(c >> 16))) * 65536.0 + (double)row_sum4_i(row16_sum_i((int)(c & 0xffffu)));
+                else
+                  m = red.sum_wide((int)(c >> 12), (int)(c & 4095u));
+                if (__builtin_amdgcn_readfirstlane(m >= want))
+                  lo = mid;
+                else
+                  hi = mid - 1;
+              }
+              if (kPairs && t == 0) s_lb = lo;
+            }
+            if constexpr (kPairs) {
+              __syncthreads();
+              lo = hi = __builtin_amdgcn_readfirstlane(s_lb);
+            }
+            break;
+          }
+        }
         const uint32_t mid = (lo + hi + 1) >> 1;
         float mm;
         MASS_GE(mid, mm);
-        if (mm >= target)
+        if (__builtin_amdgcn_readfirstlane(mm >= target)) {
           lo = mid;
-        else
+        } else {
           hi = mid - 1;
+          over = mm;
+        }
       }
       tau = max(lo, L0);
       check = false;
     }
 #undef MASS_GE
+#undef COLLECT
     token = found;
   }
   if (TOPK && t < 64) {  // one wave: rank-sort the collected top-K candidates (value desc, index asc)
@@ -774,12 +1015,19 @@ extern "C" int lwc_sample(const void* logits, int ld, int V, int B, const float*
   const bool proc = bias || mask || counts;
 #define LWC_SAMPLE(S)                                                                                                \
   do {                                                                                                               \
-    if (proc && num_logprobs > 0) sample_kernel<S, true, true><<<B, kSampT, 0, s>>>(p);                              \
-    else if (proc) sample_kernel<S, true, false><<<B, kSampT, 0, s>>>(p);                                            \
-    else if (num_logprobs > 0) sample_kernel<S, false, true><<<B, kSampT, 0, s>>>(p);                                \
-    else sample_kernel<S, false, false><<<B, kSampT, 0, s>>>(p);                                                     \
+    if (proc && num_logprobs > 0) sample_kernel<kSampT, S, S, true, true><<<B, kSampT, 0, s>>>(p);                   \
+    else if (proc) sample_kernel<kSampT, S, S, true, false><<<B, kSampT, 0, s>>>(p);                                 \
+    else if (num_logprobs > 0) sample_kernel<kSampT, S, S, false, true><<<B, kSampT, 0, s>>>(p);                     \
+    else sample_kernel<kSampT, S, S, false, false><<<B, kSampT, 0, s>>>(p);                                          \
   } while (0)
-  if (slots <= 4)
+  // 65537 to 131072 tokens, plain rows: two rows per compute unit from four rows per unit on, so that one's load goes on under
+  // the other's passes; a thread of a pair does twice the work, and with fewer rows their latency is what counts
+  // (128256 tokens, us, one row per unit against two: 64 rows top-p 0.95 35 / 61, 512 72 / 77, 1024 104 / 101, 4096 300 / 280;
+  // 4096 rows greedy 206 / 206, temperature alone 258 / 229, top-k 40 537 / 403, 20 logprobs 511 / 399)
+  if (slots > 8 && slots <= 16 && !proc && B >= 1024) {
+    if (num_logprobs > 0) sample_kernel<512, 16, kRegSlots, false, true><<<B, 512, 0, s>>>(p);
+    else sample_kernel<512, 16, kRegSlots, false, false><<<B, 512, 0, s>>>(p);
+  } else if (slots <= 4)
     LWC_SAMPLE(4);
   else if (slots <= 8)
     LWC_SAMPLE(8);

@@ -69,6 +69,8 @@ def _torch_flags(name: str = "_kernels") -> tuple[list[str], list[str]]:
 # 32-key tile).
 PER_FILE_FLAGS = {f: ["-mllvm", "-amdgpu-mfma-vgpr-form=1"] for f in ("attention_prefill.hip", "attention_decode.hip",
                                                                       "wattn.hip", "wattn_decode_wide.hip", "retention.hip")}
+# the sampler's two accumulators per thread, paired up into vectors, keep both halves' operands in registers: 270 spills
+PER_FILE_FLAGS["sampler.hip"] = ["-fno-slp-vectorize"]
 
 
 # hipcc -O3 forms packed fp32 instructions by itself from scalar float code; this keeps it from doing so.  ``_res32`` is
