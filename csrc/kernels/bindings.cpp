@@ -16,6 +16,9 @@ int lwc_rope_kv_write(void*, const int*, const int*, const float*, const float*,
                       int, int, hipStream_t);
 int lwc_silu_mul(const void*, void*, int, int, int, hipStream_t);
 int lwc_embedding_gather(const void*, const int*, void*, int, int, int, hipStream_t);
+int lwc_encoder_few_ok(int, int, int, int);
+int lwc_encoder_few(const void*, const void*, const int*, const int*, int, int, const void*, const void*, float, const void* const*, int,
+                    const int*, int, int, int, int, int, float, float*, void*, void*, void*, void*, hipStream_t);
 int lwc_embedding_step(const void*, const int*, void*, float*, int*, int, int, int, int, hipStream_t);
 int lwc_kv_block_copy(void*, const int*, int, int, int, long long, hipStream_t);
 int lwc_kv_gather(const void*, const void*, const long long*, void*, void*, int, int, int, int, hipStream_t);
@@ -913,6 +916,38 @@ c10::optional<at::Tensor> encoder_layers(at::Tensor x, const std::vector<at::Ten
   return x;
 }
 
+// A post-norm encoder over few packed rows, embeddings to last hidden rows (encoder_few.hip): weights as encoder_layers takes
+// them.  Nothing, and nothing launched, for shapes, counts of rows or layouts that those kernels do not take.
+c10::optional<at::Tensor> encoder_few(const at::Tensor& word, const at::Tensor& pos, const at::Tensor& ids, const at::Tensor& positions,
+                                      const at::Tensor& g, const at::Tensor& b, const std::vector<at::Tensor>& weights,
+                                      const at::Tensor& cu, int64_t H, double scale, double eps) {
+  if (weights.empty() || weights.size() % 12 != 0 || word.dim() != 2 || ids.dim() != 1) return c10::nullopt;
+  const int64_t T = ids.size(0), d = word.size(1), f = weights[6].dim() == 2 ? weights[6].size(0) : 0;
+  if (T > 4096 || !lwc_encoder_few_ok((int)T, (int)d, (int)H, (int)f)) return c10::nullopt;
+  const std::vector<std::vector<int64_t>> sizes = {{3 * d, d}, {3 * d}, {d, d}, {d}, {d}, {d}, {f, d}, {f}, {d, f}, {d}, {d}, {d}};
+  auto bf16 = [&](const at::Tensor& t, at::IntArrayRef size) {
+    return t.device() == word.device() && t.is_contiguous() && t.scalar_type() == at::kBFloat16 && t.sizes() == size && ((uintptr_t)t.data_ptr() & 15) == 0;
+  };
+  auto ints = [&](const at::Tensor& t) { return t.device() == word.device() && t.is_contiguous() && t.scalar_type() == at::kInt && t.dim() == 1; };
+  if (!word.is_cuda() || !bf16(word, word.sizes()) || pos.dim() != 2 || pos.size(1) != d || !bf16(pos, pos.sizes()) || !bf16(g, {d}) ||
+      !bf16(b, {d}) || !ints(ids) || !ints(positions) || positions.size(0) != T || !ints(cu) || cu.size(0) < 2 || cu.size(0) > 64 || word.size(0) == 0 ||
+      pos.size(0) == 0 || word.size(0) > INT_MAX || pos.size(0) > INT_MAX)
+    return c10::nullopt;
+  std::vector<const void*> w(weights.size());
+  for (size_t i = 0; i < weights.size(); ++i) {
+    if (!bf16(weights[i], sizes[i % 12])) return c10::nullopt;
+    w[i] = weights[i].data_ptr();
+  }
+  at::Tensor x = at::empty({T, d}, word.options()), a = at::empty({T, d}, word.options()), h = at::empty({T, f}, word.options());
+  at::Tensor part = at::empty({4, T, d}, word.options().dtype(at::kFloat)), y = at::empty({T, d}, word.options());
+  CHECK_RC(lwc_encoder_few(word.data_ptr(), pos.data_ptr(), ids.data_ptr<int>(), positions.data_ptr<int>(), (int)word.size(0),
+                           (int)pos.size(0), g.data_ptr(), b.data_ptr(), (float)eps, w.data(), (int)(w.size() / 12), cu.data_ptr<int>(),
+                           (int)cu.size(0) - 1, (int)T, (int)d, (int)H, (int)f, (float)scale, part.data_ptr<float>(), x.data_ptr(),
+                           y.data_ptr(), a.data_ptr(), h.data_ptr(), cur_stream()),
+           "encoder_few");
+  return x;
+}
+
 void prefill_attention_mx(const at::Tensor& q, const at::Tensor& k, const at::Tensor& v, at::Tensor& out8, at::Tensor& mx,
                           const at::Tensor& cu_seqlens, int64_t max_seqlen, int64_t Hq, int64_t Hkv, double scale,
                           bool causal) {
@@ -1152,6 +1187,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("set_decode_wave_min_items", &lwc_set_decode_wave_min_items,
         "B*Hkv*splits threshold of the wave-per-item decode kernel; returns the previous value");
   m.def("prefill_attention", &prefill_attention);
+  m.def("encoder_few", &encoder_few, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("encoder_layers", &encoder_layers, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("prefill_attention_mx", &prefill_attention_mx);
   m.def("prefill_attention_paged", &prefill_attention_paged);

@@ -529,6 +529,14 @@ def encoder_layers(x: torch.Tensor, weights: Sequence[torch.Tensor], cu: torch.T
                                     bool(fuse_f), part, count)
 
 
+def encoder_few(word: torch.Tensor, pos: torch.Tensor, ids: torch.Tensor, positions: torch.Tensor, g: torch.Tensor, b: torch.Tensor,
+                weights: Sequence[torch.Tensor], cu: torch.Tensor, H: int, scale: float, eps: float) -> Optional[torch.Tensor]:
+    """The last hidden rows of a post-norm encoder over few packed rows (csrc/kernels/encoder_few.hip), from the embedding
+    tables on; ``g`` / ``b``: the embeddings' norm, ``weights`` 12 tensors a layer as :func:`encoder_layers` takes them.
+    None, and nothing done, for other shapes, layouts or more rows than those kernels take."""
+    return kernels().encoder_few(word, pos, ids, positions, g, b, weights, cu, int(H), float(scale), float(eps))
+
+
 def gemm2w_ok(N: int, K: int, *operands: Optional[torch.Tensor], swiglu: bool = False) -> bool:
     """Whether :func:`gemm2w` takes a call: its sizes, and 16-byte rows and pointers of every operand."""
     return K % 64 == 0 and N % (64 if swiglu else 8) == 0 and all(

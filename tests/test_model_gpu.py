@@ -420,3 +420,37 @@ def test_folded_norms_keep_encode_and_logits_with_real_norm_weights(gpu):
     la = a.prefill(toks, pos, pos, cu, P, last, KVCache(cfg, 16, 16, gpu)).float()
     lb = b.prefill(toks, pos, pos, cu, P, last, KVCache(cfg, 16, 16, gpu)).float()
     assert _cos(la, lb) > 0.9995
+
+
+@pytest.mark.parametrize("arch", ["bge-small-en-v1.5", "bge-base-en-v1.5", "bge-large-en-v1.5"])
+@pytest.mark.parametrize("lens", [[1], [12], [16], [17], [32], [5, 1, 9], [3, 13, 1, 15], [1] * 32])
+def test_few_row_encoder_matches_reference(gpu, monkeypatch, arch, lens):
+    """The encoder's kernels for few rows at the edges of their row tiles and of texts within them, against the fp32 layers:
+    no further off than the general kernels are, but for the spread of two roundings (2 x).  A weight at an odd address is
+    left to the general ones."""
+    from llm_weighted_consensus_amd import ops
+    from llm_weighted_consensus_amd.models import bert
+    from llm_weighted_consensus_amd.models.config import encoder_config
+
+    m = bert.BertEncoder(encoder_config(arch), device=gpu, seed=5)
+    for L in m.layers:   # biases and gains that matter
+        for n in ("bqkv", "bo", "b1", "b2", "ln1_b", "ln2_b"):
+            getattr(L, n).normal_(0.0, 0.1)
+        L.ln1_g.normal_(1.0, 0.1)
+        L.ln2_g.normal_(1.0, 0.1)
+    args = m.pack([[(37 * i + 11 * j) % 900 + 1 for j in range(n)] for i, n in enumerate(lens)])
+    taken, few = [], ops.encoder_few
+    monkeypatch.setattr(ops, "encoder_few", lambda *a: taken.append(few(*a)) or taken[-1])
+    y = m.forward_packed(*args)
+    assert len(taken) == 1 and taken[0] is y
+    monkeypatch.undo()
+    ref = m.forward_reference(*args[:3])
+    monkeypatch.setattr(bert, "FEW_ROWS", 0)
+    plain = m.forward_packed(*args)
+    err = lambda t: ((t.float() - ref).norm() / ref.norm()).item()  # noqa: E731
+    assert err(y) < 2 * err(plain) and err(y) < 0.03, (err(y), err(plain))
+    monkeypatch.setattr(bert, "FEW_ROWS", 32)
+    w = m.layers[-1].w2
+    m.layers[-1].w2 = torch.cat([w.flatten()[:1], w.flatten()])[1:].view(w.shape)   # two bytes off
+    assert ops.encoder_few(m.word, m.pos_type, args[0], args[1], m.emb_ln_g, m.emb_ln_b,
+                           [t for L in m.layers for t in bert._layer_tensors(L)], args[2], m.cfg.heads, m.scale, 1e-12) is None
