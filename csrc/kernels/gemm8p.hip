@@ -7,7 +7,8 @@
 //
 // Tile pipeline (cdna_hip_programming.md §5 "The 256² 8-phase template", written for this kernel's operand split):
 //   workgroup : 8 waves (512 threads) = 2 (M) x 4 (N); wave tile 128 x 64 = 8 x 4 MFMA 16x16 tiles,
-//               mfma_f32_16x16x32_bf16, 128 fp32 accumulators per lane.
+//               mfma_f32_16x16x32_bf16, 128 fp32 accumulators per lane.  Row tiles of 224 and 192 (R1 = 3, 2, row_tile): the
+//               second quadrant has R1 instead of 4 tiles of 16 rows, the rest of unit A1 is not loaded.
 //   K tile    : BK = 64 (128 B per row), staged global -> LDS by LDS-DMA (global_load_lds_dwordx4) in four
 //               16 KiB UNITS, each of which is exactly what one compute phase reads:
 //                 A0 = rows {0..63, 128..191}   (quadrant mi=0 of both wave rows)
@@ -60,6 +61,7 @@ constexpr int kUnitB = 128 * 128;   // 128 rows x 128 B
 constexpr int kBufB = 4 * kUnitB;   // one K tile: A0 A1 B0 B1
 constexpr int kLdsB = 2 * kBufB;    // 128 KiB
 constexpr int kUA0 = 0, kUA1 = kUnitB, kUB0 = 2 * kUnitB, kUB1 = 3 * kUnitB;
+constexpr int kDeep = 2;  // 16-row tiles of a partial that the finaliser has in flight: 8 loads (4 were a longer chain, 16 spill)
 constexpr int kPartialF = 256 * 256;  // fp32 partial tile per workgroup
 
 enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4 };
@@ -106,8 +108,9 @@ LWC_DEVICE void tile_mn(const Params& p, int t, int& m, int& n) {
   n = in / gsz;
 }
 
-template <int EPI>
+template <int EPI, int R1>
 __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
+  constexpr int BMH = 64 + 16 * R1;  // rows of a wave row
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int KT = p.KT;
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
@@ -135,7 +138,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
     }
     int tm, tn;
     tile_mn(p, tile, tm, tn);
-    const int m0 = tm * 256, n0 = tn * 256;
+    const int m0 = tm * 2 * BMH, n0 = tn * 256;
     // Lane geometry is re-derived per item from an opaque copy of threadIdx.x: hoisted out of the
     // item loop, the ~100 epilogue / fragment addresses it feeds would stay live and spill.
     int tid = threadIdx.x;
@@ -152,7 +155,8 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
     for (int i = 0; i < 2; ++i)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        voA[h][i] = (uint32_t)(((i * 128 + h * 64 + (tid >> 3)) * p.lda + chk) * 2);
+        // (R1 < 4: the rest of unit A1 lies past the resource's end, no memory request)
+        voA[h][i] = h == 0 || (tid >> 3) < 16 * R1 ? (uint32_t)(((i * BMH + h * 64 + (tid >> 3)) * p.lda + chk) * 2) : 0x60000000u;
         voW[h][i] = (uint32_t)((((2 * i + (tid >> 8)) * 64 + h * 32 + ((tid >> 3) & 31)) * p.K + chk) * 2);
       }
     const int dst_lane0 = wid * 64 * 16;  // wave-uniform LDS destination of instruction 0 inside a unit
@@ -161,7 +165,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
 
     // buffer descriptors of the tile's A rows / W rows: rows past M / N fall outside num_records and
     // load as zeros (their outputs are not stored)
-    const __amdgpu_buffer_rsrc_t rA = uniform_rsrc(p.A + (size_t)m0 * p.lda, (p.M - m0) * p.lda * 2);
+    const __amdgpu_buffer_rsrc_t rA = uniform_rsrc(p.A + (size_t)m0 * p.lda, min(p.M - m0, 2 * BMH) * p.lda * 2);
     const __amdgpu_buffer_rsrc_t rW = uniform_rsrc(p.W + (size_t)n0 * p.K, min(p.N - n0, 256) * p.K * 2);
     auto stage = [&](int u, uint8_t* buf, int kt) {
 #pragma unroll
@@ -180,9 +184,9 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
 
     // acc[i][jj] = 16 x 16 tile (i, jj) of the wave's 128 x 64 (lane: rows 4q..4q+3 of column r16).
     // (The 32x32x16 MFMA with the same units and phases measured ~10 % slower on every shape.)
-    float4v acc[8][4];
+    float4v acc[4 + R1][4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 4 + R1; ++i)
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) acc[i][jj] = float4v{0.f, 0.f, 0.f, 0.f};
 
@@ -191,13 +195,13 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < (i0 == 0 ? 4 : R1); ++i)
 #pragma unroll
           for (int jj = 0; jj < 2; ++jj) acc[i0 + i][j0 + jj] = mfma(a[i][s], bb[jj][s], acc[i0 + i][j0 + jj]);
     };
     auto rdA = [&](const uint8_t* buf, int u) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) rd(buf + u, wr * 64 + i * 16, a[i][0], a[i][1]);
+      for (int i = 0; i < (u == kUA0 ? 4 : R1); ++i) rd(buf + u, wr * 64 + i * 16, a[i][0], a[i][1]);
     };
     auto rdB = [&](const uint8_t* buf, int u, uint4v (&bb)[2][2]) {
 #pragma unroll
@@ -259,7 +263,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
     if (khi < KT) {  // contributor: publish the fp32 partial, no store of C
       float4v* wsp = reinterpret_cast<float4v*>(p.ws + (size_t)blockIdx.x * kPartialF);
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < 4 + R1; ++i)
 #pragma unroll
         for (int jj = 0; jj < 4; ++jj) wsp[(wid * 32 + i * 4 + jj) * 64 + lane] = acc[i][jj];
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -287,12 +291,23 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
           __hip_atomic_store(p.flags + blk, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
-        const float4v* wsq = reinterpret_cast<const float4v*>(p.ws + (size_t)blk * kPartialF);
+        const __amdgpu_buffer_rsrc_t rP = uniform_rsrc(p.ws + (size_t)blk * kPartialF, kPartialF * 4);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+        for (int i0 = 0; i0 < 4 + R1; i0 += kDeep) {
+          float4v part[kDeep][4];
 #pragma unroll
-          for (int jj = 0; jj < 4; ++jj) acc[i][jj] += wsq[(wid * 32 + i * 4 + jj) * 64 + lane];
-          __builtin_amdgcn_sched_barrier(0);  // 4 loads in flight at a time: no 128-VGPR load burst
+          for (int i = 0; i < kDeep; ++i)
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj)
+              if (i0 + i < 4 + R1)
+                part[i][jj] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rP, lane * 16, (wid * 32 + (i0 + i) * 4 + jj) * 1024, 0));
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int i = 0; i < kDeep; ++i)
+#pragma unroll
+            for (int jj = 0; jj < 4; ++jj)
+              if (i0 + i < 4 + R1) acc[i0 + i < 4 + R1 ? i0 + i : 0][jj] += part[i][jj];
+          __builtin_amdgcn_sched_barrier(0);
         }
         if (pa <= tile_begin) break;
       }
@@ -305,7 +320,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
     constexpr int NJ = CW / 16;
     if constexpr (EPI == EPI_SWIGLU) {
 #pragma unroll
-      for (int i = 0; i < 8; ++i)
+      for (int i = 0; i < 4 + R1; ++i)
 #pragma unroll
         for (int jj = 0; jj < 2; ++jj)
 #pragma unroll
@@ -319,7 +334,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
         const int col = n0 + wc * 64 + jj * 16 + r16;
         const float bv = col < p.N ? bf2f(p.R[col]) : 0.f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < 4 + R1; ++i)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const float y = acc[i][jj][r] + bv;
@@ -329,7 +344,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
     }
     bf16_t* ot = reinterpret_cast<bf16_t*>(smem) + wid * 128 * CW;
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+    for (int i = 0; i < 4 + R1; ++i)
 #pragma unroll
       for (int jj = 0; jj < NJ; ++jj)
 #pragma unroll
@@ -347,11 +362,11 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
       // residual rows through a buffer resource (rows past M read zeros, no request), all of a group's loads
       // in flight before the first add — inside the store's bounds branch each 16 B load waited its own
       // HBM round trip
-      const int row0 = m0 + wr * 128;
-      const int rows_here = max(0, min(p.M - row0, 128));
+      const int row0 = m0 + wr * BMH;
+      const int rows_here = max(0, min(p.M - row0, BMH));
       const __amdgpu_buffer_rsrc_t rR = uniform_rsrc(p.R + (size_t)row0 * p.ldc, rows_here * p.ldc * 2);
       const int gn = ncol0 + cch * 8;
-      constexpr int kIt = 128 / RPI, kGrp = kIt < 16 ? kIt : 16;
+      constexpr int kIt = BMH / RPI, kGrp = kIt < 16 ? kIt : 16;
       static_assert(kIt % kGrp == 0, "residual epilogue groups must tile the wave's rows");
 #pragma unroll 1
       for (int k0 = 0; k0 < kIt; k0 += kGrp) {
@@ -374,9 +389,9 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
       }
     } else {
 #pragma unroll 4
-      for (int k = 0; k < 128 / RPI; ++k) {
+      for (int k = 0; k < BMH / RPI; ++k) {
         const int row = lane / CPR + RPI * k;
-        const int gm = m0 + wr * 128 + row;
+        const int gm = m0 + wr * BMH + row;
         const int gn = ncol0 + cch * 8;
         if (gm < p.M && gn < ncols)
           *reinterpret_cast<uint4v*>(p.C + (size_t)gm * p.ldc + gn) =
@@ -387,15 +402,20 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
   }
 }
 
-template <int EPI>
+template <int EPI, int R1>
 int launch(const Params& p, hipStream_t s) {
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)gemm8p_kernel<EPI>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsB);
+    (void)hipFuncSetAttribute((const void*)gemm8p_kernel<EPI, R1>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsB);
     attr = true;
   }
-  gemm8p_kernel<EPI><<<8 * p.wpx, 512, kLdsB, s>>>(p);
+  gemm8p_kernel<EPI, R1><<<8 * p.wpx, 512, kLdsB, s>>>(p);
   return (int)hipGetLastError();
+}
+
+template <int EPI>
+int launch(const Params& p, int r1, hipStream_t s) {
+  return r1 == 4 ? launch<EPI, 4>(p, s) : r1 == 3 ? launch<EPI, 3>(p, s) : launch<EPI, 2>(p, s);
 }
 
 // Experiment knob (A/B in one process, scripts/microbench.py g8ab): LWC_G8_GM, the tile group height
@@ -413,6 +433,32 @@ int device_cus() {
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 8) cus = 256;
   }
   return cus;
+}
+
+// Workgroups per XCD: at least ~8 K iterations per stream-K workgroup, so small problems get a smaller grid.
+int grid_wpx(int tiles, int KT) {
+  const int wpx = device_cus() / 8;
+  const long long iters = (long long)tiles * KT;
+  return iters < 8LL * 8 * wpx ? (int)std::max(1LL, iters / 64) : wpx;
+}
+
+// The row tile (R1: 256, 224 or 192 rows).  256 rows are 1.56 us per K iteration and round, 224 0.89 and 192 0.83 of that
+// (28672 x 4096 and 4096 x 14336, whole rounds of tiles), so a smaller one pays where it saves rows past M: 1095 rows are five
+// tiles either way.  To it comes the hand-off of the tiles cut between workgroups (256 KiB through one compute unit each way):
+// over whole rounds 10 us and 45 times the last round's share, with fewer tiles than workgroups 15 us a part, 10 if all are cut
+// evenly.  The rule's choice, us, against 256 rows: gate|up 28672 x 4096 of 520 / 1095 / 1300 / 3333 rows 137 / 222 / 274 / 615
+// for 163 / 238 / 304 / 624, down 4096 x 14336 of 520 / 1095 / 1300 / 2200 rows 97 / 137 / 147 / 221 for 112 / 165 / 159 / 238.
+int row_tile(int M, int tiles_n, int KT) {
+  constexpr double kIter = 1.56, kCost[5] = {0, 0, 0.83, 0.89, 1.0};
+  int best = 4;
+  double least = 0;
+  for (int r1 = 4; r1 >= 2; --r1) {
+    const int bm = 128 + 32 * r1, tiles = (M + bm - 1) / bm * tiles_n, G = 8 * grid_wpx(tiles, KT), rest = tiles % G;
+    const double cut = rest == 0 ? 0 : tiles > G ? 10 + 45.0 * rest / G : G % tiles == 0 ? 10 : 15.0 * G / tiles;
+    const double us = kCost[r1] * kIter * KT * tiles / G + cut;
+    if (r1 == 4 || us < least) best = r1, least = us;
+  }
+  return best;
 }
 
 }  // namespace g8p
@@ -433,12 +479,8 @@ extern "C" int lwc_gemm8p(const void* A, const void* W, void* C, const void* R, 
   if (epi == EPI_SWIGLU && N % 64 != 0) return -1;
   if ((epi == EPI_RESIDUAL || epi == EPI_BIAS || epi == EPI_BIAS_GELU) && R == nullptr) return -1;
   if (M == 0 || N == 0) return 0;
-  const int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256, tiles = tiles_m * tiles_n, KT = K / 64;
-  int wpx = device_cus() / 8;
-  // at least ~8 K iterations per stream-K workgroup: shrink the grid for small problems
-  const long long iters = (long long)tiles * KT;
-  if (iters < 8LL * 8 * wpx) wpx = (int)std::max(1LL, iters / 64);
-  const int G = 8 * wpx;
+  const int tiles_n = (N + 255) / 256, KT = K / 64, r1 = lda < (1 << 20) ? row_tile(M, tiles_n, KT) : 4;
+  const int bm = 128 + 32 * r1, tiles_m = (M + bm - 1) / bm, tiles = tiles_m * tiles_n, wpx = grid_wpx(tiles, KT), G = 8 * wpx;
   int sk = 0, dp = tiles / G;
   if (tiles % G != 0) {
     dp = std::max(0, tiles / G - 1);
@@ -447,11 +489,11 @@ extern "C" int lwc_gemm8p(const void* A, const void* W, void* C, const void* R, 
   Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, ws, flags,
            M, N, K, lda, ldc, tiles_m, tiles_n, KT, std::max(1, env_int("LWC_G8_GM", 8)), wpx, sk, dp};
   switch (epi) {
-    case EPI_PLAIN: return launch<EPI_PLAIN>(p, s);
-    case EPI_RESIDUAL: return launch<EPI_RESIDUAL>(p, s);
-    case EPI_SWIGLU: return launch<EPI_SWIGLU>(p, s);
-    case EPI_BIAS: return launch<EPI_BIAS>(p, s);
-    case EPI_BIAS_GELU: return launch<EPI_BIAS_GELU>(p, s);
+    case EPI_PLAIN: return launch<EPI_PLAIN>(p, r1, s);
+    case EPI_RESIDUAL: return launch<EPI_RESIDUAL>(p, r1, s);
+    case EPI_SWIGLU: return launch<EPI_SWIGLU>(p, r1, s);
+    case EPI_BIAS: return launch<EPI_BIAS>(p, r1, s);
+    case EPI_BIAS_GELU: return launch<EPI_BIAS_GELU>(p, r1, s);
   }
   return -1;
 }

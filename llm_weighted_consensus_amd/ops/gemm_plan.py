@@ -87,8 +87,12 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
     Many rows of a gate|up projection: the library needs a SwiGLU pass over its [M, N] result, gemm8p none. Beyond 8192
     rows, N x K 8192 x 1024 to 27648 x 5120: 0.65 to 1.02; from 4609 rows on N decides how full the last round of tiles is:
     14336 x 2048, 8192 and 16384 x 1024, 16384 x 2048, 22016 and 28672 x 4096, 27648 x 5120 0.72 to 1.01, but 8192 x 4096
-    0.65 to 1.09, 11264 x 4096 0.76 to 1.07, 9216 x 1152 up to 1.09, 4096 x 2048 up to 1.24. Fewer rows: either way (28672 x
-    4096, 4500: 817 and 840 us, 2200: 416 and 459, 3333: 706 and 622). 32768 x 8192: 0.90 to 1.05.
+    0.65 to 1.09, 11264 x 4096 0.76 to 1.07, 9216 x 1152 up to 1.09, 4096 x 2048 up to 1.24. 32768 x 8192: 0.90 to 1.05.
+
+    Hundreds of rows, where gemm8p's row tile fits them (22 counts of 545 to 3600): gate|up 22016 and 28672 x 4096, 27648 x 5120
+    0.65 to 1.04 from 545 to 1900 rows and 0.75 to 0.98 from 2401 to 3600, between them up to 1.10, fewer columns either way
+    (14336 x 4096 0.74 to 1.17, 8192 x 4096 0.88 to 1.20), 32768 x 4096 up to 1.11. Down into 16 column tiles, 4096 x 11008 and
+    14336: 0.53 to 1.00 from 545 to 1900 rows; 2048 x 14336 up to 1.15, 5120 x 13824 1.10, 8192 x 14336 1.11, 4096 x 8192 1.14.
 
     Few rows (prefill: a batch of prompts' last layer runs on their last tokens only, and short prompts on few rows
     everywhere): the weight's read bounds them. gate|up, which saves its SwiGLU pass, up to 64 rows on gemm2w: 11264, 14336
@@ -103,7 +107,11 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
         if M > 4608:  # (M * N: 32-bit byte offsets)
             wide = N >= (8192 if M > 8192 or K <= 1024 else 14336)
             return "g8" if wide and 1 << 23 <= size < 1 << 28 and M * N < 1 << 30 else "blas"
+        if 22016 <= N <= 28672 and 4096 <= K <= 5120 and (544 < M <= 1900 or 2400 < M <= 3600):
+            return "g8"
         return "g2" if M <= 64 and N >= 8192 and K <= 4096 and 1 << 25 <= size <= 1 << 27 else "blas"
+    if epi == "residual" and 3840 < N <= 4096 and 11008 <= K <= 14336 and 544 < M <= 1900:
+        return "g8"
     if M <= 16 and K <= 4096 and N <= 8 * K and 1 << 22 <= size <= 1 << 24:
         return "gv"
     return "g2" if 32 < M <= 64 and (N < 8192 or K <= 2048) and 1 << 24 <= size <= 1 << 26 else "blas"
