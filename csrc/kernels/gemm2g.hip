@@ -37,6 +37,7 @@ struct Params {
   const uint8_t* a_mx;
   uint8_t* mx_out;
   int s_rows;
+  int turned;  // a tile's walk over K starts at a step of its own
 };
 
 LWC_DEVICE float4v mfma8(const uint4v& a0, const uint4v& a1, const uint4v& b0, const uint4v& b1, const float4v& c, int sb) {
@@ -118,7 +119,10 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
   // kMxA: the rows' scales of a step, four bytes (its blocks of 32) a row
   const uint32_t voS = m_begin + tid < m_end ? (uint32_t)((m_begin + tid) * 4) : 0x7fffffffu;
   const __amdgpu_buffer_rsrc_t rS = uniform_rsrc(p.a_mx, MXA ? (p.K / 128) * p.s_rows * 4 : 0);
-  auto stage = [&](uint8_t* buf, int kt) {
+  const int nk = p.K / 128, live = m_end - m_begin;
+  const int k0 = p.turned ? (int)((unsigned)(3 * (ntile >> 3) + 15 * g) % (unsigned)nk) : 0;
+  auto stage = [&](uint8_t* buf, int step) {
+    const int kt = step + k0 < nk ? step + k0 : step + k0 - nk;
 #pragma unroll
     for (int i = 0; i < IA; ++i) dma16(rA, buf + (i * 4 + wid) * 1024, voA[i], kt * 128);
 #pragma unroll
@@ -143,7 +147,6 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) acc[i][c][h] = float4v{0.f, 0.f, 0.f, 0.f};
 
-  const int nk = p.K / 128, live = m_end - m_begin;
 #pragma unroll
   for (int k = 0; k < NST; ++k)
     if (k < nk) stage(smem + k * kStage, k);
@@ -265,8 +268,8 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
                               int rows, int mode, const void* a_mx, void* mx_out, int s_rows, hipStream_t s) {
   using namespace lwc::g2g;
   if ((!row_off && G != 1) || K % 128 != 0 || K < 128 || N % 8 != 0 || rows <= 0) return -1;
-  const Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, a_scale, w_scale, G, N, K, lda, ldc, rows_a,
-                 rows, 0, 0, (const uint8_t*)a_mx, (uint8_t*)mx_out, s_rows};
+  Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, a_scale, w_scale, G, N, K, lda, ldc, rows_a,
+                 rows, 0, 0, (const uint8_t*)a_mx, (uint8_t*)mx_out, s_rows, 0};
   // The tile that most groups' rows fit, with room for an uneven routing: a second tile reads the weights again, and where the
   // columns give every CU a workgroup already some CUs walk K once more.  us at 64 / 128 / 192 rows a tile, 32 rows a group: bf16
   // [4096, 14336] x 8 (256 columns) 164 / 166 / 172, one expert with four times the rows 238 / 190 / 193, with 130 rows 254 /
@@ -275,6 +278,13 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
   // 34 / 42 / 46.  More, where it is one of many: bf16 [14336, 4096] x 8 (896) 204 / 203 / 205, four times 190 / 193 / 202.
   // Dense (no table): tiles of 64 rows while they give a CU two workgroups at most, else of 128.
   const int per = (rows + G - 1) / G;
+  // 128 rows of a stride whose low bits are zero lie on few memory channels, and all tiles walk K in step: starting each tile's
+  // walk at another step of K spreads them.  bf16, 8 experts of 8 / 64 rows, us, before -> after: [4096, 8192] 148 / 137 -> 97 /
+  // 99, [14336, 4096] 199 / 210 -> 165 / 181, [4096, 2048] 33 / 36 -> 25 / 28, [14336, 6144] 273 / 299 -> 243 / 271; rows of 11008
+  // and 22016 bytes, [4096, 5504] 78 / 88 -> 67 / 74, [4096, 11008] 148 / 160 -> 126 / 140; 3072, 5120 and 7168 bytes level.  Odd
+  // multiples of 2048 bytes gain nothing (14336: 82 / 94 -> 85 / 95).  With many rows the tiles of a row tile no longer share its
+  // rows' way through L2: [14336, 4096] at 160 rows 236 -> 254, but [4096, 4096] 72 -> 66.
+  p.turned = (K % 4096 == 0 || K % 2048 != 0) && (per <= 104 || (row_off && N <= 4096 && per <= 192));
   const long long nt = (N + 127) / 128, cols = nt * G;
   int tm = per <= (cols <= 128 ? 44 : 16) ? 64 : per <= 104 && !(cols > 128 && cols <= 256) ? 128 : 192;
   if (!row_off) tm = nt * ((rows + 63) / 64) <= 512 ? 64 : 128;

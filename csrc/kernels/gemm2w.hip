@@ -35,6 +35,7 @@ struct Params {
   int* count;   // [tiles] finished ranges (zero between launches)
   RowSumsq ss;  // NORM: read by EPI_PLAIN, EPI_SWIGLU and EPI_ROPE_KV, written by EPI_RESIDUAL
   RopeKV kv;    // EPI_ROPE_KV
+  int turned;   // a tile's walk over its K range starts at a step of its own
 };
 
 LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
@@ -97,7 +98,10 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
     const int row = (i * 4 + wid) * 8 + (lane >> 3);
     voW[i] = row < rows_n ? (uint32_t)((row + (EPI == EPI_ROPE_KV && row >= 32 ? far : 0)) * p.K * 2 + (((lane & 7) ^ ((row >> 3 & 3) * 2 + (row >> 1 & 1))) << 4)) : 0x7fffffffu;
   }
-  auto stage = [&](uint8_t* buf, int kt) {
+  const int KT = p.K / 64, k0 = KT * split / p.splits, nk = KT * (split + 1) / p.splits - k0;
+  const int turn0 = p.turned ? (int)((unsigned)(in / gsz * 3) % (unsigned)nk) : 0;
+  auto stage = [&](uint8_t* buf, int step) {
+    const int kt = k0 + (step + turn0 < nk ? step + turn0 : step + turn0 - nk);
 #pragma unroll
     for (int i = 0; i < IA; ++i) dma16(rA, buf + (i * 4 + wid) * 1024, voA[i], kt * 128);
 #pragma unroll
@@ -135,10 +139,9 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
   RopeAhead<8> ahead;
   if constexpr (EPI == EPI_ROPE_KV) rope_kv_row(p.kv, ahead, min(m0 + wr * 16 + r16, p.M - 1), n0 / p.kv.D);
   __builtin_amdgcn_sched_barrier(0);
-  const int KT = p.K / 64, k0 = KT * split / p.splits, nk = KT * (split + 1) / p.splits - k0;
 #pragma unroll
   for (int k = 0; k < NST; ++k)  // (NORM: steps past the range too, rows that nothing reads: behind a branch the sums would wait for all)
-    if (NORM || k < nk) stage(smem + k * kStage, k0 + k);
+    if (NORM || k < nk) stage(smem + k * kStage, k);
   __builtin_amdgcn_sched_barrier(0);
   if constexpr (EPI == EPI_ROPE_KV) rope_kv_angles(p.kv, ahead, n0 / p.kv.D, n0 % p.kv.D + 8 * q);
   if constexpr (kScale) {
@@ -176,7 +179,7 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();  // every wave holds the step's operands: its buffer takes the step after next
     asm volatile("" ::: "memory");
-    if (kt + NST < nk) stage(buf, k0 + kt + NST);
+    if (kt + NST < nk) stage(buf, kt + NST);
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -326,6 +329,12 @@ int launch(Params p, hipStream_t s) {
   (void)attr;
   p.tiles_m = (p.M + TM - 1) / TM;
   p.tiles_n = (p.N + TN - 1) / TN;
+  // W rows of a stride whose low bits are zero lie on few memory channels, and all tiles walk K in step (gemm2g.hip): another
+  // first step for each column tile spreads them.  N x K at 24 / 64 / 128 rows, us, before -> after: 16384 x 2048 17 / 17 / 26 -> 15 /
+  // 15 / 23, 28672 x 4096 50 / 54 / 59 -> 48 / 52 / 51, 32000 x 4096 55 / 57 / 64 -> 55 / 57 / 52, 8192 x 8192 33 / 33 / 44 -> 27 /
+  // 29 / 42, 4096 x 11008 23 / 25 / 35 -> 21 / 24 / 33; 4096 x 14336 and 6144 x 4096 level.  Many rounds of tiles spread by
+  // themselves (128256 x 4096 185 / 202 / 212 -> 199 / 213 / 217), and from 300 rows on the matrix cores are the bound.
+  p.turned = p.M <= 256 && (long long)p.tiles_m * p.tiles_n <= 1024 && (p.K % 2048 == 0 || p.K % 1024 != 0);
   gemm2w_kernel<EPI, TM, TN, NST, NORM><<<p.tiles_m * p.tiles_n * p.splits, 256, kLds, s>>>(p);
   return (int)hipGetLastError();
 }
@@ -382,7 +391,7 @@ extern "C" int lwc_gemm2w(const void* A, const void* W, void* C, const void* R, 
   if (M == 0 || N == 0) return 0;
   if (((long long)M + 63) / 64 * ((N + 63) / 64) * splits >= (1LL << 31)) return -1;
   const Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc, 0, 0,
-                 splits, part, count, ss != nullptr ? *ss : lwc::RowSumsq{}, kv != nullptr ? *kv : lwc::RopeKV{}};
+                 splits, part, count, ss != nullptr ? *ss : lwc::RowSumsq{}, kv != nullptr ? *kv : lwc::RopeKV{}, 0};
   if (ss != nullptr) switch (epi) {
     case EPI_PLAIN: return launch<EPI_PLAIN, 64, 64, 4, true>(p, s);
     case EPI_RESIDUAL: return launch<EPI_RESIDUAL, 64, 64, 4, true>(p, s);

@@ -319,8 +319,8 @@ def grouped_gemm(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tensor, max_sl
     K over that many workgroups per tile (fp32 atomics into a workspace, then one bf16 pass); default:
     chosen so a small-M launch (MoE decode down projection: 8 experts x 32 column tiles) still puts
     ~4 workgroups on every CU.  That is the 128-row kernel's; by their sizes (bf16: :func:`_grouped_bf16`,
-    fp8 from 32 rows per group: ``weight_bound`` in csrc/kernels/gemm8g.hip) calls run on tiles of 64 to 192
-    rows (csrc/kernels/gemm2g.hip) or the 8-phase 256-row tiles (csrc/kernels/gemm8g.hip) instead.
+    fp8: :func:`_few_fp8`, from 32 rows per group on ``weight_bound`` in csrc/kernels/gemm8g.hip) calls run on tiles of 64 to
+    192 rows (csrc/kernels/gemm2g.hip) or the 8-phase 256-row tiles (csrc/kernels/gemm8g.hip) instead.
     ``swiglu=True``: W's rows are gate / up interleaved in blocks of 32 (:func:`swiglu_interleave` per group)
     and the result is silu(gate) * up [rows, N/2] — from those two kernels' epilogues when one of them takes
     the batch, else GEMM + the SwiGLU pass.  ``a_mx`` [K/128, rows, 4] uint8: A carries MX block scales (from
@@ -339,12 +339,13 @@ def grouped_gemm(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tensor, max_sl
             out = torch.empty(rows, N // 2 if swiglu else N, dtype=torch.bfloat16, device=A.device)
         kernels().gemm8g_bf16(A, W, out, row_off, -(-rows // 256) + G, a_rows, bool(swiglu), core)
         return out
-    if _use_gemm8g(A, W, rows, G, N, K, bias, splits, out) and (not swiglu or N % 64 == 0):
-        # fp8 expert batches of 32 rows per expert and more: the 8-phase kernel or the small tiles, by sizes
+    few = rows < 32 * G and max_slots is None and _few_fp8(rows, G, N, K) and _few_fp8_layout(A, W, rows, N, K, out, a_rows, a_scale, w_scale)
+    if _use_gemm8g(A, W, rows, G, N, K, bias, splits, out, few) and (not swiglu or N % 64 == 0):
+        # fp8 expert batches: of few rows per expert the small tiles, else the 8-phase kernel or the small tiles, by sizes
         if out is None:
             out = torch.empty(rows, N // 2 if swiglu else N, dtype=torch.bfloat16, device=A.device)
         kernels().gemm8g_fp8(A, W, out, row_off, -(-rows // 256) + G, a_rows, a_scale, w_scale.contiguous(),
-                             int(bool(swiglu)), None, None, _moe_core())
+                             int(bool(swiglu)), None, None, _moe_core() or (2 if few else 0))
         return out
     if swiglu:
         return silu_mul(grouped_gemm(A, W, row_off, max_slots=max_slots, a_scale=a_scale, w_scale=w_scale,
@@ -401,6 +402,30 @@ def moe_mx_ok(A: torch.Tensor, W13: torch.Tensor, W2: torch.Tensor, rows: int) -
     return rows * (N // 2) < (1 << 31) and (N // 256) * rows * 4 < (1 << 31)
 
 
+def _hit_groups(rows: int, G: int) -> float:
+    """How many of G groups a routing of few rows reaches, each row any group alike."""
+    return float(G) if rows >= 4 * G else G * (1.0 - (1.0 - 1.0 / G) ** rows)
+
+
+def _few_fp8(rows: int, G: int, N: int, K: int) -> bool:
+    """Whether an fp8 call of less than 32 rows per group (row scales) takes the small tiles instead of the 128-row kernel, which
+    splits K over workgroups: where the tiles that the routing reaches are enough for the length of K.  us on one MI355X, N x K x
+    groups at 0.25 / 0.5 / 1 / 4 / 31 rows per group, 128-row kernel / small tiles: 28672 x 4096 x 8 SwiGLU 75 / 43, 112 / 85, 172 /
+    123, 243 / 157, 339 / 164; 4096 x 14336 x 8 37 / 48, 65 / 53, 85 / 63, 127 / 81, 178 / 87; 4096 x 16384 x 8 43 / 53, 73 / 57,
+    107 / 71, 154 / 95, 209 / 104; 2048 x 7168 x 8 21 / 26, 25 / 27, 28 / 28, 43 / 29, 56 / 32; 2816 x 2048 x 32 31 / 14 to 95 / 41;
+    4096 x 4096 x 2 17 / 15 to 37 / 18; short K keeps the 128-row kernel: 2048 x 768 x 128 56 / 73, 59 / 70, 63 / 70, 72 / 69, 92 /
+    91, 2048 x 512 x 256 174 / 256 to 210 / 264."""
+    return K >= 1024 and 160 * _hit_groups(rows, G) * -(-N // 128) >= K
+
+
+def _few_fp8_layout(A, W, rows, N, K, out, a_rows, a_scale, w_scale) -> bool:
+    """Rows of 16 bytes that do not overlap, one output row per row: what else the 128-row kernel takes or refuses stays with it."""
+    return (A.dtype == W.dtype == torch.float8_e4m3fn and N % 16 == 0 and A.stride(1) == 1 and A.stride(0) >= K
+            and A.data_ptr() % 16 == 0 and W.data_ptr() % 16 == 0 and W.is_contiguous() and (a_rows is not None or rows == A.shape[0])
+            and all(t is not None and t.dtype == torch.float32 and t.is_contiguous() for t in (a_scale, w_scale))
+            and (out is None or (out.shape[0] == rows and out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)))
+
+
 # rows per group (on average) from which bf16 groups take the small-tile and 8-phase kernels (csrc/kernels/gemm2g.hip,
 # gemm8g.hip): below, the two GEMMs of an expert together gain little or nothing, and the 128-row kernel's split of K over
 # workgroups stays
@@ -452,18 +477,16 @@ def _bf16_core(A, W, rows, G, N, K, bias, splits, out, a_rows) -> int:
     return _grouped_bf16(rows, G, N, K) or (0 if N % 16 == 0 else 8 if rows > 176 * G else 2)
 
 
-def _use_gemm8g(A, W, rows, G, N, K, bias, splits, out) -> bool:
+def _use_gemm8g(A, W, rows, G, N, K, bias, splits, out, few: bool = False) -> bool:
     if MOE_GEMM == "classic" or A.dtype != torch.float8_e4m3fn or bias is not None or (splits or 1) > 1:
         return False
     if K % 128 or N % 8 or A.stride(0) % 16 or A.shape[0] * A.stride(0) >= (1 << 31) or 256 * K >= (1 << 31):
         return False
     if out is not None and (out.stride(1) != 1 or out.stride(0) % 8):
         return False
-    # Fewer rows keep the 128-row kernel: with this answer the expert FFN also takes its middle in MX form, and block scales
-    # would change what those sizes' activations keep.  With row scales the small tiles are faster there too, which nothing uses
-    # yet: 4 to 31 rows a group, us, 128-row kernel / small tiles, 28672 x 4096 x 8 248 / 186 to 308 / 201, 4096 x 14336 x 8
-    # 130 / 81 to 164 / 86, 2048 x 7168 x 8 45 / 30 to 53 / 32, 2048 x 1408 x 32 30 / 22 to 33 / 25
-    return _moe_core() != 0 or rows >= 32 * G
+    # (From 32 rows a group on the expert FFN also takes its middle in MX form; block scales would change what fewer rows'
+    # activations keep, so those keep row scales.)
+    return _moe_core() != 0 or rows >= 32 * G or few
 
 
 def gemm8p(A: torch.Tensor, W: torch.Tensor, residual: Optional[torch.Tensor] = None,

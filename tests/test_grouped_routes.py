@@ -98,6 +98,44 @@ def test_bf16_kernel_by_sizes(taken, monkeypatch, N, K, G, rows, core, swiglu):
     assert taken[0] == (("gemm8g_bf16", core) if core else ("grouped_gemm", None))
 
 
+@pytest.mark.parametrize("N,K,G,rows,few", [
+    # (what measured fastest, ``ops._few_fp8``: rows of all groups)
+    (28672, 4096, 8, 2, True), (4096, 14336, 8, 2, False), (4096, 14336, 8, 4, True), (4096, 16384, 8, 4, True), (2816, 2048, 32, 8, True),
+    (4096, 4096, 2, 1, True), (2048, 768, 128, 400, False), (2048, 512, 256, 64, False), (2048, 7168, 8, 255, True)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_fp8_kernel_of_few_rows(taken, monkeypatch, N, K, G, rows, few, swiglu):
+    """Row scales either way: the middle of an expert stays out of MX form below 32 rows a group."""
+    monkeypatch.setattr(ops, "silu_mul", lambda *a, **kw: None)
+    _call(rows, G=G, N=N // 64 * 64, K=K, fp8=True, swiglu=swiglu) if N * K * G < 1 << 28 else None
+    assert ops._few_fp8(rows, G, N, K) == few
+    assert not taken or taken[0] == (("gemm8g_fp8", 2) if few else ("grouped_gemm", None))
+    assert not ops.moe_mx_ok(torch.zeros(rows, 128, dtype=torch.float8_e4m3fn), torch.zeros(G, 256, 128, dtype=torch.float8_e4m3fn),
+                             torch.zeros(G, 128, 128, dtype=torch.float8_e4m3fn), rows)
+
+
+@pytest.mark.parametrize("form", ["expanded rows", "overlapping rows", "output beyond A", "fewer rows than A", "slots", "strided scales", "N off 16"])
+def test_fp8_forms_of_few_rows_that_stay_with_the_128_row_kernel(taken, form):
+    G, N, K, rows = 4, 256, 1024, 16
+    f8 = lambda *s: torch.zeros(*s, dtype=torch.float8_e4m3fn)  # noqa: E731
+    A, sc, kw = f8(rows, K), torch.ones(rows), {}
+    if form == "expanded rows":
+        A = f8(1, K).expand(rows, K)
+    elif form == "overlapping rows":
+        A = f8(rows * 64 + K).as_strided((rows, K), (64, 1))
+    elif form == "output beyond A":
+        kw["rows"] = rows + 16
+    elif form == "fewer rows than A":
+        kw["rows"] = rows - 2
+    elif form == "slots":
+        kw["max_slots"] = 9
+    elif form == "strided scales":
+        sc = torch.ones(2 * rows)[::2]
+    else:
+        N = 264
+    ops.grouped_gemm(A, f8(G, N, K), torch.zeros(G + 1, dtype=torch.int32), a_scale=sc, w_scale=torch.ones(G, N), **kw)
+    assert [n for n, _ in taken] == ["grouped_gemm"]
+
+
 class _Shape:
     """A contiguous bf16 operand of which only the layout is looked at."""
     dtype, device = torch.bfloat16, "cpu"
