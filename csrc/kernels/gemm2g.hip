@@ -15,6 +15,8 @@
 // 270 -> 217, 155 -> 115.  Dense calls of few tiles likewise: 512 rows x 4096 x K 4096 from MX 45 -> 21.
 // bf16, 8 experts of 16 rows: [14336, 4096] 194 (the 128-row kernel with split K, its clear and its conversion 204), [4096, 7168] 82
 // (103).
+#include <algorithm>
+
 #include "common.h"
 
 namespace lwc {
@@ -278,14 +280,19 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
   // 34 / 42 / 46.  More, where it is one of many: bf16 [14336, 4096] x 8 (896) 204 / 203 / 205, four times 190 / 193 / 202.
   // Dense (no table): tiles of 64 rows while they give a CU two workgroups at most, else of 128.
   const int per = (rows + G - 1) / G;
+  const long long nt = (N + 127) / 128, cols = nt * G;
   // 128 rows of a stride whose low bits are zero lie on few memory channels, and all tiles walk K in step: starting each tile's
   // walk at another step of K spreads them.  bf16, 8 experts of 8 / 64 rows, us, before -> after: [4096, 8192] 148 / 137 -> 97 /
   // 99, [14336, 4096] 199 / 210 -> 165 / 181, [4096, 2048] 33 / 36 -> 25 / 28, [14336, 6144] 273 / 299 -> 243 / 271; rows of 11008
   // and 22016 bytes, [4096, 5504] 78 / 88 -> 67 / 74, [4096, 11008] 148 / 160 -> 126 / 140; 3072, 5120 and 7168 bytes level.  Odd
   // multiples of 2048 bytes gain nothing (14336: 82 / 94 -> 85 / 95).  With many rows the tiles of a row tile no longer share its
-  // rows' way through L2: [14336, 4096] at 160 rows 236 -> 254, but [4096, 4096] 72 -> 66.
-  p.turned = (K % 4096 == 0 || K % 2048 != 0) && (per <= 104 || (row_off && N <= 4096 && per <= 192));
-  const long long nt = (N + 127) / 128, cols = nt * G;
+  // rows' way through L2: what an XCD's 64 workgroups have in use, the rows of so many groups, has to fit its 4 MiB ([28672, 4096]
+  // fp8 to MX at 64 / 128 / 160 rows 203 / 214 / 221 -> 170 / 186 / 198, bf16 [14336, 4096] at 96 / 128 / 160 209 / 219 / 224 -> 200 /
+  // 225 / 248, [8192, 4096] at 64 / 96 118 / 119 -> 103 / 125), unless every workgroup has a CU to itself ([4096, 4096] at 160 rows
+  // 72 -> 66, fp8 [4096, 8192] at 176 74 -> 71).
+  const long long nj = (nt + 7) / 8, groups = std::min<long long>(G, (64 + nj - 1) / nj);
+  p.turned = (K % 4096 == 0 || K % 2048 != 0) && ((groups * per * K <= 4 << 20 && per <= (K <= 4096 ? 160 : 144)) ||
+                                                  (row_off && cols <= 256 && per <= 192));
   int tm = per <= (cols <= 128 ? 44 : 16) ? 64 : per <= 104 && !(cols > 128 && cols <= 256) ? 128 : 192;
   if (!row_off) tm = nt * ((rows + 63) / 64) <= 512 ? 64 : 128;
 #define LWC_G2G(M) \
