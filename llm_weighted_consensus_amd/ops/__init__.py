@@ -427,9 +427,21 @@ def _few_fp8_layout(A, W, rows, N, K, out, a_rows, a_scale, w_scale) -> bool:
 
 
 # rows per group (on average) from which bf16 groups take the small-tile and 8-phase kernels (csrc/kernels/gemm2g.hip,
-# gemm8g.hip): below, the two GEMMs of an expert together gain little or nothing, and the 128-row kernel's split of K over
-# workgroups stays
+# gemm8g.hip) by :func:`_grouped_bf16`; below, :func:`_few_bf16`
 GROUPED_BF16_ROWS = 4
+
+
+def _few_bf16(rows: int, G: int, N: int, K: int) -> int:
+    """The kernel of a bf16 call of less than three rows per group (from three to four: the 128-row kernel): 2, the small tiles,
+    where the tiles that the routing reaches are enough for the length of K, else 0.  us on one MI355X, N x K x groups at 0.25 /
+    0.5 / 1 / 2 rows per group, 128-row kernel with its split of K / small tiles: 28672 x 4096 x 8 SwiGLU 111 / 84, 190 / 164, 260
+    / 248, 351 / 307; 14336 x 4096 x 8 64 / 42, 114 / 81, 159 / 121, 208 / 165; 4096 x 14336 x 8 66 / 93, 102 / 101, 142 / 122, 189 /
+    158; 4096 x 7168 x 8 36 / 48, 61 / 53, 81 / 62, 102 / 81; 2048 x 7168 x 8 25 / 46, 38 / 48, 47 / 50, 63 / 53; 1536 x 2048 x 128
+    154 / 91 to 188 / 143; but 2048 x 768 x 128 63 / 76 to 86 / 82, 2048 x 512 x 256 178 / 259 to 167 / 210, 4096 x 4096 x 2 17 / 27
+    to 23 / 29, 6144 x 16384 x 8 92 / 106, 164 / 143, 222 / 271, 300 / 287."""
+    tiles = _hit_groups(rows, G) * -(-N // 128)
+    return 2 if rows < 3 * G and K >= 1024 and N % 16 == 0 and tiles >= 96 and 96 * tiles >= K and \
+        not (K % 8192 == 0 and -(-N // 128) * G > 256) else 0
 
 
 def _grouped_bf16(rows: int, G: int, N: int, K: int) -> int:
@@ -472,8 +484,10 @@ def _bf16_core(A, W, rows, G, N, K, bias, splits, out, a_rows) -> int:
         return 0
     if out is not None and (out.shape[0] != rows or out.stride(1) != 1 or out.stride(0) % 8 or out.data_ptr() % 16):
         return 0
-    if _moe_core() or rows < GROUPED_BF16_ROWS * G:
+    if _moe_core():
         return _moe_core()
+    if rows < GROUPED_BF16_ROWS * G:
+        return _few_bf16(rows, G, N, K)
     return _grouped_bf16(rows, G, N, K) or (0 if N % 16 == 0 else 8 if rows > 176 * G else 2)
 
 
