@@ -68,6 +68,7 @@ struct DecodeParams {
   const float* rope_sin;
   const int* positions;
   int* counts = nullptr;  // [B, Hkv] finished splits, zero between calls: the last split of a sequence's KV head adds them up
+  int rounds = 0;         // paged_decode_kernel: > 0: workgroups take the sequences by length, that many of them resident per CU
 };
 
 // K and V registers of one PAIR of 16-token blocks for one wave (K: 8 x 16 B, V: 16 x 8 B per lane).
@@ -325,15 +326,21 @@ LWC_DEVICE void split_sum(const float* part_o, const float* part_lse, bf16_t* ou
 // and its waves meet in LDS (a second kernel that adds splits up takes 5 to 7 us of a step, whatever the batch; the last split
 // to finish doing it, about as much behind the longest sequence); with counts the splits there are meet in this launch.
 // Dynamic LDS: [W][G] running maxima and sums, [W][G][kD + 4] output rows.
-template <int W>
+template <int W, bool RANKED>
 __global__ void __launch_bounds__(64 * W, 4)
     paged_decode_kernel(DecodeParams p, const int* __restrict__ block_tables, const int* __restrict__ ctx_lens) {
-  const int item = blockIdx.x, kvh = blockIdx.y, split = blockIdx.z;
+  int item = blockIdx.x, kvh = blockIdx.y;
+  const int split = blockIdx.z;
   // wid through readfirstlane: the compiler then knows everything derived from it (sequence, block
   // indices) is wave-uniform and loads block tables / ctx lens with SCALAR loads — as vector loads each
   // one needed an s_waitcnt vmcnt(0) that drained the K/V loads in flight (the pipeline collapsed)
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
+  if constexpr (RANKED) {
+    const int B = gridDim.x, at = ranked_place(item + B * kvh, B * p.Hkv, p.rounds);
+    item = ranked_row(B, at / p.Hkv, lane, p.max_blocks, [&](int i) { return (ctx_lens[i] + kBS - 1) / kBS; });
+    kvh = at % p.Hkv;
+  }
 
   const int nrows = p.G;
   const int ctx = ctx_lens[item];
@@ -827,6 +834,21 @@ extern "C" int lwc_set_decode_wave_min_items(int n) {
 
 // Plain split-K paged decode (the small-batch / no-shared-prompt path; the engine's large batches with
 // forked prompts use the cascade kernel below).
+template <int W, bool RANKED>
+static void launch_decode_as(const lwc::DecodeParams& p, dim3 grid, int lds, const int* block_tables, const int* ctx_lens, hipStream_t s) {
+  if (W > 4) {
+    static const hipError_t attr = hipFuncSetAttribute((const void*)lwc::paged_decode_kernel<W, RANKED>, hipFuncAttributeMaxDynamicSharedMemorySize, W * 16 * 134 * 4);
+    (void)attr;
+  }
+  lwc::paged_decode_kernel<W, RANKED><<<grid, 64 * W, lds, s>>>(p, block_tables, ctx_lens);
+}
+
+template <int W>
+static void launch_decode(const lwc::DecodeParams& p, bool ranked, dim3 grid, int lds, const int* block_tables, const int* ctx_lens, hipStream_t s) {
+  if (ranked) launch_decode_as<W, true>(p, grid, lds, block_tables, ctx_lens, s);
+  else launch_decode_as<W, false>(p, grid, lds, block_tables, ctx_lens, s);
+}
+
 extern "C" int lwc_paged_decode(const void* q, int q_stride, const void* kc, const void* vc, const int* block_tables,
                                 const int* ctx_lens, void* out, float* part_o, float* part_lse, int B, int Hq,
                                 int Hkv, int D, int BS, int max_blocks, int num_splits, float scale,
@@ -855,18 +877,17 @@ extern "C" int lwc_paged_decode(const void* q, int q_stride, const void* kc, con
     p.num_splits = std::min(num_splits, std::max((4 * num_splits + waves - 1) / waves, room));
     p.counts = p.num_splits > 1 ? counts : nullptr;
     num_splits = p.num_splits;
+    // More workgroups than CUs take the sequences by length: a CU with the two longest would otherwise end the launch (and where
+    // B divides 256, its workgroups are different heads of ONE sequence).  Contexts within 80 % of their mean, us: 64 x 900 keys
+    // 57.3 -> 47.6, 128 x 600 72.3 -> 59.8, 100 x 1500 140.7 -> 124.0, 61 x 900 51.2 -> 44.3, 40 x 700 36.8 -> 30.3; equal ones
+    // 43.8 and 43.9.  Up to one workgroup per CU nothing can be paired.
+    if (p.num_splits == 1 && B * Hkv > 256) p.rounds = 16 / waves;
     const dim3 grid(B, Hkv, p.num_splits);
     const int lds = waves * p.G * (2 + kD + 4) * 4;
-    if (waves == 4) paged_decode_kernel<4><<<grid, 256, lds, s>>>(p, block_tables, ctx_lens);
-    else if (waves == 8) {
-      static const hipError_t attr = hipFuncSetAttribute((const void*)paged_decode_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, 8 * 16 * 134 * 4);
-      (void)attr;
-      paged_decode_kernel<8><<<grid, 512, lds, s>>>(p, block_tables, ctx_lens);
-    } else {
-      static const hipError_t attr = hipFuncSetAttribute((const void*)paged_decode_kernel<16>, hipFuncAttributeMaxDynamicSharedMemorySize, 16 * 16 * 134 * 4);
-      (void)attr;
-      paged_decode_kernel<16><<<grid, 1024, lds, s>>>(p, block_tables, ctx_lens);
-    }
+    const bool ranked = p.rounds > 0;
+    if (waves == 4) launch_decode<4>(p, ranked, grid, lds, block_tables, ctx_lens, s);
+    else if (waves == 8) launch_decode<8>(p, ranked, grid, lds, block_tables, ctx_lens, s);
+    else launch_decode<16>(p, ranked, grid, lds, block_tables, ctx_lens, s);
     if (p.counts) return (int)hipGetLastError();
   }
   if (num_splits > 1)

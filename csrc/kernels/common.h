@@ -152,6 +152,36 @@ LWC_DEVICE int xcd_remap(int orig, int nwg) {
   return (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + orig / 8;
 }
 
+// ---- rows of different lengths over the CUs ----
+// The place of workgroup w of n among the items sorted by work, most first, so that every CU gets about as much.  Workgroup w
+// starts on CU w % 256 as long as that has room: the rounds of 256 that are resident walk the order back and forth, the last
+// one forwards; after them the next longest goes to the CU that is done first.
+LWC_DEVICE int ranked_place(int w, int n, int rounds) {
+  const int k = w / 256, resident = min((n + 255) / 256, rounds);
+  return k < resident && ((resident - 1 - k) & 1) ? 256 * k + 255 - w % 256 : w;
+}
+
+// The row of rank `rank` among rows 0 .. B - 1 (0: the largest key(i); equal ones in their order), found bit by bit of the keys
+// (0 .. max_key; larger ones count as that) from ballots: each wave for itself, without a sort, a barrier or LDS, 0.3 us.  Beyond
+// 64 rows the n = ceil(B / 64) sets of every n-th one are ranked each for itself and take turns, the order of all but for
+// neighbours (with all of them at once, two and more keys a lane, the decode attention spilled 43 registers).
+template <typename Key>
+LWC_DEVICE int ranked_row(int B, int rank, int lane, int max_key, Key key_of) {
+  const int n = (B + 63) / 64, set = rank % n, i = set + n * lane;
+  rank /= n;
+  const int key = i < B ? min(key_of(i), max_key) : 0;
+  unsigned long long mask = __ballot(i < B);
+  for (int bit = 31 - __clz(max_key); bit >= 0; --bit) {
+    const unsigned long long ones = __ballot((key >> bit) & 1) & mask;
+    const int c = __popcll(ones);
+    const bool in = rank < c;
+    rank -= in ? 0 : c;
+    mask = in ? ones : mask & ~ones;
+  }
+  const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
+  return set + n * (int)__builtin_ctzll(__ballot(((mask >> lane) & 1) && below == rank));
+}
+
 }  // namespace lwc
 
 #define LWC_CHECK_LAUNCH() (void)hipGetLastError()
