@@ -532,6 +532,11 @@ static int g_wave_min_items = 2048;
 //
 // Workgroup = kCWaves waves = one SUPER-TILE (row_start, nseq, prefix_blocks) x one KV head; wave w
 // owns sequences row_start + w*per .. (+per), per = 16/G, as its 16 MFMA query rows (seq, head).
+// Few full tiles: two workgroups take half of a tile each, with half the sequences per wave (a grid of two
+// layers; where more than 128 tiles and heads are in use the second layer leaves at once).  The layers are the
+// slowest grid dimension: a workgroup that only leaves still waits for a CU's LDS (64 groups of 8 candidates
+// take 53 us so, 85 with the layers next to each other).  Tiles of up to 8 sequences: two per wave
+// (64 groups of 8: 54.7 -> 51.7 us, 128: 104.3 -> 99.2; one each 57.6, as every wave attends the whole prompt).
 //  phase 1 (prefix): the super-tile's sequences share their first `prefix_blocks` blocks.  The WG
 //    stages kCPairs block pairs at a time into LDS (K rows XOR-swizzled by 16 B chunk, V^T linear),
 //    and every wave runs the pair loop for its 16 rows out of LDS: the prompt's KV is read from HBM
@@ -578,13 +583,17 @@ __global__ void __launch_bounds__(kCWaves * 64)
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   // heads are the fast grid dimension: the real tiles (a prefix of the table) are dispatched first,
   // the graph-capture slack (nseq = 0 entries) last
-  const int tile = blockIdx.y, kvh = blockIdx.x;
+  const int tile = blockIdx.y, kvh = blockIdx.x, part = blockIdx.z;
   const int* t = tiles + 3 * tile;
-  const int row_start = t[0], nseq = t[1], pblk = t[2];
+  int per = t[1] <= kCWaves ? min(16 / p.G, 2) : 16 / p.G;
+  if (gridDim.z == 2) {
+    const int few = 128 / p.Hkv;  // (the tiles in use are the table's first)
+    if (2 * t[1] > kCWaves * per && (few >= (int)gridDim.y || tiles[3 * few + 1] <= 0)) per = (t[1] + 2 * kCWaves - 1) / (2 * kCWaves);
+  }
+  const int row_start = t[0] + part * kCWaves * per, nseq = t[1] - part * kCWaves * per, pblk = t[2];
   if (nseq <= 0) return;  // uniform for the whole workgroup, before any barrier
   const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);  // see above
   const int r16 = lane & 15, g = lane >> 4;
-  const int per = 16 / p.G;
   const int s0 = row_start + wid * per;
   const int nseq_w = max(0, min(per, nseq - wid * per));
   const int nrows = nseq_w * p.G;
@@ -832,8 +841,6 @@ extern "C" int lwc_set_decode_wave_min_items(int n) {
   return old;
 }
 
-// Plain split-K paged decode (the small-batch / no-shared-prompt path; the engine's large batches with
-// forked prompts use the cascade kernel below).
 template <int W, bool RANKED>
 static void launch_decode_as(const lwc::DecodeParams& p, dim3 grid, int lds, const int* block_tables, const int* ctx_lens, hipStream_t s) {
   if (W > 4) {
@@ -849,6 +856,8 @@ static void launch_decode(const lwc::DecodeParams& p, bool ranked, dim3 grid, in
   else launch_decode_as<W, false>(p, grid, lds, block_tables, ctx_lens, s);
 }
 
+// Plain split-K paged decode (the small-batch / no-shared-prompt path; the engine's large batches with
+// forked prompts use the cascade kernel below).
 extern "C" int lwc_paged_decode(const void* q, int q_stride, const void* kc, const void* vc, const int* block_tables,
                                 const int* ctx_lens, void* out, float* part_o, float* part_lse, int B, int Hq,
                                 int Hkv, int D, int BS, int max_blocks, int num_splits, float scale,
@@ -899,7 +908,7 @@ extern "C" int lwc_paged_decode(const void* q, int q_stride, const void* kc, con
 // (row_start, nseq <= kCWaves*16/G, prefix_blocks), unused entries nseq = 0.
 extern "C" int lwc_paged_decode_cascade(const void* q, int q_stride, const void* kc, const void* vc,
                                         const int* block_tables, const int* ctx_lens, const int* tiles, int max_tiles,
-                                        void* out, int Hq, int Hkv, int D, int BS, int max_blocks, float scale,
+                                        int B, void* out, int Hq, int Hkv, int D, int BS, int max_blocks, float scale,
                                         const float* rope_cos, const float* rope_sin, const int* positions,
                                         void* out8, void* mx, int mx_rows, hipStream_t s) {
   using namespace lwc;
@@ -923,7 +932,12 @@ extern "C" int lwc_paged_decode_cascade(const void* q, int q_stride, const void*
     const char* e = getenv("LWC_CASCADE_PAIRS");  // experiment knob, re-read per launch
     if (e) pairs = atoi(e);
   }
-  const dim3 grid(Hkv, max_tiles);
+  // Two workgroups share a tile while the tiles leave half of the CUs without one; each reads the prompt, which costs less than
+  // the CUs (32 heads on 8, prompt 256, 64 own keys, us: 128 sequences 28.6 -> 22.4, 256 29.4 -> 23.7, 512 38.4 -> 33.7; prompt 600
+  // and 128 own, 128 sequences: 64.8 -> 44.5).  At 768 sequences 49.9 would become 60.9, at 4096 226 become 280; tiles of half the
+  // rows and less stay whole (16 candidates each, 512 sequences: 37.2 would become 40.8).
+  const int rows = kCWaves * (16 / p.G), full = (B + rows - 1) / rows * Hkv;
+  const dim3 grid(Hkv, max_tiles, full <= 128 ? 2 : 1);
   if (pairs == 2)
     paged_decode_cascade_kernel<2><<<grid, kCWaves * 64, 2 * kPairBytes, s>>>(p, block_tables, ctx_lens, tiles);
   else if (pairs == 4)

@@ -25,7 +25,7 @@ int lwc_kv_gather(const void*, const void*, const long long*, void*, void*, int,
 int lwc_paged_decode(const void*, int, const void*, const void*, const int*, const int*, void*, float*, float*, int,
                      int, int, int, int, int, int, float, const float*, const float*, const int*, int*, hipStream_t);
 int lwc_set_decode_wave_min_items(int);
-int lwc_paged_decode_cascade(const void*, int, const void*, const void*, const int*, const int*, const int*, int, void*,
+int lwc_paged_decode_cascade(const void*, int, const void*, const void*, const int*, const int*, const int*, int, int, void*,
                              int, int, int, int, int, float, const float*, const float*, const int*, void*, void*, int, hipStream_t);
 int lwc_cascade_rows_per_tile(int);
 int lwc_grouped_gemm(const void*, const void*, void*, const int*, const float*, const float*, const void*, const int*,
@@ -362,7 +362,7 @@ void paged_decode_cascade(const at::Tensor& q, const at::Tensor& k_cache, const 
   const QRope qr = q_rope(rope_cos, rope_sin, positions, B, D, "paged_decode_cascade");
   CHECK_RC(lwc_paged_decode_cascade(q.data_ptr(), (int)q.stride(0), k_cache.data_ptr(), v_cache.data_ptr(),
                                     block_tables.data_ptr<int>(), ctx_lens.data_ptr<int>(), tiles.data_ptr<int>(),
-                                    (int)tiles.size(0), outp, (int)Hq, Hkv, D, BS,
+                                    (int)tiles.size(0), B, outp, (int)Hq, Hkv, D, BS,
                                     (int)block_tables.size(1), (float)scale, qr.cos, qr.sin, qr.pos, o8, mxp, mx_rows,
                                     cur_stream()),
            "paged_decode_cascade");
