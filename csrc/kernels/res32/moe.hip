@@ -398,21 +398,39 @@ __global__ void moe_combine_kernel(const YT* __restrict__ Y, const int* __restri
   }
 }
 
-// four columns per thread (d a multiple of four, aligned bases)
-template <typename AT, typename YT>
-__global__ void moe_combine_vec_kernel(const YT* __restrict__ Y, const int* __restrict__ inv, const float* __restrict__ wts,
-                                       const AT* __restrict__ h, int ldh, int k, float* __restrict__ out, int d,
-                                       const AT* __restrict__ add, int lda, const float* __restrict__ gate, int ldg) {
-  const int t = blockIdx.x;
+// 4 NCH columns per thread (d a multiple of four, aligned bases), 1024 NCH a workgroup: the loads of a choice's row, and of the
+// next choice's, are on their way at once.  64 tokens of 4096, top 2: 6.4 -> 4.8 us (a loop over the columns and the
+// choices, a load at a time); 16384 tokens (0.6 GB) 119 -> 109.
+template <typename AT, typename YT, int NCH>
+__global__ void __launch_bounds__(256) moe_combine_vec_kernel(const YT* __restrict__ Y, const int* __restrict__ inv,
+                                                               const float* __restrict__ wts, const AT* __restrict__ h, int ldh,
+                                                               int k, float* __restrict__ out, int d, const AT* __restrict__ add,
+                                                               int lda, const float* __restrict__ gate, int ldg) {
+  const int t = blockIdx.x, c0 = (blockIdx.y * 256 * NCH + threadIdx.x) * 4;
   const float ga = gate ? sigmoid_f(gate[(size_t)t * ldg]) : 1.0f;
-  for (int c = threadIdx.x * 4; c < d; c += blockDim.x * 4) {
-    float4v s = add ? Vec4<AT>::ld(add + (size_t)t * lda + c) * ga : float4v{0.f, 0.f, 0.f, 0.f};
-    for (int j = 0; j < k; ++j) {
-      const int r = inv[(size_t)t * k + j];
-      const float4v v = r >= 0 ? Vec4<YT>::ld(Y + (size_t)r * d + c) : Vec4<AT>::ld(h + (size_t)t * ldh + c);
-      s += v * wts[(size_t)t * k + j];
+  float4v s[NCH];
+#pragma unroll
+  for (int u = 0; u < NCH; ++u) {
+    const int c = c0 + 1024 * u;
+    s[u] = add && c < d ? Vec4<AT>::ld(add + (size_t)t * lda + c) * ga : float4v{0.f, 0.f, 0.f, 0.f};
+  }
+#pragma unroll 2
+  for (int j = 0; j < k; ++j) {
+    const int r = inv[(size_t)t * k + j];
+    const float wt = wts[(size_t)t * k + j];
+    float4v v[NCH];
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) {
+      const int c = c0 + 1024 * u, at = c < d ? c : 0;
+      v[u] = r >= 0 ? Vec4<YT>::ld(Y + (size_t)r * d + at) : Vec4<AT>::ld(h + (size_t)t * ldh + at);
     }
-    Vec4<float>::st(out + (size_t)t * d + c, s);
+#pragma unroll
+    for (int u = 0; u < NCH; ++u) s[u] += v[u] * wt;
+  }
+#pragma unroll
+  for (int u = 0; u < NCH; ++u) {
+    const int c = c0 + 1024 * u;
+    if (c < d) Vec4<float>::st(out + (size_t)t * d + c, s[u]);
   }
 }
 
@@ -475,15 +493,25 @@ extern "C" int r32_moe_combine(const void* Y, int y_f32, const int* inv, const f
                                int k, float* out, int d, const void* add, int lda, const float* gate, int ldg, int f32,
                                hipStream_t s) {
   if (T <= 0) return 0;
-  if (d % 4 == 0 && ldh % 4 == 0 && lda % 4 == 0 && aligned_to(add, f32 ? 16 : 8) && aligned_to(Y, y_f32 ? 16 : 8) && aligned_to(h, f32 ? 16 : 8) && aligned_to(out, 16)) {
-    if (f32 && y_f32)
-      moe_combine_vec_kernel<float, float><<<T, 256, 0, s>>>((const float*)Y, inv, wts, (const float*)h, ldh, k, out, d, (const float*)add, lda, gate, ldg);
-    else if (!f32 && y_f32)
-      moe_combine_vec_kernel<bf16_t, float><<<T, 256, 0, s>>>((const float*)Y, inv, wts, (const bf16_t*)h, ldh, k, out, d, (const bf16_t*)add, lda, gate, ldg);
-    else if (!f32 && !y_f32)
-      moe_combine_vec_kernel<bf16_t, bf16_t><<<T, 256, 0, s>>>((const bf16_t*)Y, inv, wts, (const bf16_t*)h, ldh, k, out, d, (const bf16_t*)add, lda, gate, ldg);
-    else
+  if (d > 0 && d % 4 == 0 && ldh % 4 == 0 && lda % 4 == 0 && aligned_to(add, f32 ? 16 : 8) && aligned_to(Y, y_f32 ? 16 : 8) && aligned_to(h, f32 ? 16 : 8) && aligned_to(out, 16)) {
+#define LWC_COMBINE(AT, YT, NCH)                                                                                              \
+  moe_combine_vec_kernel<AT, YT, NCH><<<dim3(T, (d + 1024 * NCH - 1) / (1024 * NCH)), 256, 0, s>>>(                            \
+      (const YT*)Y, inv, wts, (const AT*)h, ldh, k, out, d, (const AT*)add, lda, gate, ldg)
+#define LWC_COMBINE_N(AT, YT)                  \
+  if (d <= 1024) LWC_COMBINE(AT, YT, 1);       \
+  else if (d <= 2048) LWC_COMBINE(AT, YT, 2);  \
+  else LWC_COMBINE(AT, YT, 4)
+    if (f32 && y_f32) {
+      LWC_COMBINE_N(float, float);
+    } else if (!f32 && y_f32) {
+      LWC_COMBINE_N(bf16_t, float);
+    } else if (!f32 && !y_f32) {
+      LWC_COMBINE_N(bf16_t, bf16_t);
+    } else {
       return -1;
+    }
+#undef LWC_COMBINE_N
+#undef LWC_COMBINE
     LWC_CHECK_LAUNCH();
     return 0;
   }

@@ -725,3 +725,38 @@ def test_loader_refuses_wrong_shapes(gpu, tmp_path):
     save_file(bad, str(d / "model.safetensors"))
     with pytest.raises(KeyError):
         load_model(str(d))
+
+
+@pytest.mark.parametrize("d", [4, 30, 1020, 1024, 1028, 2048, 2052, 4096, 4100, 8192, 8196])
+def test_row_kernels_at_the_edges_of_their_widths(gpu, d):
+    """Rows a chunk long, just below and above, and longer than the kernels hold in registers: embedding, gated norm and
+    residual, row norm, routed sum.  Bounds: the embedding is exact; fp32 sums of d terms (2^-24 each, random: sqrt(d) of
+    them) on values of up to 16; bf16 outputs half a unit in the last place more (2^-8 of the value)."""
+    from llm_weighted_consensus_amd.ops import res32
+
+    g = torch.Generator().manual_seed(d)
+    T, V, k, tol = 3, 7, 3, 16 * 2 ** -24 * (d ** 0.5 + 8)
+    r = lambda *s: torch.randn(*s, generator=g)  # noqa: E731
+    table, toks = r(V, d).to(torch.bfloat16), torch.tensor([6, 0, 9], dtype=torch.int32)
+    cast = torch.empty(T, d, dtype=torch.bfloat16, device=gpu)
+    x = res32.embed_rows(table.to(gpu), toks.to(gpu), scale=2.0, cast=cast)
+    assert (x.cpu() == 2 * table[[6, 0, 6]].float()).all() and (cast.cpu() == 2 * table[[6, 0, 6]]).all()
+    x0, w, wn = x.cpu().double(), r(d), r(d)
+    for y, gate in ((r(T, d).to(torch.bfloat16), r(T, d).to(torch.bfloat16)), (r(T, d), None)):
+        z = y.double() * (torch.sigmoid(gate.double()) if gate is not None else 1)
+        want = x0 + z / (z.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * w.double()
+        nxt = want / (want.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * wn.double()
+        for next_w, ref in ((None, want), (wn.to(gpu), nxt)):
+            xs = x.clone()
+            res32.gated_norm_residual(xs, y.to(gpu), w.to(gpu), 1e-6, gate_logits=None if gate is None else gate.to(gpu), x_cast=cast,
+                                      next_w=next_w)
+            assert (xs.cpu().double() - want).abs().max() < tol
+            assert ((cast.cpu().double() - ref).abs() <= ref.abs() * 2 ** -8 + tol).all()
+    got = res32.rmsnorm_rows(x, w.to(gpu), 1e-6, torch.float32, rows=torch.tensor([2, 0], device=gpu)).cpu().double()
+    assert (got - (x0 / (x0.pow(2).mean(1, keepdim=True) + 1e-6).sqrt() * w.double())[[2, 0]]).abs().max() < tol
+    Y, h, add = r(5, d).to(torch.bfloat16), r(T, d).to(torch.bfloat16), r(T, d).to(torch.bfloat16)
+    inv, wt = torch.tensor([[0, 4, -1], [-1, -1, 2], [3, 1, 0]], dtype=torch.int32), torch.rand(T, k, generator=g)
+    rows = torch.where(inv[..., None] >= 0, Y.double()[inv.clamp(min=0)], h.double()[:, None])
+    want = (wt.double()[..., None] * rows).sum(1)
+    assert (res32.moe_combine(Y.to(gpu), inv.to(gpu), wt.to(gpu), h.to(gpu)).cpu().double() - want).abs().max() < tol
+    assert (res32.moe_combine(Y.to(gpu), inv.to(gpu), wt.to(gpu), h.to(gpu), add=add.to(gpu)).cpu().double() - want - add.double()).abs().max() < tol
