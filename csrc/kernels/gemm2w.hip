@@ -216,13 +216,19 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
     float sum[kAcc];
 #pragma unroll
     for (int e = 0; e < kAcc; ++e) sum[e] = 0.f;
-    for (int s = 0; s < p.splits; ++s) {
-      const float* part = p.part + ((size_t)t * p.splits + s) * (TM * TN) + tid;
-      float x[kAcc];
+    // (four ranges on their way at once: 61 x 4096 x 4096 in four 12.8 -> 12.1 us, 64 x 64 x 4096 in eight 9.2 -> 8.1)
+    for (int s = 0; s < p.splits; s += 4) {
+      float x[4][kAcc];
 #pragma unroll
-      for (int e = 0; e < kAcc; ++e) x[e] = __hip_atomic_load(part + e * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int j = 0; j < 4; ++j) {
+        const float* part = p.part + ((size_t)t * p.splits + min(s + j, p.splits - 1)) * (TM * TN) + tid;
 #pragma unroll
-      for (int e = 0; e < kAcc; ++e) sum[e] += x[e];
+        for (int e = 0; e < kAcc; ++e) x[j][e] = __hip_atomic_load(part + e * 256, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int e = 0; e < kAcc; ++e) sum[e] += s + j < p.splits ? x[j][e] : 0.f;
     }
 #pragma unroll
     for (int e = 0; e < kAcc; ++e) acc[e / (NP * 8)][e / 8 % NP][e / 4 % 2][e % 4] = sum[e];
@@ -352,10 +358,11 @@ int launch(Params p, hipStream_t s) {
 // The tile and the K ranges of a call (max_splits: what the caller's workspace holds, in 64 x 64 partial tiles).
 // 64 x 64 up to 512 tiles (two workgroups per CU) and for any call of up to 64 rows.  Measured (us, 64 x 64 against 128 x 128):
 // 512 rows x 4096 x K 1024 9.9 / 14.8, 512 x 4096 x 4096 35.5 / 42.8, 1000 x 3072 x 1024 (768 tiles) 14.9 / 13.8, 1000 x 4096 x
-// 4096 (1024 tiles) 62 / 44.  Its K ranges: as many as fit one workgroup per CU, none below 16 steps.  Measured, one / two /
-// four / eight ranges: 61 x 4096 x 4096 21.9 / 15.6 / 12.9 / 15.5, 61 x 6144 x 4096 22.2 / 17.0 / 17.6 / 21.3, 61 x 4096 x 14336
-// 70 / 42 / 28 / 32, 128 x 4096 x 4096 22.1 / 16.1 / 17.3 / 25.4, 256 x 1024 x 4096 21.1 / 14.9 / 12.2 / 13.7, 61 x 3072 x 1024
-// 7.4 / 7.9 / 8.2.
+// 4096 (1024 tiles) 62 / 44.  Its K ranges: as many as fit one workgroup per CU, none below 16 steps, or 8 up to 32 tiles.
+// Measured, one / two / four / eight ranges: 61 x 4096 x 4096 22.3 / 15.7 / 12.1 / 14.8, 61 x 6144 x 4096 23.1 / 18.9 / 17.6 / 21.0,
+// 61 x 4096 x 14336 70 / 44 / 28 / 31, 128 x 4096 x 4096 22.2 / 17.3 / 16.8 / 23.6, 256 x 1024 x 4096 21.5 / 15.1 / 11.3 / 12.4, 61 x
+// 3072 x 1024 7.7 / 8.0 / 7.6 / 9.8; up to 32 tiles 64 x 64 x 4096 20.7 / 13.8 / 9.4 / 8.1 (sixteen 8.8), 64 x 1024 x 4096 21.4 / 14.8 /
+// 10.5 / 9.8, 16 x 2048 x 2048 12.1 / 10.0 / 8.1 / 8.9, 61 x 1024 x 1024 7.4 / 7.3 / 6.5 / 7.6.
 // Larger ones: the tile that takes the least time in whole rounds of two workgroups per CU, the larger of two that tie.
 // Measured (128 x 128 against 128 x 192): 3600 x 2304 x 768 (522 and 348 tiles) 25.3 / 20.3, 3600 x 4096 x 1024 (928 and
 // 638) 40.8 / 46.7, 7155 x 3072 x 768 (1344 and 896) 51.5 / 48.1.
@@ -365,7 +372,7 @@ extern "C" void lwc_gemm2w_plan(int M, int N, int K, int epi, long long max_spli
   const long long small = tiles(64, 64);
   if (M <= 64 || small <= 512) {
     *tile = 3;
-    const long long s = std::min(std::min(256 / std::max(small, 1LL), (long long)K / 1024), max_splits / std::max(small, 1LL));
+    const long long s = std::min(std::min(256 / std::max(small, 1LL), (long long)K / (small <= 32 ? 512 : 1024)), max_splits / std::max(small, 1LL));
     *splits = (int)std::max(1LL, s);
     return;
   }
