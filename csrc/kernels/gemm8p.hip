@@ -61,7 +61,6 @@ constexpr int kUnitB = 128 * 128;   // 128 rows x 128 B
 constexpr int kBufB = 4 * kUnitB;   // one K tile: A0 A1 B0 B1
 constexpr int kLdsB = 2 * kBufB;    // 128 KiB
 constexpr int kUA0 = 0, kUA1 = kUnitB, kUB0 = 2 * kUnitB, kUB1 = 3 * kUnitB;
-constexpr int kDeep = 2;  // 16-row tiles of a partial that the finaliser has in flight: 8 loads (4 were a longer chain, 16 spill)
 constexpr int kPartialF = 256 * 256;  // fp32 partial tile per workgroup
 
 enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4 };
@@ -291,22 +290,13 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
           __hip_atomic_store(p.flags + blk, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
         __syncthreads();
-        const __amdgpu_buffer_rsrc_t rP = uniform_rsrc(p.ws + (size_t)blk * kPartialF, kPartialF * 4);
+        // four loads at a time: with eight the 256-row tile spills 37 to 41 registers instead of 16 to 19 (9000 x 4096 x 1024 115 ->
+        // 124 us, 4096 x 28672 x 4096 695 -> 723), the 224-row one 12 instead of none
+        const float4v* wsq = reinterpret_cast<const float4v*>(p.ws + (size_t)blk * kPartialF);
 #pragma unroll
-        for (int i0 = 0; i0 < 4 + R1; i0 += kDeep) {
-          float4v part[kDeep][4];
+        for (int i = 0; i < 4 + R1; ++i) {
 #pragma unroll
-          for (int i = 0; i < kDeep; ++i)
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj)
-              if (i0 + i < 4 + R1)
-                part[i][jj] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rP, lane * 16, (wid * 32 + (i0 + i) * 4 + jj) * 1024, 0));
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int i = 0; i < kDeep; ++i)
-#pragma unroll
-            for (int jj = 0; jj < 4; ++jj)
-              if (i0 + i < 4 + R1) acc[i0 + i < 4 + R1 ? i0 + i : 0][jj] += part[i][jj];
+          for (int jj = 0; jj < 4; ++jj) acc[i][jj] += wsq[(wid * 32 + i * 4 + jj) * 64 + lane];
           __builtin_amdgcn_sched_barrier(0);
         }
         if (pa <= tile_begin) break;
