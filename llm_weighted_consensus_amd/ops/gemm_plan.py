@@ -286,9 +286,16 @@ def _enc_ok(n: str, x: torch.Tensor, w: torch.Tensor, epi: str, other: torch.Ten
     return n != "g2" or gemm2w_ok(N, K, w, other)
 
 
+# gemm8p is taken for an encoder's projection where it leads by this much: between an encoder's other kernels it does not keep a
+# small lead (24 layers of bge-large over 7156 rows with its FFN1 of 70 us on gemm8p 6116 us, on the library 5998, on gemm2w 6079)
+G8_LEAD = 0.95
+
+
 def _pick(key, runs) -> str:
     t = {name: _time(fn, iters=2, rounds=3) for name, fn in runs.items()}
     TIMINGS[key] = t
+    if "g8" in t and min(t, key=t.get) == "g8" and t["g8"] > G8_LEAD * min(t[n] for n in t if n != "g8"):
+        t = {n: v for n, v in t.items() if n != "g8"}
     own = min((n for n in t if n != "blas"), key=lambda n: t[n], default="blas")
     return own if t[own] <= t["blas"] * (1 + OWN_MARGIN) else "blas"
 
