@@ -282,17 +282,17 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
   const int per = (rows + G - 1) / G;
   const long long nt = (N + 127) / 128, cols = nt * G;
   // 128 rows of a stride whose low bits are zero lie on few memory channels, and all tiles walk K in step: starting each tile's
-  // walk at another step of K spreads them.  bf16, 8 experts of 8 / 64 rows, us, before -> after: [4096, 8192] 148 / 137 -> 97 /
-  // 99, [14336, 4096] 199 / 210 -> 165 / 181, [4096, 2048] 33 / 36 -> 25 / 28, [14336, 6144] 273 / 299 -> 243 / 271; rows of 11008
-  // and 22016 bytes, [4096, 5504] 78 / 88 -> 67 / 74, [4096, 11008] 148 / 160 -> 126 / 140; 3072, 5120 and 7168 bytes level.  Odd
-  // multiples of 2048 bytes gain nothing (14336: 82 / 94 -> 85 / 95).  With many rows the tiles of a row tile no longer share its
-  // rows' way through L2: what an XCD's 64 workgroups have in use, the rows of so many groups, has to fit its 4 MiB ([28672, 4096]
-  // fp8 to MX at 64 / 128 / 160 rows 203 / 214 / 221 -> 170 / 186 / 198, bf16 [14336, 4096] at 96 / 128 / 160 209 / 219 / 224 -> 200 /
-  // 225 / 248, [8192, 4096] at 64 / 96 118 / 119 -> 103 / 125), unless every workgroup has a CU to itself ([4096, 4096] at 160 rows
-  // 72 -> 66, fp8 [4096, 8192] at 176 74 -> 71).
+  // walk at another step of K spreads them.  fp8, 8 experts, us, before -> after: [28672, 4096] to MX at 64 / 128 / 160 rows 203 /
+  // 214 / 221 -> 170 / 186 / 198, [4096, 8192] at 176 74 -> 71; odd multiples of 2048 bytes gain nothing (14336: 82 / 94 -> 85 / 95).
+  // With many rows the tiles of a row tile no longer share its rows' way through L2: what an XCD's 64 workgroups have in use, the
+  // rows of so many groups, has to fit its 4 MiB, unless every workgroup has a CU to itself.
+  // bf16 experts walk K from its start: the next layer's router reads their sums, and in another order of them rows whose second
+  // and third expert nearly tie change experts (2 of 1280 rows behind one such layer; one moved by a tenth of its norm), for
+  // [14336, 4096] x 8 of 8 rows at 199 us instead of 165.  fp8 rows are rounded to e4m3 in front of every product, which moves
+  // them more than an order does.
   const long long nj = (nt + 7) / 8, groups = std::min<long long>(G, (64 + nj - 1) / nj);
-  p.turned = (K % 4096 == 0 || K % 2048 != 0) && ((groups * per * K <= 4 << 20 && per <= (K <= 4096 ? 160 : 144)) ||
-                                                  (row_off && cols <= 256 && per <= 192));
+  p.turned = mode != kBf16 && mode != kBf16Swiglu && (K % 4096 == 0 || K % 2048 != 0) &&
+             ((groups * per * K <= 4 << 20 && per <= (K <= 4096 ? 160 : 144)) || (row_off && cols <= 256 && per <= 192));
   int tm = per <= (cols <= 128 ? 44 : 16) ? 64 : per <= 104 && !(cols > 128 && cols <= 256) ? 128 : 192;
   if (!row_off) tm = nt * ((rows + 63) / 64) <= 512 ? 64 : 128;
 #define LWC_G2G(M) \

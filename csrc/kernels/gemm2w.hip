@@ -216,7 +216,7 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
     float sum[kAcc];
 #pragma unroll
     for (int e = 0; e < kAcc; ++e) sum[e] = 0.f;
-    // (four ranges on their way at once: 61 x 4096 x 4096 in four 12.8 -> 12.1 us, 64 x 64 x 4096 in eight 9.2 -> 8.1)
+    // (four ranges on their way at once: 61 x 4096 x 4096 in four 12.8 -> 12.1 us)
     for (int s = 0; s < p.splits; s += 4) {
       float x[4][kAcc];
 #pragma unroll
@@ -339,8 +339,10 @@ int launch(Params p, hipStream_t s) {
   // first step for each column tile spreads them.  N x K at 24 / 64 / 128 rows, us, before -> after: 16384 x 2048 17 / 17 / 26 -> 15 /
   // 15 / 23, 28672 x 4096 50 / 54 / 59 -> 48 / 52 / 51, 32000 x 4096 55 / 57 / 64 -> 55 / 57 / 52, 8192 x 8192 33 / 33 / 44 -> 27 /
   // 29 / 42, 4096 x 11008 23 / 25 / 35 -> 21 / 24 / 33; 4096 x 14336 and 6144 x 4096 level.  Many rounds of tiles spread by
-  // themselves (128256 x 4096 185 / 202 / 212 -> 199 / 213 / 217), and from 300 rows on the matrix cores are the bound.
-  p.turned = p.M <= 256 && (long long)p.tiles_m * p.tiles_n <= 1024 && (p.K % 2048 == 0 || p.K % 1024 != 0);
+  // themselves (128256 x 4096 185 / 202 / 212 -> 199 / 213 / 217), and from 300 rows on the matrix cores are the bound.  Plain
+  // products without the folded norm, the projections of the models with routed experts, walk K from its start: behind them a
+  // router picks experts, and another order of the sums moves rows that nearly tie (gemm2g.hip).
+  p.turned = (NORM || EPI != EPI_PLAIN) && p.M <= 256 && (long long)p.tiles_m * p.tiles_n <= 1024 && (p.K % 2048 == 0 || p.K % 1024 != 0);
   gemm2w_kernel<EPI, TM, TN, NST, NORM><<<p.tiles_m * p.tiles_n * p.splits, 256, kLds, s>>>(p);
   return (int)hipGetLastError();
 }
@@ -358,11 +360,11 @@ int launch(Params p, hipStream_t s) {
 // The tile and the K ranges of a call (max_splits: what the caller's workspace holds, in 64 x 64 partial tiles).
 // 64 x 64 up to 512 tiles (two workgroups per CU) and for any call of up to 64 rows.  Measured (us, 64 x 64 against 128 x 128):
 // 512 rows x 4096 x K 1024 9.9 / 14.8, 512 x 4096 x 4096 35.5 / 42.8, 1000 x 3072 x 1024 (768 tiles) 14.9 / 13.8, 1000 x 4096 x
-// 4096 (1024 tiles) 62 / 44.  Its K ranges: as many as fit one workgroup per CU, none below 16 steps, or 8 up to 32 tiles.
+// 4096 (1024 tiles) 62 / 44.  Its K ranges: as many as fit one workgroup per CU, none below 16 steps.
 // Measured, one / two / four / eight ranges: 61 x 4096 x 4096 22.3 / 15.7 / 12.1 / 14.8, 61 x 6144 x 4096 23.1 / 18.9 / 17.6 / 21.0,
 // 61 x 4096 x 14336 70 / 44 / 28 / 31, 128 x 4096 x 4096 22.2 / 17.3 / 16.8 / 23.6, 256 x 1024 x 4096 21.5 / 15.1 / 11.3 / 12.4, 61 x
-// 3072 x 1024 7.7 / 8.0 / 7.6 / 9.8; up to 32 tiles 64 x 64 x 4096 20.7 / 13.8 / 9.4 / 8.1 (sixteen 8.8), 64 x 1024 x 4096 21.4 / 14.8 /
-// 10.5 / 9.8, 16 x 2048 x 2048 12.1 / 10.0 / 8.1 / 8.9, 61 x 1024 x 1024 7.4 / 7.3 / 6.5 / 7.6.
+// 3072 x 1024 7.7 / 8.0 / 7.6 / 9.8.  (Ranges of 8 steps up to 32 tiles, 64 x 64 x 4096 9.4 -> 8.1, would be
+// another order of sums in front of a router, as a walk from another step is.)
 // Larger ones: the tile that takes the least time in whole rounds of two workgroups per CU, the larger of two that tie.
 // Measured (128 x 128 against 128 x 192): 3600 x 2304 x 768 (522 and 348 tiles) 25.3 / 20.3, 3600 x 4096 x 1024 (928 and
 // 638) 40.8 / 46.7, 7155 x 3072 x 768 (1344 and 896) 51.5 / 48.1.
@@ -372,7 +374,7 @@ extern "C" void lwc_gemm2w_plan(int M, int N, int K, int epi, long long max_spli
   const long long small = tiles(64, 64);
   if (M <= 64 || small <= 512) {
     *tile = 3;
-    const long long s = std::min(std::min(256 / std::max(small, 1LL), (long long)K / (small <= 32 ? 512 : 1024)), max_splits / std::max(small, 1LL));
+    const long long s = std::min(std::min(256 / std::max(small, 1LL), (long long)K / 1024), max_splits / std::max(small, 1LL));
     *splits = (int)std::max(1LL, s);
     return;
   }

@@ -434,14 +434,16 @@ GROUPED_BF16_ROWS = 4
 def _few_bf16(rows: int, G: int, N: int, K: int) -> int:
     """The kernel of a bf16 call of less than three rows per group (from three to four: the 128-row kernel): 2, the small tiles,
     where the tiles that the routing reaches are enough for the length of K, else 0.  us on one MI355X, N x K x groups at 0.25 /
-    0.5 / 1 / 2 rows per group, 128-row kernel with its split of K / small tiles: 28672 x 4096 x 8 SwiGLU 111 / 84, 190 / 164, 260
-    / 248, 351 / 307; 14336 x 4096 x 8 64 / 42, 114 / 81, 159 / 121, 208 / 165; 4096 x 14336 x 8 66 / 93, 102 / 101, 142 / 122, 189 /
-    158; 4096 x 7168 x 8 36 / 48, 61 / 53, 81 / 62, 102 / 81; 2048 x 7168 x 8 25 / 46, 38 / 48, 47 / 50, 63 / 53; 1536 x 2048 x 128
-    154 / 91 to 188 / 143; but 2048 x 768 x 128 63 / 76 to 86 / 82, 2048 x 512 x 256 178 / 259 to 167 / 210, 4096 x 4096 x 2 17 / 27
-    to 23 / 29, 6144 x 16384 x 8 92 / 106, 164 / 143, 222 / 271, 300 / 287."""
+    0.5 / 1 / 2 rows per group, 128-row kernel with its split of K / small tiles: 4096 x 14336 x 8 65 / 97, 105 / 118, 148 / 145, 192
+    / 174; 4096 x 7168 x 8 39 / 50, 61 / 61, 82 / 66, 102 / 85; 2048 x 7168 x 8 26 / 48, 38 / 49, 45 / 56, 61 / 60; 1536 x 2048 x
+    128 158 / 94 to 191 / 151; 5632 x 2048 x 64 183 / 104 to 285 / 242; but 2048 x 768 x 128 68 / 78 to 89 / 85, 2048 x 512 x 256
+    178 / 259 to 167 / 210, 4096 x 4096 x 2 17 / 27 to 23 / 29.  K of multiples of 4096, whose rows lie on few memory channels:
+    up to half a row per group, 14336 x 4096 x 8 SwiGLU 65 / 52, 109 / 101, 158 / 161, 192 / 212; 28672 x 4096 x 8 114 / 105, 194 /
+    192, 269 / 307, 362 / 381; 8192 x 4096 x 16 77 / 57, 105 / 100, 155 / 156, 178 / 190; 4096 x 8192 x 8 never, 45 / 57, 71 / 73,
+    101 / 108, 131 / 150."""
     tiles = _hit_groups(rows, G) * -(-N // 128)
     return 2 if rows < 3 * G and K >= 1024 and N % 16 == 0 and tiles >= 96 and 96 * tiles >= K and \
-        not (K % 8192 == 0 and -(-N // 128) * G > 256) else 0
+        (K % 4096 != 0 or (K == 4096 and 2 * rows <= G)) else 0
 
 
 def _grouped_bf16(rows: int, G: int, N: int, K: int) -> int:

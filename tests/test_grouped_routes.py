@@ -100,8 +100,8 @@ def test_bf16_kernel_by_sizes(taken, monkeypatch, N, K, G, rows, core, swiglu):
 
 @pytest.mark.parametrize("N,K,G,rows,core", [
     # (less than three rows a group, ``ops._few_bf16``: rows of all groups)
-    (14336, 4096, 8, 2, 2), (14336, 4096, 8, 23, 2), (14336, 4096, 8, 24, 0), (14336, 4096, 8, 31, 0), (4096, 14336, 8, 4, 0),
-    (4096, 14336, 8, 8, 2), (4096, 7168, 8, 2, 0), (4096, 7168, 8, 4, 2), (1536, 2048, 128, 64, 2), (2048, 768, 128, 128, 0),
+    (14336, 4096, 8, 2, 2), (14336, 4096, 8, 4, 2), (14336, 4096, 8, 5, 0), (14336, 4096, 8, 24, 0), (14336, 4096, 8, 31, 0), (4096, 14336, 8, 4, 0),
+    (4096, 14336, 8, 8, 2), (4096, 14336, 8, 23, 2), (4096, 14336, 8, 24, 0), (4096, 7168, 8, 2, 0), (4096, 7168, 8, 4, 2), (4096, 8192, 8, 4, 0), (1536, 2048, 128, 64, 2), (2048, 768, 128, 128, 0),
     (4096, 4096, 2, 4, 0), (6144, 16384, 8, 8, 0), (328, 4096, 64, 128, 0)])
 def test_bf16_kernel_of_few_rows(taken, monkeypatch, N, K, G, rows, core):
     monkeypatch.setattr(torch, "empty", lambda *a, **kw: None)   # (no result is needed)
