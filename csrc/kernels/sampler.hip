@@ -301,9 +301,12 @@ __global__ void __launch_bounds__(T, RS < SLOTS * (kSampT / T) ? 4 : SLOTS <= 4 
   // One: every thread's (64 rows, top-p 0.95, 50 us by one wave, 35 by all; 4096 rows of 32000 in pairs 83 by one, 92 by all)
   constexpr bool kPairs = LS > 0 || SLOTS <= 4;
   constexpr int kList = LS > 0 ? 3456 : kPairs ? 2048 : 8192;  // 16-bit keys in LDS, which the pairs share
+  // Masses are searched in lists of as many keys in every build of a vocabulary: a round over the row decides by fp32 sums, a list
+  // by exact ones, and a row's draw must not depend on how many rows there are (counts are whole numbers either way)
+  constexpr int kMassList = SLOTS == 16 ? 3456 : kList;
   __shared__ uint32_t s_tkey[kList / 2];
   uint16_t* const s_list = reinterpret_cast<uint16_t*>(s_tkey);
-  static_assert(kList >= 2 * kSampT, "s_tkey holds the maxima of 1024 threads too");
+  static_assert(kList >= 2 * kSampT && kMassList <= kList, "s_tkey holds the maxima of 1024 threads too");
   __shared__ uint32_t s_lb, s_fkey;
   __shared__ uint32_t s_own[SLOTS * 4];
   __shared__ float s_oexcl;
@@ -633,9 +636,9 @@ OPAQUE_ROW(row);
     MASS_LOCAL(KEY, _l);         \
     OUT = red.sum(_l);           \
   } while (0)
-    // The keys in [LO, HI] (LO >= 1) go to s_list if they are at most kList, thread by thread; N: how many they are.  A search
+    // The keys in [LO, HI] (LO >= 1) go to s_list if they are at most MAX, thread by thread; N: how many they are.  A search
     // over the list takes 2 us, over the row 14 rounds of 1.3 (counts) or 2 us (masses).
-#define COLLECT(LO, HI, N)                                                             \
+#define COLLECT(LO, HI, N, MAX)                                                        \
   do {                                                                                 \
     OPAQUE_ROW(row);                                                                   \
     const uint32_t _a = thr1x2(LO), _b = thr1x2((HI) + 1u);                            \
@@ -660,7 +663,7 @@ OPAQUE_ROW(row);
       _tot += sw;                                                                      \
     }                                                                                  \
     N = __builtin_amdgcn_readfirstlane((int)_tot);                                     \
-    if (N <= kList && __builtin_amdgcn_ballot_w64(_c > 0.f)) {                         \
+    if (N <= (MAX) && __builtin_amdgcn_ballot_w64(_c > 0.f)) {                         \
       int _p = (int)_off;                                                              \
       _Pragma("unroll") for (int s = 0; s < NS; ++s) {                                 \
         const uint4v x = SLOT(s);                                                      \
@@ -693,7 +696,7 @@ OPAQUE_ROW(row);
         lo = __builtin_amdgcn_readfirstlane(s_lb);
         const uint32_t from = max(lo, 1u);
         int n;
-        COLLECT(from, hi, n);
+        COLLECT(from, hi, n, kList);
         if (n <= kList) {
           if (t < 64) {  // (one wave: the list is short)
             while (lo < hi) {
@@ -916,8 +919,8 @@ OPAQUE_ROW(row);
       for (int round = 0; lo < hi; ++round) {
         if (round % 4 == 0) {
           int n;
-          COLLECT(lo, hi, n);
-          if (n <= kList) {
+          COLLECT(lo, hi, n, kMassList);
+          if (n <= kMassList) {
             // masses as whole numbers of 2^-24 (every fp16 u is one): exact in any order
             const double want = ((double)target - (double)over) * 16777216.0;
             if (!kPairs || t < 64) {
