@@ -343,6 +343,10 @@ __global__ void __launch_bounds__(T, RS < SLOTS * (kSampT / T) ? 4 : SLOTS <= 4 
     const int w0 = __builtin_amdgcn_readfirstlane(t >> 6) * 64;
 #pragma unroll
     for (int i = 0; i < NS; ++i) {
+      if (i == LS) {  // (the wait below counts on it: the loads to LDS are the older ones)
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+      }
       const int s = i < LS ? RS + i : i - LS, v0 = s % SLOTS * kSampT + s / SLOTS * T;
       const __amdgpu_buffer_rsrc_t r = uniform_rsrc(lrow + v0 * 8, max(0, nvec - v0) * 16);
       if (i < LS)
@@ -350,6 +354,7 @@ __global__ void __launch_bounds__(T, RS < SLOTS * (kSampT / T) ? 4 : SLOTS <= 4 
       else
         row[i < LS ? 0 : s] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(r, t * 16, 0, 0));
     }
+    __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RS) : "memory");
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
