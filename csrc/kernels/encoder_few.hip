@@ -316,17 +316,35 @@ __global__ void __launch_bounds__(kT) qkv_attn_kernel(Attn p) {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");  // the wave's own rows of p
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+  float4v o[DH / 16];
+  float all = 0.f;
 #pragma unroll
   for (int c = 0; c < DH / 16; ++c) {
-    float4v o = float4v{0.f, 0.f, 0.f, 0.f};
+    o[c] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < TK / 32; ++s)
-      o = mfma(*reinterpret_cast<const uint4v*>(vs + (16 * c + r16) * (TK + 8) + s * 32 + 8 * g),
-               *reinterpret_cast<const uint4v*>(ps + qi * (TK + 8) + s * 32 + 8 * g), o);
+      o[c] = mfma(*reinterpret_cast<const uint4v*>(vs + (16 * c + r16) * (TK + 8) + s * 32 + 8 * g),
+                  *reinterpret_cast<const uint4v*>(ps + qi * (TK + 8) + s * 32 + 8 * g), o[c]);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) o[r] *= inv;
-    if (qi < p.T) *reinterpret_cast<uint2v*>(p.a + (size_t)qi * D + h * DH + 16 * c + 4 * g) = narrow4(o);
+    for (int r = 0; r < 4; ++r) {
+      o[c][r] *= inv;
+      all = fmaf(o[c][r], 0.f, all);  // 0, or NaN
+    }
   }
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(all != 0.f) != 0, 0)) {
+    // an infinity or NaN among the values: a weight of zero does not keep it to its own text, so each query's keys alone
+#pragma unroll
+    for (int c = 0; c < DH / 16; ++c)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float t = 0.f;
+        for (int key = lo; key < hi; ++key) t += bf2f(ps[qi * (TK + 8) + key]) * bf2f(vs[(16 * c + 4 * g + r) * (TK + 8) + key]);
+        o[c][r] = t * inv;
+      }
+  }
+#pragma unroll
+  for (int c = 0; c < DH / 16; ++c)
+    if (qi < p.T) *reinterpret_cast<uint2v*>(p.a + (size_t)qi * D + h * DH + 16 * c + 4 * g) = narrow4(o[c]);
 }
 
 enum Out { OUT_PART = 0, OUT_BIAS = 1, OUT_GELU = 2 };

@@ -454,3 +454,27 @@ def test_few_row_encoder_matches_reference(gpu, monkeypatch, arch, lens):
     m.layers[-1].w2 = torch.cat([w.flatten()[:1], w.flatten()])[1:].view(w.shape)   # two bytes off
     assert ops.encoder_few(m.word, m.pos_type, args[0], args[1], m.emb_ln_g, m.emb_ln_b,
                            [t for L in m.layers for t in bert._layer_tensors(L)], args[2], m.cfg.heads, m.scale, 1e-12) is None
+
+
+@pytest.mark.parametrize("arch", ["bge-small-en-v1.5", "bge-base-en-v1.5"])
+@pytest.mark.parametrize("lens", [[5, 4, 6], [12, 17, 3]])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf")])
+def test_few_row_encoder_keeps_infinities_to_their_text(gpu, monkeypatch, arch, lens, value):
+    """A text with a token whose embedding is not finite changes no other text of its batch, as with the general kernels: the
+    others' rows are what they are beside an ordinary token, but for the order of the attention's sums (bf16 layers: 0.01)."""
+    from llm_weighted_consensus_amd.models import bert
+    from llm_weighted_consensus_amd.models.config import encoder_config
+
+    m = bert.BertEncoder(encoder_config(arch), device=gpu, seed=5)
+    texts = [[(37 * i + 11 * j) % 900 + 1 for j in range(n)] for i, n in enumerate(lens)]
+    args = m.pack(texts)
+    want = m.forward_packed(*args).float()
+    texts[1][1] = 29999
+    m.word[29999] = value
+    bad = slice(lens[0], lens[0] + lens[1])
+    for few in (32, 0):
+        monkeypatch.setattr(bert, "FEW_ROWS", few)
+        got = m.forward_packed(*m.pack(texts)).float()
+        assert not torch.isfinite(got[bad]).any()
+        for rows in (slice(0, lens[0]), slice(lens[0] + lens[1], None)):
+            assert torch.isfinite(got[rows]).all() and (got[rows] - want[rows]).norm() < 0.02 * want[rows].norm(), few
