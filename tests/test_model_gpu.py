@@ -478,3 +478,94 @@ def test_few_row_encoder_keeps_infinities_to_their_text(gpu, monkeypatch, arch, 
         assert not torch.isfinite(got[bad]).any()
         for rows in (slice(0, lens[0]), slice(lens[0] + lens[1], None)):
             assert torch.isfinite(got[rows]).all() and (got[rows] - want[rows]).norm() < 0.02 * want[rows].norm(), few
+
+
+# the core of each projection of a decode step (None: the library, with the norm and RoPE kernels in front of it)
+_STEP_CORES = {"gv": ["gv"] * 5, "g2": ["g2"] * 5, "library o and head": ["gv", None, "g2", "g2", None], "library qkv and down": [None, "gv", "g2", None, "gv"],
+               "library gate|up": ["g2", "g2", None, "gv", "g2"]}
+
+
+@pytest.mark.parametrize("cores", list(_STEP_CORES))
+@pytest.mark.parametrize("B,longest,splits", [(1, 600, 1), (1, 600, 4), (17, 400, 3), (64, 60, 1)])
+def test_decode_step_without_kernels_between_its_gemms(gpu, monkeypatch, cores, B, longest, splits):
+    """The decode step of few rows (norms, RoPE and cache writes in the projections, splits added up in the attention) over
+    three layers with norm weights other than one, every projection on a core of its own and some on the library: logits
+    and cached rows against the fp32 forward, no further off than the step of separate kernels but for the spread of two
+    roundings (2 x); nothing else in the cache changes, a row without a slot writes nothing; a captured step gives the same bits."""
+    from llm_weighted_consensus_amd import ops
+    from llm_weighted_consensus_amd.models.config import decoder_config
+    from llm_weighted_consensus_amd.models.llama import KVCache, LlamaModel
+    from llm_weighted_consensus_amd.ops import gemm_plan
+
+    cfg = decoder_config("llama-tiny", layers=3, ffn=1536)   # (every projection of a shape of its own)
+    gen = torch.Generator(device="cpu").manual_seed(B + splits)
+    m = LlamaModel(cfg, device=gpu, seed=7, max_position=1024, fold_norms=False)
+    norm = lambda: (0.5 + torch.rand(cfg.hidden, generator=gen)).to(gpu, torch.bfloat16)  # noqa: E731
+    for L in m.layers:
+        L.attn_norm, L.mlp_norm = norm(), norm()
+    m.final_norm = norm()
+    m._fold_norms()
+    lens = [int(n) for n in torch.randint(3, longest, (B,), generator=gen)]
+    lens[0] = longest                                     # the last position is what the step decodes
+    texts = [torch.randint(0, cfg.vocab_size, (n,), generator=gen).to(gpu) for n in lens]
+    nb = [-(-n // 16) for n in lens]
+    width, first = max(nb), [1 + sum(nb[:b]) for b in range(B)]
+    cache = KVCache(cfg, sum(nb) + 1, 16, gpu)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=gpu)  # noqa: E731
+    tables = torch.zeros(B, width, dtype=torch.int32, device=gpu)
+    for b in range(B):
+        tables[b, :nb[b]] = torch.arange(first[b], first[b] + nb[b])
+    past = [n - 1 for n in lens]
+    cu = i32([0] + torch.tensor(past).cumsum(0).tolist())
+    m.prefill(torch.cat([t[:-1] for t in texts]).int(), i32([p for n in past for p in range(n)]),
+              i32([first[b] * 16 + p for b in range(B) for p in range(past[b])]), cu, max(past), (cu[1:] - 1).long(), cache)
+    slots = [first[b] * 16 + past[b] for b in range(B)]
+    live = list(range(B))
+    if B == 17:                                           # a padded row, as the engine has them
+        slots[5], lens[5], past[5] = -1, 1, 0
+        tables[5] = 0
+        live.remove(5)
+    args = (torch.stack([t[-1] for t in texts]).int(), i32(past), i32(slots), tables, i32(lens), cache)
+    before = cache.pool.clone()
+    taken = []
+    for name in ("step_qkv", "step_project"):
+        f = getattr(ops, name)
+        monkeypatch.setattr(ops, name, lambda x, w, core, *a, _f=f, _n=name, **kw: taken.append((_n, tuple(w.shape), core)) or _f(x, w, core, *a, **kw))
+    monkeypatch.setattr(gemm_plan, "MODE", "auto")
+    L, want, ss = m.layers[0], [], True
+    shapes = [(L.wqkv, "plain"), (L.wo, "residual"), (L.w_gate_up, "swiglu"), (L.w_down, "residual"), (m.lm_head, "plain")]
+    for (w, epi), c in zip(shapes, _STEP_CORES[cores]):
+        monkeypatch.setitem(gemm_plan._CHOICE, (B, w.shape[0], w.shape[1], epi), c or "blas")
+    for li in range(cfg.layers):                          # who takes part: a projection behind one that left no sums does not
+        for (w, epi), c in list(zip(shapes, _STEP_CORES[cores]))[:4] + ([(shapes[4], _STEP_CORES[cores][4])] if li + 1 == cfg.layers else []):
+            if c and (ss or epi == "residual"):
+                want.append(("step_qkv" if w is L.wqkv else "step_project", tuple(w.shape), {"gv": 1, "g2": 2}[c]))
+            ss = bool(c) if epi == "residual" else ss
+    got = m.decode(*args, num_splits=splits)
+    assert taken == want
+    after = cache.pool.clone()
+    cache.pool.copy_(before)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = m.decode(*args, num_splits=splits)
+    for _ in range(3):
+        cache.pool.copy_(before)
+        out.fill_(float("nan"))
+        graph.replay()
+        assert torch.equal(out[live], got[live]) and torch.equal(cache.pool, after)
+        assert torch.equal(m.decode(*args, num_splits=splits)[live], got[live])
+    cache.pool.copy_(before)
+    monkeypatch.setenv("LWC_DECODE_QROPE", "0")           # the step of separate kernels
+    n = len(taken)
+    plain = m.decode(*args, num_splits=splits)
+    assert len(taken) == n
+    refs = torch.stack([ref.llama_forward(m, texts[b])[-1] for b in live])
+    err = lambda t: ((t[live].float() - refs).norm() / refs.norm()).item()  # noqa: E731
+    assert err(got) < 2 * err(plain) and err(got) < 0.03, (err(got), err(plain))
+    ours, theirs, was = (t.view(cfg.layers, 2, -1, cfg.kv_heads, 16 * cfg.head_dim) for t in (after, cache.pool, before))
+    blocks = torch.zeros(ours.shape[2], dtype=torch.bool, device=gpu)
+    blocks[[slots[b] // 16 for b in live]] = True
+    assert torch.equal(ours[:, :, ~blocks], was[:, :, ~blocks])
+    wrote, expect = (after != before), (cache.pool != before)
+    assert (wrote.sum() - expect.sum()).abs() <= 0.01 * expect.sum()      # (a value may round to what was there)
+    assert ((ours.float() - theirs.float()).norm() <= 0.02 * (theirs.float() - was.float()).norm())
