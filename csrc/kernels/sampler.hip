@@ -3,10 +3,12 @@
 //
 // Bound by the row a compute unit holds: its load takes 11 us at the CU's share of the memory rate, its passes 8 us and more
 // (a round of exps 6, of masses 2).  Large batches of large vocabularies hold two rows per CU, 512 threads each with 23 of 32
-// slots in registers and 9 in LDS, so that the two overlap; thresholds are searched in a list of the few elements that can
-// matter, and a draw that carries 1 - top_p by itself is accepted without a pass.  4096 rows, one MI355X, us, before -> after
-// these: vocabulary 128256 greedy 208 -> 206, temperature 0.8 258 -> 229, with top-p 0.95 344 -> 280, with top-k 40 and top-p
-// 0.9 818 -> 403, with 20 logprobs 589 -> 399; vocabulary 32000 top-p 0.95 99 -> 83, top-k 240 -> 161, 20 logprobs 239 -> 166.
+// slots in registers and 9 in LDS, so that the two overlap; thresholds are searched in a list of the elements that can
+// matter where those are few, and a draw that carries 1 - top_p by itself is accepted without a pass.  4096 rows, one MI355X, us,
+// before -> after these: vocabulary 128256 greedy 216 -> 224, temperature 0.8 264 -> 242, with top-p 0.95 356 -> 285, with top-k 40
+// and top-p 0.9 814 -> 405, with top-p 0.95 and 20 logprobs 598 -> 411; vocabulary 32000 top-p 0.95 110 -> 99, top-k 40 199 -> 157, with
+// 20 logprobs 254 -> 188, with a bias and a mask 189 -> 138.  What two rows per unit cost: greedy rows a power of two of bytes apart
+// (131072 tokens) 213 -> 242.
 //
 // One workgroup per row, of 1024 threads or of 512 that stand for two each.  The row (bf16, V <= 8*1024*SLOTS) is
 // loaded ONCE from HBM as packed bf16 (16 B per load, SLOTS loads per thread) and every later phase — raw max and
@@ -210,6 +212,20 @@ struct Red {
     __syncthreads();
     return row16_sum(sc[threadIdx.x & 15]);
   }
+  // (and the block's sum of c)
+  LWC_DEVICE float sum(const float (&x)[VT], int c, int& count) {
+    float* sc = set();
+#pragma unroll
+    for (int v = 0; v < VT; ++v) {
+      const float w = row_sum4(row16_sum(x[v]));
+      if ((threadIdx.x & 63) == 0) sc[(threadIdx.x >> 6) + v * kW] = w;
+    }
+    c = row_sum4_i(row16_sum_i(c));
+    if ((threadIdx.x & 63) == 0) reinterpret_cast<int*>(sc)[16 + (threadIdx.x >> 6)] = c;
+    __syncthreads();
+    count = row16_sum_i((threadIdx.x & 15) < kW ? reinterpret_cast<int*>(sc)[16 + (threadIdx.x & (kW - 1))] : 0);
+    return row16_sum(sc[threadIdx.x & 15]);
+  }
   LWC_DEVICE float max(float v) {
     float* sc = set();
     v = row_max4(row16_max(v));
@@ -286,8 +302,10 @@ LWC_DEVICE float uniform_f(float x) { return __int_as_float(__builtin_amdgcn_rea
 // that asks for neither carries neither's registers.
 // T threads: 1024, or 512 of which each stands for two of the 1024 (element order, sums and draws are those of 1024: slot
 // v * SLOTS + j of thread t is slot j of thread v * T + t).  RS of the VT * SLOTS slots are in registers, the rest in LDS.
+// Waves per SIMD: two workgroups of the shortest rows; with 5 for 8 slots the next row's workgroup comes in beside the last waves of
+// the one before it (the wave that ranks the logprobs: 4096 rows of 65536 tokens, 5 logprobs, 256 -> 241 us).
 template <int T, int SLOTS, int RS, bool PROC, bool TOPK>
-__global__ void __launch_bounds__(T, RS < SLOTS * (kSampT / T) ? 4 : SLOTS <= 4 && !PROC ? 8 : 4) sample_kernel(SampleParams p) {
+__global__ void __launch_bounds__(T, SLOTS <= 4 ? (PROC && TOPK ? 7 : 8) : SLOTS == 8 ? 5 : 4) sample_kernel(SampleParams p) {
   constexpr int VT = kSampT / T, NS = SLOTS * VT, LS = NS - RS;
   static_assert(!PROC || VT == 1, "processed rows are held by 1024 threads");
   __shared__ uint4v held[LS > 0 ? LS * T : 1];
@@ -303,7 +321,11 @@ __global__ void __launch_bounds__(T, RS < SLOTS * (kSampT / T) ? 4 : SLOTS <= 4 
   constexpr int kList = LS > 0 ? 3456 : kPairs ? 2048 : 8192;  // 16-bit keys in LDS, which the pairs share
   // Masses are searched in lists of as many keys in every build of a vocabulary: a round over the row decides by fp32 sums, a list
   // by exact ones, and a row's draw must not depend on how many rows there are (counts are whole numbers either way)
-  constexpr int kMassList = SLOTS == 16 ? 3456 : kList;
+  // (4 slots: a list is one wave's, and a round over so short a row 1 us: 64 rows of 32000 tokens, top-p 0.5, 29 us by rounds, 35 in
+  // lists of up to 2048)
+  constexpr int kMassList = SLOTS == 16 ? 3456 : SLOTS <= 4 ? 512 : kList;
+  constexpr int kFewest = LS > 0 ? 40 * SLOTS : 24 * SLOTS + (SLOTS <= 8 ? 32 : 0);  // a top-k up to which the list of the largest pays
+  static_assert(kFewest <= kSampT, "one of the threads' maxima each");
   __shared__ uint32_t s_tkey[kList / 2];
   uint16_t* const s_list = reinterpret_cast<uint16_t*>(s_tkey);
   static_assert(kList >= 2 * kSampT && kMassList <= kList, "s_tkey holds the maxima of 1024 threads too");
@@ -684,9 +706,11 @@ OPAQUE_ROW(row);
     uint32_t tau_k = 0;  // top-k: keep elements with key >= tau_k
     if (k > 0) {
       uint32_t lo = 0, hi = 0x3C00u;  // keys of [0, 1.0]
-      // Few (k <= 1024): the k largest of the threads' own maxima bound the k-th largest element from below (0: fewer than
-      // k threads hold any mass); the elements from there on, rarely more than a few times k, are searched in a list
-      if (k <= kSampT) {
+      // Few: the k largest of the threads' own maxima bound the k-th largest element from below (0: fewer than k threads hold
+      // any mass); the elements from there on, rarely more than a few times k, are searched in a list.  As k comes near the 1024
+      // maxima the bound falls and the list grows: 64 rows of 128256 tokens 37.6 us at k = 40, 48.4 at 400, 59.2 at 600, 136 at 1000
+      // (rounds over the row 48), 64 of 32000 26 at 100, 29 at 200, 60 at 1000 (26); two rows per unit 512 at 600, 621 at 800 (671)
+      if (k <= kFewest) {
 #pragma unroll
         for (int v = 0; v < VT; ++v) {
           const float um = __builtin_amdgcn_exp2f(__builtin_fmaf(mxv[v], c1, c0));
@@ -914,57 +938,65 @@ OPAQUE_ROW(row);
       // (The margin is wider than the sums' rounding, 256 terms each: what the sum would answer is what this answers)
       const float rest = total - (float)__builtin_bit_cast(_Float16, (uint16_t)ks);
       if (__builtin_amdgcn_readfirstlane(rest * 1.0001f < target)) break;
-      float above;
-      MASS_GE(ks + 1u, above);
+      float mass[VT];
+      MASS_LOCAL(ks + 1u, mass);
+      int eighth = 0;  // of the keys above, those among an eighth of the row's
+      if (T == 512 || t < 512) {
+        const uint32_t t2 = thr1x2(ks + 1u);
+        uint32_t c2 = 0u;
+#pragma unroll
+        for (int j = 0; j < SLOTS; j += 2) count2(c2, row[j][0], row[j + 1][0], t2, kOne2);
+        eighth = (int)((c2 & 0xffffu) + (c2 >> 16));
+      }
+      const float above = red.sum(mass, eighth, eighth);
       if (above < target) break;  // accepted (block-uniform)
       // rejected: tau_p > ks.  Exact search for the largest key with mass(>= key) >= target.
-      // The keys left in the interval go to a list once they are few; until then rounds over the row halve it.
+      // Keys in the interval that are few go to a list; otherwise rounds over the row halve it.  (A list that does not fit costs
+      // a pass: tried again every four rounds, 64 rows of 128256 tokens at top-p 0.9 took 61.5 us, by rounds alone 56.7.)
       uint32_t lo = ks + 1u, hi = 0x3C00u;
-      float over = 0.f;  // the mass above hi
-      for (int round = 0; lo < hi; ++round) {
-        if (round % 4 == 0) {
-          int n;
-          COLLECT(lo, hi, n, kMassList);
-          if (n <= kMassList) {
-            // masses as whole numbers of 2^-24 (every fp16 u is one): exact in any order
-            const double want = ((double)target - (double)over) * 16777216.0;
-            if (!kPairs || t < 64) {
-              while (lo < hi) {
-                const uint32_t mid = (lo + hi + 1) >> 1;
-                uint32_t c = 0;
+      bool listed = lo < hi && __builtin_amdgcn_readfirstlane(eighth) * 8 <= kMassList;
+      if (listed) {
+        int n;
+        COLLECT(lo, hi, n, kMassList);
+        listed = n <= kMassList;
+        if (listed) {
+          // masses as whole numbers of 2^-24 (every fp16 u is one): exact in any order
+          const double want = (double)target * 16777216.0;
+          if (!kPairs || t < 64) {
+            while (lo < hi) {
+              const uint32_t mid = (lo + hi + 1) >> 1;
+              uint32_t c = 0;
 #pragma unroll 4
-                for (int i = t; i < n; i += kPairs ? 64 : T) {
-                  const uint16_t kk = s_list[i];
-                  c += kk >= mid ? (uint32_t)((float)__builtin_bit_cast(_Float16, kk) * 16777216.f) : 0u;
-                }
-                double m;
-                if constexpr (kPairs)
-                  m = (double)row_sum4_i(row16_sum_i((int)(c >> 16))) * 65536.0 + (double)row_sum4_i(row16_sum_i((int)(c & 0xffffu)));
-                else
-                  m = red.sum_wide((int)(c >> 12), (int)(c & 4095u));
-                if (__builtin_amdgcn_readfirstlane(m >= want))
-                  lo = mid;
-                else
-                  hi = mid - 1;
+              for (int i = t; i < n; i += kPairs ? 64 : T) {
+                const uint16_t kk = s_list[i];
+                c += kk >= mid ? (uint32_t)((float)__builtin_bit_cast(_Float16, kk) * 16777216.f) : 0u;
               }
-              if (kPairs && t == 0) s_lb = lo;
+              double m;
+              if constexpr (kPairs)
+                m = (double)row_sum4_i(row16_sum_i((int)(c >> 16))) * 65536.0 + (double)row_sum4_i(row16_sum_i((int)(c & 0xffffu)));
+              else
+                m = red.sum_wide((int)(c >> 12), (int)(c & 4095u));
+              if (__builtin_amdgcn_readfirstlane(m >= want))
+                lo = mid;
+              else
+                hi = mid - 1;
             }
-            if constexpr (kPairs) {
-              __syncthreads();
-              lo = hi = __builtin_amdgcn_readfirstlane(s_lb);
-            }
-            break;
+            if (kPairs && t == 0) s_lb = lo;
+          }
+          if constexpr (kPairs) {
+            __syncthreads();
+            lo = __builtin_amdgcn_readfirstlane(s_lb);
           }
         }
+      }
+      while (!listed && lo < hi) {
         const uint32_t mid = (lo + hi + 1) >> 1;
         float mm;
         MASS_GE(mid, mm);
-        if (__builtin_amdgcn_readfirstlane(mm >= target)) {
+        if (__builtin_amdgcn_readfirstlane(mm >= target))
           lo = mid;
-        } else {
+        else
           hi = mid - 1;
-          over = mm;
-        }
       }
       tau = max(lo, L0);
       check = false;
@@ -1031,7 +1063,7 @@ extern "C" int lwc_sample(const void* logits, int ld, int V, int B, const float*
   // 65537 to 131072 tokens, plain rows: two rows per compute unit from four rows per unit on, so that one's load goes on under
   // the other's passes; a thread of a pair does twice the work, and with fewer rows their latency is what counts
   // (128256 tokens, us, one row per unit against two: 64 rows top-p 0.95 35 / 61, 512 72 / 77, 1024 104 / 101, 4096 300 / 280;
-  // 4096 rows greedy 206 / 206, temperature alone 258 / 229, top-k 40 537 / 403, 20 logprobs 511 / 399)
+  // 4096 rows greedy 216 / 224, temperature alone 258 / 229, top-k 40 537 / 403, 20 logprobs 511 / 399)
   if (slots > 8 && slots <= 16 && !proc && B >= 1024) {
     if (num_logprobs > 0) sample_kernel<512, 16, kRegSlots, false, true><<<B, 512, 0, s>>>(p);
     else sample_kernel<512, 16, kRegSlots, false, false><<<B, 512, 0, s>>>(p);
