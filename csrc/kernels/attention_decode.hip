@@ -876,27 +876,31 @@ extern "C" int lwc_paged_decode(const void* q, int q_stride, const void* kc, con
     paged_decode_wave_kernel<<<dim3((items + kWaves - 1) / kWaves, Hkv), 256, 0, s>>>(p, items, block_tables,
                                                                                       ctx_lens);
   } else {
-    // As many waves per (sequence, KV head) as num_splits workgroups of four, in workgroups of up to 16, and further workgroups
-    // while there are fewer than CUs; of eight where the CUs have room for half the splits (a CU reads 50 to 60 GB/s, and one
-    // sequence of 2000 keys took 14.4 us in 16s, 13.5 in 16 splits of four).  Against splits of four waves and a second kernel
-    // (us, 32 heads on 8): 1 x 247 keys 12.2 -> 9, 8 x 900 19.0 -> 16.1, 32 x 900 30.0 -> 25.6, 64 x 60 13.0 -> 8.5, 64 x 900
-    // 53.2 -> 45.5, 128 x 600 (one split) 64.3 -> 61.1.
-    const int room = 256 / std::max(1, B * Hkv);
-    waves = num_splits == 1 ? 4 : num_splits == 2 || room >= (num_splits + 1) / 2 ? 8 : 16;
-    p.num_splits = std::min(num_splits, std::max((4 * num_splits + waves - 1) / waves, room));
+    // Waves per workgroup and splits, by how many (sequence, KV head) pairs there are.  Measured over 20 to 4000 keys, equal and
+    // within 80 % of their mean, 2 to 1952 pairs (863 settings; us, mean time relative to the best choice of each):
+    //   above 512      workgroups of four, whole sequences (1.01 to 1.08; of eight 1.15, of sixteen 1.5)
+    //   to 512         of eight, two a CU: 61 x 900 ragged 43.8, of four 47.0, of sixteen 46.7
+    //   to 399         more pairs than CUs and too few for two each: four splits of four waves (1.06, second kernel 1.10; whole in
+    //                  sixteens 1.5: 40 x 250 20.7 against 16.0)
+    //   224 to 256     of eight, one a CU (1.03)
+    //   below          some three workgroups of four a CU (1.03 to 1.07, second kernel 1.13 to 1.18)
+    // A sequence takes fewer splits than that if it has no pair of blocks for every wave, and then needs no adding up.
+    const int pairs = B * Hkv;
+    const bool two = pairs <= 512 && pairs >= (counts ? 400 : 384), one = pairs <= 256 && pairs >= 224;
+    waves = two || one ? 8 : 4;
+    p.num_splits = std::min(num_splits, two || one || pairs > 512 ? 1 : pairs > 256 && !counts ? 4 : (768 + pairs - 1) / pairs);
     p.counts = p.num_splits > 1 ? counts : nullptr;
     num_splits = p.num_splits;
     // More workgroups than CUs take the sequences by length: a CU with the two longest would otherwise end the launch (and where
     // B divides 256, its workgroups are different heads of ONE sequence).  Contexts within 80 % of their mean, us: 64 x 900 keys
-    // 57.3 -> 47.6, 128 x 600 72.3 -> 59.8, 100 x 1500 140.7 -> 124.0, 61 x 900 51.2 -> 44.3, 40 x 700 36.8 -> 30.3; equal ones
-    // 43.8 and 43.9.  Up to one workgroup per CU nothing can be paired.
+    // 57.3 -> 47.6, 128 x 600 72.3 -> 59.8, 100 x 1500 140.7 -> 124.0, 61 x 900 51.2 -> 44.3; equal ones 43.8 and 43.9.  Up to one
+    // workgroup per CU nothing can be paired.
     if (p.num_splits == 1 && B * Hkv > 256) p.rounds = 16 / waves;
     const dim3 grid(B, Hkv, p.num_splits);
     const int lds = waves * p.G * (2 + kD + 4) * 4;
     const bool ranked = p.rounds > 0;
     if (waves == 4) launch_decode<4>(p, ranked, grid, lds, block_tables, ctx_lens, s);
-    else if (waves == 8) launch_decode<8>(p, ranked, grid, lds, block_tables, ctx_lens, s);
-    else launch_decode<16>(p, ranked, grid, lds, block_tables, ctx_lens, s);
+    else launch_decode<8>(p, ranked, grid, lds, block_tables, ctx_lens, s);
     if (p.counts) return (int)hipGetLastError();
   }
   if (num_splits > 1)
