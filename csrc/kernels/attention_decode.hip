@@ -336,14 +336,18 @@ __global__ void __launch_bounds__(64 * W, 4)
   // one needed an s_waitcnt vmcnt(0) that drained the K/V loads in flight (the pipeline collapsed)
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
+  int ctx;
   if constexpr (RANKED) {
     const int B = gridDim.x, at = ranked_place(item + B * kvh, B * p.Hkv, p.rounds);
-    item = ranked_row(B, at / p.Hkv, lane, p.max_blocks, [&](int i) { return (ctx_lens[i] + kBS - 1) / kBS; });
+    int mine = 0, from;
+    item = ranked_row(B, at / p.Hkv, lane, p.max_blocks, [&](int i) { return ((mine = ctx_lens[i]) + kBS - 1) / kBS; }, from);
     kvh = at % p.Hkv;
+    ctx = __builtin_amdgcn_readlane(mine, from);
+  } else {
+    ctx = ctx_lens[item];
   }
 
   const int nrows = p.G;
-  const int ctx = ctx_lens[item];
   const int nblk_total = (ctx + kBS - 1) / kBS;
   const int per_split = max((nblk_total + p.num_splits - 1) / p.num_splits, 2 * W);
   const int splits = max(1, (nblk_total + per_split - 1) / per_split);

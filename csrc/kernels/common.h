@@ -164,14 +164,15 @@ LWC_DEVICE int ranked_place(int w, int n, int rounds) {
 // The row of rank `rank` among rows 0 .. B - 1 (0: the largest key(i); equal ones in their order), found bit by bit of the keys
 // (0 .. max_key; larger ones count as that) from ballots: each wave for itself, without a sort, a barrier or LDS, 0.3 us.  Beyond
 // 64 rows the n = ceil(B / 64) sets of every n-th one are ranked each for itself and take turns, the order of all but for
-// neighbours (with all of them at once, two and more keys a lane, the decode attention spilled 43 registers).
+// neighbours (with all of them at once, two and more keys a lane, the decode attention spilled 43 registers).  from: the lane
+// whose key it is, so that what the key is made of need not be read again.
 template <typename Key>
-LWC_DEVICE int ranked_row(int B, int rank, int lane, int max_key, Key key_of) {
+LWC_DEVICE int ranked_row(int B, int rank, int lane, int max_key, Key key_of, int& from) {
   const int n = (B + 63) / 64, set = rank % n, i = set + n * lane;
   rank /= n;
   const int key = i < B ? min(key_of(i), max_key) : 0;
   unsigned long long mask = __ballot(i < B);
-  for (int bit = 31 - __clz(max_key); bit >= 0; --bit) {
+  for (int bit = __ballot(key >> 4) ? 31 - __clz(max_key) : 3; bit >= 0; --bit) {
     const unsigned long long ones = __ballot((key >> bit) & 1) & mask;
     const int c = __popcll(ones);
     const bool in = rank < c;
@@ -179,7 +180,8 @@ LWC_DEVICE int ranked_row(int B, int rank, int lane, int max_key, Key key_of) {
     mask = in ? ones : mask & ~ones;
   }
   const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-  return set + n * (int)__builtin_ctzll(__ballot(((mask >> lane) & 1) && below == rank));
+  from = (int)__builtin_ctzll(__ballot(((mask >> lane) & 1) && below == rank));
+  return set + n * from;
 }
 
 }  // namespace lwc

@@ -199,23 +199,38 @@ __global__ void __launch_bounds__(256) gated_norm_residual_vec_kernel(float* __r
   float* xr = x + (size_t)t * d;
   float4v z[NCH], g[NCH], xv[NCH], wv[NCH];
   float s = 0.f;
+  if constexpr (NCH == 1) {
+    // (one access a thread: x asked for behind the sum and nothing past the row; on their way during the sum, and from any place of
+    // the row past it, 16384 rows of 256 took 20 us instead of 14, 4000 of 1024 9.1 instead of 8.1)
+    const int i = threadIdx.x * 4;
+    z[0] = float4v{0.f, 0.f, 0.f, 0.f};
+    if (i < d) {
+      z[0] = Vec4<YT>::ld(yr + i);
+      if (rr) {
+        const float4v q = Vec4<GT>::ld(rr + i);
+        z[0] *= float4v{sigmoid_f(q[0]), sigmoid_f(q[1]), sigmoid_f(q[2]), sigmoid_f(q[3])};
+      }
+      s += z[0][0] * z[0][0] + z[0][1] * z[0][1] + z[0][2] * z[0][2] + z[0][3] * z[0][3];
+    }
+  } else {
 #pragma unroll
-  for (int u = 0; u < NCH; ++u) {
-    const int i = (threadIdx.x + 256 * u) * 4, at = i < d ? i : 0;  // (past the row: any place in it)
-    z[u] = Vec4<YT>::ld(yr + at);
-    if (rr) g[u] = Vec4<GT>::ld(rr + at);
-  }
+    for (int u = 0; u < NCH; ++u) {
+      const int i = (threadIdx.x + 256 * u) * 4, at = i < d ? i : 0;  // (past the row: any place in it)
+      z[u] = Vec4<YT>::ld(yr + at);
+      if (rr) g[u] = Vec4<GT>::ld(rr + at);
+    }
 #pragma unroll
-  for (int u = 0; u < NCH; ++u) {  // on their way during the sum
-    const int i = (threadIdx.x + 256 * u) * 4, at = i < d ? i : 0;
-    xv[u] = Vec4<float>::ld(xr + at);
-    wv[u] = Vec4<float>::ld(w + at);
-  }
+    for (int u = 0; u < NCH; ++u) {  // on their way during the sum
+      const int i = (threadIdx.x + 256 * u) * 4, at = i < d ? i : 0;
+      xv[u] = Vec4<float>::ld(xr + at);
+      wv[u] = Vec4<float>::ld(w + at);
+    }
 #pragma unroll
-  for (int u = 0; u < NCH; ++u) {
-    const int i = (threadIdx.x + 256 * u) * 4;
-    if (rr) z[u] *= float4v{sigmoid_f(g[u][0]), sigmoid_f(g[u][1]), sigmoid_f(g[u][2]), sigmoid_f(g[u][3])};
-    s += i < d ? z[u][0] * z[u][0] + z[u][1] * z[u][1] + z[u][2] * z[u][2] + z[u][3] * z[u][3] : 0.f;
+    for (int u = 0; u < NCH; ++u) {
+      const int i = (threadIdx.x + 256 * u) * 4;
+      if (rr) z[u] *= float4v{sigmoid_f(g[u][0]), sigmoid_f(g[u][1]), sigmoid_f(g[u][2]), sigmoid_f(g[u][3])};
+      s += i < d ? z[u][0] * z[u][0] + z[u][1] * z[u][1] + z[u][2] * z[u][2] + z[u][3] * z[u][3] : 0.f;
+    }
   }
   const float rstd = 1.0f / sqrtf(block_sum(s, scratch) / (float)d + eps);
   float s2 = 0.f;
@@ -223,7 +238,7 @@ __global__ void __launch_bounds__(256) gated_norm_residual_vec_kernel(float* __r
   for (int u = 0; u < NCH; ++u) {
     const int i = (threadIdx.x + 256 * u) * 4;
     if (i < d) {
-      const float4v v = xv[u] + z[u] * rstd * wv[u];
+      const float4v v = NCH == 1 ? Vec4<float>::ld(xr + i) + z[u] * rstd * Vec4<float>::ld(w + i) : xv[u] + z[u] * rstd * wv[u];
       Vec4<float>::st(xr + i, v);
       if (x_cast && !w_next) Vec4<bf16_t>::st(x_cast + (size_t)t * d + i, v);
       z[u] = v;

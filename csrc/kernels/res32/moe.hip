@@ -407,6 +407,7 @@ __global__ void __launch_bounds__(256) moe_combine_vec_kernel(const YT* __restri
                                                                int k, float* __restrict__ out, int d, const AT* __restrict__ add,
                                                                int lda, const float* __restrict__ gate, int ldg) {
   const int t = blockIdx.x, c0 = (blockIdx.y * 256 * NCH + threadIdx.x) * 4;
+  if (c0 >= d) return;
   const float ga = gate ? sigmoid_f(gate[(size_t)t * ldg]) : 1.0f;
   float4v s[NCH];
 #pragma unroll
@@ -497,9 +498,12 @@ extern "C" int r32_moe_combine(const void* Y, int y_f32, const int* inv, const f
 #define LWC_COMBINE(AT, YT, NCH)                                                                                              \
   moe_combine_vec_kernel<AT, YT, NCH><<<dim3(T, (d + 1024 * NCH - 1) / (1024 * NCH)), 256, 0, s>>>(                            \
       (const YT*)Y, inv, wts, (const AT*)h, ldh, k, out, d, (const AT*)add, lda, gate, ldg)
+    // as few workgroups a row as hold it in 4096 columns each, of as few columns as that leaves (5120: two of 3072)
+    const int groups = (d + 4095) / 4096, nch = (d + 1024 * groups - 1) / (1024 * groups);
 #define LWC_COMBINE_N(AT, YT)                  \
-  if (d <= 1024) LWC_COMBINE(AT, YT, 1);       \
-  else if (d <= 2048) LWC_COMBINE(AT, YT, 2);  \
+  if (nch == 1) LWC_COMBINE(AT, YT, 1);        \
+  else if (nch == 2) LWC_COMBINE(AT, YT, 2);   \
+  else if (nch == 3) LWC_COMBINE(AT, YT, 3);   \
   else LWC_COMBINE(AT, YT, 4)
     if (f32 && y_f32) {
       LWC_COMBINE_N(float, float);

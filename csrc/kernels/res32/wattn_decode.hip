@@ -106,13 +106,6 @@ extern "C" int r32_window_attn_decode(const float* q, const void* k_cache, const
   p.min_keys = D > 192 ? 128 : 64;
   const int Hg = H / G;
   const dim3 grid(B, G * ((Hg + 15) / 16), S);
-  p.max_tiles = (int)std::min<long long>(1 << 30, std::max<long long>(1, ((long long)bt_width * block_size + 31) / 32));
-  // Rows of 128 and more entries for 32 and more sequences are taken by length (unordered, the eight waves of a CU are one
-  // sequence's where B divides 256).  Contexts within 50 % of their mean, 32 heads on 8 of 128, us: 64 x 1000 keys 64.8 -> 60.0,
-  // 100 x 700 78.5 -> 69.8; within 80 % 32 x 1000 40.4 -> 36.7, 128 x 600 81.6 -> 75.3; equal ones 57.9 -> 57.5, 128 x 600 65.6 ->
-  // 67.5.  Finding the row costs 1 us: rows of 64 entries lose as much as they gain (64 x 1000 24.5 -> 23.6, equal ones 21.0 ->
-  // 21.8), and so do the wide rows' workgroups (39.1 -> 40.1).  With fewer sequences most splits of a short one have no keys.
-  p.rounds = D <= 192 && D >= 128 && Dv >= 128 && B >= 32 && (long long)grid.x * grid.y * grid.z > 256 ? 8 : 0;
   int rc = -1;
   if (D > 192) {  // one wide row for all heads: a low-rank attention's cached latent + rotated part
     const int chunks = (Hg + 15) / 16, nc = chunks > 1 ? 2 : 1;  // more than 16 heads: two chunks per workgroup

@@ -18,7 +18,7 @@ LWC_DEVICE float4v mfma16(const short8& a, const short8& b, const float4v& c) {
 // cache into the operands — no LDS: a K row's 16 bytes are an A operand as they lie, the interleaved V word is a
 // B operand as it lies.  Same arithmetic as the portion kernel (hi + lo halves of q and of the weights, bias
 // table, fp32 online softmax).  Bound by the reads of the cache: 64 sequences of 500 to 1500 keys (1000 on average), 32
-// heads over 8 of 128 entries, take 60 us for 254 MB (41 us at the rate of a plain read of memory) in tables of 4096 keys.
+// heads over 8 of 128 entries, take 54 us for 258 MB (42 us at the rate of a plain read of memory) in tables of 4096 keys.
 // With the splits cut for the table's width and every load of a tile waited for on its own it took 137 us, and 189 instead
 // of 104 us at 2048 keys each.  Each split leaves an unnormalised partial (o, m, l); the reduce kernel merges
 // them (splits == 1: still through the reduce, which then only normalises).
@@ -37,8 +37,6 @@ struct WAttnDecodeParams {
   float cap;               // > 0: scores become cap tanh(score / cap)
   float* part_o;           // [B, H, S, Dv]
   float* part_ml;          // [B, H, S, 2]
-  int max_tiles;           // tiles of 32 keys of the longest row there could be, at least 1
-  int rounds;              // > 0: workgroups take the rows by their keys, that many of them resident per CU
   int H, G, S, min_keys;  // min_keys: the fewest keys a split takes before the next one gets any (a multiple of 32)
 };
 
@@ -56,22 +54,13 @@ template <int ND, int NV, int NW = 1, bool QLO = true, bool VK = false, int NC =
 __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const WAttnDecodeParams p) {
   constexpr int D = 32 * ND, DV = 16 * NV, NVW = NV / NW, NT = 64 * NW * NC;  // NT: threads of the workgroup
   static_assert(NV % NW == 0, "value tiles divide among the waves");
-  int b = blockIdx.x, split = blockIdx.z, gy = blockIdx.y;
+  const int b = blockIdx.x, split = blockIdx.z;
   const int H = p.H, G = p.G, Hg = H / G, chunks = (Hg + 15) / 16;
   // (one wave: the wave index is a compile-time zero, so the value tiles' offsets stay immediates)
   const int lane = NT > 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x, wv_all = NT > 64 ? (int)(threadIdx.x >> 6) : 0;
   const int wv = NC > 1 ? wv_all % NW : wv_all, cw = NC > 1 ? wv_all / NW : 0;
   const int cgroups = (chunks + NC - 1) / NC;  // workgroups per kv head
-  if (NT == 64 && p.rounds > 0) {
-    const int per = gridDim.y * p.S, at = ranked_place(b + gridDim.x * (gy + gridDim.y * split), gridDim.x * per, p.rounds);
-    b = ranked_row(gridDim.x, at / per, lane, p.max_tiles, [&](int row) {
-      const int i = p.positions[row], lo = max(max(0, i - p.window + 1), p.chunk > 0 ? i - i % p.chunk : 0);
-      return (i + 1 - lo + 31) / 32;
-    });
-    gy = at % per % gridDim.y;
-    split = at % per / gridDim.y;
-  }
-  const int g = gy / cgroups, h0 = g * Hg + ((gy % cgroups) * NC + cw) * 16;
+  const int g = blockIdx.y / cgroups, h0 = g * Hg + ((blockIdx.y % cgroups) * NC + cw) * 16;
   const int nh = min(16, g * Hg + Hg - h0);  // heads of this chunk (<= 0: a wave past the last chunk only helps staging)
   const int r16 = lane & 15, g4 = lane >> 4;
   const int i = p.positions[b];
