@@ -412,10 +412,11 @@ def _few_fp8(rows: int, G: int, N: int, K: int) -> bool:
     splits K over workgroups: where the tiles that the routing reaches are enough for the length of K.  us on one MI355X, N x K x
     groups at 0.25 / 0.5 / 1 / 4 / 31 rows per group, 128-row kernel / small tiles: 28672 x 4096 x 8 SwiGLU 75 / 43, 112 / 85, 172 /
     123, 243 / 157, 339 / 164; 4096 x 14336 x 8 37 / 48, 65 / 53, 85 / 63, 127 / 81, 178 / 87; 4096 x 16384 x 8 43 / 53, 73 / 57,
-    107 / 71, 154 / 95, 209 / 104; 2048 x 7168 x 8 21 / 26, 25 / 27, 28 / 28, 43 / 29, 56 / 32; 2816 x 2048 x 32 31 / 14 to 95 / 41;
-    4096 x 4096 x 2 17 / 15 to 37 / 18; short K keeps the 128-row kernel: 2048 x 768 x 128 56 / 73, 59 / 70, 63 / 70, 72 / 69, 92 /
+    107 / 71, 154 / 95, 209 / 104; 2048 x 7168 x 8 21 / 26, 25 / 27, 29 / 32, 43 / 29, 56 / 32; 2816 x 2048 x 32 31 / 14 to 95 / 41;
+    4096 x 4096 x 2 17 / 15 to 37 / 18; 4096 x 7168 and 8192 x 8 at 0.25 26 / 27 and 26 / 30; short K keeps the 128-row kernel: 2048 x 768 x 128 56 / 73, 59 / 70, 63 / 70, 72 / 69, 92 /
     91, 2048 x 512 x 256 174 / 256 to 210 / 264."""
-    return K >= 1024 and 160 * _hit_groups(rows, G) * -(-N // 128) >= K
+    tiles = _hit_groups(rows, G) * -(-N // 128)
+    return K >= 1024 and 160 * tiles >= K and (tiles >= 96 or K <= 4096)
 
 
 def _few_fp8_layout(A, W, rows, N, K, out, a_rows, a_scale, w_scale) -> bool:
@@ -438,12 +439,12 @@ def _few_bf16(rows: int, G: int, N: int, K: int) -> int:
     / 174; 4096 x 7168 x 8 39 / 50, 61 / 61, 82 / 66, 102 / 85; 2048 x 7168 x 8 26 / 48, 38 / 49, 45 / 56, 61 / 60; 1536 x 2048 x
     128 158 / 94 to 191 / 151; 5632 x 2048 x 64 183 / 104 to 285 / 242; but 2048 x 768 x 128 68 / 78 to 89 / 85, 2048 x 512 x 256
     178 / 259 to 167 / 210, 4096 x 4096 x 2 17 / 27 to 23 / 29.  K of multiples of 4096, whose rows lie on few memory channels:
-    up to half a row per group, 14336 x 4096 x 8 SwiGLU 65 / 52, 109 / 101, 158 / 161, 192 / 212; 28672 x 4096 x 8 114 / 105, 194 /
-    192, 269 / 307, 362 / 381; 8192 x 4096 x 16 77 / 57, 105 / 100, 155 / 156, 178 / 190; 4096 x 8192 x 8 never, 45 / 57, 71 / 73,
+    up to a quarter of a row per group, 14336 x 4096 x 8 SwiGLU 65 / 52, 109 / 101, 158 / 161, 192 / 212; 28672 x 4096 x 8 114 / 105, 188
+    / 203, 269 / 307, 362 / 381; 8192 x 4096 x 16 77 / 57, 105 / 100, 155 / 156, 178 / 190; 4096 x 8192 x 8 never, 45 / 57, 71 / 73,
     101 / 108, 131 / 150."""
     tiles = _hit_groups(rows, G) * -(-N // 128)
     return 2 if rows < 3 * G and K >= 1024 and N % 16 == 0 and tiles >= 96 and 96 * tiles >= K and \
-        (K % 4096 != 0 or (K == 4096 and 2 * rows <= G)) else 0
+        (K % 4096 != 0 or (K == 4096 and 4 * rows <= G)) else 0
 
 
 def _grouped_bf16(rows: int, G: int, N: int, K: int) -> int:

@@ -80,6 +80,19 @@ def choice(M: int, N: int, K: int, epi: str) -> str:
     return "blas"
 
 
+def _g8_fill(M: int, N: int, K: int) -> float:
+    """How much of gemm8p's time on 256 CUs is its product's, by the costs that its row tile is chosen by (``row_tile`` in
+    csrc/kernels/gemm8p.hip: us per K iteration and round of 256, 224 and 192 rows, the hand-off of cut tiles)."""
+    KT, least = K // 64, float("inf")
+    for bm, cost in ((256, 1.0), (224, 0.89), (192, 0.83)):
+        tiles = -(-M // bm) * -(-N // 256)
+        G = 256 if tiles * KT >= 2048 else 8 * max(1, tiles * KT // 64)
+        rest = tiles % G
+        cut = 0.0 if rest == 0 else 10 + 45.0 * rest / G if tiles > G else 10.0 if G % tiles == 0 else 15.0 * G / tiles
+        least = min(least, 1.56 * cost * KT * tiles / G + cut)
+    return 1.56 * KT * (M / 256) * (N / 256) / 256 / least
+
+
 def _untuned(M: int, N: int, K: int, epi: str) -> str:
     """The backend of a shape that no one tuned: a core of its own where it was as fast as the library or faster over a range of
     sizes (times relative to the library, weights from memory), else the library.
@@ -89,10 +102,12 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
     14336 x 2048, 8192 and 16384 x 1024, 16384 x 2048, 22016 and 28672 x 4096, 27648 x 5120 0.72 to 1.01, but 8192 x 4096
     0.65 to 1.09, 11264 x 4096 0.76 to 1.07, 9216 x 1152 up to 1.09, 4096 x 2048 up to 1.24. 32768 x 8192: 0.90 to 1.05.
 
-    Hundreds of rows, where gemm8p's row tile fits them (22 counts of 545 to 3600): gate|up 22016 and 28672 x 4096, 27648 x 5120
-    0.65 to 1.04 from 545 to 1900 rows and 0.75 to 0.98 from 2401 to 3600, between them up to 1.10, fewer columns either way
-    (14336 x 4096 0.74 to 1.17, 8192 x 4096 0.88 to 1.20), 32768 x 4096 up to 1.11. Down into 16 column tiles, 4096 x 11008 and
-    14336: 0.53 to 1.00 from 545 to 1900 rows; 2048 x 14336 up to 1.15, 5120 x 13824 1.10, 8192 x 14336 1.11, 4096 x 8192 1.14.
+    Hundreds of rows, where gemm8p's row tile fits them (90 counts of 545 to 3600): gate|up 22016, 24576 and 28672 x 4096, 24576 x
+    4608, 25600 and 27648 x 5120 0.63 to 1.06 from 545 to 1900 rows and 0.76 to 1.04 from 2401 to 3600 where its tiles fill their
+    rounds (:func:`_g8_fill`), else up to 1.16 (25600 x 5120, 913 rows); between the two up to 1.10, fewer columns either way
+    (14336 x 4096 0.74 to 1.17, 8192 x 4096 0.88 to 1.20), 32768 x 4096 up to 1.11. Down into 16 column tiles, 3968 x 12288, 4096 x
+    11008, 12800 and 14336: 0.49 to 1.02 from 545 to 1900 rows but for 897 to 960 (1.03 to 1.08 at K 11008, 0.94 to 1.04 above); 2048
+    x 14336 up to 1.15, 5120 x 13824 1.10, 8192 x 14336 1.11, 4096 x 8192 1.14.
 
     Few rows (prefill: a batch of prompts' last layer runs on their last tokens only, and short prompts on few rows
     everywhere): the weight's read bounds them. gate|up, which saves its SwiGLU pass, up to 64 rows on gemm2w: 11264, 14336
@@ -107,7 +122,7 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
         if M > 4608:  # (M * N: 32-bit byte offsets)
             wide = N >= (8192 if M > 8192 or K <= 1024 else 14336)
             return "g8" if wide and 1 << 23 <= size < 1 << 28 and M * N < 1 << 30 else "blas"
-        if 22016 <= N <= 28672 and 4096 <= K <= 5120 and (544 < M <= 1900 or 2400 < M <= 3600):
+        if 22016 <= N <= 28672 and 4096 <= K <= 5120 and (544 < M <= 1900 or 2400 < M <= 3600) and _g8_fill(M, N, K) >= 0.8:
             return "g8"
         return "g2" if M <= 64 and N >= 8192 and K <= 4096 and 1 << 25 <= size <= 1 << 27 else "blas"
     if epi == "residual" and 3840 < N <= 4096 and 11008 <= K <= 14336 and 544 < M <= 1900:

@@ -61,7 +61,7 @@ def test_transforms_modes_and_traces_keep_the_library():
     (16, 16384, 1024, "plain", "blas"), (5, 6144, 4096, "plain", "blas"), (17, 4096, 4096, "plain", "blas"),
     (32, 4096, 14336, "residual", "blas"), (33, 4096, 14336, "residual", "g2"), (64, 16384, 1024, "plain", "g2"),
     (48, 8192, 4096, "plain", "blas"), (64, 14336, 4096, "plain", "blas"), (65, 4096, 14336, "plain", "blas"),
-    (545, 22016, 4096, "swiglu", "g8"), (1900, 27648, 5120, "swiglu", "g8"), (544, 28672, 4096, "swiglu", "blas"),
+    (654, 22016, 4096, "swiglu", "g8"), (1900, 27648, 5120, "swiglu", "g8"), (913, 25600, 5120, "swiglu", "blas"), (1283, 25600, 5120, "swiglu", "g8"), (544, 28672, 4096, "swiglu", "blas"),
     (1901, 28672, 4096, "swiglu", "blas"), (2401, 28672, 4096, "swiglu", "g8"), (3601, 28672, 4096, "swiglu", "blas"),
     (1095, 14336, 4096, "swiglu", "blas"), (1095, 32768, 4096, "swiglu", "blas"), (777, 4096, 14336, "residual", "g8"),
     (777, 4096, 14336, "plain", "blas"), (1901, 4096, 14336, "residual", "blas"), (777, 5120, 13824, "residual", "blas")])

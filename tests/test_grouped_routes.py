@@ -100,7 +100,7 @@ def test_bf16_kernel_by_sizes(taken, monkeypatch, N, K, G, rows, core, swiglu):
 
 @pytest.mark.parametrize("N,K,G,rows,core", [
     # (less than three rows a group, ``ops._few_bf16``: rows of all groups)
-    (14336, 4096, 8, 2, 2), (14336, 4096, 8, 4, 2), (14336, 4096, 8, 5, 0), (14336, 4096, 8, 24, 0), (14336, 4096, 8, 31, 0), (4096, 14336, 8, 4, 0),
+    (14336, 4096, 8, 2, 2), (14336, 4096, 8, 3, 0), (14336, 4096, 8, 5, 0), (14336, 4096, 8, 24, 0), (14336, 4096, 8, 31, 0), (4096, 14336, 8, 4, 0),
     (4096, 14336, 8, 8, 2), (4096, 14336, 8, 23, 2), (4096, 14336, 8, 24, 0), (4096, 7168, 8, 2, 0), (4096, 7168, 8, 4, 2), (4096, 8192, 8, 4, 0), (1536, 2048, 128, 64, 2), (2048, 768, 128, 128, 0),
     (4096, 4096, 2, 4, 0), (6144, 16384, 8, 8, 0), (328, 4096, 64, 128, 0)])
 def test_bf16_kernel_of_few_rows(taken, monkeypatch, N, K, G, rows, core):
@@ -112,7 +112,7 @@ def test_bf16_kernel_of_few_rows(taken, monkeypatch, N, K, G, rows, core):
 @pytest.mark.parametrize("N,K,G,rows,few", [
     # (what measured fastest, ``ops._few_fp8``: rows of all groups)
     (28672, 4096, 8, 2, True), (4096, 14336, 8, 2, False), (4096, 14336, 8, 4, True), (4096, 16384, 8, 4, True), (2816, 2048, 32, 8, True),
-    (4096, 4096, 2, 1, True), (2048, 768, 128, 400, False), (2048, 512, 256, 64, False), (2048, 7168, 8, 255, True)])
+    (4096, 4096, 2, 1, True), (2048, 768, 128, 400, False), (2048, 512, 256, 64, False), (2048, 7168, 8, 255, True), (2048, 7168, 8, 8, False), (2048, 7168, 8, 16, True), (4096, 8192, 8, 2, False)])
 @pytest.mark.parametrize("swiglu", [False, True])
 def test_fp8_kernel_of_few_rows(taken, monkeypatch, N, K, G, rows, few, swiglu):
     """Row scales either way: the middle of an expert stays out of MX form below 32 rows a group."""
