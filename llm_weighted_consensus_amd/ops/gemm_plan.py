@@ -302,7 +302,8 @@ def _enc_ok(n: str, x: torch.Tensor, w: torch.Tensor, epi: str, other: torch.Ten
 
 
 # gemm8p is taken for an encoder's projection where it leads by this much: between an encoder's other kernels it does not keep a
-# small lead (24 layers of bge-large over 7156 rows with its FFN1 of 70 us on gemm8p 6116 us, on the library 5998, on gemm2w 6079)
+# small lead.  The stacks of three widths at eight counts of 1577 to 32498 tokens, chosen with this lead and without: bge-large 7078
+# (FFN1) 5697 / 5716 us, 16252 (qkv) 9830 / 10015, bge-base 11904 (FFN2) 3643 / 3713; at the others the choice is the same
 G8_LEAD = 0.95
 
 
