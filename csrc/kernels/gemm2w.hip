@@ -33,10 +33,18 @@ struct Params {
   int splits;   // K ranges per tile
   float* part;  // splits > 1: [tiles][splits][TM * TN] partial tiles
   int* count;   // [tiles] finished ranges (zero between launches)
-  RowSumsq ss;  // NORM: read by EPI_PLAIN, EPI_SWIGLU and EPI_ROPE_KV, written by EPI_RESIDUAL
-  RopeKV kv;    // EPI_ROPE_KV
-  int turned;   // a tile's walk over its K range starts at a step of its own
+  int turned;   // > 0: a tile's walk over its K range starts at a step of its own, 0 .. turned
 };
+
+// Of the builds with the folded norm alone (as arguments of every call they cost each 0.3 us)
+struct NormParams : Params {
+  RowSumsq ss;  // read by EPI_PLAIN, EPI_SWIGLU and EPI_ROPE_KV, written by EPI_RESIDUAL
+  RopeKV kv;    // EPI_ROPE_KV
+};
+template <bool NORM>
+struct ArgsOf { using type = Params; };
+template <>
+struct ArgsOf<true> { using type = NormParams; };
 
 LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
@@ -58,7 +66,7 @@ constexpr int kGroupM = 8;
 // EPI_ROPE_KV (64 x 64 tiles, step_fuse.h): a tile takes 32 columns of a head and the 32 that rotate with them, D / 2 further.
 // NORM (64 x 64 tiles): the folded RMSNorm of step_fuse.h.
 template <int EPI, int TM, int TN, int NST, bool NORM>
-__global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
+__global__ void __launch_bounds__(256, 2) gemm2w_kernel(const typename ArgsOf<NORM>::type p) {
   static_assert((!NORM && EPI != EPI_ROPE_KV) || (TM == 64 && TN == 64), "one row of partial sums per lane group");
   constexpr bool kPairs = EPI == EPI_SWIGLU || EPI == EPI_ROPE_KV;  // columns that meet in a lane: groups of 32, two by two
   constexpr int WC = kPairs && TN == 64 ? 1 : 2, WR = 4 / WC;  // waves across the tile's columns and rows
@@ -99,13 +107,16 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
     voW[i] = row < rows_n ? (uint32_t)((row + (EPI == EPI_ROPE_KV && row >= 32 ? far : 0)) * p.K * 2 + (((lane & 7) ^ ((row >> 3 & 3) * 2 + (row >> 1 & 1))) << 4)) : 0x7fffffffu;
   }
   const int KT = p.K / 64, k0 = KT * split / p.splits, nk = KT * (split + 1) / p.splits - k0;
-  const int turn0 = p.turned ? (int)((unsigned)(in / gsz * 3) % (unsigned)nk) : 0;
-  auto stage = [&](uint8_t* buf, int step) {
-    const int kt = k0 + (step + turn0 < nk ? step + turn0 : step + turn0 - nk);
+  // (the steps are asked for in order: the byte of K that the next one begins at)
+  const int first_k = k0 * 128, past_k = first_k + nk * 128;
+  int next_k = first_k + (in / gsz * 3 & p.turned) * 128;
+  auto stage = [&](uint8_t* buf) {
 #pragma unroll
-    for (int i = 0; i < IA; ++i) dma16(rA, buf + (i * 4 + wid) * 1024, voA[i], kt * 128);
+    for (int i = 0; i < IA; ++i) dma16(rA, buf + (i * 4 + wid) * 1024, voA[i], next_k);
 #pragma unroll
-    for (int i = 0; i < IW; ++i) dma16(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], kt * 128);
+    for (int i = 0; i < IW; ++i) dma16(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], next_k);
+    next_k += 128;
+    next_k = next_k == past_k ? first_k : next_k;
   };
   // operand reads: A tile i holds rows 16 i + r16; W tile (g, h) holds rows 32 g + 8 (r16 / 4) + 4 h + r16 % 4, so that a
   // lane's accumulators of the pair h = 0, 1 are the eight consecutive columns 32 g + 8 q .. of output row r16
@@ -138,11 +149,11 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
   }
   RopeAhead<8> ahead;
   if constexpr (EPI == EPI_ROPE_KV) rope_kv_row(p.kv, ahead, min(m0 + wr * 16 + r16, p.M - 1), n0 / p.kv.D);
-  __builtin_amdgcn_sched_barrier(0);
+  if constexpr (NORM) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int k = 0; k < NST; ++k)  // (NORM: steps past the range too, rows that nothing reads: behind a branch the sums would wait for all)
-    if (NORM || k < nk) stage(smem + k * kStage, k);
-  __builtin_amdgcn_sched_barrier(0);
+    if (NORM || k < nk) stage(smem + k * kStage);
+  if constexpr (NORM) __builtin_amdgcn_sched_barrier(0);
   if constexpr (EPI == EPI_ROPE_KV) rope_kv_angles(p.kv, ahead, n0 / p.kv.D, n0 % p.kv.D + 8 * q);
   if constexpr (kScale) {
 #pragma unroll
@@ -179,7 +190,7 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();  // every wave holds the step's operands: its buffer takes the step after next
     asm volatile("" ::: "memory");
-    if (kt + NST < nk) stage(buf, kt + NST);
+    if (kt + NST < nk) stage(buf);
     __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
@@ -328,7 +339,7 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const Params p) {
 }
 
 template <int EPI, int TM, int TN, int NST, bool NORM = false>
-int launch(Params p, hipStream_t s) {
+int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
   constexpr int kLds = NST * (TM + TN) * 128;
   static const hipError_t attr =
       hipFuncSetAttribute((const void*)gemm2w_kernel<EPI, TM, TN, NST, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
@@ -342,7 +353,9 @@ int launch(Params p, hipStream_t s) {
   // themselves (128256 x 4096 185 / 202 / 212 -> 199 / 213 / 217), and from 300 rows on the matrix cores are the bound.  Plain
   // products without the folded norm, the projections of the models with routed experts, walk K from its start: behind them a
   // router picks experts, and another order of the sums moves rows that nearly tie (gemm2g.hip).
-  p.turned = (NORM || EPI != EPI_PLAIN) && p.M <= 256 && (long long)p.tiles_m * p.tiles_n <= 1024 && (p.K % 2048 == 0 || p.K % 1024 != 0);
+  const bool turned = (NORM || EPI != EPI_PLAIN) && p.M <= 256 && (long long)p.tiles_m * p.tiles_n <= 1024 && (p.K % 2048 == 0 || p.K % 1024 != 0);
+  p.turned = 0;  // (a power of two less one: a division would hold the first loads back)
+  while (turned && 2 * p.turned + 2 <= p.K / 64 / p.splits) p.turned = 2 * p.turned + 1;
   gemm2w_kernel<EPI, TM, TN, NST, NORM><<<p.tiles_m * p.tiles_n * p.splits, 256, kLds, s>>>(p);
   return (int)hipGetLastError();
 }
@@ -400,12 +413,15 @@ extern "C" int lwc_gemm2w(const void* A, const void* W, void* C, const void* R, 
   if (M == 0 || N == 0) return 0;
   if (((long long)M + 63) / 64 * ((N + 63) / 64) * splits >= (1LL << 31)) return -1;
   const Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc, 0, 0,
-                 splits, part, count, ss != nullptr ? *ss : lwc::RowSumsq{}, kv != nullptr ? *kv : lwc::RopeKV{}, 0};
-  if (ss != nullptr) switch (epi) {
-    case EPI_PLAIN: return launch<EPI_PLAIN, 64, 64, 4, true>(p, s);
-    case EPI_RESIDUAL: return launch<EPI_RESIDUAL, 64, 64, 4, true>(p, s);
-    case EPI_SWIGLU: return launch<EPI_SWIGLU, 64, 64, 4, true>(p, s);
-    default: return launch<EPI_ROPE_KV, 64, 64, 4, true>(p, s);
+                 splits, part, count, 0};
+  if (ss != nullptr) {
+    const NormParams np{p, *ss, kv != nullptr ? *kv : lwc::RopeKV{}};
+    switch (epi) {
+      case EPI_PLAIN: return launch<EPI_PLAIN, 64, 64, 4, true>(np, s);
+      case EPI_RESIDUAL: return launch<EPI_RESIDUAL, 64, 64, 4, true>(np, s);
+      case EPI_SWIGLU: return launch<EPI_SWIGLU, 64, 64, 4, true>(np, s);
+      default: return launch<EPI_ROPE_KV, 64, 64, 4, true>(np, s);
+    }
   }
 #define LWC_G2W(E)                                                                     \
   case E:                                                                              \
