@@ -106,8 +106,8 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
     4608, 25600 and 27648 x 5120 0.63 to 1.06 from 545 to 1900 rows and 0.76 to 1.04 from 2401 to 3600 where its tiles fill their
     rounds (:func:`_g8_fill`), else up to 1.16 (25600 x 5120, 913 rows); between the two up to 1.10, fewer columns either way
     (14336 x 4096 0.74 to 1.17, 8192 x 4096 0.88 to 1.20), 32768 x 4096 up to 1.11. Down into 16 column tiles, 3968 x 12288, 4096 x
-    11008, 12800 and 14336: 0.49 to 1.02 from 545 to 1900 rows but for 897 to 960 (1.03 to 1.08 at K 11008, 0.94 to 1.04 above); 2048
-    x 14336 up to 1.15, 5120 x 13824 1.10, 8192 x 14336 1.11, 4096 x 8192 1.14.
+    11008, 12800 and 14336: 0.49 to 1.03 from 545 to 1900 rows but for 897 to 960 at the narrower K (0.97 to
+    1.08; 0.94 to 0.99 at 14336); 2048 x 14336 up to 1.15, 5120 x 13824 1.10, 8192 x 14336 1.11, 4096 x 8192 1.14.
 
     Few rows (prefill: a batch of prompts' last layer runs on their last tokens only, and short prompts on few rows
     everywhere): the weight's read bounds them. gate|up, which saves its SwiGLU pass, up to 64 rows on gemm2w: 11264, 14336
@@ -125,8 +125,8 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
         if 22016 <= N <= 28672 and 4096 <= K <= 5120 and (544 < M <= 1900 or 2400 < M <= 3600) and _g8_fill(M, N, K) >= 0.8:
             return "g8"
         return "g2" if M <= 64 and N >= 8192 and K <= 4096 and 1 << 25 <= size <= 1 << 27 else "blas"
-    if epi == "residual" and 3840 < N <= 4096 and 11008 <= K <= 14336 and 544 < M <= 1900:
-        return "g8"
+    if epi == "residual" and 3840 < N <= 4096 and 11008 <= K <= 14336 and 544 < M <= 1900 and not (896 < M <= 960 and K <= 12800):
+        return "g8"  # (from 897 to 960 rows a fifth row tile, of 192 or 224, has little to do)
     if M <= 16 and K <= 4096 and N <= 8 * K and 1 << 22 <= size <= 1 << 24:
         return "gv"
     return "g2" if 32 < M <= 64 and (N < 8192 or K <= 2048) and 1 << 24 <= size <= 1 << 26 else "blas"

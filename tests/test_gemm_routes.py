@@ -64,7 +64,8 @@ def test_transforms_modes_and_traces_keep_the_library():
     (654, 22016, 4096, "swiglu", "g8"), (1900, 27648, 5120, "swiglu", "g8"), (913, 25600, 5120, "swiglu", "blas"), (1283, 25600, 5120, "swiglu", "g8"), (544, 28672, 4096, "swiglu", "blas"),
     (1901, 28672, 4096, "swiglu", "blas"), (2401, 28672, 4096, "swiglu", "g8"), (3601, 28672, 4096, "swiglu", "blas"),
     (1095, 14336, 4096, "swiglu", "blas"), (1095, 32768, 4096, "swiglu", "blas"), (777, 4096, 14336, "residual", "g8"),
-    (777, 4096, 14336, "plain", "blas"), (1901, 4096, 14336, "residual", "blas"), (777, 5120, 13824, "residual", "blas")])
+    (777, 4096, 14336, "plain", "blas"), (896, 4096, 11008, "residual", "g8"), (897, 4096, 11008, "residual", "blas"), (960, 4096, 12800, "residual", "blas"),
+    (961, 4096, 12800, "residual", "g8"), (913, 4096, 14336, "residual", "g8"), (1901, 4096, 14336, "residual", "blas"), (777, 5120, 13824, "residual", "blas")])
 def test_untuned_rule(M, N, K, epi, core):
     assert gemm_plan._untuned(M, N, K, epi) == core
 
