@@ -36,7 +36,7 @@ struct Params {
   int turned;   // > 0: a tile's walk over its K range starts at a step of its own, 0 .. turned
 };
 
-// Of the builds with the folded norm alone (as arguments of every call they cost each 0.3 us)
+// Arguments of the builds with the folded norm alone: the others neither take nor load them
 struct NormParams : Params {
   RowSumsq ss;  // read by EPI_PLAIN, EPI_SWIGLU and EPI_ROPE_KV, written by EPI_RESIDUAL
   RopeKV kv;    // EPI_ROPE_KV
