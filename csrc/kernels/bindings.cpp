@@ -884,11 +884,17 @@ c10::optional<at::Tensor> encoder_layers(at::Tensor x, const std::vector<at::Ten
     const at::Tensor &t = weights[i], &first = weights[i % 12];
     if (!t.is_contiguous() || t.scalar_type() != at::kBFloat16 || t.sizes() != first.sizes() || ((uintptr_t)t.data_ptr() & 15)) return c10::nullopt;
   }
+  at::Tensor ws, flags;
+  if (std::find(cores.begin(), cores.end(), 3) != cores.end()) {
+    if (!part.has_value() || !count.has_value()) return c10::nullopt;
+    ws = *part, flags = *count;
+  }
   at::Tensor qkv = at::empty({T, 3 * d}, x.options()), a = at::empty({T, d}, x.options()), h = at::empty({T, f}, x.options());
   at::Tensor y = at::empty({T, d}, x.options()), z = at::empty({T, d}, x.options());
   const at::Tensor q = qkv.narrow(1, 0, d), k = qkv.narrow(1, d, d), v = qkv.narrow(1, 2 * d, d);
   auto gemm = [&](int64_t core, const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const at::Tensor& R, int64_t epi) {
     if (core == 1) skinny_gemm(A, W, C, R, epi);
+    else if (core == 3) gemm8p(A, W, C, R, epi, ws, flags);
     else gemm2w(A, W, C, R, epi, -1, 1, part, count);
   };
   for (size_t l = 0; l < weights.size(); l += 12) {

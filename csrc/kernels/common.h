@@ -83,15 +83,22 @@ LWC_DEVICE float block_max(float v, float* scratch) {
   return wave_max(r);
 }
 
-// erf by Abramowitz & Stegun 7.1.26 (|error| < 1.5e-7, far below bf16's resolution): one exp, one rcp and a
-// 5-term polynomial — the libm erff's branches made the fused epilogue cost more than a separate pass.
-LWC_DEVICE float erf_as(float x) {
-  const float a = fabsf(x);
-  const float t = __builtin_amdgcn_rcpf(1.f + 0.3275911f * a);  // v_rcp_f32 (1 ulp): __frcp_rn is a full division sequence
-  const float y = t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
-  return copysignf(1.f - y * __expf(-a * a), x);
+// x Phi(x), the erf form of GELU, as max(x, 0) - |x| Phi(-|x|), with log2 Phi(-a) a polynomial over 0 <= a <= 5.6 (least squares at
+// Chebyshev nodes, weights moved towards the minimax of |x| times the error; beyond 5.6 the last term stays at 6e-8).  One exp2 and
+// eleven other instructions per element, where erf by Abramowitz & Stegun 7.1.26 took one exp, one rcp and fourteen: a tile of 256 x
+// 256 spends 0.4 us on each.  Error in fp32 arithmetic over N(0, 1) and a grid of [-6, 6]: at most 2.4e-7, rms 8.6e-8 (with erf
+// 4.7e-7 and 8.8e-8), and of the value at most 2.2e-5 for |x| < 4 (with erf 9.3e-4).  NaN stays NaN (minimum, not min).
+LWC_DEVICE float gelu_erf(float x) {
+  const float a = __builtin_elementwise_minimum(fabsf(x), 5.6f);
+  float l = fmaf(-1.437473542864609e-06f, a, 5.503627471625805e-05f);
+  l = fmaf(l, a, -0.0008901672554202378f);
+  l = fmaf(l, a, 0.008395220153033733f);
+  l = fmaf(l, a, -0.05382503569126129f);
+  l = fmaf(l, a, -0.45850393176078796f);
+  l = fmaf(l, a, -1.1512768268585205f);
+  l = fmaf(l, a, -0.9999866485595703f);
+  return fmaf(-a, __builtin_amdgcn_exp2f(l), fmaxf(x, 0.f));
 }
-LWC_DEVICE float gelu_erf(float x) { return 0.5f * x * (1.f + erf_as(x * 0.70710678118654752f)); }
 
 // Reductions over the 4 lanes {l, l^16, l^32, l^48} holding one query row's tokens: two VALU
 // half-swaps (v_permlane32_swap / v_permlane16_swap, gfx950) instead of LDS ds_bpermute round trips.

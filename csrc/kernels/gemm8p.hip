@@ -1,11 +1,11 @@
-// K6 dense projection GEMM, 8-phase schedule + stream-K tail: C = A . W^T for the decode-batch projections
+// K6 dense projection GEMM in two-phase K tiles + stream-K tail: C = A . W^T for the decode-batch projections
 // (M = decode batch 512..4096; N, K >= 4096), with fused epilogues.
 //
 //   C[M, N]  = A[M, K] . W[N, K]^T  (+ R)            EPI_PLAIN / EPI_RESIDUAL
 //   H[M, N/2] = silu(A . Wg^T) * (A . Wu^T)          EPI_SWIGLU, W rows gate/up interleaved in blocks of 32
 //                                                     (ops.swiglu_interleave), so one tile holds both halves
 //
-// Tile pipeline (cdna_hip_programming.md §5 "The 256² 8-phase template", written for this kernel's operand split):
+// Tile pipeline:
 //   workgroup : 8 waves (512 threads) = 2 (M) x 4 (N); wave tile 128 x 64 = 8 x 4 MFMA 16x16 tiles,
 //               mfma_f32_16x16x32_bf16, 128 fp32 accumulators per lane.  Row tiles of 224 and 192 (R1 = 3, 2, row_tile): the
 //               second quadrant has R1 instead of 4 tiles of 16 rows, the rest of unit A1 is not loaded.
@@ -16,39 +16,44 @@
 //                 B0 = W rows {0..31, 64..95, 128..159, 192..223} (ni=0 of the 4 wave columns)
 //                 B1 = the other 128 W rows (ni=1)
 //               Two K-tile buffers (128 KiB LDS).
-//   phases    : 4 per K tile, one C quadrant (4 x 2 MFMA tiles x K 64 = 16 MFMAs) each:
-//                 P1 reads B0 + A0 -> acc[0..3][0..1]     stage A0(t+1)  vmcnt(4) (retires B1(t))
-//                 P2 reads B1      -> acc[0..3][2..3]     stage B0(t+1)  vmcnt(4) (retires A1(t))
-//                 P3 reads A1      -> acc[4..7][2..3]     stage B1(t+1)
-//                 P4 (registers)   -> acc[4..7][0..1]     stage A1(t+1)  vmcnt(4) (retires A0, B0 (t+1))
-//               Each phase: ds_reads, 2 x glds, counted vmcnt, s_barrier, MFMA cluster at raised priority,
-//               s_barrier.  vmcnt never reaches 0 inside the loop: 2-3 units stay in flight across the
+//   phases    : 2 per K tile, half of the wave's rows times all of its columns (32 MFMAs) each:
+//                 P1 reads B0 B1 A0 -> acc[0..3]   stages A1 of tile t+1           vmcnt(8) (retires A1(t))
+//                 P2 reads A1       -> acc[4..7]   stages A0, B0, B1 of tile t+2   vmcnt(8) (retires A0, B0, B1 (t+1))
+//               Each phase: ds_reads, LDS-DMA, counted vmcnt, lgkmcnt(0), s_barrier, MFMA cluster at raised priority,
+//               s_barrier.  vmcnt never reaches 0 inside the loop: a whole K tile stays in flight across the
 //               barriers.  The two wave rows run one barrier apart (wr == 1 passes an extra barrier first),
-//               so on every SIMD one wave issues MFMAs while its partner reads LDS and issues loads.
+//               so on every SIMD one wave issues MFMAs while its partner reads LDS and issues loads.  What bounds the loop is
+//               the MFMAs and the hand-over of the matrix cores at the barriers.  Measured, us: four phases of 16 MFMAs with
+//               the wait for their reads behind the barrier 719 at 8192^3, 657 at 4096 x 28672 x 4096; two phases 686 and
+//               618; two with the DMA between the MFMAs instead 791 and 716; four with reads a phase ahead 736 and 662.
 //   hazards   : RAW - a unit is read in the phase after the wait that retired it (every wave waits for its
-//               own DMAs, then the barrier).  WAR - a unit buffer is re-staged 4-5 phases after its last read
-//               (>= 2 needed with the staggered wave rows).
-//   LDS image : lane-linear DMA image, 16 B chunk c of unit row r stored at chunk c ^ ((r >> 1) & 7): the
-//               16 lanes of a ds_read_b128 group (16 consecutive rows, same chunk) hit 16 distinct bank quads.
-//               The swizzle is applied to the DMA SOURCE address and to the read (both sides).
+//               own DMAs, then the barrier).  WAR - a wave comes to a phase's first barrier with its operands in registers;
+//               a partner that stages in the next phase has passed that barrier.
+//   tiles     : the loads run ahead over the end of a tile: its last K tile stages the first of the next one, and the epilogue
+//               goes from the registers to memory while they are on their way (its stores are counted in the waits that
+//               follow).  Through LDS, with nothing in flight, a tile of K 768 took 27 us, so 21.
+//   LDS image : lane-linear DMA image, 16 B chunk c of A's unit row r stored at chunk c ^ ((r >> 1) & 7), of W's at c ^ ((r >> 3 &
+//               3) * 2 + (r >> 1 & 1)): the 16 lanes of a ds_read_b128 group (A: 16 consecutive rows, W: rows 8 (l / 4) + l % 4,
+//               same chunk) hit 16 distinct bank quads.  The swizzle is applied to the DMA SOURCE address and to the read.
 //
 // Work distribution (persistent, one workgroup per CU, grid = 8 XCDs x wpx):
 //   The decode shapes do not divide into whole rounds of 256 tiles (qkv at M=3072: 288 tiles = 1.1 rounds;
 //   o / down: 192 = 0.75; gate_up: 1344 = 5.25), so a plain one-tile-per-workgroup grid idles 12-44 % of the
 //   chip in its last round.  Here the first `sk_tiles` tiles (the remainder plus one full round) are split
-//   by K iterations (stream-K): each XCD owns a contiguous, tile-aligned share of them and its wpx workgroups
+//   by K iterations (stream-K; where that costs less than it saves, rest_cost): each XCD owns a contiguous, tile-aligned share of them and its wpx workgroups
 //   split that share's K iterations evenly.  The remaining tiles run data-parallel, one per workgroup per
 //   round, XCD x taking wpx consecutive tiles (m fastest: the XCD's tiles share W panels in its L2).
 //   A tile cut between workgroups is finished by the one holding its last K iteration (the finaliser),
 //   which adds the fp32 partials the others wrote to the workspace.  Each workgroup walks its stream-K
 //   range backwards, so it publishes its partial (range end) first and finalises (range start) last, and
 //   a finaliser only waits on LOWER block ids of its own XCD — workgroups dispatched earlier, hence
-//   resident: no co-residency assumption, no deadlock.  Partial hand-off: plain stores, vmcnt(0), barrier,
-//   agent-scope release + flag store; the reader polls the flag, agent-scope acquire, resets the flag for
-//   the next launch (flags start zeroed), barrier, plain loads.
-//   epilogue  : accumulators -> bf16 (SwiGLU / residual applied in registers) -> LDS -> 16 B row stores.
+//   resident: no co-residency assumption, no deadlock.  Partial hand-off: stores of device scope, vmcnt(0), barrier, flag
+//   store; the reader polls the flag, resets it for the next launch (flags start zeroed), barrier, loads of device
+//   scope.  (With fences instead, each of which writes an XCD's L2 back or drops it: 1095 rows x 6144 x 4096 72 us, so 67; 4096 x
+//   14336 143 and 135.)
 #include <algorithm>
 #include <cstdlib>
+#include <type_traits>
 
 #include "common.h"
 
@@ -61,6 +66,8 @@ constexpr int kUnitB = 128 * 128;   // 128 rows x 128 B
 constexpr int kBufB = 4 * kUnitB;   // one K tile: A0 A1 B0 B1
 constexpr int kLdsB = 2 * kBufB;    // 128 KiB
 constexpr int kUA0 = 0, kUA1 = kUnitB, kUB0 = 2 * kUnitB, kUB1 = 3 * kUnitB;
+// cache policy of buffer loads and stores: device scope (past the caches of one XCD), streaming
+constexpr int kSC1 = 16, kNT = 2;
 constexpr int kPartialF = 256 * 256;  // fp32 partial tile per workgroup
 
 enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4 };
@@ -76,6 +83,7 @@ struct Params {
   int tiles_m, tiles_n, KT;
   int gm;  // tile order: groups of gm m-tiles, n fastest across a group (32 consecutive tiles ~ 4 x 8)
   int wpx, sk_tiles, dp_rounds;
+  int nt;  // the output is larger than the last-level cache: its stores pass the caches by
 };
 
 LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
@@ -107,289 +115,295 @@ LWC_DEVICE void tile_mn(const Params& p, int t, int& m, int& n) {
   n = in / gsz;
 }
 
+// A piece of a workgroup's work: the K iterations [klo, khi) of a tile.
+struct Item {
+  int it, round;  // the items before it: what is left of the stream-K range, data-parallel rounds
+  int tile, klo, khi;
+};
+
 template <int EPI, int R1>
 __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
   constexpr int BMH = 64 + 16 * R1;  // rows of a wave row
+  constexpr int CW = EPI == EPI_SWIGLU ? 32 : 64, NH = CW / 32;  // output columns of a wave, in groups of 32
+  constexpr int kStores = (4 + R1) * NH;  // store instructions of an epilogue
+  constexpr bool kBias = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int KT = p.KT;
   const int xcd = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int tid = threadIdx.x, lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int r16 = lane & 15, q = lane >> 4;
+  const int wr = wid >> 2, wc = wid & 3;
 
   int sk_a = 0, sk_e = 0;
   if (p.sk_tiles > 0) sk_range(p, xcd, j, sk_a, sk_e);
-  int it = sk_e, round = 0;
-
-  while (true) {
-    // ---- next work item: stream-K segments (backwards), then data-parallel tiles ----
-    int tile, klo, khi;
-    if (it > sk_a) {
-      tile = (it - 1) / KT;
-      const int seg = max(sk_a, tile * KT);
-      klo = seg - tile * KT;
-      khi = it - tile * KT;
-      it = seg;
-    } else if (round < p.dp_rounds) {
-      tile = p.sk_tiles + round * 8 * p.wpx + xcd * p.wpx + j;
-      klo = 0;
-      khi = KT;
-      ++round;
-    } else {
-      break;
+  // (divisions run on the vector units; what follows from their results is to stay scalar)
+  auto uni = [](int x) { return __builtin_amdgcn_readfirstlane(x); };
+  sk_a = uni(sk_a), sk_e = uni(sk_e);
+  // ---- the work items, one after the other: stream-K segments (backwards), then data-parallel tiles ----
+  auto next = [&](Item& w) -> bool {
+    if (w.it > sk_a) {
+      w.tile = uni((w.it - 1) / KT);
+      const int seg = max(sk_a, w.tile * KT);
+      w.klo = seg - w.tile * KT;
+      w.khi = w.it - w.tile * KT;
+      w.it = seg;
+      return true;
     }
+    if (w.round >= p.dp_rounds) return false;
+    // (a last round that is not full is spread over the XCDs)
+    const int begin = p.sk_tiles + w.round * 8 * p.wpx, each = min(p.wpx, (p.tiles_m * p.tiles_n - begin + 7) / 8);
+    w.tile = begin + xcd * each + j;
+    if (j >= each || w.tile >= p.tiles_m * p.tiles_n) return false;
+    w.klo = 0;
+    w.khi = KT;
+    ++w.round;
+    return true;
+  };
+
+  // per-thread DMA geometry (byte offsets from the tile's buffer base): unit u, instruction i -> unit row
+  // ru = i*64 + tid/8 at LDS chunk tid%8, which holds a global chunk of that row (swizzle on the source): chunk c of A row r
+  // lies at c ^ (r / 2 % 8), of W row r at c ^ (r / 8 % 4 * 2 + r / 2 % 2)
+  const int chkA = ((tid & 7) ^ ((tid >> 4) & 7)) * 8, chkW = ((tid & 7) ^ ((tid >> 6 & 3) * 2 + (tid >> 4 & 1))) * 8;
+  uint32_t voA[2][2], voW[2][2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      // (R1 < 4: the rest of unit A1 lies past the resource's end, no memory request)
+      voA[h][i] = h == 0 || (tid >> 3) < 16 * R1 ? (uint32_t)(((i * BMH + h * 64 + (tid >> 3)) * p.lda + chkA) * 2) : 0x60000000u;
+      voW[h][i] = (uint32_t)((((2 * i + (tid >> 8)) * 64 + h * 32 + ((tid >> 3) & 31)) * p.K + chkW) * 2);
+    }
+  const int dst_lane0 = wid * 64 * 16;  // wave-uniform LDS destination of instruction 0 inside a unit
+  // operand reads: A tile i holds rows 16 i + r16; W tile h holds rows 8 (r16 / 4) + 4 h + r16 % 4, so that a lane's
+  // accumulators of the pair h = 0, 1 are the eight consecutive columns 8 q .. of output row r16
+  const int pos = (q ^ (r16 >> 1)) << 4;  // of K entries 0 .. 31; 32 .. 63 lie at pos ^ 64
+  const int offA = (wr * 64 + r16) * 128, offW = (wc * 32 + 8 * (r16 >> 2) + (r16 & 3)) * 128;
+
+  // the K tile that is being staged, of an item that may be ahead of the one being multiplied: rows past M / N fall outside
+  // num_records and load as zeros (their outputs are not stored); behind the last K tile nothing is asked for
+  Item ahead{sk_e, 0, 0, 0, 0};
+  const bf16_t *srcA = nullptr, *srcW = nullptr;
+  int numA = 0, numW = 0, kt = -1;
+  auto advance = [&] {
+    kt = uni(kt + 1);
+    if (kt < ahead.khi) return;
+    numA = numW = 0;
+    if (!next(ahead)) return;
     int tm, tn;
-    tile_mn(p, tile, tm, tn);
-    const int m0 = tm * 2 * BMH, n0 = tn * 256;
-    // Lane geometry is re-derived per item from an opaque copy of threadIdx.x: hoisted out of the
-    // item loop, the ~100 epilogue / fragment addresses it feeds would stay live and spill.
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));
-    const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r16 = lane & 15, q = lane >> 4;
-    const int wr = wid >> 2, wc = wid & 3;
-
-    // per-thread DMA geometry (byte offsets from the tile's buffer base): unit u, instruction i -> unit row
-    // ru = i*64 + tid/8 at LDS chunk tid%8, which holds global chunk chk of that row (swizzle on the source)
-    const int chk = ((tid & 7) ^ ((tid >> 4) & 7)) * 8;
-    uint32_t voA[2][2], voW[2][2];
+    tile_mn(p, ahead.tile, tm, tn);
+    const int m0 = uni(tm) * 2 * BMH, n0 = uni(tn) * 256;
+    srcA = p.A + (size_t)m0 * p.lda;
+    srcW = p.W + (size_t)n0 * p.K;
+    numA = min(p.M - m0, 2 * BMH) * p.lda * 2;
+    numW = min(p.N - n0, 256) * p.K * 2;
+    kt = uni(ahead.klo);
+  };
+  auto stage = [&](int u, uint8_t* buf) {
+    const __amdgpu_buffer_rsrc_t r = u < 2 ? uniform_rsrc(srcA, numA) : uniform_rsrc(srcW, numW);
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        // (R1 < 4: the rest of unit A1 lies past the resource's end, no memory request)
-        voA[h][i] = h == 0 || (tid >> 3) < 16 * R1 ? (uint32_t)(((i * BMH + h * 64 + (tid >> 3)) * p.lda + chk) * 2) : 0x60000000u;
-        voW[h][i] = (uint32_t)((((2 * i + (tid >> 8)) * 64 + h * 32 + ((tid >> 3) & 31)) * p.K + chk) * 2);
-      }
-    const int dst_lane0 = wid * 64 * 16;  // wave-uniform LDS destination of instruction 0 inside a unit
-    const int sw = (r16 >> 1) & 7;
-    const int off0 = r16 * 128 + ((q ^ sw) << 4), off1 = r16 * 128 + (((4 + q) ^ sw) << 4);
+    for (int i = 0; i < 2; ++i) {
+      auto* dst = (__attribute__((address_space(3))) void*)(buf + u * kUnitB + i * 512 * 16 + dst_lane0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, u < 2 ? voA[u][i] : voW[u - 2][i], kt * 128, 0, 0);
+    }
+  };
 
-    // buffer descriptors of the tile's A rows / W rows: rows past M / N fall outside num_records and
-    // load as zeros (their outputs are not stored)
-    const __amdgpu_buffer_rsrc_t rA = uniform_rsrc(p.A + (size_t)m0 * p.lda, min(p.M - m0, 2 * BMH) * p.lda * 2);
-    const __amdgpu_buffer_rsrc_t rW = uniform_rsrc(p.W + (size_t)n0 * p.K, min(p.N - n0, 256) * p.K * 2);
-    auto stage = [&](int u, uint8_t* buf, int kt) {
+  // acc[i][jj]: 16 rows (tile i) x columns 32 (jj / 2) + 8 q + 4 (jj % 2) .. of the wave's 128 x 64, row r16 of the tile.
+  // (The 32x32x16 MFMA with the same units and phases measured ~10 % slower on every shape.)
+  float4v acc[4 + R1][4];
+  uint4v a[4][2], b[4][2];
+  auto mma = [&](auto n, int i0) {
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        auto* dst = (__attribute__((address_space(3))) void*)(buf + u * kUnitB + i * 512 * 16 + dst_lane0);
-        if (u < 2)
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, dst, 16, voA[u][i], kt * 128, 0, 0);
-        else
-          __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, dst, 16, voW[u - 2][i], kt * 128, 0, 0);
-      }
-    };
-    auto rd = [&](const uint8_t* u, int row0, uint4v& f0, uint4v& f1) {
-      f0 = *reinterpret_cast<const uint4v*>(u + row0 * 128 + off0);
-      f1 = *reinterpret_cast<const uint4v*>(u + row0 * 128 + off1);
-    };
+    for (int s = 0; s < 2; ++s)
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+        for (int i = 0; i < decltype(n)::value; ++i) acc[i0 + i][jj] = mfma(b[jj][s], a[i][s], acc[i0 + i][jj]);
+  };
+  auto rdA = [&](const uint8_t* unit, auto n) {
+#pragma unroll
+    for (int i = 0; i < decltype(n)::value; ++i) {
+      a[i][0] = *reinterpret_cast<const uint4v*>(unit + offA + pos + i * 2048);
+      a[i][1] = *reinterpret_cast<const uint4v*>(unit + offA + (pos ^ 64) + i * 2048);
+    }
+  };
+  auto rdB = [&](const uint8_t* unit, int j0) {
+#pragma unroll
+    for (int jj = 0; jj < 2; ++jj) {
+      b[j0 + jj][0] = *reinterpret_cast<const uint4v*>(unit + offW + pos + jj * 512);
+      b[j0 + jj][1] = *reinterpret_cast<const uint4v*>(unit + offW + (pos ^ 64) + jj * 512);
+    }
+  };
+  constexpr std::integral_constant<int, 4> n4{};
+  constexpr std::integral_constant<int, R1> n1{};
 
-    // acc[i][jj] = 16 x 16 tile (i, jj) of the wave's 128 x 64 (lane: rows 4q..4q+3 of column r16).
-    // (The 32x32x16 MFMA with the same units and phases measured ~10 % slower on every shape.)
-    float4v acc[4 + R1][4];
+#define G8_BAR() __builtin_amdgcn_s_barrier()
+#define G8_VM(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
+// (a wave comes to the barrier with its operands in registers: behind it their units may be filled anew)
+#define G8_MFMA(n, i0)                               \
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); \
+  G8_BAR();                                          \
+  __builtin_amdgcn_s_setprio(1);                     \
+  mma(n, i0);                                        \
+  __builtin_amdgcn_s_setprio(0);                     \
+  G8_BAR()
+
+  advance();
+  stage(0, smem), stage(2, smem), stage(3, smem), stage(1, smem);
+  advance();
+  stage(0, smem + kBufB), stage(2, smem + kBufB), stage(3, smem + kBufB);
+  G8_VM(8);
+  G8_BAR();
+  if (wr == 1) G8_BAR();  // stagger the two wave rows by one barrier
+  int at = 0;           // LDS buffer of the K tile at hand
+  bool stored = false;  // an epilogue's stores have gone out after unit B1 of the next K tile
+  uint4v bias[2];
+
+  for (Item cur{sk_e, 0, 0, 0, 0}; next(cur);) {
 #pragma unroll
     for (int i = 0; i < 4 + R1; ++i)
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) acc[i][jj] = float4v{0.f, 0.f, 0.f, 0.f};
+    int tm, tn;
+    tile_mn(p, cur.tile, tm, tn);
+    const int m0 = uni(tm) * 2 * BMH, n0 = uni(tn) * 256;
 
-    uint4v a[4][2], b0[2][2], b1[2][2];
-    auto mma = [&](int i0, int j0, const uint4v (&bb)[2][2]) {
+    int left = cur.khi - cur.klo;  // (at least one)
+    do {
+      uint8_t* cb = smem + at;
+      at ^= kBufB;
+      uint8_t* nb = smem + at;
+      if constexpr (kBias) {
+        if (left == 1) {
+          const int col = n0 + wc * 64 + 8 * q;
+          const __amdgpu_buffer_rsrc_t rb = uniform_rsrc(p.R, p.N * 2);
 #pragma unroll
-      for (int s = 0; s < 2; ++s)
-#pragma unroll
-        for (int i = 0; i < (i0 == 0 ? 4 : R1); ++i)
-#pragma unroll
-          for (int jj = 0; jj < 2; ++jj) acc[i0 + i][j0 + jj] = mfma(a[i][s], bb[jj][s], acc[i0 + i][j0 + jj]);
-    };
-    auto rdA = [&](const uint8_t* buf, int u) {
-#pragma unroll
-      for (int i = 0; i < (u == kUA0 ? 4 : R1); ++i) rd(buf + u, wr * 64 + i * 16, a[i][0], a[i][1]);
-    };
-    auto rdB = [&](const uint8_t* buf, int u, uint4v (&bb)[2][2]) {
-#pragma unroll
-      for (int jj = 0; jj < 2; ++jj) rd(buf + u, wc * 32 + jj * 16, bb[jj][0], bb[jj][1]);
-    };
-
-#define G8_BAR() __builtin_amdgcn_s_barrier()
-#define G8_MFMA(i0, j0, bb)                          \
-  G8_BAR();                                          \
-  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); \
-  __builtin_amdgcn_s_setprio(1);                     \
-  mma(i0, j0, bb);                                   \
-  __builtin_amdgcn_s_setprio(0);                     \
-  G8_BAR()
-
-    const int nt = khi - klo;  // K tiles of this item; tile r lives in LDS buffer r & 1
-#define G8_STAGE(U, R) stage(U, smem + ((R) & 1) * kBufB, klo + (R))
-#define G8_VM(N) asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory")
-#define G8_TILE(R, ST1, ST2, ST3, ST4, W1, W2, W4) \
-  {                                                \
-    uint8_t* cb = smem + ((R) & 1) * kBufB;        \
-    rdB(cb, kUB0, b0);                             \
-    __builtin_amdgcn_sched_barrier(0);             \
-    rdA(cb, kUA0);                                 \
-    ST1;                                           \
-    W1;                                            \
-    G8_MFMA(0, 0, b0);                             \
-    rdB(cb, kUB1, b1);                             \
-    ST2;                                           \
-    W2;                                            \
-    G8_MFMA(0, 2, b1);                             \
-    rdA(cb, kUA1);                                 \
-    ST3;                                           \
-    G8_MFMA(4, 2, b1);                             \
-    ST4;                                           \
-    W4;                                            \
-    G8_MFMA(4, 0, b0);                             \
-  }
-    // unit issue runs 4 units ahead of consumption: tile r stages tile r+1 (A0 B0 B1 A1 in P1..P4), 2 units
-    // in flight at each wait.  (A 6-unit lead — B1, A1 of r+1 and A0, B0 of r+2, vmcnt(8) — measured the
-    // same at 4096^3 and on the decode shapes: the DMA latency is covered, the cost is in the barriers.)
-    G8_STAGE(0, 0); G8_STAGE(2, 0); G8_STAGE(3, 0); G8_STAGE(1, 0);
-    G8_VM(4);
-    G8_BAR();
-    if (wr == 1) G8_BAR();  // stagger the two wave rows by one barrier
-    int r = 0;
-    for (; r < nt - 1; ++r)
-      G8_TILE(r, G8_STAGE(0, r + 1), G8_STAGE(2, r + 1), G8_STAGE(3, r + 1), G8_STAGE(1, r + 1), G8_VM(4), G8_VM(4),
-              G8_VM(4))
-    G8_TILE(r, , , , , G8_VM(2), G8_VM(0), )
-#undef G8_TILE
-#undef G8_VM
-#undef G8_STAGE
-    if (wr == 0) G8_BAR();  // re-align the wave rows
-#undef G8_MFMA
-#undef G8_BAR
-
-    // ---- stream-K hand-off ----
-    if (khi < KT) {  // contributor: publish the fp32 partial, no store of C
-      float4v* wsp = reinterpret_cast<float4v*>(p.ws + (size_t)blockIdx.x * kPartialF);
-#pragma unroll
-      for (int i = 0; i < 4 + R1; ++i)
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) wsp[(wid * 32 + i * 4 + jj) * 64 + lane] = acc[i][jj];
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      __syncthreads();
-      if (tid == 0) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __hip_atomic_store(p.flags + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      }
-      continue;  // the next item's prologue only touches LDS after this item's last barrier
-    }
-    if (klo > 0) {  // finaliser: add the partials of the lower workgroups of this XCD covering [0, klo)
-      const int tile_begin = tile * KT;
-      for (int jp = j - 1; jp >= 0; --jp) {
-        int pa, pe;
-        sk_range(p, xcd, jp, pa, pe);
-        if (pe <= tile_begin) break;
-        if (pa == pe) continue;  // empty range: no partial
-        const int blk = jp * 8 + xcd;
-        if (tid == 0) {
-          while (__hip_atomic_load(p.flags + blk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-            __builtin_amdgcn_s_sleep(1);
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          __hip_atomic_store(p.flags + blk, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          for (int h = 0; h < 2; ++h) bias[h] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rb, (col + 32 * h) * 2, 0, 0));
         }
-        __syncthreads();
-        // four loads at a time: with eight the 256-row tile spills 37 to 41 registers instead of 16 to 19 (9000 x 4096 x 1024 115 ->
-        // 124 us, 4096 x 28672 x 4096 695 -> 723), the 224-row one 12 instead of none
-        const float4v* wsq = reinterpret_cast<const float4v*>(p.ws + (size_t)blk * kPartialF);
-#pragma unroll
-        for (int i = 0; i < 4 + R1; ++i) {
-#pragma unroll
-          for (int jj = 0; jj < 4; ++jj) acc[i][jj] += wsq[(wid * 32 + i * 4 + jj) * 64 + lane];
-          __builtin_amdgcn_sched_barrier(0);
-        }
-        if (pa <= tile_begin) break;
       }
-    }
+      rdB(cb + kUB0, 0);
+      rdB(cb + kUB1, 2);
+      rdA(cb + kUA0, n4);
+      stage(1, nb);
+      if (stored) G8_VM(8 + kStores);
+      else G8_VM(8);
+      G8_MFMA(n4, 0);
+      advance();
+      rdA(cb + kUA1, n1);
+      stage(0, cb), stage(2, cb), stage(3, cb);
+      if (stored) G8_VM(8 + kStores);
+      else G8_VM(8);
+      G8_MFMA(n1, 4);
+      stored = false;
+    } while (--left > 0);
 
-    __syncthreads();  // every wave is done reading the K buffers: LDS is reused by the epilogue
-
-    // ---- epilogue: per wave 128 rows x CW bf16 columns through LDS, then 16 B stores ----
-    constexpr int CW = EPI == EPI_SWIGLU ? 32 : 64;
-    constexpr int NJ = CW / 16;
-    if constexpr (EPI == EPI_SWIGLU) {
-#pragma unroll
-      for (int i = 0; i < 4 + R1; ++i)
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc[i][jj][r] = silu(acc[i][jj][r]) * acc[i][jj + 2][r];
-    }
-    if constexpr (EPI == EPI_BIAS || EPI == EPI_BIAS_GELU) {
-      // bias (+ exact erf GELU) on the fp32 accumulators, before the one bf16 rounding: the encoder's
-      // FFN1 needs no separate bias_gelu pass over [M, ffn]
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) {
-        const int col = n0 + wc * 64 + jj * 16 + r16;
-        const float bv = col < p.N ? bf2f(p.R[col]) : 0.f;
+    // (an opaque copy of the lane: what follows is computed here, not ahead of the loop, where it would cost it registers)
+    int el = lane, ew = wid;
+    asm volatile("" : "+v"(el), "+s"(ew));
+    // ---- stream-K hand-off (the wave rows meet for it and part again) ----
+    const bool whole = cur.khi == KT;
+    if (!whole || cur.klo > 0) {
+      if (wr == 0) G8_BAR();
+      if (!whole) {  // contributor: publish the fp32 partial, no store of C
+        const __amdgpu_buffer_rsrc_t rp = uniform_rsrc(p.ws + (size_t)blockIdx.x * kPartialF, kPartialF * 4);
 #pragma unroll
         for (int i = 0; i < 4 + R1; ++i)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float y = acc[i][jj][r] + bv;
-            acc[i][jj][r] = EPI == EPI_BIAS_GELU ? gelu_erf(y) : y;
+          for (int jj = 0; jj < 4; ++jj)
+            __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4v, acc[i][jj]), rp, (ew * 2048 + el) * 16, (i * 4 + jj) * 1024, kSC1);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid == 0) __hip_atomic_store(p.flags + blockIdx.x, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      } else {  // finaliser: add the partials of the lower workgroups of this XCD covering [0, klo)
+        const int tile_begin = cur.tile * KT;
+        for (int jp = j - 1; jp >= 0; --jp) {
+          int pa, pe;
+          sk_range(p, xcd, jp, pa, pe);
+          if (pe <= tile_begin) break;
+          if (pa == pe) continue;  // empty range: no partial
+          const int blk = jp * 8 + xcd;
+          if (tid == 0) {
+            while (__hip_atomic_load(p.flags + blk, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
+              __builtin_amdgcn_s_sleep(1);
+            __hip_atomic_store(p.flags + blk, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           }
+          __syncthreads();
+          const __amdgpu_buffer_rsrc_t rp = uniform_rsrc(p.ws + (size_t)blk * kPartialF, kPartialF * 4);
+#pragma unroll
+          for (int i = 0; i < 4 + R1; i += 2) {
+            float4v part[2][4];
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              if (i + k / 4 < 4 + R1)
+                part[k / 4][k % 4] = __builtin_bit_cast(float4v, __builtin_amdgcn_raw_buffer_load_b128(rp, (ew * 2048 + el) * 16, (i * 4 + k) * 1024, kSC1));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+              if (i + k / 4 < 4 + R1) acc[i + k / 4][k % 4] += part[k / 4][k % 4];
+            __builtin_amdgcn_sched_barrier(0);
+          }
+          if (pa <= tile_begin) break;
+        }
       }
+      if (wr == 1) G8_BAR();
     }
-    bf16_t* ot = reinterpret_cast<bf16_t*>(smem) + wid * 128 * CW;
+
+    // ---- epilogue: a lane holds eight consecutive columns of a row, so its 16 bytes go out from the registers.  Stores past M or
+    // N fall outside the resource: the number of store instructions, which the waits above count, is always the same ----
+    if (whole) {
+      const int ncols = EPI == EPI_SWIGLU ? p.N / 2 : p.N;
+      const int ncol0 = EPI == EPI_SWIGLU ? n0 / 2 + wc * 32 : n0 + wc * 64, row0 = m0 + wr * BMH;
+      const int cols_here = max(0, min(ncols - ncol0, CW));
+      uint32_t vo[NH];
 #pragma unroll
-    for (int i = 0; i < 4 + R1; ++i)
+      for (int h = 0; h < NH; ++h) {
+        const int col = 32 * h + 8 * (el >> 4);
+        vo[h] = col < cols_here ? (uint32_t)(((el & 15) * p.ldc + col) * 2) : 0xfffffff0u;
+      }
+      auto rows_of = [&](const bf16_t* base, int i) {
+        const int rows = cols_here == 0 ? 0 : min(p.M - row0 - 16 * i, 16);
+        return uniform_rsrc(base + (size_t)(row0 + 16 * i) * p.ldc + ncol0, rows > 0 ? ((rows - 1) * p.ldc + cols_here) * 2 : 0);
+      };
+      // the residual of all rows is asked for before the first store, behind which it would have to wait for it
+      uint4v rv[EPI == EPI_RESIDUAL ? 4 + R1 : 1][NH];
+      if constexpr (EPI == EPI_RESIDUAL) {
 #pragma unroll
-      for (int jj = 0; jj < NJ; ++jj)
+        for (int i = 0; i < 4 + R1; ++i) {
+          const __amdgpu_buffer_rsrc_t rr = rows_of(p.R, i);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = i * 16 + 4 * q + r, col = jj * 16 + r16;
-          ot[row * CW + (col ^ (((row & 7) << 3) % CW))] = f2bf(acc[i][jj][r]);
+          for (int h = 0; h < NH; ++h) rv[i][h] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rr, vo[h], 0, 0));
         }
-    __syncthreads();
-    constexpr int CPR = CW / 8;    // 16 B chunks per row
-    constexpr int RPI = 64 / CPR;  // rows per store instruction
-    const int cch = lane % CPR;
-    const int ncol0 = EPI == EPI_SWIGLU ? n0 / 2 + wc * 32 : n0 + wc * 64;
-    const int ncols = EPI == EPI_SWIGLU ? p.N / 2 : p.N;
-    if constexpr (EPI == EPI_RESIDUAL) {
-      // residual rows through a buffer resource (rows past M read zeros, no request), all of a group's loads
-      // in flight before the first add — inside the store's bounds branch each 16 B load waited its own
-      // HBM round trip
-      const int row0 = m0 + wr * BMH;
-      const int rows_here = max(0, min(p.M - row0, BMH));
-      const __amdgpu_buffer_rsrc_t rR = uniform_rsrc(p.R + (size_t)row0 * p.ldc, rows_here * p.ldc * 2);
-      const int gn = ncol0 + cch * 8;
-      constexpr int kIt = BMH / RPI, kGrp = kIt < 16 ? kIt : 16;
-      static_assert(kIt % kGrp == 0, "residual epilogue groups must tile the wave's rows");
-#pragma unroll 1
-      for (int k0 = 0; k0 < kIt; k0 += kGrp) {
-        uint4v rv[kGrp];
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      auto store = [&](auto policy) {
 #pragma unroll
-        for (int u = 0; u < kGrp; ++u) {
-          const int row = lane / CPR + RPI * (k0 + u);
-          rv[u] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rR, (row * p.ldc + gn) * 2, 0, 0));
-        }
+      for (int i = 0; i < 4 + R1; ++i) {
+        const __amdgpu_buffer_rsrc_t rc = rows_of(p.C, i);
 #pragma unroll
-        for (int u = 0; u < kGrp; ++u) {
-          const int row = lane / CPR + RPI * (k0 + u);
+        for (int h = 0; h < NH; ++h) {
           float x[8], y[8];
-          unpack8(*reinterpret_cast<const uint4v*>(ot + row * CW + ((cch * 8) ^ (((row & 7) << 3) % CW))), x);
-          unpack8(rv[u], y);
+          if constexpr (kBias) unpack8(bias[h], y);
+          if constexpr (EPI == EPI_RESIDUAL) unpack8(rv[i][h], y);
 #pragma unroll
-          for (int e = 0; e < 8; ++e) x[e] += y[e];
-          if (row0 + row < p.M && gn < ncols) *reinterpret_cast<uint4v*>(p.C + (size_t)(row0 + row) * p.ldc + gn) = pack8(x);
+          for (int e = 0; e < 8; ++e) {
+            x[e] = acc[i][2 * h + e / 4][e % 4];
+            if constexpr (EPI == EPI_SWIGLU) x[e] = silu(x[e]) * acc[i][2 + e / 4][e % 4];
+            if constexpr (kBias || EPI == EPI_RESIDUAL) x[e] += y[e];
+            if constexpr (EPI == EPI_BIAS_GELU) x[e] = gelu_erf(x[e]);
+          }
+          __builtin_amdgcn_raw_buffer_store_b128(pack8(x), rc, vo[h], 0, decltype(policy)::value);
         }
       }
-    } else {
-#pragma unroll 4
-      for (int k = 0; k < BMH / RPI; ++k) {
-        const int row = lane / CPR + RPI * k;
-        const int gm = m0 + wr * BMH + row;
-        const int gn = ncol0 + cch * 8;
-        if (gm < p.M && gn < ncols)
-          *reinterpret_cast<uint4v*>(p.C + (size_t)gm * p.ldc + gn) =
-              *reinterpret_cast<const uint4v*>(ot + row * CW + ((cch * 8) ^ (((row & 7) << 3) % CW)));
-      }
+      };
+      if (p.nt) store(std::integral_constant<int, kNT>{});
+      else store(std::integral_constant<int, 0>{});
+      stored = true;
     }
-    __syncthreads();  // LDS free for the next item's prologue
   }
+  if (wr == 0) G8_BAR();  // re-align the wave rows
+  G8_VM(0);               // the last K tile's requests have ended before the LDS is given back
+#undef G8_MFMA
+#undef G8_VM
+#undef G8_BAR
 }
 
 template <int EPI, int R1>
@@ -432,20 +446,35 @@ int grid_wpx(int tiles, int KT) {
   return iters < 8LL * 8 * wpx ? (int)std::max(1LL, iters / 64) : wpx;
 }
 
-// The row tile (R1: 256, 224 or 192 rows).  256 rows are 1.56 us per K iteration and round, 224 0.89 and 192 0.83 of that
-// (28672 x 4096 and 4096 x 14336, whole rounds of tiles), so a smaller one pays where it saves rows past M: 1095 rows are five
-// tiles either way.  To it comes the hand-off of the tiles cut between workgroups (256 KiB through one compute unit each way):
-// over whole rounds 10 us and 45 times the last round's share, with fewer tiles than workgroups 15 us a part, 10 if all are cut
-// evenly.  The rule's choice, us, against 256 rows: gate|up 28672 x 4096 of 520 / 1095 / 1300 / 3333 rows 137 / 222 / 274 / 615
-// for 163 / 238 / 304 / 624, down 4096 x 14336 of 520 / 1095 / 1300 / 2200 rows 97 / 137 / 147 / 221 for 112 / 165 / 159 / 238.
+// What is lost beside the K iterations of `tiles` tiles on G workgroups, us (iter: one of a tile's KT): the tiles of a last
+// round that is not full are cut between all workgroups, or (cut: false) run as they are while the others idle (and the rest run
+// at a higher clock: three quarters of the idle time), whichever is less.  A cut costs its hand-off, 256 KiB through one compute
+// unit each way, and workgroups that walk K apart no longer share their rows' way through an XCD's L2.  Cut less uncut, us, by how
+// full the last round is: K 768 0.05 / 0.38 / 0.75 / 0.89 -3 / +3 / +9 / +10; K 2048 0.06 / 0.5 / 0.88 -18 / -7 / +29; K 4096 -46 /
+// -16 / +50; K 8192 -99 / -34 / +81; K 14336 0.25 / 0.88 -129 / +123; K 384 0.05 / 0.89 +2 / +8.  With fewer tiles than workgroups,
+// down 4096 x 14336 of 520 / 1095 / 1300 / 2200 / 3333 rows (5.3 / 3.2 / 2.7 / 1.8 / 1.1 workgroups a tile) lost 31 / 23 / 15 / 34 / 5.
+double rest_cost(int tiles, int G, int KT, double iter, bool* cut) {
+  const int rest = tiles % G;
+  const double full = (double)rest / G, idle = rest == 0 ? 0 : 0.75 * iter * KT * (1 - full);
+  const double split = rest == 0 ? 0 : tiles > G ? 6 + KT * (0.2 + 0.7 * std::max(0.0, full - 0.3))
+                                     : G % tiles == 0 ? 4.5 * G / tiles : 3 + 6.5 * G / tiles;
+  *cut = rest != 0 && split < idle;
+  return std::min(split, idle);
+}
+
+// The row tile (R1: 256, 224 or 192 rows).  256 rows are 1.45 us per K iteration and round, 224 0.93 and 192 0.85 of that
+// (28672 x 4096 and 4096 x 14336, whole rounds of tiles), so a smaller one pays where it saves rows past M (1095 rows are five
+// tiles either way) or fills the last round.  Measured, us, 256 / 224 / 192 rows: gate|up 28672 x 4096 of 520 / 1095 / 1700 / 3333 rows
+// 130 / 128 / 122, 207 / 203 / 243, 291 / 304 / 347, 555 / 585 / 662; down 4096 x 14336 of 900 / 1095 / 2200 rows 101 / 114 / 114,
+// 124 / 121 / 116, 216 / 207 / 215.
+constexpr double kIter[5] = {0, 0, 1.45 * 0.85, 1.45 * 0.93, 1.45};
 int row_tile(int M, int tiles_n, int KT) {
-  constexpr double kIter = 1.56, kCost[5] = {0, 0, 0.83, 0.89, 1.0};
   int best = 4;
   double least = 0;
   for (int r1 = 4; r1 >= 2; --r1) {
-    const int bm = 128 + 32 * r1, tiles = (M + bm - 1) / bm * tiles_n, G = 8 * grid_wpx(tiles, KT), rest = tiles % G;
-    const double cut = rest == 0 ? 0 : tiles > G ? 10 + 45.0 * rest / G : G % tiles == 0 ? 10 : 15.0 * G / tiles;
-    const double us = kCost[r1] * kIter * KT * tiles / G + cut;
+    bool cut;
+    const int bm = 128 + 32 * r1, tiles = (M + bm - 1) / bm * tiles_n, G = 8 * grid_wpx(tiles, KT);
+    const double us = kIter[r1] * KT * tiles / G + rest_cost(tiles, G, KT, kIter[r1], &cut);
     if (r1 == 4 || us < least) best = r1, least = us;
   }
   return best;
@@ -465,19 +494,18 @@ extern "C" int lwc_gemm8p(const void* A, const void* W, void* C, const void* R, 
                           int K, int lda, int ldc, int epi, hipStream_t s) {
   using namespace lwc::g8p;
   if (K % 64 != 0 || K < 64 || N % 8 != 0 || lda % 8 != 0 || ldc % 8 != 0) return -1;
-  if ((long long)M * lda * 2 >= (1LL << 31) || 256LL * K * 2 >= (1LL << 31)) return -1;  // 32-bit buffer offsets
+  if ((long long)M * lda * 2 >= (1LL << 31) || 256LL * K * 2 >= (1LL << 31) || ldc >= (1 << 26)) return -1;  // 32-bit buffer offsets
   if (epi == EPI_SWIGLU && N % 64 != 0) return -1;
   if ((epi == EPI_RESIDUAL || epi == EPI_BIAS || epi == EPI_BIAS_GELU) && R == nullptr) return -1;
   if (M == 0 || N == 0) return 0;
   const int tiles_n = (N + 255) / 256, KT = K / 64, r1 = lda < (1 << 20) ? row_tile(M, tiles_n, KT) : 4;
   const int bm = 128 + 32 * r1, tiles_m = (M + bm - 1) / bm, tiles = tiles_m * tiles_n, wpx = grid_wpx(tiles, KT), G = 8 * wpx;
-  int sk = 0, dp = tiles / G;
-  if (tiles % G != 0) {
-    dp = std::max(0, tiles / G - 1);
-    sk = tiles - dp * G;
-  }
+  bool cut;
+  rest_cost(tiles, G, KT, kIter[r1], &cut);
+  const int dp = cut ? std::max(0, tiles / G - 1) : (tiles + G - 1) / G, sk = cut ? tiles - dp * G : 0;
   Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, ws, flags,
-           M, N, K, lda, ldc, tiles_m, tiles_n, KT, std::max(1, env_int("LWC_G8_GM", 8)), wpx, sk, dp};
+           M, N, K, lda, ldc, tiles_m, tiles_n, KT, std::max(1, env_int("LWC_G8_GM", 8)), wpx, sk, dp,
+           (long long)M * N * (epi == EPI_SWIGLU ? 1 : 2) > 256LL << 20};
   switch (epi) {
     case EPI_PLAIN: return launch<EPI_PLAIN>(p, r1, s);
     case EPI_RESIDUAL: return launch<EPI_RESIDUAL>(p, r1, s);

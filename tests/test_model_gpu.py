@@ -130,6 +130,26 @@ def test_engine_export_import_prefill_equivalence(tiny, gpu):
     assert b.bm.num_free == 256
 
 
+@pytest.mark.parametrize("fused", ["0", "ffn2", "all"])
+def test_encoder_layers_on_gemm8p_launched_natively(gpu, monkeypatch, fused):
+    """Projections on gemm8p are launched from native code too, over the stream's workspace: the loop's bits."""
+    from llm_weighted_consensus_amd import ops
+    from llm_weighted_consensus_amd.models.bert import BertEncoder
+    from llm_weighted_consensus_amd.models.config import encoder_config
+    from llm_weighted_consensus_amd.ops import gemm_plan
+
+    m = BertEncoder(encoder_config("bge-small-en-v1.5"), device=gpu, seed=5)
+    m.fused_residual = fused
+    args = m.pack([[(7 * i + j) % 900 + 1 for j in range(n)] for i, n in enumerate([300, 2, 64, 129])])
+    monkeypatch.setattr(gemm_plan, "MODE", "g8")
+    taken, native = [], ops.encoder_layers
+    monkeypatch.setattr(ops, "encoder_layers", lambda *a: taken.append(native(*a)) or taken[-1])
+    y = m.forward_packed(*args)
+    assert len(taken) == 1 and taken[0] is not None
+    monkeypatch.setattr(ops, "encoder_layers", lambda *a: None)
+    assert torch.equal(y, m.forward_packed(*args))
+
+
 @pytest.mark.parametrize("core,lens", [("gv", [5, 1, 40]), ("g2", [5, 1, 40]), ("g2", [300, 2, 64, 129])])
 @pytest.mark.parametrize("fused", ["0", "ffn2", "all"])
 def test_encoder_layers_launched_natively(gpu, monkeypatch, core, lens, fused):
