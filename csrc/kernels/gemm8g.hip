@@ -1,4 +1,4 @@
-// K6g' grouped GEMM on the 8-phase 256x256 schedule (the MoE expert FFNs), fp8 and bf16:
+// K6g' grouped GEMM in the 256x256 tiles of gemm8p.hip (the MoE expert FFNs), fp8 and bf16:
 //   C[r, :] = (A[a_rows[r], :] . W_g^T) * a_scale[a_rows[r]] * w_scale[g, :]   for rows r of group g
 // with groups = the experts' contiguous row segments row_off[g]..row_off[g+1] (device table, no host
 // sync, graph-capturable) and A gathered through a_rows (MoE dispatch without a permute copy).
@@ -6,28 +6,29 @@
 // Why a second grouped kernel: the 128x128 register-staged kernel (gemm.hip) pays two barriers and a
 // full LDS rewrite per 128-byte K step for 16 block-scaled MFMAs per wave — latency-bound at ~1.0-1.3
 // PF/s fp8 (profiles/moe_r32.md: MFMA busy ~20 %).  Large decode batches give every expert >= 2 full
-// 256-row tiles (T = 2048 tokens, top-2, 8 experts: 512 rows each), which is the dense 8-phase template's
-// regime (csrc/kernels/gemm8p.hip, cdna_hip_programming.md §5 "The 256² 8-phase template"):
+// 256-row tiles (T = 2048 tokens, top-2, 8 experts: 512 rows each), which is the dense tile's regime (gemm8p.hip):
 //   * 8 waves = 2 (M) x 4 (N), wave tile 128 x 64; K tile = 128 BYTES (= 128 e4m3), four 16 KiB LDS
 //     units A0 A1 B0 B1 per K tile, two K-tile buffers (128 KiB), LDS-DMA (buffer_load ... lds) staging
-//     with the swizzle on the SOURCE address, 4 phases per K tile with counted vmcnt, raw s_barrier and
-//     the two wave rows staggered by one barrier — byte for byte the gemm8p pipeline;
+//     with the swizzle on the SOURCE address, two phases per K tile with counted vmcnt, operands in registers at the
+//     raw s_barrier and the two wave rows staggered by one barrier — byte for byte the gemm8p pipeline;
 //   * MFMA: the block-scaled mfma_scale_f32_16x16x128_f8f6f4 with unit e8m0 scales: a lane's two 16 B
 //     fragments (k-chunks q and 4+q of the 128-byte slice) form one 32-byte operand, so a phase issues
-//     8 MFMAs of twice the bf16 cycle count — the same MFMA cycles per phase as gemm8p at 2x the FLOPs;
+//     16 MFMAs of twice the bf16 cycle count — the same MFMA cycles per phase as gemm8p at 2x the FLOPs;
 //   * A rows: per-lane DMA source offsets from a_rows (rows past the group's end load a valid row of
 //     the group and are masked at the store); W: the group's [N, K] slab through its own descriptor;
-//   * epilogue: fp32 accumulators x activation row scale x weight channel scale -> bf16 -> LDS -> 16 B
-//     row stores (rows < the group's end only).
+//   * epilogue: a lane holds eight consecutive columns of eight rows: eight activation scales and 16 channel scales
+//     instead of 32 and 4, no LDS, 16 B stores (rows < the group's end only).
+// Measured against four phases of half the MFMAs with the wait for their reads behind the barrier and an epilogue through LDS, us:
+// dense fp8 8682 rows x 28672 x 4096 SwiGLU 794 -> 751, x 4096 x 14336 468 -> 449; 8 bf16 experts of 4096 rows, [14336, 4096] 2931 ->
+// 2908, [4096, 7168] 1661 -> 1617 (bound by the card's power there).  64 documents through three e5 layers 4255 -> 4045.
 // Work distribution: one 256 x 256 tile per workgroup; workgroup ids are dealt round-robin to the 8
 // XCDs, and XCD x walks the n-tiles n = x (mod 8) with all m-tiles of an n-tile consecutive, so the
 // weight tile of an expert is read from HBM once per XCD and reused from its L2 by the expert's other
 // m-tiles.  Surplus slots (routing decides the m-tile count at run time) exit immediately.
 //
 // bf16 (kBf16 / kBf16Swiglu): the same bytes move through the same pipeline — a K tile of 128 bytes is 64 bf16, a
-// phase's 8 double-length fp8 MFMAs become 16 bf16 ones as in gemm8p — without scales.  Bound by the matrix cores:
-// 8 experts of 4096 rows, [14336, 4096] weights 2988 us (1.29 PF/s; the 128-row kernel 4720), [4096, 7168] 1481 us
-// (1.30 PF/s; 2376), one MI355X.
+// phase's 16 double-length fp8 MFMAs become 32 bf16 ones as in gemm8p — without scales.  Bound by the matrix cores (the
+// 128-row kernel 4720 and 2376 us at the experts above).
 #include "common.h"
 
 namespace lwc {
@@ -72,31 +73,17 @@ constexpr int kBf16 = 4;        // bf16 A and W, bf16 out
 constexpr int kBf16Swiglu = 5;  // bf16 A and W, SwiGLU epilogue, bf16 out
 constexpr int kMxLds = 4096;  // kMxA: the two K buffers' scale tiles (256 rows x 4 blocks, twice: see the DMA)
 
-// A block-scaled: the lane's e8m0 scale is byte OP of sa (its row's scale for the lane's K block)
-template <int OP>
-LWC_DEVICE float4v mfma8s(const uint4v& a0, const uint4v& a1, const uint4v& b0, const uint4v& b1, const float4v& c,
-                          int sa) {
+// sb: the lane's e8m0 scale of the second operand (its row's, for the lane's K block)
+LWC_DEVICE float4v mfma8(const uint4v& a0, const uint4v& a1, const uint4v& b0, const uint4v& b1, const float4v& c, int sb) {
   const v8i32 av = {(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w, (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
   const v8i32 bv = {(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w, (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, OP, sa, 0, 127);
-}
-
-// max over each quad of lanes
-LWC_DEVICE float quad_max(float x) {
-  x = fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0xB1, 0xF, 0xF, false)));  // ^1
-  return fmaxf(x, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), 0x4E, 0xF, 0xF, false)));  // ^2
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, 0, 127, 0, sb);
 }
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 LWC_DEVICE float4v mfma16(const uint4v& a, const uint4v& b, const float4v& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
                                                  0, 0);
-}
-
-LWC_DEVICE float4v mfma8(const uint4v& a0, const uint4v& a1, const uint4v& b0, const uint4v& b1, const float4v& c) {
-  const v8i32 av = {(int)a0.x, (int)a0.y, (int)a0.z, (int)a0.w, (int)a1.x, (int)a1.y, (int)a1.z, (int)a1.w};
-  const v8i32 bv = {(int)b0.x, (int)b0.y, (int)b0.z, (int)b0.w, (int)b1.x, (int)b1.y, (int)b1.z, (int)b1.w};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, 0, 127, 0, 127);
 }
 
 // grouped default: an XCD takes all of its n-tiles for one m-slot before the next slot (gn = n-tiles per XCD).
@@ -154,15 +141,14 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
   const int n0 = ntile * 256;
   const int KT = p.K / 128;
 
-  int tid = threadIdx.x;
-  asm volatile("" : "+v"(tid));
+  const int tid = threadIdx.x;
   const int lane = tid & 63, wid = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, q = lane >> 4;
   const int wr = wid >> 2, wc = wid & 3;
 
-  // per-thread DMA geometry: unit u, instruction i -> unit row ru = i*64 + tid/8 at LDS chunk tid%8, holding
-  // global chunk chk of that row (swizzle on the source).  A rows are gathered: source row of tile row t.
-  const int chk = ((tid & 7) ^ ((tid >> 4) & 7)) * 16;
+  // per-thread DMA geometry: unit u, instruction i -> unit row ru = i*64 + tid/8 at LDS chunk tid%8, holding a
+  // global chunk of that row (swizzle on the source, gemm8p.hip's).  A rows are gathered: source row of tile row t.
+  const int chkA = ((tid & 7) ^ ((tid >> 4) & 7)) * 16, chkW = ((tid & 7) ^ ((tid >> 6 & 3) * 2 + (tid >> 4 & 1))) * 16;
   uint32_t voA[2][2], voW[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
@@ -171,12 +157,12 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
       int r = m_begin + i * 128 + h * 64 + (tid >> 3);
       if (r >= m_end) r = m_begin;  // a valid row of the group; its outputs are never stored
       const int src = p.a_rows ? p.a_rows[r] : r;
-      voA[h][i] = (uint32_t)(src * p.lda + chk);
-      voW[h][i] = (uint32_t)(((2 * i + (tid >> 8)) * 64 + h * 32 + ((tid >> 3) & 31)) * p.K + chk);
+      voA[h][i] = (uint32_t)(src * p.lda + chkA);
+      voW[h][i] = (uint32_t)(((2 * i + (tid >> 8)) * 64 + h * 32 + ((tid >> 3) & 31)) * p.K + chkW);
     }
   const int dst_lane0 = wid * 64 * 16;
-  const int sw = (r16 >> 1) & 7;
-  const int off0 = r16 * 128 + ((q ^ sw) << 4), off1 = r16 * 128 + (((4 + q) ^ sw) << 4);
+  const int pos = (q ^ (r16 >> 1)) << 4;
+  const int offA = (wr * 64 + r16) * 128, offW = (wc * 32 + 8 * (r16 >> 2) + (r16 & 3)) * 128;
 
   // kMxA: the tile's scales ([row][4 blocks], one dword per row) DMA'd with unit A0, one dword piece per thread
   // (an LDS-DMA lands every lane's piece on a 4-byte slot, so no narrower piece packs): threads 256..511 load
@@ -187,227 +173,165 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
     if (r >= m_end) r = m_begin;
     voS = (uint32_t)(r * 4);
   }
-  const __amdgpu_buffer_rsrc_t rS = uniform_rsrc(p.a_mx, MXA ? (p.K / 128) * p.s_rows * 4 : 0);
-  const __amdgpu_buffer_rsrc_t rA = uniform_rsrc(p.A, p.rows_a * p.lda);
-  const __amdgpu_buffer_rsrc_t rW = uniform_rsrc(p.W + ((size_t)g * p.N + n0) * p.K, min(p.N - n0, 256) * p.K);
-  auto stage = [&](int u, uint8_t* buf, int kt) {
+  const int numA = p.rows_a * p.lda, numW = min(p.N - n0, 256) * p.K, numS = MXA ? (p.K / 128) * p.s_rows * 4 : 0;
+  const uint8_t* srcW = p.W + ((size_t)g * p.N + n0) * p.K;
+  // unit u of K tile kt; past the last one the same instructions without a memory request
+  auto stage = [&](int u, int kt) {
+    uint8_t* buf = smem + (kt & 1) * kBufB;
+    const bool live = kt < KT;
+    const __amdgpu_buffer_rsrc_t r = u < 2 ? uniform_rsrc(p.A, live ? numA : 0) : uniform_rsrc(srcW, live ? numW : 0);
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
       auto* dst = (__attribute__((address_space(3))) void*)(buf + u * kUnitB + i * 512 * 16 + dst_lane0);
-      if (u < 2)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rA, dst, 16, voA[u][i], kt * 128, 0, 0);
-      else
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rW, dst, 16, voW[u - 2][i], kt * 128, 0, 0);
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, u < 2 ? voA[u][i] : voW[u - 2][i], kt * 128, 0, 0);
     }
     if constexpr (MXA) {
       if (u == 0) {
         auto* dst = (__attribute__((address_space(3))) void*)(smem + kLdsB + (kt & 1) * 2048 + (wid >> 2) * 1024 +
                                                               (wid & 3) * 256);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rS, dst, 4, voS, kt * p.s_rows * 4, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(uniform_rsrc(p.a_mx, live ? numS : 0), dst, 4, voS, kt * p.s_rows * 4, 0, 0);
       }
     }
   };
-  auto rd = [&](const uint8_t* u, int row0, uint4v& f0, uint4v& f1) {
-    f0 = *reinterpret_cast<const uint4v*>(u + row0 * 128 + off0);
-    f1 = *reinterpret_cast<const uint4v*>(u + row0 * 128 + off1);
-  };
 
+  // acc[i][jj]: 16 rows (tile i) x columns 32 (jj / 2) + 8 q + 4 (jj % 2) .. of the wave's 128 x 64, row r16 of the tile
   float4v acc[8][4];
 #pragma unroll
   for (int i = 0; i < 8; ++i)
 #pragma unroll
     for (int jj = 0; jj < 4; ++jj) acc[i][jj] = float4v{0.f, 0.f, 0.f, 0.f};
 
-  uint4v a[4][2], b0[2][2], b1[2][2];
+  uint4v a[4][2], b[4][2];
   int sc[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // kMxA: this K tile's scale (block q) of the lane's 8 row fragments
-  auto mma = [&](int i0, int j0, const uint4v (&bb)[2][2]) {
+  auto mma = [&](int i0) {
     if constexpr (BF) {
 #pragma unroll
       for (int s = 0; s < 2; ++s)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
-          for (int jj = 0; jj < 2; ++jj) acc[i0 + i][j0 + jj] = mfma16(a[i][s], bb[jj][s], acc[i0 + i][j0 + jj]);
-    } else if constexpr (MXA) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-          acc[i0 + i][j0 + jj] = mfma8s<0>(a[i][0], a[i][1], bb[jj][0], bb[jj][1], acc[i0 + i][j0 + jj], sc[i0 + i]);
+          for (int i = 0; i < 4; ++i) acc[i0 + i][jj] = mfma16(b[jj][s], a[i][s], acc[i0 + i][jj]);
     } else {
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
-        for (int jj = 0; jj < 2; ++jj)
-          acc[i0 + i][j0 + jj] = mfma8(a[i][0], a[i][1], bb[jj][0], bb[jj][1], acc[i0 + i][j0 + jj]);
+        for (int i = 0; i < 4; ++i)
+          acc[i0 + i][jj] = mfma8(b[jj][0], b[jj][1], a[i][0], a[i][1], acc[i0 + i][jj], MXA ? sc[i0 + i] : 127);
     }
   };
-  auto rdA = [&](const uint8_t* buf, int u) {
+  auto rdA = [&](const uint8_t* unit) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) rd(buf + u, wr * 64 + i * 16, a[i][0], a[i][1]);
+    for (int i = 0; i < 4; ++i) {
+      a[i][0] = *reinterpret_cast<const uint4v*>(unit + offA + pos + i * 2048);
+      a[i][1] = *reinterpret_cast<const uint4v*>(unit + offA + (pos ^ 64) + i * 2048);
+    }
   };
-  auto rdB = [&](const uint8_t* buf, int u, uint4v (&bb)[2][2]) {
+  auto rdB = [&](const uint8_t* unit, int j0) {
 #pragma unroll
-    for (int jj = 0; jj < 2; ++jj) rd(buf + u, wc * 32 + jj * 16, bb[jj][0], bb[jj][1]);
+    for (int jj = 0; jj < 2; ++jj) {
+      b[j0 + jj][0] = *reinterpret_cast<const uint4v*>(unit + offW + pos + jj * 512);
+      b[j0 + jj][1] = *reinterpret_cast<const uint4v*>(unit + offW + (pos ^ 64) + jj * 512);
+    }
   };
 
 #define G8_BAR() __builtin_amdgcn_s_barrier()
+#define G8_VM(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
   // rows of this wave row that hold data (wave-uniform): a ragged last tile of an expert (on average half of
   // it) skips the MFMAs of its empty 64-row blocks — the barriers, LDS reads and DMA stay, so the two wave
   // rows keep their schedule
   const int live = p.skip_empty ? __builtin_amdgcn_readfirstlane(m_end - m_begin - wr * 128) : 256;
-#define G8_MFMA(i0, j0, bb)                          \
-  G8_BAR();                                          \
+#define G8_MFMA(i0)                                  \
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); \
+  G8_BAR();                                          \
   __builtin_amdgcn_s_setprio(1);                     \
-  if ((i0) * 16 < live) mma(i0, j0, bb);             \
+  if ((i0) * 16 < live) mma(i0);                     \
   __builtin_amdgcn_s_setprio(0);                     \
   G8_BAR()
-#define G8_STAGE(U, R) stage(U, smem + ((R) & 1) * kBufB, (R))
-#define G8_VM(N) asm volatile("s_waitcnt vmcnt(" #N ")" ::: "memory")
-  // kMxA stages 1 more piece with unit A0: the waits after A0 / B0 of the next tile leave 5 in flight, not 4
-#define G8_VMX() \
-  if constexpr (MXA) G8_VM(5); \
-  else G8_VM(4)
-#define G8_TILE(R, ST1, ST2, ST3, ST4, W1, W2, W4) \
-  {                                                \
-    uint8_t* cb = smem + ((R) & 1) * kBufB;        \
-    rdB(cb, kUB0, b0);                             \
-    __builtin_amdgcn_sched_barrier(0);             \
-    rdA(cb, kUA0);                                 \
-    if constexpr (MXA) {                           \
-      const uint8_t* st = smem + kLdsB + ((R) & 1) * 2048 + (wr * 128 + r16) * 4 + q; \
-      _Pragma("unroll") for (int i = 0; i < 8; ++i) sc[i] = st[i * 64]; \
-    }                                              \
-    ST1;                                           \
-    W1;                                            \
-    G8_MFMA(0, 0, b0);                             \
-    rdB(cb, kUB1, b1);                             \
-    ST2;                                           \
-    W2;                                            \
-    G8_MFMA(0, 2, b1);                             \
-    rdA(cb, kUA1);                                 \
-    ST3;                                           \
-    G8_MFMA(4, 2, b1);                             \
-    ST4;                                           \
-    W4;                                            \
-    G8_MFMA(4, 0, b0);                             \
-  }
-  // the same unit lead / vmcnt schedule as gemm8p: tile r stages tile r+1 (A0 B0 B1 A1 in P1..P4)
-  G8_STAGE(0, 0); G8_STAGE(2, 0); G8_STAGE(3, 0); G8_STAGE(1, 0);
-  G8_VM(4);
+  // gemm8p.hip's two phases per K tile: P1 reads B0, B1 and A0 of tile t and stages A1 of t + 1, P2 reads A1 and stages A0
+  // (kMxA: and the scales), B0 and B1 of t + 2; a whole K tile is in flight at each wait
+  constexpr int kAhead = MXA ? 9 : 8;
+  stage(0, 0), stage(2, 0), stage(3, 0), stage(1, 0);
+  stage(0, 1), stage(2, 1), stage(3, 1);
+  G8_VM(kAhead);
   G8_BAR();
   if (wr == 1) G8_BAR();  // stagger the two wave rows by one barrier
-  int r = 0;
-  for (; r < KT - 1; ++r)
-    G8_TILE(r, G8_STAGE(0, r + 1), G8_STAGE(2, r + 1), G8_STAGE(3, r + 1), G8_STAGE(1, r + 1), G8_VMX(), G8_VMX(),
-            G8_VM(4))
-  G8_TILE(r, , , , , G8_VM(2), G8_VM(0), )
-#undef G8_TILE
-#undef G8_VMX
-#undef G8_VM
-#undef G8_STAGE
-  if (wr == 0) G8_BAR();  // re-align the wave rows
-#undef G8_MFMA
-#undef G8_BAR
-  __syncthreads();  // every wave is done reading the K buffers: LDS is reused by the epilogue
-
-  // ---- epilogue: scales in registers, per wave 128 rows x 64 bf16 columns through LDS, 16 B stores ----
-  // (row loop outermost: one activation scale live at a time — hoisting all 32 of them spills)
-  __builtin_amdgcn_sched_barrier(0);
-  if constexpr (!BF) {
-    float ws[4];
+  for (int r = 0; r < KT; ++r) {
+    const uint8_t* cb = smem + (r & 1) * kBufB;
+    rdB(cb + kUB0, 0);
+    rdB(cb + kUB1, 2);
+    rdA(cb + kUA0);
+    if constexpr (MXA) {
+      const uint8_t* st = smem + kLdsB + (r & 1) * 2048 + (wr * 128 + r16) * 4 + q;
 #pragma unroll
-    for (int jj = 0; jj < 4; ++jj) {
-      const int col = n0 + wc * 64 + jj * 16 + r16;
-      ws[jj] = col < p.N ? p.w_scale[(size_t)g * p.N + col] : 0.f;
+      for (int i = 0; i < 8; ++i) sc[i] = st[i * 64];
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int rr = 0; rr < 4; ++rr) {
-        int row = m_begin + wr * 128 + i * 16 + 4 * q + rr;
-        if (row >= m_end) row = m_begin;
-        const float as = MXA ? 1.f : p.a_scale[p.a_rows ? p.a_rows[row] : row];
-#pragma unroll
-        for (int jj = 0; jj < 4; ++jj) acc[i][jj][rr] *= as * ws[jj];
-        __builtin_amdgcn_sched_barrier(0);  // one scale load in flight at a time: no 32-load VGPR burst
-      }
+    stage(1, r + 1);
+    G8_VM(kAhead);
+    G8_MFMA(0);
+    rdA(cb + kUA1);
+    stage(0, r + 2), stage(2, r + 2), stage(3, r + 2);
+    G8_VM(kAhead);
+    G8_MFMA(4);
   }
-  if constexpr (SWIGLU) {
-    // columns jj 0, 1 of the wave are gate, jj 2, 3 the matching up columns: 32 outputs per row
-    constexpr int CW = 32;
-    bf16_t* ot = reinterpret_cast<bf16_t*>(smem) + wid * 128 * CW;
+  if (wr == 0) G8_BAR();  // re-align the wave rows
+  G8_VM(0);               // the requests past the end have landed before the LDS is given back
+#undef G8_MFMA
+#undef G8_VM
+#undef G8_BAR
+
+  // ---- epilogue: a lane holds eight consecutive columns of a row: scales, SwiGLU and 16 B stores from the registers ----
+  const int col0 = n0 + wc * 64 + 8 * q;
+  float ws[2][8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
+  for (int c = 0; c < 2; ++c)
 #pragma unroll
-      for (int jj = 0; jj < 2; ++jj)
+    for (int e = 0; e < 8; ++e) ws[c][e] = !BF && col0 + 32 * c < p.N ? p.w_scale[(size_t)g * p.N + col0 + 32 * c + e] : 1.f;
+  float as[8];
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int row = i * 16 + 4 * q + rr, col = jj * 16 + r16;
-          ot[row * CW + (col ^ ((row & 3) << 3))] = f2bf(silu8(acc[i][jj][rr]) * acc[i][jj + 2][rr]);
-        }
-    __syncthreads();
-    const int cch = lane % 4, nout = p.N / 2;
-    if constexpr (MODE == kMxOut) {
-      // e4m3 rows with one e8m0 scale per (row, MX block): the wave's 32 outputs of a row are exactly block wc of
-      // the workgroup's 128 (= one K slice of the down GEMM), held by one quad of lanes (8 each)
-      uint8_t* q8 = reinterpret_cast<uint8_t*>(p.C);
-#pragma unroll 4
-      for (int k = 0; k < 8; ++k) {
-        const int row = lane / 4 + 16 * k;
-        const int gm = m_begin + wr * 128 + row;
-        const int gn = n0 / 2 + wc * 32 + cch * 8;
+  for (int i = 0; i < 8; ++i) {
+    const int m = m_begin + wr * 128 + 16 * i + r16, row = m < m_end ? m : m_begin;
+    as[i] = MXA || BF ? 1.f : p.a_scale[p.a_rows ? p.a_rows[row] : row];
+  }
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const int m = m_begin + wr * 128 + 16 * i + r16;
+    float x[2][8];
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) x[c][e] = BF ? acc[i][2 * c + e / 4][e % 4] : acc[i][2 * c + e / 4][e % 4] * (as[i] * ws[c][e]);
+    if constexpr (!SWIGLU) {
+#pragma unroll
+      for (int c = 0; c < 2; ++c)
+        if (m < m_end && col0 + 32 * c < p.N) *reinterpret_cast<uint4v*>(p.C + (size_t)m * p.ldc + col0 + 32 * c) = pack8(x[c]);
+    } else {  // the wave's first 32 columns are gate, the other 32 the matching up columns
+      const int col = n0 / 2 + wc * 32 + 8 * q;
+      float y[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) y[e] = silu8(x[0][e]) * x[1][e];
+      const uint4v packed = pack8(y);
+      if constexpr (MODE != kMxOut) {
+        if (m < m_end && col < p.N / 2) *reinterpret_cast<uint4v*>(p.C + (size_t)m * p.ldc + col) = packed;
+      } else {
+        // e4m3 rows with one e8m0 scale per (row, MX block): the wave's 32 outputs of a row are exactly block wc of
+        // the workgroup's 128 (= one K slice of the down GEMM), held by four lanes (8 each)
         float v[8];
-        unpack8(*reinterpret_cast<const uint4v*>(ot + row * CW + ((cch * 8) ^ ((row & 3) << 3))), v);
-        float m = 0.f;
+        unpack8(packed, v);
+        float mx = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(v[e]));
-        const int e = mx_exp(quad_max(m));
+        for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[e]));
+        const int e = mx_exp(row_max4(mx));
         const float inv = __builtin_amdgcn_ldexpf(1.f, -e);
         uint32_t lo = 0, hi = 0;
         lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0] * inv, v[1] * inv, lo, false);
         lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[2] * inv, v[3] * inv, lo, true);
         hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4] * inv, v[5] * inv, hi, false);
         hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6] * inv, v[7] * inv, hi, true);
-        if (gm < m_end && gn < nout) {
-          *reinterpret_cast<uint2*>(q8 + (size_t)gm * p.ldc + gn) = uint2{lo, hi};
-          if (cch == 0) p.mx_out[((size_t)(n0 / 256) * p.s_rows + gm) * 4 + wc] = (uint8_t)(e + 127);
+        if (m < m_end && col < p.N / 2) {
+          *reinterpret_cast<uint2*>(reinterpret_cast<uint8_t*>(p.C) + (size_t)m * p.ldc + col) = uint2{lo, hi};
+          if (q == 0) p.mx_out[((size_t)(n0 / 256) * p.s_rows + m) * 4 + wc] = (uint8_t)(e + 127);
         }
       }
-    } else {
-#pragma unroll 4
-      for (int k = 0; k < 8; ++k) {
-        const int row = lane / 4 + 16 * k;
-        const int gm = m_begin + wr * 128 + row;
-        const int gn = n0 / 2 + wc * 32 + cch * 8;
-        if (gm < m_end && gn < nout)
-          *reinterpret_cast<uint4v*>(p.C + (size_t)gm * p.ldc + gn) =
-              *reinterpret_cast<const uint4v*>(ot + row * CW + ((cch * 8) ^ ((row & 3) << 3)));
-      }
-    }
-  } else {
-    constexpr int CW = 64;
-    bf16_t* ot = reinterpret_cast<bf16_t*>(smem) + wid * 128 * CW;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj)
-#pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-          const int row = i * 16 + 4 * q + rr, col = jj * 16 + r16;
-          ot[row * CW + (col ^ ((row & 7) << 3))] = f2bf(acc[i][jj][rr]);
-        }
-    __syncthreads();
-    const int cch = lane % 8;
-#pragma unroll 4
-    for (int k = 0; k < 16; ++k) {
-      const int row = lane / 8 + 8 * k;
-      const int gm = m_begin + wr * 128 + row;
-      const int gn = n0 + wc * 64 + cch * 8;
-      if (gm < m_end && gn < p.N)
-        *reinterpret_cast<uint4v*>(p.C + (size_t)gm * p.ldc + gn) =
-            *reinterpret_cast<const uint4v*>(ot + row * CW + ((cch * 8) ^ ((row & 7) << 3)));
     }
   }
 }
@@ -419,7 +343,7 @@ extern "C" int lwc_gemm2g(const void*, const void*, void*, const int*, const int
                               int, int, int, int, const void*, void*, int, hipStream_t);
 
 // Whether the weights bound a grouped fp8 call, and gemm2g.hip takes it: rows per group on average, and cols, its columns of
-// 128 in all groups (one workgroup each, two of them a CU: 512 in a round).  us, 8-phase / gemm2g, equal groups:
+// 128 in all groups (one workgroup each, two of them a CU: 512 in a round).  us, 8-phase / gemm2g, equal groups (8-phase: this kernel, before its two phases per K tile):
 // Up to 256 columns every CU has one workgroup or none there, and half as many here: from MX [4096, 14336] x 8 at 128 rows 153
 // / 107, 144 rows 156 / 113; [2048, 7168] x 8 at 144 rows 0.74.  Above 144 rows an uneven routing needs a second tile.
 // More of them without the SwiGLU (short K, or several rounds): [4096, 6400] x 16 (512) at 80 rows 88 / 86, at 112 rows from MX
@@ -442,7 +366,7 @@ static bool weight_bound(long long rows, int G, int N, int K, bool swiglu) {
 // 4096 (128) 48 / 34, 256 x 28672 SwiGLU to MX (112) 51 / 43, 2048 x 6144 (192) 49 / 66, 512 x 28672 (224) 61 / 73
 constexpr long long kSmallTiles = 128;
 
-// Grouped fp8 GEMM on the 8-phase schedule.  Requires K % 128 == 0, N % 8 == 0, lda / ldc % 16 == 0 (bytes
+// Grouped fp8 GEMM in 256 x 256 tiles.  Requires K % 128 == 0, N % 8 == 0, lda / ldc % 16 == 0 (bytes
 // / elements: 16-byte rows), rows_a * lda < 2^31 and 256 * K < 2^31 (32-bit buffer offsets); max_slots >=
 // sum_g ceil(M_g / 256) (ceil(rows / 256) + G always is).  row_off == null: dense, G = 1, rows [0, rows_c).
 // mode: 0 plain, 1 SwiGLU epilogue (bf16 out), 2 SwiGLU epilogue with e4m3 + MX block-scale output (C is
