@@ -32,7 +32,7 @@ int lwc_grouped_gemm(const void*, const void*, void*, const int*, const float*, 
                      int, int, int, int, int, int, long long, int, float*, int, long long, hipStream_t);
 int lwc_gemm8p(const void*, const void*, void*, const void*, float*, int*, int, int, int, int, int, int, hipStream_t);
 int lwc_gemm8p_slots();
-void lwc_gemm2w_plan(int, int, int, int, long long, int*, int*);
+void lwc_gemm2w_plan(int, int, int, int, bool, long long, int*, int*);
 int lwc_gemm2w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, int, float*, int*,
                const lwc::RowSumsq*, const lwc::RopeKV*, hipStream_t);
 int lwc_gemm4w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, float*, int, int, int,
@@ -469,8 +469,10 @@ void gemm2w(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::
   if (tile < 0) {
     int t = 0, s = 1;
     const bool ws = part.has_value() && count.has_value();
-    lwc_gemm2w_plan(M, N, K, (int)epi, ws ? part->numel() / 4096 : 0, &t, &s);
+    lwc_gemm2w_plan(M, N, K, (int)epi, false, ws ? part->numel() / 4096 : 0, &t, &s);
     tile = t, splits = s;
+  } else if (tile > 3) {
+    tile = 5;  // (none; 4, the weight streams, by the sizes only)
   }
   if (splits > 1) {
     const int64_t tiles = ((int64_t)M + 63) / 64 * ((N + 63) / 64);
@@ -541,7 +543,7 @@ void skinny_gemm(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const 
 }
 
 // A projection of a decode step of at most 64 rows with what lies between it and its neighbours (step_fuse.h), on the weight
-// stream (core 1, skinny.hip) or the 64 x 64 tiles (core 2, gemm2w.hip).  epi 0 plain, 1 residual (R; may be C), 2 SwiGLU:
+// stream (core 1, skinny.hip) or the tiles of gemm2w.hip and gemm1s.hip (core 2).  epi 0 plain, 1 residual (R; may be C), 2 SwiGLU:
 // ss [M, P] fp32 partial sums of squares scale the rows of 0 and 2 and are left by 1 (P = N / 16 of core 1, N / 32 of core 2).
 void step_gemm(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::optional<at::Tensor>& R, int64_t epi, int64_t core,
                const at::Tensor& ss, double eps, const lwc::RopeKV* kv, const c10::optional<at::Tensor>& part,
@@ -553,11 +555,13 @@ void step_gemm(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c1
   const lwc::RowSumsq rs{ss.data_ptr<float>(), (int)ss.size(1), (float)eps};
   const void* r = R.has_value() && R->defined() ? R->data_ptr() : nullptr;
   int tile = 3, splits = 1;
+  int64_t held = 0;
   if (core == 2 && part.has_value() && count.has_value()) {
     CHECK_GPU(*part); CHECK_DTYPE(*part, at::kFloat); CHECK_CONTIG(*part);
     CHECK_GPU(*count); CHECK_DTYPE(*count, at::kInt); CHECK_CONTIG(*count);
-    lwc_gemm2w_plan(M, N, K, (int)epi, std::min<int64_t>(part->numel() / 4096, count->numel()), &tile, &splits);
+    held = std::min<int64_t>(part->numel() / 4096, count->numel());
   }
+  if (core == 2) lwc_gemm2w_plan(M, N, K, (int)epi, true, held, &tile, &splits);
   CHECK_RC(core == 1 ? lwc_skinny_gemm(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, M, N, K, (int)A.stride(0), (int)C.stride(0),
                                        (int)epi, &rs, kv, cur_stream())
                      : lwc_gemm2w(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, M, N, K, (int)A.stride(0), (int)C.stride(0), (int)epi,

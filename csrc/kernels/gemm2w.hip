@@ -363,14 +363,20 @@ int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
 }  // namespace g2w
 }  // namespace lwc
 
+extern "C" int lwc_gemm1s_plan(int M, int N, int K, int epi, bool norm, long long max_splits);
+extern "C" int lwc_gemm1s(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, float*, int*, const lwc::RowSumsq*,
+                          const lwc::RopeKV*, hipStream_t);
+
 // epi 0: C = A W^T; 1: C = A W^T + R (R may be C); 2: C[:, :N/2] = silu(gate) * up over 32-row interleaved W (N % 64 == 0);
 // 3: C = A W^T + bias (R = bias [N]); 4: C = gelu(A W^T + bias) (exact erf GELU).
 // tile 0: 128 x 128, 1: 192 x 128, 2: 128 x 192 (not epi 2), 3: 64 x 64, there with splits K ranges per tile (part: tiles x
-// splits x 4096 floats, count: tiles ints, zero on the first call; the kernel leaves them zero).
+// splits x 4096 floats, count: tiles ints, zero on the first call; the kernel leaves them zero), 4: gemm1s.hip's weight streams (as
+// lwc_gemm2w_plan says, with its K ranges over the same workspace).
 // epi 5: the qkv projection with k and v written into the paged cache (kv; tile 3).  ss (tile 3): the folded RMSNorm: epi 0, 2
 // and 5 scale their rows by it (epi 5 always), epi 1 writes N / 32 partials per row (N % 32 == 0).
 // Requires K % 64 == 0, K / 64 >= splits, N % 8 == 0 and 16-byte rows and pointers.
-// The tile and the K ranges of a call (max_splits: what the caller's workspace holds, in 64 x 64 partial tiles).
+// The tile and the K ranges of a call (max_splits: what the caller's workspace holds, in 64 x 64 partial tiles; norm: with the
+// folded norm).  Up to 64 rows the weight streams where they take the call (lwc_gemm1s_plan); else:
 // 64 x 64 up to 512 tiles (two workgroups per CU) and for any call of up to 64 rows.  Measured (us, 64 x 64 against 128 x 128):
 // 512 rows x 4096 x K 1024 9.9 / 14.8, 512 x 4096 x 4096 35.5 / 42.8, 1000 x 3072 x 1024 (768 tiles) 14.9 / 13.8, 1000 x 4096 x
 // 4096 (1024 tiles) 62 / 44.  Its K ranges: as many as fit one workgroup per CU, none below 16 steps.
@@ -381,7 +387,12 @@ int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
 // Larger ones: the tile that takes the least time in whole rounds of two workgroups per CU, the larger of two that tie.
 // Measured (128 x 128 against 128 x 192): 3600 x 2304 x 768 (522 and 348 tiles) 25.3 / 20.3, 3600 x 4096 x 1024 (928 and
 // 638) 40.8 / 46.7, 7155 x 3072 x 768 (1344 and 896) 51.5 / 48.1.
-extern "C" void lwc_gemm2w_plan(int M, int N, int K, int epi, long long max_splits, int* tile, int* splits) {
+extern "C" void lwc_gemm2w_plan(int M, int N, int K, int epi, bool norm, long long max_splits, int* tile, int* splits) {
+  if (const int s = lwc_gemm1s_plan(M, N, K, epi, norm, max_splits)) {
+    *tile = 4;
+    *splits = s;
+    return;
+  }
   auto tiles = [&](int tm, int tn) { return ((long long)M + tm - 1) / tm * ((N + tn - 1) / tn); };
   *splits = 1;
   const long long small = tiles(64, 64);
@@ -401,17 +412,18 @@ extern "C" int lwc_gemm2w(const void* A, const void* W, void* C, const void* R, 
                           int tile, int splits, float* part, int* count, const lwc::RowSumsq* ss, const lwc::RopeKV* kv,
                           hipStream_t s) {
   using namespace lwc::g2w;
-  if (K % 64 != 0 || K < 64 || N % 8 != 0 || lda % 8 != 0 || ldc % 8 != 0 || tile < 0 || tile > 3) return -1;
+  if (K % 64 != 0 || K < 64 || N % 8 != 0 || lda % 8 != 0 || ldc % 8 != 0 || tile < 0 || tile > 4) return -1;
   if (192LL * (lda + K) * 2 >= (1LL << 31)) return -1;  // 32-bit buffer offsets in a tile
   if (((uintptr_t)A | (uintptr_t)W | (uintptr_t)C | (uintptr_t)R) & 15) return -1;
-  if (splits < 1 || splits > K / 64 || (splits > 1 && (tile != 3 || part == nullptr || count == nullptr))) return -1;
+  if (splits < 1 || splits > K / 64 || (splits > 1 && (tile < 3 || part == nullptr || count == nullptr))) return -1;
   if (epi == EPI_SWIGLU && (N % 64 != 0 || tile == 2)) return -1;
   if ((epi == EPI_RESIDUAL || epi == EPI_BIAS || epi == EPI_BIAS_GELU) && R == nullptr) return -1;
-  if (ss != nullptr && (tile != 3 || epi == EPI_BIAS || epi == EPI_BIAS_GELU || ss->P < 4 || ss->P % 4 != 0 || ss->P > 256 ||
+  if (ss != nullptr && (tile < 3 || epi == EPI_BIAS || epi == EPI_BIAS_GELU || ss->P < 4 || ss->P % 4 != 0 || ss->P > 256 ||
                         (epi == EPI_RESIDUAL && (N % 32 != 0 || ss->P != N / 32)))) return -1;
   if (epi == EPI_ROPE_KV && (ss == nullptr || kv == nullptr || !lwc::rope_kv_ok(*kv, N) || (64LL + kv->D) * K * 2 >= (1LL << 31))) return -1;
   if (M == 0 || N == 0) return 0;
   if (((long long)M + 63) / 64 * ((N + 63) / 64) * splits >= (1LL << 31)) return -1;
+  if (tile == 4) return lwc_gemm1s(A, W, C, R, M, N, K, lda, ldc, epi, splits, part, count, ss, kv, s);
   const Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc, 0, 0,
                  splits, part, count, 0};
   if (ss != nullptr) {

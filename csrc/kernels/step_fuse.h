@@ -1,5 +1,5 @@
 // What the projections of a decode step of few rows do besides their product, so that no kernel runs between them and
-// the attention (csrc/kernels/skinny.hip, gemm2w.hip): a kernel of a few rows takes 4 to 5 us however little it does.
+// the attention (csrc/kernels/skinny.hip, gemm2w.hip, gemm1s.hip): a kernel of a few rows takes 4 to 5 us however little it does.
 //
 //   * RMSNorm whose weight is folded into the projection behind it: rmsnorm(x) W^T = (x W^T) / rms(x), so the projection
 //     that writes the residual stream leaves the sums of squares of its columns and the next one scales its rows;
@@ -32,10 +32,11 @@ template <int n>
 LWC_DEVICE void rope_kv_angles(const RopeKV& r, RopeAhead<n>& a, int h, int c) {
   if (h < r.Hq || h >= r.Hq + r.Hkv) return;
   const size_t at = (size_t)a.position * (r.D / 2) + c;
+  typedef float vec __attribute__((ext_vector_type(n < 4 ? n : 4)));
 #pragma unroll
   for (int e = 0; e < n; e += 4) {
-    *reinterpret_cast<float4v*>(a.cs + e) = *reinterpret_cast<const float4v*>(r.cos + at + e);
-    *reinterpret_cast<float4v*>(a.sn + e) = *reinterpret_cast<const float4v*>(r.sin + at + e);
+    *reinterpret_cast<vec*>(a.cs + e) = *reinterpret_cast<const vec*>(r.cos + at + e);
+    *reinterpret_cast<vec*>(a.sn + e) = *reinterpret_cast<const vec*>(r.sin + at + e);
   }
 }
 

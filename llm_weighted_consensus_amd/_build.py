@@ -77,7 +77,7 @@ PER_FILE_FLAGS["sampler.hip"] = ["-fno-slp-vectorize"]
 # built with it.  ``_kernels`` is not: the one headline run of a build that had it (together with a rewritten gemm4w loop,
 # now switched off) ended in a GPU fault whose cause is not known, so its kernels stay as they ran before
 NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-PER_FILE_FLAGS.update({f: NO_PACKED_FP32 for f in ("encoder_few.hip", "gemm8p.hip", "gemm8g.hip", "gemm2s.hip")})
+PER_FILE_FLAGS.update({f: NO_PACKED_FP32 for f in ("encoder_few.hip", "gemm8p.hip", "gemm8g.hip", "gemm2s.hip", "gemm1s.hip")})
 
 
 def build_kernels(jobs: int = 8, force: bool = False) -> Path:

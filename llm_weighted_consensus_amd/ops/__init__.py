@@ -538,7 +538,7 @@ def gemm2w(A: torch.Tensor, W: torch.Tensor, residual: Optional[torch.Tensor] = 
     """MFMA GEMM in tiles for two workgroups per CU (K6, csrc/kernels/gemm2w.hip): the calls and epilogues of
     :func:`gemm8p`, rows and pointers at 16 bytes (:func:`gemm2w_ok`).  ``tile`` 0: 128 x 128, 1: 192 x 128, 2: 128 x 192 (not
     SwiGLU), 3: 64 x 64, there with ``splits`` K ranges per tile over the workspace ``ws`` (gemm8p's; default: the one of
-    the current stream); -1: by the sizes."""
+    the current stream); -1: by the sizes, up to 64 rows also the weight streams of csrc/kernels/gemm1s.hip."""
     if (swiglu and residual is not None) or (bias is not None and (swiglu or residual is not None)):
         raise ValueError("gemm2w: swiglu, residual and bias do not combine")
     if gelu and bias is None:
@@ -618,8 +618,8 @@ def step_project(x: torch.Tensor, w: torch.Tensor, core: int, ss: torch.Tensor, 
                  swiglu: bool = False, ws=None) -> torch.Tensor:
     """A projection of a decode step of at most 64 rows with the RMSNorm folded into it (csrc/kernels/step_fuse.h): scales the
     rows of ``x w^T`` (or of its gate and up halves, ``swiglu``) by 1 / rms from the partials ``ss`` [M, P], or adds into
-    ``residual`` in place and leaves its partials in ``ss``.  ``core``: 1 the weight stream, 2 the 64 x 64 tiles (with K ranges
-    over the workspace ``ws``)."""
+    ``residual`` in place and leaves its partials in ``ss``.  ``core``: 1 the weight stream, 2 the tiles of :func:`gemm2w` (with K
+    ranges over the workspace ``ws``)."""
     out = residual if residual is not None else torch.empty(x.shape[0], w.shape[0] // 2 if swiglu else w.shape[0], dtype=x.dtype,
                                                             device=x.device)
     part, count = ws if ws is not None else (None, None)

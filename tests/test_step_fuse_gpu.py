@@ -70,6 +70,15 @@ def test_residual_leaves_sums_of_squares(core, M, K, N):
     torch.testing.assert_close(ss.double(), _partials(r, P).double(), rtol=1e-5, atol=0)  # (32 fp32 terms)
 
 
+def test_many_columns_on_weight_streams():
+    """Core 2 with more than four units of 16 columns a CU and with two tiles a CU (csrc/kernels/gemm1s.hip): rows scaled in both, and
+    sums of squares of pairs of units."""
+    test_row_scaled(2, 61, 256, 35328, 8)
+    test_row_scaled(2, 64, 512, 22016, 16)
+    test_residual_leaves_sums_of_squares(2, 37, 5120, 6144)
+    test_qkv_into_the_cache(2, 33, 152, 10, 128, 256)
+
+
 @pytest.mark.parametrize("core", [1, 2])
 @pytest.mark.parametrize("M,Hq,Hkv,D,K", [(1, 32, 8, 128, 4096), (3, 4, 1, 64, 256), (17, 6, 2, 192, 512), (64, 8, 8, 128, 1024)])
 def test_qkv_into_the_cache(core, M, Hq, Hkv, D, K):
