@@ -32,6 +32,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..ops import gemm_plan
+from ..utils.pinned import to_device
 from .config import EncoderConfig
 from .packing import pack_ids
 
@@ -224,8 +225,9 @@ class BertEncoder:
     def embed(self, token_lists: Sequence[Sequence[int]], max_tokens: Optional[int] = None):
         """Embed sequences (token ids in this encoder's vocab; ids are folded into range) ->
         (unit f32 [n, d], unit bf16 [n, d])."""
-        ids, pos, cu, max_len = self.pack(token_lists, max_tokens)
-        return self.embed_packed(ids, pos, cu, max_len)
+        cap = min(max_tokens or self.cfg.max_position, self.cfg.max_position)
+        *packed, max_len = pack_ids(token_lists, cap, self.cfg.vocab_size)
+        return self.embed_packed(*to_device(self.device, *packed), max_len)
 
     def embed_packed(self, ids, pos, cu, max_len):
         h = self.forward_packed(ids, pos, cu, max_len)

@@ -13,6 +13,7 @@ from typing import Optional, Sequence
 import torch
 
 from .. import ops
+from ..utils.pinned import to_device
 from .config import DecoderConfig
 from .packing import pack_ids
 
@@ -31,13 +32,14 @@ class DecoderEmbedder:
         """Varlen packing keeping each sequence's END (the last token is pooled), numpy-vectorised
         (models/packing.py)."""
         cap = min(max_tokens or self.max_tokens, self.max_tokens)
-        ids, pos, cu, max_len = pack_ids(token_lists, cap, self.cfg.vocab_size, tail=True)
-        dev = self.device
-        return (torch.from_numpy(ids).to(dev), torch.from_numpy(pos).to(dev), torch.from_numpy(cu).to(dev), max_len)
+        *packed, max_len = pack_ids(token_lists, cap, self.cfg.vocab_size, tail=True)
+        return (*(torch.from_numpy(a).to(self.device) for a in packed), max_len)
 
     def embed(self, token_lists: Sequence[Sequence[int]], max_tokens: Optional[int] = None):
         """-> (unit f32 [n, d], unit bf16 [n, d])"""
-        ids, pos, cu, max_len = self.pack(token_lists, max_tokens)
+        cap = min(max_tokens or self.max_tokens, self.max_tokens)
+        *packed, max_len = pack_ids(token_lists, cap, self.cfg.vocab_size, tail=True)
+        ids, pos, cu = to_device(self.device, *packed)
         # only each sequence's last token is pooled: the last layer's o projection, MLP and the final norm run
         # on those rows alone (LlamaModel._layers ``keep``)
         last = (cu[1:] - 1).long()

@@ -23,6 +23,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..ops import gemm_plan, res32
+from ..utils.pinned import to_device
 from .cache import PagedLayerCache
 from .state import RecurrentStatePool
 
@@ -319,15 +320,12 @@ class LatentDecoder:
             first = np.concatenate([[0], np.cumsum(last - skip)])
             item = np.repeat(np.arange(len(k_lens)), k_lens - lo)
             pos = np.concatenate([np.arange(a, n) for a, n in zip(lo, k_lens)]) if len(k_lens) else np.zeros(0, np.int64)
-            dev = self.device
-            item_d, pos_d = torch.from_numpy(item).to(dev), torch.from_numpy(pos).to(dev)
-            blk = ch["block_tables"][item_d, pos_d // bs].long()
             tables = np.zeros((len(k_lens), max(1, int(last.max()))), np.int32)
             for i in range(len(k_lens)):
                 tables[i, skip[i]:last[i]] = first[i] + np.arange(last[i] - skip[i])
-            ctx = plan.scratch[("ctx", window)] = {
-                "blk": blk, "off": pos_d % bs, "slots": torch.from_numpy((first[item] - skip[item]) * bs + pos).to(dev),
-                "tables": torch.from_numpy(tables).to(dev), "pages": int(first[-1])}
+            item_d, page, off, slots, tables_d = to_device(self.device, item, pos // bs, pos % bs, (first[item] - skip[item]) * bs + pos, tables)
+            ctx = plan.scratch[("ctx", window)] = {"blk": ch["block_tables"][item_d, page].long(), "off": off, "slots": slots,
+                                                   "tables": tables_d, "pages": int(first[-1])}
         return ctx
 
     def _expanded_attention(self, q, positions, x, m, ci: int, cache: PagedLayerCache, plan: StepAttention, sink) -> torch.Tensor:
@@ -408,10 +406,9 @@ class LatentDecoder:
         if cu[-1] != T or state_slots.numel() != n_dec + len(q_lens):
             raise ValueError(f"{self.design}: rows, portions and state slots disagree")
         row_item = np.concatenate([np.arange(n_dec, dtype=np.int64), n_dec + np.repeat(np.arange(len(q_lens)), q_lens)])
-        dev = self.device
+        row_item_d, cu_d = to_device(self.device, row_item.astype(np.int32), cu.astype(np.int32))
         lens = [1] * min(n_dec, 1) + [int(n) for n in q_lens]
-        return res32.StepItems(torch.from_numpy(row_item.astype(np.int32)).to(dev), torch.from_numpy(cu.astype(np.int32)).to(dev),
-                               state_slots, positions, span=(min(lens), max(lens)) if lens else (0, 0))
+        return res32.StepItems(row_item_d, cu_d, state_slots, positions, span=(min(lens), max(lens)) if lens else (0, 0))
 
     def prefill(self, tokens, positions, slots, cu_seqlens, max_seqlen, last_idx, cache, ctx=None):
         raise RuntimeError(f"{self.design} prefills through forward_mixed over the paged cache (paged_prefill)")

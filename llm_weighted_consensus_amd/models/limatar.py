@@ -209,9 +209,13 @@ class LimatarModel(LatentDecoder):
         cq = res32.latent_kv_write(proj, m.q_rank, C, R, x["dq_norm"], x["dkv_norm"], x["freq"], x["rot_mult"], positions,
                                    slots, cache.k[ci], cache.v[ci], self.cfg.norm_eps)
         q = self._linear(cq, x["w_uq"])                                            # [T, H (D + R)]
-        a = torch.empty(T, H * m.vdim, dtype=dt, device=self.device)
-        for rows, o in self._latent_attention(q, x, m, ci, positions, cache, plan, sink=x["sink"]):
-            a[rows].view(-1, H, m.vdim).copy_(o)
+        parts = self._latent_attention(q, x, m, ci, positions, cache, plan, sink=x["sink"])
+        if len(parts) == 1 and parts[0][1].is_contiguous():   # all rows, as the gate reads them: 16384 x 4096 48 us less
+            a = parts[0][1].view(T, H * m.vdim)
+        else:
+            a = torch.empty(T, H * m.vdim, dtype=dt, device=self.device)
+            for rows, o in parts:
+                a[rows].view(-1, H, m.vdim).copy_(o)
         res32.gate_mul(a, proj[:, m.q_rank + C + R:], "sigmoid")
         return a
 

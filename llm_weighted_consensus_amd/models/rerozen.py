@@ -38,6 +38,7 @@ import torch.nn.functional as F
 
 from .. import ops
 from ..ops import gemm_plan, res32
+from ..utils.pinned import to_device
 from .cache import PagedLayerCache
 from .config import RerozenConfig
 from .state import RecurrentStatePool
@@ -428,9 +429,7 @@ class RerozenModel:
         if cu[-1] != T or state_slots.numel() != n_dec + len(q_lens):
             raise ValueError("Rerozen: rows, portions and state slots disagree")
         row_item = np.concatenate([np.arange(n_dec, dtype=np.int64), n_dec + np.repeat(np.arange(len(q_lens)), q_lens)])
-        dev = self.device
-        items = res32.StepItems(torch.from_numpy(row_item.astype(np.int32)).to(dev), torch.from_numpy(cu.astype(np.int32)).to(dev),
-                                state_slots, positions)
+        items = res32.StepItems(*to_device(self.device, row_item.astype(np.int32), cu.astype(np.int32)), state_slots, positions)
         dec_run = self._attend(cache, positions, dec["block_tables"]) if n_dec else None
         chk_run = (self._attend(cache, positions, chunk["block_tables"], cu_q=chunk["cu_q"], k_lens=chunk.get("k_lens"),
                                 max_q=int(chunk.get("max_q", 0))) if T > n_dec else None)
