@@ -271,6 +271,8 @@ class _PinnedRing:
         if size > self.n // 4:
             return t.pin_memory().to(dev, non_blocking=True)
         if self.head + size > self.n:
+            while self.live and self.live[0][0] >= self.head:
+                self.live.popleft()[2].synchronize()  # (what the last round left at the arena's end, which this one passes over)
             self.head = 0
         start, end = self.head, self.head + size
         while self.live and self.live[0][0] < end and start < self.live[0][1]:
