@@ -2,10 +2,14 @@
 // forward for packed variable-length sequences (cu_seqlens), head_dim 32 (bge-small), 64 or 128,
 // bf16 in/out.
 //
-// Workgroup = 4 waves = 64 query rows of one (sequence, query head); each wave owns 16 rows and
-// walks 32-key tiles that all 4 waves share through a double-buffered, XOR-swizzled LDS image
-// (register-staged: next tile's global loads are issued before the current tile's MFMAs and written
-// to LDS after them — cdna_hip_programming.md T14).
+// Workgroup = 4 waves = 64 or 128 query rows of one (sequence, query head); each wave owns one or two sets of 16
+// rows and walks 32-key tiles that all 4 waves share through three XOR-swizzled LDS stages filled by LDS-DMA.
+// What bounds it: with one set a wave, of long sequences, the reads of K and V from LDS (twice the time of the
+// MFMAs: each wave reads a whole tile for 16 rows), which two sets halve; of short ones the reads of q, k and v from
+// memory.  The row tiles and query heads that share keys run next to each other on one XCD and find them in its L2.
+// Measured (us, 64 rows a workgroup spread over the XCDs -> here): 8 x 2048 rows x 32 (8) heads of 128, causal, 593 -> 304 (900
+// TFLOP/s), 1 x 8192 785 -> 493, 64 x 129 62 -> 46; encoders, 4096 x 128 x 12 heads of 64 693 -> 580 (5.5 TB/s), 300 x 500 558 -> 376, 64 of 45 to 180
+// rows x 16 heads 24 -> 19; 400 x 256 x 12 heads of 32 211 -> 104.
 //
 // Per wave and key tile (mfma_f32_16x16x32_bf16; lane l: r16 = l & 15, g = l >> 4):
 //   S^T = K Q^T :  A = K rows from LDS (ds_read_b128, chunk XOR row swizzle: T2),
@@ -26,6 +30,7 @@
 // one ds_read_b64 returns a lane's 4 consecutive keys of one dim — the PV B operand without a transpose.
 // V elements of keys past k_lens (the tail of the last block, stale bytes) are zeroed: P is 0 there, but
 // 0 x a stale Inf / NaN would not be.  No per-layer gather of the cached keys into contiguous buffers.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -40,7 +45,10 @@ LWC_DEVICE float4v mfma16p(const short8& a, const short8& b, const float4v& c) {
                                                  0, 0);
 }
 
-constexpr int kQT = 64;  // query rows per workgroup
+LWC_DEVICE void dma16(const __amdgpu_buffer_rsrc_t& r, char* dst, uint32_t vo) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, 0, 0, 0);
+}
+
 constexpr float kLazyRescale = 8.f;
 constexpr int kKT = 32;  // keys per tile
 
@@ -70,8 +78,10 @@ struct PrefillParams {
 // The block tables come in as a const __restrict__ kernel argument (not through the params struct): the
 // compiler may then read them with SCALAR loads.  As vector loads each block id needed an s_waitcnt
 // vmcnt(0) — which also waits for the LDS-DMA of the tiles in flight and serialises the pipeline.
-template <int D, bool PAGED>
+// MR: sets of 16 query rows a wave takes
+template <int D, bool PAGED, int MR>
 __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, const int* __restrict__ block_tables) {
+  constexpr int kQT = 64 * MR;              // query rows per workgroup
   constexpr int CPR = D / 8;                // 16-byte chunks per row
   constexpr int KS = D / 32;                // k-steps for S
   constexpr int NS = D / 16;                // n-subtiles for O
@@ -83,8 +93,14 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
   static_assert(PER_WAVE >= 1 && (2 * INSTR) % 4 == 0, "tile must split evenly over 4 waves");
   __shared__ __attribute__((aligned(16))) char smem[NST * 2 * TILE_BYTES];  // [stage][K|V]
 
-  const int seq = blockIdx.x / p.max_tiles, qtile = blockIdx.x % p.max_tiles;
-  const int hq = blockIdx.y, kvh = hq / (p.Hq / p.Hkv);
+  // The workgroups that read the same keys and values, a sequence's row tiles times the query heads of a key head, are
+  // neighbours on one XCD (x % 8 with x fastest): they find them in its L2.
+  const int unit = (int)((blockIdx.z * gridDim.y + blockIdx.y) * 8 + (blockIdx.x & 7)), in = blockIdx.x >> 3;
+  if (unit >= p.nseq * p.Hkv) return;
+  // (the next sequence's heads move on by one: an XCD that met the same one of each would use few channels of its L2, as a row of
+  // q, k and v is often a multiple of 2 KiB: 1024 x 128 rows of 16 heads of 64 249 us instead of 194)
+  const int seq = unit / p.Hkv, kvh = (unit + seq) % p.Hkv, group = p.Hq / p.Hkv;
+  const int hq = kvh * group + in % group, qtile = p.causal ? p.max_tiles - 1 - in / group : in / group;  // (causal: the longest first)
   const int s0 = p.cu_seqlens[seq], len = p.cu_seqlens[seq + 1] - s0;
   const int q0 = qtile * kQT;
   if (q0 >= len) return;  // whole workgroup exits together (uniform)
@@ -98,16 +114,25 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
   const int qoff = klen - len;  // key position of query row 0
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, g = lane >> 4;
-  const int qrow = q0 + wid * 16 + r16;  // this lane's query (as B-operand column)
+  // the wave's sets are every fourth, so that the rows a short tile has divide between the waves
+  const int wrow = q0 + wid * 16, qrow = wrow + r16;  // the first query of its first set, the lane's (as B-operand column)
 
-  short8 qf[KS];
-  {
-    const int qr = qrow < len ? qrow : len - 1;
-    const bf16_t* qp = p.q + (size_t)(s0 + qr) * p.q_stride + hq * D;
+  short8 qf[MR][KS];
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qf[s] = *reinterpret_cast<const short8*>(qp + 32 * s + 8 * g);
+  for (int i = 0; i < MR; ++i) {
+    const bf16_t* qp = p.q + (size_t)(s0 + min(qrow + 64 * i, len - 1)) * p.q_stride + hq * D;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[i][s] = *reinterpret_cast<const short8*>(qp + 32 * s + 8 * g);
   }
-  const float sl2 = p.scale * 1.4426950408889634f;
+  // (the largest score times the scale is the largest scaled one where the scale is positive: else q changes its sign.  0 as a
+  // scale that leaves every score 0 and a masked one -inf)
+  if (p.scale < 0.f) {
+#pragma unroll
+    for (int i = 0; i < MR; ++i)
+#pragma unroll
+      for (int s = 0; s < KS; ++s) qf[i][s] ^= (short)0x8000;
+  }
+  const float sl2 = fmaxf(fabsf(p.scale) * 1.4426950408889634f, 1e-37f);
 
   const int q_last = min(len, q0 + kQT) - 1;
   const int kv_end = p.causal ? q_last + 1 + qoff : klen;
@@ -121,6 +146,17 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
   //  Paged V image: the tile's two interleaved block segments [4 token groups][D][4], odd groups' bytes
   //  XOR bit 7 (the layout the ds_read_b64 PV operand reads conflict-free).
   const int lrow = lane / CPR, lpc = lane % CPR;
+  // not PAGED: a tile's rows follow the last one's: an instruction's offset moves on by a tile with every issue
+  uint32_t vo[PER_WAVE];
+  if constexpr (!PAGED) {
+#pragma unroll
+    for (int i = 0; i < PER_WAVE; ++i) {
+      const int j = wid + 4 * i, r = (j >= INSTR ? j - INSTR : j) * RPI + lrow;
+      vo[i] = (uint32_t)(r * (j >= INSTR ? p.v_stride : p.k_stride) * 2 + ((lpc ^ (r % CPR)) * 16));
+    }
+  }
+  const __amdgpu_buffer_rsrc_t rK = uniform_rsrc(PAGED ? p.k : p.k + (size_t)ks0 * p.k_stride + kvh * D, PAGED ? 0 : klen * p.k_stride * 2);
+  const __amdgpu_buffer_rsrc_t rV = uniform_rsrc(PAGED ? p.v : p.v + (size_t)ks0 * p.v_stride + kvh * D, PAGED ? 0 : klen * p.v_stride * 2);
   auto issue = [&](int tile, int stage) {
     char* kb = smem + stage * 2 * TILE_BYTES;
 #pragma unroll
@@ -152,22 +188,24 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
             (void*)segp, (short)0, __builtin_amdgcn_readfirstlane(nrec), 0x00020000);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)dst, 16, vo, 0, 0, 0);
       } else {
-        const int r = jj * RPI + lrow;
-        const int key = tile * kKT + r;
-        const int stride = isv ? p.v_stride : p.k_stride;
-        const bf16_t* base = (isv ? p.v : p.k) + (size_t)ks0 * stride + kvh * D;
-        const uint32_t vo = (uint32_t)(key * stride * 2 + ((lpc ^ (r % CPR)) * 16));
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-            (void*)base, (short)0, (uint32_t)(klen * stride * 2), 0x00020000);
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (__attribute__((address_space(3))) void*)dst, 16, vo, 0, 0, 0);
+        if (isv) dma16(rV, dst, vo[i]);
+        else dma16(rK, dst, vo[i]);
+        vo[i] += (uint32_t)(kKT * (isv ? p.v_stride : p.k_stride) * 2);
       }
     }
   };
 
-  float4v o[NS];
+  float4v o[MR][NS];
+  float m[MR], l[MR];
 #pragma unroll
-  for (int n = 0; n < NS; ++n) o[n] = float4v{0.f, 0.f, 0.f, 0.f};
-  float m = -1e30f, l = 0.f;
+  for (int i = 0; i < MR; ++i) {
+#pragma unroll
+    for (int n = 0; n < NS; ++n) o[i][n] = float4v{0.f, 0.f, 0.f, 0.f};
+    m[i] = -1e30f, l[i] = 0.f;
+  }
+  // the wave's sets with rows, and the tiles they see (it loads for the others all the same)
+  const int sets = wrow >= len ? 0 : MR > 1 && wrow + 64 < len ? MR : 1, last_row = min(wrow + 64 * (sets - 1) + 16, len);
+  const int wtiles = sets == 0 ? 0 : p.causal ? min(ntiles, (last_row + qoff + kKT - 1) / kKT) : ntiles;
 
   issue(0, 0);
   if (ntiles > 1) issue(1, 1);
@@ -185,8 +223,8 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
       vofs[n] = (rowA * CPR + (chunk ^ (rowA & (CPR - 1)))) * 16 + (pp & 1) * 8;
     }
   }
-  auto tile_step = [&](const int t, auto stage) {
-    constexpr int buf = decltype(stage)::value;
+  auto tile_step = [&](const int t, auto stage, auto nsets) {
+    constexpr int buf = decltype(stage)::value, SETS = decltype(nsets)::value;
     // own DMA of tile t landed (tile t+1's may stay in flight), then every wave's (barrier); the barrier also
     // ends every wave's reads of tile t-1, whose stage tile t+2 now refills
     if (t + 1 < ntiles)
@@ -214,156 +252,151 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
     }
     const char* kb = smem + buf * 2 * TILE_BYTES;  // compile-time stage: LDS reads take immediate offsets
     const char* vb = kb + TILE_BYTES;
+    if (t >= wtiles) return;
     // ---- S^T for the two 16-key subtiles ----
-    float4v sa = {0.f, 0.f, 0.f, 0.f}, sb = {0.f, 0.f, 0.f, 0.f};
+    float4v sa[SETS], sb[SETS];
+#pragma unroll
+    for (int i = 0; i < SETS; ++i) sa[i] = sb[i] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const short8 ka = *reinterpret_cast<const short8*>(kb + kofs[s]);
       const short8 kbv = *reinterpret_cast<const short8*>(kb + kofs[s] + 16 * CPR * 16);  // keys 16..31
-      sa = mfma16p(ka, qf[s], sa);
-      sb = mfma16p(kbv, qf[s], sb);
-    }
-    // ---- mask + online softmax (per query r16) ----
-    float pa[4], pb[4];
-    float mx = -1e30f;
-    // interior tile (every key in range and, causal, at or before the wave's first query): no mask
-    const int tlast = t * kKT + kKT - 1;
-    if (tlast < klen && (!p.causal || tlast <= q0 + wid * 16 + qoff)) {  // wave-uniform
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        pa[r] = sa[r] * sl2;
-        pb[r] = sb[r] * sl2;
-        mx = fmaxf(mx, fmaxf(pa[r], pb[r]));
-      }
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int ka_ = t * kKT + 4 * g + r, kb_ = ka_ + 16;
-        const bool va = ka_ < klen && (!p.causal || ka_ <= qrow + qoff);
-        const bool vbk = kb_ < klen && (!p.causal || kb_ <= qrow + qoff);
-        pa[r] = va ? sa[r] * sl2 : -INFINITY;
-        pb[r] = vbk ? sb[r] * sl2 : -INFINITY;
-        mx = fmaxf(mx, fmaxf(pa[r], pb[r]));
+      for (int i = 0; i < SETS; ++i) {
+        sa[i] = mfma16p(ka, qf[i][s], sa[i]);
+        sb[i] = mfma16p(kbv, qf[i][s], sb[i]);
       }
     }
-    mx = row_max4(mx);
-    // lazy rescale (log2 domain): the running max only moves — and O / l are rescaled — when some row's new
-    // scores exceed it by more than kLazyRescale, so P <= 2^8 and most tiles skip the cross-lane alpha
-    // shuffles and the O multiplies
-    if (__any(mx > m + kLazyRescale)) {  // wave-uniform
-      const float m_new = fmaxf(m, mx);
-      const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-      l *= alpha;
-      m = m_new;
-      float al[4];
+    // ---- mask + online softmax (per query r16 of a set) ----
+    short8 pf[SETS];
 #pragma unroll
-      for (int r = 0; r < 4; ++r) al[r] = __shfl(alpha, 4 * g + r, 64);
-#pragma unroll
-      for (int n = 0; n < NS; ++n)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) o[n][r] *= al[r];
-    }
-    float rs = 0.f;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      pa[r] = __builtin_amdgcn_exp2f(pa[r] - m);  // raw v_exp_f32: -inf -> 0, arguments <= 8
-      pb[r] = __builtin_amdgcn_exp2f(pb[r] - m);
-      rs += pa[r] + pb[r];
-    }
-    l += row_sum4(rs);
-    short8 pf;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      pf[r] = (short)f2bf(pa[r]);
-      pf[4 + r] = (short)f2bf(pb[r]);
-    }
-    // ---- O += P V, V columns via the hardware transpose read ----
-    if constexpr (PAGED) {
-      // lane: keys 4g..4g+3 (block A half) and 16+4g..16+4g+3 (block B half) of dim 16n + r16, 8 B each
-#pragma unroll
-      for (int n = 0; n < NS; ++n) {
-        const int off = vofs[n];
-        const short4v va4 = *reinterpret_cast<const short4v*>(vb + off);
-        const short4v vb4 = *reinterpret_cast<const short4v*>(vb + TILE_BYTES / 2 + off);
-        short8 vf;
+    for (int i = 0; i < SETS; ++i) {
+      // interior tile (every key in range and, causal, at or before the set's first query): no mask
+      const int tlast = t * kKT + kKT - 1;
+      if (!(tlast < klen && (!p.causal || tlast <= wrow + 64 * i + qoff))) {  // wave-uniform
+        // of the lane's keys 4 g + r and 16 + 4 g + r, those below lim are seen
+        const int lim = (p.causal ? min(klen, qrow + 64 * i + qoff + 1) : klen) - t * kKT - 4 * g;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          vf[r] = va4[r];
-          vf[4 + r] = vb4[r];
+          sa[i][r] = r < lim ? sa[i][r] : -INFINITY;
+          sb[i][r] = 16 + r < lim ? sb[i][r] : -INFINITY;
         }
-        o[n] = mfma16p(pf, vf, o[n]);
       }
-    } else
+      float mx = fmaxf(fmaxf(sa[i][0], sa[i][1]), sa[i][2]);
+      mx = fmaxf(fmaxf(mx, sa[i][3]), sb[i][0]);
+      mx = fmaxf(fmaxf(mx, sb[i][1]), sb[i][2]);
+      mx = fmaxf(mx, sb[i][3]) * sl2;
+      // lazy rescale (log2 domain): the running max only moves, and O / l are rescaled, when some row's new
+      // scores exceed it by more than kLazyRescale, so P <= 2^8 and most tiles neither reduce their maximum over the lanes of a
+      // row nor shuffle alphas nor multiply O
+      if (t == 0) {
+        m[i] = fmaxf(m[i], row_max4(mx));
+      } else if (__any(mx > m[i] + kLazyRescale)) {  // wave-uniform
+        const float m_new = fmaxf(m[i], row_max4(mx));
+        const float alpha = __builtin_amdgcn_exp2f(m[i] - m_new);
+        l[i] *= alpha;
+        m[i] = m_new;
+        float al[4];
 #pragma unroll
-    for (int n = 0; n < NS; ++n) {
-      const int offA = vofs[n], offB = vofs[n] + 16 * CPR * 16;  // rows 4g+qq and 16+4g+qq: same swizzle
-      const short4v va4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vb + offA));
-      const short4v vb4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vb + offB));
-      short8 vf;
+        for (int r = 0; r < 4; ++r) al[r] = __shfl(alpha, 4 * g + r, 64);
+#pragma unroll
+        for (int n = 0; n < NS; ++n)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) o[i][n][r] *= al[r];
+      }
+      float pa[4], pb[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        vf[r] = va4[r];
-        vf[4 + r] = vb4[r];
+        pa[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sa[i][r], sl2, -m[i]));  // raw v_exp_f32: -inf -> 0, arguments <= 8
+        pb[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(sb[i][r], sl2, -m[i]));
       }
-      o[n] = mfma16p(pf, vf, o[n]);
+      l[i] += ((pa[0] + pa[1]) + (pa[2] + pa[3])) + ((pb[0] + pb[1]) + (pb[2] + pb[3]));  // (the lane's keys; the row's at the end)
+      pf[i] = __builtin_bit_cast(short8, uint4v{pack_bf16x2(pa[0], pa[1]), pack_bf16x2(pa[2], pa[3]),
+                                                pack_bf16x2(pb[0], pb[1]), pack_bf16x2(pb[2], pb[3])});
+    }
+    // ---- O += P V ----
+#pragma unroll
+    for (int n = 0; n < NS; ++n) {
+      short4v va4, vb4;
+      if constexpr (PAGED) {  // lane: keys 4g..4g+3 (block A half) and 16+4g..16+4g+3 (block B half) of dim 16n + r16, 8 B each
+        va4 = *reinterpret_cast<const short4v*>(vb + vofs[n]);
+        vb4 = *reinterpret_cast<const short4v*>(vb + TILE_BYTES / 2 + vofs[n]);
+      } else {  // V columns via the hardware transpose read; rows 4g+qq and 16+4g+qq: same swizzle
+        va4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vb + vofs[n]));
+        vb4 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4*)(vb + vofs[n] + 16 * CPR * 16));
+      }
+      const short8 vf = __builtin_shufflevector(va4, vb4, 0, 1, 2, 3, 4, 5, 6, 7);
+#pragma unroll
+      for (int i = 0; i < SETS; ++i) o[i][n] = mfma16p(pf[i], vf, o[i][n]);
     }
   };
-  for (int t = 0; t < ntiles; t += NST) {  // unrolled by the stage count: every stage base is a constant
-    tile_step(t, std::integral_constant<int, 0>{});
-    if (t + 1 < ntiles) tile_step(t + 1, std::integral_constant<int, 1>{});
-    if (t + 2 < ntiles) tile_step(t + 2, std::integral_constant<int, 2>{});
-  }
+  auto walk = [&](auto nsets) {
+    for (int t = 0; t < ntiles; t += NST) {  // unrolled by the stage count: every stage base is a constant
+      tile_step(t, std::integral_constant<int, 0>{}, nsets);
+      if (t + 1 < ntiles) tile_step(t + 1, std::integral_constant<int, 1>{}, nsets);
+      if (t + 2 < ntiles) tile_step(t + 2, std::integral_constant<int, 2>{}, nsets);
+    }
+  };
+  if (MR == 1 || sets < MR) walk(std::integral_constant<int, 1>{});
+  else walk(std::integral_constant<int, MR>{});
 
-  // ---- epilogue: normalise, stage the wave's 16 x D tile through LDS, 16 B stores ----
-  float linv[4];
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const float lr = __shfl(l, 4 * g + r, 64);
-    linv[r] = lr > 0.f ? 1.f / lr : 0.f;
-  }
+  // ---- epilogue: normalise, stage the wave's rows through LDS, 16 B stores ----
   __syncthreads();
-  bf16_t* ot = reinterpret_cast<bf16_t*>(smem) + wid * 16 * D;
+  bf16_t* ot = reinterpret_cast<bf16_t*>(smem) + wid * 16 * MR * D;
 #pragma unroll
-  for (int n = 0; n < NS; ++n)
+  for (int i = 0; i < MR; ++i) {
+    const float li = row_sum4(l[i]);
+    float linv[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) ot[(4 * g + r) * D + 16 * n + r16] = f2bf(o[n][r] * linv[r]);
+    for (int r = 0; r < 4; ++r) {
+      const float lr = __shfl(li, 4 * g + r, 64);
+      linv[r] = lr > 0.f ? 1.f / lr : 0.f;
+    }
+#pragma unroll
+    for (int n = 0; n < NS; ++n)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ot[(16 * i + 4 * g + r) * D + 16 * n + r16] = f2bf(o[i][n][r] * linv[r]);
+  }
   __syncthreads();
   if constexpr (D == 128) {
     if (p.out8 != nullptr) {  // uniform
-      // lane: row lane / 4 of the wave's 16, 32-dim block lane % 4 -> 32 e4m3 bytes + one e8m0 scale
-      const int row = lane >> 2, b = lane & 3;
-      const int qr = q0 + wid * 16 + row;
-      float v[32];
+      // lane: row lane / 4 of 16, 32-dim block lane % 4 -> 32 e4m3 bytes + one e8m0 scale
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        float f[8];
-        unpack8(*reinterpret_cast<const uint4v*>(ot + row * D + 32 * b + 8 * c), f);
+      for (int i = 0; i < MR; ++i) {
+        const int row = 16 * i + (lane >> 2), b = lane & 3;
+        const int qr = wrow + 64 * i + (lane >> 2);
+        float v[32];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[8 * c + j] = f[j];
-      }
-      float amax = 0.f;
+        for (int c = 0; c < 4; ++c) {
+          float f[8];
+          unpack8(*reinterpret_cast<const uint4v*>(ot + row * D + 32 * b + 8 * c), f);
 #pragma unroll
-      for (int j = 0; j < 32; ++j) amax = fmaxf(amax, fabsf(v[j]));
-      const int e = mx_exp(amax);
-      const float sc = __builtin_amdgcn_ldexpf(1.f, -e);
-      uint32_t w[8];
+          for (int j = 0; j < 8; ++j) v[8 * c + j] = f[j];
+        }
+        float amax = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        uint32_t x = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * i] * sc, v[4 * i + 1] * sc, 0, false);
-        w[i] = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * i + 2] * sc, v[4 * i + 3] * sc, x, true);
-      }
-      if (qr < len) {
-        uint8_t* dst = p.out8 + (size_t)(s0 + qr) * p.o_stride + hq * D + 32 * b;
-        *reinterpret_cast<uint4v*>(dst) = uint4v{w[0], w[1], w[2], w[3]};
-        *reinterpret_cast<uint4v*>(dst + 16) = uint4v{w[4], w[5], w[6], w[7]};
-        p.mx[((size_t)hq * p.mx_rows + s0 + qr) * 4 + b] = (uint8_t)(e + 127);
+        for (int j = 0; j < 32; ++j) amax = fmaxf(amax, fabsf(v[j]));
+        const int e = mx_exp(amax);
+        const float sc = __builtin_amdgcn_ldexpf(1.f, -e);
+        uint32_t w[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          uint32_t x = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * k] * sc, v[4 * k + 1] * sc, 0, false);
+          w[k] = __builtin_amdgcn_cvt_pk_fp8_f32(v[4 * k + 2] * sc, v[4 * k + 3] * sc, x, true);
+        }
+        if (qr < len) {
+          uint8_t* dst = p.out8 + (size_t)(s0 + qr) * p.o_stride + hq * D + 32 * b;
+          *reinterpret_cast<uint4v*>(dst) = uint4v{w[0], w[1], w[2], w[3]};
+          *reinterpret_cast<uint4v*>(dst + 16) = uint4v{w[4], w[5], w[6], w[7]};
+          p.mx[((size_t)hq * p.mx_rows + s0 + qr) * 4 + b] = (uint8_t)(e + 127);
+        }
       }
       return;
     }
   }
-  for (int c = lane; c < 16 * CPR; c += 64) {
+  for (int c = lane; c < 16 * MR * CPR; c += 64) {
     const int row = c / CPR, ch = c % CPR;
-    const int qr = q0 + wid * 16 + row;
+    const int qr = wrow + row / 16 * 64 + row % 16;
     if (qr < len)
       *reinterpret_cast<uint4v*>(p.out + (size_t)(s0 + qr) * p.o_stride + hq * D + ch * 8) =
           *reinterpret_cast<const uint4v*>(ot + row * D + ch * 8);
@@ -372,27 +405,41 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
 
 }  // namespace lwc
 
+namespace lwc {
+template <int D, bool PAGED, int MR>
+void launch_rows(PrefillParams p, int max_seqlen, hipStream_t s) {
+  p.max_tiles = (max_seqlen + 64 * MR - 1) / (64 * MR);
+  // 8 x (row tiles x query heads of a key head) by the eighths of (sequences x key heads)
+  const int rows = (int)(((long long)p.nseq * p.Hkv + 7) / 8), y = std::min(rows, 32768);
+  prefill_attn_kernel<D, PAGED, MR><<<dim3(8 * p.max_tiles * (p.Hq / p.Hkv), y, (rows + y - 1) / y), 256, 0, s>>>(p, p.block_tables);
+}
+// Two sets of rows a wave (128 rows a workgroup) where that leaves the chip enough workgroups and a sequence's last one enough
+// rows.  us, one set / two: 1024 sequences x 16 heads of 64, of 40 rows 67 / 89, 70 136 / 122, 96 172 / 152, 128 194 / 192, 132 263 / 318, 160 286 /
+// 325, 192 344 / 378, 200 453 / 418, 256 546 / 495; 64 x 32 (8) heads of 128, of 100 rows 39 / 38, 160 61 / 59, 260 125 / 118; few workgroups (of
+// 128 rows): 1 x 1000 (256) 25 / 32, 4 x 500 (512) 24 / 26, 5 x 260 (480) 17 / 19, 20 x 120 with up to 192 rows (1280) 18 / 21, but 8 x 300 (768)
+// 23 / 20, 2 x 1500 (768) 59 / 53
+template <int D, bool PAGED>
+int launch_prefill(const PrefillParams& p, int max_seqlen, hipStream_t s) {
+  const long long wgs = (long long)p.nseq * ((max_seqlen + 127) / 128) * p.Hq;
+  const bool short_second = max_seqlen > 128 && max_seqlen <= 192;
+  if (max_seqlen > 64 && wgs >= 768 && !(short_second && (D < 128 || wgs < 2048))) launch_rows<D, PAGED, 2>(p, max_seqlen, s);
+  else launch_rows<D, PAGED, 1>(p, max_seqlen, s);
+  return (int)hipGetLastError();
+}
+}  // namespace lwc
+
 extern "C" int lwc_prefill_attention(const void* q, const void* k, const void* v, void* out, const int* cu_seqlens,
                                      const int* cu_seqlens_k, int nseq, int max_seqlen, int q_stride, int k_stride, int v_stride, int o_stride,
                                      int Hq, int Hkv, int D, float scale, int causal, hipStream_t s) {
   using namespace lwc;
   if (Hq % Hkv != 0) return -1;
   if (nseq == 0 || max_seqlen == 0) return 0;
-  const int max_tiles = (max_seqlen + kQT - 1) / kQT;
   PrefillParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (bf16_t*)out, cu_seqlens, cu_seqlens_k,
                   q_stride, k_stride,
-                  v_stride, o_stride, Hq, Hkv, nseq, max_tiles, scale, causal, nullptr, nullptr, 0,
+                  v_stride, o_stride, Hq, Hkv, nseq, 0, scale, causal, nullptr, nullptr, 0,
                   nullptr, nullptr, 0};
-  dim3 grid(nseq * max_tiles, Hq);
-  if (D == 128)
-    prefill_attn_kernel<128, false><<<grid, 256, 0, s>>>(p, nullptr);
-  else if (D == 64)
-    prefill_attn_kernel<64, false><<<grid, 256, 0, s>>>(p, nullptr);
-  else if (D == 32)
-    prefill_attn_kernel<32, false><<<grid, 256, 0, s>>>(p, nullptr);
-  else
-    return -1;
-  return (int)hipGetLastError();
+  return D == 128 ? launch_prefill<128, false>(p, max_seqlen, s) : D == 64 ? launch_prefill<64, false>(p, max_seqlen, s)
+         : D == 32 ? launch_prefill<32, false>(p, max_seqlen, s) : -1;
 }
 
 // The same with the output in MX form (D = 128, keys = queries): out8 [T, Hq * 128] e4m3 (row stride o8_stride
@@ -405,13 +452,10 @@ extern "C" int lwc_prefill_attention_mx(const void* q, const void* k, const void
   using namespace lwc;
   if (Hq % Hkv != 0 || o8_stride % 16 != 0) return -1;
   if (nseq == 0 || max_seqlen == 0) return 0;
-  const int max_tiles = (max_seqlen + kQT - 1) / kQT;
   PrefillParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, nullptr, cu_seqlens, nullptr, q_stride,
-                  k_stride, v_stride, o8_stride, Hq, Hkv, nseq, max_tiles, scale, causal, nullptr, nullptr, 0,
+                  k_stride, v_stride, o8_stride, Hq, Hkv, nseq, 0, scale, causal, nullptr, nullptr, 0,
                   (uint8_t*)out8, (uint8_t*)mx, mx_rows};
-  dim3 grid(nseq * max_tiles, Hq);
-  prefill_attn_kernel<128, false><<<grid, 256, 0, s>>>(p, nullptr);
-  return (int)hipGetLastError();
+  return launch_prefill<128, false>(p, max_seqlen, s);
 }
 
 // Causal prefill of query chunks against a PAGED KV cache (D = 128, block size 16): sequence s has queries
@@ -424,11 +468,8 @@ extern "C" int lwc_prefill_attention_paged(const void* q, const void* kc, const 
   using namespace lwc;
   if (Hq % Hkv != 0 || D != 128) return -1;
   if (nseq == 0 || max_seqlen == 0) return 0;
-  const int max_tiles = (max_seqlen + kQT - 1) / kQT;
   PrefillParams p{(const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, (bf16_t*)out, cu_seqlens, nullptr,
-                  q_stride, 0, 0, o_stride, Hq, Hkv, nseq, max_tiles, scale, 1, block_tables, k_lens, bt_stride,
+                  q_stride, 0, 0, o_stride, Hq, Hkv, nseq, 0, scale, 1, block_tables, k_lens, bt_stride,
                   nullptr, nullptr, 0};
-  dim3 grid(nseq * max_tiles, Hq);
-  prefill_attn_kernel<128, true><<<grid, 256, 0, s>>>(p, block_tables);
-  return (int)hipGetLastError();
+  return launch_prefill<128, true>(p, max_seqlen, s);
 }
