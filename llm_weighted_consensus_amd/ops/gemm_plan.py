@@ -111,6 +111,12 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
     11008, 12800 and 14336: 0.49 to 1.03 from 545 to 1900 rows but for 897 to 960 at the narrower K (0.97 to
     1.08; 0.94 to 0.99 at 14336); 2048 x 14336 up to 1.15, 5120 x 13824 1.10, 8192 x 14336 1.11, 4096 x 8192 1.14.
 
+    Down into the same 16 column tiles by other counts (94 counts at 3968 x 12288, 4096 x 11008, 12800 and 14336): 385 to 544 rows
+    0.79 to 1.00, 321 to 384 up to 1.02. Beyond 4096 rows it is the library that changes: 4096 rows x 14336 take it 309 us, 4097
+    722, gemm8p 319 and 347, whose tail of tiles is cut over all CUs. 4097 to 4608 rows 0.47 to 0.52, 6145 to 7424 0.60 to 0.90,
+    8193 to 12032 0.64 to 0.92, 12289 to 13824 0.82 to 0.92; between them the library's tiles fit again: 4609 to 5120 0.90 to 1.04,
+    5121 to 5632 0.60 to 1.09, 5633 to 6144 up to 1.06, 7425 to 8192 to 1.06, 12033 to 12288 to 1.04.
+
     Few rows (prefill: a batch of prompts' last layer runs on their last tokens only, and short prompts on few rows
     everywhere): the weight's read bounds them. gate|up, which saves its SwiGLU pass, up to 64 rows on gemm2w: 11264, 14336
     and 28672 x 4096, 16384 x 2048, 12288 x 3072, 32768 x 4096 0.74 to 0.98, 22016 x 4096 0.77 to 1.05, 8192 x 4096 0.94 to
@@ -118,7 +124,9 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
     x 2048, 1024 x 4096 to 4096 x 4096 0.54 to 0.99, but 16384 x 1024 1.06 to 1.25, 6144 x 4096 0.90 to 1.23; on gemm2w from
     33 to 64: 2048 to 6144 x 4096 to 14336 0.56 to 0.99, 8192 x 2048 and 16384 x 1024 0.70 to 0.90, but 8192 and 14336 x
     4096 1.04 to 1.09. From 17 to 32 rows the library keeps all: both cores gain on some weights (4096 x 2048 0.72 and 0.91,
-    4096 x 14336 1.2 and 0.87) and lose on others (8192 x 4096 1.27 and 1.18)."""
+    4096 x 14336 1.2 and 0.87) and lose on others (8192 x 4096 1.27 and 1.18). Down from 65 to 128 on gemm2w, whose K ranges fill
+    the CUs that a few column tiles leave idle: 14 weights of 2048 to 4096 x 8192 to 18688 0.30 to 0.95, but 4608 x 12288,
+    5120 x 8192 and 13824 0.92 to 1.37; 129 to 144 rows, a third row tile, up to 1.40."""
     size = N * K
     if epi == "swiglu":
         if M > 4608:  # (M * N: 32-bit byte offsets)
@@ -127,8 +135,12 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
         if 22016 <= N <= 28672 and 4096 <= K <= 5120 and (544 < M <= 1900 or 2400 < M <= 3600) and _g8_fill(M, N, K) >= 0.8:
             return "g8"
         return "g2" if M <= 64 and N >= 8192 and K <= 4096 and 1 << 25 <= size <= 1 << 27 else "blas"
-    if epi == "residual" and 3840 < N <= 4096 and 11008 <= K <= 14336 and 544 < M <= 1900 and not (896 < M <= 960 and K <= 12800):
-        return "g8"  # (from 897 to 960 rows a fifth row tile, of 192 or 224, has little to do)
+    if epi == "residual" and 3840 < N <= 4096 and 11008 <= K <= 14336 and (
+            384 < M <= 1900 and not (896 < M <= 960 and K <= 12800) or  # (a fifth row tile, of 192 or 224, has little to do)
+            4096 < M <= 4608 or 6144 < M <= 7424 or 8192 < M <= 12032 or 12288 < M <= 13824):
+        return "g8"
+    if epi == "residual" and 64 < M <= 128 and 2048 <= N <= 4096 and K >= 8192 and size <= 1 << 26:
+        return "g2"
     if M <= 16 and K <= 4096 and N <= 8 * K and 1 << 22 <= size <= 1 << 24:
         return "gv"
     return "g2" if 32 < M <= 64 and (N < 8192 or K <= 2048) and 1 << 24 <= size <= 1 << 26 else "blas"

@@ -70,6 +70,26 @@ def test_untuned_rule(M, N, K, epi, core):
     assert gemm_plan._untuned(M, N, K, epi) == core
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,rows", [
+    (4096, 11008, {384: "blas", 385: "g8", 4096: "blas", 4097: "g8", 4608: "g8", 4609: "blas", 6145: "g8", 7425: "blas"}),
+    (3848, 14336, {544: "g8", 7424: "g8", 8193: "g8", 12033: "blas", 13824: "g8", 13825: "blas"}), (3840, 14336, {385: "blas", 4097: "blas"}),
+    (2048, 8192, {65: "g2", 128: "g2", 129: "blas"}), (3840, 17472, {100: "g2"}), (3848, 17472, {100: "blas"}), (4104, 8192, {65: "blas"}),
+    (2040, 8192, {65: "blas"}), (2048, 8128, {65: "blas"})])
+def test_untuned_down_projections(gpu, N, K, rows):
+    """Both sides of the rule's lines, and its results against fp64 of the same operands (bound: one bf16 rounding, doubled; fp32 sums)."""
+    g = torch.Generator().manual_seed(K)
+    W = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).to(gpu)
+    for M, core in rows.items():
+        A, C = (torch.randn(M, n, generator=g).to(torch.bfloat16).to(gpu) for n in (K, N))
+        if (M, N, K, "residual") not in gemm_plan._CHOICE and (N, K, "residual") not in gemm_plan._BUCKETS and gemm_plan.MODE == "auto":
+            assert gemm_plan._backend(A, W, "residual", None, C)[0] == core
+        if core == "blas":
+            continue
+        ref = A.double() @ W.double().t() + C.double()
+        torch.testing.assert_close(gemm_plan.linear_add_(A, W, C).double(), ref, rtol=2 ** -8, atol=2e-4)
+
+
 @pytest.mark.parametrize("room", [True, False])
 def test_timings_without_room_say_so(monkeypatch, caplog, room):
     """A shape timed on cached weights, because the buffer that passes them through found no room, is named in the log and table."""
