@@ -316,17 +316,20 @@ def _enc_ok(n: str, x: torch.Tensor, w: torch.Tensor, epi: str, other: torch.Ten
     return n != "g2" or gemm2w_ok(N, K, w, other)
 
 
-# gemm8p is taken for an encoder's projection where it leads by this much, about what two timings of :func:`_time_between` differ by.
-# Stacks with a lead of 0.85 / 0.92 / 0.96 / 1 asked for, ms (two runs each): bge-base, 16391 tokens 4.11 3.95 / 3.94 4.11 / 3.94 4.11 /
-# 4.12 4.11, 100000 21.1 / 20.9 / 20.8 / 20.8, bge-large, 10000 8.39 / 8.31 / 8.25 / 8.25, 25600 17.2 / 17.3 / 17.3 / 17.5, bge-small,
-# 32000 3.45 / 3.36 / 3.35 / 3.35, 102400 10.1 / 9.98 / 9.90 / 9.90
-G8_LEAD = 0.95
+# gemm8p is taken for an encoder's projection where it leads by this much: a stack runs at the clock that its power leaves, where gemm8p
+# falls 2 to 5 % behind what :func:`_time_between` gives.  Its time there over the library's, and what a pass changes by with gemm8p for
+# that projection alone, at 32 projections of stacks of 9600 to 102400 tokens: up to 0.92 (9 projections) -0.5 to -6.5 % of the pass; 0.95 to
+# 1.00 (7) -1.4 to +2.7 %, four of them slower; above 1.00 +0.5 to +8.3 %, but two.  (Seven samples a core, in one round, gave 0.88 to 0.92
+# for three projections that slow the pass by 1.5 to 2.7 %: bge-large on 38400 tokens 23.4 -> 24.4 ms.)
+G8_LEAD = 0.9
 
 
 def _pick(key, runs, x: torch.Tensor) -> str:
+    # (twice round: the first that a process times runs slow, the library's 233 us a call that takes 201 the next time)
     t = {name: _time_between(fn, x) for name, fn in runs.items()}
+    t = {name: min(t[name], _time_between(fn, x)) for name, fn in runs.items()}
     TIMINGS[key] = t
-    if "g8" in t and min(t, key=t.get) == "g8" and t["g8"] > G8_LEAD * min(t[n] for n in t if n != "g8"):
+    if "g8" in t and t["g8"] > G8_LEAD * min(t[n] for n in t if n != "g8"):
         t = {n: v for n, v in t.items() if n != "g8"}
     own = min((n for n in t if n != "blas"), key=lambda n: t[n], default="blas")
     # (a tie goes to the own core, whose layers are launched from native code: bge-large on 7156 tokens with qkv at 52 us on the
@@ -373,21 +376,24 @@ def _time(fn, iters: int = 5, rounds: int = 3) -> float:
     return sorted(ts)[len(ts) // 2]
 
 
-def _time_between(fn, x: torch.Tensor, iters: int = 7) -> float:
+def _time_between(fn, x: torch.Tensor, ms: float = 8.0) -> float:
     """Median time of ``fn`` with a pass over its rows ``x`` before each call, as in a stack, where another kernel comes between
     any two of them: calls of one kernel in a row run on each other's heels (FFN1 of bge-base on 16391 rows, gemm8p and the
-    library: 87 and 93 us a call in a row, 105 and 105 with a pass between them, 107 and 95 in the stack)."""
+    library: 87 and 93 us a call in a row, 105 and 105 with a pass between them, 107 and 95 in the stack).  Of 7 to 40 calls, as
+    ``ms`` milliseconds hold them."""
+    def median(n: int) -> float:
+        marks = []
+        for _ in range(n):
+            x.sum()
+            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            s.record()
+            fn()
+            e.record()
+            marks.append((s, e))
+        torch.cuda.synchronize()
+        return sorted(s.elapsed_time(e) for s, e in marks)[n // 2]
     fn()
-    marks = []
-    for _ in range(iters):
-        x.sum()
-        s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        s.record()
-        fn()
-        e.record()
-        marks.append((s, e))
-    torch.cuda.synchronize()
-    return sorted(s.elapsed_time(e) for s, e in marks)[iters // 2] * 1e3
+    return median(min(40, max(7, int(ms / max(median(3), 1e-3))))) * 1e3
 
 
 def _evict_buffer(device) -> Optional[torch.Tensor]:

@@ -70,6 +70,18 @@ def test_untuned_rule(M, N, K, epi, core):
     assert gemm_plan._untuned(M, N, K, epi) == core
 
 
+@pytest.mark.parametrize("times,core", [
+    ({"blas": 100, "g8": 89}, "g8"), ({"blas": 100, "g8": 91}, "blas"), ({"blas": 100, "g8": 101}, "blas"), ({"blas": 100, "g2": 102}, "g2"),
+    ({"blas": 100, "g2": 104}, "blas"), ({"blas": 100, "g8": 95, "g2": 102}, "g2"), ({"blas": 100, "g8": 95, "g2": 104}, "blas"),
+    ({"blas": 100, "g8": 85, "g2": 95}, "g8"), ({"blas": 100}, "blas")])
+def test_encoder_core_of_timings(monkeypatch, times, core):
+    """gemm8p needs its lead over every other core, in front of the library as behind it; a tie goes to the other own cores."""
+    monkeypatch.setattr(gemm_plan, "TIMINGS", {})
+    monkeypatch.setattr(gemm_plan, "_time_between", lambda fn, x: fn())
+    assert gemm_plan._pick("key", {n: (lambda v=v: v) for n, v in times.items()}, None) == core
+    assert gemm_plan.TIMINGS == {"key": times}
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,K,rows", [
     (4096, 11008, {384: "blas", 385: "g8", 4096: "blas", 4097: "g8", 4608: "g8", 4609: "blas", 6145: "g8", 7425: "blas"}),
