@@ -448,6 +448,13 @@ const void* gemm_operands(const at::Tensor& A, const at::Tensor& W, const at::Te
 void gemm8p(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::optional<at::Tensor>& R, int64_t epi,
             at::Tensor& ws, at::Tensor& flags) {
   const void* r = gemm_operands(A, W, C, R, epi);
+  // the epilogue's buffer instructions want 16-byte rows and 32-bit offsets within 16 of them
+  if ((((uintptr_t)C.data_ptr() | (epi == 1 ? (uintptr_t)r : 0)) & 15) || C.stride(0) >= (1 << 26)) {
+    at::Tensor c = at::empty(C.sizes(), C.options());
+    gemm8p(A, W, c, epi == 1 ? c10::optional<at::Tensor>(at::empty(C.sizes(), C.options()).copy_(*R)) : R, epi, ws, flags);
+    C.copy_(c);
+    return;
+  }
   const int M = (int)A.size(0), K = (int)A.size(1), N = (int)W.size(0);
   // stream-K workspace: one fp32 256x256 partial tile and one flag per workgroup (flags zero between calls)
   const int slots = lwc_gemm8p_slots();

@@ -1,7 +1,7 @@
 // Grouped fp8 and bf16 GEMM of few rows per group (gfx950): the calls of the 256-row kernel (gemm8g.hip: the same operands, epilogues
 // and MX form) while the weights, not the matrix cores, bound them.
 //
-// The 8-phase kernel keeps one workgroup per CU with 32 KiB of weights on their way, and hands its CU over with nothing in
+// That kernel keeps one workgroup per CU with 32 KiB of weights on their way, and hands its CU over with nothing in
 // flight: the experts of a decode step read their weights at 2.7 to 3.6 TB/s.  Here a tile is 64, 128 or 192 rows of a group
 // by 128 weight rows, as in gemm2w.hip (LDS layout and operand order are the same): two workgroups per CU, each with three (64
 // rows) or two steps of 128 bytes of every row in flight.  Rows past the group's end are neither loaded nor multiplied.
@@ -10,7 +10,7 @@
 // More steps in flight for calls that give a CU one workgroup (six, five, four) gain nothing and cost dear where a second round
 // follows, us, so / here: fp8, 8 experts of 16 rows [4096, 8192] (256 workgroups) 66 / 65, [4608, 8192] (288) 89 / 77; dense
 // 700 rows x 6144 x 4096 (288) 50 / 31.
-// Measured, 8 experts, us, 8-phase kernel -> here ([28672, 4096] SwiGLU to MX, [4096, 14336] from MX; 154 and 77 at the rate of
+// Measured, 8 experts, us, 256-row kernel (before its two phases per K tile) -> here ([28672, 4096] SwiGLU to MX, [4096, 14336] from MX; 154 and 77 at the rate of
 // a plain read): 4 rows an expert 257 -> 182, 144 -> 81; 32 rows 259 -> 189, 145 -> 84; 64 rows 264 -> 200, 150 -> 90; 128 rows
 // 270 -> 217, 155 -> 115.  Dense calls of few tiles likewise: 512 rows x 4096 x K 4096 from MX 45 -> 21.
 // bf16, 8 experts of 16 rows: [14336, 4096] 194 (the 128-row kernel with split K, its clear and its conversion 204), [4096, 7168] 82
