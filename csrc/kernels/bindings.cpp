@@ -449,9 +449,9 @@ void gemm8p(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::
             at::Tensor& ws, at::Tensor& flags) {
   const void* r = gemm_operands(A, W, C, R, epi);
   // the epilogue's buffer instructions want 16-byte rows and 32-bit offsets within 16 of them
-  if ((((uintptr_t)C.data_ptr() | (epi == 1 ? (uintptr_t)r : 0)) & 15) || C.stride(0) >= (1 << 26)) {
+  if ((((uintptr_t)C.data_ptr() | (uintptr_t)r) & 15) || C.stride(0) >= (1 << 26)) {
     at::Tensor c = at::empty(C.sizes(), C.options());
-    gemm8p(A, W, c, epi == 1 ? c10::optional<at::Tensor>(at::empty(C.sizes(), C.options()).copy_(*R)) : R, epi, ws, flags);
+    gemm8p(A, W, c, r ? c10::optional<at::Tensor>(R->clone(at::MemoryFormat::Contiguous)) : R, epi, ws, flags);
     C.copy_(c);
     return;
   }
