@@ -206,6 +206,9 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
   // the wave's sets with rows, and the tiles they see (it loads for the others all the same)
   const int sets = wrow >= len ? 0 : MR > 1 && wrow + 64 < len ? MR : 1, last_row = min(wrow + 64 * (sets - 1) + 16, len);
   const int wtiles = sets == 0 ? 0 : p.causal ? min(ntiles, (last_row + qoff + kKT - 1) / kKT) : ntiles;
+  // those that the first set sees: its rows end 64 before the second's, and the values past them may be infinite or NaN (times a
+  // probability of 0)
+  const int first_tiles = MR > 1 && sets > 1 && p.causal ? max(0, min(ntiles, (wrow + 16 + qoff + kKT - 1) / kKT)) : ntiles;
 
   issue(0, 0);
   if (ntiles > 1) issue(1, 1);
@@ -223,8 +226,9 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
       vofs[n] = (rowA * CPR + (chunk ^ (rowA & (CPR - 1)))) * 16 + (pp & 1) * 8;
     }
   }
-  auto tile_step = [&](const int t, auto stage, auto nsets) {
-    constexpr int buf = decltype(stage)::value, SETS = decltype(nsets)::value;
+  // for the sets SET0 .. SETS - 1
+  auto tile_step = [&](const int t, const auto buf, auto set0, auto nsets) {
+    constexpr int SET0 = decltype(set0)::value, SETS = decltype(nsets)::value;
     // own DMA of tile t landed (tile t+1's may stay in flight), then every wave's (barrier); the barrier also
     // ends every wave's reads of tile t-1, whose stage tile t+2 now refills
     if (t + 1 < ntiles)
@@ -250,19 +254,19 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
         __syncthreads();
       }
     }
-    const char* kb = smem + buf * 2 * TILE_BYTES;  // compile-time stage: LDS reads take immediate offsets
+    const char* kb = smem + buf * 2 * TILE_BYTES;  // (a compile-time stage: LDS reads take immediate offsets)
     const char* vb = kb + TILE_BYTES;
     if (t >= wtiles) return;
     // ---- S^T for the two 16-key subtiles ----
     float4v sa[SETS], sb[SETS];
 #pragma unroll
-    for (int i = 0; i < SETS; ++i) sa[i] = sb[i] = float4v{0.f, 0.f, 0.f, 0.f};
+    for (int i = SET0; i < SETS; ++i) sa[i] = sb[i] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int s = 0; s < KS; ++s) {
       const short8 ka = *reinterpret_cast<const short8*>(kb + kofs[s]);
       const short8 kbv = *reinterpret_cast<const short8*>(kb + kofs[s] + 16 * CPR * 16);  // keys 16..31
 #pragma unroll
-      for (int i = 0; i < SETS; ++i) {
+      for (int i = SET0; i < SETS; ++i) {
         sa[i] = mfma16p(ka, qf[i][s], sa[i]);
         sb[i] = mfma16p(kbv, qf[i][s], sb[i]);
       }
@@ -270,7 +274,7 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
     // ---- mask + online softmax (per query r16 of a set) ----
     short8 pf[SETS];
 #pragma unroll
-    for (int i = 0; i < SETS; ++i) {
+    for (int i = SET0; i < SETS; ++i) {
       // interior tile (every key in range and, causal, at or before the set's first query): no mask
       const int tlast = t * kKT + kKT - 1;
       if (!(tlast < klen && (!p.causal || tlast <= wrow + 64 * i + qoff))) {  // wave-uniform
@@ -327,18 +331,23 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
       }
       const short8 vf = __builtin_shufflevector(va4, vb4, 0, 1, 2, 3, 4, 5, 6, 7);
 #pragma unroll
-      for (int i = 0; i < SETS; ++i) o[i][n] = mfma16p(pf[i], vf, o[i][n]);
+      for (int i = SET0; i < SETS; ++i) o[i][n] = mfma16p(pf[i], vf, o[i][n]);
     }
   };
+  constexpr std::integral_constant<int, 0> n0{};
   auto walk = [&](auto nsets) {
-    for (int t = 0; t < ntiles; t += NST) {  // unrolled by the stage count: every stage base is a constant
-      tile_step(t, std::integral_constant<int, 0>{}, nsets);
-      if (t + 1 < ntiles) tile_step(t + 1, std::integral_constant<int, 1>{}, nsets);
-      if (t + 2 < ntiles) tile_step(t + 2, std::integral_constant<int, 2>{}, nsets);
+    for (int t = 0; t < first_tiles; t += NST) {  // unrolled by the stage count: every stage base is a constant
+      tile_step(t, n0, n0, nsets);
+      if (t + 1 < first_tiles) tile_step(t + 1, std::integral_constant<int, 1>{}, n0, nsets);
+      if (t + 2 < first_tiles) tile_step(t + 2, std::integral_constant<int, 2>{}, n0, nsets);
     }
   };
   if (MR == 1 || sets < MR) walk(std::integral_constant<int, 1>{});
   else walk(std::integral_constant<int, MR>{});
+  if constexpr (MR > 1) {
+#pragma unroll 1
+    for (int t = first_tiles; t < ntiles; ++t) tile_step(t, t % NST, std::integral_constant<int, MR - 1>{}, std::integral_constant<int, MR>{});
+  }
 
   // ---- epilogue: normalise, stage the wave's rows through LDS, 16 B stores ----
   __syncthreads();
