@@ -62,6 +62,7 @@ struct PrefillParams {
                             // queries are the LAST len_q of those positions (cached-prefix prefill)
   int q_stride, k_stride, v_stride, o_stride;  // elements per token row
   int Hq, Hkv, nseq, max_tiles;
+  int part_bits;  // log2 of the XCDs that share a sequence's key head (prefill_part_bits)
   float scale;
   int causal;
   // PAGED: block tables [nseq, bt_stride] of the key cache; k_lens [nseq] key positions per sequence
@@ -94,12 +95,13 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
   __shared__ __attribute__((aligned(16))) char smem[NST * 2 * TILE_BYTES];  // [stage][K|V]
 
   // The workgroups that read the same keys and values, a sequence's row tiles times the query heads of a key head, are
-  // neighbours on one XCD (x % 8 with x fastest): they find them in its L2.
-  const int unit = (int)((blockIdx.z * gridDim.y + blockIdx.y) * 8 + (blockIdx.x & 7)), in = blockIdx.x >> 3;
-  if (unit >= p.nseq * p.Hkv) return;
+  // neighbours on one XCD (x % 8 with x fastest), or, taken in turn, on as many as parts says: they find them in its L2.
+  const int share = (int)((blockIdx.z * gridDim.y + blockIdx.y) * 8 + (blockIdx.x & 7));
+  const int unit = share >> p.part_bits, in = (int)(blockIdx.x >> 3 << p.part_bits) + (share & ((1 << p.part_bits) - 1));
   // (the next sequence's heads move on by one: an XCD that met the same one of each would use few channels of its L2, as a row of
   // q, k and v is often a multiple of 2 KiB: 1024 x 128 rows of 16 heads of 64 249 us instead of 194)
   const int seq = unit / p.Hkv, kvh = (unit + seq) % p.Hkv, group = p.Hq / p.Hkv;
+  if (unit >= p.nseq * p.Hkv || in >= p.max_tiles * group) return;
   const int hq = kvh * group + in % group, qtile = p.causal ? p.max_tiles - 1 - in / group : in / group;  // (causal: the longest first)
   const int s0 = p.cu_seqlens[seq], len = p.cu_seqlens[seq + 1] - s0;
   const int q0 = qtile * kQT;
@@ -415,56 +417,84 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
 }  // namespace lwc
 
 namespace lwc {
-template <int D, bool PAGED, int MR>
-void launch_rows(PrefillParams p, int max_seqlen, hipStream_t s) {
-  p.max_tiles = (max_seqlen + 64 * MR - 1) / (64 * MR);
-  // 8 x (row tiles x query heads of a key head) by the eighths of (sequences x key heads)
-  const int rows = (int)(((long long)p.nseq * p.Hkv + 7) / 8), y = std::min(rows, 32768);
-  prefill_attn_kernel<D, PAGED, MR><<<dim3(8 * p.max_tiles * (p.Hq / p.Hkv), y, (rows + y - 1) / y), 256, 0, s>>>(p, p.block_tables);
-}
 // Two sets of rows a wave (128 rows a workgroup) where that leaves the chip enough workgroups and a sequence's last one enough
 // rows.  us, one set / two: 1024 sequences x 16 heads of 64, of 40 rows 67 / 89, 70 136 / 122, 96 172 / 152, 128 194 / 192, 132 263 / 318, 160 286 /
 // 325, 192 344 / 378, 200 453 / 418, 256 546 / 495; 64 x 32 (8) heads of 128, of 100 rows 39 / 38, 160 61 / 59, 260 125 / 118; few workgroups (of
 // 128 rows): 1 x 1000 (256) 25 / 32, 4 x 500 (512) 24 / 26, 5 x 260 (480) 17 / 19, 20 x 120 with up to 192 rows (1280) 18 / 21, but 8 x 300 (768)
 // 23 / 20, 2 x 1500 (768) 59 / 53
-template <int D, bool PAGED>
-int launch_prefill(const PrefillParams& p, int max_seqlen, hipStream_t s) {
-  const long long wgs = (long long)p.nseq * ((max_seqlen + 127) / 128) * p.Hq;
+inline int prefill_sets(int nseq, int max_seqlen, int Hq, int D) {
+  const long long wgs = (long long)nseq * ((max_seqlen + 127) / 128) * Hq;
   const bool short_second = max_seqlen > 128 && max_seqlen <= 192;
-  if (max_seqlen > 64 && wgs >= 768 && !(short_second && (D < 128 || wgs < 2048))) launch_rows<D, PAGED, 2>(p, max_seqlen, s);
+  return max_seqlen > 64 && wgs >= 768 && !(short_second && (D < 128 || wgs < 2048)) ? 2 : 1;
+}
+// The XCDs over which a sequence's key head goes: as few as leave none of them with an eighth more than its share because of the
+// longest sequence (the others in equal parts of the rest of all rows; work by the square of the rows).
+// us, a key head on one XCD / so, 32 (1) heads of 128, causal: 1 x 8192 rows 3333 / 581, 1 x 2048 293 / 57, 4096 beside 30 x 60 894 / 182; 32 (2)
+// 1901 / 576, 32 (4) 987 / 555; 12 heads of 64, 1 x 8192 338 / 274; 9 heads 323 / 245.  More XCDs than that read the keys more often:
+// 32 (8) heads 1 x 2048 on 1 / 2 / 4 / 8 52 / 57 / 59 / 67, 40 x 300 rows of 12 heads 30 / 37 / 40 / 63.
+inline int prefill_part_bits(int nseq, int rows, int max_seqlen, int Hq, int Hkv, int sets) {
+  const double longest = (double)max_seqlen * max_seqlen, other = nseq > 1 ? std::max(0.0, (double)rows - max_seqlen) / (nseq - 1) : 0;
+  const double fair = Hkv / 8.0 * (longest + (nseq - 1) * other * other);
+  const int workgroups = (max_seqlen + 64 * sets - 1) / (64 * sets) * (Hq / Hkv);
+  int bits = 0;
+  auto over = [&] { return ((((Hkv << bits) + 7) / 8) / (double)(1 << bits) - Hkv / 8.0) * longest; };
+  while (bits < 3 && 2 << bits <= workgroups && over() > 0.125 * fair) ++bits;
+  return bits;
+}
+template <int D, bool PAGED, int MR>
+void launch_rows(PrefillParams p, int max_seqlen, hipStream_t s) {
+  p.max_tiles = (max_seqlen + 64 * MR - 1) / (64 * MR);
+  // 8 x (a part of row tiles x query heads of a key head) by the eighths of (sequences x key heads x parts)
+  const int parts = 1 << p.part_bits, per = (p.max_tiles * (p.Hq / p.Hkv) + parts - 1) / parts;
+  const int shares = (int)(((long long)p.nseq * p.Hkv * parts + 7) / 8), y = std::min(shares, 32768);
+  prefill_attn_kernel<D, PAGED, MR><<<dim3(8 * per, y, (shares + y - 1) / y), 256, 0, s>>>(p, p.block_tables);
+}
+// rows: of all sequences
+template <int D, bool PAGED>
+int launch_prefill(PrefillParams p, int rows, int max_seqlen, hipStream_t s) {
+  const int sets = prefill_sets(p.nseq, max_seqlen, p.Hq, D);
+  p.part_bits = prefill_part_bits(p.nseq, rows, max_seqlen, p.Hq, p.Hkv, sets);
+  if (sets == 2) launch_rows<D, PAGED, 2>(p, max_seqlen, s);
   else launch_rows<D, PAGED, 1>(p, max_seqlen, s);
   return (int)hipGetLastError();
 }
 }  // namespace lwc
 
+// How a call is cut up: query rows of a workgroup, XCDs that share a sequence's key head.
+extern "C" void lwc_prefill_plan(int nseq, int rows, int max_seqlen, int Hq, int Hkv, int D, int* tile, int* parts) {
+  const int sets = lwc::prefill_sets(nseq, max_seqlen, Hq, D);
+  *tile = 64 * sets;
+  *parts = 1 << lwc::prefill_part_bits(nseq, rows, max_seqlen, Hq, Hkv, sets);
+}
+
+// rows: of q
 extern "C" int lwc_prefill_attention(const void* q, const void* k, const void* v, void* out, const int* cu_seqlens,
-                                     const int* cu_seqlens_k, int nseq, int max_seqlen, int q_stride, int k_stride, int v_stride, int o_stride,
-                                     int Hq, int Hkv, int D, float scale, int causal, hipStream_t s) {
+                                     const int* cu_seqlens_k, int nseq, int rows, int max_seqlen, int q_stride, int k_stride, int v_stride,
+                                     int o_stride, int Hq, int Hkv, int D, float scale, int causal, hipStream_t s) {
   using namespace lwc;
   if (Hq % Hkv != 0) return -1;
   if (nseq == 0 || max_seqlen == 0) return 0;
   PrefillParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, (bf16_t*)out, cu_seqlens, cu_seqlens_k,
                   q_stride, k_stride,
-                  v_stride, o_stride, Hq, Hkv, nseq, 0, scale, causal, nullptr, nullptr, 0,
+                  v_stride, o_stride, Hq, Hkv, nseq, 0, 0, scale, causal, nullptr, nullptr, 0,
                   nullptr, nullptr, 0};
-  return D == 128 ? launch_prefill<128, false>(p, max_seqlen, s) : D == 64 ? launch_prefill<64, false>(p, max_seqlen, s)
-         : D == 32 ? launch_prefill<32, false>(p, max_seqlen, s) : -1;
+  return D == 128 ? launch_prefill<128, false>(p, rows, max_seqlen, s) : D == 64 ? launch_prefill<64, false>(p, rows, max_seqlen, s)
+         : D == 32 ? launch_prefill<32, false>(p, rows, max_seqlen, s) : -1;
 }
 
 // The same with the output in MX form (D = 128, keys = queries): out8 [T, Hq * 128] e4m3 (row stride o8_stride
 // bytes), mx [Hq][mx_rows >= T][4] e8m0 — what the fp8 o projection's block-scaled MFMAs read, so the bf16
 // output and its row quantisation pass are gone.
 extern "C" int lwc_prefill_attention_mx(const void* q, const void* k, const void* v, void* out8, void* mx,
-                                        int mx_rows, const int* cu_seqlens, int nseq, int max_seqlen, int q_stride,
-                                        int k_stride, int v_stride, int o8_stride, int Hq, int Hkv, float scale,
-                                        int causal, hipStream_t s) {
+                                        int mx_rows, const int* cu_seqlens, int nseq, int rows, int max_seqlen,
+                                        int q_stride, int k_stride, int v_stride, int o8_stride, int Hq, int Hkv, float scale, int causal, hipStream_t s) {
   using namespace lwc;
   if (Hq % Hkv != 0 || o8_stride % 16 != 0) return -1;
   if (nseq == 0 || max_seqlen == 0) return 0;
   PrefillParams p{(const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, nullptr, cu_seqlens, nullptr, q_stride,
-                  k_stride, v_stride, o8_stride, Hq, Hkv, nseq, 0, scale, causal, nullptr, nullptr, 0,
+                  k_stride, v_stride, o8_stride, Hq, Hkv, nseq, 0, 0, scale, causal, nullptr, nullptr, 0,
                   (uint8_t*)out8, (uint8_t*)mx, mx_rows};
-  return launch_prefill<128, false>(p, max_seqlen, s);
+  return launch_prefill<128, false>(p, rows, max_seqlen, s);
 }
 
 // Causal prefill of query chunks against a PAGED KV cache (D = 128, block size 16): sequence s has queries
@@ -472,13 +502,13 @@ extern "C" int lwc_prefill_attention_mx(const void* q, const void* k, const void
 // kc / vc through block_tables[s] (bt_stride entries per row, covering ceil(k_lens[s] / 16) blocks).
 extern "C" int lwc_prefill_attention_paged(const void* q, const void* kc, const void* vc, void* out,
                                            const int* cu_seqlens, const int* block_tables, const int* k_lens,
-                                           int bt_stride, int nseq, int max_seqlen, int q_stride, int o_stride, int Hq,
-                                           int Hkv, int D, float scale, hipStream_t s) {
+                                           int bt_stride, int nseq, int rows, int max_seqlen, int q_stride, int o_stride,
+                                           int Hq, int Hkv, int D, float scale, hipStream_t s) {
   using namespace lwc;
   if (Hq % Hkv != 0 || D != 128) return -1;
   if (nseq == 0 || max_seqlen == 0) return 0;
   PrefillParams p{(const bf16_t*)q, (const bf16_t*)kc, (const bf16_t*)vc, (bf16_t*)out, cu_seqlens, nullptr,
-                  q_stride, 0, 0, o_stride, Hq, Hkv, nseq, 0, scale, 1, block_tables, k_lens, bt_stride,
+                  q_stride, 0, 0, o_stride, Hq, Hkv, nseq, 0, 0, scale, 1, block_tables, k_lens, bt_stride,
                   nullptr, nullptr, 0};
-  return launch_prefill<128, true>(p, max_seqlen, s);
+  return launch_prefill<128, true>(p, rows, max_seqlen, s);
 }

@@ -54,11 +54,12 @@ int lwc_ep_unpack(const void*, int, int, int, int, int, int, void*, float*, int*
 int lwc_ep_back(const void*, const int*, int, int, int, void*, hipStream_t);
 int lwc_ep_combine(const void*, const int*, const int*, const float*, int, int, int, int, int, int, void*, hipStream_t);
 int lwc_silu_mul_quant_fp8(const void*, int, int, int, void*, float*, hipStream_t);
-int lwc_prefill_attention(const void*, const void*, const void*, void*, const int*, const int*, int, int, int, int, int, int, int,
+int lwc_prefill_attention(const void*, const void*, const void*, void*, const int*, const int*, int, int, int, int, int, int, int, int,
                           int, int, float, int, hipStream_t);
-int lwc_prefill_attention_mx(const void*, const void*, const void*, void*, void*, int, const int*, int, int, int, int,
+void lwc_prefill_plan(int, int, int, int, int, int, int*, int*);
+int lwc_prefill_attention_mx(const void*, const void*, const void*, void*, void*, int, const int*, int, int, int, int, int,
                              int, int, int, int, float, int, hipStream_t);
-int lwc_prefill_attention_paged(const void*, const void*, const void*, void*, const int*, const int*, const int*, int, int,
+int lwc_prefill_attention_paged(const void*, const void*, const void*, void*, const int*, const int*, const int*, int, int, int,
                                 int, int, int, int, int, int, float, hipStream_t);
 int lwc_sample(const void*, int, int, int, const float*, const float*, const int*, const float*, const float*,
                const float*, const float*, const float*, void*, const int*, const float*, const int*,
@@ -872,10 +873,18 @@ void prefill_attention(const at::Tensor& q, const at::Tensor& k, const at::Tenso
               "prefill_attention: head shape mismatch");
   const int nseq = (int)cu_seqlens.numel() - 1;
   CHECK_RC(lwc_prefill_attention(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), cu_seqlens.data_ptr<int>(),
-                                 cuk, nseq, (int)max_seqlen, (int)q.stride(0), (int)k.stride(0), (int)v.stride(0),
+                                 cuk, nseq, (int)q.size(0), (int)max_seqlen, (int)q.stride(0), (int)k.stride(0), (int)v.stride(0),
                                  (int)out.stride(0), (int)Hq, (int)Hkv, (int)D, (float)scale, causal ? 1 : 0,
                                  cur_stream()),
            "prefill_attention");
+}
+
+// (query rows of a workgroup, XCDs that share a sequence's key head) of a prefill attention call
+std::pair<int64_t, int64_t> prefill_plan(int64_t nseq, int64_t rows, int64_t max_seqlen, int64_t Hq, int64_t Hkv, int64_t D) {
+  TORCH_CHECK(nseq > 0 && rows > 0 && max_seqlen > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0, "prefill_plan: sizes");
+  int tile = 0, parts = 0;
+  lwc_prefill_plan((int)nseq, (int)rows, (int)max_seqlen, (int)Hq, (int)Hkv, (int)D, &tile, &parts);
+  return {tile, parts};
 }
 
 // The layers of a post-norm encoder over packed rows x [T, d], launched from here: a forward of few rows is bound by the
@@ -982,7 +991,7 @@ void prefill_attention_mx(const at::Tensor& q, const at::Tensor& k, const at::Te
               "prefill_attention_mx: mx [Hq, >= T, 4]");
   const int nseq = (int)cu_seqlens.numel() - 1;
   CHECK_RC(lwc_prefill_attention_mx(q.data_ptr(), k.data_ptr(), v.data_ptr(), out8.data_ptr(), mx.data_ptr(),
-                                    (int)mx.size(1), cu_seqlens.data_ptr<int>(), nseq, (int)max_seqlen,
+                                    (int)mx.size(1), cu_seqlens.data_ptr<int>(), nseq, (int)q.size(0), (int)max_seqlen,
                                     (int)q.stride(0), (int)k.stride(0), (int)v.stride(0), (int)out8.stride(0), (int)Hq,
                                     (int)Hkv, (float)scale, causal ? 1 : 0, cur_stream()),
            "prefill_attention_mx");
@@ -1010,7 +1019,7 @@ void prefill_attention_paged(const at::Tensor& q, const at::Tensor& k_cache, con
               "prefill_attention_paged: q / out shapes");
   CHECK_RC(lwc_prefill_attention_paged(q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), out.data_ptr(),
                                        cu_seqlens.data_ptr<int>(), block_tables.data_ptr<int>(), k_lens.data_ptr<int>(),
-                                       (int)block_tables.size(1), nseq, (int)max_seqlen, (int)q.stride(0),
+                                       (int)block_tables.size(1), nseq, (int)q.size(0), (int)max_seqlen, (int)q.stride(0),
                                        (int)out.stride(0), (int)Hq, Hkv, D, (float)scale, cur_stream()),
            "prefill_attention_paged");
 }
@@ -1204,6 +1213,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("set_decode_wave_min_items", &lwc_set_decode_wave_min_items,
         "B*Hkv*splits threshold of the wave-per-item decode kernel; returns the previous value");
   m.def("prefill_attention", &prefill_attention);
+  m.def("prefill_plan", &prefill_plan);
   m.def("encoder_few", &encoder_few, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("encoder_layers", &encoder_layers, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("prefill_attention_mx", &prefill_attention_mx);

@@ -23,8 +23,8 @@
 #include "common.h"
 
 extern "C" int lwc_prefill_attention(const void* q, const void* k, const void* v, void* out, const int* cu_q, const int* cu_k, int nseq,
-                                     int max_seqlen, int ldq, int ldk, int ldv, int ldo, int Hq, int Hkv, int D, float scale,
-                                     int causal, hipStream_t s);
+                                     int rows, int max_seqlen, int ldq, int ldk, int ldv, int ldo, int Hq, int Hkv, int D,
+                                     float scale, int causal, hipStream_t s);
 
 namespace lwc {
 namespace efew {
@@ -469,7 +469,7 @@ int run(Norm n, const Call& c) {
     } else {
       lds<project_kernel<MT, D, PF, OUT_BIAS>>(kLn);
       project_kernel<MT, D, PF, OUT_BIAS><<<3 * D / 16, kT, kLn, c.s>>>(Proj{n, nullptr, t(0), t(1), nullptr, c.h, T, 3 * D, D});
-      const int rc = lwc_prefill_attention(c.h, c.h + D, c.h + 2 * D, c.a, c.cu, c.cu, c.nseq, T, 3 * D, 3 * D, 3 * D, D, H, H, DH,
+      const int rc = lwc_prefill_attention(c.h, c.h + D, c.h + 2 * D, c.a, c.cu, c.cu, c.nseq, T, T, 3 * D, 3 * D, 3 * D, D, H, H, DH,
                                            c.scale, 0, c.s);
       if (rc != 0) return rc;
     }
