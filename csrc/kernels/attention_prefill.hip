@@ -7,9 +7,9 @@
 // What bounds it: with one set a wave, of long sequences, the reads of K and V from LDS (twice the time of the
 // MFMAs: each wave reads a whole tile for 16 rows), which two sets halve; of short ones the reads of q, k and v from
 // memory.  The row tiles and query heads that share keys run next to each other on one XCD and find them in its L2.
-// Measured (us, 64 rows a workgroup spread over the XCDs -> here): 8 x 2048 rows x 32 (8) heads of 128, causal, 593 -> 304 (900
-// TFLOP/s), 1 x 8192 785 -> 493, 64 x 129 62 -> 46; encoders, 4096 x 128 x 12 heads of 64 693 -> 580 (5.5 TB/s), 300 x 500 558 -> 376, 64 of 45 to 180
-// rows x 16 heads 24 -> 19; 400 x 256 x 12 heads of 32 211 -> 104.
+// Measured (us, 64 rows a workgroup spread over the XCDs -> here): 8 x 2048 rows x 32 (8) heads of 128, causal, 593 -> 297 (920
+// TFLOP/s), 1 x 8192 798 -> 506, 64 x 129 62 -> 45; encoders, 4096 x 128 x 12 heads of 64 693 -> 580 (5.5 TB/s), 300 x 500 558 -> 372, 64 of 45 to 180
+// rows x 16 heads 24 -> 18; 400 x 256 x 12 heads of 32 211 -> 112; paged, 8 x 2048 697 -> 364, 24 x 16 rows of 900 keys 40 -> 32.
 //
 // Per wave and key tile (mfma_f32_16x16x32_bf16; lane l: r16 = l & 15, g = l >> 4):
 //   S^T = K Q^T :  A = K rows from LDS (ds_read_b128, chunk XOR row swizzle: T2),
@@ -275,6 +275,7 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
     }
     // ---- mask + online softmax (per query r16 of a set) ----
     short8 pf[SETS];
+    float mxs[SETS];
 #pragma unroll
     for (int i = SET0; i < SETS; ++i) {
       // interior tile (every key in range and, causal, at or before the set's first query): no mask
@@ -292,24 +293,38 @@ __global__ void __launch_bounds__(256) prefill_attn_kernel(PrefillParams p, cons
       mx = fmaxf(fmaxf(mx, sa[i][3]), sb[i][0]);
       mx = fmaxf(fmaxf(mx, sb[i][1]), sb[i][2]);
       mx = fmaxf(mx, sb[i][3]) * sl2;
-      // lazy rescale (log2 domain): the running max only moves, and O / l are rescaled, when some row's new
-      // scores exceed it by more than kLazyRescale, so P <= 2^8 and most tiles neither reduce their maximum over the lanes of a
-      // row nor shuffle alphas nor multiply O
-      if (t == 0) {
-        m[i] = fmaxf(m[i], row_max4(mx));
-      } else if (__any(mx > m[i] + kLazyRescale)) {  // wave-uniform
-        const float m_new = fmaxf(m[i], row_max4(mx));
-        const float alpha = __builtin_amdgcn_exp2f(m[i] - m_new);
-        l[i] *= alpha;
-        m[i] = m_new;
-        float al[4];
+      mxs[i] = mx;
+    }
+    // lazy rescale (log2 domain): the running max only moves, and O / l are rescaled, when some row's new
+    // scores exceed it by more than kLazyRescale, so P <= 2^8 and most tiles neither reduce their maximum over the lanes of a
+    // row nor shuffle alphas nor multiply O.  One branch for both sets: with one each, registers are copied around them (188 of them
+    // instead of 166, and two workgroups a CU instead of three: 8 x 2048 rows x 32 heads of 128 345 us, so 297)
+    if (t == 0) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) al[r] = __shfl(alpha, 4 * g + r, 64);
+      for (int i = SET0; i < SETS; ++i) m[i] = fmaxf(m[i], row_max4(mxs[i]));
+    } else {
+      bool need = false;
 #pragma unroll
-        for (int n = 0; n < NS; ++n)
+      for (int i = SET0; i < SETS; ++i) need |= mxs[i] > m[i] + kLazyRescale;
+      if (__any(need)) {  // wave-uniform
 #pragma unroll
-          for (int r = 0; r < 4; ++r) o[i][n][r] *= al[r];
+        for (int i = SET0; i < SETS; ++i) {
+          const float m_new = fmaxf(m[i], row_max4(mxs[i]));
+          const float alpha = __builtin_amdgcn_exp2f(m[i] - m_new);
+          l[i] *= alpha;
+          m[i] = m_new;
+          float al[4];
+#pragma unroll
+          for (int r = 0; r < 4; ++r) al[r] = __shfl(alpha, 4 * g + r, 64);
+#pragma unroll
+          for (int n = 0; n < NS; ++n)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[i][n][r] *= al[r];
+        }
       }
+    }
+#pragma unroll
+    for (int i = SET0; i < SETS; ++i) {
       float pa[4], pb[4];
 #pragma unroll
       for (int r = 0; r < 4; ++r) {

@@ -74,10 +74,12 @@ PER_FILE_FLAGS["sampler.hip"] = ["-fno-slp-vectorize"]
 
 
 # hipcc -O3 forms packed fp32 instructions by itself from scalar float code; this keeps it from doing so.  ``_res32`` is
-# built with it.  ``_kernels`` is not: the one headline run of a build that had it (together with a rewritten gemm4w loop,
-# now switched off) ended in a GPU fault whose cause is not known, so its kernels stay as they ran before
+# built with it, and so are the files of ``_kernels`` written or rewritten since.  Its others are not: the one headline run of a
+# build that had it throughout (together with a rewritten gemm4w loop, now switched off) ended in a GPU fault whose cause is not
+# known, so those kernels stay as they ran before
 NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
-PER_FILE_FLAGS.update({f: NO_PACKED_FP32 for f in ("encoder_few.hip", "gemm8p.hip", "gemm8g.hip", "gemm2s.hip", "gemm1s.hip")})
+for _f in ("attention_prefill.hip", "encoder_few.hip", "gemm8p.hip", "gemm8g.hip", "gemm2s.hip", "gemm1s.hip"):
+    PER_FILE_FLAGS[_f] = PER_FILE_FLAGS.get(_f, []) + NO_PACKED_FP32
 
 
 def build_kernels(jobs: int = 8, force: bool = False) -> Path:
