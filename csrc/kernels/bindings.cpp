@@ -449,11 +449,18 @@ const void* gemm_operands(const at::Tensor& A, const at::Tensor& W, const at::Te
 void gemm8p(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::optional<at::Tensor>& R, int64_t epi,
             at::Tensor& ws, at::Tensor& flags) {
   const void* r = gemm_operands(A, W, C, R, epi);
-  // the epilogue's buffer instructions want 16-byte rows and 32-bit offsets within 16 of them
+  // the epilogue's buffer instructions want 16-byte rows and 32-bit offsets within 16 of them: else through contiguous results,
+  // of at most half the columns that it reaches
   if ((((uintptr_t)C.data_ptr() | (uintptr_t)r) & 15) || C.stride(0) >= (1 << 26)) {
-    at::Tensor c = at::empty(C.sizes(), C.options());
-    gemm8p(A, W, c, r ? c10::optional<at::Tensor>(R->clone(at::MemoryFormat::Contiguous)) : R, epi, ws, flags);
-    C.copy_(c);
+    const int64_t cols = C.size(1), rows_per_col = epi == 2 ? 2 : 1;
+    for (int64_t at = 0; at < cols; at += 1 << 25) {
+      const int64_t n = std::min<int64_t>(cols - at, 1 << 25);
+      at::Tensor c = at::empty({C.size(0), n}, C.options());
+      c10::optional<at::Tensor> part = R;
+      if (r) part = R->narrow(epi == 1 ? 1 : 0, at, n).clone(at::MemoryFormat::Contiguous);
+      gemm8p(A, W.narrow(0, at * rows_per_col, n * rows_per_col), c, part, epi, ws, flags);
+      C.narrow(1, at, n).copy_(c);
+    }
     return;
   }
   const int M = (int)A.size(0), K = (int)A.size(1), N = (int)W.size(0);
