@@ -317,8 +317,8 @@ def _enc_ok(n: str, x: torch.Tensor, w: torch.Tensor, epi: str, other: torch.Ten
 
 
 # gemm8p is taken for an encoder's projection where it leads by this much: a stack runs at the clock that its power leaves, where gemm8p
-# falls 2 to 5 % behind what :func:`_time_between` gives.  Its time there over the library's, and what a pass changes by with gemm8p for
-# that projection alone, at 32 projections of stacks of 9600 to 102400 tokens: up to 0.92 (9 projections) -0.5 to -6.5 % of the pass; 0.95 to
+# falls 2 to 5 % behind what :func:`_time_between` gives.  Its time there over the library's (in medians of 20 calls and more; in the
+# few calls of now up to 0.05 less), and what a pass changes by with gemm8p for that projection alone, at 32 projections of stacks of 9600 to 102400 tokens: up to 0.92 (9 projections) -0.5 to -6.5 % of the pass; 0.95 to
 # 1.00 (7) -1.4 to +2.7 %, four of them slower; above 1.00 +0.5 to +8.3 %, but two.  (Seven samples a core, in one round, gave 0.88 to 0.92
 # for three projections that slow the pass by 1.5 to 2.7 %: bge-large on 38400 tokens 23.4 -> 24.4 ms.)
 G8_LEAD = 0.9
@@ -376,12 +376,13 @@ def _time(fn, iters: int = 5, rounds: int = 3) -> float:
     return sorted(ts)[len(ts) // 2]
 
 
-def _time_between(fn, x: torch.Tensor, ms: float = 8.0) -> float:
+def _time_between(fn, x: torch.Tensor, n: int = 7) -> float:
     """Median time of ``fn`` with a pass over its rows ``x`` before each call, as in a stack, where another kernel comes between
     any two of them: calls of one kernel in a row run on each other's heels (FFN1 of bge-base on 16391 rows, gemm8p and the
-    library: 87 and 93 us a call in a row, 105 and 105 with a pass between them, 107 and 95 in the stack).  Of 7 to 40 calls, as
-    ``ms`` milliseconds hold them."""
-    def median(n: int) -> float:
+    library: 87 and 93 us a call in a row, 105 and 105 with a pass between them, 107 and 95 in the stack).  Of ``n`` calls behind
+    the first, 3 where that takes a millisecond: a request waits for them (with 7 to 40, behind four: the first pass of bge-large on 38400
+    tokens 176 ms, so 60, of bge-base on 524288 429 and 227, of bge-small on 1661 45 and 10; gemm8p's time over the library's up to 0.05 higher)."""
+    def calls(n: int) -> list:
         marks = []
         for _ in range(n):
             x.sum()
@@ -391,9 +392,9 @@ def _time_between(fn, x: torch.Tensor, ms: float = 8.0) -> float:
             e.record()
             marks.append((s, e))
         torch.cuda.synchronize()
-        return sorted(s.elapsed_time(e) for s, e in marks)[n // 2]
-    fn()
-    return median(min(40, max(7, int(ms / max(median(3), 1e-3))))) * 1e3
+        return sorted(s.elapsed_time(e) for s, e in marks)
+    times = calls(3 if calls(1)[0] > 1 else n)
+    return times[len(times) // 2] * 1e3
 
 
 def _evict_buffer(device) -> Optional[torch.Tensor]:

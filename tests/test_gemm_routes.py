@@ -83,6 +83,21 @@ def test_encoder_core_of_timings(monkeypatch, times, core):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,most", [(256, 16), (16384, 8)])
+def test_encoder_cores_are_timed_in_few_calls(gpu, monkeypatch, n, most):
+    """A request waits while the cores of a new size are timed: sixteen calls of each, eight of those that take a millisecond."""
+    monkeypatch.setattr(gemm_plan, "TIMINGS", {})
+    x, w = torch.ones(n, n, device=gpu, dtype=torch.bfloat16), torch.ones(n, n, device=gpu, dtype=torch.bfloat16)
+    made = {"blas": 0, "g2": 0, "g8": 0}
+
+    def call(core):
+        made[core] += 1
+        x @ w
+    assert gemm_plan._pick("key", {c: (lambda c=c: call(c)) for c in made}, x) in made
+    assert all(0 < v <= most for v in made.values()) and all(v > 0 for v in gemm_plan.TIMINGS["key"].values())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("N,K,rows", [
     (4096, 11008, {384: "blas", 385: "g8", 4096: "blas", 4097: "g8", 4608: "g8", 4609: "blas", 6145: "g8", 7425: "blas"}),
     (3848, 14336, {544: "g8", 7424: "g8", 8193: "g8", 12033: "blas", 13824: "g8", 13825: "blas"}), (3840, 14336, {385: "blas", 4097: "blas"}),
