@@ -176,9 +176,10 @@ class BertEncoder:
         fuse_o, fuse_f = mode == "all", mode in ("all", "ffn2")
         if x.dtype == torch.bfloat16 and self.layers:
             L = self.layers[0]
-            cores = gemm_plan.encoder_cores(T, ((L.wqkv, L.bqkv, "bias"), (L.wo, None if fuse_o else L.bo, "enc_residual" if fuse_o else "bias"),
-                                                (L.w1, L.b1, "bias_gelu"),
-                                                (L.w2, None if fuse_f else L.b2, "enc_residual" if fuse_f else "bias")))
+            projections = ((L.wqkv, L.bqkv, "bias"), (L.wo, None if fuse_o else L.bo, "enc_residual" if fuse_o else "bias"),
+                           (L.w1, L.b1, "bias_gelu"), (L.w2, None if fuse_f else L.b2, "enc_residual" if fuse_f else "bias"))
+            gemm_plan.choose_encoder(x, projections)
+            cores = gemm_plan.encoder_cores(T, projections)
             y = None if cores is None else ops.encoder_layers(x, [t for L in self.layers for t in _layer_tensors(L)], cu, max_len, H, Dh,
                                                               self.scale, c.ln_eps, cores, fuse_o, fuse_f)
             if y is not None:

@@ -335,10 +335,28 @@ def _pick(key, runs, x: torch.Tensor) -> str:
     lead = 1.0 if key[-1] == "bias_gelu" else G8_LEAD
     if "g8" in t and t["g8"] > lead * min(t[n] for n in t if n != "g8"):
         t = {n: v for n, v in t.items() if n != "g8"}
-    own = min((n for n in t if n != "blas"), key=lambda n: t[n], default="blas")
-    # (a tie goes to the own core, whose layers are launched from native code: bge-large on 7156 tokens with qkv at 52 us on the
-    # library and 53 on gemm2w: 6.31 ms with the library's, 6.08 with gemm2w's)
-    return own if t[own] <= t["blas"] * (1.03 + OWN_MARGIN) else "blas"
+    # (a tie goes to an own core that is launched from native code: bge-large on 7156 tokens with qkv at 52 us on the library and 53 on
+    # gemm2w: 6.31 ms with the library's, 6.08 with gemm2w's.  Where the layer is not launched so, choose_encoder takes it back)
+    return min((n for n in t if n != "blas" and t[n] <= t["blas"] * ((1.03 if n in _ENC_NATIVE else 1.0) + OWN_MARGIN)),
+               key=lambda n: t[n], default="blas")
+
+
+def choose_encoder(x: torch.Tensor, projections) -> None:
+    """Choose the cores of an encoder layer's projections (as :func:`encoder_cores` takes them) for rows like ``x`` before the first
+    of them runs, each by its time; a core that is no faster than the library is kept only if all four are launched from native code, or
+    for its exact GELU."""
+    keys = [(_m_bucket(x.shape[0]), *w.shape, epi) for w, _, epi in projections]
+    if MODE in ENC_BACKENDS or all(k in _CHOICE for k in keys) or not x.is_cuda or torch.cuda.is_current_stream_capturing():
+        return
+    y = x
+    for i, (w, b, epi) in enumerate(projections):
+        a = y if i == 3 else x   # (down reads what up gives)
+        y = linear_residual_(a, w, x.clone()) if b is None else linear_bias(a, w, b, gelu=epi == "bias_gelu")
+    if not all(_CHOICE[k] in _ENC_NATIVE for k in keys):
+        for k in keys:
+            t = TIMINGS.get(k)
+            if t and k[-1] != "bias_gelu" and t.get(_CHOICE[k], 0) > t["blas"] * (1 + OWN_MARGIN):
+                _CHOICE[k] = "blas"
 
 
 def linear_residual_(x: torch.Tensor, w: torch.Tensor, acc: torch.Tensor, ws=None) -> torch.Tensor:

@@ -150,6 +150,43 @@ def test_encoder_layers_on_gemm8p_launched_natively(gpu, monkeypatch, fused):
     assert torch.equal(y, m.forward_packed(*args))
 
 
+@pytest.mark.parametrize("down,choices", [(150, ["g2", "g2", "g2", "g2"]),       # all native: the ties keep their cores
+                                          (90, ["blas", "g2", "g2", "blas"])])    # the library for one: what is faster than it, and the exact GELU
+def test_encoder_ties_go_to_native_layers_alone(gpu, monkeypatch, down, choices):
+    """A core that is no faster than the library is taken where the whole layer is launched from native code, and nowhere else; all are
+    chosen before the first projection runs, so that the first pass gives the later ones' bits."""
+    from llm_weighted_consensus_amd import ops
+    from llm_weighted_consensus_amd.models.bert import BertEncoder
+    from llm_weighted_consensus_amd.models.config import encoder_config
+    from llm_weighted_consensus_amd.ops import gemm_plan
+
+    m = BertEncoder(encoder_config("bge-small-en-v1.5"), device=gpu, seed=5)
+    m.fused_residual = "ffn2"
+    args = m.pack([[(7 * i + j) % 900 + 1 for j in range(n)] for i, n in enumerate([300, 2, 64, 129])])
+    for d in ("_CHOICE", "TIMINGS"):
+        monkeypatch.setattr(gemm_plan, d, {})
+    blas = {1152: 100, 384: 120, 1536: 100}
+    picked = gemm_plan._pick
+
+    def pick(key, runs, x):
+        lib = down if key[3] == "enc_residual" else blas[key[1]]
+        for f in runs.values():
+            f()
+        times = {n: lambda: 102 for n in runs} | {"blas": lambda: lib}
+        return picked(key, times, x)
+    monkeypatch.setattr(gemm_plan, "_pick", pick)
+    monkeypatch.setattr(gemm_plan, "_time_between", lambda fn, x: fn())
+    monkeypatch.setattr(gemm_plan, "EXCLUDE", gemm_plan.EXCLUDE | {"g8", "gv"})
+    native, run = [], ops.encoder_layers
+    monkeypatch.setattr(ops, "encoder_layers", lambda *a: native.append(1) or run(*a))
+    first = m.forward_packed(*args)
+    L = m.layers[0]
+    got = [gemm_plan._CHOICE[(gemm_plan._m_bucket(args[0].shape[0]), *w.shape, e)]
+           for w, e in ((L.wqkv, "bias"), (L.wo, "bias"), (L.w1, "bias_gelu"), (L.w2, "enc_residual"))]
+    assert got == choices and len(native) == (down == 150)
+    assert torch.equal(first, m.forward_packed(*args))
+
+
 @pytest.mark.parametrize("core,lens", [("gv", [5, 1, 40]), ("g2", [5, 1, 40]), ("g2", [300, 2, 64, 129])])
 @pytest.mark.parametrize("fused", ["0", "ffn2", "all"])
 def test_encoder_layers_launched_natively(gpu, monkeypatch, core, lens, fused):
