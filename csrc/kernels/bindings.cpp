@@ -897,14 +897,16 @@ std::pair<int64_t, int64_t> prefill_plan(int64_t nseq, int64_t rows, int64_t max
 // The layers of a post-norm encoder over packed rows x [T, d], launched from here: a forward of few rows is bound by the
 // host's launches (12 layers of 7 kernels, from Python 6.3 us each: bge-small, 12 tokens 565 us a call, 399 so).
 // weights: 12 tensors a layer (qkv, its bias, o, its bias, norm 1 gain and bias, FFN up and bias, FFN down and bias, norm 2
-// gain and bias).  cores: the planner's choice for qkv, o, up, down (1 skinny_gemm, 2 gemm2w).  fuse_o / fuse_f: the
-// projection adds into x in its epilogue and its bias enters the norm.  Returns the last hidden rows; nothing, and nothing
-// launched, if a layer's weights are not laid out as these cores read them (the caller's own loop takes any).
+// gain and bias).  cores: the planner's choice for qkv, o, up, down (1 skinny_gemm, 2 gemm2w, 3 gemm8p over the
+// workspace part and count).  fuse_o / fuse_f: the projection adds into x in its epilogue and its bias enters the norm.  Returns the
+// last hidden rows; nothing, and nothing launched, if a layer's weights are not laid out as these cores read them or core 3 has no
+// workspace (the caller's own loop takes any).
 c10::optional<at::Tensor> encoder_layers(at::Tensor x, const std::vector<at::Tensor>& weights, const at::Tensor& cu, int64_t max_len,
                           int64_t H, int64_t Dh, double scale, double eps, const std::vector<int64_t>& cores, bool fuse_o,
                           bool fuse_f, const c10::optional<at::Tensor>& part, const c10::optional<at::Tensor>& count) {
   CHECK_BF16(x); CHECK_CONTIG(x);
   TORCH_CHECK(x.dim() == 2 && weights.size() % 12 == 0 && !weights.empty() && cores.size() == 4, "encoder_layers: arguments");
+  for (int64_t c : cores) TORCH_CHECK(c >= 1 && c <= 3, "encoder_layers: cores are 1 to 3, not ", c);
   const int64_t T = x.size(0), d = x.size(1), f = weights[6].size(0);
   TORCH_CHECK(H * Dh == d && (d <= 1024 || !(fuse_o || fuse_f)), "encoder_layers: head shape or fused rows");
   for (size_t i = 0; i < weights.size(); ++i) {

@@ -150,6 +150,20 @@ def test_encoder_layers_on_gemm8p_launched_natively(gpu, monkeypatch, fused):
     assert torch.equal(y, m.forward_packed(*args))
 
 
+@pytest.mark.parametrize("core", [0, 4, -1])
+def test_encoder_layers_refuse_other_cores(gpu, core):
+    """A core that no kernel stands for is an error, not gemm2w."""
+    from llm_weighted_consensus_amd import ops
+
+    d, f = 64, 256
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=gpu)  # noqa: E731
+    weights = [z(3 * d, d), z(3 * d), z(d, d), z(d), z(d), z(d), z(f, d), z(f), z(d, f), z(d), z(d), z(d)]
+    cu = torch.tensor([0, 5], dtype=torch.int32, device=gpu)
+    assert ops.encoder_layers(z(5, d), weights, cu, 5, 2, 32, 0.2, 1e-6, [2, 2, 2, 3], False, False).shape == (5, d)
+    with pytest.raises(RuntimeError, match="cores are 1 to 3"):
+        ops.encoder_layers(z(5, d), weights, cu, 5, 2, 32, 0.2, 1e-6, [2, core, 2, 2], False, False)
+
+
 @pytest.mark.parametrize("down,choices", [(150, ["g2", "g2", "g2", "g2"]),       # all native: the ties keep their cores
                                           (90, ["blas", "g2", "g2", "blas"])])    # the library for one: what is faster than it, and the exact GELU
 def test_encoder_ties_go_to_native_layers_alone(gpu, monkeypatch, down, choices):
