@@ -57,6 +57,7 @@ int lwc_silu_mul_quant_fp8(const void*, int, int, int, void*, float*, hipStream_
 int lwc_prefill_attention(const void*, const void*, const void*, void*, const int*, const int*, int, int, int, int, int, int, int, int,
                           int, int, float, int, hipStream_t);
 void lwc_prefill_plan(int, int, int, int, int, int, int*, int*);
+int lwc_gemm2s_rows(int, int, int, int);
 int lwc_prefill_attention_mx(const void*, const void*, const void*, void*, void*, int, const int*, int, int, int, int, int,
                              int, int, int, int, float, int, hipStream_t);
 int lwc_prefill_attention_paged(const void*, const void*, const void*, void*, const int*, const int*, const int*, int, int, int,
@@ -1223,6 +1224,18 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         "B*Hkv*splits threshold of the wave-per-item decode kernel; returns the previous value");
   m.def("prefill_attention", &prefill_attention);
   m.def("prefill_plan", &prefill_plan);
+  // the tile (4: the weight streams) and the K ranges of a gemm2w call by the sizes; rows of a tile of a grouped bf16 call on gemm2s.hip's
+  // weight streams, 0 for one on gemm2g.hip's small tiles
+  m.def("gemm2w_plan", [](int M, int N, int K, int epi, bool norm, int64_t max_splits) {
+    TORCH_CHECK(M > 0 && N > 0 && K > 0 && epi >= 0 && epi <= 5, "gemm2w_plan: sizes");
+    int tile = 0, splits = 0;
+    lwc_gemm2w_plan(M, N, K, epi, norm, max_splits, &tile, &splits);
+    return std::make_pair(tile, splits);
+  });
+  m.def("gemm2s_rows", [](int rows, int G, int N, int K) {
+    TORCH_CHECK(rows > 0 && G > 0 && N > 0 && K > 0 && K <= INT_MAX / 2, "gemm2s_rows: sizes");
+    return lwc_gemm2s_rows(rows, G, N, 2 * K);
+  });
   m.def("encoder_few", &encoder_few, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("encoder_layers", &encoder_layers, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("prefill_attention_mx", &prefill_attention_mx);

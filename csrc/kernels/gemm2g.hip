@@ -265,6 +265,20 @@ int launch(Params p, int rows, hipStream_t s) {
 
 extern "C" int lwc_gemm2s(const void*, const void*, void*, const int*, const int*, int, int, int, int, int, int, int, int, hipStream_t);
 
+// bf16 weights whose rows lie 8 KiB or a multiple apart, as many tiles of 256 columns as fill their rounds of 256 CUs: gemm2s.hip's
+// weight streams.  us, here / there, uneven groups, N x K x groups of 3 / 16 / 40 / 100 rows: 14336 x 4096 x 8 (1.75 rounds) 184 /
+// 153, 195 / 162, 196 / 171, 208 / 207; 4096 x 4096 x 32 (2) 213 / 189, 210 / 187, 215 / 201, 239 / 316; 28672 x 8192 x 2 (0.88) 211 / 168, 208 /
+// 167, 203 / 184, 207 / 235; 28672 x 4096 x 8 (3.5) 365 / 355, 361 / 358, 372 / 376, 388 / 440; 3072 x 4096 x 64 (3) 296 / 278, 304 / 307, 316
+// / 314; but 22016 x 4096 x 4 (1.34) 150 / 161, and with other K 8192 x 7168 x 8 159 / 159, 4096 x 7168 x 8 (0.5) 71 / 95, 5632 x 2048 x
+// 64 262 / 288
+// Rows of a tile there, 0 for the small tiles (K in bytes).
+extern "C" int lwc_gemm2s_rows(int rows, int G, int N, int K) {
+  const int per = (rows + G - 1) / G;
+  const long long wide = (long long)((N + 255) / 256) * G, rounds = (wide + 255) / 256;
+  if (K % 8192 != 0 || per > 48 || 20 * wide < 17 * 256 * rounds) return 0;
+  return per > 16 ? 192 : 64;
+}
+
 // The operands of lwc_gemm8g_fp8 (checked there), row_off null for a dense call, or of lwc_gemm8g_bf16 (K and lda in bytes);
 // mode 3: A carries MX scales; 4, 5: bf16.  rows: all groups' rows.
 extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_off, const int* a_rows,
@@ -295,17 +309,11 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
   const long long nj = (nt + 7) / 8, groups = std::min<long long>(G, (64 + nj - 1) / nj);
   p.turned = mode != kBf16 && mode != kBf16Swiglu && (K % 4096 == 0 || K % 2048 != 0) &&
              ((groups * per * K <= 4 << 20 && per <= (K <= 4096 ? 160 : 144)) || (row_off && cols <= 256 && per <= 192));
-  // bf16 weights whose rows lie 8 KiB or a multiple apart, as many tiles of 256 columns as fill their rounds of 256 CUs: gemm2s.hip's
-  // weight streams.  us, here / there, uneven groups, N x K x groups of 3 / 16 / 40 / 100 rows: 14336 x 4096 x 8 (1.75 rounds) 184 /
-  // 153, 195 / 162, 196 / 171, 208 / 207; 4096 x 4096 x 32 (2) 213 / 189, 210 / 187, 215 / 201, 239 / 316; 28672 x 8192 x 2 (0.88) 211 / 168, 208 /
-  // 167, 203 / 184, 207 / 235; 28672 x 4096 x 8 (3.5) 365 / 355, 361 / 358, 372 / 376, 388 / 440; 3072 x 4096 x 64 (3) 296 / 278, 304 / 307, 316
-  // / 314; but 22016 x 4096 x 4 (1.34) 150 / 161, and with other K 8192 x 7168 x 8 159 / 159, 4096 x 7168 x 8 (0.5) 71 / 95, 5632 x 2048 x
-  // 64 262 / 288
-  const long long wide = (N + 255) / 256 * G, rounds = (wide + 255) / 256;
-  if ((mode == kBf16 || mode == kBf16Swiglu) && row_off && K % 8192 == 0 && per <= 48 && 20 * wide >= 17 * 256 * rounds) {
-    const int rc = lwc_gemm2s(A, W, C, row_off, a_rows, G, N, K, lda, ldc, rows_a, mode == kBf16Swiglu, per > 16 ? 192 : 64, s);
-    if (rc != -1) return rc;
-  }
+  if ((mode == kBf16 || mode == kBf16Swiglu) && row_off)
+    if (const int rt = lwc_gemm2s_rows(rows, G, N, K)) {
+      const int rc = lwc_gemm2s(A, W, C, row_off, a_rows, G, N, K, lda, ldc, rows_a, mode == kBf16Swiglu, rt, s);
+      if (rc != -1) return rc;
+    }
   int tm = per <= (cols <= 128 ? 44 : 16) ? 64 : per <= 104 && !(cols > 128 && cols <= 256) ? 128 : 192;
   if (!row_off) tm = nt * ((rows + 63) / 64) <= 512 ? 64 : 128;
 #define LWC_G2G(M) \
