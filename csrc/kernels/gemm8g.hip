@@ -14,8 +14,8 @@
 //   * MFMA: the block-scaled mfma_scale_f32_16x16x128_f8f6f4 with unit e8m0 scales: a lane's two 16 B
 //     fragments (k-chunks q and 4+q of the 128-byte slice) form one 32-byte operand, so a phase issues
 //     16 MFMAs of twice the bf16 cycle count — the same MFMA cycles per phase as gemm8p at 2x the FLOPs;
-//   * A rows: per-lane DMA source offsets from a_rows (rows past the group's end load a valid row of
-//     the group and are masked at the store); W: the group's [N, K] slab through its own descriptor;
+//   * A rows: per-lane DMA source offsets from a_rows (rows past the group's end are not loaded and are
+//     masked at the store); W: the group's [N, K] slab through its own descriptor;
 //   * epilogue: a lane holds eight consecutive columns of eight rows: eight activation scales and 16 channel scales
 //     instead of 32 and 4, no LDS, 16 B stores (rows < the group's end only).
 // Measured against four phases of half the MFMAs with the wait for their reads behind the barrier and an epilogue through LDS, us:
@@ -54,7 +54,7 @@ struct Params {
   int slots, n_tiles;     // m-tile slots per n-tile, n-tiles
   int rows_c;             // output rows when row_off is null (dense: G = 1)
   int gn;                 // grouped: n-tiles an XCD walks per m-slot before the next slot (>= 1)
-  int skip_empty;         // skip the MFMAs of empty 64-row blocks (LWC_G8G_SKIP=0: A/B off)
+  int skip_empty;         // skip the MFMAs of empty 64-row blocks (skips_empty)
   // MX activations (kMxOut producer / kMxA consumer): e8m0 block scales [K / 128][s_rows][4] bytes, block b
   // of a 128-byte K slice = its bytes [32b, 32b + 32).  (The block-scaled MFMA takes a lane's two 16-byte
   // fragments as K [16q, 16q + 16) and [64 + 16q, ...) of its 128 and scales K block b by the byte lane
@@ -154,10 +154,9 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      int r = m_begin + i * 128 + h * 64 + (tid >> 3);
-      if (r >= m_end) r = m_begin;  // a valid row of the group; its outputs are never stored
-      const int src = p.a_rows ? p.a_rows[r] : r;
-      voA[h][i] = (uint32_t)(src * p.lda + chkA);
+      const int r = m_begin + i * 128 + h * 64 + (tid >> 3);
+      // (past the group's end: past the resource's, zeros and no memory request)
+      voA[h][i] = r < m_end ? (uint32_t)((p.a_rows ? p.a_rows[r] : r) * p.lda + chkA) : 0x7fffffffu;
       voW[h][i] = (uint32_t)(((2 * i + (tid >> 8)) * 64 + h * 32 + ((tid >> 3) & 31)) * p.K + chkW);
     }
   const int dst_lane0 = wid * 64 * 16;
@@ -237,7 +236,7 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
 #define G8_BAR() __builtin_amdgcn_s_barrier()
 #define G8_VM(N) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory")
   // rows of this wave row that hold data (wave-uniform): a ragged last tile of an expert (on average half of
-  // it) skips the MFMAs of its empty 64-row blocks — the barriers, LDS reads and DMA stay, so the two wave
+  // it) may skip the MFMAs of its empty 64-row blocks — the barriers, LDS reads and DMA stay, so the two wave
   // rows keep their schedule
   const int live = p.skip_empty ? __builtin_amdgcn_readfirstlane(m_end - m_begin - wr * 128) : 256;
 #define G8_MFMA(i0)                                  \
@@ -342,6 +341,18 @@ __global__ void __launch_bounds__(512) gemm8g_kernel(Params p) {
 extern "C" int lwc_gemm2g(const void*, const void*, void*, const int*, const int*, const float*, const float*, int, int, int, int,
                               int, int, int, int, const void*, void*, int, hipStream_t);
 
+// Whether a group's last tile skips the MFMAs of its empty rows.  Where it does it walks K ahead of the tile that shares its weights, and
+// where nearly every group has a nearly empty tile beside a full one, its part of the weights comes from memory twice: groups of 300 rows,
+// MB fetched skipping / not (and as four phases per K tile, whose barriers held the lead back): bf16 [1536, 2048] x 64 1070 / 864 (905), [4096, 14336]
+// x 8 2320 / 2275 (2010).  us, skipping / not (and in four phases), 258 to 340 rows a group, bf16 [4096, 14336] x 8 362 to 369 / 328 to 334 (345 to
+// 352), [4096, 7168] x 8 177 to 181 / 167 to 171 (167 to 176), [2048, 2048] x 32 118 to 126 / 110 to 115 (107 to 116), [1536, 2048] x 64 227 to 242 / 216
+// to 227 (205 to 220), fp8 [4096, 14336] x 8 180 to 182 / 171 to 174 (170 to 175); the SwiGLU's of short K: [3072, 2048] x 32 198 / 192 (191), [1536,
+// 2048] x 64 220 / 207 (200).  But SwiGLU [14336, 4096] x 8 330 / 350, fp8 [28672, 4096] x 8 345 / 361; from 400 rows on level, and for uneven groups of 400 on
+// average [4096, 14336] x 8 516 / 542; K 768 112 / 114.
+static int skips_empty(long long rows, int G, int K, bool swiglu, bool bf16) {
+  return rows <= 256LL * G || rows > 384LL * G || K <= 2048 || (swiglu && !(bf16 && K <= 4096));
+}
+
 // Whether the weights bound a grouped fp8 call, and gemm2g.hip takes it: rows per group on average, and cols, its columns of
 // 128 in all groups (one workgroup each, two of them a CU: 512 in a round).  us, 8-phase / gemm2g, equal groups (8-phase: this kernel, before its two phases per K tile):
 // Up to 256 columns every CU has one workgroup or none there, and half as many here: from MX [4096, 14336] x 8 at 128 rows 153
@@ -403,7 +414,7 @@ extern "C" int lwc_gemm8g_fp8(const void* A, const void* W, void* C, const int* 
   const char* gv = getenv("LWC_G8G_GN");
   const int nj = (n_tiles + 7) / 8, gn = std::max(1, std::min(gv ? atoi(gv) : kDefaultGn, nj));
   Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, a_scale, w_scale,
-           G, N, K, lda, ldc, rows_a, max_slots, n_tiles, rows_c, gn, 1,
+           G, N, K, lda, ldc, rows_a, max_slots, n_tiles, rows_c, gn, row_off ? skips_empty(rows_c, G, K, swiglu, false) : 1,
            (const uint8_t*)a_mx, (uint8_t*)mx_out, s_rows};
   if (const char* sv = getenv("LWC_G8G_SKIP")) p.skip_empty = atoi(sv);
   // dense: 8 XCD ranges of ceil(tiles / 8) grouped tiles; grouped: per XCD, windows of gn n-tiles x
@@ -443,7 +454,7 @@ extern "C" int lwc_gemm8g_bf16(const void* A, const void* W, void* C, const int*
   }
   const int n_tiles = (N + 255) / 256, nj = (n_tiles + 7) / 8;
   Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, nullptr, nullptr,
-           G, N, K * 2, lda * 2, ldc, rows_a, max_slots, n_tiles, rows_c, nj, 1, nullptr, nullptr, 0};
+           G, N, K * 2, lda * 2, ldc, rows_a, max_slots, n_tiles, rows_c, nj, skips_empty(rows_c, G, K * 2, swiglu, true), nullptr, nullptr, 0};
   const unsigned grid = (unsigned)(nj * max_slots * 8);
   if (swiglu)
     gemm8g_kernel<kBf16Swiglu><<<grid, 512, kLdsB, s>>>(p);
