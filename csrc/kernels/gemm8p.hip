@@ -40,7 +40,7 @@
 //   The decode shapes do not divide into whole rounds of 256 tiles (qkv at M=3072: 288 tiles = 1.1 rounds;
 //   o / down: 192 = 0.75; gate_up: 1344 = 5.25), so a plain one-tile-per-workgroup grid idles 12-44 % of the
 //   chip in its last round.  Here the first `sk_tiles` tiles (the remainder plus one full round) are split
-//   by K iterations (stream-K; where that costs less than it saves, rest_cost): each XCD owns a contiguous, tile-aligned share of them and its wpx workgroups
+//   by K iterations (stream-K; where that costs less than it saves, call_cost): each XCD owns a contiguous, tile-aligned share of them and its wpx workgroups
 //   split that share's K iterations evenly.  The remaining tiles run data-parallel, one per workgroup per
 //   round, XCD x taking wpx consecutive tiles (m fastest: the XCD's tiles share W panels in its L2).
 //   A tile cut between workgroups is finished by the one holding its last K iteration (the finaliser),
@@ -446,35 +446,48 @@ int grid_wpx(int tiles, int KT) {
   return iters < 8LL * 8 * wpx ? (int)std::max(1LL, iters / 64) : wpx;
 }
 
-// What is lost beside the K iterations of `tiles` tiles on G workgroups, us (iter: one of a tile's KT): the tiles of a last
-// round that is not full are cut between all workgroups, or (cut: false) run as they are while the others idle (and the rest run
-// at a higher clock: three quarters of the idle time), whichever is less.  A cut costs its hand-off, 256 KiB through one compute
-// unit each way, and workgroups that walk K apart no longer share their rows' way through an XCD's L2.  Cut less uncut, us, by how
-// full the last round is: K 768 0.05 / 0.38 / 0.75 / 0.89 -3 / +3 / +9 / +10; K 2048 0.06 / 0.5 / 0.88 -18 / -7 / +29; K 4096 -46 /
-// -16 / +50; K 8192 -99 / -34 / +81; K 14336 0.25 / 0.88 -129 / +123; K 384 0.05 / 0.89 +2 / +8.  With fewer tiles than workgroups,
-// down 4096 x 14336 of 520 / 1095 / 1300 / 2200 / 3333 rows (5.3 / 3.2 / 2.7 / 1.8 / 1.1 workgroups a tile) lost 31 / 23 / 15 / 34 / 5.
-double rest_cost(int tiles, int G, int KT, double iter, bool* cut) {
-  const int rest = tiles % G;
-  const double full = (double)rest / G, idle = rest == 0 ? 0 : 0.75 * iter * KT * (1 - full);
-  const double split = rest == 0 ? 0 : tiles > G ? 6 + KT * (0.2 + 0.7 * std::max(0.0, full - 0.3))
-                                     : G % tiles == 0 ? 4.5 * G / tiles : 3 + 6.5 * G / tiles;
+// The time of `tiles` tiles on 8 x wpx workgroups, us, and whether those of a last round that is not full are cut between all
+// workgroups (or run as they are while the others idle), whichever is less.  R1: tiles of 256, 224 or 192 rows.
+//   With whole rounds, 256 rows are 1.45 us per K iteration and round, 224 0.93 and 192 0.85 of that (28672 x 4096 and 4096 x 14336).  A
+// round that is not full: the others run at a higher clock, three quarters of the idle time are lost.  A cut costs its hand-off, 256
+// KiB through one compute unit each way, and workgroups that walk K apart no longer share their rows' way through an XCD's L2.  Cut less
+// uncut, us, by how full the last round is: K 768 0.05 / 0.38 / 0.75 / 0.89 -3 / +3 / +9 / +10; K 2048 0.06 / 0.5 / 0.88 -18 / -7 / +29; K 4096
+// -46 / -16 / +50; K 8192 -99 / -34 / +81; K 14336 0.25 / 0.88 -129 / +123; K 384 0.05 / 0.89 +2 / +8.
+//   With fewer tiles than workgroups the times were fitted to 253 calls of 200 to 7156 rows, 384 to 8192 columns and K 256 to 14336, each with
+// every row tile, cut and uncut (rms 0.10 and 0.04): uncut a start, an end and the iterations, slower as more CUs run; cut the
+// iterations of the XCD that has the most tiles, a hand-off per workgroup of a tile, more where these do not divide a tile's K evenly
+// and for each tile of an XCD.  The choice is 1.008 of the best of the six on average, 1.12 at worst.  us, uncut / cut, 192 rows: 520 x 768 x 3072 (9 tiles)
+// 51 / 33, 200 x 2304 x 3072 (18) 52 / 36, 520 x 768 x 2048 38 / 28, 520 x 4096 x 14336 (48) 218 / 86; 1095 x 4096 x 1024 (96) 26 / 29, 2200 x
+// 3072 x 768 (144) 24 / 31.
+constexpr double kIter[5] = {0, 0, 1.45 * 0.85, 1.45 * 0.93, 1.45};
+constexpr double kUncut[5][3] = {{}, {}, {10.9, 0.83, 0.26}, {11.8, 0.86, 0.37}, {12.5, 0.88, 0.42}};
+constexpr double kCut[5][5] = {{}, {}, {2.8, 1.29, 3.8, 3.8, 0.42}, {1.7, 1.33, 4.8, 4.2, 0.61}, {0.7, 1.46, 5.2, 4.3, 0.71}};
+double call_cost(int tiles, int wpx, int KT, int r1, bool* cut) {
+  const int G = 8 * wpx, rest = tiles % G;
+  if (tiles < G) {
+    const double *u = kUncut[r1], *c = kCut[r1];
+    const int share = (tiles + 7) / 8;  // the most tiles of an XCD
+    const double uncut = u[0] + KT * (u[1] + u[2] * tiles / 256);
+    const double split = c[0] + c[1] * KT * share / wpx + c[2] * wpx / share + (wpx % share ? c[3] : 0) + c[4] * tiles / 8;
+    *cut = split < uncut;
+    return std::min(split, uncut);
+  }
+  const double full = (double)rest / G, idle = rest == 0 ? 0 : 0.75 * kIter[r1] * KT * (1 - full);
+  const double split = rest == 0 ? 0 : 6 + KT * (0.2 + 0.7 * std::max(0.0, full - 0.3));
   *cut = rest != 0 && split < idle;
-  return std::min(split, idle);
+  return 6 + kIter[r1] * KT * tiles / G + std::min(split, idle);
 }
 
-// The row tile (R1: 256, 224 or 192 rows).  256 rows are 1.45 us per K iteration and round, 224 0.93 and 192 0.85 of that
-// (28672 x 4096 and 4096 x 14336, whole rounds of tiles), so a smaller one pays where it saves rows past M (1095 rows are five
-// tiles either way) or fills the last round.  Measured, us, 256 / 224 / 192 rows: gate|up 28672 x 4096 of 520 / 1095 / 1700 / 3333 rows
-// 130 / 128 / 122, 207 / 203 / 243, 291 / 304 / 347, 555 / 585 / 662; down 4096 x 14336 of 900 / 1095 / 2200 rows 101 / 114 / 114,
-// 124 / 121 / 116, 216 / 207 / 215.
-constexpr double kIter[5] = {0, 0, 1.45 * 0.85, 1.45 * 0.93, 1.45};
+// The row tile (R1): a smaller one pays where it saves rows past M (1095 rows are five tiles either way) or fills the last round.
+// Measured, us, 256 / 224 / 192 rows: gate|up 28672 x 4096 of 520 / 1095 / 1700 / 3333 rows 130 / 128 / 122, 207 / 203 / 243, 291 / 304 / 347, 555 / 585 /
+// 662; down 4096 x 14336 of 900 / 1095 / 2200 rows 101 / 114 / 114, 124 / 121 / 116, 216 / 207 / 215.
 int row_tile(int M, int tiles_n, int KT) {
   int best = 4;
   double least = 0;
   for (int r1 = 4; r1 >= 2; --r1) {
     bool cut;
-    const int bm = 128 + 32 * r1, tiles = (M + bm - 1) / bm * tiles_n, G = 8 * grid_wpx(tiles, KT);
-    const double us = kIter[r1] * KT * tiles / G + rest_cost(tiles, G, KT, kIter[r1], &cut);
+    const int bm = 128 + 32 * r1, tiles = (M + bm - 1) / bm * tiles_n;
+    const double us = call_cost(tiles, grid_wpx(tiles, KT), KT, r1, &cut);
     if (r1 == 4 || us < least) best = r1, least = us;
   }
   return best;
@@ -501,7 +514,7 @@ extern "C" int lwc_gemm8p(const void* A, const void* W, void* C, const void* R, 
   const int tiles_n = (N + 255) / 256, KT = K / 64, r1 = lda < (1 << 20) ? row_tile(M, tiles_n, KT) : 4;
   const int bm = 128 + 32 * r1, tiles_m = (M + bm - 1) / bm, tiles = tiles_m * tiles_n, wpx = grid_wpx(tiles, KT), G = 8 * wpx;
   bool cut;
-  rest_cost(tiles, G, KT, kIter[r1], &cut);
+  call_cost(tiles, wpx, KT, r1, &cut);
   const int dp = cut ? std::max(0, tiles / G - 1) : (tiles + G - 1) / G, sk = cut ? tiles - dp * G : 0;
   Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, ws, flags,
            M, N, K, lda, ldc, tiles_m, tiles_n, KT, std::max(1, env_int("LWC_G8_GM", 8)), wpx, sk, dp,

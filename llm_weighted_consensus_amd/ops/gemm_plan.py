@@ -83,7 +83,7 @@ def choice(M: int, N: int, K: int, epi: str) -> str:
 def _g8_fill(M: int, N: int, K: int) -> float:
     """How full gemm8p's rounds of 256 CUs are at a call's sizes: the product's share of a time in us per K iteration and round of
     256, 224 and 192 rows and for the hand-off of cut tiles.  The costs are those at which :func:`_untuned` was measured; the
-    kernel's own (``row_tile`` and ``rest_cost`` in csrc/kernels/gemm8p.hip) have fallen since, 0.79 to 1.0 of the time that these
+    kernel's own (``row_tile`` and ``call_cost`` in csrc/kernels/gemm8p.hip) have fallen since, 0.79 to 1.0 of the time that these
     give, so that the calls which they let pass are the faster for it."""
     KT, least = K // 64, float("inf")
     for bm, cost in ((256, 1.0), (224, 0.89), (192, 0.83)):
