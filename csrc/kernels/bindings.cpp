@@ -625,9 +625,9 @@ void rms_rowsumsq(const at::Tensor& x, at::Tensor& ss) {
            "rms_rowsumsq");
 }
 
-// grouped bf16 GEMM on the 8-phase schedule (gemm8g.hip): A [rows_a, K], W [G, N, K], C [rows, N] (swiglu: [rows, N / 2],
+// grouped bf16 GEMM in 256-row tiles (gemm8g.hip): A [rows_a, K], W [G, N, K], C [rows, N] (swiglu: [rows, N / 2],
 // W's rows gate / up interleaved in blocks of 32); row_off [G + 1] int32 and a_rows [rows] int32 on the device.  core: 2
-// gemm2g.hip's kernel, 8 the 8-phase one (gemm8g_fp8: also 0, the one that the sizes call for).
+// gemm2g.hip's kernel, 8 the 256-row one (gemm8g_fp8: also 0, the one that the sizes call for).
 void gemm8g_bf16(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const at::Tensor& row_off, int64_t max_slots,
                  const c10::optional<at::Tensor>& a_rows, bool swiglu, int64_t core) {
   CHECK_GPU(A); CHECK_GPU(W); CHECK_GPU(C); CHECK_BF16(A); CHECK_BF16(W); CHECK_BF16(C); CHECK_CONTIG(W);
@@ -656,7 +656,7 @@ void gemm8g_fp8(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c
                 int64_t max_slots, const c10::optional<at::Tensor>& a_rows, const c10::optional<at::Tensor>& a_scale,
                 const at::Tensor& w_scale, int64_t mode, const c10::optional<at::Tensor>& a_mx,
                 const c10::optional<at::Tensor>& mx_out, int64_t core) {
-  // grouped fp8 GEMM on the 8-phase schedule (gemm8g.hip): A [rows_a, K] e4m3, W [G, N, K] e4m3, C [rows, N] bf16;
+  // grouped fp8 GEMM in 256-row tiles (gemm8g.hip): A [rows_a, K] e4m3, W [G, N, K] e4m3, C [rows, N] bf16;
   // row_off None: the dense projection (G = 1, every output row).  mode 1: SwiGLU epilogue, C [rows, N / 2] bf16;
   // mode 2: SwiGLU epilogue with MX output, C [rows, N / 2] e4m3 + mx_out [N / 256, rows, 4] e8m0 (uint8);
   // a_mx [K / 128, rows_a, 4] e8m0: A's MX block scales (mode 0, no a_rows; a_scale unused)

@@ -10,8 +10,8 @@
 // More steps in flight for calls that give a CU one workgroup (six, five, four) gain nothing and cost dear where a second round
 // follows, us, so / here: fp8, 8 experts of 16 rows [4096, 8192] (256 workgroups) 66 / 65, [4608, 8192] (288) 89 / 77; dense
 // 700 rows x 6144 x 4096 (288) 50 / 31.
-// Measured, 8 experts, us, 256-row kernel (before its two phases per K tile) -> here ([28672, 4096] SwiGLU to MX, [4096, 14336] from MX; 154 and 77 at the rate of
-// a plain read): 4 rows an expert 257 -> 182, 144 -> 81; 32 rows 259 -> 189, 145 -> 84; 64 rows 264 -> 200, 150 -> 90; 128 rows
+// Measured, 8 experts, us, 256-row kernel (in four phases per K tile; in its two some 6 % less) -> here ([28672, 4096] SwiGLU to MX, [4096, 14336] from MX; 154
+// and 77 at the rate of a plain read): 4 rows an expert 257 -> 182, 144 -> 81; 32 rows 259 -> 189, 145 -> 84; 64 rows 264 -> 200, 150 -> 90; 128 rows
 // 270 -> 217, 155 -> 115.  Dense calls of few tiles likewise: 512 rows x 4096 x K 4096 from MX 45 -> 21.
 // bf16, 8 experts of 16 rows: [14336, 4096] 194 (the 128-row kernel with split K, its clear and its conversion 204), [4096, 7168] 82
 // (103).
@@ -292,7 +292,7 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
   // columns give every CU a workgroup already some CUs walk K once more.  us at 64 / 128 / 192 rows a tile, 32 rows a group: bf16
   // [4096, 14336] x 8 (256 columns) 164 / 166 / 172, one expert with four times the rows 238 / 190 / 193, with 130 rows 254 /
   // 292 / 193; two workgroups a CU, fp8 [4096, 6400] x 16 (512) at 40 rows 79 / 80 / 80, one with twice the rows 96 / 82 / 82
-  // (8-phase 86).  Fewer columns, where a second tile finds an idle CU: fp8 [2048, 7168] x 8 (128) at 40 rows 34 / 40 / 44, twice
+  // (256-row kernel 86).  Fewer columns, where a second tile finds an idle CU: fp8 [2048, 7168] x 8 (128) at 40 rows 34 / 40 / 44, twice
   // 34 / 42 / 46.  More, where it is one of many: bf16 [14336, 4096] x 8 (896) 204 / 203 / 205, four times 190 / 193 / 202.
   // Dense (no table): tiles of 64 rows while they give a CU two workgroups at most, else of 128.
   const int per = (rows + G - 1) / G;

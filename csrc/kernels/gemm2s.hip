@@ -9,8 +9,9 @@
 // in flight.  Rows past the group's end are neither loaded nor multiplied.  LDS layout, operand order and the order of sums are
 // gemm2g's: the same bits.
 // Measured, gemm2g -> here, us: 8 experts of 16 / 64 rows [14336, 4096] 199 / 206 -> 162 / 175, of 106 to 143 227 -> 192, [28672, 4096] of
-// 16 365 -> 355; with as many columns as give a workgroup half a tile, [4096, 7168] 82 -> 104.  fp8 rows, whose walk over K may
-// start anywhere, gain nothing: [28672, 4096] of 16 / 128 rows 158 / 201 in gemm2g, 187 / 212 so.
+// 16 365 -> 355; with as many columns as give a workgroup half a tile, [4096, 7168] 82 -> 104.  Those are calls in a row; in a routed
+// decode step of 64 requests, behind other kernels, [14336, 4096] x 8 takes 191 to 203, gemm2g 207 to 214.  fp8 rows, whose walk
+// over K may start anywhere, gain nothing: [28672, 4096] of 16 / 128 rows 158 / 201 in gemm2g, 187 / 212 so.
 #include <algorithm>
 
 #include "common.h"

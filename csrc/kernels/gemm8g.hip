@@ -354,16 +354,16 @@ static int skips_empty(long long rows, int G, int K, bool swiglu, bool bf16) {
 }
 
 // Whether the weights bound a grouped fp8 call, and gemm2g.hip takes it: rows per group on average, and cols, its columns of
-// 128 in all groups (one workgroup each, two of them a CU: 512 in a round).  us, 8-phase / gemm2g, equal groups (8-phase: this kernel, before its two phases per K tile):
-// Up to 256 columns every CU has one workgroup or none there, and half as many here: from MX [4096, 14336] x 8 at 128 rows 153
-// / 107, 144 rows 156 / 113; [2048, 7168] x 8 at 144 rows 0.74.  Above 144 rows an uneven routing needs a second tile.
-// More of them without the SwiGLU (short K, or several rounds): [4096, 6400] x 16 (512) at 80 rows 88 / 86, at 112 rows from MX
-// 89 / 101; [2048, 1408] x 64 (1024) at 80 rows 66 / 63, at 144 rows from MX 74 / 104; [4096, 1536] x 128 (4096) at 32 rows
-// 268 / 251, at 64 rows 292 / 282 but with K 1408 1.01, at 100 rows 324 / 347.  Rows of a multiple of 16 KiB: 128 of them at
-// a time meet on fewer memory channels than 256 do: [6144, 16384] x 8 (384) at 32 rows 184 / 210, with K 14336 or 18432 0.87.
-// With the SwiGLU (K 2048 to 6144): [28672, 4096] x 8 (1792) at 128 rows 270 / 217, at 176 rows 0.85; one round not quite full,
-// x 2 (448): at 104 rows 56 to 67 / 58 to 62 by where the weights lie, at 176 rows 59 to 69 / 65 to 67; x 4 (896): at 144 rows
-// 118 / 117, at 176 rows 118 / 122.
+// 128 in all groups (one workgroup each, two of them a CU: 512 in a round).  The lines were laid when this kernel had four phases per K
+// tile; it has become 1 to 16 % faster since, which the figures say (us, here / gemm2g, equal groups), but the lines stand:
+// Up to 256 columns every CU has one workgroup or none there, and half as many here: from MX [4096, 14336] x 8 at 128 rows 142
+// / 117, 144 rows 143 / 114; [2048, 7168] x 8 at 144 rows 67 / 52.  Above 144 rows an uneven routing needs a second tile.
+// More of them without the SwiGLU (short K, or several rounds): [4096, 6400] x 16 (512) at 80 rows 86 / 87 (then 92 / 88), at 112 rows from MX
+// 90 / 103; [2048, 1408] x 64 (1024) at 80 rows 57 / 63 (63 / 63), at 144 rows from MX 71 / 98; [4096, 1536] x 128 (4096) at 32 rows
+// 229 / 230 (265 / 230), at 64 rows 261 / 283, at 100 rows 300 / 351.  Rows of a multiple of 16 KiB: 128 of them at
+// a time meet on fewer memory channels than 256 do: [6144, 16384] x 8 (384) at 32 rows 166 / 166 (177 / 166), with K 14336 or 18432 1.06 (0.89).
+// With the SwiGLU (K 2048 to 6144): [28672, 4096] x 8 (1792) at 128 rows 251 / 185, at 176 rows 257 / 225; one round not quite full,
+// x 2 (448): at 104 rows 63 / 49, at 176 rows 64 / 64; x 4 (896): at 144 rows 120 / 108, at 176 rows 122 / 130.
 static bool weight_bound(long long rows, int G, int N, int K, bool swiglu) {
   const long long cols = (long long)((N + 127) / 128) * G;
   long long most = swiglu ? 176 : 144;
@@ -373,8 +373,8 @@ static bool weight_bound(long long rows, int G, int N, int K, bool swiglu) {
   }
   return rows <= most * G;
 }
-// and the dense calls: up to this many 256 x 256 tiles.  us, 8-phase / gemm2g, K 4096: 512 rows x 4096 (32 tiles) 45 / 21, 2048 x
-// 4096 (128) 48 / 34, 256 x 28672 SwiGLU to MX (112) 51 / 43, 2048 x 6144 (192) 49 / 66, 512 x 28672 (224) 61 / 73
+// and the dense calls: up to this many 256 x 256 tiles.  us, here / gemm2g, K 4096: 512 rows x 4096 (32 tiles) 44 / 20, 2048 x
+// 4096 (128) 49 / 36, 256 x 28672 SwiGLU to MX (112) 52 / 44, 2048 x 6144 (192) 48 / 58, 512 x 28672 (224) 52 / 76
 constexpr long long kSmallTiles = 128;
 
 // Grouped fp8 GEMM in 256 x 256 tiles.  Requires K % 128 == 0, N % 8 == 0, lda / ldc % 16 == 0 (bytes

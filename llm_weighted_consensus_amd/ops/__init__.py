@@ -320,7 +320,7 @@ def grouped_gemm(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tensor, max_sl
     chosen so a small-M launch (MoE decode down projection: 8 experts x 32 column tiles) still puts
     ~4 workgroups on every CU.  That is the 128-row kernel's; by their sizes (bf16: :func:`_grouped_bf16`,
     fp8: :func:`_few_fp8`, from 32 rows per group on ``weight_bound`` in csrc/kernels/gemm8g.hip) calls run on tiles of 64 to
-    192 rows (csrc/kernels/gemm2g.hip) or the 8-phase 256-row tiles (csrc/kernels/gemm8g.hip) instead.
+    192 rows (csrc/kernels/gemm2g.hip) or on tiles of 256 rows (csrc/kernels/gemm8g.hip) instead.
     ``swiglu=True``: W's rows are gate / up interleaved in blocks of 32 (:func:`swiglu_interleave` per group)
     and the result is silu(gate) * up [rows, N/2] — from those two kernels' epilogues when one of them takes
     the batch, else GEMM + the SwiGLU pass.  ``a_mx`` [K/128, rows, 4] uint8: A carries MX block scales (from
@@ -341,7 +341,7 @@ def grouped_gemm(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tensor, max_sl
         return out
     few = rows < 32 * G and max_slots is None and _few_fp8(rows, G, N, K) and _few_fp8_layout(A, W, rows, N, K, out, a_rows, a_scale, w_scale)
     if _use_gemm8g(A, W, rows, G, N, K, bias, splits, out, few) and (not swiglu or N % 64 == 0):
-        # fp8 expert batches: of few rows per expert the small tiles, else the 8-phase kernel or the small tiles, by sizes
+        # fp8 expert batches: of few rows per expert the small tiles, else the 256-row kernel or the small tiles, by sizes
         if out is None:
             out = torch.empty(rows, N // 2 if swiglu else N, dtype=torch.bfloat16, device=A.device)
         kernels().gemm8g_fp8(A, W, out, row_off, -(-rows // 256) + G, a_rows, a_scale, w_scale.contiguous(),
@@ -363,7 +363,7 @@ def grouped_gemm(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tensor, max_sl
 
 
 # the experts' GEMMs, fp8 and bf16: auto (by sizes), classic (the 128 x 128 kernel, csrc/kernels/gemm.hip), g2 (gemm2g.hip) or
-# g8 (the 8-phase one, gemm8g.hip) at any row count; fp8 keeps its MX middle with all but classic
+# g8 (the 256-row one, gemm8g.hip) at any row count; fp8 keeps its MX middle with all but classic
 MOE_GEMM = os.environ.get("LWC_MOE_GEMM", "auto")
 
 
@@ -372,7 +372,7 @@ def _moe_core() -> int:
 
 
 # fp8 expert FFN middle in MX form (gate|up epilogue writes e4m3 + e8m0 block scales, the down GEMM's MFMAs
-# apply them): "1" (default) where both GEMMs take the 8-phase kernel or the small tiles, "0" = SwiGLU epilogue + row quantisation
+# apply them): "1" (default) where both GEMMs take the 256-row kernel or the small tiles, "0" = SwiGLU epilogue + row quantisation
 MOE_MX = os.environ.get("LWC_MOE_MX", "1") != "0"
 
 
@@ -393,7 +393,7 @@ def grouped_gemm_swiglu_mx(A: torch.Tensor, W: torch.Tensor, row_off: torch.Tens
 
 
 def moe_mx_ok(A: torch.Tensor, W13: torch.Tensor, W2: torch.Tensor, rows: int) -> bool:
-    """Whether the expert FFN runs its middle in MX form (both GEMMs on the 8-phase kernel or the small tiles)."""
+    """Whether the expert FFN runs its middle in MX form (both GEMMs on the 256-row kernel or the small tiles)."""
     if not MOE_MX or A.dtype != torch.float8_e4m3fn or W2.dtype != torch.float8_e4m3fn:
         return False
     G, N, K = W13.shape
@@ -427,7 +427,7 @@ def _few_fp8_layout(A, W, rows, N, K, out, a_rows, a_scale, w_scale) -> bool:
             and (out is None or (out.shape[0] == rows and out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0)))
 
 
-# rows per group (on average) from which bf16 groups take the small-tile and 8-phase kernels (csrc/kernels/gemm2g.hip,
+# rows per group (on average) from which bf16 groups take the small-tile and 256-row kernels (csrc/kernels/gemm2g.hip,
 # gemm8g.hip) by :func:`_grouped_bf16`; below, :func:`_few_bf16`
 GROUPED_BF16_ROWS = 4
 
@@ -448,12 +448,13 @@ def _few_bf16(rows: int, G: int, N: int, K: int) -> int:
 
 
 def _grouped_bf16(rows: int, G: int, N: int, K: int) -> int:
-    """The kernel of a bf16 call by its sizes: 0 the 128-row kernel, 2 the small tiles (gemm2g.hip), 8 the 8-phase one.
+    """The kernel of a bf16 call by its sizes: 0 the 128-row kernel, 2 the small tiles (gemm2g.hip), 8 the 256-row one (gemm8g.hip).
 
     us on one MI355X, equal groups, weights from memory, N x K x groups at rows per group (the SwiGLU adds 3 to 5 to the 128-row
-    kernel's, whose pass the others save); 128-row kernel / small tiles / 8-phase.  What each needs:
-    * the 8-phase kernel some 112 of its tiles: 4096 x 14336 x 8 at 400 rows (256) 740 / 629 / 318, 14336 x 4096 x 2 at 192
-      (112) 140 / 67 / 87, but 2048 x 7168 x 8 at 192 (64) 135 / 111 / 144, 4096 x 14336 x 2 at 256 (32) 137 / 199 / 281;
+    kernel's, whose pass the others save); 128-row kernel / small tiles / 256-row kernel (in two phases per K tile; the lines were laid when it
+    had four and took up to 7 % more).  What each needs:
+    * the 256-row kernel some 112 of its tiles: 4096 x 14336 x 8 at 400 rows (256) 740 / 592 / 351, 14336 x 4096 x 2 at 192
+      (112) 140 / 67 / 81, but 2048 x 7168 x 8 at 192 (64) 135 / 104 / 130, 4096 x 14336 x 2 at 256 (32) 137 / 199 / 262;
     * the small tiles, whose workgroups walk all of K, workgroups for half the CUs, and more the longer K is (the 128-row
       kernel splits K): 2048 x 7168 x 8 at 16 rows (128) 64 / 54, 14336 x 4096 x 2 (224) 65 / 49, but 4096 x 14336 x 4 (128) 109 / 118,
       x 2 (64) 65 / 96, 2048 x 7168 x 4 (64) 44 / 49; short K repays fewer: 512 x 1024 x 8 (32) 21 / 12;
@@ -473,7 +474,7 @@ def _grouped_bf16(rows: int, G: int, N: int, K: int) -> int:
 
 
 def _bf16_core(A, W, rows, G, N, K, bias, splits, out, a_rows) -> int:
-    """The kernel of a bf16 call (:func:`_grouped_bf16`, or as forced).  The small tiles and the 8-phase one want 16-byte rows
+    """The kernel of a bf16 call (:func:`_grouped_bf16`, or as forced).  The small tiles and the 256-row one want 16-byte rows
     that do not overlap (an expanded A has them all at one address, and the kernels' buffers end where ``rows * stride`` does)
     and 32-bit spans.  What else the 128-row kernel takes or refuses (output rows beyond A's, or fewer) stays with it; it does
     not take N off 16."""
@@ -901,7 +902,7 @@ class Fp8Weight:
         self.shape = tuple(w.shape)
 
 
-# dense fp8 projections (config 5): "auto" times the hand-written 8-phase fp8 core (gemm8g in dense mode)
+# dense fp8 projections (config 5): "auto" times the hand-written fp8 core (gemm8g in dense mode)
 # against hipBLASLt's row-scaled fp8 GEMM per (row bucket, N, K) on the first eager call and keeps the
 # hand-written one unless the library is faster by more than FP8_OWN_MARGIN; "g8g" / "blas" force one.
 FP8_GEMM = os.environ.get("LWC_FP8_GEMM", "auto")
@@ -926,7 +927,7 @@ G8G_SPAN = 1 << 31  # bytes of A one gemm8g launch may address (its buffer range
 
 def gemm8g_dense(xq: torch.Tensor, xs: torch.Tensor, w: "Fp8Weight", out: Optional[torch.Tensor] = None,
                  swiglu: bool = False):
-    """Dense fp8 GEMM on the hand-written 8-phase core (csrc/kernels/gemm8g.hip, G = 1, no row table):
+    """Dense fp8 GEMM on the hand-written 256-row core (csrc/kernels/gemm8g.hip, G = 1, no row table):
     (xq [M, K] e4m3 . w.q^T) * xs[row] * w.s[col] -> bf16 [M, N]; ``swiglu``: w's rows are gate|up interleaved
     in blocks of 32 (:func:`swiglu_interleave`) and the epilogue writes silu(gate) * up, bf16 [M, N / 2].
     The kernel addresses A through a 32-bit buffer range: row blocks of < 2 GiB of A go one launch each
@@ -951,7 +952,7 @@ def _fp8_blas(xq, xs, w):
 
 
 def linear_fp8_q(xq: torch.Tensor, xs: torch.Tensor, w: Fp8Weight) -> torch.Tensor:
-    """(e4m3 rows xq [M, K], row scales xs [M]) . w^T -> bf16 [M, N] (K6 fp8).  The hand-written 8-phase fp8
+    """(e4m3 rows xq [M, K], row scales xs [M]) . w^T -> bf16 [M, N] (K6 fp8).  The hand-written 256-row fp8
     core (:func:`gemm8g_dense`) or hipBLASLt's row-scaled fp8 GEMM (``torch._scaled_mm``), chosen per
     (row bucket, N, K) by timing (see FP8_GEMM); shapes the hand-written core does not take use the library."""
     if not _g8g_dense_ok(xq, w) or FP8_GEMM == "blas":

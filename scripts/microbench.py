@@ -130,7 +130,7 @@ def grouped(dev):
 
 
 def gemm8p_study(dev, Ms):
-    """8-phase 256x256 GEMM (csrc/kernels/gemm8p.hip) vs hipBLASLt, interleaved
+    """256x256-tile GEMM (csrc/kernels/gemm8p.hip) vs hipBLASLt, interleaved
     rounds in one process (median of 3), random operands; plus the fused SwiGLU epilogue against
     hipBLASLt gate_up + silu_mul."""
     from llm_weighted_consensus_amd import ops

@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """A/B of the fp8 MoE expert GEMMs (Mixtral-8x7B shapes, top-2 of 8 experts, random routing, A rows gathered
-like the model does): the 128x128 grouped kernel (gemm.hip) vs the 8-phase grouped kernel (gemm8g.hip),
+like the model does): the 128x128 grouped kernel (gemm.hip) vs the 256-row grouped kernel (gemm8g.hip),
 interleaved rounds in one process, median of 3.  TF/s = 2 * rows * N * K / time."""
 import os
 import sys

@@ -51,7 +51,7 @@ def _bf16(*shape):
 
 @pytest.mark.parametrize("form", ["expanded rows", "overlapping rows", "output beyond A", "fewer rows than A", "longer output", "no K"])
 def test_bf16_forms_that_stay_with_the_128_row_kernel(taken, form):
-    """Calls that the small-tile and 8-phase kernels answer differently from the 128-row kernel: A's rows at one address or
+    """Calls that the small-tile and 256-row kernels answer differently from the 128-row kernel: A's rows at one address or
     overlapping (their buffers would end early: zeros), and what they would refuse, or take though it was refused."""
     G, N, K, rows, out, kw = 4, 128, 128, 512, None, {}
     A = _bf16(rows, K)
