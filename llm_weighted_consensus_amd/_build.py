@@ -81,6 +81,11 @@ NO_PACKED_FP32 = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 for _f in ("attention_prefill.hip", "encoder_few.hip", "gemm8p.hip", "gemm8g.hip", "gemm2s.hip", "gemm1s.hip"):
     PER_FILE_FLAGS[_f] = PER_FILE_FLAGS.get(_f, []) + NO_PACKED_FP32
 
+# gemm8g's K loop (1140 to 1300 bytes an iteration) from the start of a line of the instruction cache: the same instructions
+# 8 / 16 / 0 bytes into one, us: dense fp8 8682 x 28672 x 4096 SwiGLU 760 / 768 / 748, x 4096 x 14336 426 / 433 / 421, x 6144 x 4096 196 / 199 / 194;
+# bf16 experts level
+PER_FILE_FLAGS["gemm8g.hip"].append("-falign-loops=64")
+
 
 def build_kernels(jobs: int = 8, force: bool = False) -> Path:
     """Compile every csrc/kernels/*.hip for gfx950 and link the torch extension."""
