@@ -18,7 +18,8 @@ int lwc_silu_mul(const void*, void*, int, int, int, hipStream_t);
 int lwc_embedding_gather(const void*, const int*, void*, int, int, int, hipStream_t);
 int lwc_encoder_few_ok(int, int, int, int);
 int lwc_encoder_few(const void*, const void*, const int*, const int*, int, int, const void*, const void*, float, const void* const*, int,
-                    const int*, int, int, int, int, int, float, float*, void*, void*, void*, void*, hipStream_t);
+                    const int*, int, int, int, int, int, float, void*, void*, hipStream_t);
+long long lwc_encoder_few_scratch(int, int, int);
 int lwc_embedding_step(const void*, const int*, void*, float*, int*, int, int, int, int, hipStream_t);
 int lwc_kv_block_copy(void*, const int*, int, int, int, long long, hipStream_t);
 int lwc_kv_gather(const void*, const void*, const long long*, void*, void*, int, int, int, int, hipStream_t);
@@ -974,12 +975,12 @@ c10::optional<at::Tensor> encoder_few(const at::Tensor& word, const at::Tensor& 
     if (!bf16(weights[i], sizes[i % 12])) return c10::nullopt;
     w[i] = weights[i].data_ptr();
   }
-  at::Tensor x = at::empty({T, d}, word.options()), a = at::empty({T, d}, word.options()), h = at::empty({T, f}, word.options());
-  at::Tensor part = at::empty({4, T, d}, word.options().dtype(at::kFloat)), y = at::empty({T, d}, word.options());
+  const int layers = (int)(w.size() / 12);
+  at::Tensor x = at::empty({T, d}, word.options());
+  at::Tensor scratch = at::empty({(int64_t)lwc_encoder_few_scratch(layers, (int)T, (int)d)}, word.options().dtype(at::kByte));
   CHECK_RC(lwc_encoder_few(word.data_ptr(), pos.data_ptr(), ids.data_ptr<int>(), positions.data_ptr<int>(), (int)word.size(0),
-                           (int)pos.size(0), g.data_ptr(), b.data_ptr(), (float)eps, w.data(), (int)(w.size() / 12), cu.data_ptr<int>(),
-                           (int)cu.size(0) - 1, (int)T, (int)d, (int)H, (int)f, (float)scale, part.data_ptr<float>(), x.data_ptr(),
-                           y.data_ptr(), a.data_ptr(), h.data_ptr(), cur_stream()),
+                           (int)pos.size(0), g.data_ptr(), b.data_ptr(), (float)eps, w.data(), layers, cu.data_ptr<int>(),
+                           (int)cu.size(0) - 1, (int)T, (int)d, (int)H, (int)f, (float)scale, x.data_ptr(), scratch.data_ptr(), cur_stream()),
            "encoder_few");
   return x;
 }

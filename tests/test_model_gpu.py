@@ -551,6 +551,62 @@ def test_few_row_encoder_keeps_infinities_to_their_text(gpu, monkeypatch, arch, 
             assert torch.isfinite(got[rows]).all() and (got[rows] - want[rows]).norm() < 0.02 * want[rows].norm(), few
 
 
+@pytest.mark.parametrize("arch,n", [("bge-small-en-v1.5", 14), ("bge-small-en-v1.5", 32), ("bge-base-en-v1.5", 9), ("bge-large-en-v1.5", 20)])
+def test_few_row_encoder_hands_on_what_this_call_made(gpu, arch, n):
+    """One launch holds the whole stack and its stages hand rows to each other through scratch memory that the next call gets
+    again: calls on other inputs, one after the other, on two streams at once and as a graph that is replayed on them, all
+    give the bits of a call by itself."""
+    from llm_weighted_consensus_amd.models import bert
+    from llm_weighted_consensus_amd.models.config import encoder_config
+
+    m = bert.BertEncoder(encoder_config(arch), device=gpu, seed=5)
+    inputs = [m.pack([[(37 * i + 11 * j + 50 * k) % 900 + 1 for j in range(n // 2)] for i in range(2)])[:3] for k in range(3)]
+    want = []
+    for a in inputs:
+        want.append(m.forward_packed(*a, n))
+        torch.cuda.synchronize()
+    assert not torch.equal(want[0], want[1])
+    got = [(k % 3, m.forward_packed(*inputs[k % 3], n)) for k in range(12)]
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for s in streams:
+        s.wait_stream(torch.cuda.current_stream())
+    for k in range(40):
+        with torch.cuda.stream(streams[k % 2]):
+            got.append((k % 3, m.forward_packed(*inputs[k % 3], n)))
+    torch.cuda.synchronize()
+    assert all(torch.equal(y, want[k]) for k, y in got)
+    ids = inputs[0][0].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = m.forward_packed(ids, *inputs[0][1:], n)
+    for k in (0, 1, 2, 1, 0):
+        ids.copy_(inputs[k][0])
+        graph.replay()
+        assert torch.equal(y, want[k])
+        m.forward_packed(*inputs[2], n)
+
+
+def test_few_row_encoder_of_more_layers_than_a_launch(gpu, monkeypatch):
+    """A stack of 26 layers is two launches: the second goes on from what the first left.  The bound as above."""
+    from dataclasses import replace
+
+    from llm_weighted_consensus_amd import ops
+    from llm_weighted_consensus_amd.models import bert
+    from llm_weighted_consensus_amd.models.config import encoder_config
+
+    m = bert.BertEncoder(replace(encoder_config("bge-small-en-v1.5"), layers=26), device=gpu, seed=5)
+    args = m.pack([[7, 9, 11, 13, 500], [3] * 6])
+    taken, few = [], ops.encoder_few
+    monkeypatch.setattr(ops, "encoder_few", lambda *a: taken.append(few(*a)) or taken[-1])
+    y = m.forward_packed(*args)
+    assert len(taken) == 1 and taken[0] is y
+    ref = m.forward_reference(*args[:3])
+    monkeypatch.setattr(bert, "FEW_ROWS", 0)
+    plain = m.forward_packed(*args)
+    err = lambda t: ((t.float() - ref).norm() / ref.norm()).item()  # noqa: E731
+    assert err(y) < 2 * err(plain) and err(y) < 0.03, (err(y), err(plain))
+
+
 # the core of each projection of a decode step (None: the library, with the norm and RoPE kernels in front of it)
 _STEP_CORES = {"gv": ["gv"] * 5, "g2": ["g2"] * 5, "library o and head": ["gv", None, "g2", "g2", None], "library qkv and down": [None, "gv", "g2", None, "gv"],
                "library gate|up": ["g2", "g2", None, "gv", "g2"]}
