@@ -32,6 +32,7 @@ int lwc_cascade_rows_per_tile(int);
 int lwc_grouped_gemm(const void*, const void*, void*, const int*, const float*, const float*, const void*, const int*,
                      int, int, int, int, int, int, long long, int, float*, int, long long, hipStream_t);
 int lwc_gemm8p(const void*, const void*, void*, const void*, float*, int*, int, int, int, int, int, int, hipStream_t);
+int lwc_gemm8p_fp8(const void*, const void*, void*, const float*, const float*, float*, int*, int, int, int, int, int, int, hipStream_t);
 int lwc_gemm8p_slots();
 void lwc_gemm2w_plan(int, int, int, int, bool, long long, int*, int*);
 int lwc_gemm2w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, int, float*, int*,
@@ -475,6 +476,37 @@ void gemm8p(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::
   CHECK_RC(lwc_gemm8p(A.data_ptr(), W.data_ptr(), C.data_ptr(), r, ws.data_ptr<float>(), flags.data_ptr<int>(), M, N,
                       K, (int)A.stride(0), (int)C.stride(0), (int)epi, cur_stream()),
            "gemm8p");
+}
+
+// The dense fp8 projection on gemm8p's kernel: A [M, K] and W [N, K] e4m3, C [M, N] bf16 (swiglu: [M, N / 2], W's rows gate / up interleaved in
+// blocks of 32); ws and flags as gemm8p's, or none: K is not cut then
+void gemm8p_fp8(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const at::Tensor& a_scale, const at::Tensor& w_scale, bool swiglu,
+                const c10::optional<at::Tensor>& ws, const c10::optional<at::Tensor>& flags) {
+  CHECK_GPU(A); CHECK_GPU(W); CHECK_CONTIG(W); CHECK_BF16(C);
+  TORCH_CHECK(A.scalar_type() == at::kFloat8_e4m3fn && W.scalar_type() == at::kFloat8_e4m3fn, "gemm8p_fp8: e4m3 A and W");
+  TORCH_CHECK(A.dim() == 2 && A.stride(1) == 1 && C.dim() == 2 && C.stride(1) == 1 && W.dim() == 2, "gemm8p_fp8: layouts");
+  TORCH_CHECK(W.size(0) < INT_MAX && W.size(1) < INT_MAX && A.size(0) * A.stride(0) < (int64_t(1) << 31), "gemm8p_fp8: 32-bit sizes");
+  const int M = (int)A.size(0), N = (int)W.size(0), K = (int)W.size(1);
+  TORCH_CHECK(A.size(1) == K && C.size(0) == M && C.size(1) == (swiglu ? N / 2 : N), "gemm8p_fp8: shape mismatch");
+  TORCH_CHECK(C.stride(0) < (1 << 26), "gemm8p_fp8: output rows too far apart");
+  TORCH_CHECK((((uintptr_t)A.data_ptr() | (uintptr_t)W.data_ptr() | (uintptr_t)C.data_ptr()) & 15) == 0, "gemm8p_fp8: 16-byte aligned operands");
+  for (const at::Tensor* t : {&a_scale, &w_scale}) {
+    CHECK_DTYPE(*t, at::kFloat); CHECK_CONTIG(*t);
+  }
+  TORCH_CHECK(a_scale.numel() >= M && w_scale.numel() == N, "gemm8p_fp8: scale shapes");
+  float* part = nullptr;
+  int* count = nullptr;
+  if (ws.has_value() && ws->defined()) {
+    const int slots = lwc_gemm8p_slots();
+    TORCH_CHECK(flags.has_value() && flags->defined(), "gemm8p_fp8: a workspace has its flags");
+    CHECK_GPU(*ws); CHECK_DTYPE(*ws, at::kFloat); CHECK_CONTIG(*ws);
+    CHECK_GPU(*flags); CHECK_DTYPE(*flags, at::kInt); CHECK_CONTIG(*flags);
+    TORCH_CHECK(ws->numel() >= (int64_t)slots * 65536 && flags->numel() >= slots, "gemm8p_fp8: workspace too small (", slots, " slots)");
+    part = ws->data_ptr<float>(), count = flags->data_ptr<int>();
+  }
+  CHECK_RC(lwc_gemm8p_fp8(A.data_ptr(), W.data_ptr(), C.data_ptr(), a_scale.data_ptr<float>(), w_scale.data_ptr<float>(), part, count, M, N, K,
+                          (int)A.stride(0), (int)C.stride(0), swiglu ? 1 : 0, cur_stream()),
+           "gemm8p_fp8");
 }
 
 // gemm2w: tiles of 128 x 128 (tile 0), 192 x 128 (1), 128 x 192 (2) or 64 x 64 (3, in splits K ranges: part and count, the
@@ -1207,6 +1239,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_decode", &paged_decode);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("gemm8p", &gemm8p);
+  m.def("gemm8p_fp8", &gemm8p_fp8);
   m.def("gemm2w", &gemm2w);
   m.def("gemm4w", &gemm4w);
   m.def("skinny_gemm", &skinny_gemm);

@@ -51,6 +51,10 @@
 //   store; the reader polls the flag, resets it for the next launch (flags start zeroed), barrier, loads of device
 //   scope.  (With fences instead, each of which writes an XCD's L2 back or drops it: 1095 rows x 6144 x 4096 72 us, so 67; 4096 x
 //   14336 143 and 135.)
+// fp8 (EPI_FP8, EPI_FP8_SWIGLU): e4m3 rows are the same bytes; a phase's 32 bf16 MFMAs are 16 scaled ones of four times the K at twice the
+// cycles, and the scales of a tile's rows and columns come into LDS with its last K tile.  Against one tile per workgroup (gemm8g.hip's dense
+// mode), whose last round of 32 to 48 tiles idles most of the chip, us, 8682 rows: x 28672 x 4096 SwiGLU 731 -> 690 (2.95 PFLOP/s), x 4096
+// x 14336 410 -> 336, x 6144 x 4096 194 -> 171, x 4096 x 4096 143 -> 116; 64 documents through three e5 layers 3916 -> 3655.
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -70,7 +74,9 @@ constexpr int kUA0 = 0, kUA1 = kUnitB, kUB0 = 2 * kUnitB, kUB1 = 3 * kUnitB;
 constexpr int kSC1 = 16, kNT = 2;
 constexpr int kPartialF = 256 * 256;  // fp32 partial tile per workgroup
 
-enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4 };
+// (fp8: e4m3 A and W, their element counts halved as of bf16, scales of A's rows and W's rows applied to the accumulators)
+enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4, EPI_FP8 = 5, EPI_FP8_SWIGLU = 6 };
+constexpr int kScalesB = 2 * 2048;  // fp8: the scales of two tiles, behind the K tiles
 
 struct Params {
   const bf16_t* A;
@@ -83,12 +89,20 @@ struct Params {
   int tiles_m, tiles_n, KT;
   int gm;  // tile order: groups of gm m-tiles, n fastest across a group (32 consecutive tiles ~ 4 x 8)
   int wpx, sk_tiles, dp_rounds;
+  const float *a_scale, *w_scale;  // fp8: [M], [N]
   int nt;  // the output is larger than the last-level cache: its stores pass the caches by
 };
 
 LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
                                                  0, 0);
+}
+
+typedef int v8i32 __attribute__((ext_vector_type(8)));
+LWC_DEVICE float4v mfma8(const uint4v (&a)[2], const uint4v (&b)[2], const float4v& c) {
+  const v8i32 av = {(int)a[0].x, (int)a[0].y, (int)a[0].z, (int)a[0].w, (int)a[1].x, (int)a[1].y, (int)a[1].z, (int)a[1].w};
+  const v8i32 bv = {(int)b[0].x, (int)b[0].y, (int)b[0].z, (int)b[0].w, (int)b[1].x, (int)b[1].y, (int)b[1].z, (int)b[1].w};
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, 0, 127, 0, 127);  // (block scales of one)
 }
 
 // x * sigmoid(x) with v_rcp_f32 (1 ulp) instead of the IEEE division sequence (v_div_scale x2, v_div_fmas,
@@ -124,7 +138,8 @@ struct Item {
 template <int EPI, int R1>
 __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
   constexpr int BMH = 64 + 16 * R1;  // rows of a wave row
-  constexpr int CW = EPI == EPI_SWIGLU ? 32 : 64, NH = CW / 32;  // output columns of a wave, in groups of 32
+  constexpr bool kF8 = EPI == EPI_FP8 || EPI == EPI_FP8_SWIGLU, kSwiglu = EPI == EPI_SWIGLU || EPI == EPI_FP8_SWIGLU;
+  constexpr int CW = kSwiglu ? 32 : 64, NH = CW / 32;  // output columns of a wave, in groups of 32
   constexpr int kStores = (4 + R1) * NH;  // store instructions of an epilogue
   constexpr bool kBias = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
@@ -212,6 +227,19 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
   float4v acc[4 + R1][4];
   uint4v a[4][2], b[4][2];
   auto mma = [&](auto n, int i0) {
+    if constexpr (kF8) {
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+        for (int i = 0; i < decltype(n)::value; ++i) acc[i0 + i][jj] = mfma8(b[jj], a[i], acc[i0 + i][jj]);
+      // (else the compiler sinks the scaled MFMAs past the barriers into the next phase: 8682 x 28672 x 4096 SwiGLU 814 us for 690)
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int jj = 0; jj < 4; ++jj)
+#pragma unroll
+        for (int i = 0; i < decltype(n)::value; ++i) asm volatile("" : "+v"(acc[i0 + i][jj]));
+      return;
+    }
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
@@ -257,6 +285,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
   int at = 0;           // LDS buffer of the K tile at hand
   bool stored = false;  // an epilogue's stores have gone out after unit B1 of the next K tile
   uint4v bias[2];
+  int scales = kLdsB;  // fp8: where the scales of the tile at hand lie
 
   for (Item cur{sk_e, 0, 0, 0, 0}; next(cur);) {
 #pragma unroll
@@ -280,6 +309,13 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
           for (int h = 0; h < 2; ++h) bias[h] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(rb, (col + 32 * h) * 2, 0, 0));
         }
       }
+      if constexpr (kF8) {
+        if (left == 1) {  // the scales of the tile's rows (waves 0 .. 3) and columns, one a thread
+          auto* dst = (__attribute__((address_space(3))) void*)(smem + scales + wid * 256);
+          const __amdgpu_buffer_rsrc_t rs = wr == 0 ? uniform_rsrc(p.a_scale + m0, min(p.M - m0, 256) * 4) : uniform_rsrc(p.w_scale + n0, min(p.N - n0, 256) * 4);
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 4, (tid & 255) * 4, 0, 0, 0);
+        }
+      }
       rdB(cb + kUB0, 0);
       rdB(cb + kUB1, 2);
       rdA(cb + kUA0, n4);
@@ -290,7 +326,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
       advance();
       rdA(cb + kUA1, n1);
       stage(0, cb), stage(2, cb), stage(3, cb);
-      if (stored) G8_VM(8 + kStores);
+      if (stored && !(kF8 && left == 1)) G8_VM(8 + kStores);  // (the scales have landed with the tile's last K tile)
       else G8_VM(8);
       G8_MFMA(n1, 4);
       stored = false;
@@ -350,8 +386,8 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
     // ---- epilogue: a lane holds eight consecutive columns of a row, so its 16 bytes go out from the registers.  Stores past M or
     // N fall outside the resource: the number of store instructions, which the waits above count, is always the same ----
     if (whole) {
-      const int ncols = EPI == EPI_SWIGLU ? p.N / 2 : p.N;
-      const int ncol0 = EPI == EPI_SWIGLU ? n0 / 2 + wc * 32 : n0 + wc * 64, row0 = m0 + wr * BMH;
+      const int ncols = kSwiglu ? p.N / 2 : p.N;
+      const int ncol0 = kSwiglu ? n0 / 2 + wc * 32 : n0 + wc * 64, row0 = m0 + wr * BMH;
       const int cols_here = max(0, min(ncols - ncol0, CW));
       uint32_t vo[NH];
 #pragma unroll
@@ -374,10 +410,20 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
         }
         __builtin_amdgcn_sched_barrier(0);
       }
+      float ws[kF8 ? 2 : 1][8];
+      if constexpr (kF8) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int e = 0; e < 8; e += 4)
+            *reinterpret_cast<float4v*>(&ws[c][e]) = *reinterpret_cast<const float4v*>(smem + scales + 1024 + (wc * 64 + 32 * c + 8 * (el >> 4) + e) * 4);
+      }
       auto store = [&](auto policy) {
 #pragma unroll
       for (int i = 0; i < 4 + R1; ++i) {
         const __amdgpu_buffer_rsrc_t rc = rows_of(p.C, i);
+        float as = 1.f;
+        if constexpr (kF8) as = *reinterpret_cast<const float*>(smem + scales + (wr * BMH + 16 * i + (el & 15)) * 4);
 #pragma unroll
         for (int h = 0; h < NH; ++h) {
           float x[8], y[8];
@@ -386,7 +432,9 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
 #pragma unroll
           for (int e = 0; e < 8; ++e) {
             x[e] = acc[i][2 * h + e / 4][e % 4];
+            if constexpr (kF8) x[e] *= as * ws[h][e];
             if constexpr (EPI == EPI_SWIGLU) x[e] = silu(x[e]) * acc[i][2 + e / 4][e % 4];
+            if constexpr (EPI == EPI_FP8_SWIGLU) x[e] = silu(x[e]) * (acc[i][2 + e / 4][e % 4] * (as * ws[1][e]));
             if constexpr (kBias || EPI == EPI_RESIDUAL) x[e] += y[e];
             if constexpr (EPI == EPI_BIAS_GELU) x[e] = gelu_erf(x[e]);
           }
@@ -398,6 +446,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
       else store(std::integral_constant<int, 0>{});
       stored = true;
     }
+    if constexpr (kF8) scales ^= kLdsB ^ (kLdsB + 2048);
   }
   if (wr == 0) G8_BAR();  // re-align the wave rows
   G8_VM(0);               // the last K tile's requests have ended before the LDS is given back
@@ -408,12 +457,13 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
 
 template <int EPI, int R1>
 int launch(const Params& p, hipStream_t s) {
+  constexpr int kLds = kLdsB + (EPI >= EPI_FP8 ? kScalesB : 0);
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)gemm8p_kernel<EPI, R1>, hipFuncAttributeMaxDynamicSharedMemorySize, kLdsB);
+    (void)hipFuncSetAttribute((const void*)gemm8p_kernel<EPI, R1>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
     attr = true;
   }
-  gemm8p_kernel<EPI, R1><<<8 * p.wpx, 512, kLdsB, s>>>(p);
+  gemm8p_kernel<EPI, R1><<<8 * p.wpx, 512, kLds, s>>>(p);
   return (int)hipGetLastError();
 }
 
@@ -493,6 +543,24 @@ int row_tile(int M, int tiles_n, int KT) {
   return best;
 }
 
+// How a call is cut: its row tiles, grid, stream-K tiles (none without a workspace) and rounds of whole tiles
+int plan(Params& p, bool swiglu) {
+  p.tiles_n = (p.N + 255) / 256, p.KT = p.K / 64;
+  const int r1 = p.lda < (1 << 20) ? row_tile(p.M, p.tiles_n, p.KT) : 4, bm = 128 + 32 * r1;
+  p.tiles_m = (p.M + bm - 1) / bm;
+  const int tiles = p.tiles_m * p.tiles_n;
+  p.wpx = grid_wpx(tiles, p.KT);
+  const int G = 8 * p.wpx;
+  bool cut;
+  call_cost(tiles, p.wpx, p.KT, r1, &cut);
+  if (!p.ws) cut = false;
+  p.dp_rounds = cut ? std::max(0, tiles / G - 1) : (tiles + G - 1) / G;
+  p.sk_tiles = cut ? tiles - p.dp_rounds * G : 0;
+  p.gm = std::max(1, env_int("LWC_G8_GM", 8));
+  p.nt = (long long)p.M * p.N * (swiglu ? 1 : 2) > 256LL << 20;
+  return r1;
+}
+
 }  // namespace g8p
 }  // namespace lwc
 
@@ -511,14 +579,10 @@ extern "C" int lwc_gemm8p(const void* A, const void* W, void* C, const void* R, 
   if (epi == EPI_SWIGLU && N % 64 != 0) return -1;
   if ((epi == EPI_RESIDUAL || epi == EPI_BIAS || epi == EPI_BIAS_GELU) && R == nullptr) return -1;
   if (M == 0 || N == 0) return 0;
-  const int tiles_n = (N + 255) / 256, KT = K / 64, r1 = lda < (1 << 20) ? row_tile(M, tiles_n, KT) : 4;
-  const int bm = 128 + 32 * r1, tiles_m = (M + bm - 1) / bm, tiles = tiles_m * tiles_n, wpx = grid_wpx(tiles, KT), G = 8 * wpx;
-  bool cut;
-  call_cost(tiles, wpx, KT, r1, &cut);
-  const int dp = cut ? std::max(0, tiles / G - 1) : (tiles + G - 1) / G, sk = cut ? tiles - dp * G : 0;
-  Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, ws, flags,
-           M, N, K, lda, ldc, tiles_m, tiles_n, KT, std::max(1, env_int("LWC_G8_GM", 8)), wpx, sk, dp,
-           (long long)M * N * (epi == EPI_SWIGLU ? 1 : 2) > 256LL << 20};
+  Params p{};
+  p.A = (const lwc::bf16_t*)A, p.W = (const lwc::bf16_t*)W, p.C = (lwc::bf16_t*)C, p.R = (const lwc::bf16_t*)R, p.ws = ws, p.flags = flags;
+  p.M = M, p.N = N, p.K = K, p.lda = lda, p.ldc = ldc;
+  const int r1 = plan(p, epi == EPI_SWIGLU);
   switch (epi) {
     case EPI_PLAIN: return launch<EPI_PLAIN>(p, r1, s);
     case EPI_RESIDUAL: return launch<EPI_RESIDUAL>(p, r1, s);
@@ -527,4 +591,21 @@ extern "C" int lwc_gemm8p(const void* A, const void* W, void* C, const void* R, 
     case EPI_BIAS_GELU: return launch<EPI_BIAS_GELU>(p, r1, s);
   }
   return -1;
+}
+
+// C [M, N] = (A [M, K] . W [N, K]^T) * a_scale[row] * w_scale[column] of e4m3 A and W, or (swiglu, W's rows gate / up interleaved in
+// blocks of 32) silu(gate) * up [M, N / 2], bf16.  Requires K % 128 == 0, N % 8 == 0 (SwiGLU: 64), lda % 16 == 0 (bytes), ldc % 8 == 0, A, W and
+// C at 16 bytes; ws and flags as lwc_gemm8p's, or null: K is not cut then.
+extern "C" int lwc_gemm8p_fp8(const void* A, const void* W, void* C, const float* a_scale, const float* w_scale, float* ws, int* flags, int M,
+                              int N, int K, int lda, int ldc, int swiglu, hipStream_t s) {
+  using namespace lwc::g8p;
+  if (K % 128 != 0 || K < 128 || N % (swiglu ? 64 : 8) != 0 || lda % 16 != 0 || ldc % 8 != 0 || !a_scale || !w_scale) return -1;
+  if ((long long)M * lda >= (1LL << 31) || 256LL * K >= (1LL << 31) || ldc >= (1 << 26)) return -1;  // 32-bit buffer offsets
+  if (M == 0 || N == 0) return 0;
+  Params p{};
+  p.A = (const lwc::bf16_t*)A, p.W = (const lwc::bf16_t*)W, p.C = (lwc::bf16_t*)C, p.ws = ws, p.flags = flags;
+  p.a_scale = a_scale, p.w_scale = w_scale;
+  p.M = M, p.N = N, p.K = K / 2, p.lda = lda / 2, p.ldc = ldc;
+  const int r1 = plan(p, swiglu);
+  return swiglu ? launch<EPI_FP8_SWIGLU>(p, r1, s) : launch<EPI_FP8>(p, r1, s);
 }

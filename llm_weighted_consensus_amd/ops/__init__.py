@@ -922,12 +922,21 @@ def _g8g_dense_ok(xq: torch.Tensor, w: "Fp8Weight") -> bool:
             and M >= 0 and 256 * K < (1 << 31) and xq.dtype == torch.float8_e4m3fn)
 
 
+def _fp8_few(M: int, N: int, K: int, ws) -> bool:
+    """Whether a dense fp8 product goes in gemm2g.hip's small tiles: up to 128 of gemm8p's 256 x 256 ones, unless K is long and
+    gemm8p may cut it (``ws``).  us, gemm2g / gemm8p, at 64, 128 and 144 to 160 tiles: K 2048 14.1 / 23.6, 22.2 / 24.4, 32.7 / 25.1; K 4096 23.5 /
+    34.1, 34.9 / 37.9, 47.6 / 37.1; K 8192 40.0 / 42.3, 60.7 / 60.9, 100.2 / 69.7; K 14336 66.0 / 55.1, 101.3 / 91.3, 167.4 / 115.3, at 48 tiles 53.1 to
+    65.6 / 57.6 to 67.3, at 32 53.2 / 46.8."""
+    tiles = -(-M // 256) * -(-N // 256)
+    return tiles <= 128 and (ws is None or K < 12288 or tiles < 64)
+
+
 G8G_SPAN = 1 << 31  # bytes of A one gemm8g launch may address (its buffer range is 32-bit)
 
 
 def gemm8g_dense(xq: torch.Tensor, xs: torch.Tensor, w: "Fp8Weight", out: Optional[torch.Tensor] = None,
                  swiglu: bool = False):
-    """Dense fp8 GEMM on the hand-written 256-row core (csrc/kernels/gemm8g.hip, G = 1, no row table):
+    """Dense fp8 GEMM on the hand-written cores (csrc/kernels/gemm8p.hip; of few tiles gemm2g.hip's through gemm8g.hip):
     (xq [M, K] e4m3 . w.q^T) * xs[row] * w.s[col] -> bf16 [M, N]; ``swiglu``: w's rows are gate|up interleaved
     in blocks of 32 (:func:`swiglu_interleave`) and the epilogue writes silu(gate) * up, bf16 [M, N / 2].
     The kernel addresses A through a 32-bit buffer range: row blocks of < 2 GiB of A go one launch each
@@ -939,11 +948,18 @@ def gemm8g_dense(xq: torch.Tensor, xs: torch.Tensor, w: "Fp8Weight", out: Option
     if M == 0:
         return out
     step = max(256, (G8G_SPAN - 1) // xq.stride(0) // 256 * 256)
-    s, ws, wq = xs.reshape(-1).contiguous(), w.s.reshape(-1), w.q.view(1, N, K)
+    s, ws = xs.reshape(-1).contiguous(), w.s.reshape(-1)
     for r0 in range(0, M, step):
         r1 = min(M, r0 + step)
-        kernels().gemm8g_fp8(xq[r0:r1], wq, out[r0:r1], None, -(-(r1 - r0) // 256), None, s[r0:r1], ws,
-                             int(bool(swiglu)), None, None)
+        work = _split_workspace(xq.device)
+        # (gemm8p's rows, pointers and reach; anything else goes where those were never asked for)
+        wide = out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.stride(0) < 1 << 26 and not (xq.data_ptr() | out.data_ptr() | w.q.data_ptr()) & 15
+        if wide and not _fp8_few(r1 - r0, N, K, work):
+            part, flags = work or (None, None)
+            kernels().gemm8p_fp8(xq[r0:r1], w.q, out[r0:r1], s[r0:r1], ws, bool(swiglu), part, flags)
+        else:
+            kernels().gemm8g_fp8(xq[r0:r1], w.q.view(1, N, K), out[r0:r1], None, -(-(r1 - r0) // 256), None, s[r0:r1], ws,
+                                 int(bool(swiglu)), None, None)
     return out
 
 
