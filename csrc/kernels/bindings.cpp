@@ -931,16 +931,15 @@ std::pair<int64_t, int64_t> prefill_plan(int64_t nseq, int64_t rows, int64_t max
 // The layers of a post-norm encoder over packed rows x [T, d], launched from here: a forward of few rows is bound by the
 // host's launches (12 layers of 7 kernels, from Python 6.3 us each: bge-small, 12 tokens 565 us a call, 399 so).
 // weights: 12 tensors a layer (qkv, its bias, o, its bias, norm 1 gain and bias, FFN up and bias, FFN down and bias, norm 2
-// gain and bias).  cores: the planner's choice for qkv, o, up, down (1 skinny_gemm, 2 gemm2w, 3 gemm8p over the
+// gain and bias).  cores: the planner's choice for qkv, o, up, down (0 the library, 1 skinny_gemm, 2 gemm2w, 3 gemm8p over the
 // workspace part and count).  fuse_o / fuse_f: the projection adds into x in its epilogue and its bias enters the norm.  Returns the
 // last hidden rows; nothing, and nothing launched, if a layer's weights are not laid out as these cores read them or core 3 has no
 // workspace (the caller's own loop takes any).
-c10::optional<at::Tensor> encoder_layers(at::Tensor x, const std::vector<at::Tensor>& weights, const at::Tensor& cu, int64_t max_len,
+c10::optional<at::Tensor> run_encoder_layers(at::Tensor x, const std::vector<at::Tensor>& weights, const at::Tensor& cu, int64_t max_len,
                           int64_t H, int64_t Dh, double scale, double eps, const std::vector<int64_t>& cores, bool fuse_o,
                           bool fuse_f, const c10::optional<at::Tensor>& part, const c10::optional<at::Tensor>& count) {
   CHECK_BF16(x); CHECK_CONTIG(x);
   TORCH_CHECK(x.dim() == 2 && weights.size() % 12 == 0 && !weights.empty() && cores.size() == 4, "encoder_layers: arguments");
-  for (int64_t c : cores) TORCH_CHECK(c >= 1 && c <= 3, "encoder_layers: cores are 1 to 3, not ", c);
   const int64_t T = x.size(0), d = x.size(1), f = weights[6].size(0);
   TORCH_CHECK(H * Dh == d && (d <= 1024 || !(fuse_o || fuse_f)), "encoder_layers: head shape or fused rows");
   for (size_t i = 0; i < weights.size(); ++i) {
@@ -956,7 +955,10 @@ c10::optional<at::Tensor> encoder_layers(at::Tensor x, const std::vector<at::Ten
   at::Tensor y = at::empty({T, d}, x.options()), z = at::empty({T, d}, x.options());
   const at::Tensor q = qkv.narrow(1, 0, d), k = qkv.narrow(1, d, d), v = qkv.narrow(1, 2 * d, d);
   auto gemm = [&](int64_t core, const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const at::Tensor& R, int64_t epi) {
-    if (core == 1) skinny_gemm(A, W, C, R, epi);
+    if (core == 0) {  // what the caller's loop asks of the library, into the same results
+      if (epi == 4) at::_addmm_activation_out(C, R, A, W.t(), 1, 1, true);
+      else at::addmm_out(C, R, A, W.t());
+    } else if (core == 1) skinny_gemm(A, W, C, R, epi);
     else if (core == 3) gemm8p(A, W, C, R, epi, ws, flags);
     else gemm2w(A, W, C, R, epi, -1, 1, part, count);
   };
@@ -983,6 +985,26 @@ c10::optional<at::Tensor> encoder_layers(at::Tensor x, const std::vector<at::Ten
     }
   }
   return x;
+}
+
+c10::optional<at::Tensor> encoder_layers(at::Tensor x, const std::vector<at::Tensor>& weights, const at::Tensor& cu, int64_t max_len,
+                          int64_t H, int64_t Dh, double scale, double eps, const std::vector<int64_t>& cores, bool fuse_o,
+                          bool fuse_f, const c10::optional<at::Tensor>& part, const c10::optional<at::Tensor>& count) {
+  for (int64_t c : cores) TORCH_CHECK(c >= 1 && c <= 3, "encoder_layers: cores are 1 to 3, not ", c);
+  return run_encoder_layers(x, weights, cu, max_len, H, Dh, scale, eps, cores, fuse_o, fuse_f, part, count);
+}
+
+// The same with projections on the library too (core 0).  us a call of `embed`, these layers from Python / from here: bge-small 7680 and 24000 tokens
+// 1032 / 1004, 2458 / 2328; bge-base 3200 and 7680 1225 / 1160, 2162 / 2138; bge-large 960, 3200 and 7680 1876 / 1765, 3204 / 3198, 5849 / 5798
+c10::optional<at::Tensor> encoder_layers_mixed(at::Tensor x, const std::vector<at::Tensor>& weights, const at::Tensor& cu, int64_t max_len,
+                          int64_t H, int64_t Dh, double scale, double eps, const std::vector<int64_t>& cores, bool fuse_o,
+                          bool fuse_f, const c10::optional<at::Tensor>& part, const c10::optional<at::Tensor>& count) {
+  for (int64_t c : cores) TORCH_CHECK(c >= 0 && c <= 3, "encoder_layers_mixed: cores are 0 to 3, not ", c);
+  // (the library's results go into tensors that are there: nothing that a gradient is asked of)
+  if (at::GradMode::is_enabled())
+    for (const at::Tensor& t : weights)
+      if (t.requires_grad()) return c10::nullopt;
+  return run_encoder_layers(x, weights, cu, max_len, H, Dh, scale, eps, cores, fuse_o, fuse_f, part, count);
 }
 
 // A post-norm encoder over few packed rows, embeddings to last hidden rows (encoder_few.hip): weights as encoder_layers takes
@@ -1270,6 +1292,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     TORCH_CHECK(rows > 0 && G > 0 && N > 0 && K > 0 && K <= INT_MAX / 2, "gemm2s_rows: sizes");
     return lwc_gemm2s_rows(rows, G, N, 2 * K);
   });
+  m.def("encoder_layers_mixed", &encoder_layers_mixed, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("encoder_few", &encoder_few, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("encoder_layers", &encoder_layers, pybind11::call_guard<pybind11::gil_scoped_release>());
   m.def("prefill_attention_mx", &prefill_attention_mx);

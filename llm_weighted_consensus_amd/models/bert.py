@@ -180,8 +180,9 @@ class BertEncoder:
                            (L.w1, L.b1, "bias_gelu"), (L.w2, None if fuse_f else L.b2, "enc_residual" if fuse_f else "bias"))
             gemm_plan.choose_encoder(x, projections)
             cores = gemm_plan.encoder_cores(T, projections)
-            y = None if cores is None else ops.encoder_layers(x, [t for L in self.layers for t in _layer_tensors(L)], cu, max_len, H, Dh,
-                                                              self.scale, c.ln_eps, cores, fuse_o, fuse_f)
+            run = None if cores is None else ops.encoder_layers if all(cores) else ops.encoder_layers_mixed
+            y = None if run is None else run(x, [t for L in self.layers for t in _layer_tensors(L)], cu, max_len, H, Dh, self.scale,
+                                             c.ln_eps, cores, fuse_o, fuse_f)
             if y is not None:
                 return y
         for L in self.layers:

@@ -570,6 +570,14 @@ def encoder_layers(x: torch.Tensor, weights: Sequence[torch.Tensor], cu: torch.T
                                     bool(fuse_f), part, count)
 
 
+def encoder_layers_mixed(x: torch.Tensor, weights: Sequence[torch.Tensor], cu: torch.Tensor, max_len: int, H: int, Dh: int,
+                         scale: float, eps: float, cores: Sequence[int], fuse_o: bool, fuse_f: bool) -> Optional[torch.Tensor]:
+    """:func:`encoder_layers` where ``cores`` may name the library (0)."""
+    part, count = _split_workspace(x.device) or (None, None)
+    return kernels().encoder_layers_mixed(x, weights, cu, int(max_len), int(H), int(Dh), float(scale), float(eps), cores, bool(fuse_o),
+                                          bool(fuse_f), part, count)
+
+
 def encoder_few(word: torch.Tensor, pos: torch.Tensor, ids: torch.Tensor, positions: torch.Tensor, g: torch.Tensor, b: torch.Tensor,
                 weights: Sequence[torch.Tensor], cu: torch.Tensor, H: int, scale: float, eps: float) -> Optional[torch.Tensor]:
     """The last hidden rows of a post-norm encoder over few packed rows (csrc/kernels/encoder_few.hip), from the embedding

@@ -291,12 +291,15 @@ _ENC_NATIVE = {**_NATIVE, "g8": 3}
 
 def encoder_cores(M: int, projections) -> Optional[list]:
     """The cores of an encoder layer's projections ((weight, its bias or None where it adds into the stream, epilogue
-    name) each) at M rows as ``ops.encoder_layers`` numbers them; None until all are timed, or if one's choice is another
-    core or does not take the call."""
+    name) each) at M rows as ``ops.encoder_layers`` numbers them, 0 the library (``ops.encoder_layers_mixed``); None until all are
+    timed, or if one's choice is another core or does not take the call."""
     out = []
     for w, b, epi in projections:
         N, K = w.shape
         c = MODE if MODE in ENC_BACKENDS else _CHOICE.get((_m_bucket(M), N, K, epi))
+        if c == "blas":
+            out.append(0)
+            continue
         n = _ENC_NATIVE.get(c)
         if n is None or not _g8_ok(N, K, epi) or c in EXCLUDE:
             return None

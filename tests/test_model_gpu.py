@@ -150,6 +150,47 @@ def test_encoder_layers_on_gemm8p_launched_natively(gpu, monkeypatch, fused):
     assert torch.equal(y, m.forward_packed(*args))
 
 
+@pytest.mark.parametrize("fused", ["0", "ffn2", "all"])
+@pytest.mark.parametrize("cores", [["blas"] * 4, ["blas", "g2", "g8", "blas"], ["g2", "blas", "blas", "g8"]])
+def test_encoder_layers_with_the_library_launched_natively(gpu, monkeypatch, cores, fused):
+    """Layers with projections on the library are launched from native code as well: the loop's bits, eagerly and as a graph; a
+    weight that asks for a gradient leaves them to the loop."""
+    from llm_weighted_consensus_amd import ops
+    from llm_weighted_consensus_amd.models.bert import BertEncoder
+    from llm_weighted_consensus_amd.models.config import encoder_config
+    from llm_weighted_consensus_amd.ops import gemm_plan
+
+    m = BertEncoder(encoder_config("bge-small-en-v1.5"), device=gpu, seed=5)
+    for L in m.layers:
+        for n in ("bqkv", "bo", "b1", "b2"):
+            getattr(L, n).normal_(0.0, 0.1)
+    m.fused_residual = fused
+    args = m.pack([[(7 * i + j) % 900 + 1 for j in range(n)] for i, n in enumerate([300, 2, 64, 129])])
+    L, T = m.layers[0], args[0].shape[0]
+    epis = ("bias", "enc_residual" if fused == "all" else "bias", "bias_gelu", "bias" if fused == "0" else "enc_residual")
+    monkeypatch.setattr(gemm_plan, "_CHOICE", {(gemm_plan._m_bucket(T), *w.shape, e): c
+                                               for w, e, c in zip((L.wqkv, L.wo, L.w1, L.w2), epis, cores)})
+    taken, native = [], ops.encoder_layers_mixed
+    monkeypatch.setattr(ops, "encoder_layers_mixed", lambda *a: taken.append(native(*a)) or taken[-1])
+    y = m.forward_packed(*args)
+    assert len(taken) == 1 and taken[0] is y
+    if "g8" not in cores:   # (the capture's stream has no workspace)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            z = m.forward_packed(*args)
+        for _ in range(3):
+            graph.replay()
+            assert torch.equal(y, z)
+            m.forward_packed(*args)
+    monkeypatch.setattr(ops, "encoder_layers_mixed", lambda *a: None)
+    assert torch.equal(y, m.forward_packed(*args))
+    monkeypatch.setattr(ops, "encoder_layers_mixed", native)
+    m.layers[2].wo.requires_grad_(True)
+    assert native(torch.zeros_like(y), [t for L in m.layers for t in (L.wqkv, L.bqkv, L.wo, L.bo, L.ln1_g, L.ln1_b, L.w1, L.b1, L.w2, L.b2,
+                                                                     L.ln2_g, L.ln2_b)], args[2], 300, 12, 32, m.scale, 1e-12, [0] * 4,
+                  False, False) is None
+
+
 @pytest.mark.parametrize("core", [0, 4, -1])
 def test_encoder_layers_refuse_other_cores(gpu, core):
     """A core that no kernel stands for is an error, not gemm2w."""
