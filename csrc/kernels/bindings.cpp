@@ -32,7 +32,8 @@ int lwc_cascade_rows_per_tile(int);
 int lwc_grouped_gemm(const void*, const void*, void*, const int*, const float*, const float*, const void*, const int*,
                      int, int, int, int, int, int, long long, int, float*, int, long long, hipStream_t);
 int lwc_gemm8p(const void*, const void*, void*, const void*, float*, int*, int, int, int, int, int, int, hipStream_t);
-int lwc_gemm8p_fp8(const void*, const void*, void*, const float*, const float*, float*, int*, int, int, int, int, int, int, hipStream_t);
+int lwc_gemm8p_fp8(const void*, const void*, void*, const float*, const float*, const void*, void*, int, float*, int*, int, int, int, int, int,
+                   int, hipStream_t);
 int lwc_gemm8p_slots();
 void lwc_gemm2w_plan(int, int, int, int, bool, long long, int*, int*);
 int lwc_gemm2w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, int, float*, int*,
@@ -478,22 +479,54 @@ void gemm8p(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::
            "gemm8p");
 }
 
-// The dense fp8 projection on gemm8p's kernel: A [M, K] and W [N, K] e4m3, C [M, N] bf16 (swiglu: [M, N / 2], W's rows gate / up interleaved in
-// blocks of 32); ws and flags as gemm8p's, or none: K is not cut then
-void gemm8p_fp8(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const at::Tensor& a_scale, const at::Tensor& w_scale, bool swiglu,
-                const c10::optional<at::Tensor>& ws, const c10::optional<at::Tensor>& flags) {
-  CHECK_GPU(A); CHECK_GPU(W); CHECK_CONTIG(W); CHECK_BF16(C);
+// MX scale planes [K / 128][rows][4] bytes: a row-range view of a larger tensor is accepted (the plane stride is then the full
+// tensor's row count)
+int plane_rows(const at::Tensor& t, const char* what) {
+  CHECK_GPU(t); CHECK_DTYPE(t, at::kByte);
+  TORCH_CHECK(t.dim() == 3 && t.size(2) == 4 && t.stride(2) == 1 && t.stride(1) == 4 && t.stride(0) % 4 == 0 && t.stride(0) / 4 >= t.size(1),
+              what, ": MX scales must be [K / 128, rows, 4] bytes with rows contiguous");
+  return (int)(t.stride(0) / 4);
+}
+
+// The dense fp8 projection on gemm8p's kernel: A [M, K] and W [N, K] e4m3, C [M, N] bf16, or (swiglu 1, W's rows gate / up
+// interleaved in blocks of 32) [M, N / 2], or (2) that as e4m3 with mx_out [N / 256, M, 4]; a_mx [K / 128, M, 4]: A's block scales in place of a_scale;
+// ws and flags as gemm8p's, or none: K is not cut then
+void gemm8p_fp8(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c10::optional<at::Tensor>& a_scale, const at::Tensor& w_scale,
+                int64_t swiglu, const c10::optional<at::Tensor>& ws, const c10::optional<at::Tensor>& flags,
+                const c10::optional<at::Tensor>& a_mx, const c10::optional<at::Tensor>& mx_out) {
+  CHECK_GPU(A); CHECK_GPU(W); CHECK_CONTIG(W); CHECK_GPU(C);
+  TORCH_CHECK(swiglu >= 0 && swiglu <= 2, "gemm8p_fp8: swiglu 0, 1 or 2");
   TORCH_CHECK(A.scalar_type() == at::kFloat8_e4m3fn && W.scalar_type() == at::kFloat8_e4m3fn, "gemm8p_fp8: e4m3 A and W");
+  CHECK_DTYPE(C, swiglu == 2 ? at::kFloat8_e4m3fn : at::kBFloat16);
   TORCH_CHECK(A.dim() == 2 && A.stride(1) == 1 && C.dim() == 2 && C.stride(1) == 1 && W.dim() == 2, "gemm8p_fp8: layouts");
   TORCH_CHECK(W.size(0) < INT_MAX && W.size(1) < INT_MAX && A.size(0) * A.stride(0) < (int64_t(1) << 31), "gemm8p_fp8: 32-bit sizes");
   const int M = (int)A.size(0), N = (int)W.size(0), K = (int)W.size(1);
   TORCH_CHECK(A.size(1) == K && C.size(0) == M && C.size(1) == (swiglu ? N / 2 : N), "gemm8p_fp8: shape mismatch");
   TORCH_CHECK(C.stride(0) < (1 << 26), "gemm8p_fp8: output rows too far apart");
-  TORCH_CHECK((((uintptr_t)A.data_ptr() | (uintptr_t)W.data_ptr() | (uintptr_t)C.data_ptr()) & 15) == 0, "gemm8p_fp8: 16-byte aligned operands");
-  for (const at::Tensor* t : {&a_scale, &w_scale}) {
-    CHECK_DTYPE(*t, at::kFloat); CHECK_CONTIG(*t);
+  CHECK_GPU(w_scale); CHECK_DTYPE(w_scale, at::kFloat); CHECK_CONTIG(w_scale);
+  TORCH_CHECK(w_scale.numel() == N, "gemm8p_fp8: w_scale shape");
+  const float* as = nullptr;
+  const void* amx = nullptr;
+  void* mxo = nullptr;
+  int s_rows = 0;
+  if (a_mx.has_value() && a_mx->defined()) {
+    TORCH_CHECK(!swiglu, "gemm8p_fp8: an A with block scales takes the plain epilogues");
+    s_rows = plane_rows(*a_mx, "gemm8p_fp8 a_mx");
+    TORCH_CHECK(a_mx->size(0) == K / 128 && a_mx->size(1) >= M, "gemm8p_fp8: a_mx must be [K / 128, M, 4]");
+    amx = a_mx->data_ptr();
+  } else {
+    TORCH_CHECK(a_scale.has_value() && a_scale->defined(), "gemm8p_fp8: a_scale or a_mx required");
+    CHECK_GPU(*a_scale); CHECK_DTYPE(*a_scale, at::kFloat); CHECK_CONTIG(*a_scale);
+    TORCH_CHECK(a_scale->numel() >= M, "gemm8p_fp8: a_scale shape");
+    as = a_scale->data_ptr<float>();
   }
-  TORCH_CHECK(a_scale.numel() >= M && w_scale.numel() == N, "gemm8p_fp8: scale shapes");
+  if (swiglu == 2) {
+    TORCH_CHECK(mx_out.has_value() && mx_out->defined(), "gemm8p_fp8: swiglu 2 writes mx_out");
+    s_rows = plane_rows(*mx_out, "gemm8p_fp8 mx_out");
+    TORCH_CHECK(N % 256 == 0 && mx_out->size(0) == N / 256 && mx_out->size(1) >= M, "gemm8p_fp8: mx_out must be [N / 256, M, 4]");
+    mxo = mx_out->data_ptr();
+  }
+  TORCH_CHECK((((uintptr_t)A.data_ptr() | (uintptr_t)W.data_ptr() | (uintptr_t)C.data_ptr()) & 15) == 0, "gemm8p_fp8: 16-byte aligned operands");
   float* part = nullptr;
   int* count = nullptr;
   if (ws.has_value() && ws->defined()) {
@@ -504,8 +537,8 @@ void gemm8p_fp8(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const a
     TORCH_CHECK(ws->numel() >= (int64_t)slots * 65536 && flags->numel() >= slots, "gemm8p_fp8: workspace too small (", slots, " slots)");
     part = ws->data_ptr<float>(), count = flags->data_ptr<int>();
   }
-  CHECK_RC(lwc_gemm8p_fp8(A.data_ptr(), W.data_ptr(), C.data_ptr(), a_scale.data_ptr<float>(), w_scale.data_ptr<float>(), part, count, M, N, K,
-                          (int)A.stride(0), (int)C.stride(0), swiglu ? 1 : 0, cur_stream()),
+  CHECK_RC(lwc_gemm8p_fp8(A.data_ptr(), W.data_ptr(), C.data_ptr(), as, w_scale.data_ptr<float>(), amx, mxo, s_rows, part, count, M, N, K,
+                          (int)A.stride(0), (int)C.stride(0), (int)swiglu, cur_stream()),
            "gemm8p_fp8");
 }
 
@@ -733,15 +766,6 @@ void gemm8g_fp8(const at::Tensor& A, const at::Tensor& W, at::Tensor& C, const c
   } else {
     TORCH_CHECK(C.size(0) <= A.size(0), "gemm8g: more output rows than A rows");
   }
-  // scale planes [K / 128][rows][4] bytes; a row-range view of a larger tensor is accepted (the plane stride
-  // is then the full tensor's row count)
-  auto plane_rows = [](const at::Tensor& t, const char* what) {
-    CHECK_GPU(t); CHECK_DTYPE(t, at::kByte);
-    TORCH_CHECK(t.dim() == 3 && t.size(2) == 4 && t.stride(2) == 1 && t.stride(1) == 4 && t.stride(0) % 4 == 0 &&
-                    t.stride(0) / 4 >= t.size(1),
-                what, ": MX scales must be [K / 128, rows, 4] bytes with rows contiguous");
-    return (int)(t.stride(0) / 4);
-  };
   int s_rows = 0;
   const void* amx = nullptr;
   void* mxo = nullptr;
@@ -1261,7 +1285,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("paged_decode", &paged_decode);
   m.def("grouped_gemm", &grouped_gemm);
   m.def("gemm8p", &gemm8p);
-  m.def("gemm8p_fp8", &gemm8p_fp8);
+  m.def("gemm8p_fp8", &gemm8p_fp8, py::arg("A"), py::arg("W"), py::arg("C"), py::arg("a_scale"), py::arg("w_scale"), py::arg("swiglu"),
+        py::arg("ws"), py::arg("flags"), py::arg("a_mx") = py::none(), py::arg("mx_out") = py::none());
   m.def("gemm2w", &gemm2w);
   m.def("gemm4w", &gemm4w);
   m.def("skinny_gemm", &skinny_gemm);

@@ -54,7 +54,9 @@
 // fp8 (EPI_FP8, EPI_FP8_SWIGLU): e4m3 rows are the same bytes; a phase's 32 bf16 MFMAs are 16 scaled ones of four times the K at twice the
 // cycles, and the scales of a tile's rows and columns come into LDS with its last K tile.  Against one tile per workgroup (gemm8g.hip's dense
 // mode), whose last round of 32 to 48 tiles idles most of the chip, us, 8682 rows: x 28672 x 4096 SwiGLU 731 -> 690 (2.95 PFLOP/s), x 4096
-// x 14336 410 -> 336, x 6144 x 4096 194 -> 171, x 4096 x 4096 143 -> 116; 64 documents through three e5 layers 3916 -> 3655.
+// x 14336 410 -> 336, x 6144 x 4096 194 -> 171, x 4096 x 4096 143 -> 116; with block scales, which come with each K tile, from MX x 4096 x 4096 151 -> 121,
+// x 4096 x 14336 449 -> 356, SwiGLU to MX of 16641 rows x 28672 x 4096 1407 -> 1334; 64 documents through three e5 layers 3897 -> 3605.  (The
+// residual added here spilled, and cost 32 to 38 us for the 17 that the norm behind it gains.)
 #include <algorithm>
 #include <cstdlib>
 #include <type_traits>
@@ -75,8 +77,11 @@ constexpr int kSC1 = 16, kNT = 2;
 constexpr int kPartialF = 256 * 256;  // fp32 partial tile per workgroup
 
 // (fp8: e4m3 A and W, their element counts halved as of bf16, scales of A's rows and W's rows applied to the accumulators)
-enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4, EPI_FP8 = 5, EPI_FP8_SWIGLU = 6 };
-constexpr int kScalesB = 2 * 2048;  // fp8: the scales of two tiles, behind the K tiles
+enum Epi { EPI_PLAIN = 0, EPI_RESIDUAL = 1, EPI_SWIGLU = 2, EPI_BIAS = 3, EPI_BIAS_GELU = 4, EPI_FP8 = 5, EPI_FP8_SWIGLU = 6,
+  EPI_FP8_MX_OUT = 7,    // SwiGLU, its result as e4m3 with a scale per row and 32 columns
+  EPI_FP8_MX = 8 };      // A with such scales, a scale per row and 32 of K, instead of one a row
+// fp8: the scales of two tiles, behind the K tiles, and of A's blocks in two K tiles, [256 rows][4] (twice: the waves' loads are as many)
+constexpr int kScalesB = 2 * 2048, kMxB = 2 * 2048;
 
 struct Params {
   const bf16_t* A;
@@ -90,6 +95,10 @@ struct Params {
   int gm;  // tile order: groups of gm m-tiles, n fastest across a group (32 consecutive tiles ~ 4 x 8)
   int wpx, sk_tiles, dp_rounds;
   const float *a_scale, *w_scale;  // fp8: [M], [N]
+  // e8m0 block scales [K / 128][s_rows][4] of A, [N / 256][s_rows][4] of the result (as in gemm8g.hip)
+  const uint8_t* a_mx;
+  uint8_t* mx_out;
+  int s_rows;
   int nt;  // the output is larger than the last-level cache: its stores pass the caches by
 };
 
@@ -98,11 +107,13 @@ LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
                                                  0, 0);
 }
 
+typedef uint32_t uint2v __attribute__((ext_vector_type(2)));
 typedef int v8i32 __attribute__((ext_vector_type(8)));
-LWC_DEVICE float4v mfma8(const uint4v (&a)[2], const uint4v (&b)[2], const float4v& c) {
+// (sb: the scale of b's row, its block of the lane's K; 127: one)
+LWC_DEVICE float4v mfma8(const uint4v (&a)[2], const uint4v (&b)[2], const float4v& c, int sb) {
   const v8i32 av = {(int)a[0].x, (int)a[0].y, (int)a[0].z, (int)a[0].w, (int)a[1].x, (int)a[1].y, (int)a[1].z, (int)a[1].w};
   const v8i32 bv = {(int)b[0].x, (int)b[0].y, (int)b[0].z, (int)b[0].w, (int)b[1].x, (int)b[1].y, (int)b[1].z, (int)b[1].w};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, 0, 127, 0, 127);  // (block scales of one)
+  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, 0, 127, 0, sb);
 }
 
 // x * sigmoid(x) with v_rcp_f32 (1 ulp) instead of the IEEE division sequence (v_div_scale x2, v_div_fmas,
@@ -138,9 +149,11 @@ struct Item {
 template <int EPI, int R1>
 __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
   constexpr int BMH = 64 + 16 * R1;  // rows of a wave row
-  constexpr bool kF8 = EPI == EPI_FP8 || EPI == EPI_FP8_SWIGLU, kSwiglu = EPI == EPI_SWIGLU || EPI == EPI_FP8_SWIGLU;
+  constexpr bool kF8 = EPI >= EPI_FP8, kMx = EPI == EPI_FP8_MX, kMxOut = EPI == EPI_FP8_MX_OUT;
+  constexpr bool kSwiglu = EPI == EPI_SWIGLU || EPI == EPI_FP8_SWIGLU || kMxOut;
+  constexpr int kAhead = kMx ? 9 : 8;  // loads of a K tile
   constexpr int CW = kSwiglu ? 32 : 64, NH = CW / 32;  // output columns of a wave, in groups of 32
-  constexpr int kStores = (4 + R1) * NH;  // store instructions of an epilogue
+  constexpr int kStores = (4 + R1) * (kMxOut ? 2 : NH);  // store instructions of an epilogue
   constexpr bool kBias = EPI == EPI_BIAS || EPI == EPI_BIAS_GELU;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   const int KT = p.KT;
@@ -198,7 +211,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
   // num_records and load as zeros (their outputs are not stored); behind the last K tile nothing is asked for
   Item ahead{sk_e, 0, 0, 0, 0};
   const bf16_t *srcA = nullptr, *srcW = nullptr;
-  int numA = 0, numW = 0, kt = -1;
+  int numA = 0, numW = 0, kt = -1, mS = 0;
   auto advance = [&] {
     kt = uni(kt + 1);
     if (kt < ahead.khi) return;
@@ -211,6 +224,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
     srcW = p.W + (size_t)n0 * p.K;
     numA = min(p.M - m0, 2 * BMH) * p.lda * 2;
     numW = min(p.N - n0, 256) * p.K * 2;
+    mS = m0;
     kt = uni(ahead.klo);
   };
   auto stage = [&](int u, uint8_t* buf) {
@@ -220,18 +234,26 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
       auto* dst = (__attribute__((address_space(3))) void*)(buf + u * kUnitB + i * 512 * 16 + dst_lane0);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(r, dst, 16, u < 2 ? voA[u][i] : voW[u - 2][i], kt * 128, 0, 0);
     }
+    if constexpr (kMx) {
+      if (u == 0) {  // the scales of the K tile's rows, four bytes a row
+        auto* dst = (__attribute__((address_space(3))) void*)(smem + kLdsB + kScalesB + (buf == smem ? 0 : 2048) + wid * 256);
+        const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(p.a_mx + (size_t)mS * 4, numA ? (KT * p.s_rows - mS) * 4 : 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 4, (tid & 255) * 4, kt * p.s_rows * 4, 0, 0);
+      }
+    }
   };
 
   // acc[i][jj]: 16 rows (tile i) x columns 32 (jj / 2) + 8 q + 4 (jj % 2) .. of the wave's 128 x 64, row r16 of the tile.
   // (The 32x32x16 MFMA with the same units and phases measured ~10 % slower on every shape.)
   float4v acc[4 + R1][4];
   uint4v a[4][2], b[4][2];
+  int sc[kMx ? 4 + R1 : 1];
   auto mma = [&](auto n, int i0) {
     if constexpr (kF8) {
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj)
 #pragma unroll
-        for (int i = 0; i < decltype(n)::value; ++i) acc[i0 + i][jj] = mfma8(b[jj], a[i], acc[i0 + i][jj]);
+        for (int i = 0; i < decltype(n)::value; ++i) acc[i0 + i][jj] = mfma8(b[jj], a[i], acc[i0 + i][jj], kMx ? sc[kMx ? i0 + i : 0] : 127);
       // (else the compiler sinks the scaled MFMAs past the barriers into the next phase: 8682 x 28672 x 4096 SwiGLU 814 us for 690)
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -279,7 +301,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
   stage(0, smem), stage(2, smem), stage(3, smem), stage(1, smem);
   advance();
   stage(0, smem + kBufB), stage(2, smem + kBufB), stage(3, smem + kBufB);
-  G8_VM(8);
+  G8_VM(kAhead);
   G8_BAR();
   if (wr == 1) G8_BAR();  // stagger the two wave rows by one barrier
   int at = 0;           // LDS buffer of the K tile at hand
@@ -312,22 +334,27 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
       if constexpr (kF8) {
         if (left == 1) {  // the scales of the tile's rows (waves 0 .. 3) and columns, one a thread
           auto* dst = (__attribute__((address_space(3))) void*)(smem + scales + wid * 256);
-          const __amdgpu_buffer_rsrc_t rs = wr == 0 ? uniform_rsrc(p.a_scale + m0, min(p.M - m0, 256) * 4) : uniform_rsrc(p.w_scale + n0, min(p.N - n0, 256) * 4);
+          const __amdgpu_buffer_rsrc_t rs = wr == 0 ? uniform_rsrc(p.a_scale + m0, kMx ? 0 : min(p.M - m0, 256) * 4) : uniform_rsrc(p.w_scale + n0, min(p.N - n0, 256) * 4);
           __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 4, (tid & 255) * 4, 0, 0, 0);
         }
       }
       rdB(cb + kUB0, 0);
       rdB(cb + kUB1, 2);
       rdA(cb + kUA0, n4);
+      if constexpr (kMx) {
+        const uint8_t* st = smem + kLdsB + kScalesB + (cb == smem ? 0 : 2048) + (wr * BMH + r16) * 4 + q;
+#pragma unroll
+        for (int i = 0; i < 4 + R1; ++i) sc[i] = st[i * 64];
+      }
       stage(1, nb);
-      if (stored) G8_VM(8 + kStores);
-      else G8_VM(8);
+      if (stored) G8_VM(kAhead + kStores);
+      else G8_VM(kAhead);
       G8_MFMA(n4, 0);
       advance();
       rdA(cb + kUA1, n1);
       stage(0, cb), stage(2, cb), stage(3, cb);
-      if (stored && !(kF8 && left == 1)) G8_VM(8 + kStores);  // (the scales have landed with the tile's last K tile)
-      else G8_VM(8);
+      if (stored && !(kF8 && left == 1)) G8_VM(kAhead + kStores);  // (the scales have landed with the tile's last K tile)
+      else G8_VM(kAhead);
       G8_MFMA(n1, 4);
       stored = false;
     } while (--left > 0);
@@ -423,7 +450,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
       for (int i = 0; i < 4 + R1; ++i) {
         const __amdgpu_buffer_rsrc_t rc = rows_of(p.C, i);
         float as = 1.f;
-        if constexpr (kF8) as = *reinterpret_cast<const float*>(smem + scales + (wr * BMH + 16 * i + (el & 15)) * 4);
+        if constexpr (kF8 && !kMx) as = *reinterpret_cast<const float*>(smem + scales + (wr * BMH + 16 * i + (el & 15)) * 4);
 #pragma unroll
         for (int h = 0; h < NH; ++h) {
           float x[8], y[8];
@@ -434,11 +461,30 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
             x[e] = acc[i][2 * h + e / 4][e % 4];
             if constexpr (kF8) x[e] *= as * ws[h][e];
             if constexpr (EPI == EPI_SWIGLU) x[e] = silu(x[e]) * acc[i][2 + e / 4][e % 4];
-            if constexpr (EPI == EPI_FP8_SWIGLU) x[e] = silu(x[e]) * (acc[i][2 + e / 4][e % 4] * (as * ws[1][e]));
+            if constexpr (kF8 && kSwiglu) x[e] = silu(x[e]) * (acc[i][2 + e / 4][e % 4] * (as * ws[1][e]));
             if constexpr (kBias || EPI == EPI_RESIDUAL) x[e] += y[e];
             if constexpr (EPI == EPI_BIAS_GELU) x[e] = gelu_erf(x[e]);
           }
-          __builtin_amdgcn_raw_buffer_store_b128(pack8(x), rc, vo[h], 0, decltype(policy)::value);
+          if constexpr (!kMxOut) {
+            __builtin_amdgcn_raw_buffer_store_b128(pack8(x), rc, vo[h], 0, decltype(policy)::value);
+          } else {  // the wave's 32 columns of a row are a block, held by four lanes
+            float v[8];
+            unpack8(pack8(x), v);
+            float mx = 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) mx = fmaxf(mx, fabsf(v[e]));
+            const int exp = mx_exp(row_max4(mx)), m = row0 + 16 * i, rows = min(max(p.M - m, 0), 16);
+            const float inv = __builtin_amdgcn_ldexpf(1.f, -exp);
+            uint32_t lo = 0, hi = 0;
+            lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0] * inv, v[1] * inv, lo, false);
+            lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[2] * inv, v[3] * inv, lo, true);
+            hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4] * inv, v[5] * inv, hi, false);
+            hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6] * inv, v[7] * inv, hi, true);
+            const __amdgpu_buffer_rsrc_t r8 = uniform_rsrc((uint8_t*)p.C + (size_t)m * p.ldc + ncol0, rows > 0 ? (rows - 1) * p.ldc + 32 : 0);
+            __builtin_amdgcn_raw_buffer_store_b64(uint2v{lo, hi}, r8, (el & 15) * p.ldc + 8 * (el >> 4), 0, decltype(policy)::value);
+            const __amdgpu_buffer_rsrc_t rm = uniform_rsrc(p.mx_out + ((size_t)(n0 / 256) * p.s_rows + m) * 4, rows * 4);
+            __builtin_amdgcn_raw_buffer_store_b8((uint8_t)(exp + 127), rm, el < 16 ? el * 4 + wc : 0x7ffffff0, 0, 0);
+          }
         }
       }
       };
@@ -457,7 +503,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
 
 template <int EPI, int R1>
 int launch(const Params& p, hipStream_t s) {
-  constexpr int kLds = kLdsB + (EPI >= EPI_FP8 ? kScalesB : 0);
+  constexpr int kLds = kLdsB + (EPI >= EPI_FP8 ? kScalesB : 0) + (EPI == EPI_FP8_MX ? kMxB : 0);
   static bool attr = false;
   if (!attr) {
     (void)hipFuncSetAttribute((const void*)gemm8p_kernel<EPI, R1>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
@@ -593,19 +639,25 @@ extern "C" int lwc_gemm8p(const void* A, const void* W, void* C, const void* R, 
   return -1;
 }
 
-// C [M, N] = (A [M, K] . W [N, K]^T) * a_scale[row] * w_scale[column] of e4m3 A and W, or (swiglu, W's rows gate / up interleaved in
-// blocks of 32) silu(gate) * up [M, N / 2], bf16.  Requires K % 128 == 0, N % 8 == 0 (SwiGLU: 64), lda % 16 == 0 (bytes), ldc % 8 == 0, A, W and
-// C at 16 bytes; ws and flags as lwc_gemm8p's, or null: K is not cut then.
-extern "C" int lwc_gemm8p_fp8(const void* A, const void* W, void* C, const float* a_scale, const float* w_scale, float* ws, int* flags, int M,
-                              int N, int K, int lda, int ldc, int swiglu, hipStream_t s) {
+// C [M, N] = (A [M, K] . W [N, K]^T) * a_scale[row] * w_scale[column] of e4m3 A and W, or (swiglu 1, W's rows gate / up interleaved in
+// blocks of 32) silu(gate) * up [M, N / 2], bf16; swiglu 2: that as e4m3 with block scales mx_out (N % 256 == 0, ldc % 16 == 0, bytes).  a_mx: A's
+// block scales in place of a_scale (swiglu 0).  Scale planes of s_rows rows (gemm8g.hip).  Requires K % 128 == 0, N % 8 == 0 (SwiGLU: 64), lda % 16 == 0
+// (bytes), ldc % 8 == 0, operands at 16 bytes; ws and flags as lwc_gemm8p's, or null: K is not cut then. 
+extern "C" int lwc_gemm8p_fp8(const void* A, const void* W, void* C, const float* a_scale, const float* w_scale, const void* a_mx,
+                              void* mx_out, int s_rows, float* ws, int* flags, int M, int N, int K, int lda, int ldc, int swiglu, hipStream_t s) {
   using namespace lwc::g8p;
-  if (K % 128 != 0 || K < 128 || N % (swiglu ? 64 : 8) != 0 || lda % 16 != 0 || ldc % 8 != 0 || !a_scale || !w_scale) return -1;
+  if (K % 128 != 0 || K < 128 || N % (swiglu ? 64 : 8) != 0 || lda % 16 != 0 || ldc % 8 != 0 || (!a_scale && !a_mx) || !w_scale) return -1;
   if ((long long)M * lda >= (1LL << 31) || 256LL * K >= (1LL << 31) || ldc >= (1 << 26)) return -1;  // 32-bit buffer offsets
+  if (swiglu < 0 || swiglu > 2 || (swiglu && a_mx)) return -1;
+  if (swiglu == 2 && (N % 256 != 0 || !mx_out || s_rows < M || ldc % 16 != 0)) return -1;
+  if (a_mx && (s_rows < M || (long long)(K / 128) * s_rows * 4 >= (1LL << 31))) return -1;
   if (M == 0 || N == 0) return 0;
   Params p{};
   p.A = (const lwc::bf16_t*)A, p.W = (const lwc::bf16_t*)W, p.C = (lwc::bf16_t*)C, p.ws = ws, p.flags = flags;
-  p.a_scale = a_scale, p.w_scale = w_scale;
+  p.a_scale = a_scale, p.w_scale = w_scale, p.a_mx = (const uint8_t*)a_mx, p.mx_out = (uint8_t*)mx_out, p.s_rows = s_rows;
   p.M = M, p.N = N, p.K = K / 2, p.lda = lda / 2, p.ldc = ldc;
   const int r1 = plan(p, swiglu);
-  return swiglu ? launch<EPI_FP8_SWIGLU>(p, r1, s) : launch<EPI_FP8>(p, r1, s);
+  if (swiglu == 2) return launch<EPI_FP8_MX_OUT>(p, r1, s);
+  if (swiglu) return launch<EPI_FP8_SWIGLU>(p, r1, s);
+  return a_mx ? launch<EPI_FP8_MX>(p, r1, s) : launch<EPI_FP8>(p, r1, s);
 }

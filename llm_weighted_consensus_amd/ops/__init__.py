@@ -930,13 +930,16 @@ def _g8g_dense_ok(xq: torch.Tensor, w: "Fp8Weight") -> bool:
             and M >= 0 and 256 * K < (1 << 31) and xq.dtype == torch.float8_e4m3fn)
 
 
-def _fp8_few(M: int, N: int, K: int, ws) -> bool:
-    """Whether a dense fp8 product goes in gemm2g.hip's small tiles: up to 128 of gemm8p's 256 x 256 ones, unless K is long and
-    gemm8p may cut it (``ws``).  us, gemm2g / gemm8p, at 64, 128 and 144 to 160 tiles: K 2048 14.1 / 23.6, 22.2 / 24.4, 32.7 / 25.1; K 4096 23.5 /
-    34.1, 34.9 / 37.9, 47.6 / 37.1; K 8192 40.0 / 42.3, 60.7 / 60.9, 100.2 / 69.7; K 14336 66.0 / 55.1, 101.3 / 91.3, 167.4 / 115.3, at 48 tiles 53.1 to
-    65.6 / 57.6 to 67.3, at 32 53.2 / 46.8."""
+def _fp8_gemm8p(M: int, N: int, K: int, ws, *operands: torch.Tensor) -> bool:
+    """Whether a dense fp8 product goes to gemm8p's kernel, and not to gemm8g_fp8's (of few tiles gemm2g.hip's small ones): more
+    than 128 tiles of 256 x 256, or from 64 on where K is long and may be cut (``ws``).  us, gemm2g / gemm8p, at 64, 128 and 144 to 160 tiles: K
+    2048 14.1 / 23.6, 22.2 / 24.4, 32.7 / 25.1; K 4096 23.5 / 34.1, 34.9 / 37.9, 47.6 / 37.1; K 8192 40.0 / 42.3, 60.7 / 60.9, 100.2 / 69.7; K 14336 66.0 /
+    55.1, 101.3 / 91.3, 167.4 / 115.3, at 48 tiles 53.1 to 65.6 / 57.6 to 67.3, at 32 53.2 / 46.8.  K from 512 on: 8682 x 4096 x 512 from MX, gemm8g / gemm8p, 42.8 / 33.0,
+    8682 x 8192 x 512 SwiGLU to MX 69.5 / 57.5, but at K 256 and 128 22.8 / 33.0 and 22.7 / 62.3.
+    ``operands``: rows and pointers that gemm8p wants at 16 bytes; for others gemm8g_fp8 says what it takes."""
     tiles = -(-M // 256) * -(-N // 256)
-    return tiles <= 128 and (ws is None or K < 12288 or tiles < 64)
+    return K >= 512 and (tiles > 128 or (tiles >= 64 and K >= 12288 and ws is not None)) and all(
+        t.stride(1) == 1 and t.stride(0) * t.element_size() % 16 == 0 and t.stride(0) < 1 << 26 and t.data_ptr() % 16 == 0 for t in operands)
 
 
 G8G_SPAN = 1 << 31  # bytes of A one gemm8g launch may address (its buffer range is 32-bit)
@@ -960,11 +963,8 @@ def gemm8g_dense(xq: torch.Tensor, xs: torch.Tensor, w: "Fp8Weight", out: Option
     for r0 in range(0, M, step):
         r1 = min(M, r0 + step)
         work = _split_workspace(xq.device)
-        # (gemm8p's rows, pointers and reach; anything else goes where those were never asked for)
-        wide = out.stride(1) == 1 and out.stride(0) % 8 == 0 and out.stride(0) < 1 << 26 and not (xq.data_ptr() | out.data_ptr() | w.q.data_ptr()) & 15
-        if wide and not _fp8_few(r1 - r0, N, K, work):
-            part, flags = work or (None, None)
-            kernels().gemm8p_fp8(xq[r0:r1], w.q, out[r0:r1], s[r0:r1], ws, bool(swiglu), part, flags)
+        if _fp8_gemm8p(r1 - r0, N, K, work, xq[r0:r1], w.q, out[r0:r1]):
+            kernels().gemm8p_fp8(xq[r0:r1], w.q, out[r0:r1], s[r0:r1], ws, int(bool(swiglu)), *(work or (None, None)))
         else:
             kernels().gemm8g_fp8(xq[r0:r1], w.q.view(1, N, K), out[r0:r1], None, -(-(r1 - r0) // 256), None, s[r0:r1], ws,
                                  int(bool(swiglu)), None, None)
@@ -1076,23 +1076,31 @@ def linear_fp8_swiglu_mx(x, w: Fp8Weight):
     N, K = w.q.shape
     q = torch.empty(M, N // 2, dtype=torch.float8_e4m3fn, device=xq.device)
     mx = torch.empty(N // 256, M, 4, dtype=torch.uint8, device=xq.device)
-    s, ws, wq = xs.reshape(-1).contiguous(), w.s.reshape(-1), w.q.view(1, N, K)
+    s, ws = xs.reshape(-1).contiguous(), w.s.reshape(-1)
     for r0, r1 in _row_blocks(M, xq.stride(0)):
-        kernels().gemm8g_fp8(xq[r0:r1], wq, q[r0:r1], None, -(-(r1 - r0) // 256), None, s[r0:r1], ws, 2, None,
-                             mx[:, r0:r1])
+        work = _split_workspace(xq.device)
+        if _fp8_gemm8p(r1 - r0, N, K, work, xq[r0:r1], w.q, q[r0:r1]):
+            kernels().gemm8p_fp8(xq[r0:r1], w.q, q[r0:r1], s[r0:r1], ws, 2, *(work or (None, None)), mx_out=mx[:, r0:r1])
+        else:
+            kernels().gemm8g_fp8(xq[r0:r1], w.q.view(1, N, K), q[r0:r1], None, -(-(r1 - r0) // 256), None, s[r0:r1], ws, 2, None,
+                                 mx[:, r0:r1])
     return q, mx
 
 
 def linear_fp8_mx(aq: torch.Tensor, amx: torch.Tensor, w: Fp8Weight) -> torch.Tensor:
-    """(e4m3 [M, K] with MX block scales [K/128, M, 4]) . w^T -> bf16 [M, N] on gemm8g (the scales applied by
-    the block-scaled MFMA)."""
+    """(e4m3 [M, K] with MX block scales [K/128, M, 4]) . w^T -> bf16 [M, N] on the cores of :func:`gemm8g_dense` (the
+    scales applied by the block-scaled MFMA)."""
     M = aq.shape[0]
     N, K = w.q.shape
     out = torch.empty(M, N, dtype=torch.bfloat16, device=aq.device)
-    ws, wq = w.s.reshape(-1), w.q.view(1, N, K)
+    ws = w.s.reshape(-1)
     for r0, r1 in _row_blocks(M, aq.stride(0)):
-        kernels().gemm8g_fp8(aq[r0:r1], wq, out[r0:r1], None, -(-(r1 - r0) // 256), None, None, ws, 0,
-                             amx[:, r0:r1], None)
+        work = _split_workspace(aq.device)
+        if _fp8_gemm8p(r1 - r0, N, K, work, aq[r0:r1], w.q, out[r0:r1]):
+            kernels().gemm8p_fp8(aq[r0:r1], w.q, out[r0:r1], None, ws, 0, *(work or (None, None)), a_mx=amx[:, r0:r1])
+        else:
+            kernels().gemm8g_fp8(aq[r0:r1], w.q.view(1, N, K), out[r0:r1], None, -(-(r1 - r0) // 256), None, None, ws, 0,
+                                 amx[:, r0:r1], None)
     return out
 
 
