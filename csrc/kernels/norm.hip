@@ -61,11 +61,9 @@ __global__ void __launch_bounds__(1024) rmsnorm_kernel(const bf16_t* __restrict_
   }
 }
 
-// Wave-per-row RMSNorm for the decode rows (d = 64 * 8 * VPL, e.g. 4096 -> VPL = 8): a wave owns a whole
-// row, each lane VPL 16-byte vectors (lane-interleaved, so every load / store instruction moves 1 KiB
-// contiguous), all loads issued before the first use, and the reduction is a wave reduction — no LDS, no
-// workgroup barrier.  The workgroup-per-row kernel above spends most of a 4096-wide row's time in its two
-// barriers and a single 16 B load per lane (4.4 TB/s at [4096, 4096]).
+// Wave-per-row RMSNorm (d = 64 * 8 * VPL, 2048 -> VPL = 4): a wave owns a whole row, each lane VPL 16-byte vectors
+// (lane-interleaved, so every load / store instruction moves 1 KiB contiguous), all loads issued before the first use, and the
+// reduction is a wave reduction — no LDS, no workgroup barrier.
 // kQuant: the normalised row is also quantised per row to OCP e4m3 for the fp8 projection that consumes it
 // (config 5's dense fp8 layers): scale = max|bf16(y)| / 448 over the row, q = e4m3(bf16(y) / scale) —
 // exactly quant_fp8_rows(rmsnorm(x)) without writing and re-reading the bf16 row (y may be null then).
@@ -146,28 +144,111 @@ __global__ void __launch_bounds__(256) rmsnorm_wave_kernel(const bf16_t* __restr
   }
 }
 
-template <int VPL>
-static void launch_rmsnorm_wave(const void* x, void* residual, const void* w, void* y, int rows, int d, float eps,
-                                hipStream_t s) {
-  const dim3 grid((rows + 3) / 4);
-  if (residual)
-    rmsnorm_wave_kernel<VPL, true><<<grid, 256, 0, s>>>((const bf16_t*)x, (bf16_t*)residual, (const bf16_t*)w,
-                                                        (bf16_t*)y, rows, d, eps);
-  else
-    rmsnorm_wave_kernel<VPL, false><<<grid, 256, 0, s>>>((const bf16_t*)x, nullptr, (const bf16_t*)w, (bf16_t*)y,
-                                                         rows, d, eps);
+// A workgroup of four waves per row, the row in registers (d = 256 * 8 * NV): the same function, one barrier (two with the
+// quantisation), every load of the row, the residual and the weight on its way before the first use.  Bound by memory, and by one trip
+// to it below some 1000 rows.  us, a wave per row / so, with residual and e4m3 rows: 512 rows of 4096 5.9 / 4.3, 1095 8.1 / 6.4,
+// 8682 39.5 / 36.4 (6.8 TB/s), 512 of 8192 9.2 / 6.0, 4096 42.7 / 35.2; bf16 rows alone: 512 of 4096 3.6 / 3.1, 4096 10.8 / 11.3,
+// 8682 21.8 / 21.5.
+template <int NV, bool kResidual, bool kQuant>
+__global__ void __launch_bounds__(256) rmsnorm_row_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ residual,
+                                                          const bf16_t* __restrict__ w, bf16_t* __restrict__ y, int d, float eps,
+                                                          uint8_t* __restrict__ q, float* __restrict__ qscale) {
+  __shared__ float red[2][4];
+  const size_t row = blockIdx.x;
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const uint4v* xr = reinterpret_cast<const uint4v*>(x + row * d);
+  uint4v* rr = reinterpret_cast<uint4v*>(residual + row * d);
+  const uint4v* wr = reinterpret_cast<const uint4v*>(w);
+  uint4v raw[NV], res[NV], wt[NV];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) raw[k] = xr[tid + 256 * k];
+  if (kResidual) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) res[k] = rr[tid + 256 * k];
+  }
+#pragma unroll
+  for (int k = 0; k < NV; ++k) wt[k] = wr[tid + 256 * k];
+  float ss = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    float a[8];
+    unpack8(raw[k], a);
+    if (kResidual) {
+      float b[8];
+      unpack8(res[k], b);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[j] += b[j];
+      raw[k] = pack8(a);  // the normalised value is computed from the bf16-rounded sum, as the stream holds it
+      rr[tid + 256 * k] = raw[k];
+      unpack8(raw[k], a);
+    }
+#pragma unroll
+    for (int j = 0; j < 8; ++j) ss += a[j] * a[j];
+  }
+  ss = wave_sum(ss);
+  if ((tid & 63) == 0) red[0][wave] = ss;
+  __syncthreads();
+  const float inv = rsqrtf((((red[0][0] + red[0][1]) + red[0][2]) + red[0][3]) / (float)d + eps);
+  float amax = 0.f;
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    float a[8], wf[8], o[8];
+    unpack8(raw[k], a);
+    unpack8(wt[k], wf);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) o[j] = a[j] * inv * wf[j];
+    raw[k] = pack8(o);
+    if (!kQuant || y != nullptr) reinterpret_cast<uint4v*>(y + row * d)[tid + 256 * k] = raw[k];
+    if (kQuant) {
+      unpack8(raw[k], o);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(o[j]));
+    }
+  }
+  if (kQuant) {
+    amax = wave_max(amax);
+    if ((tid & 63) == 0) red[1][wave] = amax;
+    __syncthreads();
+    amax = fmaxf(fmaxf(red[1][0], red[1][1]), fmaxf(red[1][2], red[1][3]));
+    const float sc = fmaxf(amax, 1e-12f) / 448.f;
+    const float qi = 1.f / sc;
+    if (tid == 0) qscale[row] = sc;
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {
+      float v[8];
+      unpack8(raw[k], v);
+      uint32_t lo = 0, hi = 0;
+      lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[0] * qi, v[1] * qi, lo, false);
+      lo = __builtin_amdgcn_cvt_pk_fp8_f32(v[2] * qi, v[3] * qi, lo, true);
+      hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[4] * qi, v[5] * qi, hi, false);
+      hi = __builtin_amdgcn_cvt_pk_fp8_f32(v[6] * qi, v[7] * qi, hi, true);
+      reinterpret_cast<uint2*>(q + row * d)[tid + 256 * k] = make_uint2(lo, hi);
+    }
+  }
 }
 
-template <int VPL>
-static void launch_rmsnorm_wave_q(const void* x, void* residual, const void* w, void* y, int rows, int d, float eps,
-                                  void* q, float* qscale, hipStream_t s) {
-  const dim3 grid((rows + 3) / 4);
-  if (residual)
-    rmsnorm_wave_kernel<VPL, true, true><<<grid, 256, 0, s>>>((const bf16_t*)x, (bf16_t*)residual, (const bf16_t*)w,
-                                                              (bf16_t*)y, rows, d, eps, (uint8_t*)q, qscale);
-  else
-    rmsnorm_wave_kernel<VPL, false, true><<<grid, 256, 0, s>>>((const bf16_t*)x, nullptr, (const bf16_t*)w, (bf16_t*)y,
-                                                               rows, d, eps, (uint8_t*)q, qscale);
+// Rows of 2048 leave a workgroup's thread one vector: above 1024 of them the chip is full of waves either way and a wave per row
+// comes out ahead (512 rows 2.8 / 2.7 us a wave / a workgroup per row, with e4m3 rows 3.5 / 3.2; 2048 rows 4.1 / 4.4 and 4.3 / 4.8).
+constexpr int kRowGroupRows = 1024;
+
+template <int NV, bool kQuant>
+static void launch_rmsnorm(const void* x, void* residual, const void* w, void* y, int rows, int d, float eps, void* q,
+                           float* qscale, hipStream_t s) {
+  const bf16_t* xb = (const bf16_t*)x;
+  const bf16_t* wb = (const bf16_t*)w;
+  bf16_t* rb = (bf16_t*)residual;
+  bf16_t* yb = (bf16_t*)y;
+  uint8_t* qb = (uint8_t*)q;
+  if constexpr (NV == 1) {
+    if (rows > kRowGroupRows) {
+      const int grid = (rows + 3) / 4;
+      if (rb) rmsnorm_wave_kernel<4, true, kQuant><<<grid, 256, 0, s>>>(xb, rb, wb, yb, rows, d, eps, qb, qscale);
+      else rmsnorm_wave_kernel<4, false, kQuant><<<grid, 256, 0, s>>>(xb, rb, wb, yb, rows, d, eps, qb, qscale);
+      return;
+    }
+  }
+  if (rb) rmsnorm_row_kernel<NV, true, kQuant><<<rows, 256, 0, s>>>(xb, rb, wb, yb, d, eps, qb, qscale);
+  else rmsnorm_row_kernel<NV, false, kQuant><<<rows, 256, 0, s>>>(xb, rb, wb, yb, d, eps, qb, qscale);
 }
 
 // LayerNorm with affine: y = (h - mean)/sqrt(var+eps) * g + b, h = x (+ residual);
@@ -353,10 +434,10 @@ extern "C" int lwc_rmsnorm(const void* x, void* residual, const void* w, void* y
   using namespace lwc;
   if (d % 8 != 0 || d > kMaxVec * 8 * 1024) return -1;
   if (rows == 0) return 0;
-  if (rows >= 256 && (d == 4096 || d == 2048 || d == 8192)) {  // decode / prefill rows: a wave per row
-    if (d == 2048) launch_rmsnorm_wave<4>(x, residual, w, y, rows, d, eps, s);
-    else if (d == 4096) launch_rmsnorm_wave<8>(x, residual, w, y, rows, d, eps, s);
-    else launch_rmsnorm_wave<16>(x, residual, w, y, rows, d, eps, s);
+  if (rows >= 256 && (d == 4096 || d == 2048 || d == 8192)) {  // decode / prefill rows, in registers
+    if (d == 2048) launch_rmsnorm<1, false>(x, residual, w, y, rows, d, eps, nullptr, nullptr, s);
+    else if (d == 4096) launch_rmsnorm<2, false>(x, residual, w, y, rows, d, eps, nullptr, nullptr, s);
+    else launch_rmsnorm<4, false>(x, residual, w, y, rows, d, eps, nullptr, nullptr, s);
     return (int)hipGetLastError();
   }
   const int t = norm_threads(d);
@@ -367,7 +448,7 @@ extern "C" int lwc_rmsnorm(const void* x, void* residual, const void* w, void* y
   return (int)hipGetLastError();
 }
 
-// RMSNorm (+ residual) with the per-row e4m3 quantisation of its output fused (wave per row; d in
+// RMSNorm (+ residual) with the per-row e4m3 quantisation of its output fused (the row in registers; d in
 // {2048, 4096, 8192}); y (bf16 output) is optional.  Returns -1 for other widths (the caller runs the two
 // kernels).
 extern "C" int lwc_rmsnorm_quant_fp8(const void* x, void* residual, const void* w, void* y, int rows, int d, float eps,
@@ -375,9 +456,9 @@ extern "C" int lwc_rmsnorm_quant_fp8(const void* x, void* residual, const void* 
   using namespace lwc;
   if (d != 2048 && d != 4096 && d != 8192) return -1;
   if (rows == 0) return 0;
-  if (d == 2048) launch_rmsnorm_wave_q<4>(x, residual, w, y, rows, d, eps, q, qscale, s);
-  else if (d == 4096) launch_rmsnorm_wave_q<8>(x, residual, w, y, rows, d, eps, q, qscale, s);
-  else launch_rmsnorm_wave_q<16>(x, residual, w, y, rows, d, eps, q, qscale, s);
+  if (d == 2048) launch_rmsnorm<1, true>(x, residual, w, y, rows, d, eps, q, qscale, s);
+  else if (d == 4096) launch_rmsnorm<2, true>(x, residual, w, y, rows, d, eps, q, qscale, s);
+  else launch_rmsnorm<4, true>(x, residual, w, y, rows, d, eps, q, qscale, s);
   return (int)hipGetLastError();
 }
 

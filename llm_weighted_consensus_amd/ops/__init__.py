@@ -73,7 +73,7 @@ class QAct:
 def rmsnorm_quant_fp8(x: torch.Tensor, w: torch.Tensor, eps: float, residual: Optional[torch.Tensor] = None,
                       keep_bf16: bool = False) -> QAct:
     """RMSNorm (+ in-place residual update, as :func:`rmsnorm`) with the per-row e4m3 quantisation of its
-    output fused into the same pass (csrc/kernels/norm.hip, wave per row): equal to
+    output fused into the same pass (csrc/kernels/norm.hip): equal to
     ``quant_fp8_rows(rmsnorm(x, ...))``.  Widths the fused kernel does not take run the two kernels."""
     d = x.shape[-1]
     if d not in (2048, 4096, 8192):
