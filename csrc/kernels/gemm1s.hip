@@ -35,6 +35,7 @@ struct Params {
   int tiles, wide;   // a run's tiles, and the blocks of each
   float* part;       // splits > 1: [N / 16][splits][1024] partial sums
   int* count;        // splits > 1: [runs * tiles] finished ranges (zero between launches)
+  int nt;            // weights_pass (common.h)
   int turned;        // a run's walk over its K range starts at a step of its own, 0 .. turned
   RowSumsq ss;       // NORM: read by EPI_PLAIN, EPI_SWIGLU and EPI_ROPE_KV, written by EPI_RESIDUAL
   RopeKV kv;         // EPI_ROPE_KV
@@ -45,8 +46,9 @@ LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
 }
 LWC_DEVICE float silu(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 LWC_DEVICE int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+template <int CP = 0>
 LWC_DEVICE void dma16(const __amdgpu_buffer_rsrc_t& r, uint8_t* dst, uint32_t vo, int so) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, CP);
 }
 LWC_DEVICE void unpack4(const uint2& v, float (&x)[4]) {
   x[0] = __uint_as_float(v.x << 16), x[1] = __uint_as_float(v.x & 0xffff0000u);
@@ -111,10 +113,14 @@ __global__ void __launch_bounds__(512, 2) gemm1s_kernel(const Params p) {
     uint8_t* b = smem + buf * kStage;
 #pragma unroll
     for (int s = 0; s < 2; ++s) dma16(rX, b + s * kA + wid * 1024, voA, load_k + s * 128);
+    auto weights = [&](auto cp) {
 #pragma unroll
-    for (int j = 0; j < IW; ++j)
+      for (int j = 0; j < IW; ++j)
 #pragma unroll
-      for (int s = 0; s < 2; ++s) dma16(rW, b + 2 * kA + s * UW * kUnit + mu * kUnit + (j + mr) * 1024, voW[j], load_k + s * 128);
+        for (int s = 0; s < 2; ++s) dma16<decltype(cp)::value>(rW, b + 2 * kA + s * UW * kUnit + mu * kUnit + (j + mr) * 1024, voW[j], load_k + s * 128);
+    };
+    if (p.nt) weights(std::integral_constant<int, kNT>{});
+    else weights(std::integral_constant<int, 0>{});
     load_k += 256;
     load_k = load_k == past_k ? first_k : load_k;
     if (--load_left == 0) {
@@ -385,7 +391,7 @@ extern "C" int lwc_gemm1s(const void* A, const void* W, void* C, const void* R, 
   while (2 * turned + 2 <= K / 128 / splits) turned = 2 * turned + 1;
   const int blocks = N / (16 * grain);
   const Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc, c.runs, splits,
-                 blocks / c.runs, blocks % c.runs, c.tiles, c.wide, part, count, turned, ss != nullptr ? *ss : lwc::RowSumsq{},
+                 blocks / c.runs, blocks % c.runs, c.tiles, c.wide, part, count, lwc::weights_pass(2LL * N * K), turned, ss != nullptr ? *ss : lwc::RowSumsq{},
                  kv != nullptr ? *kv : lwc::RopeKV{}};
   if (ss != nullptr) {
     switch (epi) {

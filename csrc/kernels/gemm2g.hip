@@ -40,6 +40,7 @@ struct Params {
   uint8_t* mx_out;
   int s_rows;
   int turned;  // a tile's walk over K starts at a step of its own
+  int nt;  // weights_pass (common.h)
 };
 
 LWC_DEVICE float4v mfma8(const uint4v& a0, const uint4v& a1, const uint4v& b0, const uint4v& b1, const float4v& c, int sb) {
@@ -52,8 +53,9 @@ LWC_DEVICE float4v mfma16(const uint4v& a, const uint4v& b, const float4v& c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 LWC_DEVICE float silu8(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
+template <int CP = 0>
 LWC_DEVICE void dma16(const __amdgpu_buffer_rsrc_t& r, uint8_t* dst, uint32_t vo, int so) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, CP);
 }
 LWC_DEVICE void dma4(const __amdgpu_buffer_rsrc_t& r, uint8_t* dst, uint32_t vo, int so) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, vo, so, 0, 0);
@@ -127,8 +129,12 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
     const int kt = step + k0 < nk ? step + k0 : step + k0 - nk;
 #pragma unroll
     for (int i = 0; i < IA; ++i) dma16(rA, buf + (i * 4 + wid) * 1024, voA[i], kt * 128);
+    auto weights = [&](auto cp) {
 #pragma unroll
-    for (int i = 0; i < IW; ++i) dma16(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], kt * 128);
+      for (int i = 0; i < IW; ++i) dma16<decltype(cp)::value>(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], kt * 128);
+    };
+    if (p.nt) weights(std::integral_constant<int, kNT>{});
+    else weights(std::integral_constant<int, 0>{});
     if constexpr (MXA) dma4(rS, buf + kS + wid * 256, voS, kt * p.s_rows * 4);
   };
   // the wave's row tiles are every other one, so that the rows a short group has divide between the waves
@@ -287,7 +293,7 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
   using namespace lwc::g2g;
   if ((!row_off && G != 1) || K % 128 != 0 || K < 128 || N % 8 != 0 || rows <= 0) return -1;
   Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, a_scale, w_scale, G, N, K, lda, ldc, rows_a,
-                 rows, 0, 0, (const uint8_t*)a_mx, (uint8_t*)mx_out, s_rows, 0};
+                 rows, 0, 0, (const uint8_t*)a_mx, (uint8_t*)mx_out, s_rows, 0, 0};
   // The tile that most groups' rows fit, with room for an uneven routing: a second tile reads the weights again, and where the
   // columns give every CU a workgroup already some CUs walk K once more.  us at 64 / 128 / 192 rows a tile, 32 rows a group: bf16
   // [4096, 14336] x 8 (256 columns) 164 / 166 / 172, one expert with four times the rows 238 / 190 / 193, with 130 rows 254 /
@@ -316,6 +322,8 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
     }
   int tm = per <= (cols <= 128 ? 44 : 16) ? 64 : per <= 104 && !(cols > 128 && cols <= 256) ? 128 : 192;
   if (!row_off) tm = nt * ((rows + 63) / 64) <= 512 ? 64 : 128;
+  // (160 rows a group on average: most of an uneven routing's still fit a tile of 192)
+  p.nt = per <= (row_off ? 160 : tm) && lwc::weights_pass((long long)G * N * K);
 #define LWC_G2G(M) \
   case M:          \
     return tm == 64 ? launch<M, 64, 3>(p, rows, s) : tm == 128 ? launch<M, 128, 2>(p, rows, s) : launch<M, 192, 2>(p, rows, s);

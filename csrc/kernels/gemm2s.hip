@@ -28,6 +28,7 @@ struct Params {
   const int* row_off;  // [G + 1]
   const int* a_rows;
   int G, N, K, lda, ldc, rows_a;
+  int nt;  // weights_pass (common.h)
 };
 
 LWC_DEVICE float4v mfma16(const uint4v& a, const uint4v& b, const float4v& c) {
@@ -35,8 +36,9 @@ LWC_DEVICE float4v mfma16(const uint4v& a, const uint4v& b, const float4v& c) {
 }
 LWC_DEVICE float silu8(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 LWC_DEVICE int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+template <int CP = 0>
 LWC_DEVICE void dma16(const __amdgpu_buffer_rsrc_t& r, uint8_t* dst, uint32_t vo, int so) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, CP);
 }
 template <int N>
 LWC_DEVICE void wait_rows() {
@@ -125,8 +127,12 @@ __global__ void __launch_bounds__(512) gemm2s_kernel(const Params p) {
       }
     }
     const __amdgpu_buffer_rsrc_t r = uniform_rsrc(src_w, num_w);
+    auto weights = [&](auto cp) {
 #pragma unroll
-    for (int i = 0; i < IW; ++i) dma16(r, smem + atw + (i * 8 + wid) * 1024, voW[i], uni(kw * 128));
+      for (int i = 0; i < IW; ++i) dma16<decltype(cp)::value>(r, smem + atw + (i * 8 + wid) * 1024, voW[i], uni(kw * 128));
+    };
+    if (p.nt) weights(std::integral_constant<int, kNT>{});
+    else weights(std::integral_constant<int, 0>{});
     ++kw;
     atw = atw == (NW - 1) * kW ? 0 : atw + kW;
   };
@@ -265,7 +271,8 @@ extern "C" int lwc_gemm2s(const void* A, const void* W, void* C, const int* row_
   using namespace lwc::g2s;
   // (a cursor is at most four steps ahead; 32-bit offsets in a tile)
   if (!row_off || K % 128 != 0 || K < 4 * 128 || N % (swiglu ? 64 : 8) != 0 || 256LL * K >= (1LL << 31) || 32LL * ldc >= (1LL << 30)) return -1;
-  const Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, G, N, K, lda, ldc, rows_a};
+  const Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, G, N, K, lda, ldc, rows_a,
+                 lwc::weights_pass((long long)G * N * K)};
   if (swiglu) return tm == 64 ? launch<true, 64, 4, 2>(p, s) : launch<true, 192, 3, 2>(p, s);
   return tm == 64 ? launch<false, 64, 4, 2>(p, s) : launch<false, 192, 3, 2>(p, s);
 }

@@ -33,6 +33,7 @@ struct Params {
   int splits;   // K ranges per tile
   float* part;  // splits > 1: [tiles][splits][TM * TN] partial tiles
   int* count;   // [tiles] finished ranges (zero between launches)
+  int nt;       // weights_pass (common.h)
   int turned;   // > 0: a tile's walk over its K range starts at a step of its own, 0 .. turned
 };
 
@@ -51,8 +52,9 @@ LWC_DEVICE float4v mfma(const uint4v& a, const uint4v& b, const float4v& c) {
 }
 LWC_DEVICE float silu(float x) { return x * __builtin_amdgcn_rcpf(1.f + __expf(-x)); }
 
+template <int CP = 0>
 LWC_DEVICE void dma16(const __amdgpu_buffer_rsrc_t& r, uint8_t* dst, uint32_t vo, int so) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, 0);
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, vo, so, 0, CP);
 }
 
 // every outstanding load but the last N, and all LDS reads
@@ -113,8 +115,12 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const typename ArgsOf<NO
   auto stage = [&](uint8_t* buf) {
 #pragma unroll
     for (int i = 0; i < IA; ++i) dma16(rA, buf + (i * 4 + wid) * 1024, voA[i], next_k);
+    auto weights = [&](auto cp) {
 #pragma unroll
-    for (int i = 0; i < IW; ++i) dma16(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], next_k);
+      for (int i = 0; i < IW; ++i) dma16<decltype(cp)::value>(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], next_k);
+    };
+    if (p.nt) weights(std::integral_constant<int, kNT>{});
+    else weights(std::integral_constant<int, 0>{});
     next_k += 128;
     next_k = next_k == past_k ? first_k : next_k;
   };
@@ -346,6 +352,7 @@ int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
   (void)attr;
   p.tiles_m = (p.M + TM - 1) / TM;
   p.tiles_n = (p.N + TN - 1) / TN;
+  p.nt = p.tiles_m == 1 && weights_pass(2LL * p.N * p.K);
   // W rows of a stride whose low bits are zero lie on few memory channels, and all tiles walk K in step (gemm2g.hip): another
   // first step for each column tile spreads them.  N x K at 24 / 64 / 128 rows, us, before -> after: 16384 x 2048 17 / 17 / 26 -> 15 /
   // 15 / 23, 28672 x 4096 50 / 54 / 59 -> 48 / 52 / 51, 32000 x 4096 55 / 57 / 64 -> 55 / 57 / 52, 8192 x 8192 33 / 33 / 44 -> 27 /
@@ -425,7 +432,7 @@ extern "C" int lwc_gemm2w(const void* A, const void* W, void* C, const void* R, 
   if (((long long)M + 63) / 64 * ((N + 63) / 64) * splits >= (1LL << 31)) return -1;
   if (tile == 4) return lwc_gemm1s(A, W, C, R, M, N, K, lda, ldc, epi, splits, part, count, ss, kv, s);
   const Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc, 0, 0,
-                 splits, part, count, 0};
+                 splits, part, count, 0, 0};
   if (ss != nullptr) {
     const NormParams np{p, *ss, kv != nullptr ? *kv : lwc::RopeKV{}};
     switch (epi) {

@@ -73,7 +73,7 @@ constexpr int kBufB = 4 * kUnitB;   // one K tile: A0 A1 B0 B1
 constexpr int kLdsB = 2 * kBufB;    // 128 KiB
 constexpr int kUA0 = 0, kUA1 = kUnitB, kUB0 = 2 * kUnitB, kUB1 = 3 * kUnitB;
 // cache policy of buffer loads and stores: device scope (past the caches of one XCD), streaming
-constexpr int kSC1 = 16, kNT = 2;
+constexpr int kSC1 = 16;
 constexpr int kPartialF = 256 * 256;  // fp32 partial tile per workgroup
 
 // (fp8: e4m3 A and W, their element counts halved as of bf16, scales of A's rows and W's rows applied to the accumulators)
