@@ -37,6 +37,7 @@ constexpr int kRegSlots = 23;  // of the 32 slots of the 512-thread build
 struct SampleParams {
   const bf16_t* logits;  // [B, ld]
   int ld, V;
+  int nt;                    // rows of more than 131072 tokens: the logits are loaded past the caches
   const float* temperature;  // [B]  (<= 0 -> greedy)
   const float* top_p;        // [B]  (>= 1 -> off)
   const int* top_k;          // [B]  (<= 0 -> off)
@@ -341,14 +342,31 @@ __global__ void __launch_bounds__(T, SLOTS <= 4 ? (PROC && TOPK ? 7 : 8) : SLOTS
   const int nvec = p.V >> 3;
 
   // ---- load the raw row once ----
+  // (With the nt bit where the logits are many: read once, they neither stay in the last-level cache nor push out what it holds.  All
+  // rows of pairs, us without / with it: 4096 rows of 128256 greedy 215 / 177, top-p 0.95 318 / 307, top-k 40 359 / 344, 1500 greedy 85 / 69,
+  // 1024 47 / 48, with the logits written just before 58 / 43; longer rows from 128 MiB of logits on: 4096 of 151936 greedy 286 / 241,
+  // 1000 73 / 68, written just before 79 / 59, 64 11.2 / 12.4.  Shorter rows level within 5 % either way, so not there.)
   uint4v row[RS];
   const uint32_t* lmask =
       (PROC && p.mask_logprobs && p.mask && p.mask_rows[b] >= 0) ? p.mask + (size_t)p.mask_rows[b] * (p.V >> 5) : nullptr;
   if constexpr (VT == 1) {
+    const uint4v none = uint4v{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
+    if (SLOTS > 16 && !PROC && p.nt) {
+#pragma unroll
+      for (int j = 0; j < SLOTS; ++j) {
+        const int vi = j * kSampT + t;
+        row[j] = vi < nvec ? __builtin_nontemporal_load(reinterpret_cast<const uint4v*>(lrow + (size_t)vi * 8)) : none;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < SLOTS; ++j) {
+        const int vi = j * kSampT + t;
+        row[j] = vi < nvec ? *reinterpret_cast<const uint4v*>(lrow + (size_t)vi * 8) : none;
+      }
+    }
 #pragma unroll
     for (int j = 0; j < SLOTS; ++j) {
       const int vi = j * kSampT + t;
-      row[j] = vi < nvec ? *reinterpret_cast<const uint4v*>(lrow + (size_t)vi * 8) : uint4v{0xff80ff80u, 0xff80ff80u, 0xff80ff80u, 0xff80ff80u};
       if (lmask && vi < nvec) {  // constrained logprobs: disallowed tokens are -inf from the start
         const uint32_t bits = (lmask[vi >> 2] >> ((vi & 3) * 8)) & 0xffu;
 #pragma unroll
@@ -372,9 +390,9 @@ __global__ void __launch_bounds__(T, SLOTS <= 4 ? (PROC && TOPK ? 7 : 8) : SLOTS
       const int s = i < LS ? RS + i : i - LS, v0 = s % SLOTS * kSampT + s / SLOTS * T;
       const __amdgpu_buffer_rsrc_t r = uniform_rsrc(lrow + v0 * 8, max(0, nvec - v0) * 16);
       if (i < LS)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(held + i * T + w0), 16, t * 16, 0, 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)(held + i * T + w0), 16, t * 16, 0, 0, kNT);
       else
-        row[i < LS ? 0 : s] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(r, t * 16, 0, 0));
+        row[i < LS ? 0 : s] = __builtin_bit_cast(uint4v, __builtin_amdgcn_raw_buffer_load_b128(r, t * 16, 0, kNT));
     }
     __builtin_amdgcn_sched_barrier(0);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(RS) : "memory");
@@ -1047,7 +1065,7 @@ extern "C" int lwc_sample(const void* logits, int ld, int V, int B, const float*
   using namespace lwc;
   if (V % 32 != 0 || num_logprobs < 0 || num_logprobs > kMaxTopK) return -1;
   if (B == 0) return 0;
-  SampleParams p{(const bf16_t*)logits, ld, V, temperature, top_p, top_k, min_p, top_a, freq_pen, pres_pen, rep_pen,
+  SampleParams p{(const bf16_t*)logits, ld, V, 2LL * B * V >= 128 << 20, temperature, top_p, top_k, min_p, top_a, freq_pen, pres_pen, rep_pen,
                  (uint16_t*)counts, count_rows, bias, bias_rows, mask, mask_rows, seeds, offsets, num_logprobs,
                  mask_logprobs, need_logprob, out_token, out_logprob, out_topk_ids, out_topk_lp};
   const int nvec = V / 8;
