@@ -198,11 +198,7 @@ LWC_DEVICE void pair_softmax(const float4v& sa, const float4v& sb, int blkA, boo
   }
   l += row_sum4(rs);
   // P operand (A): k order {A: 4g+0..3, B: 4g+0..3}
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    pf[i] = (short)f2bf(pa[i]);
-    pf[4 + i] = (short)f2bf(pb[i]);
-  }
+  pf = __builtin_bit_cast(short8, uint4v{pack_bf16x2(pa[0], pa[1]), pack_bf16x2(pa[2], pa[3]), pack_bf16x2(pb[0], pb[1]), pack_bf16x2(pb[2], pb[3])});
 }
 
 // O += P V for the pair: per n-tile pair m, four K = 16 MFMAs (block A's and block B's 4 tokens per lane
@@ -289,12 +285,15 @@ LWC_DEVICE void load_q(short8 (&qf)[4], const DecodeParams& p, int row_seq0, int
       const float4 s1 = *reinterpret_cast<const float4*>(p.rope_sin + (size_t)pos * (kD / 2) + c + 4);
       const float cs[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
       const float sn[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
+      float y1[8], y2[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
         const float x1 = bf2f((bf16_t)qf[s][e]), x2 = bf2f((bf16_t)qf[s + 2][e]);
-        qf[s][e] = (short)f2bf(x1 * cs[e] - x2 * sn[e]);
-        qf[s + 2][e] = (short)f2bf(x2 * cs[e] + x1 * sn[e]);
+        y1[e] = x1 * cs[e] - x2 * sn[e];
+        y2[e] = x2 * cs[e] + x1 * sn[e];
       }
+      qf[s] = __builtin_bit_cast(short8, pack8(y1));
+      qf[s + 2] = __builtin_bit_cast(short8, pack8(y2));
     }
   }
 }

@@ -34,8 +34,12 @@ LWC_DEVICE bf16_t f2bf(float f) {
   return *reinterpret_cast<bf16_t*>(&b);
 }
 
+// (As one conversion of a pair: put together from two single ones, of which the compiler makes each an instruction, a shift and an or, a
+// pair took four instructions instead of one.)
 LWC_DEVICE uint32_t pack_bf16x2(float lo, float hi) {
-  return (uint32_t)f2bf(lo) | ((uint32_t)f2bf(hi) << 16);
+  typedef float float2v __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(float2v{lo, hi}, bf16x2));
 }
 
 // 16-byte vector of 8 bf16 <-> 8 floats.
@@ -51,6 +55,16 @@ LWC_DEVICE uint4v pack8(const float (&f)[8]) {
 #pragma unroll
   for (int i = 0; i < 4; ++i) v[i] = pack_bf16x2(f[2 * i], f[2 * i + 1]);
   return v;
+}
+// f as hi + lo, each rounded to bf16
+LWC_DEVICE void split8(const float (&f)[8], short8& hi, short8& lo) {
+  const uint4v h = pack8(f);
+  float r[8];
+  unpack8(h, r);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) r[e] = f[e] - r[e];
+  hi = __builtin_bit_cast(short8, h);
+  lo = __builtin_bit_cast(short8, pack8(r));
 }
 
 LWC_DEVICE float wave_sum(float v) {

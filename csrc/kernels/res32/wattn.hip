@@ -297,12 +297,7 @@ __global__ void __launch_bounds__(256, 2) window_attn_mfma_kernel(const WAttnMfm
 #pragma unroll
         for (int e = 0; e < 8; ++e) x[e] = qp[e];
       }
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const bf16_t hi = f2bf(x[e]);
-        qhi[qs][kd][e] = (short)hi;
-        qlo[qs][kd][e] = (short)f2bf(x[e] - bf2f(hi));
-      }
+      split8(x, qhi[qs][kd], qlo[qs][kd]);
     }
   const int w_min = pos0 + wrow, w_max = min(w_min + 16 * QS - 1, pos_last);  // this wave's positions
   const int w_lo_min = lo_of(w_min), w_lo_max = lo_of(max(w_max, w_min));     // and their first visible keys
@@ -463,12 +458,7 @@ __global__ void __launch_bounds__(256, 2) window_attn_mfma_kernel(const WAttnMfm
         }
 #pragma unroll
         for (int e = 0; e < 8; ++e) l[qs] += pe[e];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const bf16_t hi = f2bf(pe[e]);
-          ph[qs][e] = (short)hi;
-          pl[qs][e] = (short)f2bf(pe[e] - bf2f(hi));
-        }
+        split8(pe, ph[qs], pl[qs]);
       }
 #pragma unroll
       for (int n = 0; n < NV; ++n) {

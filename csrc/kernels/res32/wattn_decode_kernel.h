@@ -251,12 +251,7 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
     l = l * alpha + psum;
     m = m_new;
     short8 ph, pl;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const bf16_t hi = f2bf(pe[e]);
-      ph[e] = (short)hi;
-      pl[e] = (short)f2bf(pe[e] - bf2f(hi));
-    }
+    split8(pe, ph, pl);
     float ar[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) ar[r] = __shfl(alpha, 4 * g4 + r, 64);
