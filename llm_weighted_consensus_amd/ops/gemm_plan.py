@@ -126,7 +126,12 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
     4096 1.04 to 1.09. From 17 to 32 rows the library keeps all: both cores gain on some weights (4096 x 2048 0.72 and 0.91,
     4096 x 14336 1.2 and 0.87) and lose on others (8192 x 4096 1.27 and 1.18). Down from 65 to 128 on gemm2w, whose K ranges fill
     the CUs that a few column tiles leave idle: 14 weights of 2048 to 4096 x 8192 to 18688 0.30 to 0.95, but 4608 x 12288,
-    5120 x 8192 and 13824 0.92 to 1.37; 129 to 144 rows, a third row tile, up to 1.40."""
+    5120 x 8192 and 13824 0.92 to 1.37; 129 to 144 rows, a third row tile, up to 1.40.
+
+    With the weights past the caches (``weights_pass``, csrc/kernels/common.h) gemm2w also leads at up to 32 rows of a head, 32000 to
+    151936 x 4096, 50304 and 151936 x 2048, 32768 x 5120, 65536 x 8192 0.46 to 0.99 (128256 x 4096, 5 rows 183 us -> 152; 33 to 64 rows
+    up to 1.07; 30522 x 1024 is 16 us on either), and down at up to 24, 4096 x 11008 and 14336, 5120 x 13824, 8192 x 28672 0.54 to 1.01
+    (4096 x 8192 up to 1.08; plain 8192 x 28672 1.07)."""
     size = N * K
     if epi == "swiglu":
         if M > 4608:  # (M * N: 32-bit byte offsets)
@@ -140,6 +145,10 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
             4096 < M <= 4608 or 6144 < M <= 7424 or 8192 < M <= 12032 or 12288 < M <= 13824):
         return "g8"
     if epi == "residual" and 64 < M <= 128 and 2048 <= N <= 4096 and K >= 8192 and size <= 1 << 26:
+        return "g2"
+    if epi == "plain" and M <= 32 and N >= 32000 and 2048 <= K <= 8192 and 3 << 25 <= size < 1 << 30:
+        return "g2"
+    if epi == "residual" and M <= 24 and 4096 <= N <= 8192 and K >= 11008 and size < 1 << 28:
         return "g2"
     if M <= 16 and K <= 4096 and N <= 8 * K and 1 << 22 <= size <= 1 << 24:
         return "gv"

@@ -70,6 +70,36 @@ def test_untuned_rule(M, N, K, epi, core):
     assert gemm_plan._untuned(M, N, K, epi) == core
 
 
+@pytest.mark.parametrize("N,K,epi,rows", [
+    (128256, 4096, "plain", {1: "g2", 32: "g2", 33: "blas"}), (32000, 4096, "plain", {5: "g2"}), (31992, 4096, "plain", {5: "blas"}),
+    (50304, 2048, "plain", {1: "g2"}), (49144, 2048, "plain", {1: "blas"}), (151936, 1984, "plain", {1: "blas"}), (65536, 8256, "plain", {1: "blas"}),
+    (131072, 8192, "plain", {1: "blas"}), (128256, 4096, "residual", {5: "blas"}),
+    (4096, 14336, "residual", {1: "g2", 24: "g2", 25: "blas"}), (4096, 14336, "plain", {5: "blas"}), (4088, 14336, "residual", {5: "blas"}),
+    (4096, 11008, "residual", {24: "g2"}), (4096, 10944, "residual", {24: "blas"}), (8192, 28672, "residual", {1: "g2"}), (8200, 28672, "residual", {1: "blas"}),
+    (8192, 32768, "residual", {1: "blas"})])
+def test_untuned_rule_of_few_rows(N, K, epi, rows):
+    assert {M: gemm_plan._untuned(M, N, K, epi) for M in rows} == rows
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("N,K,epi", [(32008, 4096, "plain"), (50304, 2048, "plain"), (4104, 11072, "residual"), (5120, 13824, "residual")])
+def test_untuned_few_rows_of_wide_and_deep_weights(gpu, N, K, epi):
+    """The results of both against fp64 of the same operands (bound: one bf16 rounding, doubled; fp32 sums), rows of another stride and
+    a residual off 16 bytes, which the library keeps, among them."""
+    g = torch.Generator().manual_seed(K)
+    W = (torch.randn(N, K, generator=g) * K ** -0.5).to(torch.bfloat16).to(gpu)
+    for M in (1, 5, 16, 17, 24):
+        A = torch.randn(M, K + 8, generator=g).to(torch.bfloat16).to(gpu)[:, :K]
+        if epi == "plain":
+            got, ref = gemm_plan.linear(A, W), A.double() @ W.double().t()
+            torch.testing.assert_close(got.double(), ref, rtol=2 ** -8, atol=2e-4)
+            continue
+        for off in (0, 1):
+            C = torch.randn(M * N + off, generator=g).to(torch.bfloat16).to(gpu)[off:].view(M, N)
+            ref = A.double() @ W.double().t() + C.double()
+            torch.testing.assert_close(gemm_plan.linear_add_(A, W, C).double(), ref, rtol=2 ** -8, atol=2e-4)
+
+
 @pytest.mark.parametrize("times,core", [
     ({"blas": 100, "g8": 89}, "g8"), ({"blas": 100, "g8": 91}, "blas"), ({"blas": 100, "g8": 101}, "blas"), ({"blas": 100, "g2": 102}, "g2"),
     ({"blas": 100, "g2": 104}, "blas"), ({"blas": 100, "g8": 95, "g2": 102}, "g2"), ({"blas": 100, "g8": 95, "g2": 104}, "blas"),
