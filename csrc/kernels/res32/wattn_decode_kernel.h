@@ -75,13 +75,19 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
   const int BS = p.block_size, bsh = p.bs_shift;
   auto page_ix = [&](int j) { return j >> bsh; };
   auto page_off = [&](int j) { return j & (BS - 1); };
-  // the split's pages, one per lane, fetched once: a key's page then comes from a lane exchange instead of a table
-  // load that every K / V load would have to wait for (splits longer than 64 pages look the table up directly)
-  const int pg_base = page_ix(base);
-  const bool pages_in_lanes = page_ix(base + keys_per_split - 1) - pg_base < 64;
-  int my_page = 0;
-  if (pages_in_lanes && pg_base + lane <= page_ix(max(i, 0)) && base <= i) my_page = table[pg_base + lane];
-  auto page_of = [&](int j) { return pages_in_lanes ? __shfl(my_page, page_ix(j) - pg_base, 64) : table[page_ix(j)]; };
+  // 64 pages from the tile at hand's, one per lane: a key's page then comes from a lane exchange instead of a table load that
+  // every K / V load would have to wait for.  A tile and the next one's rows need 64 pages at most.  (The exchange in `look_up` is the
+  // load's wait, in the branch that loads: behind it, or behind a choice between lanes and table, the compiler waits for every load on
+  // its way, three times a tile and, with wide rows, at every row that a thread stages.  us, so / here, cold: 576 / 512 entries, 32
+  // heads, 64 rows of 500 to 1500 keys 98 / 61, of 4000 199 / 122, one of 4000 54 / 33; 320 / 256, 16 heads 49 / 32, 97 / 68, 36 / 25; 128 /
+  // 128, 32 heads over 8, 255 rows of 400 58 / 51, 64 of 20 to 60 15.6 / 13.1, 64 of 500 to 1500 67 / 68, which memory bounds.)
+  int pg_base = 0, my_page = 0;
+  auto look_up = [&](int t0) {
+    pg_base = page_ix(t0);
+    my_page = __shfl(table[min(pg_base + lane, page_ix(i))], lane, 64);
+  };
+  if (base <= last) look_up(base);
+  auto page_of = [&](int j) { return __shfl(my_page, page_ix(j) - pg_base, 64); };
   const bool h_valid = r16 < nh;
   const int h = h0 + (h_valid ? r16 : 0);
 
@@ -94,21 +100,23 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
   short8 qhi[NDW], qlo[QLO ? NDW : 1];
 #pragma unroll
   for (int kd = 0; kd < NDW; ++kd) {
+    typedef float float4u __attribute__((ext_vector_type(4), aligned(4)));
+    const float4u* qp = reinterpret_cast<const float4u*>(p.q + ((size_t)b * H + h) * D + (kd0 + kd) * 32 + 8 * g4);
+    const float4u x0 = qp[0], x1 = qp[1];
+    float x[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      float x = 0.f;
-      if (h_valid) x = p.q[((size_t)b * H + h) * D + (kd0 + kd) * 32 + 8 * g4 + e];
-      const bf16_t hi = f2bf(x);
-      qhi[kd][e] = (short)hi;
-      if (QLO) qlo[kd][e] = (short)f2bf(x - bf2f(hi));
-    }
+    for (int e = 0; e < 8; ++e) x[e] = h_valid ? e < 4 ? x0[e] : x1[e - 4] : 0.f;
+    short8 lo;
+    split8(x, qhi[kd], lo);
+    if (QLO) qlo[kd] = lo;
   }
   float4v O[NVW];
 #pragma unroll
   for (int n = 0; n < NVW; ++n) O[n] = float4v{0.f, 0.f, 0.f, 0.f};
   float m = -1e30f, l = 0.f;
   const float cap_k = p.cap > 0.f ? 2.0f * 1.4426950408889634f / p.cap : 0.f;
-  const float* bias_h = p.bias ? p.bias + (size_t)h * p.window : nullptr;  // no table: no distance bias
+  const bool biased = p.bias != nullptr;  // no table: no distance bias
+  const float* bias_h = p.bias + (size_t)h * p.window;
 
   constexpr bool kStage = NW > 1;
   constexpr int KLD = D + 8;                                       // LDS row stride: rows start in different banks
@@ -142,7 +150,7 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
   // One wave alone (no LDS): a tile's value words and the next tile's key rows are in flight while the scores and the
   // weights of the tile are formed.  (Rows past the split's keys are masked below: any valid row does.)
   short8 kf[kStage ? 1 : 2 * ND];
-  short4v vf[kStage ? 1 : 2 * NVW];
+  uint4v vf[kStage ? 1 : NVW];
   auto load_keys = [&](int t0) {
 #pragma unroll
     for (int sub = 0; sub < 2; ++sub) {
@@ -153,13 +161,14 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
     }
   };
   auto value_row = [&](int j) {
-    return p.v_cache + (long long)page_of(j) * p.vb_stride + (long long)(page_off(j) >> 2) * (4LL * G * DV) + 4LL * (g * DV + r16);
+    return p.v_cache + (long long)page_of(j) * p.vb_stride + (long long)(page_off(j) >> 2) * (4LL * G * DV) + 4LL * (g * DV + (kStage ? 1 : 2) * r16);
   };
   if constexpr (!kStage) {
     if (base <= last) load_keys(base);
   }
 
   for (int t0 = base; t0 <= last; t0 += 32) {  // (base and last are the same for every wave of the workgroup)
+    if (page_ix(t0 + 63) - pg_base >= 64) look_up(t0);
     if (kStage && t0 + 32 <= last) fetch(t0 + 32);
     // the lane's two 4-key groups: keys t0 + 4 g4 .. and t0 + 16 + 4 g4 .. (groups past the token: any valid one,
     // their weights are 0)
@@ -170,15 +179,15 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
       vb = value_row(jb);
     }
     float bias_e[8];
-    if (bias_h) {
+    if (biased) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) bias_e[e] = bias_h[min(max(i - (t0 + (e >> 2) * 16 + 4 * g4 + (e & 3)), 0), p.window - 1)];
     }
     if constexpr (!kStage) {
 #pragma unroll
-      for (int n = 0; n < NVW; ++n) {
-        vf[2 * n] = *reinterpret_cast<const short4v*>(va + 64 * n);
-        vf[2 * n + 1] = *reinterpret_cast<const short4v*>(vb + 64 * n);
+      for (int n = 0; n < NVW; n += 2) {  // two columns, 32 n + 2 r16 and the one after it, four keys of each
+        vf[n] = *reinterpret_cast<const uint4v*>(va + 64 * n);
+        vf[n + 1] = *reinterpret_cast<const uint4v*>(vb + 64 * n);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -233,7 +242,7 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
       const int j = t0 + (e >> 2) * 16 + 4 * g4 + (e & 3);
       const int dist = i - j;
       ok[e] = h_valid && dist >= 0 && j >= j_lo && j <= last;
-      s[e] = ok[e] ? sacc[e >> 2][e & 3] - (bias_h ? bias_e[e] : 0.f) : -1e30f;
+      s[e] = ok[e] ? sacc[e >> 2][e & 3] - (biased ? bias_e[e] : 0.f) : -1e30f;
       mx = fmaxf(mx, s[e]);
     }
     mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
@@ -268,8 +277,8 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
           bb[4 + e] = (short)col[(16 + e) * KLD];
         }
       } else if constexpr (!kStage) {
-        const short4v b0 = vf[2 * n], b1 = vf[2 * n + 1];
-        bb = short8{b0[0], b0[1], b0[2], b0[3], b1[0], b1[1], b1[2], b1[3]};
+        const uint4v &b0 = vf[n & ~1], &b1 = vf[n | 1];
+        bb = __builtin_bit_cast(short8, uint4v{b0[2 * (n & 1)], b0[2 * (n & 1) + 1], b1[2 * (n & 1)], b1[2 * (n & 1) + 1]});
       } else {
         const short4v b0 = *reinterpret_cast<const short4v*>(va + 64 * (wv * NVW + n));
         const short4v b1 = *reinterpret_cast<const short4v*>(vb + 64 * (wv * NVW + n));
@@ -291,7 +300,7 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
     if (hr < nh && base <= last) {
       float* po = p.part_o + (((size_t)b * H + h0 + hr) * p.S + split) * DV;
 #pragma unroll
-      for (int n = 0; n < NVW; ++n) po[(wv * NVW + n) * 16 + r16] = O[n][r];
+      for (int n = 0; n < NVW; ++n) po[kStage ? (wv * NVW + n) * 16 + r16 : 32 * (n / 2) + 2 * r16 + n % 2] = O[n][r];
     }
   }
   if (g4 == 0 && h_valid && wv == 0) {
