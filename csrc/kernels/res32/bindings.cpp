@@ -34,7 +34,7 @@ int r32_delta_rule(float*, int, const void*, int, int, int, const float*, const 
                    const int*, const int*, float*, int, int, int, int, int, int, int, int, hipStream_t);
 int r32_head_norm_gate(const float*, int, const void*, int, const float*, void*, int, int, int, int, float, int, int,
                        hipStream_t);
-int r32_embed_rows(const void*, const int*, float*, int, int, int, float, void*, int, hipStream_t);
+int r32_embed_rows(const void*, const int*, float*, int, int, int, float, void*, float*, int, hipStream_t);
 int r32_head_norm_kv_write(const void*, int, int, int, const int*, const int*, float*, void*, void*, long long, long long,
                            int, int, int, int, int, int, float, float, float, int, int, hipStream_t);
 int r32_gate_mul(void*, int, const void*, int, int, int, int, int, hipStream_t);
@@ -478,8 +478,8 @@ void head_norm_gate(Tensor o, c10::optional<Tensor> gate, c10::optional<Tensor> 
                           stream()), "head_norm_gate");
 }
 
-// cast (bf16 [T, d], or absent) also receives the rows
-void embed_rows(Tensor table, Tensor tokens, Tensor out, double scale, c10::optional<Tensor> cast) {
+// cast (bf16 [T, d], or absent) and twin (as out, or absent) also receive the rows
+void embed_rows(Tensor table, Tensor tokens, Tensor out, double scale, c10::optional<Tensor> cast, c10::optional<Tensor> twin) {
   const int f = act_f32(table, "embed_rows table");
   TORCH_CHECK(table.dim() == 2 && table.is_contiguous(), "embed_rows: table [V, d]");
   want(tokens, torch::kInt32, "embed_rows tokens");
@@ -492,8 +492,12 @@ void embed_rows(Tensor table, Tensor tokens, Tensor out, double scale, c10::opti
     TORCH_CHECK(cast->numel() == out.numel(), "embed_rows: cast [T, d]");
     cp = cast->data_ptr();
   }
-  done(r32_embed_rows(table.data_ptr(), tokens.data_ptr<int>(), out.data_ptr<float>(), T, d, (int)table.size(0), (float)scale, cp, f,
-                      stream()), "embed_rows");
+  if (twin.has_value()) {
+    want(*twin, torch::kFloat32, "embed_rows twin");
+    TORCH_CHECK(twin->numel() == out.numel(), "embed_rows: twin [T, d]");
+  }
+  done(r32_embed_rows(table.data_ptr(), tokens.data_ptr<int>(), out.data_ptr<float>(), T, d, (int)table.size(0), (float)scale, cp,
+                      twin.has_value() ? twin->data_ptr<float>() : nullptr, f, stream()), "embed_rows");
 }
 
 // proj [T, ...] row-dense: q at column 0 (H*D), k at k_off (G*D), values at v_off (G*Dv; v_off == k_off: the keys as

@@ -1,6 +1,6 @@
 // Layer plumbing of fp32-residual designs with gated, post-normalised sublayers (gfx950, wave64).
 //
-//   embed_rows           x[t] = table[token[t]] * scale as fp32 (optionally also as bf16 rows)
+//   embed_rows           x[t] = table[token[t]] * scale as fp32 (optionally also as bf16 rows, or twice)
 //   head_norm_kv_write   from fused projection rows: q and k divided by their root mean square PER HEAD (no weight);
 //                        q times scale * (1 + coef ln(floor((p + 1) / every) + 1)) into an fp32 buffer; normalised k
 //                        into the paged K cache; the values (a projection of their own, or the keys as projected,
@@ -18,7 +18,7 @@ namespace {
 
 template <typename AT>
 __global__ void embed_rows_kernel(const AT* __restrict__ table, const int* __restrict__ tokens, float* __restrict__ out,
-                                  int d, int vocab, float scale, bf16_t* __restrict__ cast) {
+                                  int d, int vocab, float scale, bf16_t* __restrict__ cast, float* __restrict__ twin) {
   const int t = blockIdx.x;
   int tok = tokens[t];
   tok = tok < 0 ? 0 : (tok >= vocab ? vocab - 1 : tok);
@@ -27,6 +27,7 @@ __global__ void embed_rows_kernel(const AT* __restrict__ table, const int* __res
     const float v = Elem<AT>::ld(row + i) * scale;
     out[(size_t)t * d + i] = v;
     if (cast) cast[(size_t)t * d + i] = f2bf(v);
+    if (twin) twin[(size_t)t * d + i] = v;
   }
 }
 
@@ -35,7 +36,7 @@ __global__ void embed_rows_kernel(const AT* __restrict__ table, const int* __res
 template <typename AT>
 __global__ void __launch_bounds__(256) embed_rows_vec_kernel(const AT* __restrict__ table, const int* __restrict__ tokens,
                                                               float* __restrict__ out, int d, int vocab, float scale,
-                                                              bf16_t* __restrict__ cast) {
+                                                              bf16_t* __restrict__ cast, float* __restrict__ twin) {
   const size_t t = blockIdx.x;
   const int tok = min(max(tokens[t], 0), vocab - 1);
   const AT* row = table + (size_t)tok * d;
@@ -44,6 +45,7 @@ __global__ void __launch_bounds__(256) embed_rows_vec_kernel(const AT* __restric
     const float4v v = Vec4<AT>::ld(row + i) * scale;
     Vec4<float>::st(out + t * d + i, v);
     if (cast) Vec4<bf16_t>::st(cast + t * d + i, v);
+    if (twin) Vec4<float>::st(twin + t * d + i, v);
   }
 }
 
@@ -332,16 +334,16 @@ int blocks_for(long long total) { return (int)((total + 255) / 256 < 65536 ? (to
 using namespace lwc;
 
 extern "C" int r32_embed_rows(const void* table, const int* tokens, float* out, int T, int d, int vocab, float scale, void* cast,
-                              int f32, hipStream_t s) {
+                              float* twin, int f32, hipStream_t s) {
   if (T <= 0) return 0;
-  if (d % 4 == 0 && vocab > 0 && aligned_to(table, f32 ? 16 : 8) && aligned_to(out, 16) && aligned_to(cast, 8)) {
-    if (f32) embed_rows_vec_kernel<float><<<T, 256, 0, s>>>((const float*)table, tokens, out, d, vocab, scale, (bf16_t*)cast);
-    else embed_rows_vec_kernel<bf16_t><<<T, 256, 0, s>>>((const bf16_t*)table, tokens, out, d, vocab, scale, (bf16_t*)cast);
+  if (d % 4 == 0 && vocab > 0 && aligned_to(table, f32 ? 16 : 8) && aligned_to(out, 16) && aligned_to(cast, 8) && aligned_to(twin, 16)) {
+    if (f32) embed_rows_vec_kernel<float><<<T, 256, 0, s>>>((const float*)table, tokens, out, d, vocab, scale, (bf16_t*)cast, twin);
+    else embed_rows_vec_kernel<bf16_t><<<T, 256, 0, s>>>((const bf16_t*)table, tokens, out, d, vocab, scale, (bf16_t*)cast, twin);
     LWC_CHECK_LAUNCH();
     return 0;
   }
-  if (f32) embed_rows_kernel<float><<<T, 256, 0, s>>>((const float*)table, tokens, out, d, vocab, scale, (bf16_t*)cast);
-  else embed_rows_kernel<bf16_t><<<T, 256, 0, s>>>((const bf16_t*)table, tokens, out, d, vocab, scale, (bf16_t*)cast);
+  if (f32) embed_rows_kernel<float><<<T, 256, 0, s>>>((const float*)table, tokens, out, d, vocab, scale, (bf16_t*)cast, twin);
+  else embed_rows_kernel<bf16_t><<<T, 256, 0, s>>>((const bf16_t*)table, tokens, out, d, vocab, scale, (bf16_t*)cast, twin);
   LWC_CHECK_LAUNCH();
   return 0;
 }

@@ -358,9 +358,9 @@ class LatentDecoder:
         return res32.rmsnorm_rows(x, self.final_w, self.cfg.norm_eps, self.dtype, rows=rows)
 
     def _logits(self, x, rows: Optional[torch.Tensor], float_logits: bool) -> torch.Tensor:
-        lg = self._linear(self._output_rows(x, rows), self._head()).float()
+        lg = self._linear(self._output_rows(x, rows), self._head())
         if float_logits:
-            return lg
+            return lg.float()
         V, Vp = self.cfg.vocab_size, self.logit_width
         if Vp == V:
             return lg.to(torch.bfloat16)

@@ -334,8 +334,7 @@ class MerudraModel:
         T, d, eps, nl = tokens.shape[0], cfg.hidden, cfg.norm_eps, len(self.layers)
         exact = dt == torch.float32
         X = torch.empty(nl + 1, T, d, dtype=torch.float32, device=self.device)  # every layer's result stays resident
-        res32.embed_rows(self.embed, tokens, X[0])
-        X[1].copy_(X[0])
+        res32.embed_rows(self.embed, tokens, X[0], twin=X[1])
         xb = None if exact else torch.empty(T, d, dtype=dt, device=self.device)
         for li, (S, L) in enumerate(zip(cfg.layer_specs, self.layers)):
             m, x = S.mixer, X[li + 1]
@@ -383,9 +382,9 @@ class MerudraModel:
 
     def _logits(self, x: torch.Tensor, rows: Optional[torch.Tensor], float_logits: bool) -> torch.Tensor:
         h = res32.rmsnorm_rows(x, self.final_w, self.cfg.norm_eps, self.dtype, rows=rows)
-        lg = self._linear(h, self.head).float()
+        lg = self._linear(h, self.head)
         if float_logits:
-            return lg
+            return lg.float()
         V, Vp = self.cfg.vocab_size, self.logit_width
         if Vp == V:
             return lg.to(torch.bfloat16)

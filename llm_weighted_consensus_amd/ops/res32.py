@@ -199,11 +199,11 @@ def head_norm_gate(o: torch.Tensor, out: torch.Tensor, H: int, eps: float, w: Op
 
 
 def embed_rows(table: torch.Tensor, tokens: torch.Tensor, out: Optional[torch.Tensor] = None,
-               scale: float = 1.0, cast: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """x[t] = table[tokens[t]] * scale as fp32; ``cast`` (bf16 [T, d]) also receives the rows."""
+               scale: float = 1.0, cast: Optional[torch.Tensor] = None, twin: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """x[t] = table[tokens[t]] * scale as fp32; ``cast`` (bf16 [T, d]) and ``twin`` (fp32) also receive the rows."""
     if out is None:
         out = torch.empty(tokens.numel(), table.shape[1], dtype=torch.float32, device=table.device)
-    kernels().embed_rows(table, tokens, out, float(scale), cast)
+    kernels().embed_rows(table, tokens, out, float(scale), cast, twin)
     return out
 
 
