@@ -80,7 +80,7 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
   // load's wait, in the branch that loads: behind it, or behind a choice between lanes and table, the compiler waits for every load on
   // its way, three times a tile and, with wide rows, at every row that a thread stages.  us, so / here, cold: 576 / 512 entries, 32
   // heads, 64 rows of 500 to 1500 keys 98 / 61, of 4000 199 / 122, one of 4000 54 / 33; 320 / 256, 16 heads 49 / 32, 97 / 68, 36 / 25; 128 /
-  // 128, 32 heads over 8, 255 rows of 400 58 / 51, 64 of 20 to 60 15.6 / 13.1, 64 of 500 to 1500 67 / 68, which memory bounds.)
+  // 128, 32 heads over 8, 255 rows of 400 58 / 52, 64 of 20 to 60 15.6 / 13.0, 64 of 500 to 1500 67 / 66.5, which memory bounds.)
   int pg_base = 0, my_page = 0;
   auto look_up = [&](int t0) {
     pg_base = page_ix(t0);
@@ -147,8 +147,8 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
     __syncthreads();
   }
 
-  // One wave alone (no LDS): a tile's value words and the next tile's key rows are in flight while the scores and the
-  // weights of the tile are formed.  (Rows past the split's keys are masked below: any valid row does.)
+  // One wave alone (no LDS): a tile's value words are in flight while the scores and the weights of the tile are formed, the next
+  // tile's key rows while it is summed.  (Rows past the split's keys are masked below: any valid row does.)
   short8 kf[kStage ? 1 : 2 * ND];
   uint4v vf[kStage ? 1 : NVW];
   auto load_keys = [&](int t0) {
@@ -225,11 +225,6 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
       }
     }
     }  // (scores without the split)
-    if constexpr (!kStage) {
-      __builtin_amdgcn_sched_barrier(0);
-      load_keys(t0 + 32);
-      __builtin_amdgcn_sched_barrier(0);
-    }
     if (p.cap > 0.f) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) sacc[e >> 2][e & 3] = softcap_f(sacc[e >> 2][e & 3], p.cap, cap_k);
@@ -259,6 +254,11 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
     psum += __shfl_xor(psum, 32, 64);
     l = l * alpha + psum;
     m = m_new;
+    if constexpr (!kStage) {  // (ahead of the softmax, keys and values in flight at once: 64 rows of 500 to 1500 keys 68 us for 66.5)
+      __builtin_amdgcn_sched_barrier(0);
+      load_keys(t0 + 32);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     short8 ph, pl;
     split8(pe, ph, pl);
     float ar[4];
