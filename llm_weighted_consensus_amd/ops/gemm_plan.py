@@ -130,8 +130,8 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
 
     With the weights past the caches (``weights_pass``, csrc/kernels/common.h) gemm2w also leads at up to 32 rows of a head, 32000 to
     151936 x 4096, 50304 and 151936 x 2048, 32768 x 5120, 65536 x 8192 0.46 to 0.99 (128256 x 4096, 5 rows 183 us -> 152; 33 to 64 rows
-    up to 1.07; 30522 x 1024 is 16 us on either), and down at up to 24, 4096 x 11008 and 14336, 5120 x 13824, 8192 x 28672 0.54 to 1.01
-    (4096 x 8192 up to 1.08; plain 8192 x 28672 1.07)."""
+    up to 1.07; 30522 x 1024 is 16 us on either), and down at up to 24, 4096 x 11008 and 14336, 5120 x 13824 0.54 to 1.01 (4096 x
+    8192 up to 1.08)."""
     size = N * K
     if epi == "swiglu":
         if M > 4608:  # (M * N: 32-bit byte offsets)
@@ -148,7 +148,7 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
         return "g2"
     if epi == "plain" and M <= 32 and N >= 32000 and 2048 <= K <= 8192 and 3 << 25 <= size < 1 << 30:
         return "g2"
-    if epi == "residual" and M <= 24 and 4096 <= N <= 8192 and K >= 11008 and size < 1 << 28:
+    if epi == "residual" and M <= 24 and 4096 <= N <= 5120 and 11008 <= K <= 14336:
         return "g2"
     if M <= 16 and K <= 4096 and N <= 8 * K and 1 << 22 <= size <= 1 << 24:
         return "gv"

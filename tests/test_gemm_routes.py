@@ -75,8 +75,8 @@ def test_untuned_rule(M, N, K, epi, core):
     (50304, 2048, "plain", {1: "g2"}), (49144, 2048, "plain", {1: "blas"}), (151936, 1984, "plain", {1: "blas"}), (65536, 8256, "plain", {1: "blas"}),
     (131072, 8192, "plain", {1: "blas"}), (128256, 4096, "residual", {5: "blas"}),
     (4096, 14336, "residual", {1: "g2", 24: "g2", 25: "blas"}), (4096, 14336, "plain", {5: "blas"}), (4088, 14336, "residual", {5: "blas"}),
-    (4096, 11008, "residual", {24: "g2"}), (4096, 10944, "residual", {24: "blas"}), (8192, 28672, "residual", {1: "g2"}), (8200, 28672, "residual", {1: "blas"}),
-    (8192, 32768, "residual", {1: "blas"})])
+    (4096, 11008, "residual", {24: "g2"}), (4096, 10944, "residual", {24: "blas"}), (5120, 14336, "residual", {1: "g2"}), (5128, 14336, "residual", {1: "blas"}),
+    (4096, 14400, "residual", {1: "blas"})])
 def test_untuned_rule_of_few_rows(N, K, epi, rows):
     assert {M: gemm_plan._untuned(M, N, K, epi) for M in rows} == rows
 
