@@ -71,10 +71,11 @@ int launch_decode_nv(const WAttnDecodeParams& p, int nv, dim3 grid, hipStream_t 
 }
 
 // Splits for a decode step of B sequences whose windows hold at most max_keys keys: about 2048 waves (two per SIMD, the
-// registers' limit).  Measured with contexts of 500 to 1500 keys of 128, 8 kv heads: at 64 sequences 2 splits 65 us, 4
-// (2048 waves) 54 us, 6 61 us, 8 56 us, 16 66 us; at 8 sequences 8 splits 22 us, 16 19 us, 32 (2048 waves) 20 us, 64 22 us.
+// registers' limit).  Measured, cold, with contexts of 500 to 1500 keys of 128, 8 kv heads: at 64 sequences 2 splits 63 us, 4
+// (2048 waves) 67, 6 67, 8 67, 16 72; at 8 sequences of 1000 2 splits 31, 4 22, 8 19, 16 and 32 20.  (1024 waves: 0.82 to 0.98 of the time for
+// equal contexts of 128 entries, a step of 64 rows level; up to 1.15 for 100 to 3000 keys, 64 entries up to 1.48.)
 // Wide rows (D = 320, 576): workgroups of four waves, about 512 of them, or of eight (more than 16 heads), at most 256 of them
-// (one per CU: at 64 sequences x 32 heads x 576 / 512 4 splits take 74 us where 8 take 94 us), at least 128 keys each (their
+// (one per CU: at 64 sequences of 500 to 1500 keys x 32 heads x 576 / 512 2 / 4 / 8 splits take 81 / 54 / 63 us), at least 128 keys each (their
 // partials are large).
 extern "C" int r32_window_attn_decode_splits(int B, int G, int Hg, int max_keys, int D) {
   const bool wide = D > 192;
