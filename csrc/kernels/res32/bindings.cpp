@@ -23,6 +23,7 @@ int r32_window_attn_mfma(const float*, const void*, const void*, long long, long
                          hipStream_t);
 int r32_window_attn_decode_ok(int, int, int);
 int r32_window_attn_decode_splits(int, int, int, int, int);
+void r32_window_attn_decode_heads(int, int, int, int*, int*);
 int r32_window_attn_decode(const float*, const void*, const void*, long long, long long, int, const int*, const int*, int,
                            const float*, const float*, int, int, float, float*, float*, int, void*, int, int, int, int, int, int, int,
                            hipStream_t);
@@ -1113,6 +1114,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("window_attn_mfma_ok", &window_attn_mfma_ok);
   m.def("window_attn_decode_ok", &window_attn_decode_ok);
   m.def("window_attn_decode", &window_attn_decode);
+  m.def("window_attn_decode_heads", [](int64_t H, int64_t G, int64_t D) {
+    TORCH_CHECK(G > 0 && H > 0 && H % G == 0, "window_attn_decode_heads: head counts");
+    int lo, hi;
+    r32_window_attn_decode_heads((int)H, (int)G, (int)D, &lo, &hi);
+    return std::make_pair(lo, hi);
+  });
   m.def("conv_hist", &conv_hist);
   m.def("conv_hist_update", &conv_hist_update);
   m.def("delta_rule", &delta_rule);

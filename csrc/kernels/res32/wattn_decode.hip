@@ -88,6 +88,22 @@ extern "C" int r32_window_attn_decode_splits(int B, int G, int Hg, int max_keys,
   return s < 1 ? 1 : s;
 }
 
+// Head chunks that share a workgroup: two where one wide row serves more than 16 heads.
+static int chunks_per_group(int Hg, int D) { return D > 192 && Hg > 16 ? 2 : 1; }
+
+// The lowest and highest of a sequence's heads whose q and bias the decode kernel loads, over all its workgroups and waves.
+extern "C" void r32_window_attn_decode_heads(int H, int G, int D, int* lo, int* hi) {
+  const int Hg = H / G, nc = chunks_per_group(Hg, D), chunks = (Hg + 15) / 16;
+  *lo = H, *hi = -1;
+  for (int y = 0; y < G * ((chunks + nc - 1) / nc); ++y)
+    for (int cw = 0; cw < nc; ++cw)
+      for (int r16 = 0; r16 < 16; ++r16) {
+        const int h = loaded_head(head_chunk(y, cw, nc, Hg), r16);
+        if (h < *lo) *lo = h;
+        if (h > *hi) *hi = h;
+      }
+}
+
 // part_o: fp32 [B * H * S * Dv], part_ml: fp32 [B * H * S * 2] scratch of the caller.
 extern "C" int r32_window_attn_decode(const float* q, const void* k_cache, const void* v_cache, long long kb_stride,
                                       long long vb_stride, int block_size, const int* positions, const int* block_tables,
@@ -109,7 +125,7 @@ extern "C" int r32_window_attn_decode(const float* q, const void* k_cache, const
   const dim3 grid(B, G * ((Hg + 15) / 16), S);
   int rc = -1;
   if (D > 192) {  // one wide row for all heads: a low-rank attention's cached latent + rotated part
-    const int chunks = (Hg + 15) / 16, nc = chunks > 1 ? 2 : 1;  // more than 16 heads: two chunks per workgroup
+    const int chunks = (Hg + 15) / 16, nc = chunks_per_group(Hg, D);
     rc = r32_window_attn_decode_wide_launch(&p, D, B, G * ((chunks + nc - 1) / nc), S, nc, s);
   } else {
     switch (D / 32) {

@@ -40,6 +40,20 @@ struct WAttnDecodeParams {
   int H, G, S, min_keys;  // min_keys: the fewest keys a split takes before the next one gets any (a multiple of 32)
 };
 
+struct HeadChunk {
+  int g, h0, nh, last;  // kv head; first head, heads (<= 0: a wave past the last chunk only helps staging); the kv head's last one
+};
+// Chunk cw of the NC (below) of workgroup y.
+LWC_HOST_DEVICE HeadChunk head_chunk(int y, int cw, int NC, int Hg) {
+  const int cgroups = ((Hg + 15) / 16 + NC - 1) / NC;  // workgroups per kv head
+  const int g = y / cgroups, h0 = g * Hg + ((y % cgroups) * NC + cw) * 16, end = g * Hg + Hg;
+  return {g, h0, end - h0 < 16 ? end - h0 : 16, end - 1};
+}
+// The head whose q (and bias) column r16 of the MFMA loads: a column, or a whole wave, that has none loads one that there is
+LWC_HOST_DEVICE int loaded_head(const HeadChunk& c, int r16) {
+  return r16 < c.nh ? c.h0 + r16 : c.h0 < c.last ? c.h0 : c.last;
+}
+
 // NW waves per workgroup share one (sequence, head chunk, split).  With NW > 1 a tile's 32 key rows go through LDS
 // once for all the waves (fetched into registers one tile ahead), and each wave owns NV / NW of the 16-column value
 // tiles (wide value rows: the accumulators of one wave would leave no registers for loads in flight).  NW = 4: the
@@ -55,13 +69,12 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
   constexpr int D = 32 * ND, DV = 16 * NV, NVW = NV / NW, NT = 64 * NW * NC;  // NT: threads of the workgroup
   static_assert(NV % NW == 0, "value tiles divide among the waves");
   const int b = blockIdx.x, split = blockIdx.z;
-  const int H = p.H, G = p.G, Hg = H / G, chunks = (Hg + 15) / 16;
+  const int H = p.H, G = p.G;
   // (one wave: the wave index is a compile-time zero, so the value tiles' offsets stay immediates)
   const int lane = NT > 64 ? (int)(threadIdx.x & 63) : (int)threadIdx.x, wv_all = NT > 64 ? (int)(threadIdx.x >> 6) : 0;
   const int wv = NC > 1 ? wv_all % NW : wv_all, cw = NC > 1 ? wv_all / NW : 0;
-  const int cgroups = (chunks + NC - 1) / NC;  // workgroups per kv head
-  const int g = blockIdx.y / cgroups, h0 = g * Hg + ((blockIdx.y % cgroups) * NC + cw) * 16;
-  const int nh = min(16, g * Hg + Hg - h0);  // heads of this chunk (<= 0: a wave past the last chunk only helps staging)
+  const HeadChunk heads = head_chunk(blockIdx.y, cw, NC, H / G);
+  const int g = heads.g, h0 = heads.h0, nh = heads.nh;
   const int r16 = lane & 15, g4 = lane >> 4;
   const int i = p.positions[b];
   const int j_lo = max(max(0, i - p.window + 1), p.chunk > 0 ? i - i % p.chunk : 0);
@@ -89,7 +102,7 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
   if (base <= last) look_up(base);
   auto page_of = [&](int j) { return __shfl(my_page, page_ix(j) - pg_base, 64); };
   const bool h_valid = r16 < nh;
-  const int h = h0 + (h_valid ? r16 : 0);
+  const int h = loaded_head(heads, r16);
 
   // With NW = 4 staged waves the scores of a tile are formed ONCE per chunk: wave w multiplies key subtile (w & 1) with
   // half (w >> 1) of the row's 32-entry slices, the halves meet through LDS.  Such a wave keeps only its half of q.
