@@ -35,6 +35,7 @@ int lwc_gemm8p(const void*, const void*, void*, const void*, float*, int*, int, 
 int lwc_gemm8p_fp8(const void*, const void*, void*, const float*, const float*, const void*, void*, int, float*, int*, int, int, int, int, int,
                    int, hipStream_t);
 int lwc_gemm8p_slots();
+int lwc_gemm8p_mx_bytes(int, int, int, int);
 void lwc_gemm2w_plan(int, int, int, int, bool, long long, int*, int*);
 int lwc_gemm2w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, int, float*, int*,
                const lwc::RowSumsq*, const lwc::RopeKV*, hipStream_t);
@@ -1287,6 +1288,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm8p", &gemm8p);
   m.def("gemm8p_fp8", &gemm8p_fp8, py::arg("A"), py::arg("W"), py::arg("C"), py::arg("a_scale"), py::arg("w_scale"), py::arg("swiglu"),
         py::arg("ws"), py::arg("flags"), py::arg("a_mx") = py::none(), py::arg("mx_out") = py::none());
+  m.def("gemm8p_mx_bytes", &lwc_gemm8p_mx_bytes);
   m.def("gemm2w", &gemm2w);
   m.def("gemm4w", &gemm4w);
   m.def("skinny_gemm", &skinny_gemm);

@@ -116,6 +116,10 @@ LWC_DEVICE float4v mfma8(const uint4v (&a)[2], const uint4v (&b)[2], const float
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 0, 0, 0, 127, 0, sb);
 }
 
+// Bytes from row m0 of A's first plane of block scales to the end of its last one: M rows of s_rows there, which other calls' may follow,
+// or the tensor's end
+LWC_HOST_DEVICE int mx_bytes(int planes, int s_rows, int M, int m0) { return ((planes - 1) * s_rows + M - m0) * 4; }
+
 // x * sigmoid(x) with v_rcp_f32 (1 ulp) instead of the IEEE division sequence (v_div_scale x2, v_div_fmas,
 // v_div_fixup around an rcp: ~9 VALU per element in an epilogue of 256 per lane); the result is rounded
 // to bf16 (or e4m3) anyway.  x -> -inf: rcp(inf) = 0, x * 0 = -0 as the division gives
@@ -237,7 +241,7 @@ __global__ void __launch_bounds__(512) gemm8p_kernel(Params p) {
     if constexpr (kMx) {
       if (u == 0) {  // the scales of the K tile's rows, four bytes a row
         auto* dst = (__attribute__((address_space(3))) void*)(smem + kLdsB + kScalesB + (buf == smem ? 0 : 2048) + wid * 256);
-        const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(p.a_mx + (size_t)mS * 4, numA ? (KT * p.s_rows - mS) * 4 : 0);
+        const __amdgpu_buffer_rsrc_t rs = uniform_rsrc(p.a_mx + (size_t)mS * 4, numA ? mx_bytes(KT, p.s_rows, p.M, mS) : 0);
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, dst, 4, (tid & 255) * 4, kt * p.s_rows * 4, 0, 0);
       }
     }
@@ -638,6 +642,9 @@ extern "C" int lwc_gemm8p(const void* A, const void* W, void* C, const void* R, 
   }
   return -1;
 }
+
+// What a tile from row m0 on may read of A's block scales (for tests).
+extern "C" int lwc_gemm8p_mx_bytes(int planes, int s_rows, int M, int m0) { return lwc::g8p::mx_bytes(planes, s_rows, M, m0); }
 
 // C [M, N] = (A [M, K] . W [N, K]^T) * a_scale[row] * w_scale[column] of e4m3 A and W, or (swiglu 1, W's rows gate / up interleaved in
 // blocks of 32) silu(gate) * up [M, N / 2], bf16; swiglu 2: that as e4m3 with block scales mx_out (N % 256 == 0, ldc % 16 == 0, bytes).  a_mx: A's
