@@ -191,6 +191,55 @@ def test_encoder_layers_with_the_library_launched_natively(gpu, monkeypatch, cor
                   False, False) is None
 
 
+@pytest.mark.parametrize("how", ["dual weight", "dual bias", "mode", "subclass"])
+def test_encoder_layers_with_the_library_stay_visible(gpu, monkeypatch, how):
+    """Layers with projections on the library run call by call where forward-mode duals, a dispatch mode or a subclass
+    would see those calls (out= forms refuse duals), and give the same bits."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from llm_weighted_consensus_amd import ops
+    from llm_weighted_consensus_amd.models.bert import BertEncoder
+    from llm_weighted_consensus_amd.models.config import encoder_config
+    from llm_weighted_consensus_amd.ops import gemm_plan
+
+    m = BertEncoder(encoder_config("bge-small-en-v1.5"), device=gpu, seed=5)
+    args = m.pack([[(7 * i + j) % 900 + 1 for j in range(n)] for i, n in enumerate([64, 29])])
+    monkeypatch.setattr(gemm_plan, "MODE", "blas")
+    taken, native = [], ops.encoder_layers_mixed
+    monkeypatch.setattr(ops, "encoder_layers_mixed", lambda *a: taken.append(native(*a)) or taken[-1])
+    want = m.forward_packed(*args)
+    assert taken.pop() is want
+    L, calls = m.layers[3], []
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, a=(), kw=None):
+            calls.append(func.name())
+            return func(*a, **(kw or {}))
+
+    class Other(torch.Tensor):
+        @classmethod
+        def __torch_function__(cls, func, types, a=(), kw=None):
+            calls.append(func.__name__)
+            with torch._C.DisableTorchFunctionSubclass():
+                return func(*a, **(kw or {}))
+
+    if how == "mode":
+        with Seen():
+            got = m.forward_packed(*args)
+        assert calls.count("aten::addmm") >= 24
+    elif how == "subclass":
+        L.wo = L.wo.as_subclass(Other)
+        got = m.forward_packed(*args)
+        assert "linear" in calls
+    else:
+        with forward_ad.dual_level():
+            n = "wo" if how == "dual weight" else "bo"
+            monkeypatch.setattr(L, n, forward_ad.make_dual(getattr(L, n), torch.ones_like(getattr(L, n))))
+            got = forward_ad.unpack_dual(m.forward_packed(*args)).primal
+    assert taken == [None] and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("core", [0, 4, -1])
 def test_encoder_layers_refuse_other_cores(gpu, core):
     """A core that no kernel stands for is an error, not gemm2w."""
