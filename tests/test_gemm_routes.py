@@ -81,8 +81,17 @@ def test_untuned_rule_of_few_rows(N, K, epi, rows):
     assert {M: gemm_plan._untuned(M, N, K, epi) for M in rows} == rows
 
 
+@pytest.mark.parametrize("N,K,rows", [
+    (4608, 12288, {1: "blas", 24: "blas"}), (4736, 11008, {1: "blas", 24: "blas"}), (4160, 13952, {8: "blas"}), (4744, 11264, {1: "g2", 24: "g2"}),
+    (4096, 12288, {1: "blas", 16: "blas", 17: "g2"}), (4096, 13824, {16: "blas", 24: "g2"}), (4096, 13952, {1: "g2", 16: "g2"}), (4096, 11072, {1: "g2"}),
+    (5120, 13824, {1: "blas", 7: "blas", 8: "g2", 24: "g2"}), (5120, 13312, {1: "g2"}), (4992, 14080, {5: "g2"})])
+def test_untuned_down_of_few_rows(N, K, rows):
+    """Inside the range of down projections that gemm2w takes: widths and depths at which the library measured faster keep it."""
+    assert {M: gemm_plan._untuned(M, N, K, "residual") for M in rows} == rows
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("N,K,epi", [(32008, 4096, "plain"), (50304, 2048, "plain"), (4104, 11072, "residual"), (5120, 13824, "residual")])
+@pytest.mark.parametrize("N,K,epi", [(32008, 4096, "plain"), (50304, 2048, "plain"), (4104, 11072, "residual"), (5120, 13824, "residual"), (4096, 11072, "residual"), (4744, 11072, "residual")])
 def test_untuned_few_rows_of_wide_and_deep_weights(gpu, N, K, epi):
     """The results of both against fp64 of the same operands (bound: one bf16 rounding, doubled; fp32 sums), rows of another stride and
     a residual off 16 bytes, which the library keeps, among them."""
