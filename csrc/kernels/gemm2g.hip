@@ -40,7 +40,7 @@ struct Params {
   uint8_t* mx_out;
   int s_rows;
   int turned;  // a tile's walk over K starts at a step of its own
-  int nt;  // weights_pass (common.h)
+  int nt;  // weights_pass (common.h), for the groups of one tile
 };
 
 LWC_DEVICE float4v mfma8(const uint4v& a0, const uint4v& a1, const uint4v& b0, const uint4v& b1, const float4v& c, int sb) {
@@ -94,11 +94,13 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
   const int ntile = local % nj * 8 + xcd;
   if (ntile >= p.n_tiles) return;
   int slot = local / nj, g = 0, m_begin = 0, m_end = 0;
+  bool once = false;  // the weights are read by this tile alone
   for (; g < p.G; ++g) {
     const int r0 = p.row_off ? p.row_off[g] : 0, r1 = p.row_off ? p.row_off[g + 1] : p.rows, nt = (r1 - r0 + TM - 1) / TM;
     if (slot < nt) {
       m_begin = r0 + slot * TM;
       m_end = min(r1, m_begin + TM);
+      once = p.nt && nt == 1;
       break;
     }
     slot -= nt;
@@ -133,7 +135,7 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
 #pragma unroll
       for (int i = 0; i < IW; ++i) dma16<decltype(cp)::value>(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], kt * 128);
     };
-    if (p.nt) weights(std::integral_constant<int, kNT>{});
+    if (once) weights(std::integral_constant<int, kNT>{});
     else weights(std::integral_constant<int, 0>{});
     if constexpr (MXA) dma4(rS, buf + kS + wid * 256, voS, kt * p.s_rows * 4);
   };
@@ -322,7 +324,7 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
     }
   int tm = per <= (cols <= 128 ? 44 : 16) ? 64 : per <= 104 && !(cols > 128 && cols <= 256) ? 128 : 192;
   if (!row_off) tm = nt * ((rows + 63) / 64) <= 512 ? 64 : 128;
-  // (160 rows a group on average: most of an uneven routing's still fit a tile of 192)
+  // (160 rows a group on average: with more, 180 or 192 in each group, gate|up loses 1.5 % by it)
   p.nt = per <= (row_off ? 160 : tm) && lwc::weights_pass((long long)G * N * K);
 #define LWC_G2G(M) \
   case M:          \

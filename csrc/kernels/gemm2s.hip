@@ -28,7 +28,7 @@ struct Params {
   const int* row_off;  // [G + 1]
   const int* a_rows;
   int G, N, K, lda, ldc, rows_a;
-  int nt;  // weights_pass (common.h)
+  int nt;  // weights_pass (common.h), for the groups of one tile
 };
 
 LWC_DEVICE float4v mfma16(const uint4v& a, const uint4v& b, const float4v& c) {
@@ -61,9 +61,10 @@ LWC_DEVICE Groups groups_at(const Params& p, int g0, int tm) {
   return t;
 }
 
-// Tile t: columns n0 .. n1 of group g's weights times its rows begin .. end (slot: which row tile of all groups)
+// Tile t: columns n0 .. n1 of group g's weights times its rows begin .. end (slot: which row tile of all groups; once: the group's only one)
 struct Tile {
   int slot, g, begin, end, n0, n1;
+  bool once;
 };
 LWC_DEVICE Tile tile_of(const Params& p, const Groups& first, int t, int n_tiles, int tm, int tn) {
   Tile c;
@@ -81,6 +82,7 @@ LWC_DEVICE Tile tile_of(const Params& p, const Groups& first, int t, int n_tiles
   c.g = g0 + l;
   c.begin = uni(r0 + (slot - __builtin_amdgcn_readlane(gr.upto, l) + (r1 - r0 + tm - 1) / tm) * tm);
   c.end = uni(min(r1, c.begin + tm));
+  c.once = r1 - r0 <= tm;
   return c;
 }
 
@@ -115,6 +117,7 @@ __global__ void __launch_bounds__(512) gemm2s_kernel(const Params p) {
   }
   // the weights' and the rows' cursors; behind the last tile the same instructions without a memory request
   int tw = first, kw = nk, atw = 0, num_w = 0;
+  bool past = false;  // the weights at hand pass the caches by
   const uint8_t* src_w = p.W;
   auto stage_w = [&] {
     if (kw == nk) {
@@ -124,6 +127,7 @@ __global__ void __launch_bounds__(512) gemm2s_kernel(const Params p) {
         const Tile c = tile_of(p, groups, tw++, n_tiles, TM, TN);
         src_w = p.W + ((size_t)c.g * p.N + c.n0) * p.K;
         num_w = (c.n1 - c.n0) * p.K;
+        past = p.nt && c.once;
       }
     }
     const __amdgpu_buffer_rsrc_t r = uniform_rsrc(src_w, num_w);
@@ -131,7 +135,7 @@ __global__ void __launch_bounds__(512) gemm2s_kernel(const Params p) {
 #pragma unroll
       for (int i = 0; i < IW; ++i) dma16<decltype(cp)::value>(r, smem + atw + (i * 8 + wid) * 1024, voW[i], uni(kw * 128));
     };
-    if (p.nt) weights(std::integral_constant<int, kNT>{});
+    if (past) weights(std::integral_constant<int, kNT>{});
     else weights(std::integral_constant<int, 0>{});
     ++kw;
     atw = atw == (NW - 1) * kW ? 0 : atw + kW;
