@@ -36,6 +36,7 @@ int lwc_gemm8p_fp8(const void*, const void*, void*, const float*, const float*, 
                    int, hipStream_t);
 int lwc_gemm8p_slots();
 int lwc_gemm8p_mx_bytes(int, int, int, int);
+int lwc_gemm2w_past_caches(int, int, int, int, int);
 void lwc_gemm2w_plan(int, int, int, int, bool, long long, int*, int*);
 int lwc_gemm2w(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, int, float*, int*,
                const lwc::RowSumsq*, const lwc::RopeKV*, hipStream_t);
@@ -1285,6 +1286,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("gemm8p_fp8", &gemm8p_fp8, py::arg("A"), py::arg("W"), py::arg("C"), py::arg("a_scale"), py::arg("w_scale"), py::arg("swiglu"),
         py::arg("ws"), py::arg("flags"), py::arg("a_mx") = py::none(), py::arg("mx_out") = py::none());
   m.def("gemm8p_mx_bytes", &lwc_gemm8p_mx_bytes);
+  m.def("gemm2w_past_caches", [](int M, int N, int K, int tm, int tn) { return lwc_gemm2w_past_caches(M, N, K, tm, tn) != 0; });
   m.def("gemm2w", &gemm2w);
   m.def("gemm4w", &gemm4w);
   m.def("skinny_gemm", &skinny_gemm);

@@ -101,13 +101,15 @@ LWC_DEVICE float block_max(float v, float* scratch) {
 // Weights that a call reads once, in one tile of rows, are loaded with the nt bit where there are at least 32 MiB of them: a model of
 // such layers does not stay in the last-level cache (256 MiB) from one call to the next, and loads that claim no place there run at up
 // to 6.6 TB/s instead of 5.9.  us, without / with it, weights from memory: gemm1s 61 x 28672 x 4096 42.3 / 39.3, 4096 x 4096 (32 MiB) 11.7
-// / 11.0; gemm2w 16 x 128256 x 4096 182 / 158 (61 rows 196 / 199), 61 x 4096 x 14336 26.9 / 25.1; gemm2s 8 x 16 rows x 14336 x 4096 166 / 152;
-// gemm2g bf16 [4096, 7168] x 8 of 16 rows 79 / 70, fp8 [28672, 4096] x 8 of 16 and 128 rows 158 / 139 and 187 / 184, [4096, 14336] x 8 of 128
-// 108 / 94.  A second tile of rows then reads from memory too (gemm2w 1000 x 128256 x 4096 1019 / 1420, gemm2g fp8 8 x 250 rows x 28672 x 4096
-// 313 / 402), so that a group of several tiles takes its weights through the caches among others that do not: us, without it / with it for all / for
-// groups of one tile, 28672 x 4096 fp8, 8 groups, 210, 205, 200, 198, 90, 60, 40, 20 rows 236 / 277 / 231, two of 300 among 20s 228 / 246 / 216,
-// bf16 14336 x 4096 245 / 285 / 244 and 229 / 254 / 218, 4096 x 14336 331 / 343 / 311 and 283 / 302 / 278.  And weights that would have been in the cache lose: 24 MiB of 3072 x 1024 4 %, a single 10240 x 8192 called again
-// and again 46 / 73.  Partial reads of a line too (skinny.hip, 1 x 128256 x 4096 163 / 180).
+// / 11.0; gemm2w 16 x 128256 x 4096 182 / 158 (more rows: past_caches there), 61 x 4096 x 14336 26.9 / 25.1; gemm2s 8 x 16 rows x 14336 x
+// 4096 166 / 152; gemm2g bf16 [4096, 7168] x 8 of 16 rows 79 / 70, fp8 [28672, 4096] x 8 of 16 and 128 rows 158 / 139 and 187 / 184, [4096,
+// 14336] x 8 of 128 108 / 94.
+// A second tile of rows then reads from memory too (gemm2w 1000 x 128256 x 4096 1019 / 1420, gemm2g fp8 8 x 250 rows x 28672 x 4096 313 / 402), so a
+// group of several tiles takes its weights through the caches among others that do not.  us, without / with it for all / for groups of
+// one tile, 28672 x 4096 fp8, 8 groups: 210, 205, 200, 198, 90, 60, 40, 20 rows 236 / 277 / 231, two of 300 among 20s 228 / 246 / 216; bf16
+// 14336 x 4096 245 / 285 / 244 and 229 / 254 / 218, 4096 x 14336 331 / 343 / 311 and 283 / 302 / 278.
+// Weights that would have been in the cache lose: 24 MiB of 3072 x 1024 4 %, a single 10240 x 8192 called again and again 46 / 73.  Partial
+// reads of a line too (skinny.hip, 1 x 128256 x 4096 163 / 180).
 constexpr int kNT = 2;  // a buffer load's nt bit
 constexpr int weights_pass(long long bytes) { return bytes >= 32LL << 20; }
 

@@ -33,7 +33,7 @@ struct Params {
   int splits;   // K ranges per tile
   float* part;  // splits > 1: [tiles][splits][TM * TN] partial tiles
   int* count;   // [tiles] finished ranges (zero between launches)
-  int nt;       // weights_pass (common.h)
+  int nt;       // past_caches
   int turned;   // > 0: a tile's walk over its K range starts at a step of its own, 0 .. turned
 };
 
@@ -344,6 +344,16 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const typename ArgsOf<NO
   }
 }
 
+// Whether the weights of a call in tiles of tm x tn pass the caches by (weights_pass, common.h): where one tile of rows reads them, but not from
+// 49 rows on where they are wide, nor in tiles of 192 rows.  Time with it over without, weights from memory: 64 x 64 tiles up to 48 rows 0.85 to
+// 0.99 (13 weights, 28672 x 4096 to 256000 x 3584), 56 and 64 rows of 65536 columns at most 0.92 to 1.00, of 128256 and 151936 x 2048 0.96 to
+// 0.98, but 81920 to 151936 x 4096 up to 1.03; 128 x 128, 65 to 128 rows of 65536 columns at most 0.93 to 0.99, more columns up to 1.05; 128 x 192
+// 0.93 to 1.01 throughout; 192 x 128, 160 and 192 rows 0.97 to 1.04.
+bool past_caches(int M, int N, int K, int tm, int tn) {
+  if (M > tm || tm > 128 || !weights_pass(2LL * N * K)) return false;
+  return M <= 48 || N <= 65536 || tn == 192 || (tm == 64 && (long long)N * K < 5 << 26);
+}
+
 template <int EPI, int TM, int TN, int NST, bool NORM = false>
 int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
   constexpr int kLds = NST * (TM + TN) * 128;
@@ -352,7 +362,7 @@ int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
   (void)attr;
   p.tiles_m = (p.M + TM - 1) / TM;
   p.tiles_n = (p.N + TN - 1) / TN;
-  p.nt = p.tiles_m == 1 && weights_pass(2LL * p.N * p.K);
+  p.nt = past_caches(p.M, p.N, p.K, TM, TN);
   // W rows of a stride whose low bits are zero lie on few memory channels, and all tiles walk K in step (gemm2g.hip): another
   // first step for each column tile spreads them.  N x K at 24 / 64 / 128 rows, us, before -> after: 16384 x 2048 17 / 17 / 26 -> 15 /
   // 15 / 23, 28672 x 4096 50 / 54 / 59 -> 48 / 52 / 51, 32000 x 4096 55 / 57 / 64 -> 55 / 57 / 52, 8192 x 8192 33 / 33 / 44 -> 27 /
@@ -373,6 +383,9 @@ int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
 extern "C" int lwc_gemm1s_plan(int M, int N, int K, int epi, bool norm, long long max_splits);
 extern "C" int lwc_gemm1s(const void*, const void*, void*, const void*, int, int, int, int, int, int, int, float*, int*, const lwc::RowSumsq*,
                           const lwc::RopeKV*, hipStream_t);
+
+// (for tests)
+extern "C" int lwc_gemm2w_past_caches(int M, int N, int K, int tm, int tn) { return lwc::g2w::past_caches(M, N, K, tm, tn); }
 
 // epi 0: C = A W^T; 1: C = A W^T + R (R may be C); 2: C[:, :N/2] = silu(gate) * up over 32-row interleaved W (N % 64 == 0);
 // 3: C = A W^T + bias (R = bias [N]); 4: C = gelu(A W^T + bias) (exact erf GELU).

@@ -81,6 +81,18 @@ def test_untuned_rule_of_few_rows(N, K, epi, rows):
     assert {M: gemm_plan._untuned(M, N, K, epi) for M in rows} == rows
 
 
+@pytest.mark.parametrize("M,N,K,tile,past", [
+    (1, 8192, 2040, (64, 64), False), (1, 8192, 2048, (64, 64), True), (48, 256000, 3584, (64, 64), True), (49, 128256, 4096, (64, 64), False),
+    (64, 65536, 8192, (64, 64), True), (64, 128256, 2048, (64, 64), True), (64, 81920, 4096, (64, 64), False), (65, 65536, 8192, (64, 64), False),
+    (128, 65536, 8192, (128, 128), True), (128, 128256, 4096, (128, 128), False), (128, 128256, 4096, (128, 192), True), (129, 65536, 8192, (128, 192), False),
+    (160, 28672, 4096, (192, 128), False), (160, 128256, 4096, (192, 128), False)])
+def test_weights_past_the_caches_rule(M, N, K, tile, past):
+    """Weights pass the caches by where that measured faster: read by one tile of rows, and few rows or not too wide."""
+    from llm_weighted_consensus_amd import ops
+
+    assert ops.kernels().gemm2w_past_caches(M, N, K, *tile) == past
+
+
 @pytest.mark.parametrize("N,K,rows", [
     (4608, 12288, {1: "blas", 24: "blas"}), (4736, 11008, {1: "blas", 24: "blas"}), (4160, 13952, {8: "blas"}), (4744, 11264, {1: "g2", 24: "g2"}),
     (4096, 12288, {1: "blas", 16: "blas", 17: "g2"}), (4096, 13824, {16: "blas", 24: "g2"}), (4096, 13952, {1: "g2", 16: "g2"}), (4096, 11072, {1: "g2"}),
