@@ -35,7 +35,6 @@ struct Params {
   int tiles, wide;   // a run's tiles, and the blocks of each
   float* part;       // splits > 1: [N / 16][splits][1024] partial sums
   int* count;        // splits > 1: [runs * tiles] finished ranges (zero between launches)
-  int nt;            // weights_pass (common.h)
   int turned;        // a run's walk over its K range starts at a step of its own, 0 .. turned
   RowSumsq ss;       // NORM: read by EPI_PLAIN, EPI_SWIGLU and EPI_ROPE_KV, written by EPI_RESIDUAL
   RopeKV kv;         // EPI_ROPE_KV
@@ -59,7 +58,8 @@ constexpr int kRows = 64, kA = kRows * 128, kUnit = 16 * 128;  // bytes of 64 en
 constexpr int kSide = 8 * kRows * 4 + 16;                      // sums that waves exchange, and a flag
 
 // UW: the most units of a tile, 8, or 4: two waves share one, each with half of the rows.  NST steps of 128 entries in LDS.
-template <int EPI, bool NORM, int UW, int NST>
+// NT: the weights pass the caches by (weights_pass, common.h).
+template <int EPI, bool NORM, int UW, int NST, bool NT>
 __global__ void __launch_bounds__(512, 2) gemm1s_kernel(const Params p) {
   constexpr bool kPairs = EPI == EPI_SWIGLU || EPI == EPI_ROPE_KV;  // a unit is 8 columns and the 8 that meet them
   constexpr bool kScale = NORM && EPI != EPI_RESIDUAL, kSums = NORM && EPI == EPI_RESIDUAL;
@@ -113,14 +113,10 @@ __global__ void __launch_bounds__(512, 2) gemm1s_kernel(const Params p) {
     uint8_t* b = smem + buf * kStage;
 #pragma unroll
     for (int s = 0; s < 2; ++s) dma16(rX, b + s * kA + wid * 1024, voA, load_k + s * 128);
-    auto weights = [&](auto cp) {
 #pragma unroll
-      for (int j = 0; j < IW; ++j)
+    for (int j = 0; j < IW; ++j)
 #pragma unroll
-        for (int s = 0; s < 2; ++s) dma16<decltype(cp)::value>(rW, b + 2 * kA + s * UW * kUnit + mu * kUnit + (j + mr) * 1024, voW[j], load_k + s * 128);
-    };
-    if (p.nt) weights(std::integral_constant<int, kNT>{});
-    else weights(std::integral_constant<int, 0>{});
+      for (int s = 0; s < 2; ++s) dma16<NT ? kNT : 0>(rW, b + 2 * kA + s * UW * kUnit + mu * kUnit + (j + mr) * 1024, voW[j], load_k + s * 128);
     load_k += 256;
     load_k = load_k == past_k ? first_k : load_k;
     if (--load_left == 0) {
@@ -312,20 +308,24 @@ __global__ void __launch_bounds__(512, 2) gemm1s_kernel(const Params p) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (the loads past the end write zeros to LDS)
 }
 
-template <int EPI, bool NORM, int UW, int NST>
+template <int EPI, bool NORM, int UW, int NST, bool NT>
 int go(const Params& p, hipStream_t s) {
   constexpr int kLds = NST * 2 * (kA + UW * kUnit) + kSide;
   static_assert(kLds <= 160 * 1024, "LDS of a CU");
   static const hipError_t attr =
-      hipFuncSetAttribute((const void*)gemm1s_kernel<EPI, NORM, UW, NST>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+      hipFuncSetAttribute((const void*)gemm1s_kernel<EPI, NORM, UW, NST, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   (void)attr;
-  gemm1s_kernel<EPI, NORM, UW, NST><<<p.runs * p.splits, 512, kLds, s>>>(p);
+  gemm1s_kernel<EPI, NORM, UW, NST, NT><<<p.runs * p.splits, 512, kLds, s>>>(p);
   return (int)hipGetLastError();
 }
 
+// (Kernels of their own for NT: where a branch in the K loop chose, the compiler took each step for fewer loads than it has and waited for
+// later ones too early.  us, chosen so / now: residual 64 x 3072 x 4096 16.7 / 15.4, 33 x 8192 x 1024 12.8 / 10.9, 64 x 3072 x 768 10.4 / 9.3.)
 template <int EPI, bool NORM>
 int launch(const Params& p, hipStream_t s) {
-  return p.wide * (NORM && EPI == EPI_RESIDUAL ? 2 : 1) <= 4 ? go<EPI, NORM, 4, 4>(p, s) : go<EPI, NORM, 8, 3>(p, s);
+  const bool narrow = p.wide * (NORM && EPI == EPI_RESIDUAL ? 2 : 1) <= 4;
+  if (weights_pass(2LL * p.N * p.K)) return narrow ? go<EPI, NORM, 4, 4, true>(p, s) : go<EPI, NORM, 8, 3, true>(p, s);
+  return narrow ? go<EPI, NORM, 4, 4, false>(p, s) : go<EPI, NORM, 8, 3, false>(p, s);
 }
 
 // How the columns go over the CUs with K in so many ranges: as evenly as units allow (runs of a whole 64 columns each would start at rows
@@ -391,7 +391,7 @@ extern "C" int lwc_gemm1s(const void* A, const void* W, void* C, const void* R, 
   while (2 * turned + 2 <= K / 128 / splits) turned = 2 * turned + 1;
   const int blocks = N / (16 * grain);
   const Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc, c.runs, splits,
-                 blocks / c.runs, blocks % c.runs, c.tiles, c.wide, part, count, lwc::weights_pass(2LL * N * K), turned, ss != nullptr ? *ss : lwc::RowSumsq{},
+                 blocks / c.runs, blocks % c.runs, c.tiles, c.wide, part, count, turned, ss != nullptr ? *ss : lwc::RowSumsq{},
                  kv != nullptr ? *kv : lwc::RopeKV{}};
   if (ss != nullptr) {
     switch (epi) {

@@ -40,7 +40,6 @@ struct Params {
   uint8_t* mx_out;
   int s_rows;
   int turned;  // a tile's walk over K starts at a step of its own
-  int nt;  // weights_pass (common.h), for the groups of one tile
 };
 
 LWC_DEVICE float4v mfma8(const uint4v& a0, const uint4v& a1, const uint4v& b0, const uint4v& b1, const float4v& c, int sb) {
@@ -79,7 +78,8 @@ LWC_DEVICE void wait_steps(int n) {
   }
 }
 
-template <int MODE, int TM, int NST>
+// NT: the weights of groups of one tile pass the caches by (weights_pass, common.h).
+template <int MODE, int TM, int NST, bool NT>
 __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
   constexpr bool MXA = MODE == kMxA, BF = MODE == kBf16 || MODE == kBf16Swiglu;
   constexpr int TN = 128, kA = TM * 128, kS = kA + TN * 128, kStage = kS + (MXA ? 1024 : 0);  // rows, weights, scales
@@ -100,7 +100,7 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
     if (slot < nt) {
       m_begin = r0 + slot * TM;
       m_end = min(r1, m_begin + TM);
-      once = p.nt && nt == 1;
+      once = nt == 1;
       break;
     }
     slot -= nt;
@@ -135,7 +135,7 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
 #pragma unroll
       for (int i = 0; i < IW; ++i) dma16<decltype(cp)::value>(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], kt * 128);
     };
-    if (once) weights(std::integral_constant<int, kNT>{});
+    if (NT && once) weights(std::integral_constant<int, kNT>{});
     else weights(std::integral_constant<int, 0>{});
     if constexpr (MXA) dma4(rS, buf + kS + wid * 256, voS, kt * p.s_rows * 4);
   };
@@ -253,18 +253,18 @@ __global__ void __launch_bounds__(256, 2) gemm2g_kernel(const Params p) {
   }
 }
 
-template <int MODE, int TM, int NST>
+template <int MODE, int TM, int NST, bool NT>
 int launch(Params p, int rows, hipStream_t s) {
   constexpr int kLds = NST * ((TM + 128) * 128 + (MODE == kMxA ? 1024 : 0));
   static_assert(2 * kLds <= 160 * 1024 || (MODE == kMxA && TM == 192), "two workgroups share a CU's LDS");
   static const hipError_t attr =
-      hipFuncSetAttribute((const void*)gemm2g_kernel<MODE, TM, NST>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+      hipFuncSetAttribute((const void*)gemm2g_kernel<MODE, TM, NST, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   (void)attr;
   p.slots = (rows + TM - 1) / TM + p.G;
   p.n_tiles = (p.N + 127) / 128;
   const long long grid = 8LL * ((p.n_tiles + 7) / 8) * p.slots;
   if (grid >= (1LL << 31)) return -1;
-  gemm2g_kernel<MODE, TM, NST><<<(unsigned)grid, 256, kLds, s>>>(p);
+  gemm2g_kernel<MODE, TM, NST, NT><<<(unsigned)grid, 256, kLds, s>>>(p);
   return (int)hipGetLastError();
 }
 
@@ -295,7 +295,7 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
   using namespace lwc::g2g;
   if ((!row_off && G != 1) || K % 128 != 0 || K < 128 || N % 8 != 0 || rows <= 0) return -1;
   Params p{(const uint8_t*)A, (const uint8_t*)W, (lwc::bf16_t*)C, row_off, a_rows, a_scale, w_scale, G, N, K, lda, ldc, rows_a,
-                 rows, 0, 0, (const uint8_t*)a_mx, (uint8_t*)mx_out, s_rows, 0, 0};
+                 rows, 0, 0, (const uint8_t*)a_mx, (uint8_t*)mx_out, s_rows, 0};
   // The tile that most groups' rows fit, with room for an uneven routing: a second tile reads the weights again, and where the
   // columns give every CU a workgroup already some CUs walk K once more.  us at 64 / 128 / 192 rows a tile, 32 rows a group: bf16
   // [4096, 14336] x 8 (256 columns) 164 / 166 / 172, one expert with four times the rows 238 / 190 / 193, with 130 rows 254 /
@@ -325,10 +325,11 @@ extern "C" int lwc_gemm2g(const void* A, const void* W, void* C, const int* row_
   int tm = per <= (cols <= 128 ? 44 : 16) ? 64 : per <= 104 && !(cols > 128 && cols <= 256) ? 128 : 192;
   if (!row_off) tm = nt * ((rows + 63) / 64) <= 512 ? 64 : 128;
   // (160 rows a group on average: with more, 180 or 192 in each group, gate|up loses 1.5 % by it)
-  p.nt = per <= (row_off ? 160 : tm) && lwc::weights_pass((long long)G * N * K);
+  const bool past = per <= (row_off ? 160 : tm) && lwc::weights_pass((long long)G * N * K);
 #define LWC_G2G(M) \
   case M:          \
-    return tm == 64 ? launch<M, 64, 3>(p, rows, s) : tm == 128 ? launch<M, 128, 2>(p, rows, s) : launch<M, 192, 2>(p, rows, s);
+    if (past) return tm == 64 ? launch<M, 64, 3, true>(p, rows, s) : tm == 128 ? launch<M, 128, 2, true>(p, rows, s) : launch<M, 192, 2, true>(p, rows, s); \
+    return tm == 64 ? launch<M, 64, 3, false>(p, rows, s) : tm == 128 ? launch<M, 128, 2, false>(p, rows, s) : launch<M, 192, 2, false>(p, rows, s);
   switch (mode) {
     LWC_G2G(kPlain)
     LWC_G2G(kSwiglu)

@@ -33,7 +33,6 @@ struct Params {
   int splits;   // K ranges per tile
   float* part;  // splits > 1: [tiles][splits][TM * TN] partial tiles
   int* count;   // [tiles] finished ranges (zero between launches)
-  int nt;       // past_caches
   int turned;   // > 0: a tile's walk over its K range starts at a step of its own, 0 .. turned
 };
 
@@ -66,8 +65,8 @@ LWC_DEVICE void wait_rows() {
 constexpr int kGroupM = 8;
 
 // EPI_ROPE_KV (64 x 64 tiles, step_fuse.h): a tile takes 32 columns of a head and the 32 that rotate with them, D / 2 further.
-// NORM (64 x 64 tiles): the folded RMSNorm of step_fuse.h.
-template <int EPI, int TM, int TN, int NST, bool NORM>
+// NORM (64 x 64 tiles): the folded RMSNorm of step_fuse.h.  NT: the weights pass the caches by (past_caches).
+template <int EPI, int TM, int TN, int NST, bool NORM, bool NT>
 __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const typename ArgsOf<NORM>::type p) {
   static_assert((!NORM && EPI != EPI_ROPE_KV) || (TM == 64 && TN == 64), "one row of partial sums per lane group");
   constexpr bool kPairs = EPI == EPI_SWIGLU || EPI == EPI_ROPE_KV;  // columns that meet in a lane: groups of 32, two by two
@@ -115,12 +114,8 @@ __global__ void __launch_bounds__(256, 2) gemm2w_kernel(const typename ArgsOf<NO
   auto stage = [&](uint8_t* buf) {
 #pragma unroll
     for (int i = 0; i < IA; ++i) dma16(rA, buf + (i * 4 + wid) * 1024, voA[i], next_k);
-    auto weights = [&](auto cp) {
 #pragma unroll
-      for (int i = 0; i < IW; ++i) dma16<decltype(cp)::value>(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], next_k);
-    };
-    if (p.nt) weights(std::integral_constant<int, kNT>{});
-    else weights(std::integral_constant<int, 0>{});
+    for (int i = 0; i < IW; ++i) dma16<NT ? kNT : 0>(rW, buf + kA + (i * 4 + wid) * 1024, voW[i], next_k);
     next_k += 128;
     next_k = next_k == past_k ? first_k : next_k;
   };
@@ -354,15 +349,22 @@ bool past_caches(int M, int N, int K, int tm, int tn) {
   return M <= 48 || N <= 65536 || tn == 192 || (tm == 64 && (long long)N * K < 5 << 26);
 }
 
-template <int EPI, int TM, int TN, int NST, bool NORM = false>
-int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
+template <int EPI, int TM, int TN, int NST, bool NORM, bool NT>
+int go(const typename ArgsOf<NORM>::type& p, hipStream_t s) {
   constexpr int kLds = NST * (TM + TN) * 128;
   static const hipError_t attr =
-      hipFuncSetAttribute((const void*)gemm2w_kernel<EPI, TM, TN, NST, NORM>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
+      hipFuncSetAttribute((const void*)gemm2w_kernel<EPI, TM, TN, NST, NORM, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
   (void)attr;
+  gemm2w_kernel<EPI, TM, TN, NST, NORM, NT><<<p.tiles_m * p.tiles_n * p.splits, 256, kLds, s>>>(p);
+  return (int)hipGetLastError();
+}
+
+// (Kernels of their own for NT, as gemm1s.hip's.  us, by a branch / now: bias 256 x 4096 x 4096 27.5 / 26.2, 96 x 8192 x 8192 47.4 /
+// 44.8.)
+template <int EPI, int TM, int TN, int NST, bool NORM = false>
+int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
   p.tiles_m = (p.M + TM - 1) / TM;
   p.tiles_n = (p.N + TN - 1) / TN;
-  p.nt = past_caches(p.M, p.N, p.K, TM, TN);
   // W rows of a stride whose low bits are zero lie on few memory channels, and all tiles walk K in step (gemm2g.hip): another
   // first step for each column tile spreads them.  N x K at 24 / 64 / 128 rows, us, before -> after: 16384 x 2048 17 / 17 / 26 -> 15 /
   // 15 / 23, 28672 x 4096 50 / 54 / 59 -> 48 / 52 / 51, 32000 x 4096 55 / 57 / 64 -> 55 / 57 / 52, 8192 x 8192 33 / 33 / 44 -> 27 /
@@ -373,8 +375,9 @@ int launch(typename ArgsOf<NORM>::type p, hipStream_t s) {
   const bool turned = (NORM || EPI != EPI_PLAIN) && p.M <= 256 && (long long)p.tiles_m * p.tiles_n <= 1024 && (p.K % 2048 == 0 || p.K % 1024 != 0);
   p.turned = 0;  // (a power of two less one: a division would hold the first loads back)
   while (turned && 2 * p.turned + 2 <= p.K / 64 / p.splits) p.turned = 2 * p.turned + 1;
-  gemm2w_kernel<EPI, TM, TN, NST, NORM><<<p.tiles_m * p.tiles_n * p.splits, 256, kLds, s>>>(p);
-  return (int)hipGetLastError();
+  if constexpr (TM <= 128)
+    if (past_caches(p.M, p.N, p.K, TM, TN)) return go<EPI, TM, TN, NST, NORM, true>(p, s);
+  return go<EPI, TM, TN, NST, NORM, false>(p, s);
 }
 
 }  // namespace g2w
@@ -445,7 +448,7 @@ extern "C" int lwc_gemm2w(const void* A, const void* W, void* C, const void* R, 
   if (((long long)M + 63) / 64 * ((N + 63) / 64) * splits >= (1LL << 31)) return -1;
   if (tile == 4) return lwc_gemm1s(A, W, C, R, M, N, K, lda, ldc, epi, splits, part, count, ss, kv, s);
   const Params p{(const lwc::bf16_t*)A, (const lwc::bf16_t*)W, (lwc::bf16_t*)C, (const lwc::bf16_t*)R, M, N, K, lda, ldc, 0, 0,
-                 splits, part, count, 0, 0};
+                 splits, part, count, 0};
   if (ss != nullptr) {
     const NormParams np{p, *ss, kv != nullptr ? *kv : lwc::RopeKV{}};
     switch (epi) {
