@@ -133,10 +133,9 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
     151936 x 4096, 50304 and 151936 x 2048, 32768 x 5120, 65536 x 8192 0.46 to 1.00 (128256 x 4096, 5 rows 183 us -> 152; 33 to 64 rows
     up to 1.07; 30522 x 1024 is 16 us on either).
 
-    Down at up to 24 rows, 12 widths and 16 depths of 4096 to 5120 x 11008 to 14336: with 64 column tiles (4096) or 75 to 80 (4744 to 5120),
-    whose K ranges give nearly every CU a workgroup, 0.51 to 1.01, 0.58 at 4096 and 5120 x 11008; but up to 16 rows of 4096 x the
-    multiples of 512 below 14336, for which the library has its best kernels, 1.01 to 1.08, and below 8 rows of 4744 to 5120 x 13824 1.02
-    to 1.07. 65 to 74 tiles go to the weight stream: 4160 to 4736 x the same 0.76 to 1.47. (4096 x 8192 up to 1.08.)"""
+    Down at up to 24 rows, 12 widths and 16 depths of 4096 to 5120 x 11008 to 14336: 0.49 to 1.02, 0.57 at 4096 and 5120 x 11008, but for
+    the multiples of 512 below 14336, for which the library has its best kernels: 4096 up to 16 rows 0.98 to 1.04, below 8 rows 4160 to
+    4672 0.94 to 1.06 and the wider 13824 0.99 to 1.03. (4096 x 8192 up to 1.08.)"""
     size = N * K
     if epi == "swiglu":
         if M > 4608:  # (M * N: 32-bit byte offsets)
@@ -153,8 +152,8 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
         return "g2"
     if epi == "plain" and M <= 32 and N >= 32000 and 2048 <= K <= 8192 and 3 << 25 <= size < 1 << 30:
         return "g2"
-    if epi == "residual" and M <= 24 and (N == 4096 or 4736 < N <= 5120) and 11008 <= K <= 14336 and (
-            K % 512 or K > 13824 or M > 16 or N > 4096 and (M >= 8 or K < 13824)):
+    if epi == "residual" and M <= 24 and 4096 <= N <= 5120 and 11008 <= K <= 14336 and (
+            K % 512 or K > 13824 or M > 16 or N > 4096 and (M >= 8 or N >= 4736 and K < 13824)):
         return "g2"
     if M <= 16 and K <= 4096 and N <= 8 * K and 1 << 22 <= size <= 1 << 24:
         return "gv"

@@ -94,11 +94,11 @@ def test_weights_past_the_caches_rule(M, N, K, tile, past):
 
 
 @pytest.mark.parametrize("N,K,rows", [
-    (4608, 12288, {1: "blas", 24: "blas"}), (4736, 11008, {1: "blas", 24: "blas"}), (4160, 13952, {8: "blas"}), (4744, 11264, {1: "g2", 24: "g2"}),
+    (4608, 12288, {1: "blas", 7: "blas", 8: "g2", 24: "g2"}), (4736, 11008, {1: "g2", 24: "g2"}), (4160, 13952, {1: "g2"}), (4744, 11264, {1: "g2", 24: "g2"}),
     (4096, 12288, {1: "blas", 16: "blas", 17: "g2"}), (4096, 13824, {16: "blas", 24: "g2"}), (4096, 13952, {1: "g2", 16: "g2"}), (4096, 11072, {1: "g2"}),
-    (5120, 13824, {1: "blas", 7: "blas", 8: "g2", 24: "g2"}), (5120, 13312, {1: "g2"}), (4992, 14080, {5: "g2"})])
+    (5120, 13824, {1: "blas", 7: "blas", 8: "g2", 24: "g2"}), (5120, 13312, {1: "g2"}), (4672, 13312, {1: "blas", 8: "g2"}), (4992, 14080, {5: "g2"})])
 def test_untuned_down_of_few_rows(N, K, rows):
-    """Inside the range of down projections that gemm2w takes: widths and depths at which the library measured faster keep it."""
+    """Inside the range of down projections that gemm2w takes: rows, widths and depths at which the library measured faster keep it."""
     assert {M: gemm_plan._untuned(M, N, K, "residual") for M in rows} == rows
 
 
