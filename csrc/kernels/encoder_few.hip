@@ -1,4 +1,5 @@
-// A post-norm encoder over few packed rows (a search query, a handful of short texts), the whole stack in one launch.
+// A post-norm encoder over few packed rows (a search query, a handful of short texts), in two launches: begin_kernel sums the
+// embeddings and clears the flags, chain_kernel is the whole stack (of up to 24 layers; further ones two launches more).
 //
 // A text of 12 tokens through bge-small is 12 layers of dependent stages over 42 MB of weights, 7 us of reading: what counts is how
 // many stages there are, and what each waits for.  A stage is cut into items of a workgroup each:
@@ -15,13 +16,21 @@
 // before its own, by workgroups that are running: whatever else runs on the GPU, another such launch too, the lowest item that is
 // not done waits for nothing.
 //
-// As kernels of their own, four or five a layer, a stage was 4.3 us; here it is 2.9: 0.3 us until its stores are in memory, 0.4 to 1 until
+// As kernels of their own, four or five a layer, a stage was 4.3 us; here it is 2.9 (bge-small: 49 of them): 0.3 us until its stores are in memory, 0.4 to 1 until
 // the flags are seen, 0.5 to 0.7 for the rows, 0.45 for a norm, 0.6 for the products and their sum (1.2 with the attention).  One
 // MI355X, us a call, kernels / one launch (rows): bge-small 198 / 133 (3), 214 / 143 (14), 282 / 190 (32); bge-base 250 / 219, 274 / 232, 361 / 316;
 // bge-large 632 / 558, 699 / 588, 918 / 726.  On the way there, bge-small, 14 rows: 212 as the kernels were; the stage before asked
 // first and seldom, half a wave a row in the norm 184; the flags in eight copies 174, one for each XCD 153; what is
 // handed on in a place of its own, read through the caches, and 32 columns an item 160 (of 174); one item a CU at a time 143 (of 154; two:
 // bge-base 274 for 232).
+//
+// What it costs others: a workgroup waits in 81 KiB of its CU's LDS, up to 250 of them for the 130 to 720 us of a call, and kernels of another
+// stream that want more than the rest wait for it.  Queries of 12 tokens one behind the other beside decode steps, us a step alone, then a
+// step and a query beside each other, kernels / here: llama 1 545, 600 and 726 / 523, 667 and 220; 61 rows 790, 836 and 701 / 770, 1095 and 219;
+// merudra 64 1084, 1137 and 597 / 1021, 1125 and 261; bge-large beside llama 1 545, 657 and 2400 / 523, 828 and 986.  A query takes 24 to 65 us
+// from the steps beside it (28 to 67 before), bge-large's 360 (410), but there are up to three times as many.  And memory: each layer's
+// rows keep a place of their own until the call's end, layers + 1 times Rows::kBytes a row: 4 MB at bge-small's 32 rows, 13 at
+// bge-base's, 16 and 26 at bge-large's 16 and 32.
 //
 // project: 16 or 32 output columns, 8 waves over K in steps of 32 (wave w: steps w, w + 8, ..), W the A operand and the rows the B
 // operand of mfma_f32_16x16x32_bf16, so that a lane holds four consecutive columns of one row.  qkv_attn: a head, 24 (16 columns,

@@ -147,8 +147,9 @@ __global__ void __launch_bounds__(256) rmsnorm_wave_kernel(const bf16_t* __restr
 // A workgroup of four waves per row, the row in registers (d = 256 * 8 * NV): the same function, one barrier (two with the
 // quantisation), every load of the row, the residual and the weight on its way before the first use.  Bound by memory, and by one trip
 // to it below some 1000 rows.  us, a wave per row / so, with residual and e4m3 rows: 512 rows of 4096 5.9 / 4.3, 1095 8.1 / 6.4,
-// 8682 39.5 / 36.4 (6.8 TB/s), 512 of 8192 9.2 / 6.0, 4096 42.7 / 35.2; bf16 rows alone: 512 of 4096 3.6 / 3.1, 4096 10.8 / 11.3,
-// 8682 21.8 / 21.5.
+// 8682 39.5 / 36.4 (6.8 TB/s), 512 of 8192 9.2 / 6.0, 4096 42.7 / 35.2; bf16 rows alone, just written, in a stream of other kernels
+// (each with 3 us of its events): 2048 of 4096 10.1 / 9.8, 4096 14.1 / 13.8, 8682 25.2 / 24.2.  (Called again and again on the same rows, which
+// L2 then holds, 3072 of 4096 7.9 / 8.6, 4096 10.6 / 10.8.)
 template <int NV, bool kResidual, bool kQuant>
 __global__ void __launch_bounds__(256) rmsnorm_row_kernel(const bf16_t* __restrict__ x, bf16_t* __restrict__ residual,
                                                           const bf16_t* __restrict__ w, bf16_t* __restrict__ y, int d, float eps,

@@ -18,9 +18,9 @@ LWC_DEVICE float4v mfma16(const short8& a, const short8& b, const float4v& c) {
 // cache into the operands — no LDS: a K row's 16 bytes are an A operand as they lie, the interleaved V word is a
 // B operand as it lies.  Same arithmetic as the portion kernel (hi + lo halves of q and of the weights, bias
 // table, fp32 online softmax).  Bound by the reads of the cache: 64 sequences of 500 to 1500 keys (1000 on average), 32
-// heads over 8 of 128 entries, take 54 us for 258 MB (42 us at the rate of a plain read of memory) in tables of 4096 keys.
-// With the splits cut for the table's width and every load of a tile waited for on its own it took 137 us, and 189 instead
-// of 104 us at 2048 keys each.  Each split leaves an unnormalised partial (o, m, l); the reduce kernel merges
+// heads over 8 of 128 entries, take 67 us for 258 MB from memory (42 us at the rate of a plain read) in tables of 4096 keys.
+// (With the splits cut for the table's width and every load of a tile waited for on its own 2.5 times as long, 1.8 times at
+// 2048 keys each.)  Each split leaves an unnormalised partial (o, m, l); the reduce kernel merges
 // them (splits == 1: still through the reduce, which then only normalises).
 struct WAttnDecodeParams {
   const float* q;          // [B, H*D]
@@ -93,7 +93,8 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
   // load's wait, in the branch that loads: behind it, or behind a choice between lanes and table, the compiler waits for every load on
   // its way, three times a tile and, with wide rows, at every row that a thread stages.  us, so / here, cold: 576 / 512 entries, 32
   // heads, 64 rows of 500 to 1500 keys 98 / 61, of 4000 199 / 122, one of 4000 54 / 33; 320 / 256, 16 heads 49 / 32, 97 / 68, 36 / 25; 128 /
-  // 128, 32 heads over 8, 255 rows of 400 58 / 52, 64 of 20 to 60 15.6 / 13.0, 64 of 500 to 1500 67 / 66.5, which memory bounds.)
+  // 128, 32 heads over 8, 255 rows of 400 89 / 87, 64 of 20 to 60 15.6 / 13.0, 64 of 500 to 1500 67.5 / 67.4, which memory bounds; over 32,
+  // 64 of 100 to 4000 400 / 337, but of 1000 each 181 / 188 and with a bias 180 / 194: more in flight is no gain to equal rows that fill the chip.)
   int pg_base = 0, my_page = 0;
   auto look_up = [&](int t0) {
     pg_base = page_ix(t0);
@@ -198,7 +199,7 @@ __global__ void __launch_bounds__(64 * NW * NC) window_attn_decode_kernel(const 
     }
     if constexpr (!kStage) {
 #pragma unroll
-      for (int n = 0; n < NVW; n += 2) {  // two columns, 32 n + 2 r16 and the one after it, four keys of each
+      for (int n = 0; n < NVW; n += 2) {  // two columns, 16 n + 2 r16 and the one after it, four keys of each
         vf[n] = *reinterpret_cast<const uint4v*>(va + 64 * n);
         vf[n + 1] = *reinterpret_cast<const uint4v*>(vb + 64 * n);
       }

@@ -345,7 +345,9 @@ __global__ void __launch_bounds__(T, SLOTS <= 4 ? (PROC && TOPK ? 7 : 8) : SLOTS
   // (With the nt bit where the logits are many: read once, they neither stay in the last-level cache nor push out what it holds.  All
   // rows of pairs, us without / with it: 4096 rows of 128256 greedy 215 / 177, top-p 0.95 318 / 307, top-k 40 359 / 344, 1500 greedy 85 / 69,
   // 1024 47 / 48, with the logits written just before 58 / 43; longer rows from 128 MiB of logits on: 4096 of 151936 greedy 286 / 241,
-  // 1000 73 / 68, written just before 79 / 59, 64 11.2 / 12.4.  Shorter rows level within 5 % either way, so not there.)
+  // 1000 73 / 68, written just before 79 / 59, 64 11.2 / 12.4.  Shorter rows level within 5 % either way, so not there.  Rows of pairs that the
+  // last-level cache holds whole, read and written again there just before, lose: 1024 of 102400 greedy 42.4 / 44.5, top-k 40 102 / 105; written
+  // by the product with the head 54.5 / 47.6 and 107 / 103.)
   uint4v row[RS];
   const uint32_t* lmask =
       (PROC && p.mask_logprobs && p.mask && p.mask_rows[b] >= 0) ? p.mask + (size_t)p.mask_rows[b] * (p.V >> 5) : nullptr;

@@ -39,7 +39,7 @@ from .packing import pack_ids
 POOL_MODES = {"cls": ops.POOL_CLS, "mean": ops.POOL_MEAN, "last": ops.POOL_LAST}
 
 
-FEW_ROWS = 32  # up to here (what ops.encoder_few takes) its one launch leads the layers below, seven kernels each: 1.2 to 2.2x
+FEW_ROWS = 32  # up to here (what ops.encoder_few takes) its two launches lead the layers below, seven kernels each: 1.2 to 2.2x
 
 
 @dataclass
