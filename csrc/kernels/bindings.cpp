@@ -1026,6 +1026,10 @@ c10::optional<at::Tensor> encoder_layers_mixed(at::Tensor x, const std::vector<a
                           int64_t H, int64_t Dh, double scale, double eps, const std::vector<int64_t>& cores, bool fuse_o,
                           bool fuse_f, const c10::optional<at::Tensor>& part, const c10::optional<at::Tensor>& count) {
   for (int64_t c : cores) TORCH_CHECK(c >= 0 && c <= 3, "encoder_layers_mixed: cores are 0 to 3, not ", c);
+  // (the library's results go into tensors that are there: nothing that a gradient is asked of)
+  if (at::GradMode::is_enabled())
+    for (const at::Tensor& t : weights)
+      if (t.requires_grad()) return c10::nullopt;
   return run_encoder_layers(x, weights, cu, max_len, H, Dh, scale, eps, cores, fuse_o, fuse_f, part, count);
 }
 

@@ -573,10 +573,11 @@ def encoder_layers(x: torch.Tensor, weights: Sequence[torch.Tensor], cu: torch.T
 def encoder_layers_mixed(x: torch.Tensor, weights: Sequence[torch.Tensor], cu: torch.Tensor, max_len: int, H: int, Dh: int,
                          scale: float, eps: float, cores: Sequence[int], fuse_o: bool, fuse_f: bool) -> Optional[torch.Tensor]:
     """:func:`encoder_layers` where ``cores`` may name the library (0), whose results go into tensors that are there already: None,
-    and nothing done, also where something records, transforms or watches library calls (``gemm_plan._plain``)."""
-    from .gemm_plan import _plain
+    and nothing done, also where something records, transforms or watches library calls (``gemm_plan._unseen``; the native code asks for
+    requires_grad, which takes 29 us from here for 288 weights)."""
+    from .gemm_plan import _unseen
 
-    if not _plain(x, *weights):
+    if not _unseen(x, *weights):
         return None
     part, count = _split_workspace(x.device) or (None, None)
     return kernels().encoder_layers_mixed(x, weights, cu, int(max_len), int(H), int(Dh), float(scale), float(eps), cores, bool(fuse_o),

@@ -32,7 +32,6 @@ use hipBLASLt, but where :func:`_untuned` names a core.  ``LWC_GEMM=blas|g8|g4|g
 from __future__ import annotations
 
 import logging
-import operator
 import os
 from typing import Dict, Optional, Tuple
 
@@ -160,20 +159,20 @@ def _untuned(M: int, N: int, K: int, epi: str) -> str:
     return "g2" if 32 < M <= 64 and (N < 8192 or K <= 2048) and 1 << 24 <= size <= 1 << 26 else "blas"
 
 
-_asks_grad = operator.attrgetter("requires_grad")
-
-
-def _plain(*ts: torch.Tensor) -> bool:
-    """Whether a raw kernel may take these tensors' place in a torch call: nothing records, transforms or watches it (autograd,
-    forward-mode duals, vmap and the other function transforms, fake and other subclasses, dispatch modes, tracing)."""
+def _unseen(*ts: torch.Tensor) -> bool:
+    """Whether no one but autograd could see or transform a torch call of these tensors: no forward-mode duals, vmap or other function
+    transforms, fake and other subclasses, dispatch modes, tracing."""
     if not set(map(type, ts)) <= {torch.Tensor, torch.nn.Parameter}:
-        return False
-    if torch.is_grad_enabled() and any(map(_asks_grad, ts)):
         return False
     if torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_dispatch_stack() or \
             torch.jit.is_tracing() or torch.compiler.is_compiling():
         return False
     return forward_ad._current_level < 0 or all(forward_ad.unpack_dual(t).tangent is None for t in ts)
+
+
+def _plain(*ts: torch.Tensor) -> bool:
+    """Whether a raw kernel may take these tensors' place in a torch call: nothing records, transforms or watches it."""
+    return not (torch.is_grad_enabled() and any(t.requires_grad for t in ts)) and _unseen(*ts)
 
 
 def _backend(x: torch.Tensor, w: torch.Tensor, epi: str, ws, acc: Optional[torch.Tensor] = None):
