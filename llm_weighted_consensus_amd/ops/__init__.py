@@ -941,10 +941,12 @@ def _fp8_gemm8p(M: int, N: int, K: int, ws, *operands: torch.Tensor) -> bool:
     than 128 tiles of 256 x 256, or from 64 on where K is long and may be cut (``ws``).  us, gemm2g / gemm8p, at 64, 128 and 144 to 160 tiles: K
     2048 14.1 / 23.6, 22.2 / 24.4, 32.7 / 25.1; K 4096 23.5 / 34.1, 34.9 / 37.9, 47.6 / 37.1; K 8192 40.0 / 42.3, 60.7 / 60.9, 100.2 / 69.7; K 14336 66.0 /
     55.1, 101.3 / 91.3, 167.4 / 115.3, at 48 tiles 53.1 to 65.6 / 57.6 to 67.3, at 32 53.2 / 46.8.  K from 512 on: 8682 x 4096 x 512 from MX, gemm8g / gemm8p, 42.8 / 33.0,
-    8682 x 8192 x 512 SwiGLU to MX 69.5 / 57.5, but at K 256 and 128 22.8 / 33.0 and 22.7 / 62.3.
+    8682 x 8192 x 512 SwiGLU to MX 69.5 / 57.5, but at K 256 and 128 22.8 / 33.0 and 22.7 / 62.3. Up to 256 tiles, one each for gemm8g's
+    workgroups, from 1024 on: gemm8p has a workgroup for eight K steps of 128, and fewer than tiles below. gemm8p over gemm8g at 136 to 256 tiles: K 512 to
+    896 1.14 to 1.46, K 1024 0.83 to 0.97; at 264 to 768 tiles 0.76 to 0.97 (2048, 4096 and 8192 columns, plain, from and to MX).
     ``operands``: rows and pointers that gemm8p wants at 16 bytes; for others gemm8g_fp8 says what it takes."""
     tiles = -(-M // 256) * -(-N // 256)
-    return K >= 512 and (tiles > 128 or (tiles >= 64 and K >= 12288 and ws is not None)) and all(
+    return K >= (512 if tiles > 256 else 1024) and (tiles > 128 or (tiles >= 64 and K >= 12288 and ws is not None)) and all(
         t.stride(1) == 1 and t.stride(0) * t.element_size() % 16 == 0 and t.stride(0) < 1 << 26 and t.data_ptr() % 16 == 0 for t in operands)
 
 

@@ -81,6 +81,17 @@ def test_untuned_rule_of_few_rows(N, K, epi, rows):
     assert {M: gemm_plan._untuned(M, N, K, epi) for M in rows} == rows
 
 
+@pytest.mark.parametrize("M,N,K,own", [(4096, 4096, 512, False), (4097, 4096, 512, True), (4096, 4096, 896, False), (4096, 4096, 1024, True),
+                                       (2048, 4096, 1024, False), (2049, 4096, 1024, True), (5000, 2048, 768, False), (8682, 2048, 512, True),
+                                       (8682, 2048, 384, False), (1024, 4096, 12288, True), (1024, 4096, 8192, False)])
+def test_dense_fp8_core_rule(M, N, K, own):
+    """Which of the dense fp8 cores measured faster: gemm8p's from 1024 deep on where its tiles are at most the CUs, from 512 beyond."""
+    from llm_weighted_consensus_amd import ops
+
+    x, w = (torch.empty(r, K, dtype=torch.float8_e4m3fn) for r in (M, N))
+    assert ops._fp8_gemm8p(M, N, K, object(), x, w) == own
+
+
 @pytest.mark.parametrize("M,N,K,tile,past", [
     (1, 8192, 2040, (64, 64), False), (1, 8192, 2048, (64, 64), True), (48, 256000, 3584, (64, 64), True), (49, 128256, 4096, (64, 64), False),
     (64, 65536, 8192, (64, 64), True), (64, 128256, 2048, (64, 64), True), (64, 81920, 4096, (64, 64), False), (65, 65536, 8192, (64, 64), False),
